@@ -43,12 +43,16 @@ PI_ADDR KSplit cut_k(int K, int splits, int quantum) {
 struct WaveRange {
   int k0, k1;
 };
+// The w-th of `waves` shares of [kb0, kb1), in whole steps.
+PI_ADDR WaveRange wave_share(int kb0, int kb1, int waves, int wave) {
+  const int per_wave = ((kb1 - kb0 + waves * KSTEP - 1) / (waves * KSTEP)) * KSTEP;
+  const int k0 = kb0 + wave * per_wave;
+  return WaveRange{k0, imin(kb1, k0 + per_wave)};
+}
 PI_ADDR WaveRange skinny_wave_range(int K, int k_per_block, int split, int wave) {
   const int kb0 = split * k_per_block;
   const int kb1 = imin(K, kb0 + k_per_block);
-  const int per_wave = ((kb1 - kb0 + 4 * KSTEP - 1) / (4 * KSTEP)) * KSTEP;
-  const int k0 = kb0 + wave * per_wave;
-  return WaveRange{k0, imin(kb1, k0 + per_wave)};
+  return wave_share(kb0, kb1, 4, wave);
 }
 
 // Row part of a lane's weight address for row tile t of the block whose first row is n0 (lane

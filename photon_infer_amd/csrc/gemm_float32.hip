@@ -1,0 +1,462 @@
+// float32 matrix products on the matrix cores: C[M, N] (+)= A[M, K] . W[N, K]^T with 32-bit operands, products and sums
+// (v_mfma_f32_32x32x2_f32 and v_mfma_f32_16x16x4_f32; 157 TFLOP/s on this chip, twice the vector unit's rate without
+// packed instructions).  They carry the float32 path's products; gemm_general.hip keeps mixed types and odd strides.
+//
+// K and the row strides are multiples of 4 and the operands 16-byte aligned.  A row of 32 floats is 128 bytes, as a row
+// of 64 bfloat16 is, so both kernels move their operands exactly as the bfloat16 kernels do and share those kernels'
+// address arithmetic (addressing.h), in units of two bytes: every `2 *` below turns floats into such units.
+//
+// Up to 32 rows (decode steps): gemm_float32_rows_kernel, bound by the weights' way from memory.  More rows:
+// gemm_float32_tile_kernel, bound by the matrix cores; where its tiles are few, k is cut over blocks and
+// pi_splitk_reduce adds the pieces in order.
+#include "addressing.h"
+#include "mfma.h"
+
+#define FSTEP 32                      // floats of k per step: 128 bytes of a row
+#define ROWS_MAX_M 32                 // up to this many rows of activations the weight-streaming kernel is taken
+#define ROWS_SPLIT_MIN_K 4096
+
+// ------------------------------------------------------------------ few rows: stream the weights
+// The weights are the row operand, the activations the column operand.  A block is WAVES waves on the same RT * 16
+// weight rows, each on a share of k; a lane fetches 32 contiguous bytes of a weight row per step, the four lane groups
+// of a row 128, and a wave keeps DEPTH steps of loads in flight.  Activations go through the wave's own patch of LDS,
+// turned so that neither side has bank conflicts, as in the bfloat16 kernel.  The waves' sums meet in LDS, in pairs.
+// See launch_rows() for the shapes.
+template <int MB, int RT, int WAVES>
+union RowsLds {
+  float red[WAVES][RT * 16][MB * 16 + 1];
+  u32x4_t xs[WAVES][MB * 8 * 16];
+};
+
+template <int MB, int RT, int WAVES, int DEPTH, bool ACCUM>
+__global__ __launch_bounds__(WAVES * 64) void gemm_float32_rows_kernel(float* __restrict__ C, long ldc, const float* __restrict__ X, long ldx,
+                                                                       const float* __restrict__ W, long ldw, int M, int N, int K,
+                                                                       int k_per_block, float* __restrict__ part) {
+  constexpr int ROWS = RT * 16;
+  __shared__ RowsLds<MB, RT, WAVES> lds;
+  const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
+  const int lr = lane % 16, lg = lane / 16;
+  const long n0 = (long)blockIdx.x * ROWS;
+  const addressing::WaveRange range = addressing::wave_share(2 * (int)blockIdx.y * k_per_block, 2 * min(K, (int)(blockIdx.y + 1) * k_per_block), WAVES, wave);
+  const int k0 = range.k0, k1 = range.k1;                 // in units of two bytes, as all addresses below
+  const int steps = k1 > k0 ? (k1 - k0 + addressing::KSTEP - 1) / addressing::KSTEP : 0;
+  const bf16_t* Wh = reinterpret_cast<const bf16_t*>(W);
+  const bf16_t* Xh = reinterpret_cast<const bf16_t*>(X);
+
+  const bf16_t* wrow[RT];
+#pragma unroll
+  for (int t = 0; t < RT; ++t) wrow[t] = Wh + addressing::skinny_w_base(0, n0, t, lr, lg, N, 2 * K, 2 * ldw);
+  const int x_loads = __builtin_amdgcn_readfirstlane((M + 7) / 8);
+  const int xt = lane / 8, xp = lane % 8;
+  const bf16_t* xsrc[MB * 2];
+  int xdst[MB * 2];
+#pragma unroll
+  for (int i = 0; i < MB * 2; ++i) {
+    const int token = i * 8 + xt;
+    xsrc[i] = Xh + addressing::skinny_x_base(token, M, 2 * ldx, xp);
+    xdst[i] = ((token / 16) * 8 + xp) * 16 + ((token + 2 * xp) & 15);
+  }
+  u32x4_t* xs = lds.xs[wave];
+  int xfrag[MB][2];
+#pragma unroll
+  for (int c = 0; c < MB; ++c)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) xfrag[c][h] = (c * 8 + lg * 2 + h) * 16 + ((lr + 2 * (lg * 2 + h)) & 15);
+
+  f32x4_t acc[RT][MB];
+#pragma unroll
+  for (int t = 0; t < RT; ++t)
+#pragma unroll
+    for (int c = 0; c < MB; ++c) acc[t][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+  // pieces beyond k1 (the last, partial step) are fetched from a stand-in inside the row and count as zero; steps beyond
+  // the last fetch the last again, so that the loads in flight are a number the waits can count on
+  u32x4_t wq[DEPTH][RT][2], xq[DEPTH][MB * 2];
+  auto fetch = [&](const int s, const int j) {
+    const int kk = k0 + min(s, steps - 1) * addressing::KSTEP;
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) wq[j][t][h] = *reinterpret_cast<const u32x4_t*>(wrow[t] + addressing::skinny_w_step(0, false, kk, h, lg, k0, k1));
+#pragma unroll
+    for (int i = 0; i < MB * 2; ++i)
+      if (i == 0 || i < x_loads) xq[j][i] = *reinterpret_cast<const u32x4_t*>(xsrc[i] + addressing::skinny_x_step(false, kk, xp, k0, k1));
+  };
+  auto step = [&](const int s, const int j) {
+    const int kk = k0 + s * addressing::KSTEP;
+    f32x4_t w[RT][2];
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        w[t][h] = __builtin_bit_cast(f32x4_t, addressing::skinny_w_used(false, kk, h, lg, k1) ? wq[j][t][h] : u32x4_t{0u, 0u, 0u, 0u});
+    const bool x_ok = kk + xp * 8 < k1;
+#pragma unroll
+    for (int i = 0; i < MB * 2; ++i)
+      if (i == 0 || i < x_loads) xs[xdst[i]] = x_ok ? xq[j][i] : u32x4_t{0u, 0u, 0u, 0u};
+    fetch(s + DEPTH, j);
+    // the wave reads what its own lanes wrote: LDS serves one wave's accesses in order
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int c = 0; c < MB; ++c) {
+      // a quarter of the step in an accumulator of its own, then all into the running sum: chains of 8 products and one
+      // of steps instead of one of all k (at k = 2,048 off by 1e-7 of the result's norm instead of 4e-7)
+      f32x4_t sum[RT][4];
+#pragma unroll
+      for (int t = 0; t < RT; ++t)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) sum[t][u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const f32x4_t x = __builtin_bit_cast(f32x4_t, xs[xfrag[c][h]]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int t = 0; t < RT; ++t) sum[t][h * 2 + e % 2] = mfma16_f32(w[t][h][e], x[e], sum[t][h * 2 + e % 2]);
+      }
+#pragma unroll
+      for (int t = 0; t < RT; ++t) acc[t][c] += (sum[t][0] + sum[t][1]) + (sum[t][2] + sum[t][3]);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+  if (steps > 0) {
+#pragma unroll
+    for (int j = 0; j < DEPTH; ++j) fetch(j, j);
+    int s0 = 0;
+    for (; s0 + DEPTH <= steps; s0 += DEPTH) {
+#pragma unroll
+      for (int j = 0; j < DEPTH; ++j) step(s0 + j, j);
+    }
+#pragma unroll
+    for (int j = 0; j < DEPTH - 1; ++j)
+      if (s0 + j < steps) step(s0 + j, j);
+  }
+  __syncthreads();                      // the partial tiles take the place of the staged activations
+#pragma unroll
+  for (int t = 0; t < RT; ++t)
+#pragma unroll
+    for (int c = 0; c < MB; ++c)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) lds.red[wave][t * 16 + lg * 4 + r][c * 16 + lr] = acc[t][c][r];
+  __syncthreads();
+  for (int idx = tid; idx < ROWS * MB * 16; idx += WAVES * 64) {
+    const int nl = idx % ROWS, m = idx / ROWS;
+    if (m >= M || n0 + nl >= N) continue;
+    float v[WAVES];
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) v[w] = lds.red[w][nl][m];
+#pragma unroll
+    for (int gap = 1; gap < WAVES; gap *= 2)
+#pragma unroll
+      for (int w = 0; w < WAVES; w += 2 * gap) v[w] += v[w + gap];
+    if (gridDim.y > 1) {
+      part[((long)blockIdx.y * M + m) * N + n0 + nl] = v[0];
+    } else {
+      float* c = C + m * ldc + n0 + nl;
+      *c = ACCUM ? *c + v[0] : v[0];
+    }
+  }
+}
+
+// ------------------------------------------------------------------ many rows: tiles
+// A block-wide barrier that waits for this wave's LDS accesses and for all but its last LOADS loads from memory;
+// __syncthreads() would wait for every load on its way into LDS.
+template <int LOADS>
+__device__ inline void block_barrier_keeping_loads() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0x0070 | (LOADS & 15) | ((LOADS >> 4) << 14));      // vmcnt LOADS, lgkmcnt 0
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// Block tile TM x TN, four waves in 2 x 2, slabs of 32 floats of k that go from memory straight into LDS through a ring
+// of NB buffers (rows of 128 bytes, their 16-byte pieces turned by (row / 2) % 8 as in gemm_mfma.hip).  A matrix
+// instruction takes 64 cycles for two registers of operands, so LDS and its reads have time to spare and the tile only
+// has to be large enough for L2: 32 / 21 / 16 flops per byte at 128 x 128 / 128 x 64 / 64 x 64.  What decides is how the
+// tiles fill the chip, see plan().  Every output is summed over k in the same order in every tile shape.
+template <int TM, int TN, int NB, bool ACCUM>
+__global__ __launch_bounds__(256) void gemm_float32_tile_kernel(float* __restrict__ C, long ldc, const float* __restrict__ A, long lda,
+                                                                const float* __restrict__ W, long ldw, int M, int N, int K, int tiles_n,
+                                                                int k_per_split, float* __restrict__ part) {
+  extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
+  constexpr int ROW = 64;                        // a row of a slab: 128 bytes, in units of two
+  constexpr int AI = TM / 32, WI = TN / 32;      // load instructions of a wave per slab: eight rows each
+  constexpr int WM = TM / 64, WN = TN / 64;      // a wave's 32 x 32 tiles
+  uint16_t* As = lds;                            // [NB][TM][ROW]
+  uint16_t* Ws = lds + NB * TM * ROW;            // [NB][TN][ROW]
+  const int tid = threadIdx.x, lane = tid % 64;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+  const int wm = wave / 2, wn = wave % 2;
+  const int k_lo = 2 * (int)blockIdx.y * k_per_split, k_hi = 2 * min(K, (int)(blockIdx.y + 1) * k_per_split);
+  const int tiles_m = gridDim.x / tiles_n;
+  int tile_m, tile_n;
+  if (tiles_n % 8 == 0) {                        // a die streams its own slice of W and walks the row tiles of a column first
+    const int die = blockIdx.x % 8, local = blockIdx.x / 8;
+    tile_n = die * (tiles_n / 8) + local / tiles_m;
+    tile_m = local % tiles_m;
+  } else {
+    tile_m = blockIdx.x / tiles_n;
+    tile_n = blockIdx.x % tiles_n;
+  }
+  const long m0 = (long)tile_m * TM, n0 = (long)tile_n * TN;
+  const int a_rows = (int)min((long)TM, M - m0), w_rows = (int)min((long)TN, N - n0);
+#if defined(__HIP_DEVICE_COMPILE__)
+  const __amdgpu_buffer_rsrc_t a_src = operand_descriptor(reinterpret_cast<const bf16_t*>(A), addressing::tile_descriptor(m0, 2 * lda, k_lo, k_hi, a_rows));
+  const __amdgpu_buffer_rsrc_t w_src = operand_descriptor(reinterpret_cast<const bf16_t*>(W), addressing::tile_descriptor(n0, 2 * ldw, k_lo, k_hi, w_rows));
+#endif
+  unsigned a_off[AI], w_off[WI];
+  int a_piece[AI], w_piece[WI];
+#pragma unroll
+  for (int p = 0; p < AI; ++p) {
+    const int row = (wave * AI + p) * 8 + lane / 8;
+    a_piece[p] = addressing::tile_piece(lane, row);
+    a_off[p] = addressing::tile_lane_offset(row, a_rows, 2 * lda, a_piece[p]);
+  }
+#pragma unroll
+  for (int p = 0; p < WI; ++p) {
+    const int row = (wave * WI + p) * 8 + lane / 8;
+    w_piece[p] = addressing::tile_piece(lane, row);
+    w_off[p] = addressing::tile_lane_offset(row, w_rows, 2 * ldw, w_piece[p]);
+  }
+  auto load_slab = [&](int s, int buf) {         // beyond the range: offsets outside the descriptor, zeros nobody uses
+#if defined(__HIP_DEVICE_COMPILE__)
+    const int k = s * ROW;
+#pragma unroll
+    for (int p = 0; p < AI; ++p)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(a_src, (lds_ptr_t)(As + (buf * TM + (wave * AI + p) * 8) * ROW), 16,
+                                               addressing::tile_slab_offset(a_off[p], k, a_piece[p], k_hi - k_lo), 0, 0, 0);
+#pragma unroll
+    for (int p = 0; p < WI; ++p)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(w_src, (lds_ptr_t)(Ws + (buf * TN + (wave * WI + p) * 8) * ROW), 16,
+                                               addressing::tile_slab_offset(w_off[p], k, w_piece[p], k_hi - k_lo), 0, 0, 0);
+#endif
+  };
+
+  f32x16_t acc[WM][WN];
+#pragma unroll
+  for (int i = 0; i < WM; ++i)
+#pragma unroll
+    for (int j = 0; j < WN; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+
+  const int slabs = (k_hi - k_lo + ROW - 1) / ROW;
+  const int frow = lane % 32;
+  int place[4];                                  // where the four floats of this lane's k in every 8 lie in its rows
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) place[ks] = ((ks * 2 + lane / 32) ^ ((frow >> 1) & 7)) * 8;
+#pragma unroll
+  for (int s = 0; s < NB - 1; ++s) load_slab(s, s);
+  int buf = 0;
+  for (int s = 0; s < slabs; ++s) {
+    // all but the slabs asked for after this one have landed: loads return in order
+    constexpr int later = (NB - 2) * (AI + WI);
+    block_barrier_keeping_loads<later>();        // ... for every wave, and everybody has left the buffer before this one
+    load_slab(s + NB - 1, buf == 0 ? NB - 1 : buf - 1);
+    const uint16_t* a_base = As + (buf * TM + wm * (TM / 2) + frow) * ROW;
+    const uint16_t* w_base = Ws + (buf * TN + wn * (TN / 2) + frow) * ROW;
+    f32x4_t fa[2][WM], fb[2][WN];
+#pragma unroll
+    for (int i = 0; i < WM; ++i) fa[0][i] = *reinterpret_cast<const f32x4_t*>(a_base + i * 32 * ROW + place[0]);
+#pragma unroll
+    for (int j = 0; j < WN; ++j) fb[0][j] = *reinterpret_cast<const f32x4_t*>(w_base + j * 32 * ROW + place[0]);
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      if (ks < 3) {                              // the next eight k are read while these run
+#pragma unroll
+        for (int i = 0; i < WM; ++i) fa[(ks + 1) & 1][i] = *reinterpret_cast<const f32x4_t*>(a_base + i * 32 * ROW + place[(ks + 1) & 3]);
+#pragma unroll
+        for (int j = 0; j < WN; ++j) fb[(ks + 1) & 1][j] = *reinterpret_cast<const f32x4_t*>(w_base + j * 32 * ROW + place[(ks + 1) & 3]);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < WM; ++i)
+#pragma unroll
+          for (int j = 0; j < WN; ++j) acc[i][j] = mfma32_f32(fa[ks & 1][i][e], fb[ks & 1][j][e], acc[i][j]);
+      if (ks < 3) {                              // the reads go out behind the first of these products, not behind the last
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, WM + WN, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, 4 * WM * WN - 1, 0);
+      } else {
+        __builtin_amdgcn_sched_group_barrier(0x008, 4 * WM * WN, 0);
+      }
+    }
+    buf = buf == NB - 1 ? 0 : buf + 1;
+  }
+  __builtin_amdgcn_s_waitcnt(0x0F70);            // nothing may still be on its way into LDS when the block ends
+
+  // acc[i][j][v] is C[m0 + wm*TM/2 + i*32 + 8*(v/4) + 4*(lane/32) + v%4][n0 + wn*TN/2 + j*32 + lane%32]: a store
+  // instruction writes 128 contiguous bytes of two rows
+  const bool pieces = gridDim.y > 1;
+  float* out = pieces ? part + (long)blockIdx.y * M * N : C;
+  const long ld = pieces ? N : ldc;
+#pragma unroll
+  for (int j = 0; j < WN; ++j) {
+    const long n = n0 + wn * (TN / 2) + j * 32 + frow;
+    if (n >= N) continue;
+#pragma unroll
+    for (int i = 0; i < WM; ++i)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const long m = m0 + wm * (TM / 2) + i * 32 + 8 * (v / 4) + 4 * (lane / 32) + v % 4;
+        if (m >= M) continue;
+        float* c = out + m * ld + n;
+        *c = ACCUM && !pieces ? *c + acc[i][j][v] : acc[i][j][v];
+      }
+  }
+}
+
+// ------------------------------------------------------------------ which kernel, which tile, how many pieces
+struct Float32Plan {
+  int tm, tn;            // 0: the weight-streaming kernel
+  int splits, k_per_split;
+};
+
+static int compute_units() {
+  static int units = 0;
+  if (units == 0) {
+    int device = 0, count = 0;
+    if (hipGetDevice(&device) != hipSuccess || hipDeviceGetAttribute(&count, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || count <= 0)
+      count = 256;
+    units = count;
+  }
+  return units;
+}
+
+static Float32Plan cut(int tm, int tn, int K, int splits) {
+  const addressing::KSplit c = addressing::cut_k(K, splits, FSTEP);
+  return Float32Plan{tm, tn, c.splits, c.k_per_block};
+}
+
+// Tiles: the shape and the number of pieces with the least time by a model of what was measured: a unit works through
+// its blocks at 0.5 TFLOP/s (less on the smaller tiles), a block starts and ends in 3 us, pieces are written and read
+// once at 4 TB/s by a kernel of their own.  Measured, N x K = 16384 x 2048: 2,048 rows 1,002 us (137 TFLOP/s), 1,293 rows
+// 727 us (1,236 on the vector unit), 378 rows 214 us (118 TFLOP/s); 2048 x 8192: 2,048 rows 525 us, 1,293 rows 412 us in two
+// pieces, 378 rows 119 us in five.
+static Float32Plan plan(int M, int N, int K, long part_floats) {
+  const int units = compute_units();
+  if (M <= ROWS_MAX_M) {
+    // blocks of 32 rows want to be two per unit; a matrix of fewer rows whose k is long is cut over blocks, any other
+    // gets its waves in blocks of 16 rows (launch_rows)
+    int splits = K >= ROWS_SPLIT_MIN_K ? 2 * units / ceil_div(N, 32) : 1;
+    while (splits > 1 && (K / splits < 512 || (long)splits * M * N > part_floats)) --splits;
+    return cut(0, 0, K, splits < 1 ? 1 : splits);
+  }
+  static const struct { int tm, tn; float rate; } shapes[] = {{128, 128, 0.50e6f}, {128, 64, 0.49e6f}, {64, 64, 0.46e6f}};
+  Float32Plan best = {128, 128, 1, K};
+  float least = 0.f;
+  for (const auto& s : shapes) {
+    const long tiles = (long)ceil_div(M, s.tm) * ceil_div(N, s.tn);
+    for (int splits = 1; splits <= 8; ++splits) {
+      const Float32Plan p = cut(s.tm, s.tn, K, splits);
+      if (splits > 1 && (p.splits != splits || p.k_per_split < 256 || (long)splits * M * N > part_floats)) continue;
+      const long rounds = (tiles * p.splits + units - 1) / units;
+      float us = rounds * (3.f + 2.f * s.tm * s.tn * p.k_per_split / s.rate);
+      if (p.splits > 1) us += 4.f + 2.f * p.splits * M * N * 4.f / 4.0e6f;
+      if (least == 0.f || us < least) { least = us; best = p; }
+    }
+  }
+  return best;
+}
+
+// Pieces that pi_gemm_float32 makes of this product when it may leave pieces in `part_floats` floats: 1 if it writes C.
+extern "C" int pi_gemm_float32_pieces(int M, int N, int K, long part_floats) {
+  return M > 0 && N > 0 && K > 0 ? plan(M, N, K, part_floats).splits : 1;
+}
+
+template <int TM, int TN, int NB>
+static int launch_tiles(float* C, long ldc, const float* A, long lda, const float* W, long ldw, int M, int N, int K, int accumulate,
+                        const Float32Plan& p, float* part, hipStream_t stream) {
+  constexpr size_t bytes = (size_t)NB * (TM + TN) * 128;
+  static bool configured = false;
+  if (!configured) {
+    for (const void* f : {reinterpret_cast<const void*>(gemm_float32_tile_kernel<TM, TN, NB, true>), reinterpret_cast<const void*>(gemm_float32_tile_kernel<TM, TN, NB, false>)}) {
+      hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+      if (e != hipSuccess) return pi_fail("gemm_float32: cannot reserve %zu bytes of LDS: %s", bytes, hipGetErrorString(e));
+    }
+    configured = true;
+  }
+  const int tiles_n = ceil_div(N, TN);
+  const dim3 grid((unsigned)(ceil_div(M, TM) * (long)tiles_n), p.splits), block(256);
+  if (accumulate)
+    hipLaunchKernelGGL((gemm_float32_tile_kernel<TM, TN, NB, true>), grid, block, bytes, stream, C, ldc, A, lda, W, ldw, M, N, K, tiles_n, p.k_per_split, part);
+  else
+    hipLaunchKernelGGL((gemm_float32_tile_kernel<TM, TN, NB, false>), grid, block, bytes, stream, C, ldc, A, lda, W, ldw, M, N, K, tiles_n, p.k_per_split, part);
+  return pi_check_launch("gemm_float32 (tiles)");
+}
+
+// Enough waves for the memory whatever the matrix' rows are: blocks of four waves on 32 rows where that gives two per
+// unit, also by cutting k; else blocks of 16 rows with 8 or 16 waves.  Eight tokens, N x K: 16384 x 2048 25.8 us
+// (5.2 TB/s; 35.6 before, on the vector unit), 128256 x 2048 181 us (5.8 TB/s; 197), 3072 x 2048 12.5 us and
+// 2048 x 2048 10.7 us with 16 waves, 2048 x 8192 17.1 us in eight pieces and 4 to add them (with 16 waves instead: 25).
+template <int MB>
+static int launch_rows(float* C, long ldc, const float* A, long lda, const float* W, long ldw, int M, int N, int K, int accumulate,
+                       const Float32Plan& p, float* part, hipStream_t stream) {
+#define ROWS_GO(RT, WAVES, DEPTH)                                                                                                              \
+  do {                                                                                                                                         \
+    const dim3 grid(ceil_div(N, RT * 16), p.splits), block(WAVES * 64);                                                                        \
+    if (accumulate)                                                                                                                            \
+      hipLaunchKernelGGL((gemm_float32_rows_kernel<MB, RT, WAVES, DEPTH, true>), grid, block, 0, stream, C, ldc, A, lda, W, ldw, M, N, K, p.k_per_split, part);  \
+    else                                                                                                                                       \
+      hipLaunchKernelGGL((gemm_float32_rows_kernel<MB, RT, WAVES, DEPTH, false>), grid, block, 0, stream, C, ldc, A, lda, W, ldw, M, N, K, p.k_per_split, part); \
+  } while (0)
+  const int units = compute_units();
+  if (p.splits > 1 || N >= 2 * units * 24) ROWS_GO(2, 4, 1);
+  else if (MB == 1 && N <= units * 16) ROWS_GO(1, (MB == 1 ? 16 : 8), 2);     // sixteen waves have registers for 16 tokens only
+  else ROWS_GO(1, 8, 2);
+#undef ROWS_GO
+  return pi_check_launch("gemm_float32 (few rows)");
+}
+
+// C (+)= A . W^T.  `part` (may be null): float32 [part_floats] for the pieces of a product whose k is cut; when
+// pi_gemm_float32_pieces says more than one, the pieces [splits, M, N] are all that is written and C is not touched.
+extern "C" int pi_gemm_float32(void* C, long ldc, const void* A, long lda, const void* W, long ldw, int M, int N, int K, int accumulate,
+                               void* part, long part_floats, hipStream_t stream) {
+  PI_REQUIRE(M > 0 && N > 0 && K > 0 && K < (1 << 29), "gemm_float32: bad sizes M=%d N=%d K=%d", M, N, K);
+  PI_REQUIRE(lda >= K && ldw >= K && ldc >= N, "gemm_float32: row strides (%ld, %ld, %ld) smaller than the rows (K=%d, N=%d)", lda, ldw, ldc, K, N);
+  PI_REQUIRE(K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0, "gemm_float32: K (%d) and row strides (%ld, %ld) must be multiples of 4", K, lda, ldw);
+  PI_REQUIRE(128 * lda < (1L << 28) && 128 * ldw < (1L << 28), "gemm_float32: row strides (%ld, %ld) are too long for 32-bit offsets inside a tile", lda, ldw);
+  PI_REQUIRE((uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0, "gemm_float32: operands must be 16-byte aligned");
+  PI_REQUIRE((long)ceil_div(M, 64) * ceil_div(N, 64) < 2147483647L, "gemm_float32: too many tiles");
+  const Float32Plan p = plan(M, N, K, part ? part_floats : 0);
+  PI_REQUIRE(p.splits == 1 || (part && part_floats >= (long)p.splits * M * N), "gemm_float32: workspace too small (%ld floats for %ld)", part_floats, (long)p.splits * M * N);
+  float *c = (float*)C, *pieces = (float*)part;
+  const float *a = (const float*)A, *w = (const float*)W;
+  if (p.tm == 0) {
+    return M <= 16 ? launch_rows<1>(c, ldc, a, lda, w, ldw, M, N, K, accumulate, p, pieces, stream) : launch_rows<2>(c, ldc, a, lda, w, ldw, M, N, K, accumulate, p, pieces, stream);
+  }
+  if (p.tm == 128 && p.tn == 128) return launch_tiles<128, 128, 2>(c, ldc, a, lda, w, ldw, M, N, K, accumulate, p, pieces, stream);
+  if (p.tm == 128) return launch_tiles<128, 64, 3>(c, ldc, a, lda, w, ldw, M, N, K, accumulate, p, pieces, stream);
+  return launch_tiles<64, 64, 4>(c, ldc, a, lda, w, ldw, M, N, K, accumulate, p, pieces, stream);
+}
+
+// ------------------------------------------------------------------ adding pieces
+// C[m][n] (op)= sum over splits of part[s][m][n], in split order: store bfloat16 (0), store float32 (1), add into float32 (2)
+template <int EPI>
+__global__ void splitk_reduce_kernel(void* __restrict__ Cv, long ldc, const float* __restrict__ part, int splits, int M, int N) {
+  const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (idx >= (long)M * N) return;
+  const long m = idx / N, n = idx % N;
+  float sum = 0.f;
+  for (int s = 0; s < splits; ++s) sum += part[(long)s * M * N + idx];
+  if (EPI == 0) reinterpret_cast<bf16_t*>(Cv)[m * ldc + n] = from_float<bf16_t>(sum);
+  if (EPI == 1) reinterpret_cast<float*>(Cv)[m * ldc + n] = sum;
+  if (EPI == 2) reinterpret_cast<float*>(Cv)[m * ldc + n] += sum;
+}
+
+extern "C" int pi_splitk_reduce(void* C, int epilogue, long ldc, const void* part, int splits, int M, int N, hipStream_t stream) {
+  PI_REQUIRE(M > 0 && N > 0 && splits >= 1 && part, "splitk_reduce: bad arguments M=%d N=%d splits=%d", M, N, splits);
+  const long total = (long)M * N;
+  const dim3 grid((unsigned)((total + 255) / 256)), block(256);
+  switch (epilogue) {
+    case 0: hipLaunchKernelGGL(splitk_reduce_kernel<0>, grid, block, 0, stream, C, ldc, (const float*)part, splits, M, N); break;
+    case 1: hipLaunchKernelGGL(splitk_reduce_kernel<1>, grid, block, 0, stream, C, ldc, (const float*)part, splits, M, N); break;
+    case 2: hipLaunchKernelGGL(splitk_reduce_kernel<2>, grid, block, 0, stream, C, ldc, (const float*)part, splits, M, N); break;
+    default: return pi_fail("splitk_reduce: unknown epilogue %d", epilogue);
+  }
+  return pi_check_launch("splitk_reduce");
+}

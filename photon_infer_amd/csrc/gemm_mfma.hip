@@ -191,21 +191,6 @@ __device__ inline void store_rows32(float* patch, const f32x16_t& acc0, const f3
   __builtin_amdgcn_wave_barrier();
 }
 
-// Global loads go through buffer descriptors: a scalar base (the block's first row at its first
-// k), a byte length, and per-lane 32-bit offsets.  An offset at or beyond the length reads
-// zeros, which is how rows beyond the matrix and k beyond the range are filled, without a branch.
-#if defined(__HIP_DEVICE_COMPILE__)
-__device__ inline __amdgpu_buffer_rsrc_t operand_descriptor(const bf16_t* operand, addressing::Descriptor d) {
-  // made scalar by hand so that the loads take the descriptor from scalar registers
-  const long bytes = d.bytes;
-  const uint64_t v = reinterpret_cast<uint64_t>(operand + d.base);
-  const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v));
-  const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v >> 32));
-  void* p = reinterpret_cast<void*>((static_cast<uint64_t>(hi) << 32) | lo);
-  return __builtin_amdgcn_make_buffer_rsrc(p, 0, __builtin_amdgcn_readfirstlane((int)bytes), 0x00020000);
-}
-#endif
-
 template <int EPI>
 __global__ __launch_bounds__(256) void gemm_mfma_kernel(void* __restrict__ Cv, long ldc, const bf16_t* __restrict__ A, long lda,
                                                         const bf16_t* __restrict__ W, long ldw, int M, int N, int K,
@@ -277,7 +262,6 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(void* __restrict__ Cv, l
     a_off[p] = addressing::tile_lane_offset(row, a_rows, lda, piece);
     w_off[p] = addressing::tile_lane_offset(row, w_rows, ldw, piece);
   }
-  typedef __attribute__((address_space(3))) void* lds_ptr_t;
   auto load_slab = [&](int k0, int buf) {
     // k0 is relative to k_lo; a lane's 8 k of the slab may lie beyond the range (last slab)
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -442,7 +426,6 @@ __global__ __launch_bounds__(512) void gemm_mfma_big_kernel(void* __restrict__ C
     w_off[p] = addressing::big_lane_offset(row, w_rows, ldw, piece);
   }
   const int slabs = (k_hi - k_lo) / BK;
-  typedef __attribute__((address_space(3))) void* lds_ptr_t;
   auto load_slab = [&](int s, int buf) {
     const int kbytes = addressing::big_slab_bytes(s, slabs);     // past the last slab: read it again, unused
 #if defined(__HIP_DEVICE_COMPILE__)

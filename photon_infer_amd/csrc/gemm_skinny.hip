@@ -413,30 +413,6 @@ __global__ __launch_bounds__(256) void gemm_skinny_shared_kernel(void* __restric
   }
 }
 
-// C[m][n] (op)= sum over splits of part[s][m][n], in split order.
-template <int EPI>
-__global__ void splitk_reduce_kernel(void* __restrict__ Cv, long ldc, const float* __restrict__ part, int splits, int M, int N) {
-  const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (long)M * N) return;
-  const long m = idx / N, n = idx % N;
-  float sum = 0.f;
-  for (int s = 0; s < splits; ++s) sum += part[(long)s * M * N + idx];
-  epilogue_store<EPI>(Cv, ldc, m, n, sum);
-}
-
-extern "C" int pi_splitk_reduce(void* C, int epilogue, long ldc, const void* part, int splits, int M, int N, hipStream_t stream) {
-  PI_REQUIRE(M > 0 && N > 0 && splits >= 1 && part, "splitk_reduce: bad arguments M=%d N=%d splits=%d", M, N, splits);
-  const long total = (long)M * N;
-  const dim3 grid((unsigned)((total + 255) / 256)), block(256);
-  switch (epilogue) {
-    case EPI_BF16: hipLaunchKernelGGL(splitk_reduce_kernel<EPI_BF16>, grid, block, 0, stream, C, ldc, (const float*)part, splits, M, N); break;
-    case EPI_F32: hipLaunchKernelGGL(splitk_reduce_kernel<EPI_F32>, grid, block, 0, stream, C, ldc, (const float*)part, splits, M, N); break;
-    case EPI_ACCUM: hipLaunchKernelGGL(splitk_reduce_kernel<EPI_ACCUM>, grid, block, 0, stream, C, ldc, (const float*)part, splits, M, N); break;
-    default: return pi_fail("splitk_reduce: unknown epilogue %d", epilogue);
-  }
-  return pi_check_launch("splitk_reduce");
-}
-
 template <int MB>
 static int launch_mb(int epi, dim3 grid, hipStream_t stream, void* C, long ldc, const bf16_t* X, long ldx, const bf16_t* W,
                      long ldw, int M, int N, int K, int kpb, float* part, int tiled) {

@@ -7,6 +7,7 @@
 //   B operand: lane l holds 8 bf16 of column (l % 16), same k assignment as A.
 //   D:         lane l holds D[(l / 16) * 4 + i][l % 16] for i = 0..3.
 #pragma once
+#include "addressing.h"
 #include "common.h"
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
@@ -34,6 +35,11 @@ __device__ inline f32x16_t mfma32(const Frag& a, const Frag& b, f32x16_t c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.v, b.v, c, 0, 0, 0);
 }
 
+// float32 operands.  32 x 32 x 2: lane l holds row (column) l % 32 of the operand at k = l / 32, results as for mfma32;
+// 16 x 16 x 4: row (column) l % 16 at k = l / 16, results as for mfma16.  Products and sums are 32-bit throughout.
+__device__ inline f32x16_t mfma32_f32(float a, float b, f32x16_t c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0); }
+__device__ inline f32x4_t mfma16_f32(float a, float b, f32x4_t c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
 __device__ inline Frag zero_frag() {
   Frag f;
   f.q = make_uint4(0u, 0u, 0u, 0u);
@@ -48,3 +54,19 @@ __device__ inline Frag load_frag(const bf16_t* p) {
 }
 
 __device__ inline uint32_t pack_bf16x2(float lo, float hi) { return f32x2_to_bf16x2_bits(lo, hi); }
+
+// Global loads of the tile kernels go through buffer descriptors: a scalar base (the block's first row at its first
+// k), a byte length, and per-lane 32-bit offsets.  An offset at or beyond the length reads
+// zeros, which is how rows beyond the matrix and k beyond the range are filled, without a branch.
+#if defined(__HIP_DEVICE_COMPILE__)
+__device__ inline __amdgpu_buffer_rsrc_t operand_descriptor(const bf16_t* operand, addressing::Descriptor d) {
+  // made scalar by hand so that the loads take the descriptor from scalar registers
+  const long bytes = d.bytes;
+  const uint64_t v = reinterpret_cast<uint64_t>(operand + d.base);
+  const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v));
+  const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v >> 32));
+  void* p = reinterpret_cast<void*>((static_cast<uint64_t>(hi) << 32) | lo);
+  return __builtin_amdgcn_make_buffer_rsrc(p, 0, __builtin_amdgcn_readfirstlane((int)bytes), 0x00020000);
+}
+#endif
+typedef __attribute__((address_space(3))) void* lds_ptr_t;

@@ -110,7 +110,7 @@ class ModelRunner:
         # scratch memory of the kernels and the one residual update that may be pending: this
         # runner's own, handed to the parts with every step's context
         self.workspace = ops.KernelWorkspace(self.device)
-        self.workspace.prepare(self.dtype == torch.bfloat16 and ops.fast_kernels_enabled())
+        self.workspace.prepare(self.dtype == torch.bfloat16 and ops.fast_kernels_enabled(), ops.fast_kernels_enabled())
         # a second copy of the matrices that every decode step streams, in the order the kernels
         # read them; made before the cache is sized, which takes what memory is left
         self.stream_copies = 0

@@ -266,6 +266,10 @@ def gemm(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, accumulate: bool =
         from . import fast
         if fast.gemm(out, a, w, accumulate, M, N, K, lda, ldw, ldc, may_defer and out.dtype == torch.float32 and out.is_contiguous(), ws):
             return
+    if _FAST and a.dtype == torch.float32 and w.dtype == torch.float32 and out.dtype == torch.float32:
+        from . import fast
+        if fast.gemm_float32(out, a, w, accumulate, M, N, K, lda, ldw, ldc, ws):
+            return
     _lib.call("core", "pi_gemm_general", out.data_ptr(), _dt(out), ldc, a.data_ptr(), _dt(a), lda, w.data_ptr(),
               _dt(w), ldw, M, N, K, int(accumulate), _stream())
 

@@ -27,6 +27,9 @@ _SIGNATURES = {
         "pi_swiglu": [P, P, I, I, I, I, P],
         "pi_rope_kv_write": [P, L, P, L, P, L, I, P, P, P, I, I, I, I, I, I, I, P, P, P, I, I, L, P, I, I, I, I, I, I, P, P],
         "pi_gemm_general": [P, I, L, P, I, L, P, I, L, I, I, I, I, P],
+        "pi_gemm_float32_pieces": [I, I, I, L],
+        "pi_gemm_float32": [P, L, P, L, P, L, I, I, I, I, P, L, P],
+        "pi_splitk_reduce": [P, I, L, P, I, I, I, P],
         "pi_paged_attention_general": [P, L, P, L, P, P, I, P, I, P, P, I, I, I, I, I, F, I, L, I, P, L, I, P, P, P, L, F, F, I, I, P],
         "pi_branch_norm_add": [P, P, I, P, P, P, P, P, F, F, I, I, P],
         "pi_cast_stream": [P, I, P, L, P],
@@ -61,7 +64,6 @@ _SIGNATURES = {
         "pi_gemm_mfma_clamped_glu": [P, L, P, L, P, L, I, I, I, P, F, F, P],
         "pi_gemm_mfma_grouped": [P, I, L, P, L, P, L, L, P, P, P, I, I, I, L, L, F, F, P, L, P],
         "pi_gemm_skinny": [P, I, L, P, L, P, L, I, I, I, I, P, L, P, I, P],
-        "pi_splitk_reduce": [P, I, L, P, I, I, I, P],
         "pi_attention_tile_rows": [I, I, I],
         "pi_attention_prefill_mfma": [P, L, P, L, P, P, P, I, P, P, P, P, P, P, P, P, I, I, I, I, I, I, F, I, L, P, P, P, L, F, F, I, I, P],
         "pi_attention_combine_rows": [P, L, P, I, P, I, I, I, P, P, L, F, P],

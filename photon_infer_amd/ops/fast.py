@@ -34,6 +34,7 @@ SHARED_FROM_TOKENS = 32        # more tokens than this: the skinny kernel that s
 SHARED_ROWS_PER_BLOCK = 64     # ... with this many weight rows per block ...
 SHARED_BLOCKS_PER_UNIT = 1     # ... and one block wanted per compute unit
 TILE_MAX_SPLITS = 4
+FLOAT32_MAX_STRIDE = 1 << 21   # floats between rows up to which the float32 kernels' offsets inside a tile fit 32 bits
 BIG_TILES_PER_UNIT = 0.75      # 256 x 256 tiles (times k pieces) per compute unit from which the large-tile kernel is taken (the library's rule)
 DEFAULT_UNITS = 256            # compute units assumed where no device can be asked (an MI355X)
 BIG_MIN_K = 1024               # a piece of the large-tile kernel keeps at least this much of k
@@ -164,7 +165,7 @@ def _tiles_in_pieces(a, w, M, N, K, lda, ldw, splits: int, ws: Optional[KernelWo
 
 def reduce_into(out: torch.Tensor, p: Partials, accumulate: bool) -> None:
     epilogue = EPI_ACCUM if accumulate else (EPI_BF16 if out.dtype == torch.bfloat16 else EPI_F32)
-    _lib.call("bf16", "pi_splitk_reduce", out.data_ptr(), epilogue, out.stride(0), p.part.data_ptr(), p.splits, p.M, p.N,
+    _lib.call("core", "pi_splitk_reduce", out.data_ptr(), epilogue, out.stride(0), p.part.data_ptr(), p.splits, p.M, p.N,
               _stream())
 
 
@@ -197,8 +198,27 @@ def gemm(out, a, w, accumulate, M, N, K, lda, ldw, ldc, may_defer=False, ws: Opt
             ws.pending = PendingUpdate(out, pieces, accumulate)          # the next norm of this stream adds them
             ws.counts["deferred"] += 1
         else:
-            _lib.call("bf16", "pi_splitk_reduce", out.data_ptr(), epilogue, ldc, pieces.part.data_ptr(), pieces.splits,
+            _lib.call("core", "pi_splitk_reduce", out.data_ptr(), epilogue, ldc, pieces.part.data_ptr(), pieces.splits,
                       M, N, _stream())
+    return True
+
+
+def _float32_ok(a, w, K, lda, ldw) -> bool:
+    return (K % 4 == 0 and lda % 4 == 0 and ldw % 4 == 0 and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and max(lda, ldw) < FLOAT32_MAX_STRIDE)
+
+
+def gemm_float32(out, a, w, accumulate, M, N, K, lda, ldw, ldc, ws: Optional[KernelWorkspace] = None) -> bool:
+    """out (+)= a @ w^T, all float32, by the float32 matrix-core kernels; what a product of few tiles leaves in pieces is
+    added at once."""
+    if not _float32_ok(a, w, K, lda, ldw):
+        return False
+    made = _lib.load("core").pi_gemm_float32_pieces(M, N, K, GEMM_PART_FLOATS)
+    buf = _piece_buffer(ws, made * M * N, a.device) if made > 1 else None
+    _lib.call("core", "pi_gemm_float32", out.data_ptr(), ldc, a.data_ptr(), lda, w.data_ptr(), ldw, M, N, K, int(accumulate),
+              None if buf is None else buf.data_ptr(), GEMM_PART_FLOATS if buf is not None else 0, _stream())
+    if buf is not None:
+        _lib.call("core", "pi_splitk_reduce", out.data_ptr(), EPI_ACCUM if accumulate else EPI_F32, ldc, buf.data_ptr(), made, M, N, _stream())
     return True
 
 
@@ -251,7 +271,7 @@ def gemm_from_ranges(out, kr: KeyRanges, w, accumulate, N, ldw, ldc, may_defer, 
             ws.pending = PendingUpdate(out, pieces, accumulate)
             ws.counts["deferred"] += 1
         else:
-            _lib.call("bf16", "pi_splitk_reduce", out.data_ptr(), epilogue, ldc, pieces.part.data_ptr(), pieces.splits, M, N,
+            _lib.call("core", "pi_splitk_reduce", out.data_ptr(), epilogue, ldc, pieces.part.data_ptr(), pieces.splits, M, N,
                       _stream())
     return True
 

@@ -122,11 +122,12 @@ class KernelWorkspace:
         """Partial results of cut tiles, grown on demand."""
         return self._buffer("_tile_part", max(4, floats))
 
-    def prepare(self, matrix_core_kernels: bool) -> None:
+    def prepare(self, matrix_core_attention: bool, split_products: bool = True) -> None:
         """Make the buffers of fixed size now (before anything is captured into a graph)."""
         self.sample_part
-        if matrix_core_kernels:
+        if split_products:
             self.gemm_part
+        if matrix_core_attention:
             self.attn_part
 
     def add_stream_copy(self, w: torch.Tensor) -> bool:

@@ -243,6 +243,32 @@ def test_gemm_on_large_tiles_split_over_k(_ops, M, N, K):
     close(y, want, 2e-6, "large gemm without a workspace")
 
 
+# the weight-streaming kernel (up to 32 rows) and the tile kernel at the edges of its tiles, with and without pieces
+FLOAT32_SHAPES = [(1, 33, 4), (16, 64, 36), (17, 100, 132), (32, 2048, 2048), (7, 16384, 96), (33, 65, 100), (64, 64, 32), (65, 128, 96),
+                  (100, 3072, 512), (128, 130, 1000), (129, 2048, 2048), (300, 200, 8192), (513, 1500, 260), (1100, 2112, 160)]
+
+
+@pytest.mark.parametrize("M,N,K", FLOAT32_SHAPES)
+def test_float32_products_on_the_matrix_cores(_ops, M, N, K):
+    """Against 64 bits; a sum of K products in 32 bits, in whatever order, is off by about 2^-24 sqrt(K) of its size."""
+    rel = 2 ** -24 * (4 + math.sqrt(K))
+    a_full, w_full = torch.randn(M, K + 8, generator=gen(M)), torch.randn(N, K + 4, generator=gen(N))
+    a, w = a_full.to(DEV)[:, 4:K + 4], w_full.to(DEV)[:, :K]                  # rows that lie apart
+    want = a.double() @ w.double().t()
+    out_full = torch.zeros(M, N + 3, device=DEV)
+    _ops.gemm(out_full[:, 1:N + 1], a, w)
+    close(out_full[:, 1:N + 1], want.cpu(), rel, f"float32 {M}x{N}x{K}")
+    assert out_full[:, 0].abs().max() == 0 and out_full[:, N + 1:].abs().max() == 0
+    base = torch.randn(M, N, generator=gen(9)).to(DEV)
+    for space in (None, _ops.KernelWorkspace(DEV)):
+        x = base.clone()
+        _ops.gemm(x, a, w, accumulate=True, ws=space)
+        close(x, (want + base.double()).cpu(), rel, "float32 accumulate")
+    odd = torch.empty(M, N, device=DEV)                                       # operands off 16 bytes: the general kernel
+    _ops.gemm(odd, a_full.to(DEV)[:, 1:K + 1], w)
+    close(odd, (a_full[:, 1:K + 1].double() @ w.double().cpu().t()), rel, "float32, unaligned")
+
+
 @pytest.mark.parametrize("M,I,K", [(1000, 6160, 200), (1000, 6160, 192), (2048, 8192, 64)])
 def test_gemm_with_swiglu_on_large_tiles(_ops, M, I, K):
     _ops.use_fast_kernels(True)
