@@ -502,6 +502,11 @@ def paged_attention(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v
         if fast.paged_attention(out, q, k_cache, v_cache, block_table, ctx, num_heads, num_kv_heads, head_dim,
                                 page_size, scale, window, pages, ws, slopes, sinks, gate, softcap, out_scale, chunk, gate_stride, keep):
             return
+    if _FAST and q.dtype == torch.float32 and vd == head_dim and keep == 0 and not ctx.all_decode:
+        from . import fast
+        if fast.paged_attention_float32(out, q, k_cache, v_cache, block_table, ctx, num_heads, num_kv_heads, head_dim,
+                                        page_size, scale, window, pages, slopes, sinks, gate, softcap, out_scale, chunk, gate_stride):
+            return
     # a step of few tokens over long contexts: its keys cut into ranges, merged by a second kernel
     # (as many as the context-length bucket asks for, so that a step gives the same bits eagerly and replayed)
     # (chunks bound a token's keys whatever the context: one range)

@@ -27,6 +27,8 @@ _SIGNATURES = {
         "pi_swiglu": [P, P, I, I, I, I, P],
         "pi_rope_kv_write": [P, L, P, L, P, L, I, P, P, P, I, I, I, I, I, I, I, P, P, P, I, I, L, P, I, I, I, I, I, I, P, P],
         "pi_gemm_general": [P, I, L, P, I, L, P, I, L, I, I, I, I, P],
+        "pi_attention_float32_tile_tokens": [I, I],
+        "pi_attention_float32": [P, L, P, L, P, P, P, I, P, P, I, I, I, I, I, I, F, I, L, P, P, P, L, F, F, I, P],
         "pi_gemm_float32_pieces": [I, I, I, L],
         "pi_gemm_float32": [P, L, P, L, P, L, I, I, I, I, P, L, P],
         "pi_splitk_reduce": [P, I, L, P, I, I, I, P],

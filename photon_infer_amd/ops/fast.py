@@ -626,6 +626,29 @@ def paged_attention(out, q, k_cache, v_cache, block_table, ctx, num_heads, num_k
     return True
 
 
+# Below this many tokens a step of portions over contexts longer than this goes to the general kernel, which cuts the keys
+# of few tokens into ranges; a tile walks its whole context in one block
+FLOAT32_TILE_MIN_TOKENS, FLOAT32_TILE_SHORT_CONTEXT = 32, 512
+
+
+def paged_attention_float32(out, q, k_cache, v_cache, block_table, ctx, num_heads, num_kv_heads, head_dim, page_size, scale, window, pages,
+                            slopes=None, sinks=None, gate=None, softcap: float = 0.0, out_scale: float = 1.0, chunk: int = 0,
+                            gate_stride: int = 0) -> bool:
+    """Prompt portions on the float32 path, by the matrix-core tile kernel (options as for ``paged_attention``)."""
+    if (head_dim % 16 or head_dim > 128 or page_size % 16 or q.data_ptr() % 16 or out.data_ptr() % 16 or q.stride(0) % 4 or out.stride(0) % 4
+            or k_cache.data_ptr() % 16 or v_cache.data_ptr() % 16):
+        return False
+    if ctx.T < FLOAT32_TILE_MIN_TOKENS and ctx.max_kv_len > FLOAT32_TILE_SHORT_CONTEXT:
+        return False
+    rows = _lib.load("core").pi_attention_float32_tile_tokens(num_heads, num_kv_heads)
+    tiles = sum(-(-n // rows) for n in ctx.q_lens)
+    _lib.call("core", "pi_attention_float32", out.data_ptr(), out.stride(0), q.data_ptr(), q.stride(0), k_cache.data_ptr(), v_cache.data_ptr(),
+              block_table.data_ptr(), block_table.shape[1], ctx.q_start.data_ptr(), ctx.kv_len.data_ptr(), ctx.R, tiles, num_heads, num_kv_heads,
+              head_dim, page_size, float(scale), int(window), pages, None if slopes is None else slopes.data_ptr(),
+              None if sinks is None else sinks.data_ptr(), None if gate is None else gate.data_ptr(), gate_stride, softcap, out_scale, chunk, _stream())
+    return True
+
+
 def decode_attention_from_projection(out, qkv, ctx, table, num_heads, num_kv_heads, head_dim, k_cache, v_cache,
                                      block_table, page_size, scale, window, pages, write_kv,
                                      ws: Optional[KernelWorkspace] = None, leave_ranges: int = 0):

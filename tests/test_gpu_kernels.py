@@ -688,6 +688,40 @@ def test_paged_attention(_ops, case, dtype, fast):
     close(out, want, 3e-6 if dtype == F32 else 2 ** -7, "attention")
 
 
+FLOAT32_ATTN_CASES = [c for c in ATTN_CASES if c[2] <= 128 and c[3] % 16 == 0 and max(c[4]) > 1]
+
+
+@pytest.mark.parametrize("case", FLOAT32_ATTN_CASES + [(8, 4, 64, 16, [1] * 70 + [33, 16], [5] * 70 + [600, 16], None)])
+@pytest.mark.parametrize("options", [False, True])
+def test_float32_attention_of_portions_on_the_matrix_cores(_ops, case, options):
+    """The tile kernel against the general kernel, which other tests hold to the plain implementation, on portions cut at
+    the tiles' and pages' edges; with every option at once too.  Weights and sums are 32-bit in both."""
+    nh, nkv, hd, page, q_lens, kv_lens, window = case
+    g = gen(nh + hd)
+    kvs = [(torch.randn(kv, nkv, hd, generator=g), torch.randn(kv, nkv, hd, generator=g)) for kv in kv_lens]
+    paged, ctx, T = PagedKV(kvs, page, F32, seed=hd), attention_ctx(q_lens, kv_lens, F32), sum(q_lens)
+    q_full = (torch.randn(T, nh * hd + 8, generator=g) * 2).to(DEV)
+    q = q_full[:, 4:nh * hd + 4]
+    ways = [{}]
+    if options:
+        one = dict(slopes=torch.rand(nh, generator=g).to(DEV) * 0.1, sinks=torch.randn(nh, generator=g).to(DEV), softcap=20.0, out_scale=0.7, chunk=48)
+        ways = [dict(one, gate=torch.rand(T * nh, generator=g).to(DEV)), dict(one, feature_gate=torch.randn(T, nh * hd + 4, generator=g).to(DEV)[:, :nh * hd])]
+    for way in ways:
+        got, want = torch.full((T, nh * hd), float("nan"), device=DEV), torch.empty(T, nh * hd, device=DEV)
+        for out, fast in ((got, True), (want, False)):
+            _ops.use_fast_kernels(fast)
+            ctx.T = max(T, 32)          # a step of few tokens would keep to the general kernel
+            _ops.paged_attention(out, q, paged.k, paged.v, paged.table, ctx, nh, nkv, hd, page, 1.0 / math.sqrt(hd), window or 0, **way)
+        _ops.use_fast_kernels(True)
+        close(got, want.cpu(), 3e-6, "float32 attention")
+    if not options:                      # a page that is not there shows in the tokens that see it
+        table = paged.table.clone()
+        table[0, 0] = -1
+        broken = torch.zeros(T, nh * hd, device=DEV)
+        _ops.paged_attention(broken, q, paged.k, paged.v, table, ctx, nh, nkv, hd, page, 0.1, 0)
+        assert broken[:q_lens[0]].isnan().all() and not broken[q_lens[0]:].isnan().any()
+
+
 @pytest.mark.parametrize("dtype", [F32, BF16])
 @pytest.mark.parametrize("fast", [False, True])
 def test_attention_finds_one_far_key_among_hundreds(_ops, dtype, fast):
