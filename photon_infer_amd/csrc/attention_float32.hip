@@ -11,6 +11,7 @@
 // Bound by the matrix cores: 128 instructions of 32 cycles per round and wave at head size 64.  Three prompts of 345 to 517
 // tokens, 32 heads of 64 on 8 kv heads: 64 us per layer, 462 on attention_general.hip (one wave per token and head).
 #include "mfma.h"
+#include "token_tiles.h"
 
 #define KEYS 64
 
@@ -43,27 +44,8 @@ __global__ __launch_bounds__(256) void attention_float32_kernel(float* __restric
 
   // which request and which of its token tiles: the last tiles, with the longest walks, start first
   const int tile_tokens = 16 * (4 / wh);
-  int tile = (int)gridDim.x - 1 - (int)blockIdx.x, req = -1;
-  for (int r0 = 0; r0 < R; r0 += 64) {
-    const int r = r0 + lane;
-    const int mine = r < R ? (q_start[r + 1] - q_start[r] + tile_tokens - 1) / tile_tokens : 0;
-    int upto = mine;
-#pragma unroll
-    for (int d = 1; d < 64; d *= 2) {
-      const int other = __shfl_up(upto, d, 64);
-      if (lane >= d) upto += other;
-    }
-    const unsigned long long past = __ballot(upto > tile);
-    if (past) {
-      const int at = __ffsll((long long)past) - 1;
-      req = r0 + at;
-      tile -= __shfl(upto - mine, at, 64);
-      break;
-    }
-    tile -= __shfl(upto, 63, 64);
-  }
-  req = __builtin_amdgcn_readfirstlane(req);
-  tile = __builtin_amdgcn_readfirstlane(tile);
+  const TokenTile at = find_token_tile(q_start, R, tile_tokens, (int)gridDim.x - 1 - (int)blockIdx.x);
+  const int req = at.req, tile = at.tile;
   if (req < 0) return;                             // the same in every wave of the block
   const int q0 = q_start[req], n = q_start[req + 1] - q0, before = kv_len[req] - n;
   const int t0 = tile * tile_tokens;

@@ -27,14 +27,14 @@ CSRC_DIR = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__
 # matrix-core kernels that only the bfloat16 path uses.
 MODULES: Dict[str, List[str]] = {
     "core": ["elementwise.hip", "gemm_general.hip", "gemm_float32.hip", "attention_general.hip", "attention_float32.hip", "sampling.hip", "stream_norm.hip",
-             "matrix_memory.hip", "routed_experts.hip", "recurrent.hip", "latent.hip", "gated_recurrence.hip", "hyper_streams.hip", "retention.hip"],
+             "matrix_memory.hip", "routed_experts.hip", "recurrent.hip", "state_space_chunks.hip", "latent.hip", "gated_recurrence.hip", "hyper_streams.hip", "retention.hip"],
     "bf16": ["gemm_mfma.hip", "gemm_skinny.hip", "attention_mfma.hip", "attention_decode.hip"],
     # host only: cache manager bookkeeping (needs no GPU and no hipcc)
     "runtime": ["runtime/cache.cpp"],
     # host only: the engine for C / C++ programs (hosts an interpreter; links libpython)
     "api": ["api/photon_engine.cpp"],
 }
-HEADERS = ["common.h", "mfma.h", "addressing.h", "attention_mfma.h", "sampling.h"]
+HEADERS = ["common.h", "mfma.h", "addressing.h", "attention_mfma.h", "sampling.h", "token_tiles.h"]
 HOST_MODULES = {"runtime", "api"}
 HOST_HEADERS = {"api": ["api/photon_engine.h"]}
 HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-Wall"]

@@ -120,6 +120,43 @@ def test_state_space_recurrence_whole_in_portions_and_token_by_token(sizes):
         assert bool((state[0] == 0).all()) and bool((state[2] == 0).all())
 
 
+@pytest.mark.parametrize("sizes", [(2, 64, 128, 1), (4, 20, 16, 2), (2, 72, 32, 1), (1, 128, 64, 1)])
+def test_state_space_recurrence_in_chunks(sizes):
+    """Portions long enough for the chunked form, whole and cut beside, before and behind chunk edges, next to single tokens,
+    from states that earlier steps left; step sizes and decays from next to nothing to a state that is forgotten at once."""
+    from photon_infer_amd import ops
+    H, Pd, N, G = sizes
+    T = {"a": 333, "b": 129, "c": 2}
+    A_log, D, dt_bias = torch.linspace(-3.0, 3.0, H), randn(H, seed=2), torch.linspace(-4.0, 1.0, H)
+    data, want = {}, {}
+    for i, (n, t) in enumerate(T.items()):
+        x, B, C, dt = randn(t, H, Pd, seed=10 + i), randn(t, G, N, seed=20 + i, scale=0.5), randn(t, G, N, seed=30 + i, scale=0.5), randn(t, H, seed=40 + i)
+        data[n] = (torch.cat([x.reshape(t, -1), B.reshape(t, -1), C.reshape(t, -1)], dim=1), dt)
+        want[n] = P.state_space_recurrence(x, B, C, P.softplus(dt + dt_bias), A_log, D)
+    slot = {"a": 3, "b": 1, "c": 0}
+    floats = ops.scan_state_floats(H, N, Pd)
+    for cuts in ({"a": [333], "b": [129], "c": [1]}, {"a": [5, 128, 200], "b": [129], "c": [2]}, {"a": [192, 141], "b": [64, 65], "c": [1]}):
+        state = torch.zeros((4, floats + 3), device=DEV)
+        got = {n: [] for n in T}
+        for step in in_steps(T, cuts):
+            xbc, dt = (dev32(torch.cat([data[n][k][i:j] for n, i, j in step])) for k in (0, 1))
+            y = torch.empty((xbc.shape[0], H * Pd), device=DEV)
+            ops.state_space_scan(y, xbc, dt, dev32(dt_bias), dev32(A_log), dev32(D), state_ctx([j - i for _, i, j in step], [slot[n] for n, _, _ in step]),
+                                 state[:, :floats], H, Pd, N, G)
+            for (n, i, j), part in zip(step, torch.split(y, [j - i for _, i, j in step])):
+                got[n].append(part)
+        for n in T:
+            # sums of up to 64 + 128 products and a carry per chunk: some 2^-24 * 20 of the largest, and the exponentials' own error
+            close(torch.cat(got[n]), want[n][0].reshape(T[n], -1), f"{sizes} {n} cut {cuts[n]}", 1e-5)
+            close(ops.unpack_scan_state(state[slot[n]], H, N, Pd), want[n][1], f"{sizes} {n} state after {cuts[n]}", 1e-5)
+        assert bool((state[2] == 0).all())
+    xbc, dt = dev32(data["a"][0]), dev32(data["a"][1])
+    xbc[100, 1] = float("inf")                     # an input that is not finite: its column from its token on, nothing else
+    y = torch.empty((333, H * Pd), device=DEV)
+    ops.state_space_scan(y, xbc, dt, dev32(dt_bias), dev32(A_log), dev32(D), state_ctx([333], [0]), torch.zeros((1, floats), device=DEV), H, Pd, N, G)
+    assert not bool(y[:, 1].isfinite()[100:].any()) and bool(y[:100].isfinite().all()) and bool(y[:, 0].isfinite().all()) and bool(y[:, 2:].isfinite().all())
+
+
 def delta_inputs(t, H, G, d, dv, seed):
     q, k, v = randn(t, G, d, seed=seed), randn(t, G, d, seed=seed + 1), randn(t, H, dv, seed=seed + 2)
     return q, k, v, randn(t, H * d, seed=seed + 3), randn(t, H, seed=seed + 4)
