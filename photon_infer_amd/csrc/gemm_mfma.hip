@@ -365,11 +365,14 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(void* __restrict__ Cv, l
 }
 
 // ---------------------------------------------------------------------------------------------
-// The same product with block tile 256 x 256 for problems that have enough of them to fill the
+// The same product with larger block tiles, for problems that have enough of them to fill the
 // chip and a k that is a multiple of the slab: eight waves in 2 x 4 (two per SIMD), each
-// 128 x 64 as 4 x 2 tiles of v_mfma_f32_32x32x16_bf16.  Per 16 k a wave reads 6 fragments from
-// LDS for 8 matrix-core instructions, three quarters of the LDS traffic per flop of the
-// 128 x 128 kernel, and a block asks L2 for half the bytes per flop.  With one wave per SIMD
+// WI x WJ tiles of v_mfma_f32_32x32x16_bf16, so that a block's tile is 64 WI x 128 WJ: 256 x 256,
+// 192 x 384, 192 x 256, 128 x 384 or 128 x 256.  A unit holds one block, and a last round of few blocks
+// costs as much as a full one: which shape a product takes is decided by the rounds it needs (ops/fast.py).
+// At 256 x 256 a wave reads 6 fragments from
+// LDS per 16 k for 8 matrix-core instructions, three quarters of the LDS traffic per flop of the
+// 128 x 128 kernel (192 x 384: 6 for 9, 128 x 256: 4 for 4), and a block asks L2 for half the bytes per flop.  With one wave per SIMD
 // (four waves of 128 x 128, the first form of this kernel) every barrier and every wait left
 // the matrix pipe idle.  No branch in the loop (rows beyond the matrix are clamped on load and
 // skipped on store), loads through a buffer descriptor (a scalar base that moves with k plus
@@ -377,22 +380,19 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(void* __restrict__ Cv, l
 // buffer, issued at the top of a slab and awaited at its one barrier, and scheduling hints that
 // deal the memory instructions out between the matrix-core ones.
 // Per output element the sum over k runs in ascending k, as in the small kernel.
-#define GM 256
-#define GN 256
-#define BIG_TILE_ELEMS (GM * BK)
-
-template <int EPI>
+template <int EPI, int WI, int WJ>
 __global__ __launch_bounds__(512) void gemm_mfma_big_kernel(void* __restrict__ Cv, long ldc, const bf16_t* __restrict__ A, long lda,
                                                             const bf16_t* __restrict__ W, long ldw, int M, int N, int K,
                                                             int tiles_n, int k_per_split, GluArgs glu) {
   extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
   constexpr int ROW = BK;                       // rows of 128 bytes, no padding: the loads write LDS themselves, lane after lane
-  constexpr int TILE = GM * ROW;
+  constexpr int GM = 64 * WI, GN = 128 * WJ;    // the block's tile
+  constexpr int AI = WI, BI = 2 * WJ;           // load instructions of a wave per slab: eight rows each
   uint16_t* As = lds;                           // [2][GM][ROW], 16-byte pieces of a row turned by (row / 2) % 8
-  uint16_t* Ws = lds + 2 * TILE;                // [2][GN][ROW]
+  uint16_t* Ws = lds + 2 * GM * ROW;            // [2][GN][ROW]
   const int tid = threadIdx.x, lane = tid % 64;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
-  const int wm = wave / 4, wn = wave % 4;       // a wave's corner: 128 rows x 64 columns
+  const int wm = wave / 4, wn = wave % 4;       // a wave's corner: 32 WI rows x 32 WJ columns
   const int k_lo = blockIdx.y * k_per_split;
   const int k_hi = min(K, k_lo + k_per_split);
   if (gridDim.y > 1) Cv = reinterpret_cast<float*>(Cv) + (long)blockIdx.y * M * ldc;
@@ -409,7 +409,7 @@ __global__ __launch_bounds__(512) void gemm_mfma_big_kernel(void* __restrict__ C
   const long m0 = (long)tile_m * GM, n0 = (long)tile_n * GN;
 
   // global -> LDS without registers in between: load instruction p of wave w fills rows
-  // (4 w + p) * 8 .. + 7 of a tile, lane l the 16-byte piece l % 8 of row l / 8.  Which piece of
+  // (AI w + p) * 8 .. + 7 of A's tile (BI for W's), lane l the 16-byte piece l % 8 of row l / 8.  Which piece of
   // the row in memory that is depends on the row: piece c of row r lies at place c ^ ((r / 2) % 8),
   // so that the fragment reads of sixteen neighbouring rows fall on all 64 banks.
   const int a_rows = (int)min((long)GM, M - m0), w_rows = (int)min((long)GN, N - n0);
@@ -417,31 +417,35 @@ __global__ __launch_bounds__(512) void gemm_mfma_big_kernel(void* __restrict__ C
   const __amdgpu_buffer_rsrc_t a_src = operand_descriptor(A, addressing::tile_descriptor(m0, lda, k_lo, k_hi, a_rows));
   const __amdgpu_buffer_rsrc_t w_src = operand_descriptor(W, addressing::tile_descriptor(n0, ldw, k_lo, k_hi, w_rows));
 #endif
-  unsigned a_off[4], w_off[4];
+  unsigned a_off[AI], w_off[BI];
 #pragma unroll
-  for (int p = 0; p < 4; ++p) {
-    const int row = (wave * 4 + p) * 8 + lane / 8;
-    const int piece = addressing::tile_piece(lane, row);
-    a_off[p] = addressing::big_lane_offset(row, a_rows, lda, piece);
-    w_off[p] = addressing::big_lane_offset(row, w_rows, ldw, piece);
+  for (int p = 0; p < AI; ++p) {
+    const int row = (wave * AI + p) * 8 + lane / 8;
+    a_off[p] = addressing::big_lane_offset(row, a_rows, lda, addressing::tile_piece(lane, row));
+  }
+#pragma unroll
+  for (int p = 0; p < BI; ++p) {
+    const int row = (wave * BI + p) * 8 + lane / 8;
+    w_off[p] = addressing::big_lane_offset(row, w_rows, ldw, addressing::tile_piece(lane, row));
   }
   const int slabs = (k_hi - k_lo) / BK;
   auto load_slab = [&](int s, int buf) {
     const int kbytes = addressing::big_slab_bytes(s, slabs);     // past the last slab: read it again, unused
 #if defined(__HIP_DEVICE_COMPILE__)
 #pragma unroll
-    for (int p = 0; p < 4; ++p) {
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(a_src, (lds_ptr_t)(As + buf * TILE + (wave * 4 + p) * 8 * ROW), 16, a_off[p], kbytes, 0, 0);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(w_src, (lds_ptr_t)(Ws + buf * TILE + (wave * 4 + p) * 8 * ROW), 16, w_off[p], kbytes, 0, 0);
-    }
+    for (int p = 0; p < AI; ++p)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(a_src, (lds_ptr_t)(As + (buf * GM + (wave * AI + p) * 8) * ROW), 16, a_off[p], kbytes, 0, 0);
+#pragma unroll
+    for (int p = 0; p < BI; ++p)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(w_src, (lds_ptr_t)(Ws + (buf * GN + (wave * BI + p) * 8) * ROW), 16, w_off[p], kbytes, 0, 0);
 #endif
   };
 
-  f32x16_t acc[4][2];
+  f32x16_t acc[WI][WJ];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < WI; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < WJ; ++j)
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
 
@@ -449,116 +453,124 @@ __global__ __launch_bounds__(512) void gemm_mfma_big_kernel(void* __restrict__ C
   int place[4];                                  // where this lane's piece of each 16 k lies in its rows
 #pragma unroll
   for (int ks = 0; ks < 4; ++ks) place[ks] = ((ks * 2 + lane / 32) ^ ((frow >> 1) & 7)) * 8;
-  Frag fa[2][4], fb[2][2];
+  Frag fa[2][WI], fb[2][WJ];
   auto read_frags = [&](int which, int buf, int ks) {   // ks: which 16 k of the slab
-    const uint16_t* a_base = As + buf * TILE + (wm * 128 + frow) * ROW + place[ks];
-    const uint16_t* w_base = Ws + buf * TILE + (wn * 64 + frow) * ROW + place[ks];
+    const uint16_t* a_base = As + (buf * GM + wm * 32 * WI + frow) * ROW + place[ks];
+    const uint16_t* w_base = Ws + (buf * GN + wn * 32 * WJ + frow) * ROW + place[ks];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) fa[which][i].n = *reinterpret_cast<const u32x4_t*>(a_base + i * 32 * ROW);
+    for (int i = 0; i < WI; ++i) fa[which][i].n = *reinterpret_cast<const u32x4_t*>(a_base + i * 32 * ROW);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) fb[which][j].n = *reinterpret_cast<const u32x4_t*>(w_base + j * 32 * ROW);
+    for (int j = 0; j < WJ; ++j) fb[which][j].n = *reinterpret_cast<const u32x4_t*>(w_base + j * 32 * ROW);
   };
   auto products = [&](int which) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < WI; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) acc[i][j] = mfma32(fa[which][i], fb[which][j], acc[i][j]);
+      for (int j = 0; j < WJ; ++j) acc[i][j] = mfma32(fa[which][i], fb[which][j], acc[i][j]);
   };
 
   load_slab(0, 0);
   __builtin_amdgcn_s_waitcnt(0x0F70);           // vmcnt(0): this wave's pieces of the slab are in LDS
   __syncthreads();
   read_frags(0, 0, 0);
-  // the order wanted inside one scheduling region: one matrix-core instruction, then one of
-  // each kind of memory instruction named, `n` times; the rest of the 8 after that
-#define PI_DEAL(n, kind_a, kind_b)                                                   \
-  _Pragma("unroll") for (int d_ = 0; d_ < n; ++d_) {                                 \
-    __builtin_amdgcn_sched_group_barrier(PI_SCHED_MFMA, 1, 0);                       \
-    if (kind_a) __builtin_amdgcn_sched_group_barrier(kind_a, 1, 0);                  \
-    if (kind_b) __builtin_amdgcn_sched_group_barrier(kind_b, 1, 0);                  \
+  // the order wanted inside one scheduling region: after every matrix-core instruction one fragment read, as long as there
+  // are any, and (`loads`) its share of the next slab's loads
+#define PI_DEAL(loads)                                                                                            \
+  _Pragma("unroll") for (int d_ = 0; d_ < WI * WJ; ++d_) {                                                        \
+    __builtin_amdgcn_sched_group_barrier(PI_SCHED_MFMA, 1, 0);                                                    \
+    if (d_ < WI + WJ) __builtin_amdgcn_sched_group_barrier(PI_SCHED_DS_READ, 1, 0);                               \
+    const int share_ = (loads) ? (d_ + 1) * (AI + BI) / (WI * WJ) - d_ * (AI + BI) / (WI * WJ) : 0;               \
+    if (share_ > 0) __builtin_amdgcn_sched_group_barrier(PI_SCHED_VMEM_READ, 1, 0);                               \
+    if (share_ > 1) __builtin_amdgcn_sched_group_barrier(PI_SCHED_VMEM_READ, 1, 0);                               \
   }
   load_slab(1, 1);
   for (int s = 0; s < slabs; ++s) {
     const int buf = s & 1;
     read_frags(1, buf, 1);
     products(0);
-    PI_DEAL(6, PI_SCHED_DS_READ, 0)
-    PI_DEAL(2, 0, 0)
+    PI_DEAL(false)
     read_frags(0, buf, 2);
     products(1);
-    PI_DEAL(6, PI_SCHED_DS_READ, 0)
-    PI_DEAL(2, 0, 0)
+    PI_DEAL(false)
     read_frags(1, buf, 3);
     products(0);
-    PI_DEAL(6, PI_SCHED_DS_READ, 0)
-    PI_DEAL(2, 0, 0)
+    PI_DEAL(false)
     __builtin_amdgcn_s_waitcnt(0x0F70);     // slab s + 1 has landed (asked for a whole slab ago)
     __syncthreads();
     load_slab(s + 2, buf);          // into the buffer everybody has just left
     read_frags(0, buf ^ 1, 0);
     products(1);
-    PI_DEAL(6, PI_SCHED_DS_READ, PI_SCHED_VMEM_READ)
-    PI_DEAL(2, PI_SCHED_VMEM_READ, 0)
+    PI_DEAL(true)
   }
   __builtin_amdgcn_s_waitcnt(0x0F70);       // nothing may still be on its way into LDS when the patches take it over
 #undef PI_DEAL
 
-  // acc[i][j][v] is C[m0 + wm*128 + i*32 + 8*(v/4) + 4*(lane/32) + v%4][n0 + wn*64 + j*32 + lane%32].
+  // acc[i][j][v] is C[m0 + wm*32*WI + i*32 + 8*(v/4) + 4*(lane/32) + v%4][n0 + wn*32*WJ + j*32 + lane%32].
   // Offsets inside the wave's corner are 32-bit (the host checks that 128 * ldc fits).
   __syncthreads();                              // LDS is free for the waves' patches
   {
-    const long mw = m0 + wm * 128, nw = n0 + wn * 64;
-    const int rows_left = (int)min((long)128, M - mw), cols_left = (int)min((long)64, N - nw);   // may be <= 0
-    if (EPI == EPI_GATE) glu.bias += mw * glu.gate_stride + nw;
+    const long mw = m0 + wm * 32 * WI;
+    const int rows_left = (int)min((long)32 * WI, M - mw);                                                // may be <= 0
     float* patch = reinterpret_cast<float*>(lds) + wave * PATCH_FLOATS;
     const int esize = EPI_HALF(EPI) || EPI_GATED(EPI) ? 2 : 4;
-    char* corner = reinterpret_cast<char*>(Cv) + (mw * ldc + (EPI_GATED(EPI) ? nw / 2 : nw)) * esize;
-    const bool wide = (ldc * esize) % 16 == 0 && reinterpret_cast<uintptr_t>(corner) % 16 == 0;
+    if (EPI == EPI_GATE) glu.bias += mw * glu.gate_stride + n0 + wn * 32 * WJ;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) store_rows32<EPI>(patch, acc[i][0], acc[i][1], corner, (int)ldc, i * 32, rows_left, cols_left, lane, wide, glu, nw);
+    for (int j = 0; j < WJ; j += 2) {
+      const long nw = n0 + wn * 32 * WJ + j * 32;
+      const int cols_left = (int)min((long)64, N - nw);
+      char* corner = reinterpret_cast<char*>(Cv) + (mw * ldc + (EPI_GATED(EPI) ? nw / 2 : nw)) * esize;
+      const bool wide = (ldc * esize) % 16 == 0 && reinterpret_cast<uintptr_t>(corner) % 16 == 0;
+#pragma unroll
+      for (int i = 0; i < WI; ++i)
+        store_rows32<EPI>(patch, acc[i][j], acc[i][j + 1 < WJ ? j + 1 : j], corner, (int)ldc, i * 32, rows_left,
+                          j + 1 < WJ ? cols_left : min(32, cols_left), lane, wide, glu, nw);       // an odd last tile stands alone
+      if (EPI == EPI_GATE) glu.bias += 64;
+    }
   }
-}
-
-static const size_t kBigLdsBytes = 4 * BIG_TILE_ELEMS * sizeof(uint16_t);   // 131,072 bytes
-// enough 256 x 256 tiles (times k pieces) to occupy most of the chip: three quarters of its compute units
-static int big_min_tiles() {
-  static int units = 0;
-  if (units == 0) {
-    int device = 0, count = 0;
-    if (hipGetDevice(&device) != hipSuccess || hipDeviceGetAttribute(&count, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || count <= 0)
-      count = 256;
-    units = count;
-  }
-  return units * 3 / 4;
 }
 
 static const size_t kLdsBytes = 4 * TILE_ELEMS * sizeof(uint16_t);   // 65,536 bytes
 
+template <int EPI, int WI, int WJ>
+static int launch_big(void* C, long ldc, const void* A, long lda, const void* W, long ldw, int M, int N, int K, int splits, int kps,
+                      hipStream_t stream, GluArgs glu) {
+  constexpr size_t bytes = 2 * (64 * WI + 128 * WJ) * BK * sizeof(uint16_t);
+  static bool configured = false;
+  if (!configured) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_mfma_big_kernel<EPI, WI, WJ>),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+    if (e != hipSuccess) return pi_fail("gemm_mfma: cannot reserve %zu bytes of LDS: %s", bytes, hipGetErrorString(e));
+    configured = true;
+  }
+  const long tiles = (long)ceil_div(M, 64 * WI) * ceil_div(N, 128 * WJ);
+  hipLaunchKernelGGL((gemm_mfma_big_kernel<EPI, WI, WJ>), dim3((unsigned)tiles, splits), dim3(512), bytes, stream, C, ldc,
+                     (const bf16_t*)A, lda, (const bf16_t*)W, ldw, M, N, K, ceil_div(N, 128 * WJ), kps, glu);
+  return pi_check_launch("gemm_mfma_big");
+}
+
+// shape: 0 the 128 x 128 kernel, else 10 WI + WJ of the larger tiles (K a multiple of the slab)
 template <int EPI>
-static int launch(void* C, long ldc, const void* A, long lda, const void* W, long ldw, int M, int N, int K, int splits,
+static int launch(void* C, long ldc, const void* A, long lda, const void* W, long ldw, int M, int N, int K, int splits, int shape,
                   hipStream_t stream, GluArgs glu = GluArgs{nullptr, 0.f, 0.f, 0}) {
+  const addressing::KSplit cut = addressing::cut_k(K, splits, BK);
+  const int kps = cut.k_per_block;
+  splits = cut.splits;
+  PI_REQUIRE(shape == 0 || K % BK == 0, "gemm_mfma: the larger tiles take whole slabs of %d only, K is %d", BK, K);
+  switch (shape) {
+    case 0: break;
+    case 42: return launch_big<EPI, 4, 2>(C, ldc, A, lda, W, ldw, M, N, K, splits, kps, stream, glu);
+    case 33: return launch_big<EPI, 3, 3>(C, ldc, A, lda, W, ldw, M, N, K, splits, kps, stream, glu);
+    case 32: return launch_big<EPI, 3, 2>(C, ldc, A, lda, W, ldw, M, N, K, splits, kps, stream, glu);
+    case 23: return launch_big<EPI, 2, 3>(C, ldc, A, lda, W, ldw, M, N, K, splits, kps, stream, glu);
+    case 22: return launch_big<EPI, 2, 2>(C, ldc, A, lda, W, ldw, M, N, K, splits, kps, stream, glu);
+    default: return pi_fail("gemm_mfma: unknown tile shape %d", shape);
+  }
   static bool configured = false;
   if (!configured) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_mfma_kernel<EPI>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsBytes);
     if (e != hipSuccess) return pi_fail("gemm_mfma: cannot reserve %zu bytes of LDS: %s", kLdsBytes, hipGetErrorString(e));
     configured = true;
-  }
-  const addressing::KSplit cut = addressing::cut_k(K, splits, BK);
-  const int kps = cut.k_per_block;
-  splits = cut.splits;
-  const long big_tiles = (long)ceil_div(M, GM) * ceil_div(N, GN);
-  if (big_tiles * splits >= big_min_tiles() && big_tiles < 2147483647L && K % BK == 0) {
-    static bool big_configured = false;
-    if (!big_configured) {
-      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_mfma_big_kernel<EPI>),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)kBigLdsBytes);
-      if (e != hipSuccess) return pi_fail("gemm_mfma: cannot reserve %zu bytes of LDS: %s", kBigLdsBytes, hipGetErrorString(e));
-      big_configured = true;
-    }
-    hipLaunchKernelGGL((gemm_mfma_big_kernel<EPI>), dim3((unsigned)big_tiles, splits), dim3(512), kBigLdsBytes, stream, C, ldc,
-                       (const bf16_t*)A, lda, (const bf16_t*)W, ldw, M, N, K, ceil_div(N, GN), kps, glu);
-    return pi_check_launch("gemm_mfma_big");
   }
   const int tiles_m = ceil_div(M, BM), tiles_n = ceil_div(N, BN);
   hipLaunchKernelGGL((gemm_mfma_kernel<EPI>), dim3((unsigned)tiles_m * tiles_n, splits), dim3(256), kLdsBytes, stream, C, ldc,
@@ -630,7 +642,7 @@ extern "C" int pi_gemm_mfma_pieces(int K, int splits) {
 // epilogue: 0 store bf16, 1 store f32, 2 add into f32, 3 SwiGLU (W rows interleaved by 16; C is [M, N / 2] bf16),
 // 5 store max(c, 0)^2 as bf16, 6 store the exact gelu of c as bf16
 extern "C" int pi_gemm_mfma(void* C, int epilogue, long ldc, const void* A, long lda, const void* W, long ldw, int M,
-                            int N, int K, int splits, hipStream_t stream) {
+                            int N, int K, int splits, int shape, hipStream_t stream) {
   PI_REQUIRE(M > 0 && N > 0 && K > 0, "gemm_mfma: bad sizes M=%d N=%d K=%d", M, N, K);
   // splits > 1: C is a float32 workspace [splits, M, N] (ldc = N) that receives the pieces; the
   // number of pieces is ceil(K / (ceil(K / splits) rounded up to 64))
@@ -643,12 +655,12 @@ extern "C" int pi_gemm_mfma(void* C, int epilogue, long ldc, const void* A, long
   PI_REQUIRE(epilogue != EPI_SWIGLU || N % 32 == 0, "gemm_mfma: the SwiGLU epilogue needs N (%d) to be a multiple of 32", N);
   PI_REQUIRE((long)ceil_div(M, BM) * ceil_div(N, BN) < 2147483647L, "gemm_mfma: too many tiles");
   switch (epilogue) {
-    case EPI_BF16: return launch<EPI_BF16>(C, ldc, A, lda, W, ldw, M, N, K, splits, stream);
-    case EPI_F32: return launch<EPI_F32>(C, ldc, A, lda, W, ldw, M, N, K, splits, stream);
-    case EPI_ACCUM: return launch<EPI_ACCUM>(C, ldc, A, lda, W, ldw, M, N, K, splits, stream);
-    case EPI_RELU2: return launch<EPI_RELU2>(C, ldc, A, lda, W, ldw, M, N, K, splits, stream);
-    case EPI_GELU: return launch<EPI_GELU>(C, ldc, A, lda, W, ldw, M, N, K, splits, stream);
-    case EPI_SWIGLU: return launch<EPI_SWIGLU>(C, ldc, A, lda, W, ldw, M, N, K, splits, stream);
+    case EPI_BF16: return launch<EPI_BF16>(C, ldc, A, lda, W, ldw, M, N, K, splits, shape, stream);
+    case EPI_F32: return launch<EPI_F32>(C, ldc, A, lda, W, ldw, M, N, K, splits, shape, stream);
+    case EPI_ACCUM: return launch<EPI_ACCUM>(C, ldc, A, lda, W, ldw, M, N, K, splits, shape, stream);
+    case EPI_RELU2: return launch<EPI_RELU2>(C, ldc, A, lda, W, ldw, M, N, K, splits, shape, stream);
+    case EPI_GELU: return launch<EPI_GELU>(C, ldc, A, lda, W, ldw, M, N, K, splits, shape, stream);
+    case EPI_SWIGLU: return launch<EPI_SWIGLU>(C, ldc, A, lda, W, ldw, M, N, K, splits, shape, stream);
   }
   return pi_fail("gemm_mfma: unknown epilogue %d", epilogue);
 }
@@ -656,7 +668,7 @@ extern "C" int pi_gemm_mfma(void* C, int epilogue, long ldc, const void* A, long
 // C[M, N / 2] (bfloat16) = the clamped gated unit of A . W^T: W's rows and `bias` (float32 [N]) hold gate and up
 // interleaved by 16; g' = min(g + bg, limit), u' = clamp(u + bu, -limit, limit), g' * sigmoid(alpha * g') * (u' + 1).
 extern "C" int pi_gemm_mfma_clamped_glu(void* C, long ldc, const void* A, long lda, const void* W, long ldw, int M, int N, int K,
-                                        const float* bias, float limit, float alpha, hipStream_t stream) {
+                                        const float* bias, float limit, float alpha, int shape, hipStream_t stream) {
   PI_REQUIRE(M > 0 && N > 0 && K > 0 && bias, "gemm_mfma: bad sizes M=%d N=%d K=%d", M, N, K);
   PI_REQUIRE(K % 8 == 0 && lda % 8 == 0 && ldw % 8 == 0, "gemm_mfma: K (%d) and row strides (%ld, %ld) must be multiples of 8", K, lda, ldw);
   PI_REQUIRE(256 * lda < (1L << 29) && 256 * ldw < (1L << 29), "gemm_mfma: row strides (%ld, %ld) are too long for 32-bit offsets inside a tile", lda, ldw);
@@ -664,5 +676,5 @@ extern "C" int pi_gemm_mfma_clamped_glu(void* C, long ldc, const void* A, long l
   PI_REQUIRE(((uintptr_t)A % 16 == 0) && ((uintptr_t)W % 16 == 0), "gemm_mfma: operands must be 16-byte aligned");
   PI_REQUIRE(N % 32 == 0, "gemm_mfma: the gated epilogue needs N (%d) to be a multiple of 32", N);
   PI_REQUIRE((long)ceil_div(M, BM) * ceil_div(N, BN) < 2147483647L, "gemm_mfma: too many tiles");
-  return launch<EPI_CLAMPED_GLU>(C, ldc, A, lda, W, ldw, M, N, K, 1, stream, GluArgs{bias, limit, alpha, 0});
+  return launch<EPI_CLAMPED_GLU>(C, ldc, A, lda, W, ldw, M, N, K, 1, shape, stream, GluArgs{bias, limit, alpha, 0});
 }

@@ -63,9 +63,9 @@ _SIGNATURES = {
         "pi_sample_static": [P, P, L, P, P, I, I, P],
     },
     "bf16": {
-        "pi_gemm_mfma": [P, I, L, P, L, P, L, I, I, I, I, P],
+        "pi_gemm_mfma": [P, I, L, P, L, P, L, I, I, I, I, I, P],
         "pi_gemm_mfma_pieces": [I, I],
-        "pi_gemm_mfma_clamped_glu": [P, L, P, L, P, L, I, I, I, P, F, F, P],
+        "pi_gemm_mfma_clamped_glu": [P, L, P, L, P, L, I, I, I, P, F, F, I, P],
         "pi_gemm_mfma_grouped": [P, I, L, P, L, P, L, L, P, P, P, I, I, I, L, L, F, F, P, L, P],
         "pi_gemm_skinny": [P, I, L, P, L, P, L, I, I, I, I, P, L, P, I, P],
         "pi_attention_tile_rows": [I, I, I],

@@ -282,6 +282,35 @@ def test_gemm_with_swiglu_on_large_tiles(_ops, M, I, K):
     close(out, want, 2 ** -7, "fused swiglu on large tiles")
 
 
+@pytest.mark.parametrize("shape", [0, 42, 33, 32, 23, 22])
+@pytest.mark.parametrize("M,N,K", [(129, 96, 64), (193, 512, 192), (257, 800, 320), (640, 1184, 448)])
+def test_every_tile_shape_at_its_edges(_ops, monkeypatch, shape, M, N, K):
+    """Each block tile with one row more than it holds, columns that end inside a wave's corner, and one slab of k up to
+    several: stored in both types, added, in pieces, and through the gated epilogue (products of bfloat16 in 32-bit sums:
+    the bounds of the tests above)."""
+    from photon_infer_amd.ops import fast
+    monkeypatch.setattr(fast, "_tile_shape", lambda *_: shape)
+    a = (torch.randn(M, K, generator=gen(M)) * 0.5).to(BF16).to(DEV)
+    w = torch.randn(N, K, generator=gen(N)).to(BF16).to(DEV)
+    want = a.double() @ w.double().t()
+    for c_dtype, rel in ((BF16, 2 ** -8), (F32, 2e-6)):
+        full = torch.zeros(M, N + 16, dtype=c_dtype, device=DEV)
+        _ops.gemm(full[:, 8:N + 8], a, w)
+        close(full[:, 8:N + 8], want.cpu(), rel, f"tiles {shape}")
+        assert full[:, :8].abs().max() == 0 and full[:, N + 8:].abs().max() == 0
+    base = torch.randn(M, N, generator=gen(9)).to(DEV)
+    x = base.clone()
+    _ops.gemm(x, a, w, accumulate=True)
+    close(x, (want + base.double()).cpu(), 2e-6, f"tiles {shape}, added")
+    ws = _ops.KernelWorkspace(DEV)
+    p = fast._tiles_in_pieces(a, w, M, N, K, K, K, 3, ws)
+    close(p.part[:p.splits * M * N].view(p.splits, M, N).double().sum(0), want.cpu(), 2e-6, f"tiles {shape}, pieces")
+    g, u = want.view(M, N // 32, 2, 16).unbind(2)
+    out = torch.empty(M, N // 2, dtype=BF16, device=DEV)
+    _ops.gemm_swiglu(out, a, w, 16)
+    close(out, P.swiglu(g.reshape(M, -1), u.reshape(M, -1)).cpu(), 2 ** -7, f"tiles {shape}, swiglu")
+
+
 def test_gemm_reference_vectors(_ops):
     # tests/ops/test_matmul.cpp:90-204
     W = torch.tensor([[1.0, 2.0, 3.0], [4.0, 5.0, 6.0]], device=DEV)
