@@ -4,7 +4,11 @@
 // the kv group (up to 16; unused columns are padding), so a group's keys and values are read
 // once.  Every range writes its un-normalised partial result with its running maximum and
 // sum; a second small kernel merges the ranges in range order (deterministic).  With one range
-// the result is written directly.
+// the result is written directly.  A block may also hold WAVES waves that share one range's keys and
+// merge in LDS, in wave order: where a step's requests nearly fill the chip by themselves, two to four
+// such waves take the place of ranges and their merging kernel, and requests of unlike length hold up
+// the step less, as a wave alone streams some 11 GB/s (32 heads and 8 kv heads of 64: 64 requests of 2,000
+// to 4,000 keys 87.7 -> 79.9 us, 4.9 -> 5.4 TB/s; 24 of 1,000 to 2,000 23.1 + 4.6 -> 23.7 us).
 //
 // For the query at position p = kv_len - 1: keys lo..p with lo = max(0, p - window + 1)
 // (window 0: all keys), or the start of p's chunk where positions are cut into chunks.  Ranges are cut at multiples of 32 keys.
@@ -170,14 +174,15 @@ __device__ inline void store_new_kv(const DecodeSource& src, long row, int g, in
   }
 }
 
-template <int HD, bool FUSED, bool OPT = false>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(HD <= 64 ? 2 : 1))) void attention_decode_kernel(
+template <int HD, bool FUSED, bool OPT, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(HD <= 64 ? 2 : 1))) void attention_decode_kernel(
     bf16_t* __restrict__ out, long out_stride, const bf16_t* __restrict__ q, long q_stride, DecodeSource src,
     const bf16_t* k_cache, const bf16_t* v_cache,   // not restrict: the fused kernel stores into them
     const int* __restrict__ block_table,
     int table_width, const int* __restrict__ q_start, const int* __restrict__ kv_len_of, const int* __restrict__ req_ids,
     int nh, int nkv, int page_size, float scale, int window, long num_pages, float* __restrict__ part, AttnOptions opt) {
-  const int lane = threadIdx.x, lr = lane % 16, lg = lane / 16;
+  const int lane = threadIdx.x % 64, lr = lane % 16, lg = lane / 16;
+  const int wave = WAVES > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / 64) : 0;
   const int split = blockIdx.x, splits = gridDim.x, g = blockIdx.y;
   // the z-th request of this launch: all of the step's requests, or the listed ones (a step
   // that also holds prompt portions sends only its single tokens here)
@@ -205,8 +210,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(HD <= 64 ? 2
   const int first_place = OPT && kept > 0 ? 0 : first_chunk;
   const int last_chunk = p / 32 - gap;             // as a place
   const int chunks = last_chunk - first_place + 1;
-  const int per = (chunks + splits - 1) / splits;
-  const int c0 = first_place + split * per;
+  const int per = (chunks + splits * WAVES - 1) / (splits * WAVES);
+  const int c0 = first_place + (split * WAVES + wave) * per;
   const int c1 = min(last_chunk + 1, c0 + per);
   // The wave whose keys end at the new token writes that token into the cache first and waits
   // for the stores; after that it reads the token like any other key, in the same order of
@@ -229,6 +234,39 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(HD <= 64 ? 2
                      }
                    }, kept, gap);
   attn_finish(st);
+  if constexpr (WAVES > 1) {
+    // the waves' states meet in the first one; a wave without keys (m = -inf) weighs nothing
+    __shared__ f32x4_t outs[WAVES - 1][HD / 16][64];
+    __shared__ float2 sums[WAVES - 1][16];
+    if (wave > 0) {
+#pragma unroll
+      for (int db = 0; db < HD / 16; ++db) outs[wave - 1][db][lane] = st.o[db][0];
+      if (lg == 0) sums[wave - 1][lr] = make_float2(st.m[0], st.l[0]);
+    }
+    __syncthreads();
+    if (wave > 0) return;
+    const float to_base2 = scale * PI_LOG2E;
+    float m_tot = st.m[0];
+#pragma unroll
+    for (int w = 0; w < WAVES - 1; ++w) m_tot = fmaxf(m_tot, sums[w][lr].x);
+    const float own = range_weight(st.m[0] * to_base2, m_tot * to_base2);
+    st.m[0] = m_tot;
+    st.l[0] *= own;
+#pragma unroll
+    for (int db = 0; db < HD / 16; ++db) st.o[db][0] *= own;
+#pragma unroll
+    for (int w = 0; w < WAVES - 1; ++w) {
+      const float2 ml = sums[w][lr];
+      const float weight = range_weight(ml.x * to_base2, m_tot * to_base2);
+      st.l[0] = range_add(weight, ml.y, st.l[0]);
+#pragma unroll
+      for (int db = 0; db < HD / 16; ++db) {
+        const f32x4_t v = outs[w][db][lane];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) st.o[db][0][i] = range_add(weight, v[i], st.o[db][0][i]);
+      }
+    }
+  }
 
   const int head = g * G + lr;
   if (splits == 1) {
@@ -265,7 +303,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(HD <= 64 ? 2
   }
 }
 
-// Merge the key ranges of one (request, head) by one wave: lane d owns features d, d + 64, ..
+// Merge the key ranges of one (request, head), a wave per 64 features: lane d of wave w owns feature 64 w + d (one
+// wave for all features of a head of 256: 12.1 us for 4 requests with 16 heads and 64 ranges; four: 8.3).
 // Ranges are added in range order; an empty range (m = -inf) counts nothing.
 // sink2: the head's sink in base-2 units, joining the sum of weights once (-inf: none); gate: a
 // factor for the finished output; features: gates per feature, still to go through a sigmoid (null: none).
@@ -273,45 +312,39 @@ template <int HD>
 __device__ inline void combine_ranges(bf16_t* __restrict__ o, const float* base, int splits, int lane, float sink2 = -INFINITY,
                                       float gate = 1.0f, const float* features = nullptr) {
   const int rec = HD + 4;
-  constexpr int NF = (HD + 63) / 64;     // features per lane
+  const int mine = threadIdx.x;          // this lane's feature
   // lane s holds range s (splits <= 64): maxima, weights and the total in parallel
   const float ms = lane < splits ? base[lane * rec + HD] : -INFINITY;
   const float ls = lane < splits ? base[lane * rec + HD + 1] : 0.f;
   const float m_tot = fmaxf(wave_max(ms), sink2);
   const float w = range_weight(ms, m_tot);
   float l_tot = range_weight(sink2, m_tot);
-  float acc[NF];
-#pragma unroll
-  for (int i = 0; i < NF; ++i) acc[i] = 0.f;
+  float acc = 0.f;
   // ranges in order; eight loads in flight at a time
   for (int s0 = 0; s0 < splits; s0 += 8) {
-    float ov[8][NF], ws[8];
+    float ov[8], ws[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       const int s = s0 + u;
       ws[u] = __shfl(w, s < splits ? s : 0, 64);
       if (s >= splits) ws[u] = 0.f;
-#pragma unroll
-      for (int i = 0; i < NF; ++i) ov[u][i] = (s < splits && lane + i * 64 < HD) ? base[s * rec + lane + i * 64] : 0.f;
+      ov[u] = (s < splits && mine < HD) ? base[s * rec + mine] : 0.f;
     }
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       l_tot = range_add(ws[u], __shfl(ls, (s0 + u < splits) ? s0 + u : 0, 64), l_tot);
-#pragma unroll
-      for (int i = 0; i < NF; ++i) acc[i] = range_add(ws[u], ov[u][i], acc[i]);
+      acc = range_add(ws[u], ov[u], acc);
     }
   }
-#pragma unroll
-  for (int i = 0; i < NF; ++i)
-    if (lane + i * 64 < HD) {
-      const float f = features ? gate / (1.0f + __expf(-features[lane + i * 64])) : gate;
-      o[lane + i * 64] = from_float<bf16_t>(range_finish(acc[i], l_tot) * f);
-    }
+  if (mine < HD) {
+    const float f = features ? gate / (1.0f + __expf(-features[mine])) : gate;
+    o[mine] = from_float<bf16_t>(range_finish(acc, l_tot) * f);
+  }
 }
 
-// One wave per (request, head).
+// One block per (request, head).
 template <int HD>
-__global__ __launch_bounds__(64) void attention_combine_kernel(bf16_t* __restrict__ out, long out_stride,
+__global__ __launch_bounds__((HD + 63) / 64 * 64) void attention_combine_kernel(bf16_t* __restrict__ out, long out_stride,
                                                                const int* __restrict__ q_start,
                                                                const int* __restrict__ req_ids,
                                                                const int* __restrict__ rows,
@@ -321,7 +354,7 @@ __global__ __launch_bounds__(64) void attention_combine_kernel(bf16_t* __restric
   const int r = req_ids ? req_ids[blockIdx.y] : (int)blockIdx.y;
   const long out_row = rows ? rows[blockIdx.y] : q_start[r];
   combine_ranges<HD>(out + out_row * out_stride + (long)head * HD, part + ((long)blockIdx.y * nh + head) * splits * (HD + 4),
-                     splits, threadIdx.x, opt.sinks ? opt.sinks[head] * PI_LOG2E : -INFINITY,
+                     splits, threadIdx.x % 64, opt.sinks ? opt.sinks[head] * PI_LOG2E : -INFINITY,
                      (opt.gate && !opt.gate_stride ? opt.gate[out_row * nh + head] : 1.0f) * opt.out_mult,
                      opt.gate_stride ? opt.gate + out_row * opt.gate_stride + (long)head * HD : nullptr);
 }
@@ -330,7 +363,7 @@ __global__ __launch_bounds__(64) void attention_combine_kernel(bf16_t* __restric
 // token rows) or listed token rows.
 static int launch_combine(void* out, long out_stride, const int* q_start, const int* req_ids, const int* rows, int Z,
                           const void* part, int nh, int hd, int splits, hipStream_t stream, AttnOptions opt = AttnOptions{nullptr, nullptr, nullptr}) {
-  const dim3 grid(nh, Z), block(64);
+  const dim3 grid(nh, Z), block((hd + 63) / 64 * 64);
 #define GO(H) hipLaunchKernelGGL(attention_combine_kernel<H>, grid, block, 0, stream, (bf16_t*)out, out_stride, q_start, req_ids, rows, \
                                  (const float*)part, nh, splits, opt)
   switch (hd) {
@@ -362,7 +395,7 @@ static int launch_combine(void* out, long out_stride, const int* q_start, const 
 static int launch_decode(bool fused, const DecodeSource& src, void* out, long out_stride, const void* q, long q_stride,
                          const void* k_cache, const void* v_cache, const int* block_table, int table_width,
                          const int* q_start, const int* kv_len, const int* req_ids, int R, int nh, int nkv, int hd,
-                         int page_size, float scale, int window, long num_pages, int splits, void* part, long part_elems,
+                         int page_size, float scale, int window, long num_pages, int splits, int waves, void* part, long part_elems,
                          bool merge, hipStream_t stream, AttnOptions opt = AttnOptions{nullptr, nullptr, nullptr}) {
   const bool with_options = opt.any();
   PI_REQUIRE(!with_options || (!fused && merge && scale > 0.f), "attention_decode: heads with options take the separate kernels, merged here, and a positive scale");
@@ -374,15 +407,16 @@ static int launch_decode(bool fused, const DecodeSource& src, void* out, long ou
   PI_REQUIRE(out_stride % 4 == 0 && ((uintptr_t)out % 8 == 0), "attention_decode: out rows must be 8-byte aligned");
   if (!fused)
     PI_REQUIRE(q_stride % 8 == 0 && ((uintptr_t)q % 16 == 0), "attention_decode: q rows must be 16-byte aligned");
+  PI_REQUIRE(waves == 1 || ((waves == 2 || waves == 4) && splits == 1), "attention_decode: %d waves per block over %d ranges", waves, splits);
   if (splits > 1)
     PI_REQUIRE(part && part_elems >= (long)R * nh * splits * (hd + 4), "attention_decode: workspace too small for %d ranges", splits);
-  const dim3 grid(splits, nkv, R), block(64);
-#define GO(H, F) hipLaunchKernelGGL((attention_decode_kernel<H, F>), grid, block, 0, stream, (bf16_t*)out, out_stride, (const bf16_t*)q, \
+  const dim3 grid(splits, nkv, R), block(64 * waves);
+#define GO_W(H, F, O, WV) hipLaunchKernelGGL((attention_decode_kernel<H, F, O, WV>), grid, block, 0, stream, (bf16_t*)out, out_stride, (const bf16_t*)q, \
                                     q_stride, src, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_table, table_width, q_start, \
                                     kv_len, req_ids, nh, nkv, page_size, scale, window, num_pages, (float*)part, opt)
-#define GO_OPT(H) hipLaunchKernelGGL((attention_decode_kernel<H, false, true>), grid, block, 0, stream, (bf16_t*)out, out_stride, (const bf16_t*)q, \
-                                    q_stride, src, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_table, table_width, q_start, \
-                                    kv_len, req_ids, nh, nkv, page_size, scale, window, num_pages, (float*)part, opt)
+#define GO_F(H, F, O) do { if (waves == 1) GO_W(H, F, O, 1); else if (waves == 2) GO_W(H, F, O, 2); else GO_W(H, F, O, 4); } while (0)
+#define GO(H, F) GO_F(H, F, false)
+#define GO_OPT(H) GO_F(H, false, true)
   if (fused) { if (hd == 64) GO(64, true); else GO(128, true); }
   else if (with_options) {
     switch (hd) {
@@ -425,6 +459,8 @@ static int launch_decode(bool fused, const DecodeSource& src, void* out, long ou
   }
 #undef GO
 #undef GO_OPT
+#undef GO_F
+#undef GO_W
   if (pi_check_launch("attention_decode")) return -1;
   // merge == false: the caller's next kernel merges the ranges itself (nothing is in `out` then)
   if (splits > 1 && merge) return launch_combine(out, out_stride, q_start, req_ids, nullptr, R, part, nh, hd, splits, stream, opt);
@@ -434,13 +470,13 @@ static int launch_decode(bool fused, const DecodeSource& src, void* out, long ou
 extern "C" int pi_attention_decode(void* out, long out_stride, const void* q, long q_stride, const void* k_cache,
                                    const void* v_cache, const int* block_table, int table_width, const int* q_start,
                                    const int* kv_len, const int* req_ids, int R, int nh, int nkv, int hd, int page_size,
-                                   float scale, int window, long num_pages, int splits, void* part, long part_elems,
+                                   float scale, int window, long num_pages, int splits, int waves, void* part, long part_elems,
                                    const float* slopes, const float* sinks, const float* gate, long gate_stride, float softcap,
                                    float out_mult, int chunk, int keep, hipStream_t stream) {
   PI_REQUIRE(chunk >= 0 && keep >= 0, "attention_decode: chunk and kept first keys must be >= 0, got %d and %d", chunk, keep);
   PI_REQUIRE(gate_stride == 0 || (gate && gate_stride % 4 == 0 && (uintptr_t)gate % 16 == 0), "attention_decode: gates per feature must lie in 16-byte groups");
   return launch_decode(false, DecodeSource{}, out, out_stride, q, q_stride, k_cache, v_cache, block_table, table_width, q_start,
-                       kv_len, req_ids, R, nh, nkv, hd, page_size, scale, window, num_pages, splits, part, part_elems, true, stream,
+                       kv_len, req_ids, R, nh, nkv, hd, page_size, scale, window, num_pages, splits, waves, part, part_elems, true, stream,
                        AttnOptions{slopes, sinks, gate, softcap, out_mult, gate_stride, chunk, keep});
 }
 
@@ -455,7 +491,7 @@ extern "C" int pi_attention_decode_fused(void* out, long out_stride, const void*
                                          int qkv_splits, int ncols, int T, const float* table, int write_kv, void* k_cache,
                                          void* v_cache, const int* block_table, int table_width, const int* q_start,
                                          const int* kv_len, int R, int nh, int nkv, int hd, int page_size, float scale,
-                                         int window, long num_pages, int splits, void* part, long part_elems,
+                                         int window, long num_pages, int splits, int waves, void* part, long part_elems,
                                          int merge, hipStream_t stream) {
   PI_REQUIRE((qkv != nullptr) != (qkv_part != nullptr), "attention_decode_fused: give the projection as a tensor or as pieces");
   PI_REQUIRE(T == R, "attention_decode_fused: %d tokens for %d requests (single tokens only)", T, R);
@@ -484,7 +520,7 @@ extern "C" int pi_attention_decode_fused(void* out, long out_stride, const void*
   src.k_cache = (bf16_t*)k_cache;
   src.v_cache = (bf16_t*)v_cache;
   return launch_decode(true, src, out, out_stride, nullptr, 0, k_cache, v_cache, block_table, table_width, q_start, kv_len,
-                       nullptr, R, nh, nkv, hd, page_size, scale, window, num_pages, splits, part, part_elems, merge != 0, stream);
+                       nullptr, R, nh, nkv, hd, page_size, scale, window, num_pages, splits, waves, part, part_elems, merge != 0, stream);
 }
 
 // Merge partial results that the tile kernel wrote for `Z` tokens whose tiles' keys were cut in

@@ -45,6 +45,10 @@ FUSED_DECODE_HEAD_DIMS = (64, 128)                 # ... and of its form that st
 MAX_DECODE_SPLITS = 64         # the combine kernel holds one key range per lane
 DECODE_WAVES_PER_UNIT = 2      # waves of the decode attention kernel per compute unit that fill the chip (measured at batch 1 to 64: more is never faster)
 DECODE_MIN_KEYS_PER_SPLIT = 128
+# Waves that share a block's keys: only where the blocks fill their rounds over the units this far (320 blocks of a design with
+# capped scores, 1.25 rounds: a step of 783 us took 796) and, without ranges to replace, for contexts longer than this
+# (64 requests of 300 keys: 1,325 -> 1,336 us; of 600: 1,400 -> 1,384)
+DECODE_WAVES_FILL, DECODE_WAVES_MIN_KEYS = 0.75, 512
 
 
 def _stream() -> int:
@@ -608,6 +612,19 @@ def decode_splits(R: int, num_kv_heads: int, max_kv_len: int) -> int:
     return min(splits, max(1, decode_length_bucket(max_kv_len) // DECODE_MIN_KEYS_PER_SPLIT))
 
 
+def decode_block_waves(splits: int, R: int, num_kv_heads: int, max_kv_len: int) -> int:
+    """Waves per block of the decode attention, which share a request's keys of one kv head and merge in the block: they take
+    the place of ``splits`` ranges (more than 1: one range then, and no merging kernel), or 1.  Steps whose ranges the next
+    product may merge keep them."""
+    blocks = R * num_kv_heads
+    rounds = -(-blocks // compute_units())
+    if R <= RANGES_MAX_TOKENS or splits > 4 or blocks < DECODE_WAVES_FILL * rounds * compute_units():
+        return 1
+    if splits > 1:
+        return 2 if splits == 2 else 4
+    return 2 if rounds < 4 and decode_length_bucket(max_kv_len) > DECODE_WAVES_MIN_KEYS else 1
+
+
 def _attn_part(ws: Optional[KernelWorkspace], floats: int, device) -> torch.Tensor:
     return ws.attn_part if ws is not None else torch.empty(max(4, floats), dtype=torch.float32, device=device)
 
@@ -638,11 +655,14 @@ def paged_attention(out, q, k_cache, v_cache, block_table, ctx, num_heads, num_k
         if chunk:                      # a token's keys end at its chunk's start, whatever the context
             longest = min(longest, chunk + keep)
         splits = _decode_splits_that_fit(ws, n_req, num_heads, num_kv_heads, head_dim, longest)
+        waves = decode_block_waves(splits, n_req, num_kv_heads, min(longest, window) if window else longest)
+        if waves > 1:
+            splits = 1
         part = _attn_part(ws, n_req * num_heads * splits * (head_dim + 4), q.device)
         _lib.call("bf16", "pi_attention_decode", out.data_ptr(), out.stride(0), q.data_ptr(), q.stride(0),
                   k_cache.data_ptr(), v_cache.data_ptr(), block_table.data_ptr(), block_table.shape[1],
                   ctx.q_start.data_ptr(), ctx.kv_len.data_ptr(), req_ids, n_req, num_heads, num_kv_heads, head_dim,
-                  page_size, float(scale), int(window), pages, splits, part.data_ptr(), part.numel(), *opt, _stream())
+                  page_size, float(scale), int(window), pages, splits, waves, part.data_ptr(), part.numel(), *opt, _stream())
 
     if ctx.all_decode and G <= 16:
         decode_kernel(R, 0, ctx.max_kv_len)
@@ -712,14 +732,17 @@ def decode_attention_from_projection(out, qkv, ctx, table, num_heads, num_kv_hea
     if (qkv.N % 4 or qkv.part.data_ptr() % 16) if pieces else (qkv.stride(0) % 8 or qkv.stride(1) != 1 or qkv.data_ptr() % 16):
         return False
     splits = _decode_splits_that_fit(ws, R, num_heads, num_kv_heads, head_dim, ctx.max_kv_len)
-    part = _attn_part(ws, R * num_heads * splits * (head_dim + 4), out.device)
     leave = leave_ranges > 0 and ws is not None and splits > 1 and ranges_product_ok(R, head_dim, leave_ranges)
+    waves = 1 if leave else decode_block_waves(splits, R, num_kv_heads, min(ctx.max_kv_len, window) if window else ctx.max_kv_len)
+    if waves > 1:
+        splits = 1
+    part = _attn_part(ws, R * num_heads * splits * (head_dim + 4), out.device)
     _lib.call("bf16", "pi_attention_decode_fused", out.data_ptr(), out.stride(0),
               None if pieces else qkv.data_ptr(), 0 if pieces else qkv.stride(0),
               qkv.part.data_ptr() if pieces else None, qkv.splits if pieces else 0, qkv.N if pieces else 0, R,
               None if table is None else table.data_ptr(), int(bool(write_kv)), k_cache.data_ptr(), v_cache.data_ptr(),
               block_table.data_ptr(), block_table.shape[1], ctx.q_start.data_ptr(), ctx.kv_len.data_ptr(), R, num_heads,
-              num_kv_heads, head_dim, page_size, float(scale), int(window), pages, splits, part.data_ptr(),
+              num_kv_heads, head_dim, page_size, float(scale), int(window), pages, splits, waves, part.data_ptr(),
               part.numel(), int(not leave), _stream())
     if leave:
         return KeyRanges(part, splits, R, num_heads, head_dim, ctx.q_start)

@@ -751,6 +751,46 @@ def test_float32_attention_of_portions_on_the_matrix_cores(_ops, case, options):
         assert broken[:q_lens[0]].isnan().all() and not broken[q_lens[0]:].isnan().any()
 
 
+@pytest.mark.parametrize("waves", [2, 4])
+@pytest.mark.parametrize("hd,nh,nkv,page,window,options", [(64, 8, 2, 16, 0, False), (128, 4, 4, 32, 40, False), (48, 6, 3, 16, 0, True),
+                                                           (64, 16, 1, 16, 70, True), (256, 4, 2, 16, 0, True)])
+def test_decode_attention_by_the_waves_of_a_block(_ops, monkeypatch, waves, hd, nh, nkv, page, window, options):
+    """A block's waves share a request's keys: contexts that leave waves without keys, end inside a wave's share and fill
+    all of them, against plain attention (with options: the general kernel); the fused kernel leaves the same cache and bits."""
+    from photon_infer_amd.ops import fast
+    monkeypatch.setattr(fast, "decode_block_waves", lambda *a: waves)
+    kv_lens = [1, 31, 33, 64, 65, 97, 129, 300, 1000]
+    R, scale = len(kv_lens), hd ** -0.5
+    g = gen(hd + nh + waves)
+    kvs = [(torch.randn(kv, nkv, hd, generator=g).to(BF16).float(), torch.randn(kv, nkv, hd, generator=g).to(BF16).float()) for kv in kv_lens]
+    paged, ctx = PagedKV(kvs, page, BF16, seed=hd), attention_ctx([1] * R, kv_lens, BF16)
+    q = (torch.randn(R, nh * hd, generator=g) * 2).to(BF16).to(DEV)
+    got = torch.full_like(q, float("nan"))
+    if options:
+        way = dict(slopes=torch.rand(nh, generator=g).to(DEV) * 0.1, sinks=torch.randn(nh, generator=g).to(DEV), softcap=20.0, out_scale=0.7,
+                   feature_gate=torch.randn(R, nh * hd, generator=g).to(DEV))
+        want = torch.empty_like(q)
+        _ops.use_fast_kernels(False)
+        _ops.paged_attention(want, q, paged.k, paged.v, paged.table, ctx, nh, nkv, hd, page, scale, window, **way)
+        _ops.use_fast_kernels(True)
+        _ops.paged_attention(got, q, paged.k, paged.v, paged.table, ctx, nh, nkv, hd, page, scale, window, **way)
+        close(got, want.cpu(), 2 ** -6, "attention with options")   # both sides round to bfloat16
+        return
+    _ops.paged_attention(got, q, paged.k, paged.v, paged.table, ctx, nh, nkv, hd, page, scale, window)
+    want = dense_attention([x.reshape(1, nh, hd).float().cpu() for x in q], kvs, [1] * R, kv_lens, scale, window or None).reshape(R, nh * hd)
+    close(got, want, 2 ** -7, "attention")
+    table = paged.table.cpu()
+    last = [(table[r, (n - 1) // page].item(), (n - 1) % page) for r, n in enumerate(kv_lens)]
+    new_k, new_v = torch.stack([paged.k[pg, :, sl] for pg, sl in last]), torch.stack([paged.v[pg, :, :, sl] for pg, sl in last])
+    k, v = paged.k.clone(), paged.v.clone()
+    for pg, sl in last:
+        k[pg, :, sl], v[pg, :, :, sl] = 1e4, -1e4
+    qkv = torch.cat([q, new_k.reshape(R, -1), new_v.reshape(R, -1)], 1).contiguous()
+    fused = torch.full_like(q, float("nan"))
+    assert _ops.decode_attention_from_projection(fused, qkv, ctx, None, nh, nkv, hd, k, v, paged.table, page, scale, window, True)
+    assert torch.equal(k, paged.k) and torch.equal(v, paged.v) and torch.equal(fused, got)
+
+
 @pytest.mark.parametrize("dtype", [F32, BF16])
 @pytest.mark.parametrize("fast", [False, True])
 def test_attention_finds_one_far_key_among_hundreds(_ops, dtype, fast):
