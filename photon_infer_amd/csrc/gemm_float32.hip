@@ -435,28 +435,53 @@ extern "C" int pi_gemm_float32(void* C, long ldc, const void* A, long lda, const
 }
 
 // ------------------------------------------------------------------ adding pieces
-// C[m][n] (op)= sum over splits of part[s][m][n], in split order: store bfloat16 (0), store float32 (1), add into float32 (2)
-template <int EPI>
-__global__ void splitk_reduce_kernel(void* __restrict__ Cv, long ldc, const float* __restrict__ part, int splits, int M, int N) {
-  const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (long)M * N) return;
-  const long m = idx / N, n = idx % N;
-  float sum = 0.f;
-  for (int s = 0; s < splits; ++s) sum += part[(long)s * M * N + idx];
-  if (EPI == 0) reinterpret_cast<bf16_t*>(Cv)[m * ldc + n] = from_float<bf16_t>(sum);
-  if (EPI == 1) reinterpret_cast<float*>(Cv)[m * ldc + n] = sum;
-  if (EPI == 2) reinterpret_cast<float*>(Cv)[m * ldc + n] += sum;
+// C[m][n] (op)= sum over splits of part[s][m][n], in split order: store bfloat16 (0), store float32 (1), add into float32 (2).
+// Bound by latency and, with many rows, by memory: a thread takes V neighbouring columns (four where 16-byte accesses are
+// allowed) and has eight pieces in flight (one column and one piece at a time before: 2,048 tokens by 2,048 columns added into
+// float32 14.9 -> 11.5 us, 12 tokens 3.7 -> 1.8).
+template <int EPI, int V>
+__global__ __launch_bounds__(256) void splitk_reduce_kernel(void* __restrict__ Cv, long ldc, const float* __restrict__ part, int splits, int M, int N) {
+  typedef float vec_t __attribute__((ext_vector_type(V)));
+  const int n = (blockIdx.x * blockDim.x + threadIdx.x) * V;
+  if (n >= N) return;
+  for (long m = blockIdx.y; m < M; m += gridDim.y) {
+    const float* p = part + m * N + n;
+    vec_t old = 0.f, sum = 0.f;
+    if (EPI == 2) old = *reinterpret_cast<const vec_t*>((const float*)Cv + m * ldc + n);
+    for (int s0 = 0; s0 < splits; s0 += 8) {
+      vec_t v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (s0 + u < splits) v[u] = *reinterpret_cast<const vec_t*>(p + (long)(s0 + u) * M * N);
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (s0 + u < splits) sum += v[u];
+    }
+    if (EPI == 0) {
+#pragma unroll
+      for (int i = 0; i < V; ++i) reinterpret_cast<bf16_t*>(Cv)[m * ldc + n + i] = from_float<bf16_t>(sum[i]);
+    } else {
+      *reinterpret_cast<vec_t*>((float*)Cv + m * ldc + n) = EPI == 2 ? old + sum : sum;
+    }
+  }
+}
+
+template <int V>
+static int launch_reduce(void* C, int epilogue, long ldc, const float* part, int splits, int M, int N, hipStream_t stream) {
+  const int across = (N + V - 1) / V, threads = across < 256 ? (across + 63) / 64 * 64 : 256;
+  const dim3 grid((across + threads - 1) / threads, M < 65535 ? M : 65535), block(threads);
+  switch (epilogue) {
+    case 0: hipLaunchKernelGGL((splitk_reduce_kernel<0, V>), grid, block, 0, stream, C, ldc, part, splits, M, N); break;
+    case 1: hipLaunchKernelGGL((splitk_reduce_kernel<1, V>), grid, block, 0, stream, C, ldc, part, splits, M, N); break;
+    case 2: hipLaunchKernelGGL((splitk_reduce_kernel<2, V>), grid, block, 0, stream, C, ldc, part, splits, M, N); break;
+    default: return pi_fail("splitk_reduce: unknown epilogue %d", epilogue);
+  }
+  return pi_check_launch("splitk_reduce");
 }
 
 extern "C" int pi_splitk_reduce(void* C, int epilogue, long ldc, const void* part, int splits, int M, int N, hipStream_t stream) {
   PI_REQUIRE(M > 0 && N > 0 && splits >= 1 && part, "splitk_reduce: bad arguments M=%d N=%d splits=%d", M, N, splits);
-  const long total = (long)M * N;
-  const dim3 grid((unsigned)((total + 255) / 256)), block(256);
-  switch (epilogue) {
-    case 0: hipLaunchKernelGGL(splitk_reduce_kernel<0>, grid, block, 0, stream, C, ldc, (const float*)part, splits, M, N); break;
-    case 1: hipLaunchKernelGGL(splitk_reduce_kernel<1>, grid, block, 0, stream, C, ldc, (const float*)part, splits, M, N); break;
-    case 2: hipLaunchKernelGGL(splitk_reduce_kernel<2>, grid, block, 0, stream, C, ldc, (const float*)part, splits, M, N); break;
-    default: return pi_fail("splitk_reduce: unknown epilogue %d", epilogue);
-  }
-  return pi_check_launch("splitk_reduce");
+  const bool wide = N % 4 == 0 && (uintptr_t)part % 16 == 0 && (epilogue == 0 || (ldc % 4 == 0 && (uintptr_t)C % 16 == 0));
+  return wide ? launch_reduce<4>(C, epilogue, ldc, (const float*)part, splits, M, N, stream)
+              : launch_reduce<1>(C, epilogue, ldc, (const float*)part, splits, M, N, stream);
 }

@@ -8,7 +8,7 @@
 #include "common.h"
 
 #define PI_CONV_MAX_TAPS 8
-#define PI_CONV_SEGMENT 64
+#define PI_CONV_SEGMENT 16        // at least PI_CONV_MAX_TAPS - 1: only a request's first segment reads its state
 #define PI_SCAN_COLUMNS 16      // value columns of a block: four walking waves of four columns each
 #define PI_SCAN_WAVES 4
 
@@ -22,6 +22,10 @@ __device__ inline float softplus_f(float v) { return v > 20.0f ? v : log1pf(expf
 // taps - 1 inputs of earlier steps, zeros at the start of a sequence), which is brought up to
 // date here.  A thread owns a channel of one segment of a request's tokens; the thread of the
 // first segment reads the old state before it writes the new one, and nobody else touches it.
+// Bound by memory (an input in, an output out), if enough of it is asked for at a time: a segment's
+// inputs are all fetched before the first is used, and segments are short for the sake of many blocks
+// (2,048 tokens, four layers of 2,304 and 6,144 channels: 32.4 us each with one input at a time and
+// segments of 64, 16.5 so, of which some 11 are the bytes).
 template <typename TW>
 __global__ __launch_bounds__(256) void causal_conv_silu_kernel(
     float* __restrict__ out, long out_stride, const float* __restrict__ in, long in_stride, const TW* __restrict__ w,
@@ -53,12 +57,18 @@ __global__ __launch_bounds__(256) void causal_conv_silu_kernel(
     for (int j = 0; j < PI_CONV_MAX_TAPS - 1; ++j) old[j] = j < taps - 1 ? st[(long)j * C + c] : 0.f;
   }
   const float b = bias ? to_float(bias[c]) : 0.f;
-  for (int t = t0; t < t1; ++t) {
-    win[PI_CONV_MAX_TAPS - 1] = in[(long)(qs + t) * in_stride + c];
+  float u[PI_CONV_SEGMENT];
+#pragma unroll
+  for (int i = 0; i < PI_CONV_SEGMENT; ++i)
+    if (t0 + i < t1) u[i] = in[(long)(qs + t0 + i) * in_stride + c];
+#pragma unroll
+  for (int i = 0; i < PI_CONV_SEGMENT; ++i) {
+    if (t0 + i >= t1) break;
+    win[PI_CONV_MAX_TAPS - 1] = u[i];
     float acc = b;
 #pragma unroll
     for (int j = 0; j < PI_CONV_MAX_TAPS; ++j) acc = fmaf(wr[j], win[j], acc);
-    out[(long)(qs + t) * out_stride + c] = silu_f(acc);
+    out[(long)(qs + t0 + i) * out_stride + c] = silu_f(acc);
 #pragma unroll
     for (int j = 0; j < PI_CONV_MAX_TAPS - 1; ++j) win[j] = win[j + 1];
   }
@@ -309,25 +319,46 @@ extern "C" int pi_state_space_scan(float* y, long y_stride, const float* xbc, lo
 
 // ------------------------------------------------------------------ gate, then norm in equal parts
 // out[t, i] = mult * w[i] * v[i] / sqrt(mean over i's part of v^2 + eps),  v = y * silu(z).
-// One block per (token, part).
+// One block per (token, part).  Latency bounds it: a thread fetches up to PI_NORM_VALUES columns before it uses the
+// first, and keeps them over the norm; wider parts (above 1024 threads' worth) are read twice
+// (2,048 columns, a loop of one column at a time before: 12 tokens 6.5 -> 2.6 us, 2,048 tokens 14.2 -> 10.8).
+#define PI_NORM_VALUES 4
+
 template <typename TO>
-__global__ __launch_bounds__(256) void gated_group_norm_kernel(TO* __restrict__ out, long out_stride, const float* __restrict__ y,
-                                                              long y_stride, const float* __restrict__ z, long z_stride,
-                                                              const float* __restrict__ w, float eps, float mult, int size) {
+__global__ __launch_bounds__(1024) void gated_group_norm_kernel(TO* __restrict__ out, long out_stride, const float* __restrict__ y,
+                                                                long y_stride, const float* __restrict__ z, long z_stride,
+                                                                const float* __restrict__ w, float eps, float mult, int size) {
   __shared__ float scratch[16];
   const long t = blockIdx.x;
-  const int base = blockIdx.y * size;
+  const int base = blockIdx.y * size, step = blockDim.x;
   const float* yr = y + t * y_stride + base;
   const float* zr = z + t * z_stride + base;
+  float v[PI_NORM_VALUES], g[PI_NORM_VALUES], wv[PI_NORM_VALUES];
+#pragma unroll
+  for (int i = 0; i < PI_NORM_VALUES; ++i) {
+    const int c = threadIdx.x + i * step;
+    v[i] = g[i] = wv[i] = 0.f;
+    if (c < size) { v[i] = yr[c]; g[i] = zr[c]; wv[i] = w[base + c]; }
+  }
   float ss = 0.f;
-  for (int i = threadIdx.x; i < size; i += blockDim.x) {
-    const float v = yr[i] * silu_f(zr[i]);
-    ss = fmaf(v, v, ss);
+#pragma unroll
+  for (int i = 0; i < PI_NORM_VALUES; ++i) {
+    v[i] *= silu_f(g[i]);
+    ss = fmaf(v[i], v[i], ss);
+  }
+  for (int c = threadIdx.x + PI_NORM_VALUES * step; c < size; c += step) {
+    const float u = yr[c] * silu_f(zr[c]);
+    ss = fmaf(u, u, ss);
   }
   const float rinv = 1.0f / sqrtf(block_sum(ss, scratch) / size + eps);
-  for (int i = threadIdx.x; i < size; i += blockDim.x) {
-    const float v = yr[i] * silu_f(zr[i]);
-    out[t * out_stride + base + i] = from_float<TO>(v * rinv * w[base + i] * mult);
+#pragma unroll
+  for (int i = 0; i < PI_NORM_VALUES; ++i) {
+    const int c = threadIdx.x + i * step;
+    if (c < size) out[t * out_stride + base + c] = from_float<TO>(v[i] * rinv * wv[i] * mult);
+  }
+  for (int c = threadIdx.x + PI_NORM_VALUES * step; c < size; c += step) {
+    const float u = yr[c] * silu_f(zr[c]);
+    out[t * out_stride + base + c] = from_float<TO>(u * rinv * w[base + c] * mult);
   }
 }
 
@@ -337,7 +368,8 @@ extern "C" int pi_gated_group_norm(void* out, int out_dtype, long out_stride, co
   PI_REQUIRE(T >= 0 && width > 0 && parts > 0 && parts <= 65535 && width % parts == 0, "gated norm: %d columns in %d parts", width, parts);
   if (T == 0) return 0;
   const int size = width / parts;
-  const dim3 grid(T, parts), block(size >= 256 ? 256 : 64);
+  const int waves = (size + PI_NORM_VALUES * PI_WAVE - 1) / (PI_NORM_VALUES * PI_WAVE);
+  const dim3 grid(T, parts), block(PI_WAVE * (waves < 16 ? waves : 16));
   if (out_dtype == PI_F32)
     hipLaunchKernelGGL(gated_group_norm_kernel<float>, grid, block, 0, stream, (float*)out, out_stride, y, y_stride, z, z_stride, w, eps, mult, size);
   else if (out_dtype == PI_BF16)

@@ -248,6 +248,26 @@ FLOAT32_SHAPES = [(1, 33, 4), (16, 64, 36), (17, 100, 132), (32, 2048, 2048), (7
                   (100, 3072, 512), (128, 130, 1000), (129, 2048, 2048), (300, 200, 8192), (513, 1500, 260), (1100, 2112, 160)]
 
 
+@pytest.mark.parametrize("M,N,splits,ld,skip", [(1, 4, 1, 4, 0), (12, 2048, 7, 2048, 0), (3, 260, 8, 264, 0), (5, 1028, 9, 1028, 0),
+                                                (70, 37, 17, 37, 0), (2, 64, 3, 65, 0), (2, 64, 3, 64, 1)])
+@pytest.mark.parametrize("epilogue", [0, 1, 2])
+def test_pieces_are_added_in_order(M, N, splits, ld, skip, epilogue):
+    """Wide and narrow accesses (columns, rows or an output that are no multiple of 16 bytes), fewer and more pieces than are in flight."""
+    from photon_infer_amd.ops import _lib
+    g = gen(M + N)
+    part = torch.randn(splits, M, N, generator=g).to(DEV)
+    c = torch.randn(M * ld + skip + 8, generator=g).to(BF16 if epilogue == 0 else F32).to(DEV)
+    total = torch.zeros(M, N, device=DEV)
+    for piece in part:
+        total = total + piece
+    want = c.clone()
+    rows = want[skip:skip + M * ld].view(M, ld)[:, :N]
+    rows.copy_(rows + total if epilogue == 2 else total)
+    _lib.call("core", "pi_splitk_reduce", c.data_ptr() + skip * c.element_size(), epilogue, ld, part.data_ptr(), splits, M, N,
+              torch.cuda.current_stream().cuda_stream)
+    assert torch.equal(c, want)
+
+
 @pytest.mark.parametrize("M,N,K", FLOAT32_SHAPES)
 def test_float32_products_on_the_matrix_cores(_ops, M, N, K):
     """Against 64 bits; a sum of K products in 32 bits, in whatever order, is off by about 2^-24 sqrt(K) of its size."""

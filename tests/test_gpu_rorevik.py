@@ -244,6 +244,17 @@ def test_gate_then_norm_in_equal_parts(dtype, N, parts):
     close(out, want, f"gated norm {N} / {parts}", 2e-5 if dtype == "float32" else 1e-2)
 
 
+@pytest.mark.parametrize("N,parts", [(256, 1), (257, 1), (4096, 1), (4097, 1), (9000, 2), (66, 33)])
+def test_gate_then_norm_at_the_edges_of_what_a_thread_keeps(N, parts):
+    from photon_infer_amd import ops
+    T, eps = 3, 1e-5
+    y, z, w = randn(T, N, seed=1, scale=3.0), randn(T, N, seed=2), randn(N, seed=3)
+    want = P.rms_norm((y * P.silu(z)).view(T, parts, N // parts), None, eps).reshape(T, N) * w
+    out = torch.empty((T, N), device=DEV)
+    ops.gated_group_norm(out, dev32(y), dev32(z), dev32(w), eps, parts, 1.0)
+    close(out, want, f"gated norm {N} / {parts}", 2e-5)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_clamped_unit_with_biases_and_the_stream_bias(dtype):
     from photon_infer_amd import ops
