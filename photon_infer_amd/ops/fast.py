@@ -47,7 +47,8 @@ DECODE_WAVES_PER_UNIT = 2      # waves of the decode attention kernel per comput
 DECODE_MIN_KEYS_PER_SPLIT = 128
 # Waves that share a block's keys: only where the blocks fill their rounds over the units this far (320 blocks of a design with
 # capped scores, 1.25 rounds: a step of 783 us took 796) and, without ranges to replace, for contexts longer than this
-# (64 requests of 300 keys: 1,325 -> 1,336 us; of 600: 1,400 -> 1,384)
+# (64 requests of 300 keys: 1,325 -> 1,336 us; of 600: 1,400 -> 1,384; of 4,000 down to 2,000: 2,450 -> 2,331; of 4,096 each,
+# with nothing to even out: 2,530 -> 2,570)
 DECODE_WAVES_FILL, DECODE_WAVES_MIN_KEYS = 0.75, 512
 
 
