@@ -4,6 +4,7 @@ from __future__ import annotations
 import io
 import json
 import os
+from contextlib import contextmanager
 from types import SimpleNamespace
 from typing import Dict, List, Sequence
 
@@ -11,6 +12,19 @@ import numpy as np
 import torch
 
 DEV = "cuda:0"
+
+
+@contextmanager
+def library_calls():
+    """The names of the library's functions that are called meanwhile, in order."""
+    from photon_infer_amd.ops import _lib
+
+    names, call = [], _lib.call
+    _lib.call = lambda module, name, *args: names.append(name) or call(module, name, *args)
+    try:
+        yield names
+    finally:
+        _lib.call = call
 
 
 def fp32_tol(ref: torch.Tensor) -> float:

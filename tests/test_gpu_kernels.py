@@ -5,7 +5,7 @@ import pytest
 import torch
 
 import plain_llama as P
-from gpu_tools import DEV, PagedKV, attention_ctx
+from gpu_tools import DEV, PagedKV, attention_ctx, library_calls
 
 pytestmark = pytest.mark.gpu
 
@@ -769,6 +769,38 @@ def test_float32_attention_of_portions_on_the_matrix_cores(_ops, case, options):
         broken = torch.zeros(T, nh * hd, device=DEV)
         _ops.paged_attention(broken, q, paged.k, paged.v, table, ctx, nh, nkv, hd, page, 0.1, 0)
         assert broken[:q_lens[0]].isnan().all() and not broken[q_lens[0]:].isnan().any()
+
+
+@pytest.mark.parametrize("nh,nkv,hd,page", [(8, 2, 64, 16), (3, 1, 128, 32), (4, 2, 16, 16)])
+@pytest.mark.parametrize("window,chunk", [(0, 0), (50, 0), (0, 48)])
+def test_float32_attention_keeps_values_that_are_not_finite_to_the_tokens_that_see_them(_ops, nh, nkv, hd, page, window, chunk):
+    """Positions 130 .. 199 over values that are infinite or no number in the middle of the tiles, in front of a window's and in
+    front of a chunk's edge, and behind the last position of a tile but not of its request: a feature of a token is finite
+    unless the token sees such a key, as in the general kernel, and the others are what they are without them."""
+    before, n, scale = 130, 70, hd ** -0.5
+    g = gen(hd)
+    k, v = torch.randn(before + n, nkv, hd, generator=g), torch.randn(before + n, nkv, hd, generator=g)
+    bad = {(150, 0, 1): float("inf"), (100, nkv - 1, 3): float("-inf"), (143, 0, 5): float("nan"), (199, nkv - 1, 7): float("inf"), (64, 0, 2): float("nan")}
+    for at, value in bad.items():
+        v[at] = value
+    paged, ctx = PagedKV([(k, v)], page, F32, seed=hd), attention_ctx([n], [before + n], F32)
+    q = torch.randn(n, nh * hd, generator=g).to(DEV)
+    got, want = (torch.full((n, nh * hd), 7.0, device=DEV) for _ in range(2))
+    with library_calls() as names:
+        _ops.paged_attention(got, q, paged.k, paged.v, paged.table, ctx, nh, nkv, hd, page, scale, window, chunk=chunk)
+    assert names == ["pi_attention_float32"]
+    _ops.use_fast_kernels(False)
+    _ops.paged_attention(want, q, paged.k, paged.v, paged.table, ctx, nh, nkv, hd, page, scale, window, chunk=chunk)
+    seen = torch.zeros(n, nkv, nh // nkv, hd, dtype=torch.bool)
+    for t in range(n):
+        p = before + t
+        lo = max(0, p - window + 1) if window else p // chunk * chunk if chunk else 0
+        for key, head, feature in bad:
+            seen[t, head, :, feature] |= lo <= key <= p
+    seen = seen.reshape(n, nh * hd).to(DEV)
+    assert torch.equal(want.isfinite(), ~seen) and torch.equal(got.isfinite(), ~seen)
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    close(got[~seen], want[~seen].cpu(), 3e-6, "float32 attention beside values that are not finite")
 
 
 @pytest.mark.parametrize("waves", [2, 4])
