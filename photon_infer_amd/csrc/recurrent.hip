@@ -30,10 +30,10 @@ template <typename TW>
 __global__ __launch_bounds__(256) void causal_conv_silu_kernel(
     float* __restrict__ out, long out_stride, const float* __restrict__ in, long in_stride, const TW* __restrict__ w,
     const TW* __restrict__ bias, int C, int taps, const int* __restrict__ q_start, const int* __restrict__ slots,
-    float* __restrict__ state, long state_stride) {
+    float* __restrict__ state, long state_stride, int first_segment) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= C) return;
-  const int r = blockIdx.y, seg = blockIdx.z;
+  const int r = blockIdx.y, seg = first_segment + blockIdx.z;
   const int qs = q_start[r], n = q_start[r + 1] - qs;
   const int t0 = seg * PI_CONV_SEGMENT;
   if (t0 >= n) return;
@@ -99,16 +99,18 @@ extern "C" int pi_causal_conv_silu(float* out, long out_stride, const float* in,
   PI_REQUIRE(state_stride >= (long)(taps - 1) * C, "convolution: a state row of %ld floats cannot hold %d x %d inputs", state_stride, taps - 1, C);
   if (R == 0 || longest == 0) return 0;
   const int segs = (longest + PI_CONV_SEGMENT - 1) / PI_CONV_SEGMENT;
-  PI_REQUIRE(segs <= 65535, "convolution: a request brings too many tokens (%d)", longest);
-  const dim3 grid((C + 255) / 256, R, segs), block(256);
-  if (w_dtype == PI_F32)
-    hipLaunchKernelGGL(causal_conv_silu_kernel<float>, grid, block, 0, stream, out, out_stride, in, in_stride, (const float*)w,
-                       (const float*)bias, C, taps, q_start, slots, state, state_stride);
-  else if (w_dtype == PI_BF16)
-    hipLaunchKernelGGL(causal_conv_silu_kernel<bf16_t>, grid, block, 0, stream, out, out_stride, in, in_stride, (const bf16_t*)w,
-                       (const bf16_t*)bias, C, taps, q_start, slots, state, state_stride);
-  else
-    return pi_fail("convolution: unsupported weight dtype %d", w_dtype);
+  // a grid holds 65,535 segments; only the first of all touches the state, the others read inputs alone
+  for (int first = 0; first < segs; first += 65535) {
+    const dim3 grid((C + 255) / 256, R, segs - first < 65535 ? segs - first : 65535), block(256);
+    if (w_dtype == PI_F32)
+      hipLaunchKernelGGL(causal_conv_silu_kernel<float>, grid, block, 0, stream, out, out_stride, in, in_stride, (const float*)w,
+                         (const float*)bias, C, taps, q_start, slots, state, state_stride, first);
+    else if (w_dtype == PI_BF16)
+      hipLaunchKernelGGL(causal_conv_silu_kernel<bf16_t>, grid, block, 0, stream, out, out_stride, in, in_stride, (const bf16_t*)w,
+                         (const bf16_t*)bias, C, taps, q_start, slots, state, state_stride, first);
+    else
+      return pi_fail("convolution: unsupported weight dtype %d", w_dtype);
+  }
   return pi_check_launch("causal_conv_silu");
 }
 

@@ -90,6 +90,18 @@ def test_convolution_whole_in_portions_and_in_slots_used_again(taps, bias):
     assert bool((state[:, (taps - 1) * C:] == 7.0).all()) and bool((state[1] == 7.0).all()) and bool((state[3] == 7.0).all())
 
 
+def test_convolution_of_more_tokens_than_one_grid_has_segments():
+    from photon_infer_amd import ops
+    T, C, taps = 65535 * 16 + 21, 2, 4
+    u, w = torch.randn(T, C, device=DEV), randn(C, taps, seed=1)
+    state, out = torch.zeros((1, (taps - 1) * C), device=DEV), torch.empty((T, C), device=DEV)
+    ops.causal_conv_silu(out, u, dev32(w), None, state_ctx([T], [0]), state)
+    padded = torch.cat([torch.zeros(taps - 1, C, device=DEV), u])
+    want = P.silu(sum(padded[j:j + T] * dev32(w)[:, j] for j in range(taps)))
+    close(out, want.cpu(), "convolution of a million tokens")
+    assert torch.equal(state.view(taps - 1, C), u[-(taps - 1):])
+
+
 @pytest.mark.parametrize("sizes", [(2, 24, 16, 1), (4, 32, 32, 2), (3, 20, 12, 3), (1, 5, 100, 1), (2, 64, 128, 2), (6, 16, 3, 2)])
 def test_state_space_recurrence_whole_in_portions_and_token_by_token(sizes):
     from photon_infer_amd import ops
