@@ -208,8 +208,8 @@ template <int NR, bool SHORT>
 __global__ __launch_bounds__((PI_SCAN_WAVES + 1) * PI_WAVE) void state_space_scan_kernel(
     float* __restrict__ y, long y_stride, const float* __restrict__ xbc, long xbc_stride, const float* __restrict__ dt_raw,
     long dt_stride, const float* __restrict__ dt_bias, const float* __restrict__ A_log, const float* __restrict__ Dskip,
-    const int* __restrict__ q_start, const int* __restrict__ slots, float* __restrict__ state, long state_stride, int H, int P,
-    int N, int G, int vec) {
+    const int* __restrict__ q_start, const int* __restrict__ slots, int upto, float* __restrict__ state, long state_stride,
+    int H, int P, int N, int G, int vec) {
   constexpr int W = ScanShape<NR, SHORT>::W, CH = ScanShape<NR, SHORT>::CH;
   __shared__ __attribute__((aligned(16))) float sB[2][CH * W];
   __shared__ __attribute__((aligned(16))) float sC[2][CH * W];
@@ -218,7 +218,7 @@ __global__ __launch_bounds__((PI_SCAN_WAVES + 1) * PI_WAVE) void state_space_sca
   const int wave = threadIdx.x / PI_WAVE, lane = threadIdx.x % PI_WAVE, part = lane % 16;
   const int g = h / (H / G);
   const int qs = q_start[r], n = q_start[r + 1] - qs;
-  if (n <= 0) return;
+  if (n <= 0 || (upto > 0 && n > upto)) return;
   const int chunks = (n + CH - 1) / CH;
   const long b_col = (long)H * P + (long)g * N, c_col = b_col + (long)G * N, x_col = (long)h * P + z * PI_SCAN_COLUMNS;
 
@@ -292,10 +292,12 @@ __global__ __launch_bounds__((PI_SCAN_WAVES + 1) * PI_WAVE) void state_space_sca
   }
 }
 
+// `upto` > 0: requests that bring more tokens than that are left out (the chunked form takes them); `longest`: the most
+// tokens of the others.
 extern "C" int pi_state_space_scan(float* y, long y_stride, const float* xbc, long xbc_stride, const float* dt_raw, long dt_stride,
                                    const float* dt_bias, const float* A_log, const float* Dskip, const int* q_start,
-                                   const int* slots, int R, int longest, float* state, long state_stride, int H, int P, int N, int G,
-                                   hipStream_t stream) {
+                                   const int* slots, int R, int longest, int upto, float* state, long state_stride, int H, int P, int N,
+                                   int G, hipStream_t stream) {
   PI_REQUIRE(H > 0 && H <= 65535 && P > 0 && N > 0 && G > 0 && H % G == 0, "state space: bad sizes heads=%d vdim=%d state=%d groups=%d", H, P, N, G);
   const int nr = scan_rows_per_lane(N);
   PI_REQUIRE(nr > 0, "state space: a state of %d rows per head is more than 256", N);
@@ -305,7 +307,7 @@ extern "C" int pi_state_space_scan(float* y, long y_stride, const float* xbc, lo
   const dim3 grid(R, H, (P + PI_SCAN_COLUMNS - 1) / PI_SCAN_COLUMNS), block((PI_SCAN_WAVES + 1) * PI_WAVE);
 #define PI_LAUNCH_SS1(NR_, SHORT_)                                                                                                       \
   hipLaunchKernelGGL((state_space_scan_kernel<NR_, SHORT_>), grid, block, 0, stream, y, y_stride, xbc, xbc_stride, dt_raw, dt_stride, \
-                     dt_bias, A_log, Dskip, q_start, slots, state, state_stride, H, P, N, G, vec)
+                     dt_bias, A_log, Dskip, q_start, slots, upto, state, state_stride, H, P, N, G, vec)
 #define PI_LAUNCH_SS(NR_) do { if (longest <= 2) PI_LAUNCH_SS1(NR_, true); else PI_LAUNCH_SS1(NR_, false); } while (0)
   switch (nr) {
     case 1: PI_LAUNCH_SS(1); break;

@@ -1,5 +1,5 @@
 // The state-space recurrence of prompt portions, a chunk of 64 tokens at a time on the matrix cores, 32-bit throughout
-// (recurrent.hip holds the definition and the walk, which single tokens and short portions keep).  With la_t = -exp(A_log)
+// (recurrent.hip holds the definition and the walk, which requests with fewer tokens in the step keep, also beside longer ones).  With la_t = -exp(A_log)
 // dt_t and g_t its sum from the chunk's start,
 //   y_t = exp(g_t) S_0^T C_t + sum_{u <= t} exp(g_t - g_u) dt_u (C_t . B_u) x_u + D x_t
 //   S_64 = exp(g_64) S_0 + sum_u exp(g_64 - g_u) dt_u B_u x_u^T
@@ -65,12 +65,12 @@ template <int N>
 __global__ __launch_bounds__(256) void chunk_states_kernel(float* __restrict__ states, float* __restrict__ decays, const float* __restrict__ xbc,
                                                            long xbc_stride, const float* __restrict__ dt_raw, long dt_stride,
                                                            const float* __restrict__ dt_bias, const float* __restrict__ A_log,
-                                                           const int* __restrict__ q_start, int R, int H, int P, int G) {
+                                                           const int* __restrict__ q_start, int R, int from, int H, int P, int G) {
   __shared__ f32x4_t xt[64 * XROW], bt[N * XROW];
   __shared__ float weight[CHUNK];
   const int h = blockIdx.y, p0 = blockIdx.z * 64, tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
   const int lr = lane % 16, lg = lane / 16;
-  const TokenTile at = find_token_tile(q_start, R, CHUNK, blockIdx.x);
+  const TokenTile at = find_token_tile(q_start, R, CHUNK, blockIdx.x, from);
   if (at.req < 0) return;
   const long t0 = q_start[at.req] + (long)at.tile * CHUNK;
   const int tokens = min(CHUNK, (int)(q_start[at.req + 1] - t0)), cols = min(64, P - p0);
@@ -112,10 +112,10 @@ __global__ __launch_bounds__(256) void chunk_states_kernel(float* __restrict__ s
 // A thread takes one element of a request's state through its chunks: states[chunk] becomes the state at the chunk's start.
 // The state row is in the walk's order (recurrent.hip): [head][slice of four columns][i][lane], NR rows per lane.
 __global__ __launch_bounds__(256) void chunk_carry_kernel(float* __restrict__ states, const float* __restrict__ decays, const int* __restrict__ q_start,
-                                                          const int* __restrict__ slots, float* __restrict__ state, long state_stride, int H, int P,
-                                                          int N, int NR) {
+                                                          const int* __restrict__ slots, int from, float* __restrict__ state, long state_stride,
+                                                          int H, int P, int N, int NR) {
   const int r = blockIdx.x, h = blockIdx.y, e = blockIdx.z * 256 + threadIdx.x;
-  const int first = token_tiles_before(q_start, r, CHUNK), chunks = (q_start[r + 1] - q_start[r] + CHUNK - 1) / CHUNK;
+  const int first = token_tiles_before(q_start, r, CHUNK, from), chunks = token_tiles(q_start[r + 1] - q_start[r], CHUNK, from);
   if (e >= P * N || chunks == 0) return;
   const int p = e / N, n = e % N, slices = (P + 15) / 16 * 4;
   float* mine = state + (long)slots[r] * state_stride + (((long)h * slices + p / 4) * NR + n % NR) * PI_WAVE + (p % 4) * 16 + n / NR;
@@ -149,7 +149,7 @@ template <int N>
 __global__ __launch_bounds__(256) void chunk_outputs_kernel(float* __restrict__ y, long y_stride, const float* __restrict__ states,
                                                             const float* __restrict__ xbc, long xbc_stride, const float* __restrict__ dt_raw,
                                                             long dt_stride, const float* __restrict__ dt_bias, const float* __restrict__ A_log,
-                                                            const float* __restrict__ Dskip, const int* __restrict__ q_start, int R, int H, int P, int G) {
+                                                            const float* __restrict__ Dskip, const int* __restrict__ q_start, int R, int from, int H, int P, int G) {
   constexpr int NROW = N / 4 + 1, IT = 64 * (N / 4) / 256;
   __shared__ f32x4_t rows[64 * NROW];           // first the tokens' B, then the state at the chunk's start, a row per value column
   __shared__ f32x4_t xt[64 * XROW];
@@ -158,7 +158,7 @@ __global__ __launch_bounds__(256) void chunk_outputs_kernel(float* __restrict__ 
   const int h = blockIdx.y, p0 = blockIdx.z * 64, tid = threadIdx.x, lane = tid % 64;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
   const int lr = lane % 16, lg = lane / 16;
-  const TokenTile at = find_token_tile(q_start, R, CHUNK, blockIdx.x);
+  const TokenTile at = find_token_tile(q_start, R, CHUNK, blockIdx.x, from);
   if (at.req < 0) return;
   const long t0 = q_start[at.req] + (long)at.tile * CHUNK;
   const int tokens = min(CHUNK, (int)(q_start[at.req + 1] - t0)), cols = min(64, P - p0);
@@ -245,21 +245,22 @@ __global__ __launch_bounds__(256) void chunk_outputs_kernel(float* __restrict__ 
   }
 }
 
-// Tokens of a chunk, for the caller's count of chunks (sum over requests of ceil(tokens / this)), or 0: sizes that the
-// chunked form does not take.
+// Tokens of a chunk, for the caller's count of chunks (sum of ceil(tokens / this) over the requests that run in chunks), or
+// 0: sizes that the chunked form does not take.
 extern "C" int pi_state_space_chunk(int P, int N) { return P > 0 && P % 4 == 0 && (N == 16 || N == 32 || N == 64 || N == 128) ? CHUNK : 0; }
 
-// `states`: float32 [chunks, H, P, N], `decays`: float32 [chunks, H], both scratch.  Arguments otherwise as for
+// The requests that bring `from` tokens or more.  `states`: float32 [chunks, H, P, N], `decays`: float32 [chunks, H], both
+// scratch.  Arguments otherwise as for
 // pi_state_space_scan; rows of x, B, C and y must be 16-byte aligned.
 extern "C" int pi_state_space_chunks(float* y, long y_stride, const float* xbc, long xbc_stride, const float* dt_raw, long dt_stride,
                                      const float* dt_bias, const float* A_log, const float* Dskip, const int* q_start, const int* slots, int R,
-                                     int chunks, float* states, float* decays, float* state, long state_stride, int H, int P, int N, int G,
+                                     int from, int chunks, float* states, float* decays, float* state, long state_stride, int H, int P, int N, int G,
                                      hipStream_t stream) {
   PI_REQUIRE(H > 0 && H <= 65535 && P > 0 && N > 0 && G > 0 && H % G == 0, "state space: bad sizes heads=%d vdim=%d state=%d groups=%d", H, P, N, G);
   PI_REQUIRE(pi_state_space_chunk(P, N) > 0, "state space: no chunked form for heads of %d with a state of %d", P, N);
   int nr = 1;
   while (16 * nr < N) nr *= 2;
-  PI_REQUIRE(R > 0 && chunks > 0 && states && decays && state_stride >= (long)H * ((P + 15) / 16) * 4 * nr * PI_WAVE,
+  PI_REQUIRE(R > 0 && from > 0 && chunks > 0 && states && decays && state_stride >= (long)H * ((P + 15) / 16) * 4 * nr * PI_WAVE,
              "state space: bad step (%d requests, %d chunks) or a state row of %ld floats that cannot hold %d x %d x %d", R, chunks, state_stride, H, N, P);
   PI_REQUIRE(xbc_stride % 4 == 0 && y_stride % 4 == 0 && (uintptr_t)xbc % 16 == 0 && (uintptr_t)y % 16 == 0 && (uintptr_t)states % 16 == 0,
              "state space: rows must be 16-byte aligned");
@@ -267,10 +268,10 @@ extern "C" int pi_state_space_chunks(float* y, long y_stride, const float* xbc, 
 #define GO(N_)                                                                                                                                   \
   case N_:                                                                                                                                       \
     hipLaunchKernelGGL((chunk_states_kernel<N_>), grid, block, 0, stream, states, decays, xbc, xbc_stride, dt_raw, dt_stride, dt_bias, A_log,    \
-                       q_start, R, H, P, G);                                                                                                     \
-    hipLaunchKernelGGL(chunk_carry_kernel, carry, block, 0, stream, states, decays, q_start, slots, state, state_stride, H, P, N_, nr);          \
+                       q_start, R, from, H, P, G);                                                                                               \
+    hipLaunchKernelGGL(chunk_carry_kernel, carry, block, 0, stream, states, decays, q_start, slots, from, state, state_stride, H, P, N_, nr);    \
     hipLaunchKernelGGL((chunk_outputs_kernel<N_>), grid, block, 0, stream, y, y_stride, states, xbc, xbc_stride, dt_raw, dt_stride, dt_bias,     \
-                       A_log, Dskip, q_start, R, H, P, G);                                                                                       \
+                       A_log, Dskip, q_start, R, from, H, P, G);                                                                                 \
     break
   switch (N) {
     GO(16); GO(32); GO(64); GO(128);

@@ -1261,13 +1261,11 @@ def causal_conv_silu(out: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, b
               ctx.q_start.data_ptr(), ctx.slots.data_ptr(), ctx.R, longest, state.data_ptr(), state.stride(0), _stream())
 
 
-STATE_SPACE_CHUNKS_FROM = 128     # tokens of a step's longest request from which the recurrence runs in chunks (three launches against one walk)
-
-
-def _tiles_of_tokens(ctx, T: int, size: int) -> int:
-    """Tiles of up to ``size`` tokens that a step's requests are cut into (an upper bound where the host has no lengths)."""
-    lens = getattr(ctx, "q_lens", None)
-    return sum(-(-n // size) for n in lens) if lens else T // size + ctx.R
+# Tokens of a step's longest request from which the recurrence runs in chunks (three launches, some 30 us, as long as a walk of 128
+# tokens), and of the requests beside it that then do so too: all that the walk's form for a token or two does not take, for a
+# whole chunk of 64 rows is worth some 20 tokens of a walk in a full step.  32 heads of 64, state of 128, beside a request of
+# 128 tokens: 64 single tokens 81 us (walked with it 144, in chunks with it 187), 9 single tokens and 9 requests of 3 64 (69, 75).
+STATE_SPACE_CHUNKS_FROM, STATE_SPACE_CHUNKS_BESIDE = 128, 3
 
 
 def state_space_scan(y: torch.Tensor, xbc: torch.Tensor, dt: torch.Tensor, dt_bias: torch.Tensor, a_log: torch.Tensor,
@@ -1287,19 +1285,24 @@ def state_space_scan(y: torch.Tensor, xbc: torch.Tensor, dt: torch.Tensor, dt_bi
     _state_rows(state, scan_state_floats(heads, state_dim, value_dim), "state space")
     _i32(ctx.q_start, "q_start", ctx.R + 1)
     _i32(ctx.slots, "slots", ctx.R)
-    longest = int(getattr(ctx, "max_q_len", 0) or T)
+    longest, upto = int(getattr(ctx, "max_q_len", 0) or T), 0
     chunk = _lib.load("core").pi_state_space_chunk(value_dim, state_dim) if _FAST and longest >= STATE_SPACE_CHUNKS_FROM else 0
     if chunk and ldx % 4 == 0 and ldy % 4 == 0 and xbc.data_ptr() % 16 == 0 and y.data_ptr() % 16 == 0:
-        chunks = _tiles_of_tokens(ctx, T, chunk)
+        upto = STATE_SPACE_CHUNKS_BESIDE - 1
+        lens = getattr(ctx, "q_lens", None)
+        # without lengths on the host: an upper bound, and requests that may walk
+        chunks = sum(-(-n // chunk) for n in lens if n > upto) if lens else T // chunk + ctx.R
         states = torch.empty((chunks, heads, value_dim, state_dim), dtype=torch.float32, device=y.device)
         decays = torch.empty((chunks, heads), dtype=torch.float32, device=y.device)
         _lib.call("core", "pi_state_space_chunks", y.data_ptr(), ldy, xbc.data_ptr(), ldx, dt.data_ptr(), ldd, dt_bias.data_ptr(),
-                  a_log.data_ptr(), skip.data_ptr(), ctx.q_start.data_ptr(), ctx.slots.data_ptr(), ctx.R, chunks, states.data_ptr(),
+                  a_log.data_ptr(), skip.data_ptr(), ctx.q_start.data_ptr(), ctx.slots.data_ptr(), ctx.R, upto + 1, chunks, states.data_ptr(),
                   decays.data_ptr(), state.data_ptr(), state.stride(0), heads, value_dim, state_dim, groups, _stream())
-        return
+        longest = max((n for n in lens if n <= upto), default=0) if lens else min(upto, T - longest)
+        if longest == 0:
+            return
     _lib.call("core", "pi_state_space_scan", y.data_ptr(), ldy, xbc.data_ptr(), ldx, dt.data_ptr(), ldd, dt_bias.data_ptr(),
               a_log.data_ptr(), skip.data_ptr(), ctx.q_start.data_ptr(), ctx.slots.data_ptr(), ctx.R,
-              longest, state.data_ptr(), state.stride(0), heads, value_dim, state_dim, groups, _stream())
+              longest, upto, state.data_ptr(), state.stride(0), heads, value_dim, state_dim, groups, _stream())
 
 
 def gated_group_norm(out: torch.Tensor, y: torch.Tensor, z: torch.Tensor, weight: torch.Tensor, eps: float, parts: int,

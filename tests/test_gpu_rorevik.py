@@ -13,7 +13,7 @@ import torch
 
 import plain_rorevik as P
 import tiny_rorevik as TR
-from gpu_tools import DEV, attention_ctx, cut_steps, live_token_need, run_trace
+from gpu_tools import DEV, attention_ctx, cut_steps, library_calls, live_token_need, run_trace
 from tiny_models import random_tokens
 
 pytestmark = pytest.mark.gpu
@@ -167,6 +167,42 @@ def test_state_space_recurrence_in_chunks(sizes):
     y = torch.empty((333, H * Pd), device=DEV)
     ops.state_space_scan(y, xbc, dt, dev32(dt_bias), dev32(A_log), dev32(D), state_ctx([333], [0]), torch.zeros((1, floats), device=DEV), H, Pd, N, G)
     assert not bool(y[:, 1].isfinite()[100:].any()) and bool(y[:100].isfinite().all()) and bool(y[:, 0].isfinite().all()) and bool(y[:, 2:].isfinite().all())
+
+
+@pytest.mark.parametrize("lengths_on_host", [True, False])
+def test_single_tokens_walk_beside_a_request_that_runs_in_chunks(lengths_on_host):
+    """Outputs and states of requests of one and two tokens are the same bits as without the long request, which takes the chunked
+    form, as a request of three tokens then does; a step of long requests alone does not walk."""
+    from photon_infer_amd import ops
+    H, Pd, N, G = 3, 64, 32, 1
+    lens = [1, 2, 140, 1, 3, 1, 128]
+    T, floats = sum(lens), ops.scan_state_floats(H, N, Pd)
+    xbc, dt = dev32(randn(T, H * Pd + 2 * G * N, seed=1, scale=0.5)), dev32(randn(T, H, seed=2))
+    params = dev32(randn(H, seed=3)), dev32(randn(H, seed=4)), dev32(randn(H, seed=5))
+    start = dev32(randn(len(lens), floats, seed=6))
+
+    def scan(rows, slots, q_lens):
+        y, state, ctx = torch.empty((len(rows), H * Pd), device=DEV), start.clone(), state_ctx(q_lens, slots)
+        if lengths_on_host:
+            ctx.q_lens = q_lens
+        with library_calls() as names:
+            ops.state_space_scan(y, xbc[rows].contiguous(), dt[rows].contiguous(), *params, ctx, state, H, Pd, N, G)
+        return y, state, names
+
+    first = np.concatenate([[0], np.cumsum(lens)])
+    y, state, names = scan(torch.arange(T), list(range(len(lens))), lens)
+    assert names == ["pi_state_space_chunks", "pi_state_space_scan"]
+    short = [r for r, n in enumerate(lens) if n <= 2]
+    rows = torch.cat([torch.arange(first[r], first[r + 1]) for r in short])
+    y_short, state_short, names = scan(rows, short, [lens[r] for r in short])
+    assert names == ["pi_state_space_scan"]
+    assert torch.equal(y[rows], y_short) and torch.equal(state[short], state_short[short])
+    for r in (2, 4, 6):                      # the others, each alone: 64 bits as the yardstick are in the test above
+        alone, left, _ = scan(torch.arange(first[r], first[r + 1]), [r], [lens[r]])
+        close(y[first[r]:first[r + 1]], alone.double().cpu(), f"request {r}", 1e-5)
+        close(state[r], left[r].double().cpu(), f"state {r}", 1e-5)
+    if lengths_on_host:
+        assert scan(torch.arange(128), [6], [128])[2] == ["pi_state_space_chunks"]
 
 
 def delta_inputs(t, H, G, d, dv, seed):
