@@ -690,9 +690,33 @@ def paged_attention(out, q, k_cache, v_cache, block_table, ctx, num_heads, num_k
     return True
 
 
-# Below this many tokens a step of portions over contexts longer than this goes to the general kernel, which cuts the keys
-# of few tokens into ranges; a tile walks its whole context in one block
-FLOAT32_TILE_MIN_TOKENS, FLOAT32_TILE_SHORT_CONTEXT = 32, 512
+def float32_attention_us(q_lens, kv_lens, num_heads: int, num_kv_heads: int, head_dim: int, tile_tokens: int, reach: int = 0) -> Tuple[float, float]:
+    """What a step takes on the float32 path's tile kernel and on its general kernel (``reach`` > 0: a token sees at most so many
+    keys).  Tiles: a block walks its keys 64 at a time, whether its 64 rows of (token, head) are there or not; the longest
+    walk, or all of them dealt over the chip.  General: a wave per token and head, so its (query, key) pairs, and the chain
+    along the longest context, cut into ranges where the waves are few.  Fitted to 400 random steps on an MI355X - prompts,
+    portions over up to 12,000 keys, single tokens beside them; heads of 16 to 128, 1 to 12 per kv head; windows - where each
+    kernel is the faster one in about half, by up to 9 times."""
+    units, seen = compute_units(), reach or 1 << 30
+    rounds, longest, pairs, chain = 0.0, 0.0, 0.0, 0
+    for n, kv in zip(q_lens, kv_lens):
+        before, rows = kv - n, min(tile_tokens, n)
+        rounds += -(-n // tile_tokens) * (min(before + (n + rows) / 2, seen + rows) / 64 + 0.5)
+        longest = max(longest, -(-min(kv, seen + tile_tokens) // 64))
+        pairs += n * min(before + n / 2, seen)
+        chain = max(chain, min(kv, seen))
+    blocks_per_tile = num_heads * tile_tokens // 64
+    tiles = 5.3 + (1.2 + 0.053 * head_dim) * max(longest, rounds * blocks_per_tile / units)
+    if chain >= 256:
+        chain /= max(1, min(64, 4096 // (sum(q_lens) * num_heads)))
+    return tiles, 8.3 + pairs * num_heads * head_dim * 0.9e-6 + chain * (0.078 + 0.0002 * head_dim)
+
+
+# What the tile kernel must promise at most of the general kernel's time, for both are off by a fifth in places.  Of the 400
+# steps above 13 then take more than 3 % longer than on the general kernel (by a few microseconds), and the mean is 2.3 % above
+# the better of the two; with the tile kernel from 32 tokens on (the rule before) it was 121 steps and 15 %: 32 tokens at 32,768
+# keys, 24 heads of 128: 3,600 us, 2,450 now; 31 single tokens and 33 at 2,000: 590 us, 450 now.
+FLOAT32_TILES_WORTH = 0.8
 
 
 def paged_attention_float32(out, q, k_cache, v_cache, block_table, ctx, num_heads, num_kv_heads, head_dim, page_size, scale, window, pages,
@@ -702,9 +726,17 @@ def paged_attention_float32(out, q, k_cache, v_cache, block_table, ctx, num_head
     if (head_dim % 16 or head_dim > 128 or page_size % 16 or q.data_ptr() % 16 or out.data_ptr() % 16 or q.stride(0) % 4 or out.stride(0) % 4
             or k_cache.data_ptr() % 16 or v_cache.data_ptr() % 16):
         return False
-    if ctx.T < FLOAT32_TILE_MIN_TOKENS and ctx.max_kv_len > FLOAT32_TILE_SHORT_CONTEXT:
-        return False
     rows = _lib.load("core").pi_attention_float32_tile_tokens(num_heads, num_kv_heads)
+    reach = min(window or 1 << 30, chunk or 1 << 30) if window or chunk else 0
+    key = ("float32 attention", num_heads, num_kv_heads, head_dim, reach)
+    plans = getattr(ctx, "plans", None)
+    if plans is None:
+        plans = ctx.plans = {}
+    if key not in plans:
+        tiles_us, general_us = float32_attention_us(ctx.q_lens, ctx.kv_lens, num_heads, num_kv_heads, head_dim, rows, reach)
+        plans[key] = tiles_us < FLOAT32_TILES_WORTH * general_us
+    if not plans[key]:
+        return False
     tiles = sum(-(-n // rows) for n in ctx.q_lens)
     _lib.call("core", "pi_attention_float32", out.data_ptr(), out.stride(0), q.data_ptr(), q.stride(0), k_cache.data_ptr(), v_cache.data_ptr(),
               block_table.data_ptr(), block_table.shape[1], ctx.q_start.data_ptr(), ctx.kv_len.data_ptr(), ctx.R, tiles, num_heads, num_kv_heads,

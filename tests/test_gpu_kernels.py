@@ -742,9 +742,11 @@ FLOAT32_ATTN_CASES = [c for c in ATTN_CASES if c[2] <= 128 and c[3] % 16 == 0 an
 
 @pytest.mark.parametrize("case", FLOAT32_ATTN_CASES + [(8, 4, 64, 16, [1] * 70 + [33, 16], [5] * 70 + [600, 16], None)])
 @pytest.mark.parametrize("options", [False, True])
-def test_float32_attention_of_portions_on_the_matrix_cores(_ops, case, options):
+def test_float32_attention_of_portions_on_the_matrix_cores(_ops, monkeypatch, case, options):
     """The tile kernel against the general kernel, which other tests hold to the plain implementation, on portions cut at
     the tiles' and pages' edges; with every option at once too.  Weights and sums are 32-bit in both."""
+    from photon_infer_amd.ops import fast
+    monkeypatch.setattr(fast, "FLOAT32_TILES_WORTH", math.inf)          # also where the general kernel would be the faster one
     nh, nkv, hd, page, q_lens, kv_lens, window = case
     g = gen(nh + hd)
     kvs = [(torch.randn(kv, nkv, hd, generator=g), torch.randn(kv, nkv, hd, generator=g)) for kv in kv_lens]
@@ -757,26 +759,31 @@ def test_float32_attention_of_portions_on_the_matrix_cores(_ops, case, options):
         ways = [dict(one, gate=torch.rand(T * nh, generator=g).to(DEV)), dict(one, feature_gate=torch.randn(T, nh * hd + 4, generator=g).to(DEV)[:, :nh * hd])]
     for way in ways:
         got, want = torch.full((T, nh * hd), float("nan"), device=DEV), torch.empty(T, nh * hd, device=DEV)
-        for out, fast in ((got, True), (want, False)):
-            _ops.use_fast_kernels(fast)
-            ctx.T = max(T, 32)          # a step of few tokens would keep to the general kernel
-            _ops.paged_attention(out, q, paged.k, paged.v, paged.table, ctx, nh, nkv, hd, page, 1.0 / math.sqrt(hd), window or 0, **way)
+        for out, kernel in ((got, "pi_attention_float32"), (want, "pi_paged_attention_general")):
+            _ops.use_fast_kernels(out is got)
+            with library_calls() as names:
+                _ops.paged_attention(out, q, paged.k, paged.v, paged.table, ctx, nh, nkv, hd, page, 1.0 / math.sqrt(hd), window or 0, **way)
+            assert names == [kernel]
         _ops.use_fast_kernels(True)
         close(got, want.cpu(), 3e-6, "float32 attention")
     if not options:                      # a page that is not there shows in the tokens that see it
         table = paged.table.clone()
         table[0, 0] = -1
         broken = torch.zeros(T, nh * hd, device=DEV)
-        _ops.paged_attention(broken, q, paged.k, paged.v, table, ctx, nh, nkv, hd, page, 0.1, 0)
+        with library_calls() as names:
+            _ops.paged_attention(broken, q, paged.k, paged.v, table, ctx, nh, nkv, hd, page, 0.1, 0)
+        assert names == ["pi_attention_float32"]
         assert broken[:q_lens[0]].isnan().all() and not broken[q_lens[0]:].isnan().any()
 
 
 @pytest.mark.parametrize("nh,nkv,hd,page", [(8, 2, 64, 16), (3, 1, 128, 32), (4, 2, 16, 16)])
 @pytest.mark.parametrize("window,chunk", [(0, 0), (50, 0), (0, 48)])
-def test_float32_attention_keeps_values_that_are_not_finite_to_the_tokens_that_see_them(_ops, nh, nkv, hd, page, window, chunk):
+def test_float32_attention_keeps_values_that_are_not_finite_to_the_tokens_that_see_them(_ops, monkeypatch, nh, nkv, hd, page, window, chunk):
     """Positions 130 .. 199 over values that are infinite or no number in the middle of the tiles, in front of a window's and in
     front of a chunk's edge, and behind the last position of a tile but not of its request: a feature of a token is finite
     unless the token sees such a key, as in the general kernel, and the others are what they are without them."""
+    from photon_infer_amd.ops import fast
+    monkeypatch.setattr(fast, "FLOAT32_TILES_WORTH", math.inf)
     before, n, scale = 130, 70, hd ** -0.5
     g = gen(hd)
     k, v = torch.randn(before + n, nkv, hd, generator=g), torch.randn(before + n, nkv, hd, generator=g)

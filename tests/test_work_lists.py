@@ -114,3 +114,22 @@ def test_pieces_that_would_not_fit_the_workspace_are_refused():
         assert fast._tile_splits(M, N, K) * M * N <= GEMM_PART_FLOATS or fast._tile_splits(M, N, K) == 1
     for M, N, K in [(8, 128256, 2048), (128, 128256, 8192), (64, 16384, 2048), (1, 2048, 8192)]:
         assert fast._skinny_splits(M, N, K) * M * N <= GEMM_PART_FLOATS or fast._skinny_splits(M, N, K) == 1
+
+
+# (requests' tokens, contexts, heads, kv heads, head size, window, microseconds on the tile kernel, on the general kernel), measured
+FLOAT32_STEPS = [
+    ([32], [2048], 32, 8, 64, 0, 150, 127), ([32], [32768], 32, 8, 64, 0, 2316, 1687), ([32], [32768], 24, 8, 128, 0, 3604, 2452),
+    ([1] * 31 + [33], [2000] * 32, 24, 8, 128, 0, 590, 451), ([1] * 63 + [16], [4000] * 64, 24, 8, 128, 0, 2155, 1302), ([2] * 16, [4000] * 16, 24, 8, 128, 0, 732, 409),
+    ([64], [8192], 32, 8, 64, 0, 581, 1076), ([256], [8192], 24, 8, 128, 0, 912, 5003), ([1] * 8 + [64], [16000] * 9, 32, 8, 64, 0, 1147, 2562),
+    ([1] * 31 + [128], [2000] * 32, 32, 8, 64, 0, 234, 680), ([517, 431, 345], [517, 431, 345], 32, 8, 64, 0, 64, 462),
+]
+
+
+@pytest.mark.parametrize("step", FLOAT32_STEPS, ids=[f"step{i}" for i in range(len(FLOAT32_STEPS))])
+def test_the_float32_path_takes_the_attention_kernel_that_was_the_faster_one(step):
+    from photon_infer_amd.ops import fast
+    q_lens, kv_lens, heads, kv_heads, head_dim, window, tiles, general = step
+    tile_tokens = 64 if heads // kv_heads % 2 else 16
+    tiles_us, general_us = fast.float32_attention_us(q_lens, kv_lens, heads, kv_heads, head_dim, tile_tokens, window)
+    assert (tiles_us < fast.FLOAT32_TILES_WORTH * general_us) == (tiles < general)
+    assert 0.6 < tiles_us / tiles < 1.6 and 0.5 < general_us / general < 1.6       # and the estimates are of that size
