@@ -22,6 +22,7 @@
 
 #include "addressing.h"
 #include "mfma.h"
+#include "tile_plan.h"
 
 PI_DEFINE_MODULE(bf16)
 
@@ -369,7 +370,7 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(void* __restrict__ Cv, l
 // chip and a k that is a multiple of the slab: eight waves in 2 x 4 (two per SIMD), each
 // WI x WJ tiles of v_mfma_f32_32x32x16_bf16, so that a block's tile is 64 WI x 128 WJ: 256 x 256,
 // 192 x 384, 192 x 256, 128 x 384 or 128 x 256.  A unit holds one block, and a last round of few blocks
-// costs as much as a full one: which shape a product takes is decided by the rounds it needs (ops/fast.py).
+// costs as much as a full one: which shape a product takes is decided by the rounds it needs (tile_plan.h).
 // At 256 x 256 a wave reads 6 fragments from
 // LDS per 16 k for 8 matrix-core instructions, three quarters of the LDS traffic per flop of the
 // 128 x 128 kernel (192 x 384: 6 for 9, 128 x 256: 4 for 4), and a block asks L2 for half the bytes per flop.  With one wave per SIMD
@@ -637,6 +638,14 @@ extern "C" int pi_gemm_mfma_grouped(void* C, int epilogue, long ldc, const void*
 extern "C" int pi_gemm_mfma_pieces(int K, int splits) {
   if (splits < 1 || K < 1) return 0;
   return addressing::cut_k(K, splits, BK).splits;
+}
+
+// Which block tile, and how many pieces: see tile_plan.h.
+extern "C" int pi_gemm_mfma_shape(int M, int N, int K, int splits, int units) {
+  return M > 0 && N > 0 && K > 0 && splits > 0 && units > 0 ? tile_plan::shape_for(M, N, K, splits, units).code : 0;
+}
+extern "C" int pi_gemm_mfma_splits(int M, int N, int K, int units, long part_floats, double worth) {
+  return M > 0 && N > 0 && K > 0 && units > 0 ? tile_plan::splits_for(M, N, K, units, part_floats, worth) : 1;
 }
 
 // epilogue: 0 store bf16, 1 store f32, 2 add into f32, 3 SwiGLU (W rows interleaved by 16; C is [M, N / 2] bf16),

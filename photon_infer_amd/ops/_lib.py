@@ -2,7 +2,7 @@
 from __future__ import annotations
 
 import ctypes
-from ctypes import c_float, c_int, c_long, c_void_p
+from ctypes import c_double, c_float, c_int, c_long, c_void_p
 from typing import Dict
 
 import torch
@@ -10,7 +10,7 @@ import torch
 from ..errors import KernelError, KernelLibraryMissing
 from . import build
 
-P, I, L, F = c_void_p, c_int, c_long, c_float
+P, I, L, F, D = c_void_p, c_int, c_long, c_float, c_double
 
 # entry point -> argument types (all return int: 0 = ok)
 _SIGNATURES = {
@@ -65,6 +65,8 @@ _SIGNATURES = {
     "bf16": {
         "pi_gemm_mfma": [P, I, L, P, L, P, L, I, I, I, I, I, P],
         "pi_gemm_mfma_pieces": [I, I],
+        "pi_gemm_mfma_shape": [I, I, I, I, I],
+        "pi_gemm_mfma_splits": [I, I, I, I, L, D],
         "pi_gemm_mfma_clamped_glu": [P, L, P, L, P, L, I, I, I, P, F, F, I, P],
         "pi_gemm_mfma_grouped": [P, I, L, P, L, P, L, L, P, P, P, I, I, I, L, L, F, F, P, L, P],
         "pi_gemm_skinny": [P, I, L, P, L, P, L, I, I, I, I, P, L, P, I, P],

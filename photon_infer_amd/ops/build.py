@@ -34,7 +34,7 @@ MODULES: Dict[str, List[str]] = {
     # host only: the engine for C / C++ programs (hosts an interpreter; links libpython)
     "api": ["api/photon_engine.cpp"],
 }
-HEADERS = ["common.h", "mfma.h", "addressing.h", "attention_mfma.h", "sampling.h", "token_tiles.h"]
+HEADERS = ["common.h", "mfma.h", "addressing.h", "attention_mfma.h", "sampling.h", "token_tiles.h", "tile_plan.h"]
 HOST_MODULES = {"runtime", "api"}
 HOST_HEADERS = {"api": ["api/photon_engine.h"]}
 HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-Wall"]

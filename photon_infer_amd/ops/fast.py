@@ -33,8 +33,6 @@ BLOCKS_PER_UNIT = 2            # blocks of it wanted per compute unit to keep HB
 SHARED_FROM_TOKENS = 32        # more tokens than this: the skinny kernel that shares activations per block ...
 SHARED_ROWS_PER_BLOCK = 64     # ... with this many weight rows per block ...
 SHARED_BLOCKS_PER_UNIT = 1     # ... and one block wanted per compute unit
-TILE_MAX_SPLITS = 8
-TILE_MIN_K = 256               # a piece of the tile kernels keeps at least this much of k
 FLOAT32_MAX_STRIDE = 1 << 21   # floats between rows up to which the float32 kernels' offsets inside a tile fit 32 bits
 DEFAULT_UNITS = 256            # compute units assumed where no device can be asked (an MI355X)
 PIECES_WORTH = 0.95            # q, k, v of a prompt portion are left in k pieces too where that takes no more than this share of the time:
@@ -86,72 +84,25 @@ def _skinny_splits(M: int, N: int, K: int) -> int:
     return splits
 
 
-# The tile kernels: code -> (rows, columns of a block's tile, blocks a unit holds at a time, microseconds of a block that
-# has the chip nearly to itself, of one on a full chip).  Times are fitted to measurements on an MI355X of 129 to 2,627 rows
-# with nine matrices of 2,048 x 2,048 to 28,672 x 4,096, whole and in two to four pieces (k in units of 1,024): the rule
-# below takes a shape within 0.8 % of the fastest on average (the 128 x 128 and 256 x 256 tiles alone, which were all there
-# was: 5.6 %) and never one slower than those two would have been.  543 x 28,672 x 4,096: 336 tiles of 256 x 256 take two
-# rounds of 256 units, 184 us; 225 of 192 x 384 one, 130 us.  2,048 x 4,384 x 2,048: 61 us on 128 x 128, 42 to 48.
-TILE_SHAPES = {
-    0: (128, 128, 2, lambda k: 6.0 + 8.0 * k + 0.35 * k * k, lambda k: 6.0 + 16.5 * k),
-    42: (256, 256, 1, lambda k: 7.0 + 15.0 * k + 0.25 * k * k, lambda k: 6.0 + 26.0 * k),
-    33: (192, 384, 1, lambda k: 8.0 + 18.0 * k + 0.3 * k * k, lambda k: 7.0 + 32.5 * k),
-    32: (192, 256, 1, lambda k: 7.0 + 12.5 * k + 0.25 * k * k, lambda k: 5.0 + 23.5 * k),
-    23: (128, 384, 1, lambda k: 7.0 + 13.5 * k + 0.3 * k * k, lambda k: 5.0 + 28.0 * k),
-    22: (128, 256, 1, lambda k: 6.0 + 10.0 * k + 0.25 * k * k, lambda k: 4.0 + 20.5 * k),
-}
-TILE_GAIN, PIECES_GAIN = 0.96, 0.98      # what the fit, which is good to some per cent, must promise at least before another shape or one more piece is taken
-PIECES_WRITTEN, PIECES_READ = 10e6, 7e6    # bytes per microsecond: float32 pieces out of the larger tiles (beyond the times above; in those of the
-                               # 128 x 128 tiles they are hidden), and pieces or the updated stream into the norm behind the product
-
-
-def _tile_us(shape: int, M: int, N: int, K: int, splits: int, units: int) -> float:
-    rows, cols, slots, alone, full = TILE_SHAPES[shape]
-    k = -(-(-(-K // splits)) // 64) * 64 / 1024
-    rounds, rest = divmod(-(-M // rows) * -(-N // cols) * splits, slots * units)
-    top = full(k)
-    low = min(alone(k), top)
-    return rounds * top + (low + (top - low) * rest / (slots * units) if rest else 0.0)
+@functools.lru_cache(maxsize=4096)
+def _tile_shape_of(M: int, N: int, K: int, splits: int, units: int) -> int:
+    return _lib.load("bf16").pi_gemm_mfma_shape(M, N, K, splits, units)
 
 
 @functools.lru_cache(maxsize=4096)
-def _tile_plan_of(M: int, N: int, K: int, splits: int, units: int) -> Tuple[int, float]:
-    best, least = 0, _tile_us(0, M, N, K, splits, units)
-    for shape in TILE_SHAPES if K % 64 == 0 else ():      # the larger tiles take whole slabs of k only
-        us = _tile_us(shape, M, N, K, splits, units)
-        if shape and splits > 1:
-            us += 4.0 * splits * M * N / PIECES_WRITTEN
-        if us < least * (1.0 if shape == 42 else TILE_GAIN):
-            best, least = shape, us
-    return best, least
+def _tile_splits_of(M: int, N: int, K: int, units: int, worth: float) -> int:
+    return _lib.load("bf16").pi_gemm_mfma_splits(M, N, K, units, GEMM_PART_FLOATS, worth)
 
 
 def _tile_shape(M: int, N: int, K: int, splits: int) -> int:
-    """The tile shape (see TILE_SHAPES) that takes the least time for the product in ``splits`` pieces."""
-    return _tile_plan_of(M, N, K, splits, compute_units())[0]
-
-
-def _tile_plan_us(M: int, N: int, K: int, splits: int) -> float:
-    """What the product takes, with the pieces' (or the result's) way through memory."""
-    return _tile_plan_of(M, N, K, splits, compute_units())[1] + 4.0 * splits * M * N / PIECES_READ
-
-
-@functools.lru_cache(maxsize=4096)
-def _tile_splits_of(M: int, N: int, K: int, units: int) -> int:
-    best, least = 1, _tile_plan_of(M, N, K, 1, units)[1] + 4.0 * M * N / PIECES_READ      # the kernel adds into the stream
-    for splits in range(2, TILE_MAX_SPLITS + 1):
-        if K // splits < TILE_MIN_K or splits * M * N > GEMM_PART_FLOATS:
-            break
-        us = _tile_plan_of(M, N, K, splits, units)[1] + 4.0 * splits * M * N / PIECES_READ
-        if us < PIECES_GAIN * least:
-            best, least = splits, us
-    return best
+    """The block tile (its code, csrc/tile_plan.h) that takes the least time for the product in ``splits`` pieces."""
+    return _tile_shape_of(M, N, K, splits, compute_units())
 
 
 def _tile_splits(M: int, N: int, K: int) -> int:
     """k-split of the tile kernels for a product whose reader adds the pieces: as many as take the least time together
     with the pieces' way through memory."""
-    return _tile_splits_of(M, N, K, compute_units())
+    return _tile_splits_of(M, N, K, compute_units(), 1.0)
 
 
 def flush(ws: Optional[KernelWorkspace]) -> None:
@@ -338,7 +289,7 @@ def gemm_pieces(a, w, ws: Optional[KernelWorkspace]) -> Optional[Partials]:
         # a prompt portion of a few hundred tokens has too few tiles for the chip: split k there
         # too, the consumer adds the pieces
         splits = _tile_splits(M, N, K)
-        if splits <= 1 or _tile_plan_us(M, N, K, splits) > PIECES_WORTH * _tile_plan_us(M, N, K, 1):
+        if splits <= 1 or _tile_splits_of(M, N, K, compute_units(), PIECES_WORTH) <= 1:
             return None
         p = _tiles_in_pieces(a, w, M, N, K, lda, ldw, splits, ws)
         return p if p.splits > 1 else None
