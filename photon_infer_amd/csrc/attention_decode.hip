@@ -8,7 +8,8 @@
 // merge in LDS, in wave order: where a step's requests nearly fill the chip by themselves, two to four
 // such waves take the place of ranges and their merging kernel, and requests of unlike length hold up
 // the step less, as a wave alone streams some 11 GB/s (32 heads and 8 kv heads of 64: 64 requests of 2,000
-// to 4,000 keys 87.7 -> 79.9 us, 4.9 -> 5.4 TB/s; 24 of 1,000 to 2,000 23.1 + 4.6 -> 23.7 us).
+// to 4,000 keys 83 -> 76 us; 24 of 1,000 to 2,000 23.1 + 4.6 -> 23.7 us).  Requests of one length lose by
+// it (64 of 4,096 keys: 96.5 -> 99.5 us), so the second waves leave at once where the step says so (97 us).
 //
 // For the query at position p = kv_len - 1: keys lo..p with lo = max(0, p - window + 1)
 // (window 0: all keys), or the start of p's chunk where positions are cut into chunks.  Ranges are cut at multiples of 32 keys.
@@ -180,7 +181,8 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(HD <
     const bf16_t* k_cache, const bf16_t* v_cache,   // not restrict: the fused kernel stores into them
     const int* __restrict__ block_table,
     int table_width, const int* __restrict__ q_start, const int* __restrict__ kv_len_of, const int* __restrict__ req_ids,
-    int nh, int nkv, int page_size, float scale, int window, long num_pages, float* __restrict__ part, AttnOptions opt) {
+    int nh, int nkv, int page_size, float scale, int window, long num_pages, float* __restrict__ part,
+    const int* __restrict__ uneven, AttnOptions opt) {
   const int lane = threadIdx.x % 64, lr = lane % 16, lg = lane / 16;
   const int wave = WAVES > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / 64) : 0;
   const int split = blockIdx.x, splits = gridDim.x, g = blockIdx.y;
@@ -210,8 +212,13 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(HD <
   const int first_place = OPT && kept > 0 ? 0 : first_chunk;
   const int last_chunk = p / 32 - gap;             // as a place
   const int chunks = last_chunk - first_place + 1;
-  const int per = (chunks + splits * WAVES - 1) / (splits * WAVES);
-  const int c0 = first_place + (split * WAVES + wave) * per;
+  int sharing = WAVES;                             // waves that take part
+  if (WAVES > 1 && uneven && *uneven == 0) {
+    if (wave > 0) return;                          // in every block of the launch: nobody waits for these waves
+    sharing = 1;
+  }
+  const int per = (chunks + splits * sharing - 1) / (splits * sharing);
+  const int c0 = first_place + (split * sharing + wave) * per;
   const int c1 = min(last_chunk + 1, c0 + per);
   // The wave whose keys end at the new token writes that token into the cache first and waits
   // for the stores; after that it reads the token like any other key, in the same order of
@@ -234,10 +241,10 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(HD <
                      }
                    }, kept, gap);
   attn_finish(st);
-  if constexpr (WAVES > 1) {
+  if (WAVES > 1 && sharing > 1) {
     // the waves' states meet in the first one; a wave without keys (m = -inf) weighs nothing
-    __shared__ f32x4_t outs[WAVES - 1][HD / 16][64];
-    __shared__ float2 sums[WAVES - 1][16];
+    __shared__ f32x4_t outs[WAVES > 1 ? WAVES - 1 : 1][HD / 16][64];
+    __shared__ float2 sums[WAVES > 1 ? WAVES - 1 : 1][16];
     if (wave > 0) {
 #pragma unroll
       for (int db = 0; db < HD / 16; ++db) outs[wave - 1][db][lane] = st.o[db][0];
@@ -390,12 +397,13 @@ static int launch_combine(void* out, long out_stride, const int* q_start, const 
 }
 
 // part: float32 [R * nh * splits * (hd + 4)], needed when splits > 1.
+// waves: of a block, on one range; uneven: null, or on the device 0 if only the first of them is to work after all.
 // req_ids: null (requests 0 .. R-1) or the R requests of the step that this launch serves; each
 // has one query token, at row q_start[r], that sees kv_len[r] keys.
 static int launch_decode(bool fused, const DecodeSource& src, void* out, long out_stride, const void* q, long q_stride,
                          const void* k_cache, const void* v_cache, const int* block_table, int table_width,
                          const int* q_start, const int* kv_len, const int* req_ids, int R, int nh, int nkv, int hd,
-                         int page_size, float scale, int window, long num_pages, int splits, int waves, void* part, long part_elems,
+                         int page_size, float scale, int window, long num_pages, int splits, int waves, const int* uneven, void* part, long part_elems,
                          bool merge, hipStream_t stream, AttnOptions opt = AttnOptions{nullptr, nullptr, nullptr}) {
   const bool with_options = opt.any();
   PI_REQUIRE(!with_options || (!fused && merge && scale > 0.f), "attention_decode: heads with options take the separate kernels, merged here, and a positive scale");
@@ -413,7 +421,7 @@ static int launch_decode(bool fused, const DecodeSource& src, void* out, long ou
   const dim3 grid(splits, nkv, R), block(64 * waves);
 #define GO_W(H, F, O, WV) hipLaunchKernelGGL((attention_decode_kernel<H, F, O, WV>), grid, block, 0, stream, (bf16_t*)out, out_stride, (const bf16_t*)q, \
                                     q_stride, src, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_table, table_width, q_start, \
-                                    kv_len, req_ids, nh, nkv, page_size, scale, window, num_pages, (float*)part, opt)
+                                    kv_len, req_ids, nh, nkv, page_size, scale, window, num_pages, (float*)part, uneven, opt)
 #define GO_F(H, F, O) do { if (waves == 1) GO_W(H, F, O, 1); else if (waves == 2) GO_W(H, F, O, 2); else GO_W(H, F, O, 4); } while (0)
 #define GO(H, F) GO_F(H, F, false)
 #define GO_OPT(H) GO_F(H, false, true)
@@ -470,13 +478,13 @@ static int launch_decode(bool fused, const DecodeSource& src, void* out, long ou
 extern "C" int pi_attention_decode(void* out, long out_stride, const void* q, long q_stride, const void* k_cache,
                                    const void* v_cache, const int* block_table, int table_width, const int* q_start,
                                    const int* kv_len, const int* req_ids, int R, int nh, int nkv, int hd, int page_size,
-                                   float scale, int window, long num_pages, int splits, int waves, void* part, long part_elems,
+                                   float scale, int window, long num_pages, int splits, int waves, const int* uneven, void* part, long part_elems,
                                    const float* slopes, const float* sinks, const float* gate, long gate_stride, float softcap,
                                    float out_mult, int chunk, int keep, hipStream_t stream) {
   PI_REQUIRE(chunk >= 0 && keep >= 0, "attention_decode: chunk and kept first keys must be >= 0, got %d and %d", chunk, keep);
   PI_REQUIRE(gate_stride == 0 || (gate && gate_stride % 4 == 0 && (uintptr_t)gate % 16 == 0), "attention_decode: gates per feature must lie in 16-byte groups");
   return launch_decode(false, DecodeSource{}, out, out_stride, q, q_stride, k_cache, v_cache, block_table, table_width, q_start,
-                       kv_len, req_ids, R, nh, nkv, hd, page_size, scale, window, num_pages, splits, waves, part, part_elems, true, stream,
+                       kv_len, req_ids, R, nh, nkv, hd, page_size, scale, window, num_pages, splits, waves, uneven, part, part_elems, true, stream,
                        AttnOptions{slopes, sinks, gate, softcap, out_mult, gate_stride, chunk, keep});
 }
 
@@ -491,7 +499,7 @@ extern "C" int pi_attention_decode_fused(void* out, long out_stride, const void*
                                          int qkv_splits, int ncols, int T, const float* table, int write_kv, void* k_cache,
                                          void* v_cache, const int* block_table, int table_width, const int* q_start,
                                          const int* kv_len, int R, int nh, int nkv, int hd, int page_size, float scale,
-                                         int window, long num_pages, int splits, int waves, void* part, long part_elems,
+                                         int window, long num_pages, int splits, int waves, const int* uneven, void* part, long part_elems,
                                          int merge, hipStream_t stream) {
   PI_REQUIRE((qkv != nullptr) != (qkv_part != nullptr), "attention_decode_fused: give the projection as a tensor or as pieces");
   PI_REQUIRE(T == R, "attention_decode_fused: %d tokens for %d requests (single tokens only)", T, R);
@@ -520,7 +528,7 @@ extern "C" int pi_attention_decode_fused(void* out, long out_stride, const void*
   src.k_cache = (bf16_t*)k_cache;
   src.v_cache = (bf16_t*)v_cache;
   return launch_decode(true, src, out, out_stride, nullptr, 0, k_cache, v_cache, block_table, table_width, q_start, kv_len,
-                       nullptr, R, nh, nkv, hd, page_size, scale, window, num_pages, splits, waves, part, part_elems, merge != 0, stream);
+                       nullptr, R, nh, nkv, hd, page_size, scale, window, num_pages, splits, waves, uneven, part, part_elems, merge != 0, stream);
 }
 
 // Merge partial results that the tile kernel wrote for `Z` tokens whose tiles' keys were cut in

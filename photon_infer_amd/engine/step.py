@@ -285,6 +285,7 @@ class ModelRunner:
         parts = {
             "token_ids": token_ids, "positions": positions, "req_of_token": req_of_token, "q_start": q_start,
             "kv_len": np.asarray(kv_lens, np.int32), "slots": np.asarray(slots, np.int32), "logit_rows": logit_rows,
+            "uneven": np.asarray([ops.lengths_uneven(kv_lens)], np.int32),
         }
         for g in range(len(cache.groups)):
             parts[f"table{g}"] = np.ascontiguousarray(cache.table_rows(g, slots, width)).reshape(-1)
@@ -301,7 +302,7 @@ class ModelRunner:
             token_ids=views["token_ids"], positions=views["positions"], req_of_token=views["req_of_token"],
             q_start=views["q_start"], kv_len=views["kv_len"], slots=views["slots"],
             block_tables={g: views[f"table{g}"].view(R, width) for g in range(len(cache.groups))},
-            logit_rows=views["logit_rows"],
+            logit_rows=views["logit_rows"], uneven=views["uneven"],
             q_lens=q_lens, kv_lens=kv_lens, max_q_len=max(q_lens), max_kv_len=max(kv_lens),
             all_decode=all(n == 1 for n in q_lens), host_slots=slots, workspace=self.workspace,
         )
@@ -430,6 +431,8 @@ class _DecodeGraph:
             total += (R + 3) // 4 * 4
         self.off["q_start"] = (total, R + 1)
         total += (R + 1 + 3) // 4 * 4
+        self.off["uneven"] = (total, 1)
+        total += 4
         for g in range(G):
             self.off[f"table{g}"] = (total, R * self.width)
             total += (R * self.width + 3) // 4 * 4
@@ -453,7 +456,7 @@ class _DecodeGraph:
             T=R, R=R, dtype=runner.dtype, token_ids=d["token_ids"], positions=d["positions"],
             req_of_token=d["req_of_token"], q_start=d["q_start"], kv_len=d["kv_len"], slots=d["slots"],
             block_tables={g: d[f"table{g}"].view(R, self.width) for g in range(G)}, logit_rows=d["logit_rows"],
-            q_lens=[1] * R, kv_lens=(), max_q_len=1, max_kv_len=length_bucket, all_decode=True,
+            uneven=d["uneven"], q_lens=[1] * R, kv_lens=(), max_q_len=1, max_kv_len=length_bucket, all_decode=True,
             workspace=runner.workspace)
         self.feed_rows = d["feed_rows"]
         self.temps = d["temps"].view(torch.float32)
@@ -473,6 +476,7 @@ class _DecodeGraph:
             self.h["feed_rows"][:] = feed[1]
         self.h["positions"][:] = lengths
         self.h["kv_len"][:] = lengths + 1
+        self.h["uneven"][0] = ops.lengths_uneven(self.h["kv_len"])
         self.h["slots"][:] = slots
         self.hf["temps"][:] = temperatures
         self.hf["uniforms"][:] = uniforms

@@ -551,6 +551,12 @@ def sample(out: torch.Tensor, logits: torch.Tensor, temperature: Optional[torch.
 
 
 # ----------------------------------------------------------------------------- work lists
+def lengths_uneven(kv_lens) -> bool:
+    """What a step's ``uneven`` says of its requests' context lengths (see ``fast.lengths_uneven``)."""
+    from . import fast
+    return fast.lengths_uneven(kv_lens)
+
+
 def decode_length_bucket(max_kv_len: int) -> int:
     """The context-length bucket that decides a decode step's attention key ranges."""
     from . import fast

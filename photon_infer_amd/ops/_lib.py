@@ -73,8 +73,8 @@ _SIGNATURES = {
         "pi_attention_tile_rows": [I, I, I],
         "pi_attention_prefill_mfma": [P, L, P, L, P, P, P, I, P, P, P, P, P, P, P, P, I, I, I, I, I, I, F, I, L, P, P, P, L, F, F, I, I, P],
         "pi_attention_combine_rows": [P, L, P, I, P, I, I, I, P, P, L, F, P],
-        "pi_attention_decode": [P, L, P, L, P, P, P, I, P, P, P, I, I, I, I, I, F, I, L, I, I, P, L, P, P, P, L, F, F, I, I, P],
-        "pi_attention_decode_fused": [P, L, P, L, P, I, I, I, P, I, P, P, P, I, P, P, I, I, I, I, I, F, I, L, I, I, P, L, I, P],
+        "pi_attention_decode": [P, L, P, L, P, P, P, I, P, P, P, I, I, I, I, I, F, I, L, I, I, P, P, L, P, P, P, L, F, F, I, I, P],
+        "pi_attention_decode_fused": [P, L, P, L, P, I, I, I, P, I, P, P, P, I, P, P, I, I, I, I, I, F, I, L, I, I, P, P, L, I, P],
         "pi_gemm_skinny_ranges": [P, I, L, P, I, I, I, P, L, I, I, I, P, L, P, I, P],
     },
 }

@@ -43,11 +43,15 @@ FUSED_DECODE_HEAD_DIMS = (64, 128)                 # ... and of its form that st
 MAX_DECODE_SPLITS = 64         # the combine kernel holds one key range per lane
 DECODE_WAVES_PER_UNIT = 2      # waves of the decode attention kernel per compute unit that fill the chip (measured at batch 1 to 64: more is never faster)
 DECODE_MIN_KEYS_PER_SPLIT = 128
-# Waves that share a block's keys: only where the blocks fill their rounds over the units this far (320 blocks of a design with
-# capped scores, 1.25 rounds: a step of 783 us took 796) and, without ranges to replace, for contexts longer than this
-# (64 requests of 300 keys: 1,325 -> 1,336 us; of 600: 1,400 -> 1,384; of 4,000 down to 2,000: 2,450 -> 2,331; of 4,096 each,
-# with nothing to even out: 2,530 -> 2,570)
-DECODE_WAVES_FILL, DECODE_WAVES_MIN_KEYS = 0.75, 512
+# Waves that share a block's keys, against ranges with their merging kernel or one wave (lists of attention times, 32 heads, 8 kv
+# heads, 600 to 4,096 keys each).  Blocks have to fill their rounds over the units this far: 384 of them, 1.5 rounds, at 4,096
+# keys 75.7 -> 81.0 us (up to 1,024 keys 23.8 -> 21.4), 320 at head size 128 126 -> 140; 192, three quarters of one round,
+# 38.6 -> 33.7.  Without ranges to replace only at two rounds (three, head size 128: 278 -> 296 at 4,096 keys, 42 -> 46 at 600),
+# from contexts on that are longer than so many keys per 64 features (64 requests of 600 at head size 128 29.8 -> 30.2), and
+# for lengths that are uneven: 64 requests of 2,000 to 4,000 keys 83 -> 76, of 4,096 each 96.5 -> 99.5 and with the second
+# waves gone at once 97.  From 10 % between the longest and the mean on the waves gain.
+DECODE_WAVES_FILL, DECODE_WAVES_FILL_LONG, DECODE_WAVES_LONG, DECODE_WAVES_MIN_KEYS = 0.75, 0.8, 1024, 512
+UNEVEN = 1.1                   # longest context over the mean from which a step's lengths are uneven
 
 
 def _stream() -> int:
@@ -454,11 +458,12 @@ class AttentionPlanner:
                   "singles": np.asarray(singles, np.int32)}
         z, rounds = len(rows), order.shape[0]
         longest_single = max((kv_lens[r] for r in singles), default=0)
+        singles_uneven = lengths_uneven([kv_lens[r] for r in singles])
 
         def finish(views: Dict[str, torch.Tensor]) -> "TilePlan":
             return TilePlan(req=views["req"], q0=views["q0"], cut=views["cut"], z0=views["z0"], rows=views["rows"],
                             cut_tokens=z, cuts=cuts if z else 1, order=views["order"], rounds=rounds, seats=seats,
-                            singles=singles, single_ids=views["singles"], longest_single=longest_single)
+                            singles=singles, single_ids=views["singles"], longest_single=longest_single, singles_uneven=singles_uneven)
 
         return arrays, finish
 
@@ -522,6 +527,7 @@ class TilePlan:
     singles: Tuple[int, ...] = ()             # requests that bring one token beside requests that bring more
     single_ids: Optional[torch.Tensor] = None  # the same on the device
     longest_single: int = 0                   # the longest context among them
+    singles_uneven: bool = False              # their contexts are uneven (lengths_uneven)
 
 
 MAX_TILE_CUTS = 8
@@ -564,17 +570,42 @@ def decode_splits(R: int, num_kv_heads: int, max_kv_len: int) -> int:
     return min(splits, max(1, decode_length_bucket(max_kv_len) // DECODE_MIN_KEYS_PER_SPLIT))
 
 
-def decode_block_waves(splits: int, R: int, num_kv_heads: int, max_kv_len: int) -> int:
+def decode_block_waves(splits: int, R: int, num_kv_heads: int, max_kv_len: int, head_dim: int = 64) -> int:
     """Waves per block of the decode attention, which share a request's keys of one kv head and merge in the block: they take
-    the place of ``splits`` ranges (more than 1: one range then, and no merging kernel), or 1.  Steps whose ranges the next
+    the place of ``splits`` ranges (more than 1: one range then, and no merging kernel), or 1.  Where there are no ranges to
+    replace they are worth it for lengths that are uneven only (``_uneven_lengths``).  Steps whose ranges the next
     product may merge keep them."""
-    blocks = R * num_kv_heads
+    blocks, bucket = R * num_kv_heads, decode_length_bucket(max_kv_len)
     rounds = -(-blocks // compute_units())
-    if R <= RANGES_MAX_TOKENS or splits > 4 or blocks < DECODE_WAVES_FILL * rounds * compute_units():
+    fill = DECODE_WAVES_FILL_LONG if rounds > 1 and bucket > DECODE_WAVES_LONG else DECODE_WAVES_FILL
+    if R <= RANGES_MAX_TOKENS or splits > 4 or blocks < fill * rounds * compute_units():
         return 1
     if splits > 1:
         return 2 if splits == 2 else 4
-    return 2 if rounds < 4 and decode_length_bucket(max_kv_len) > DECODE_WAVES_MIN_KEYS else 1
+    return 2 if rounds < 3 and bucket > DECODE_WAVES_MIN_KEYS * max(1, head_dim // 64) else 1
+
+
+def lengths_uneven(kv_lens) -> bool:
+    """Whether a step's contexts differ enough for waves that share one: the longest against the mean."""
+    if len(kv_lens) <= RANGES_MAX_TOKENS:
+        return False
+    lens = np.asarray(kv_lens)
+    return int(lens.max()) * len(lens) > UNEVEN * int(lens.sum())
+
+
+def _waves_or_ranges(ctx, splits: int, R: int, num_kv_heads: int, head_dim: int, longest: int, bound: int, plan=None) -> Tuple[int, int, Optional[int]]:
+    """(ranges, waves, where the device reads whether the waves are to share at all) of a decode attention; ``bound`` > 0: a
+    token sees so many keys at most; ``plan``: the requests are the single tokens of a step with portions, which the host knows."""
+    bounded = 0 < bound < decode_length_bucket(longest)
+    waves = decode_block_waves(splits, R, num_kv_heads, min(longest, bound) if bounded else longest, head_dim)
+    if waves == 1 or splits > 1:
+        return (1, waves, None) if waves > 1 else (splits, 1, None)
+    if bounded:                                       # the contexts' lengths do not say how many keys are seen
+        return 1, 1, None
+    if plan is not None:
+        return 1, waves if plan.singles_uneven else 1, None
+    flag = getattr(ctx, "uneven", None)
+    return (1, 1, None) if flag is None else (1, waves, flag.data_ptr())
 
 
 def _attn_part(ws: Optional[KernelWorkspace], floats: int, device) -> torch.Tensor:
@@ -603,18 +634,16 @@ def paged_attention(out, q, k_cache, v_cache, block_table, ctx, num_heads, num_k
     G = num_heads // num_kv_heads
     R = ctx.R
 
-    def decode_kernel(n_req: int, req_ids: int, longest: int) -> None:
-        if chunk:                      # a token's keys end at its chunk's start, whatever the context
-            longest = min(longest, chunk + keep)
-        splits = _decode_splits_that_fit(ws, n_req, num_heads, num_kv_heads, head_dim, longest)
-        waves = decode_block_waves(splits, n_req, num_kv_heads, min(longest, window) if window else longest)
-        if waves > 1:
-            splits = 1
+    def decode_kernel(n_req: int, req_ids: int, longest: int, plan=None) -> None:
+        # (a token's keys end at its chunk's start, whatever the context)
+        splits = _decode_splits_that_fit(ws, n_req, num_heads, num_kv_heads, head_dim, min(longest, chunk + keep) if chunk else longest)
+        bound = min(window or 1 << 30, chunk + keep if chunk else 1 << 30) if window or chunk else 0
+        splits, waves, uneven = _waves_or_ranges(ctx, splits, n_req, num_kv_heads, head_dim, longest, bound, plan)
         part = _attn_part(ws, n_req * num_heads * splits * (head_dim + 4), q.device)
         _lib.call("bf16", "pi_attention_decode", out.data_ptr(), out.stride(0), q.data_ptr(), q.stride(0),
                   k_cache.data_ptr(), v_cache.data_ptr(), block_table.data_ptr(), block_table.shape[1],
                   ctx.q_start.data_ptr(), ctx.kv_len.data_ptr(), req_ids, n_req, num_heads, num_kv_heads, head_dim,
-                  page_size, float(scale), int(window), pages, splits, waves, part.data_ptr(), part.numel(), *opt, _stream())
+                  page_size, float(scale), int(window), pages, splits, waves, uneven, part.data_ptr(), part.numel(), *opt, _stream())
 
     if ctx.all_decode and G <= 16:
         decode_kernel(R, 0, ctx.max_kv_len)
@@ -627,7 +656,7 @@ def paged_attention(out, q, k_cache, v_cache, block_table, ctx, num_heads, num_k
     # context in one block, mostly on padding); the portions go to the tile kernel.
     plan = _tile_plan(ctx, planner, q.device)
     if plan.singles:
-        decode_kernel(len(plan.singles), plan.single_ids.data_ptr(), plan.longest_single)
+        decode_kernel(len(plan.singles), plan.single_ids.data_ptr(), plan.longest_single, plan)
     floats = plan.cut_tokens * num_heads * plan.cuts * (head_dim + 4)
     tile_part = ws.tile_part_for(floats) if ws is not None else torch.empty(max(4, floats), dtype=torch.float32, device=q.device)
     _lib.call("bf16", "pi_attention_prefill_mfma", out.data_ptr(), out.stride(0), q.data_ptr(), q.stride(0),
@@ -717,16 +746,16 @@ def decode_attention_from_projection(out, qkv, ctx, table, num_heads, num_kv_hea
         return False
     splits = _decode_splits_that_fit(ws, R, num_heads, num_kv_heads, head_dim, ctx.max_kv_len)
     leave = leave_ranges > 0 and ws is not None and splits > 1 and ranges_product_ok(R, head_dim, leave_ranges)
-    waves = 1 if leave else decode_block_waves(splits, R, num_kv_heads, min(ctx.max_kv_len, window) if window else ctx.max_kv_len)
-    if waves > 1:
-        splits = 1
+    waves, uneven = 1, None
+    if not leave:
+        splits, waves, uneven = _waves_or_ranges(ctx, splits, R, num_kv_heads, head_dim, ctx.max_kv_len, window)
     part = _attn_part(ws, R * num_heads * splits * (head_dim + 4), out.device)
     _lib.call("bf16", "pi_attention_decode_fused", out.data_ptr(), out.stride(0),
               None if pieces else qkv.data_ptr(), 0 if pieces else qkv.stride(0),
               qkv.part.data_ptr() if pieces else None, qkv.splits if pieces else 0, qkv.N if pieces else 0, R,
               None if table is None else table.data_ptr(), int(bool(write_kv)), k_cache.data_ptr(), v_cache.data_ptr(),
               block_table.data_ptr(), block_table.shape[1], ctx.q_start.data_ptr(), ctx.kv_len.data_ptr(), R, num_heads,
-              num_kv_heads, head_dim, page_size, float(scale), int(window), pages, splits, waves, part.data_ptr(),
+              num_kv_heads, head_dim, page_size, float(scale), int(window), pages, splits, waves, uneven, part.data_ptr(),
               part.numel(), int(not leave), _stream())
     if leave:
         return KeyRanges(part, splits, R, num_heads, head_dim, ctx.q_start)

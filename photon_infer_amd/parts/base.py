@@ -109,6 +109,7 @@ class StepContext:
     slots: torch.Tensor                   # [R] per-request state slot
     block_tables: Dict[int, torch.Tensor]  # cache group -> [R, width] page ids (-1 = none)
     logit_rows: torch.Tensor              # [M] token rows whose logits are wanted
+    uneven: Optional[torch.Tensor] = None  # [1] 1: the requests' lengths are uneven (ops.lengths_uneven); None: nobody says
     # host-side copies for launch planning (never read by kernels)
     q_lens: Sequence[int] = ()
     kv_lens: Sequence[int] = ()

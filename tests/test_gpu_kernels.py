@@ -850,6 +850,40 @@ def test_decode_attention_by_the_waves_of_a_block(_ops, monkeypatch, waves, hd, 
     assert torch.equal(k, paged.k) and torch.equal(v, paged.v) and torch.equal(fused, got)
 
 
+@pytest.mark.parametrize("hd,nh,nkv", [(64, 16, 8), (128, 8, 8)])
+def test_waves_share_a_request_only_when_the_step_says_its_lengths_are_uneven(_ops, hd, nh, nkv):
+    """64 requests of 8 kv heads, 33 to 1,100 keys: with the step's word for even lengths, and in a step that does not say, the
+    bits are those of one wave per request; with its word for uneven ones those of two.  The word is read when the kernel runs,
+    so a captured launch follows it."""
+    from photon_infer_amd.ops import fast
+    R, page, scale = 64, 16, hd ** -0.5
+    kv_lens = [1100 - 17 * i for i in range(R - 1)] + [33]
+    g = gen(hd)
+    paged = PagedKV([(torch.randn(n, nkv, hd, generator=g), torch.randn(n, nkv, hd, generator=g)) for n in kv_lens], page, BF16, seed=hd)
+    ctx, q = attention_ctx([1] * R, kv_lens, BF16), torch.randn(R, nh * hd, generator=g).to(BF16).to(DEV)
+
+    def run(out):
+        _ops.paged_attention(out, q, paged.k, paged.v, paged.table, ctx, nh, nkv, hd, page, scale)
+        return out
+
+    one = run(torch.empty_like(q))                        # nobody says
+    flag = ctx.uneven = torch.zeros(1, dtype=torch.int32, device=DEV)
+    assert fast.decode_splits(R, nkv, ctx.max_kv_len) == 1 and fast.decode_block_waves(1, R, nkv, ctx.max_kv_len, hd) == 2
+    assert torch.equal(run(torch.empty_like(q)), one)
+    flag.fill_(1)
+    two = run(torch.empty_like(q))
+    close(two, one.float().cpu(), 2 ** -7, "two waves")
+    out, graph = torch.empty_like(q), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        run(out)
+    for value, want in ((1, two), (0, one), (1, two)):
+        flag.fill_(value)
+        graph.replay()
+        assert torch.equal(out, want)
+    assert not torch.equal(one, two)
+
+
 @pytest.mark.parametrize("dtype", [F32, BF16])
 @pytest.mark.parametrize("fast", [False, True])
 def test_attention_finds_one_far_key_among_hundreds(_ops, dtype, fast):

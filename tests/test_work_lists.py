@@ -160,3 +160,40 @@ def test_a_token_count_that_was_not_seen_before_costs_little_to_plan(monkeypatch
                 fast._tile_shape(M, N, K, fast._tile_splits(M, N, K))
         best = min(best, (time.perf_counter() - start) / 20)
     assert best < 60e-6
+
+
+# (key ranges, requests, kv heads, longest context, head size) -> waves per block, as measured: a step of contexts of one length
+# must lose nothing, so waves that replace no ranges go to two full rounds of blocks only (and, on the device, to uneven lengths)
+@pytest.mark.parametrize("splits,R,kv_heads,longest,head_dim,waves", [
+    (1, 64, 8, 4000, 64, 2), (1, 64, 8, 4000, 128, 2), (1, 128, 4, 4000, 64, 2), (1, 64, 8, 1000, 64, 2), (1, 64, 8, 1000, 128, 1), (1, 64, 8, 300, 64, 1),
+    (1, 80, 8, 4096, 64, 1), (1, 96, 8, 4096, 128, 1), (1, 96, 8, 600, 128, 1), (1, 128, 8, 4096, 64, 1), (2, 48, 8, 4096, 64, 1), (2, 48, 8, 1024, 64, 2),
+    (2, 32, 8, 4096, 128, 2), (2, 56, 8, 4096, 64, 2), (3, 24, 8, 4096, 64, 4), (2, 40, 8, 4096, 64, 1), (4, 16, 8, 4096, 64, 1)])
+def test_waves_share_a_request_where_that_was_the_faster_way(splits, R, kv_heads, longest, head_dim, waves):
+    from photon_infer_amd.ops import fast
+    assert fast.decode_block_waves(splits, R, kv_heads, longest, head_dim) == waves
+
+
+def test_uneven_lengths():
+    from photon_infer_amd.ops import lengths_uneven
+    assert not lengths_uneven([4096] * 64) and not lengths_uneven([4000 - 10 * i for i in range(64)])
+    assert lengths_uneven([4000 - 30 * i for i in range(64)]) and lengths_uneven(np.asarray([500] * 63 + [4000], np.int32))
+    assert not lengths_uneven([1, 4000])             # a small batch: its ranges may go on to the next product
+
+
+def test_waves_of_bounded_contexts_and_of_steps_that_do_not_know_their_lengths():
+    """Windows and chunks: the lengths do not say what is seen.  The answer is the same for a step and for its length bucket's graph."""
+    from types import SimpleNamespace
+
+    import torch
+
+    from photon_infer_amd.ops import fast
+    flag = torch.zeros(1, dtype=torch.int32)
+    ctx, bare = SimpleNamespace(uneven=flag), SimpleNamespace()
+    assert fast._waves_or_ranges(ctx, 1, 64, 8, 64, 3000, 0) == (1, 2, flag.data_ptr())
+    assert fast._waves_or_ranges(bare, 1, 64, 8, 64, 3000, 0) == (1, 1, None)
+    for bound in (1024, 2500, 3500):
+        assert fast._waves_or_ranges(ctx, 1, 64, 8, 64, 3000, bound) == fast._waves_or_ranges(ctx, 1, 64, 8, 64, 4096, bound) == (1, 1, None)
+    assert fast._waves_or_ranges(ctx, 1, 64, 8, 64, 3000, 4096) == (1, 2, flag.data_ptr())
+    assert fast._waves_or_ranges(bare, 2, 32, 8, 64, 3000, 0) == (1, 2, None) and fast._waves_or_ranges(ctx, 2, 40, 8, 64, 3000, 0) == (2, 1, None)
+    for uneven in (False, True):
+        assert fast._waves_or_ranges(ctx, 1, 64, 8, 64, 3000, 0, SimpleNamespace(singles_uneven=uneven)) == (1, 1 + uneven, None)
