@@ -212,10 +212,18 @@ def _float32_ok(a, w, K, lda, ldw) -> bool:
             and max(lda, ldw) < FLOAT32_MAX_STRIDE)
 
 
+def _general_streams_faster(M: int, N: int, K: int) -> bool:
+    """Products of so few rows that the vector unit keeps up with the memory: the general kernel's form for them then streams the
+    weights faster.  One or two rows from k = 512 on (N x K, one row, general and matrix-core kernel: 2,048 x 2,048 8.0 and 9.5 us,
+    512 x 2,048 6.7 and 9.4, 16,384 x 4,096 50 and 68, 16,384 x 2,048 27.7 and 28.3; 4,096 x 256 6.6 and 4.6); up to eight rows of
+    long k in a matrix of many rows (four rows of 8,192 x 8,192 68 and 80, of 8,192 x 4,096 39 and 32)."""
+    return (M <= 2 and K > 512) or (M <= 8 and K >= 8192 and N >= 8192)
+
+
 def gemm_float32(out, a, w, accumulate, M, N, K, lda, ldw, ldc, ws: Optional[KernelWorkspace] = None) -> bool:
     """out (+)= a @ w^T, all float32, by the float32 matrix-core kernels; what a product of few tiles leaves in pieces is
     added at once."""
-    if not _float32_ok(a, w, K, lda, ldw):
+    if not _float32_ok(a, w, K, lda, ldw) or _general_streams_faster(M, N, K):
         return False
     made = _lib.load("core").pi_gemm_float32_pieces(M, N, K, GEMM_PART_FLOATS)
     buf = _piece_buffer(ws, made * M * N, a.device) if made > 1 else None

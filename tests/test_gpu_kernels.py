@@ -276,7 +276,9 @@ def test_float32_products_on_the_matrix_cores(_ops, M, N, K):
     a, w = a_full.to(DEV)[:, 4:K + 4], w_full.to(DEV)[:, :K]                  # rows that lie apart
     want = a.double() @ w.double().t()
     out_full = torch.zeros(M, N + 3, device=DEV)
-    _ops.gemm(out_full[:, 1:N + 1], a, w)
+    with library_calls() as names:
+        _ops.gemm(out_full[:, 1:N + 1], a, w)
+    assert names in (["pi_gemm_float32"], ["pi_gemm_float32", "pi_splitk_reduce"])
     close(out_full[:, 1:N + 1], want.cpu(), rel, f"float32 {M}x{N}x{K}")
     assert out_full[:, 0].abs().max() == 0 and out_full[:, N + 1:].abs().max() == 0
     base = torch.randn(M, N, generator=gen(9)).to(DEV)
@@ -285,8 +287,20 @@ def test_float32_products_on_the_matrix_cores(_ops, M, N, K):
         _ops.gemm(x, a, w, accumulate=True, ws=space)
         close(x, (want + base.double()).cpu(), rel, "float32 accumulate")
     odd = torch.empty(M, N, device=DEV)                                       # operands off 16 bytes: the general kernel
-    _ops.gemm(odd, a_full.to(DEV)[:, 1:K + 1], w)
+    with library_calls() as names:
+        _ops.gemm(odd, a_full.to(DEV)[:, 1:K + 1], w)
+    assert names == ["pi_gemm_general"]
     close(odd, (a_full[:, 1:K + 1].double() @ w.double().cpu().t()), rel, "float32, unaligned")
+
+
+@pytest.mark.parametrize("M,N,K,kernel", [(1, 2048, 2048, "pi_gemm_general"), (2, 520, 516, "pi_gemm_general"), (1, 2048, 512, "pi_gemm_float32"),
+                                          (3, 2048, 2048, "pi_gemm_float32"), (8, 8192, 8192, "pi_gemm_general"), (9, 8192, 8192, "pi_gemm_float32")])
+def test_few_float32_rows_go_to_the_kernel_that_streams_the_weights_faster(_ops, M, N, K, kernel):
+    a, w, out = torch.randn(M, K, generator=gen(M)).to(DEV), torch.randn(N, K, generator=gen(N)).to(DEV), torch.empty(M, N, device=DEV)
+    with library_calls() as names:
+        _ops.gemm(out, a, w)
+    assert names[0] == kernel
+    close(out, (a.double() @ w.double().t()).cpu(), 2 ** -24 * (4 + math.sqrt(K)), f"{M}x{N}x{K}")
 
 
 @pytest.mark.parametrize("M,I,K", [(1000, 6160, 200), (1000, 6160, 192), (2048, 8192, 64)])
