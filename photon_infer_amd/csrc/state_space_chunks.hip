@@ -17,6 +17,9 @@
 #include "token_tiles.h"
 
 #define CHUNK 64
+// A token's log decay from here on is complete forgetting: exp() of it, and of its sum with any other, is zero in 32 bits.  Taken
+// for what it is, a decay of -1e12 left the sums that follow it without the digits of theirs, one beyond 3.4e38 left NaN.
+#define LOG_DECAY_ALL (-200.0)
 #define XROW (CHUNK / 4 + 1)          // 16-byte pieces of a row of tokens in LDS: an odd number, rows fall on all banks
 
 __device__ inline float softplus_of(float v) { return v > 20.0f ? v : log1pf(expf(v)); }
@@ -29,7 +32,8 @@ struct ChunkDecay {
 __device__ inline ChunkDecay chunk_decay(const float* __restrict__ dt_raw, long dt_stride, float bias, float a_log, int tokens) {
   const int lane = threadIdx.x % PI_WAVE;
   const float dt = lane < tokens ? softplus_of(dt_raw[lane * dt_stride] + bias) : 0.f;
-  double g = -(double)expf(a_log) * (double)dt;
+  double g = lane < tokens ? -(double)expf(a_log) * (double)dt : 0.0;
+  g = g < LOG_DECAY_ALL ? LOG_DECAY_ALL : g;     // NaN stays NaN
 #pragma unroll
   for (int d = 1; d < PI_WAVE; d *= 2) {
     const double other = __shfl_up(g, d, PI_WAVE);

@@ -165,8 +165,31 @@ def test_state_space_recurrence_in_chunks(sizes):
     xbc, dt = dev32(data["a"][0]), dev32(data["a"][1])
     xbc[100, 1] = float("inf")                     # an input that is not finite: its column from its token on, nothing else
     y = torch.empty((333, H * Pd), device=DEV)
-    ops.state_space_scan(y, xbc, dt, dev32(dt_bias), dev32(A_log), dev32(D), state_ctx([333], [0]), torch.zeros((1, floats), device=DEV), H, Pd, N, G)
+    with library_calls() as names:
+        ops.state_space_scan(y, xbc, dt, dev32(dt_bias), dev32(A_log), dev32(D), state_ctx([333], [0]), torch.zeros((1, floats), device=DEV), H, Pd, N, G)
+    assert "pi_state_space_chunks" in names
     assert not bool(y[:, 1].isfinite()[100:].any()) and bool(y[:100].isfinite().all()) and bool(y[:, 0].isfinite().all()) and bool(y[:, 2:].isfinite().all())
+
+
+@pytest.mark.parametrize("a_log", [20.0, 60.0, 80.0, 90.0])
+def test_state_space_chunks_forget_at_once_and_remember_right_behind(a_log):
+    """Every other token wipes the state out - its log decay is -5e10, no 32-bit number, or infinite - and the tokens between
+    keep most of it: a sum of such decays must not swallow the small ones that follow."""
+    from photon_infer_amd import ops
+    H, Pd, N, G, T = 1, 64, 16, 1, 140
+    x, B, C = randn(T, H, Pd, seed=1), randn(T, G, N, seed=2, scale=0.5), randn(T, G, N, seed=3, scale=0.5)
+    dt = torch.full((T, H), 100.0 if a_log < 60 else 1e5, dtype=F64)
+    if a_log < 60:
+        dt[1::2] = -23.0                       # a step of 1e-10: a decay of 0.95
+    A_log, D, bias = torch.full((H,), a_log, dtype=F64), randn(H, seed=4), torch.zeros(H, dtype=F64)
+    want, last = P.state_space_recurrence(x, B, C, P.softplus(dt), A_log, D)
+    state, y = torch.ones((1, ops.scan_state_floats(H, N, Pd)), device=DEV), torch.empty((T, H * Pd), device=DEV)
+    xbc = dev32(torch.cat([x.reshape(T, -1), B.reshape(T, -1), C.reshape(T, -1)], dim=1))
+    with library_calls() as names:
+        ops.state_space_scan(y, xbc, dev32(dt), dev32(bias), dev32(A_log), dev32(D), state_ctx([T], [0]), state, H, Pd, N, G)
+    assert "pi_state_space_chunks" in names
+    close(y, want.reshape(T, -1), "outputs", 1e-5)
+    close(ops.unpack_scan_state(state[0], H, N, Pd), last, "state", 1e-5)
 
 
 @pytest.mark.parametrize("lengths_on_host", [True, False])
