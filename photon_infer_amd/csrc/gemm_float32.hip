@@ -1,6 +1,7 @@
 // float32 matrix products on the matrix cores: C[M, N] (+)= A[M, K] . W[N, K]^T with 32-bit operands, products and sums
 // (v_mfma_f32_32x32x2_f32 and v_mfma_f32_16x16x4_f32; 157 TFLOP/s on this chip, twice the vector unit's rate without
-// packed instructions).  They carry the float32 path's products; gemm_general.hip keeps mixed types and odd strides.
+// packed instructions).  They carry the float32 path's products; gemm_general.hip keeps mixed types, odd strides and the
+// products of a few rows that it streams faster (ops/fast.py).
 //
 // K and the row strides are multiples of 4 and the operands 16-byte aligned.  A row of 32 floats is 128 bytes, as a row
 // of 64 bfloat16 is, so both kernels move their operands exactly as the bfloat16 kernels do and share those kernels'
@@ -176,7 +177,8 @@ __device__ inline void block_barrier_keeping_loads() {
 // of NB buffers (rows of 128 bytes, their 16-byte pieces turned by (row / 2) % 8 as in gemm_mfma.hip).  A matrix
 // instruction takes 64 cycles for two registers of operands, so LDS and its reads have time to spare and the tile only
 // has to be large enough for L2: 32 / 21 / 16 flops per byte at 128 x 128 / 128 x 64 / 64 x 64.  What decides is how the
-// tiles fill the chip, see plan().  Every output is summed over k in the same order in every tile shape.
+// tiles fill the chip, see plan().  Every output is summed over k in the same order in every
+// tile shape; how many pieces k is cut into depends on the rows and columns, so a row's bits depend on what shares its launch.
 template <int TM, int TN, int NB, bool ACCUM>
 __global__ __launch_bounds__(256) void gemm_float32_tile_kernel(float* __restrict__ C, long ldc, const float* __restrict__ A, long lda,
                                                                 const float* __restrict__ W, long ldw, int M, int N, int K, int tiles_n,

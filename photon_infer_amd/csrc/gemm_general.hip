@@ -1,13 +1,15 @@
 // General matrix product C[M, N] (+)= A[M, K] . W[N, K]^T for any M, N, K and any mix of
 // float32 / bfloat16 operands, with float32 multiply-add throughout (no matrix cores, no
-// reduced-precision mode).  It is the whole-model float32 path and the fallback for sizes
-// the matrix-core kernels do not take.
+// reduced-precision mode).  It takes mixed types, odd strides and whatever else the matrix-core kernels
+// (gemm_mfma.hip, gemm_skinny.hip, gemm_float32.hip) do not, float32 products of so few rows that it is the
+// faster one (ops/fast.py), and every product when the fast kernels are switched off.
 //
 // Convention (include/photon/ops/kernels/matmul_kernel.hpp:54-129): activations
 // row-major [rows, in], weights row-major [out, in], y = x W^T, no bias.
 //
 // Each output element accumulates over k in ascending order, 16 at a time, so a row's
-// result does not depend on which other rows share the launch.
+// result does not depend on which other rows share the launch (the matrix-core kernels do not promise that:
+// there the number of rows decides the kernel and how k is cut).
 //
 // Up to 16 rows of activations (decode steps) take a second kernel that streams the weights:
 // a block owns a few weight rows, its waves take turns over k, their lanes four elements at a time (16-byte loads that

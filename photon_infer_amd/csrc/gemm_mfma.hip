@@ -514,7 +514,6 @@ __global__ __launch_bounds__(512) void gemm_mfma_big_kernel(void* __restrict__ C
     const int rows_left = (int)min((long)32 * WI, M - mw);                                                // may be <= 0
     float* patch = reinterpret_cast<float*>(lds) + wave * PATCH_FLOATS;
     const int esize = EPI_HALF(EPI) || EPI_GATED(EPI) ? 2 : 4;
-    if (EPI == EPI_GATE) glu.bias += mw * glu.gate_stride + n0 + wn * 32 * WJ;
 #pragma unroll
     for (int j = 0; j < WJ; j += 2) {
       const long nw = n0 + wn * 32 * WJ + j * 32;
@@ -525,7 +524,6 @@ __global__ __launch_bounds__(512) void gemm_mfma_big_kernel(void* __restrict__ C
       for (int i = 0; i < WI; ++i)
         store_rows32<EPI>(patch, acc[i][j], acc[i][j + 1 < WJ ? j + 1 : j], corner, (int)ldc, i * 32, rows_left,
                           j + 1 < WJ ? cols_left : min(32, cols_left), lane, wide, glu, nw);       // an odd last tile stands alone
-      if (EPI == EPI_GATE) glu.bias += 64;
     }
   }
 }

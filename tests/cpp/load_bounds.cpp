@@ -4,9 +4,10 @@
 //   load_bounds [old-standin] [only] [M N K splits]...
 //
 // Walks the built-in sweep of shapes (and any given as arguments) through the lanes, waves,
-// blocks and steps of gemm_skinny_kernel, gemm_skinny_shared_kernel, gemm_mfma_kernel and
-// gemm_mfma_big_kernel exactly as the kernels walk them (and, in the built-in sweep, through the
-// key and value fetches of the attention kernels' chunks for every head size and several page sizes), with the matrices row by row (two row
+// blocks and steps of gemm_skinny_kernel, gemm_skinny_shared_kernel, gemm_mfma_kernel,
+// gemm_mfma_big_kernel in its five tile shapes, gemm_float32_rows_kernel and gemm_float32_tile_kernel exactly as the kernels
+// walk them (and, in the built-in sweep, through the
+// key and value fetches of the attention kernels' chunks for every head size and several page sizes), with the matrices row by row (several row
 // strides) and, where the sizes allow, in the weight-streaming kernels' tiled order.  Prints
 // "ok <fetches>" or the first fetch that leaves its operand (exit status 1).
 // "only" leaves the built-in sweep out.  "old-standin" replaces the stand-in address of a lane beyond a partial k step by the formula
@@ -121,56 +122,109 @@ static bool shared(const Shape& s, long ldx, long ldw, int tiled, int depth) {
   return true;
 }
 
-// ------------------------------------------------------------------ tile kernels
-// One operand of one block: rows [row0, row0 + tile) of [R, K] with stride ld, k in [k_lo, k_hi).
-static bool tile_operand(const char* kernel, const char* operand, const Shape& s, long R, long ld, long row0, int tile, int waves,
-                         int k_lo, int k_hi, bool big) {
-  const int rows = (int)A::lmin(tile, R - row0);
-  const A::Descriptor d = A::tile_descriptor(row0, ld, k_lo, k_hi, rows);
-  const long operand_bytes = ((R - 1) * ld + s.K) * 2;
-  if (d.base < 0 || d.bytes <= 0 || d.base * 2 + d.bytes > operand_bytes || d.bytes >= 0x7ffffff0L)
-    return fail(kernel, operand, s, ld, 0, d.base, "the descriptor leaves the operand");
-  const int k_range = k_hi - k_lo, slabs = (k_range + 63) / 64;
-  for (int wave = 0; wave < waves; ++wave)
-    for (int p = 0; p < 4; ++p)
-      for (int lane = 0; lane < 64; ++lane) {
-        const int row = (wave * 4 + p) * 8 + lane / 8, piece = A::tile_piece(lane, row);
-        for (int sl = 0; sl < slabs + 2; ++sl) {       // the kernels ask for up to two slabs past the last
-          ++fetches;
-          long off;      // bytes inside the descriptor
-          bool used;
-          if (big) {
-            off = (long)A::big_lane_offset(row, rows, ld, piece) + A::big_slab_bytes(sl, slabs);
-            used = row < rows && sl < slabs;
-            if (off + 16 > d.bytes) return fail(kernel, operand, s, ld, 0, off, "a fetch of the large-tile kernel leaves its descriptor");
-          } else {
-            if (sl >= slabs) continue;                 // this kernel asks for existing slabs only
-            off = A::tile_slab_offset(A::tile_lane_offset(row, rows, ld, piece), sl * 64, piece, k_range);
-            used = row < rows && sl * 64 + piece * 8 < k_range;
-            if (!used && off < d.bytes) return fail(kernel, operand, s, ld, 0, off, "a fetch that should read zeros lies inside the descriptor");
-            if (used && off + 16 > d.bytes) return fail(kernel, operand, s, ld, 0, off, "a used fetch leaves its descriptor");
+// ------------------------------------------------------------------ 1..32 rows of float32, in units of two bytes
+static bool float32_rows(const Shape& s, long ldx, long ldw, int RT, int waves, int depth) {
+  const int M = s.M, N = s.N, K = s.K;
+  const A::KSplit cut = A::cut_k(K, s.splits, 32);
+  const int rows_per_block = RT * 16, MB = (M + 15) / 16;
+  const int x_loads = (M + 7) / 8;
+  for (int by = 0; by < cut.splits; ++by)
+    for (int bx = 0; bx < (N + rows_per_block - 1) / rows_per_block; ++bx)
+      for (int wave = 0; wave < waves; ++wave) {
+        const A::WaveRange r = A::wave_share(2 * by * cut.k_per_block, 2 * A::imin(K, (by + 1) * cut.k_per_block), waves, wave);
+        const int steps = r.k1 > r.k0 ? (r.k1 - r.k0 + A::KSTEP - 1) / A::KSTEP : 0;
+        if (steps == 0) continue;
+        for (int lane = 0; lane < 64; ++lane) {
+          const int lr = lane % 16, lg = lane / 16, xt = lane / 8, xp = lane % 8;
+          const long n0 = (long)bx * rows_per_block;
+          for (int st = 0; st < steps + depth; ++st) {   // the loads in flight run past the last step
+            const int kk = r.k0 + A::imin(st, steps - 1) * A::KSTEP;
+            for (int t = 0; t < RT; ++t)
+              for (int h = 0; h < 2; ++h) {
+                const long off = A::skinny_w_base(0, n0, t, lr, lg, N, 2 * K, 2 * ldw) + A::skinny_w_step(0, false, kk, h, lg, r.k0, r.k1);
+                const long row = A::lmin(n0 + t * 16 + lr, (long)N - 1);
+                ++fetches;
+                if (!in_row(off, row, 2 * ldw, 2 * K)) return fail("gemm_float32_rows", "W", s, ldw, 0, off, "outside its row");
+                if (A::skinny_w_used(false, kk, h, lg, r.k1) && off != row * 2 * ldw + kk + lg * 16 + h * 8)
+                  return fail("gemm_float32_rows", "W", s, ldw, 0, off, "a used fetch is not the lane's k");
+              }
+            for (int i = 0; i < MB * 2; ++i)
+              if (i == 0 || i < x_loads) {
+                const int token = i * 8 + xt;
+                const long off = A::skinny_x_base(token, M, 2 * ldx, xp) + A::skinny_x_step(false, kk, xp, r.k0, r.k1);
+                ++fetches;
+                if (!in_row(off, A::imin(token, M - 1), 2 * ldx, 2 * K)) return fail("gemm_float32_rows", "X", s, ldx, 0, off, "outside its row");
+              }
           }
-          if (used && d.base * 2 + off != ((row0 + row) * ld + k_lo + A::imin(sl, slabs - 1) * 64 + piece * 8) * 2)
-            return fail(kernel, operand, s, ld, 0, off, "a used fetch is not the lane's row and k");
         }
       }
   return true;
 }
 
-static bool tiles(const Shape& s, long lda, long ldw, bool big) {
-  const int tile = big ? 256 : 128, waves = big ? 8 : 4;
-  if (big && s.K % 64) return true;                    // the large-tile kernel takes whole slabs only
-  const A::KSplit cut = A::cut_k(s.K, s.splits, 64);
-  const char* kernel = big ? "gemm_mfma_big" : "gemm_mfma";
+// ------------------------------------------------------------------ tile kernels
+// A tile kernel's geometry: rows of its tiles of A and of W, waves, whether it is the larger-tile kernel, and the slabs it
+// asks for past the last.  A wave fills tile / (8 * waves) times eight rows of each per slab.
+struct Tiles {
+  const char* kernel;
+  int rows_a, rows_w, waves;
+  bool big;
+  int ahead;
+};
+
+// One operand of one block: rows [row0, row0 + tile) of [R, K] with stride ld, k in [k_lo, k_hi), in units of two bytes.
+static bool tile_operand(const Tiles& t, const char* operand, const Shape& s, long R, int K, long ld, long row0, int tile, int k_lo, int k_hi) {
+  const int rows = (int)A::lmin(tile, R - row0), loads = tile / (8 * t.waves);
+  const A::Descriptor d = A::tile_descriptor(row0, ld, k_lo, k_hi, rows);
+  const long operand_bytes = ((R - 1) * ld + K) * 2;
+  if (d.base < 0 || d.bytes <= 0 || d.base * 2 + d.bytes > operand_bytes || d.bytes >= 0x7ffffff0L)
+    return fail(t.kernel, operand, s, ld, 0, d.base, "the descriptor leaves the operand");
+  const int k_range = k_hi - k_lo, slabs = (k_range + 63) / 64;
+  for (int wave = 0; wave < t.waves; ++wave)
+    for (int p = 0; p < loads; ++p)
+      for (int lane = 0; lane < 64; ++lane) {
+        const int row = (wave * loads + p) * 8 + lane / 8, piece = A::tile_piece(lane, row);
+        for (int sl = 0; sl < slabs + t.ahead; ++sl) {
+          ++fetches;
+          long off;      // bytes inside the descriptor
+          bool used;
+          if (t.big) {
+            off = (long)A::big_lane_offset(row, rows, ld, piece) + A::big_slab_bytes(sl, slabs);
+            used = row < rows && sl < slabs;
+            if (off + 16 > d.bytes) return fail(t.kernel, operand, s, ld, 0, off, "a fetch of the larger tiles leaves its descriptor");
+          } else {
+            off = A::tile_slab_offset(A::tile_lane_offset(row, rows, ld, piece), sl * 64, piece, k_range);
+            used = row < rows && sl * 64 + piece * 8 < k_range;
+            if (!used && off < d.bytes) return fail(t.kernel, operand, s, ld, 0, off, "a fetch that should read zeros lies inside the descriptor");
+            if (used && off + 16 > d.bytes) return fail(t.kernel, operand, s, ld, 0, off, "a used fetch leaves its descriptor");
+          }
+          if (used && d.base * 2 + off != ((row0 + row) * ld + k_lo + A::imin(sl, slabs - 1) * 64 + piece * 8) * 2)
+            return fail(t.kernel, operand, s, ld, 0, off, "a used fetch is not the lane's row and k");
+        }
+      }
+  return true;
+}
+
+// per: units of two bytes per element
+static bool tiles(const Shape& s, long lda, long ldw, const Tiles& t, int per) {
+  if (t.big && s.K % 64) return true;                  // the larger tiles take whole slabs only
+  const A::KSplit cut = A::cut_k(s.K, s.splits, 64 / per);
   for (int by = 0; by < cut.splits; ++by) {
-    const int k_lo = by * cut.k_per_block, k_hi = A::imin(s.K, k_lo + cut.k_per_block);
-    for (long m0 = 0; m0 < s.M; m0 += tile)
-      if (!tile_operand(kernel, "A", s, s.M, lda, m0, tile, waves, k_lo, k_hi, big)) return false;
-    for (long n0 = 0; n0 < s.N; n0 += tile)
-      if (!tile_operand(kernel, "W", s, s.N, ldw, n0, tile, waves, k_lo, k_hi, big)) return false;
+    const int k_lo = per * by * cut.k_per_block, k_hi = per * A::imin(s.K, (by + 1) * cut.k_per_block);
+    for (long m0 = 0; m0 < s.M; m0 += t.rows_a)
+      if (!tile_operand(t, "A", s, s.M, per * s.K, per * lda, m0, t.rows_a, k_lo, k_hi)) return false;
+    for (long n0 = 0; n0 < s.N; n0 += t.rows_w)
+      if (!tile_operand(t, "W", s, s.N, per * s.K, per * ldw, n0, t.rows_w, k_lo, k_hi)) return false;
   }
   return true;
 }
+static const Tiles BFLOAT16_TILES[] = {
+    {"gemm_mfma", 128, 128, 4, false, 0},              // asks for existing slabs only
+    {"gemm_mfma_big<4, 2>", 256, 256, 8, true, 2}, {"gemm_mfma_big<3, 3>", 192, 384, 8, true, 2}, {"gemm_mfma_big<3, 2>", 192, 256, 8, true, 2},
+    {"gemm_mfma_big<2, 3>", 128, 384, 8, true, 2}, {"gemm_mfma_big<2, 2>", 128, 256, 8, true, 2},
+};
+static const Tiles FLOAT32_TILES[] = {                 // the rings of buffers, less the one in use
+    {"gemm_float32_tile<128, 128>", 128, 128, 4, false, 1}, {"gemm_float32_tile<128, 64>", 128, 64, 4, false, 2}, {"gemm_float32_tile<64, 64>", 64, 64, 4, false, 3},
+};
 
 // ------------------------------------------------------------------ attention over the paged cache
 // Every fetch of a chunk's two tiles (attn_load): the keys' fragments (16 bytes) and the values'
@@ -224,7 +278,7 @@ static bool attention(int hd, int page_size, int nkv, long num_pages) {
 }
 
 static bool check(const Shape& s) {
-  for (int pad = 0; pad <= 16; pad += 8) {             // row strides K, K + 8, K + 16
+  for (int pad = 0; pad <= 16 && s.K % 8 == 0; pad += 8) {     // row strides K, K + 8, K + 16
     const long ld = s.K + pad;
     if (s.M <= 32) {
       if (!skinny(s, ld, ld, 0, 2, A::KSTEP)) return false;
@@ -232,7 +286,17 @@ static bool check(const Shape& s) {
     } else if (s.M <= 128) {
       if (!shared(s, ld, ld, 0, 4)) return false;
     }
-    if (!tiles(s, ld, ld, false) || !tiles(s, ld, ld, true)) return false;
+    for (const Tiles& t : BFLOAT16_TILES)
+      if (!tiles(s, ld, ld, t, 1)) return false;
+  }
+  for (int pad = 0; pad <= 12 && s.K % 4 == 0; pad += 12) {    // float32: row strides K and K + 12
+    const long ld = s.K + pad;
+    if (s.M <= 32) {
+      if (!float32_rows(s, ld, ld, 2, 4, 1) || !float32_rows(s, ld, ld, 1, 8, 2) || !float32_rows(s, ld, ld, 1, 16, 2)) return false;
+    } else {
+      for (const Tiles& t : FLOAT32_TILES)
+        if (!tiles(s, ld, ld, t, 2)) return false;
+    }
   }
   if (s.N % 16 == 0 && s.K % 64 == 0) {                // the streaming copy of the weights
     if (s.M <= 32 && !skinny(s, s.K, s.K, 1, 2, A::KSTEP)) return false;
@@ -251,14 +315,14 @@ int main(int argc, char** argv) {
   for (; a + 3 < argc; a += 4) shapes.push_back(Shape{std::atoi(argv[a]), std::atoi(argv[a + 1]), std::atoi(argv[a + 2]), std::atoi(argv[a + 3])});
   const int Ms[] = {1, 2, 7, 8, 9, 16, 17, 31, 32, 33, 48, 64, 65, 100, 128, 129, 300};
   const int Ns[] = {1, 16, 31, 32, 33, 64, 100, 520, 2048};
-  const int Ks[] = {8, 16, 64, 72, 96, 128, 160, 200, 256, 272, 344, 512, 1024, 2816};
+  const int Ks[] = {4, 8, 16, 36, 64, 72, 96, 100, 128, 160, 200, 256, 272, 344, 512, 516, 1024, 2816};
   const int Ss[] = {1, 2, 3, 4, 8};
   for (int M : Ms)
     if (sweep)
     for (int N : Ns)
       for (int K : Ks)
         for (int S : Ss)
-          if (S == 1 || K / S >= 8) shapes.push_back(Shape{M, N, K, S});
+          if (S == 1 || K / S >= 4) shapes.push_back(Shape{M, N, K, S});
   for (const Shape& s : shapes)
     if (!check(s)) return 1;
   if (sweep)

@@ -4,8 +4,8 @@ A fetch whose result is discarded (a row beyond the matrix, k beyond a wave's ra
 value, so no comparison of results can see where it went; it faults only when the tensor ends
 where its mapping ends.  The kernels take their address arithmetic from ``csrc/addressing.h``;
 ``tests/cpp/load_bounds.cpp`` includes the same header, walks every block, wave, lane and step of
-the weight-streaming kernels (row-major and tiled weights) and of the two tile kernels (their
-buffer descriptors and lane offsets) for a sweep of shapes, and the key and value fetches of the
+the weight-streaming kernels (row-major and tiled weights, bfloat16 and float32) and of the tile kernels in
+every tile shape (their buffer descriptors and lane offsets) for a sweep of shapes, and the key and value fetches of the
 attention kernels' chunks (pages that are there, missing, or no pages of the pool) for every head
 size, and checks every fetch.
 """
@@ -37,7 +37,7 @@ def _args(shapes):
     """Each shape with the split counts that the dispatch rules give it, and a few more."""
     out = []
     for m, n, k in shapes:
-        if k % 8:
+        if k % 4:
             continue                      # such a product goes to the general kernel
         wanted = {1, 2, 3, fast._skinny_splits(m, n, k) if m <= fast.SKINNY_MAX_ROWS else fast._tile_splits(m, n, k)}
         for s in sorted(wanted):
