@@ -30,10 +30,10 @@ constexpr int MIN_K = 256;             // a piece keeps at least this much of k
 constexpr double SHAPE_GAIN = 0.96, PIECES_GAIN = 0.96;
 // Bytes per microsecond: float32 pieces out of the larger tiles (beyond the times above; in those of the 128 x 128 tiles
 // they are hidden), and pieces or the updated stream into the norm behind the product; and what every piece takes there
-// besides.  Fitted to product and norm together, 176 sizes of 130 to 2,627 rows in one to eight pieces: 3.1 % above the best
-// number of pieces on average.  7e6, nothing per piece and a gain of 0.98 asked for more pieces than paid (4.8 %): 300 x 2,048 x
+// besides.  Fitted to product and norm together, 176 sizes of 130 to 2,627 rows in one to eight pieces: 2.8 % above the best
+// number of pieces on average.  10e6, 7e6, nothing per piece and a gain of 0.98 asked for more pieces than paid (4.8 %): 300 x 2,048 x
 // 2,048 in eight 21.3 us, in four 18.4; 256 x 4,096 x 4,096 28.7 and 24.3; 700 x 1,024 x 1,024 in four 17.0, in two 14.9.
-constexpr double PIECES_WRITTEN = 10e6, PIECES_READ = 4e6, PIECE_US = 0.3;
+constexpr double PIECES_WRITTEN = 13e6, PIECES_READ = 4.5e6, PIECE_US = 0.4;
 
 inline double shape_us(const Shape& s, int M, int N, int K, int splits, int units) {
   const int per_piece = (K + splits - 1) / splits;
