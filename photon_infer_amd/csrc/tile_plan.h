@@ -28,12 +28,13 @@ constexpr int MAX_SPLITS = 8;
 constexpr int MIN_K = 256;             // a piece keeps at least this much of k
 // What the fit, which is good to some per cent, must promise at least before another shape or one more piece is taken.
 constexpr double SHAPE_GAIN = 0.96, PIECES_GAIN = 0.96;
-// Bytes per microsecond: float32 pieces out of the larger tiles (beyond the times above; in those of the 128 x 128 tiles
-// they are hidden), and pieces or the updated stream into the norm behind the product; and what every piece takes there
-// besides.  Fitted to product and norm together, 176 sizes of 130 to 2,627 rows in one to eight pieces: 2.8 % above the best
-// number of pieces on average.  10e6, 7e6, nothing per piece and a gain of 0.98 asked for more pieces than paid (4.8 %): 300 x 2,048 x
-// 2,048 in eight 21.3 us, in four 18.4; 256 x 4,096 x 4,096 28.7 and 24.3; 700 x 1,024 x 1,024 in four 17.0, in two 14.9.
-constexpr double PIECES_WRITTEN = 13e6, PIECES_READ = 4.5e6, PIECE_US = 0.4;
+// Bytes per microsecond of pieces, or of the updated stream, on their way into the norm behind the product, and what every
+// piece takes there besides (writing them is hidden in the times above).  Fitted to product and norm together, 176 sizes of 130
+// to 2,627 rows in one to eight pieces, and to whole prompts, whose weights are cold: 300 x 2,048 x 2,048 takes
+// 18.4 us in four pieces and 21.3 in eight, 256 x 4,096 x 4,096 24.3 and 28.7, 700 x 1,024 x 1,024 14.9 in two and 17.0 in four.
+// Rows of more than 4,096 columns go through the norm at half that rate (1,267 x 5,376 x 4,544: 104 us in one piece, 175 in two).
+constexpr double PIECES_READ = 4e6, WIDE_READ = 2e6, PIECE_US = 0.3;
+constexpr int WIDE = 4096;
 
 inline double shape_us(const Shape& s, int M, int N, int K, int splits, int units) {
   const int per_piece = (K + splits - 1) / splits;
@@ -56,8 +57,7 @@ inline Choice shape_for(int M, int N, int K, int splits, int units) {
   if (K % SLAB) return best;
   for (const Shape& s : SHAPES) {
     if (s.code == 0) continue;
-    double us = shape_us(s, M, N, K, splits, units);
-    if (splits > 1) us += 4.0 * splits * M * N / PIECES_WRITTEN;
+    const double us = shape_us(s, M, N, K, splits, units);
     if (us < best.us * (s.code == 42 ? 1.0 : SHAPE_GAIN)) best = Choice{s.code, us};
   }
   return best;
@@ -66,12 +66,13 @@ inline Choice shape_for(int M, int N, int K, int splits, int units) {
 // In how many pieces a product is left whose reader adds them: as many as take the least time together with their way
 // through memory, if they take at most `worth` of the time in one piece, and no more than `part_floats` floats hold.
 inline int splits_for(int M, int N, int K, int units, long part_floats, double worth) {
-  const double whole = shape_for(M, N, K, 1, units).us + 4.0 * M * N / PIECES_READ;      // the kernel adds into the stream
+  const double read = N > WIDE ? WIDE_READ : PIECES_READ;
+  const double whole = shape_for(M, N, K, 1, units).us + 4.0 * M * N / read;      // the kernel adds into the stream
   int best = 1;
   double least = whole;
   for (int splits = 2; splits <= MAX_SPLITS; ++splits) {
     if (K / splits < MIN_K || (long)splits * M * N > part_floats) break;
-    const double us = shape_for(M, N, K, splits, units).us + 4.0 * splits * M * N / PIECES_READ + PIECE_US * splits;
+    const double us = shape_for(M, N, K, splits, units).us + 4.0 * splits * M * N / read + PIECE_US * splits;
     if (us < PIECES_GAIN * least) { best = splits; least = us; }
   }
   return best > 1 && least > worth * whole ? 1 : best;

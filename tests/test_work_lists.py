@@ -149,7 +149,7 @@ PIECES_MEASURED = [
     (300, 2048, 2048, [23.8, 18.1, 17.9, 18.4, 19.6, 20.0, 21.8, 21.3]), (130, 2048, 8192, [74.4, 43.4, 32.5, 27.3, 24.4, 22.7, 21.5, 20.2]),
     (2048, 2048, 8192, [98.6, 83.6, 85.5, 87.7]), (1400, 2048, 8192, [88.3, 66.9, 72.1, 65.6, 71.4]), (256, 4096, 4096, [49.0, 29.8, 25.8, 24.3, 26.7, 27.8, 29.9, 28.7]),
     (1000, 4096, 4096, [58.5, 53.4, 57.7, 59.3]), (2048, 4096, 4096, [86.9, 90.5]), (200, 4096, 14336, [135.4, 74.6, 55.8, 47.8, 46.6, 43.2, 42.0, 41.4]),
-    (700, 1024, 1024, [17.6, 14.9, 15.7, 17.0]), (300, 3072, 3072, [43.5, 27.4, 24.3, 24.5, 24.3, 25.0, 26.6, 28.2]), (2600, 2048, 2048, [46.1, 47.8, 59.9]),
+    (700, 1024, 1024, [17.6, 14.9, 15.7, 17.0]), (300, 3072, 3072, [43.5, 27.4, 24.3, 24.5, 24.3, 25.0, 26.6, 28.2]), (2600, 2048, 2048, [46.1, 47.8, 59.9]), (1267, 5376, 4544, [104.3, 175.0]),
 ]
 
 
