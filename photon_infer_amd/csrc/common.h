@@ -208,3 +208,14 @@ inline int pi_check_launch(const char* what) {
   } while (0)
 
 static inline int ceil_div(long a, long b) { return (int)((a + b - 1) / b); }
+
+// Compute units of the device that is current at the first call (256 on an MI355X).
+static inline int compute_units() {
+  static const int units = [] {
+    int device = 0, count = 0;
+    if (hipGetDevice(&device) != hipSuccess || hipDeviceGetAttribute(&count, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || count <= 0)
+      count = 256;
+    return count;
+  }();
+  return units;
+}

@@ -163,16 +163,6 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_float32_rows_kernel(float* __
 }
 
 // ------------------------------------------------------------------ many rows: tiles
-// A block-wide barrier that waits for this wave's LDS accesses and for all but its last LOADS loads from memory;
-// __syncthreads() would wait for every load on its way into LDS.
-template <int LOADS>
-__device__ inline void block_barrier_keeping_loads() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt(0x0070 | (LOADS & 15) | ((LOADS >> 4) << 14));      // vmcnt LOADS, lgkmcnt 0
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-
 // Block tile TM x TN, four waves in 2 x 2, slabs of 32 floats of k that go from memory straight into LDS through a ring
 // of NB buffers (rows of 128 bytes, their 16-byte pieces turned by (row / 2) % 8 as in gemm_mfma.hip).  A matrix
 // instruction takes 64 cycles for two registers of operands, so LDS and its reads have time to spare and the tile only
@@ -328,17 +318,6 @@ struct Float32Plan {
   int tm, tn;            // 0: the weight-streaming kernel
   int splits, k_per_split;
 };
-
-static int compute_units() {
-  static int units = 0;
-  if (units == 0) {
-    int device = 0, count = 0;
-    if (hipGetDevice(&device) != hipSuccess || hipDeviceGetAttribute(&count, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || count <= 0)
-      count = 256;
-    units = count;
-  }
-  return units;
-}
 
 static Float32Plan cut(int tm, int tn, int K, int splits) {
   const addressing::KSplit c = addressing::cut_k(K, splits, FSTEP);

@@ -192,6 +192,24 @@ __device__ inline void store_rows32(float* patch, const f32x16_t& acc0, const f3
   __builtin_amdgcn_wave_barrier();
 }
 
+// Consecutive blocks go to the chip's 8 dies in turn, each with an L2 of its own.  Give every die a run of tiles, the row
+// tiles of a column before the next column: a die then streams its own share of W once and re-reads only A (768 x 19,200 x 4,096
+// 99 us; with the tiles dealt across the dies 119).  With many row tiles and a long k the dies take two by four rectangles:
+// a row of A is then read by four dies and not by all eight in the same moment (2,048 x 16,384 x 8,192 439 -> 421 us; with
+// four row tiles 2 to 5 % slower, and so are short k).
+__device__ inline void tile_of_block(int block, int tiles_m, int tiles_n, int k, int& tile_m, int& tile_n) {
+  const int die = block % 8, local = block / 8;
+  if (tiles_m >= 8 && tiles_m % 2 == 0 && tiles_n % 4 == 0 && k >= 2048) {
+    const int half = tiles_m / 2;
+    tile_m = die / 4 * half + local % half;
+    tile_n = die % 4 * (tiles_n / 4) + local / half;
+  } else {
+    const int tiles = tiles_m * tiles_n, id = die * (tiles / 8) + min(die, tiles % 8) + local;
+    tile_m = id % tiles_m;
+    tile_n = id / tiles_m;
+  }
+}
+
 template <int EPI>
 __global__ __launch_bounds__(256) void gemm_mfma_kernel(void* __restrict__ Cv, long ldc, const bf16_t* __restrict__ A, long lda,
                                                         const bf16_t* __restrict__ W, long ldw, int M, int N, int K,
@@ -210,19 +228,8 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(void* __restrict__ Cv, l
   const int k_lo = blockIdx.y * k_per_split;
   const int k_hi = min(K, k_lo + k_per_split);
   if (gridDim.y > 1) Cv = reinterpret_cast<float*>(Cv) + (long)blockIdx.y * M * ldc;
-  // Consecutive blocks go to the chip's 8 dies in turn, each with an L2 of its own.  Give every
-  // die a contiguous range of weight tiles (columns) and let it walk the row tiles of a column
-  // before the next column: a die then streams its slice of W once and re-reads only A.
-  const int tiles_m = gridDim.x / tiles_n;
   int tile_m, tile_n;
-  if (tiles_n % 8 == 0) {
-    const int die = blockIdx.x % 8, local = blockIdx.x / 8;
-    tile_n = die * (tiles_n / 8) + local / tiles_m;
-    tile_m = local % tiles_m;
-  } else {
-    tile_m = blockIdx.x / tiles_n;
-    tile_n = blockIdx.x % tiles_n;
-  }
+  tile_of_block(blockIdx.x, gridDim.x / tiles_n, tiles_n, k_hi - k_lo, tile_m, tile_n);
   // Grouped: the rows are sorted by group (a routed feed-forward's experts) and cut into tiles of
   // up to 128 rows of one group; tile t multiplies rows tile_row0[t] .. + tile_rows[t] - 1 with the
   // matrix of group group_of_tile[t] (W + group * group_stride).  The list lives on the device
@@ -366,22 +373,26 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(void* __restrict__ Cv, l
 }
 
 // ---------------------------------------------------------------------------------------------
-// The same product with larger block tiles, for problems that have enough of them to fill the
-// chip and a k that is a multiple of the slab: eight waves in 2 x 4 (two per SIMD), each
+// The same product with larger block tiles, for a k that is a multiple of the slab: eight waves in 2 x 4 (two per SIMD), each
 // WI x WJ tiles of v_mfma_f32_32x32x16_bf16, so that a block's tile is 64 WI x 128 WJ: 256 x 256,
-// 192 x 384, 192 x 256, 128 x 384 or 128 x 256.  A unit holds one block, and a last round of few blocks
+// 192 x 384, 192 x 256, 128 x 384, 128 x 256 or 128 x 128.  A unit holds one block, and a last round of few blocks
 // costs as much as a full one: which shape a product takes is decided by the rounds it needs (tile_plan.h).
 // At 256 x 256 a wave reads 6 fragments from
 // LDS per 16 k for 8 matrix-core instructions, three quarters of the LDS traffic per flop of the
 // 128 x 128 kernel (192 x 384: 6 for 9, 128 x 256: 4 for 4), and a block asks L2 for half the bytes per flop.  With one wave per SIMD
-// (four waves of 128 x 128, the first form of this kernel) every barrier and every wait left
+// (four waves of 128 x 128) every barrier and every wait left
 // the matrix pipe idle.  No branch in the loop (rows beyond the matrix are clamped on load and
 // skipped on store), loads through a buffer descriptor (a scalar base that moves with k plus
-// fixed 32-bit lane offsets, no vector arithmetic per slab) straight into the other LDS
-// buffer, issued at the top of a slab and awaited at its one barrier, and scheduling hints that
+// fixed 32-bit lane offsets, no vector arithmetic per slab) straight into LDS, and scheduling hints that
 // deal the memory instructions out between the matrix-core ones.
+// What bounds it is the loads: the loop without its matrix instructions takes 372 of 440 us (2,048 x 16,384 x 8,192), and
+// without its loads 355.  The slabs lie in rings, NA buffers for A and NW for W, as many as fit 160 KB, and a slab's one
+// barrier waits for the loads that the next slab needs and not for those behind them: W, which comes from memory, is two
+// slabs ahead.  Against two buffers of each: 128 x 256 (3 and 3) 512 x 8,192 x 4,096 57 us instead of 74, 192 x 256 (2 and 3)
+// 768 x 8,192 x 4,096 71 instead of 86, 256 x 256 (2 and 3) 1,024 x 8,192 x 4,096 87 instead of 95 and on a full chip 2 % less;
+// slabs of 32 k in five buffers were slower (rows of 64 bytes come at half the rate of rows of 128).
 // Per output element the sum over k runs in ascending k, as in the small kernel.
-template <int EPI, int WI, int WJ>
+template <int EPI, int WI, int WJ, int NA, int NW>
 __global__ __launch_bounds__(512) void gemm_mfma_big_kernel(void* __restrict__ Cv, long ldc, const bf16_t* __restrict__ A, long lda,
                                                             const bf16_t* __restrict__ W, long ldw, int M, int N, int K,
                                                             int tiles_n, int k_per_split, GluArgs glu) {
@@ -389,24 +400,16 @@ __global__ __launch_bounds__(512) void gemm_mfma_big_kernel(void* __restrict__ C
   constexpr int ROW = BK;                       // rows of 128 bytes, no padding: the loads write LDS themselves, lane after lane
   constexpr int GM = 64 * WI, GN = 128 * WJ;    // the block's tile
   constexpr int AI = WI, BI = 2 * WJ;           // load instructions of a wave per slab: eight rows each
-  uint16_t* As = lds;                           // [2][GM][ROW], 16-byte pieces of a row turned by (row / 2) % 8
-  uint16_t* Ws = lds + 2 * GM * ROW;            // [2][GN][ROW]
+  uint16_t* As = lds;                           // [NA][GM][ROW], 16-byte pieces of a row turned by (row / 2) % 8
+  uint16_t* Ws = lds + NA * GM * ROW;           // [NW][GN][ROW]
   const int tid = threadIdx.x, lane = tid % 64;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
   const int wm = wave / 4, wn = wave % 4;       // a wave's corner: 32 WI rows x 32 WJ columns
   const int k_lo = blockIdx.y * k_per_split;
   const int k_hi = min(K, k_lo + k_per_split);
   if (gridDim.y > 1) Cv = reinterpret_cast<float*>(Cv) + (long)blockIdx.y * M * ldc;
-  const int tiles_m = gridDim.x / tiles_n;
   int tile_m, tile_n;
-  if (tiles_n % 8 == 0) {                       // a die streams its own slice of W, see above
-    const int die = blockIdx.x % 8, local = blockIdx.x / 8;
-    tile_n = die * (tiles_n / 8) + local / tiles_m;
-    tile_m = local % tiles_m;
-  } else {
-    tile_m = blockIdx.x / tiles_n;
-    tile_n = blockIdx.x % tiles_n;
-  }
+  tile_of_block(blockIdx.x, gridDim.x / tiles_n, tiles_n, k_hi - k_lo, tile_m, tile_n);
   const long m0 = (long)tile_m * GM, n0 = (long)tile_n * GN;
 
   // global -> LDS without registers in between: load instruction p of wave w fills rows
@@ -430,15 +433,19 @@ __global__ __launch_bounds__(512) void gemm_mfma_big_kernel(void* __restrict__ C
     w_off[p] = addressing::big_lane_offset(row, w_rows, ldw, addressing::tile_piece(lane, row));
   }
   const int slabs = (k_hi - k_lo) / BK;
-  auto load_slab = [&](int s, int buf) {
-    const int kbytes = addressing::big_slab_bytes(s, slabs);     // past the last slab: read it again, unused
+  // past the last slab: read it again, unused
+  auto load_a = [&](int s, int buf) {
 #if defined(__HIP_DEVICE_COMPILE__)
 #pragma unroll
     for (int p = 0; p < AI; ++p)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(a_src, (lds_ptr_t)(As + (buf * GM + (wave * AI + p) * 8) * ROW), 16, a_off[p], kbytes, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(a_src, (lds_ptr_t)(As + (buf * GM + (wave * AI + p) * 8) * ROW), 16, a_off[p], addressing::big_slab_bytes(s, slabs), 0, 0);
+#endif
+  };
+  auto load_w = [&](int s, int buf) {
+#if defined(__HIP_DEVICE_COMPILE__)
 #pragma unroll
     for (int p = 0; p < BI; ++p)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(w_src, (lds_ptr_t)(Ws + (buf * GN + (wave * BI + p) * 8) * ROW), 16, w_off[p], kbytes, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(w_src, (lds_ptr_t)(Ws + (buf * GN + (wave * BI + p) * 8) * ROW), 16, w_off[p], addressing::big_slab_bytes(s, slabs), 0, 0);
 #endif
   };
 
@@ -455,9 +462,9 @@ __global__ __launch_bounds__(512) void gemm_mfma_big_kernel(void* __restrict__ C
 #pragma unroll
   for (int ks = 0; ks < 4; ++ks) place[ks] = ((ks * 2 + lane / 32) ^ ((frow >> 1) & 7)) * 8;
   Frag fa[2][WI], fb[2][WJ];
-  auto read_frags = [&](int which, int buf, int ks) {   // ks: which 16 k of the slab
-    const uint16_t* a_base = As + (buf * GM + wm * 32 * WI + frow) * ROW + place[ks];
-    const uint16_t* w_base = Ws + (buf * GN + wn * 32 * WJ + frow) * ROW + place[ks];
+  auto read_frags = [&](int which, int abuf, int wbuf, int ks) {   // ks: which 16 k of the slab
+    const uint16_t* a_base = As + (abuf * GM + wm * 32 * WI + frow) * ROW + place[ks];
+    const uint16_t* w_base = Ws + (wbuf * GN + wn * 32 * WJ + frow) * ROW + place[ks];
 #pragma unroll
     for (int i = 0; i < WI; ++i) fa[which][i].n = *reinterpret_cast<const u32x4_t*>(a_base + i * 32 * ROW);
 #pragma unroll
@@ -470,10 +477,17 @@ __global__ __launch_bounds__(512) void gemm_mfma_big_kernel(void* __restrict__ C
       for (int j = 0; j < WJ; ++j) acc[i][j] = mfma32(fa[which][i], fb[which][j], acc[i][j]);
   };
 
-  load_slab(0, 0);
-  __builtin_amdgcn_s_waitcnt(0x0F70);           // vmcnt(0): this wave's pieces of the slab are in LDS
-  __syncthreads();
-  read_frags(0, 0, 0);
+  // Slab s of A goes to buffer s % NA, of W to s % NW.  After slab s a step asks for slab s + NA of A, then for slab s + NW
+  // of W; LATER of these loads were asked for behind those that slab s + 1 needs, and loads return in order.
+  constexpr int BEHIND_A = BI + (NA - 2) * (AI + BI), BEHIND_W = (NW - 2) * (AI + BI);
+  constexpr int LATER = BEHIND_A < BEHIND_W ? BEHIND_A : BEHIND_W;
+#pragma unroll
+  for (int s = 0; s < (NA > NW ? NA : NW); ++s) {
+    if (s < NA) load_a(s, s);
+    if (s < NW) load_w(s, s);
+  }
+  block_barrier_keeping_loads<(NA - 1) * AI + (NW - 1) * BI>();
+  read_frags(0, 0, 0, 0);
   // the order wanted inside one scheduling region: after every matrix-core instruction one fragment read, as long as there
   // are any, and (`loads`) its share of the next slab's loads
 #define PI_DEAL(loads)                                                                                            \
@@ -484,24 +498,26 @@ __global__ __launch_bounds__(512) void gemm_mfma_big_kernel(void* __restrict__ C
     if (share_ > 0) __builtin_amdgcn_sched_group_barrier(PI_SCHED_VMEM_READ, 1, 0);                               \
     if (share_ > 1) __builtin_amdgcn_sched_group_barrier(PI_SCHED_VMEM_READ, 1, 0);                               \
   }
-  load_slab(1, 1);
+  int ab = 0, wb = 0;                       // slab s of A and of W
   for (int s = 0; s < slabs; ++s) {
-    const int buf = s & 1;
-    read_frags(1, buf, 1);
+    const int a_next = ab == NA - 1 ? 0 : ab + 1, w_next = wb == NW - 1 ? 0 : wb + 1;
+    read_frags(1, ab, wb, 1);
     products(0);
     PI_DEAL(false)
-    read_frags(0, buf, 2);
+    read_frags(0, ab, wb, 2);
     products(1);
     PI_DEAL(false)
-    read_frags(1, buf, 3);
+    read_frags(1, ab, wb, 3);
     products(0);
     PI_DEAL(false)
-    __builtin_amdgcn_s_waitcnt(0x0F70);     // slab s + 1 has landed (asked for a whole slab ago)
-    __syncthreads();
-    load_slab(s + 2, buf);          // into the buffer everybody has just left
-    read_frags(0, buf ^ 1, 0);
+    block_barrier_keeping_loads<LATER>();   // slab s + 1 has landed, and everybody has read slab s
+    load_a(s + NA, ab);
+    load_w(s + NW, wb);
+    read_frags(0, a_next, w_next, 0);
     products(1);
     PI_DEAL(true)
+    ab = a_next;
+    wb = w_next;
   }
   __builtin_amdgcn_s_waitcnt(0x0F70);       // nothing may still be on its way into LDS when the patches take it over
 #undef PI_DEAL
@@ -530,24 +546,26 @@ __global__ __launch_bounds__(512) void gemm_mfma_big_kernel(void* __restrict__ C
 
 static const size_t kLdsBytes = 4 * TILE_ELEMS * sizeof(uint16_t);   // 65,536 bytes
 
-template <int EPI, int WI, int WJ>
+template <int EPI, int WI, int WJ, int NA, int NW>
 static int launch_big(void* C, long ldc, const void* A, long lda, const void* W, long ldw, int M, int N, int K, int splits, int kps,
                       hipStream_t stream, GluArgs glu) {
-  constexpr size_t bytes = 2 * (64 * WI + 128 * WJ) * BK * sizeof(uint16_t);
+  constexpr size_t ring = (NA * 64 * WI + NW * 128 * WJ) * BK * sizeof(uint16_t), patches = 8 * PATCH_FLOATS * sizeof(float);
+  constexpr size_t bytes = ring > patches ? ring : patches;
+  static_assert(bytes <= 160 * 1024, "more LDS than a unit has");
   static bool configured = false;
   if (!configured) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_mfma_big_kernel<EPI, WI, WJ>),
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_mfma_big_kernel<EPI, WI, WJ, NA, NW>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
     if (e != hipSuccess) return pi_fail("gemm_mfma: cannot reserve %zu bytes of LDS: %s", bytes, hipGetErrorString(e));
     configured = true;
   }
   const long tiles = (long)ceil_div(M, 64 * WI) * ceil_div(N, 128 * WJ);
-  hipLaunchKernelGGL((gemm_mfma_big_kernel<EPI, WI, WJ>), dim3((unsigned)tiles, splits), dim3(512), bytes, stream, C, ldc,
+  hipLaunchKernelGGL((gemm_mfma_big_kernel<EPI, WI, WJ, NA, NW>), dim3((unsigned)tiles, splits), dim3(512), bytes, stream, C, ldc,
                      (const bf16_t*)A, lda, (const bf16_t*)W, ldw, M, N, K, ceil_div(N, 128 * WJ), kps, glu);
   return pi_check_launch("gemm_mfma_big");
 }
 
-// shape: 0 the 128 x 128 kernel, else 10 WI + WJ of the larger tiles (K a multiple of the slab)
+// shape: 0 a 128 x 128 tile, in whichever kernel is the faster one; else 10 WI + WJ of the larger tiles' kernel (K a multiple of the slab)
 template <int EPI>
 static int launch(void* C, long ldc, const void* A, long lda, const void* W, long ldw, int M, int N, int K, int splits, int shape,
                   hipStream_t stream, GluArgs glu = GluArgs{nullptr, 0.f, 0.f, 0}) {
@@ -556,12 +574,14 @@ static int launch(void* C, long ldc, const void* A, long lda, const void* W, lon
   splits = cut.splits;
   PI_REQUIRE(shape == 0 || K % BK == 0, "gemm_mfma: the larger tiles take whole slabs of %d only, K is %d", BK, K);
   switch (shape) {
-    case 0: break;
-    case 42: return launch_big<EPI, 4, 2>(C, ldc, A, lda, W, ldw, M, N, K, splits, kps, stream, glu);
-    case 33: return launch_big<EPI, 3, 3>(C, ldc, A, lda, W, ldw, M, N, K, splits, kps, stream, glu);
-    case 32: return launch_big<EPI, 3, 2>(C, ldc, A, lda, W, ldw, M, N, K, splits, kps, stream, glu);
-    case 23: return launch_big<EPI, 2, 3>(C, ldc, A, lda, W, ldw, M, N, K, splits, kps, stream, glu);
-    case 22: return launch_big<EPI, 2, 2>(C, ldc, A, lda, W, ldw, M, N, K, splits, kps, stream, glu);
+    case 0:
+      if (!tile_plan::ring_128_takes(M, N, K, splits, compute_units())) break;        // else the same tile in a ring
+    case 21: return launch_big<EPI, 2, 1, 3, 3>(C, ldc, A, lda, W, ldw, M, N, K, splits, kps, stream, glu);
+    case 42: return launch_big<EPI, 4, 2, 2, 3>(C, ldc, A, lda, W, ldw, M, N, K, splits, kps, stream, glu);
+    case 33: return launch_big<EPI, 3, 3, 2, 2>(C, ldc, A, lda, W, ldw, M, N, K, splits, kps, stream, glu);
+    case 32: return launch_big<EPI, 3, 2, 2, 3>(C, ldc, A, lda, W, ldw, M, N, K, splits, kps, stream, glu);
+    case 23: return launch_big<EPI, 2, 3, 2, 2>(C, ldc, A, lda, W, ldw, M, N, K, splits, kps, stream, glu);
+    case 22: return launch_big<EPI, 2, 2, 3, 3>(C, ldc, A, lda, W, ldw, M, N, K, splits, kps, stream, glu);
     default: return pi_fail("gemm_mfma: unknown tile shape %d", shape);
   }
   static bool configured = false;

@@ -70,3 +70,14 @@ __device__ inline __amdgpu_buffer_rsrc_t operand_descriptor(const bf16_t* operan
 }
 #endif
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
+
+// A block-wide barrier that waits for this wave's LDS accesses and for all but its last LOADS loads from memory;
+// __syncthreads() would wait for every load on its way into LDS.
+template <int LOADS>
+__device__ inline void block_barrier_keeping_loads() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0x0070 | (LOADS & 15) | ((LOADS >> 4) << 14));      // vmcnt LOADS, lgkmcnt 0
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+

@@ -4,36 +4,43 @@
 // count changes each time 2,520 -> 2,445 us, as fast now as with a count seen before).
 #pragma once
 
+#include <cmath>
+
 namespace tile_plan {
 
 // A block tile: its code (0: the 128 x 128 kernel; 10 WI + WJ of the larger tiles), rows and columns, blocks that a unit
 // holds at a time, and the microseconds of a block that has the chip nearly to itself and of one on a full chip, for k in
-// units of 1,024.  Fitted to measurements on an MI355X of 129 to 2,627 rows with nine matrices of 2,048 x 2,048 to
-// 28,672 x 4,096, whole and in two to four pieces.  543 x 28,672 x 4,096: 336 tiles of 256 x 256 take two rounds of 256
-// units, 184 us; 225 of 192 x 384 one, 130 us.  2,048 x 4,384 x 2,048: 61 us on 128 x 128, 42 to 48.
+// units of 1,024.  Fitted to measurements on an MI355X of 32 to 512 tiles of every shape at k of 256 to 8,192, weights cold
+// and results float32 (450 products, off by 6 to 8 % in the mean).  543 x 28,672 x 4,096: 336 tiles of 256 x 256 take two rounds of 256
+// units, 184 us; 225 of 192 x 384 one, 121 us.
 struct Shape {
   int code, rows, cols, slots;
   double alone[3], full[2];
 };
 constexpr Shape SHAPES[] = {
-    {0, 128, 128, 2, {6.0, 8.0, 0.35}, {6.0, 16.5}},
-    {42, 256, 256, 1, {7.0, 15.0, 0.25}, {6.0, 26.0}},
-    {33, 192, 384, 1, {8.0, 18.0, 0.3}, {7.0, 32.5}},
-    {32, 192, 256, 1, {7.0, 12.5, 0.25}, {5.0, 23.5}},
-    {23, 128, 384, 1, {7.0, 13.5, 0.3}, {5.0, 28.0}},
-    {22, 128, 256, 1, {6.0, 10.0, 0.25}, {4.0, 20.5}},
+    {0, 128, 128, 2, {6.533, 4.741, 0.748}, {8.62, 14.413}},
+    {42, 256, 256, 1, {7.699, 13.742, 0.347}, {12.781, 23.51}},
+    {33, 192, 384, 1, {8.2, 17.7, 0.68}, {14.8, 27.9}},
+    {32, 192, 256, 1, {7.117, 10.692, 0.274}, {10.926, 19.844}},
+    {23, 128, 384, 1, {7.3, 12.4, 1.25}, {10, 24.3}},
+    {22, 128, 256, 1, {6.449, 5.174, 2.036}, {8.406, 14.202}},
 };
+// 128 x 128 in the larger tiles' kernel, one block of eight waves to a unit, for whole slabs of k: taken in the place of the
+// 128 x 128 kernel where it is the faster one of the two (256 tiles of k = 8,192 82 us instead of 104; 512 of k = 256 15.5
+// and of k = 2,048 50 us instead of 41, two of whose blocks a unit holds).
+constexpr Shape RING_128 = {21, 128, 128, 1, {5.977, 4.279, 0.323}, {6.392, 9.063}};
 constexpr int SLAB = 64;               // k per slab: the larger tiles take whole slabs only
 constexpr int MAX_SPLITS = 8;
 constexpr int MIN_K = 256;             // a piece keeps at least this much of k
 // What the fit, which is good to some per cent, must promise at least before another shape or one more piece is taken.
-constexpr double SHAPE_GAIN = 0.96, PIECES_GAIN = 0.96;
+constexpr double SHAPE_GAIN = 0.9735, PIECES_GAIN = 0.9931;
 // Bytes per microsecond of pieces, or of the updated stream, on their way into the norm behind the product, and what every
-// piece takes there besides (writing them is hidden in the times above).  Fitted to product and norm together, 176 sizes of 130
-// to 2,627 rows in one to eight pieces, and to whole prompts, whose weights are cold: 300 x 2,048 x 2,048 takes
-// 18.4 us in four pieces and 21.3 in eight, 256 x 4,096 x 4,096 24.3 and 28.7, 700 x 1,024 x 1,024 14.9 in two and 17.0 in four.
+// piece takes there besides (writing them is hidden in the times above).  Of 21 sizes of product and norm measured together,
+// 130 to 2,627 rows in one to eight pieces with cold weights, the choice is 1.4 % above the best in the mean (the numbers above are
+// moved inside the fit's error so that it is):
+// 300 x 2,048 x 8,192 takes 68 us in one piece, 28.2 in five and 29.5 in eight, 256 x 4,096 x 4,096 48, 25.7 in three and 28.5.
 // Rows of more than 4,096 columns go through the norm at half that rate (1,267 x 5,376 x 4,544: 104 us in one piece, 175 in two).
-constexpr double PIECES_READ = 4e6, WIDE_READ = 2e6, PIECE_US = 0.3;
+constexpr double PIECES_READ = 6.869e6, WIDE_READ = PIECES_READ / 2, PIECE_US = 0.426;
 constexpr int WIDE = 4096;
 
 inline double shape_us(const Shape& s, int M, int N, int K, int splits, int units) {
@@ -44,7 +51,14 @@ inline double shape_us(const Shape& s, int M, int N, int K, int splits, int unit
   const double top = s.full[0] + s.full[1] * k;
   double low = s.alone[0] + s.alone[1] * k + s.alone[2] * k * k;
   if (low > top) low = top;
-  return rounds * top + (rest ? low + (top - low) * rest / slots : 0.0);
+  if (!rest) return rounds * top;
+  // where a unit holds two blocks, the units that have two decide
+  const double share = s.slots > 1 ? std::sqrt((double)rest / slots) : (double)rest / slots;
+  return rounds * top + low + (top - low) * share;
+}
+
+inline bool ring_128_takes(int M, int N, int K, int splits, int units) {
+  return K % SLAB == 0 && shape_us(RING_128, M, N, K, splits, units) < shape_us(SHAPES[0], M, N, K, splits, units);
 }
 
 struct Choice {
@@ -53,7 +67,7 @@ struct Choice {
 };
 // The shape that takes the least time for the product in `splits` pieces, and that time.
 inline Choice shape_for(int M, int N, int K, int splits, int units) {
-  Choice best{0, shape_us(SHAPES[0], M, N, K, splits, units)};
+  Choice best{0, shape_us(ring_128_takes(M, N, K, splits, units) ? RING_128 : SHAPES[0], M, N, K, splits, units)};
   if (K % SLAB) return best;
   for (const Shape& s : SHAPES) {
     if (s.code == 0) continue;

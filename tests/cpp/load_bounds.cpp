@@ -5,7 +5,7 @@
 //
 // Walks the built-in sweep of shapes (and any given as arguments) through the lanes, waves,
 // blocks and steps of gemm_skinny_kernel, gemm_skinny_shared_kernel, gemm_mfma_kernel,
-// gemm_mfma_big_kernel in its five tile shapes, gemm_float32_rows_kernel and gemm_float32_tile_kernel exactly as the kernels
+// gemm_mfma_big_kernel in its six tile shapes, gemm_float32_rows_kernel and gemm_float32_tile_kernel exactly as the kernels
 // walk them (and, in the built-in sweep, through the
 // key and value fetches of the attention kernels' chunks for every head size and several page sizes), with the matrices row by row (several row
 // strides) and, where the sizes allow, in the weight-streaming kernels' tiled order.  Prints
@@ -219,8 +219,9 @@ static bool tiles(const Shape& s, long lda, long ldw, const Tiles& t, int per) {
 }
 static const Tiles BFLOAT16_TILES[] = {
     {"gemm_mfma", 128, 128, 4, false, 0},              // asks for existing slabs only
-    {"gemm_mfma_big<4, 2>", 256, 256, 8, true, 2}, {"gemm_mfma_big<3, 3>", 192, 384, 8, true, 2}, {"gemm_mfma_big<3, 2>", 192, 256, 8, true, 2},
-    {"gemm_mfma_big<2, 3>", 128, 384, 8, true, 2}, {"gemm_mfma_big<2, 2>", 128, 256, 8, true, 2},
+    // the larger tiles: as many slabs past the last as their rings of buffers hold
+    {"gemm_mfma_big<4, 2>", 256, 256, 8, true, 3}, {"gemm_mfma_big<3, 3>", 192, 384, 8, true, 2}, {"gemm_mfma_big<3, 2>", 192, 256, 8, true, 3},
+    {"gemm_mfma_big<2, 3>", 128, 384, 8, true, 2}, {"gemm_mfma_big<2, 2>", 128, 256, 8, true, 3}, {"gemm_mfma_big<2, 1>", 128, 128, 8, true, 3},
 };
 static const Tiles FLOAT32_TILES[] = {                 // the rings of buffers, less the one in use
     {"gemm_float32_tile<128, 128>", 128, 128, 4, false, 1}, {"gemm_float32_tile<128, 64>", 128, 64, 4, false, 2}, {"gemm_float32_tile<64, 64>", 64, 64, 4, false, 3},

@@ -316,7 +316,7 @@ def test_gemm_with_swiglu_on_large_tiles(_ops, M, I, K):
     close(out, want, 2 ** -7, "fused swiglu on large tiles")
 
 
-@pytest.mark.parametrize("shape", [0, 42, 33, 32, 23, 22])
+@pytest.mark.parametrize("shape", [0, 42, 33, 32, 23, 22, 21])
 @pytest.mark.parametrize("M,N,K", [(129, 96, 64), (193, 512, 192), (257, 800, 320), (640, 1184, 448)])
 def test_every_tile_shape_at_its_edges(_ops, monkeypatch, shape, M, N, K):
     """Each block tile with one row more than it holds, columns that end inside a wave's corner, and one slab of k up to
