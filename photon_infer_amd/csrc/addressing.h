@@ -77,22 +77,6 @@ PI_ADDR bool skinny_w_used(bool whole, int kk, int h, int lg, int k1) { return w
 PI_ADDR long skinny_x_base(int token, int M, long ldx, int xp) { return (long)imin(token, M - 1) * ldx + xp * 8; }
 PI_ADDR long skinny_x_step(bool whole, int kk, int xp, int k0, int k1) { return (whole || kk + xp * 8 < k1) ? kk : k0 - xp * 8; }
 
-// ---------------------------------------------------------------- gemm_skinny_shared_kernel (33..128 tokens)
-// A block's waves take 16 rows each over the block's whole k-range [kb0, kb1) in steps of 64;
-// steps beyond the last are fetched again (never used) so that every step issues the same loads.
-PI_ADDR int shared_steps(int kb0, int kb1) { return (kb1 - kb0 + KSTEP - 1) / KSTEP; }
-PI_ADDR int shared_k_of(int kb0, int steps, int s) { return kb0 + imin(s, steps - 1) * KSTEP; }
-PI_ADDR long shared_w_base(int tiled, long n0, int wave, int lr, int lg, int N, int K, long ldw) {
-  return tiled ? lmin(n0 / 16 + wave, (long)N / 16 - 1) * (K / 64) * 1024 + lg * 128 + lr * 8
-               : lmin(n0 + wave * 16 + lr, (long)N - 1) * ldw;
-}
-// a piece beyond the range is fetched from the range's last 8 elements
-PI_ADDR long shared_w_step(int tiled, int kk, int h, int lg, int kb1) {
-  return tiled ? (long)kk * 16 + h * 512 : (long)imin(kk + lg * 16 + h * 8, kb1 - 8);
-}
-PI_ADDR long shared_x_base(int token, int M, long ldx) { return (long)imin(token, M - 1) * ldx; }
-PI_ADDR long shared_x_step(int kk, int xp, int kb1) { return imin(kk + xp * 8, kb1 - 8); }
-
 // ---------------------------------------------------------------- tile kernels (buffer descriptors)
 // A block's operand is read through a buffer descriptor: a base (the block's first row at its
 // first k) and a byte length; a lane's byte offset at or beyond the length reads zeros.  The
@@ -122,6 +106,22 @@ PI_ADDR unsigned big_lane_offset(int row, int rows, long ld, int piece) {
   return (unsigned)(imin(row, rows - 1) * (int)ld + piece * 8) * 2u;
 }
 PI_ADDR int big_slab_bytes(int s, int slabs) { return imin(s, slabs - 1) * 64 * 2; }   // past the last slab: read it again, unused
+
+// ---------------------------------------------------------------- gemm_skinny_ring_kernel (33..128 tokens)
+// Through descriptors too, the activations as a tile of up to 128 rows (above) and 64 weight rows: as a tile, or, `tiled`, from
+// the copy [N / 16][K / 64][2][4][16][8], of which 16 rows x 64 k are 1,024 elements in a row.  k is a multiple of 64 there.
+PI_ADDR Descriptor ring_w_descriptor(int tiled, long n0, int k_lo, int k_hi, int rows, int K, long ldw) {
+  if (!tiled) return tile_descriptor(n0, ldw, k_lo, k_hi, rows);
+  return Descriptor{n0 * K + (long)k_lo * 16, ((long)(rows / 16 - 1) * K * 16 + (long)(k_hi - k_lo) * 16) * 2};
+}
+// piece: which 8 of a step's 64 k
+PI_ADDR unsigned ring_w_lane_offset(int tiled, int row, int rows, int K, long ldw, int piece) {
+  if (!tiled) return tile_lane_offset(row, rows, ldw, piece);
+  return row < rows ? (unsigned)(row / 16 * K * 16 + (piece % 2) * 512 + (piece / 2) * 128 + (row % 16) * 8) * 2u : OUT_OF_RANGE;
+}
+PI_ADDR unsigned ring_w_step_offset(int tiled, unsigned lane_offset, int k0, int piece, int k_range) {
+  return k0 + piece * 8 < k_range ? lane_offset + (unsigned)k0 * (tiled ? 32u : 2u) : OUT_OF_RANGE;
+}
 
 // ---------------------------------------------------------------- attention over the paged cache
 // Keys [pages, kv_heads, page, HD], values transposed [pages, kv_heads, HD, page], bfloat16.  A

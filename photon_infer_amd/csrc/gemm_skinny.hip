@@ -25,7 +25,7 @@ enum { EPI_BF16 = 0, EPI_F32 = 1, EPI_ACCUM = 2, EPI_SWIGLU = 3 };
 #define RANGES_ROW_TILES 4      // row tiles per wave where the key ranges are merged on the way in (fewer blocks repeat the merge)
 #define KSTEP addressing::KSTEP
 #define SHARED_FROM_TOKENS 32   // more tokens than this: the kernel that shares an activation tile per block
-#define SHARED_DEPTH 4          // k steps of loads a wave keeps in flight (measured: more is slower)
+#define RING_MAX_STRIDE (1L << 21)  // elements between rows, and of k, up to which that kernel's byte offsets fit 31 bits
 
 template <int EPI>
 __device__ inline void epilogue_store(void* Cv, long ldc, long m, long n, float v) {
@@ -281,135 +281,143 @@ __global__ __launch_bounds__(256) void gemm_skinny_kernel(void* __restrict__ Cv,
   }
 }
 
-// The same product for 33..128 tokens, where the activations are as many bytes as a block's
-// weights: the four waves of a block take 16 weight rows each over the block's whole k-range
-// and share one activation tile per k step through LDS (loaded once per block, not once per
-// wave).  A block is alone on its compute unit, so every wave keeps DEPTH k steps of loads
-// (weights and its share of the activation tile) in flight in registers; loads return in
-// order, which is why both travel at the same distance.
-#define SHARED_ROWS_PER_BLOCK 64
+// The same product for 33..128 tokens, where the activations are as many bytes as a block's weights.  A block is eight waves
+// on 64 weight rows: wave w multiplies rows 32 (w / 4) .. + 31 with T tiles of 32 tokens (v_mfma_f32_32x32x16_bf16), and of
+// every step of 64 k takes the 16 of its quarter w % 4; the quarters are summed through LDS at the end.  So a step's
+// activations are read from LDS twice and not once per 16 rows, and the weights go into registers past LDS.  Activations go
+// from memory straight into a ring of buffers; both are asked for four steps ahead (eight: 2,048 x 8,192, 64 tokens 13.5 us
+// instead of 11.6).  The one barrier per step waits for
+// the loads that the step needs, not for those behind them.  Steps beyond the block's k, tokens beyond M and rows beyond N
+// take offsets outside the descriptors: zeros, and no bytes.
+// Bound by the weights' way from memory and, towards 128 tokens, by the activations' from L2.  In place of four waves of 16
+// rows each that staged the activations through registers, at 33 / 64 / 100 / 128 tokens, weights from memory in the copy's
+// order: 16,384 x 2,048 16.2 / 18.6 / 23.6 / 23.7 us -> 15.5 / 16.9 / 19.1 / 21.3, 2,048 x 8,192 in eight pieces 10.7 / 12.2 /
+// 16.0 / 16.6 -> 10.8 / 11.6 / 13.7 / 14.8, 6,144 x 4,096 17.1 / 19.9 / 26.4 / 28.3 in three pieces -> 15.0 / 15.7 / 18.7 / 20.1
+// in two, 28,672 x 4,096 51 / 56 / 68 / 73 -> 49 / 53 / 62 / 66.
+#define RING_ROWS 64
+#define RING_BUFFERS 5
 
-template <int MB, int EPI, int DEPTH>
-__global__ __launch_bounds__(256) void gemm_skinny_shared_kernel(void* __restrict__ Cv, long ldc, const bf16_t* __restrict__ X, long ldx,
-                                                                 const bf16_t* __restrict__ W, long ldw, int M, int N, int K,
-                                                                 int k_per_block, float* __restrict__ part, int tiled) {
-  constexpr int ROWS = SHARED_ROWS_PER_BLOCK;
-  constexpr int XL = (MB + 1) / 2;      // 16-byte pieces of an activation tile per lane
-  __shared__ union {
-    u32x4_t xs[2][MB * 128];            // [token tile][piece of the k step][token], tokens turned by the piece
-    float tile[ROWS][MB * 16 + 1];
-  } lds;
-  const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
-  const int lr = lane % 16, lg = lane / 16;
-  const long n0 = (long)blockIdx.x * ROWS;
+template <int T, int EPI>
+__global__ __launch_bounds__(512, 4) void gemm_skinny_ring_kernel(void* __restrict__ Cv, long ldc, const bf16_t* __restrict__ X, long ldx,
+                                                               const bf16_t* __restrict__ W, long ldw, int M, int N, int K,
+                                                               int k_per_block, float* __restrict__ part, int tiled) {
+  constexpr int XROWS = T == 2 ? 64 : 128, XI = XROWS / 64;        // rows of a buffer, load instructions of a wave per step
+  constexpr int NB = RING_BUFFERS, AHEAD = NB - 1, TOKENS = T * 32, PITCH = TOKENS + 1;
+  extern __shared__ __attribute__((aligned(16))) uint16_t lds[];   // [NB][XROWS][64], 16-byte pieces of a row turned by (row / 2) % 8
+  const int tid = threadIdx.x, lane = tid % 64;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+  const int rows32 = wave / 4, quarter = wave % 4;
+  const long n0 = (long)blockIdx.x * RING_ROWS;
   const int splits = gridDim.y;
-  const int kb0 = blockIdx.y * k_per_block;
-  const int kb1 = min(K, kb0 + k_per_block);
-  const int steps = addressing::shared_steps(kb0, kb1);
-  auto k_of = [&](const int s) { return addressing::shared_k_of(kb0, steps, s); };   // steps beyond the last are fetched, never used
-
-  // rows beyond N and tokens beyond M read the last valid one; their results are never stored
-  const bf16_t* wrow = W + addressing::shared_w_base(tiled, n0, wave, lr, lg, N, K, ldw);     // see gemm_skinny_kernel
-  const int xp = tid % 8;
-  const bf16_t* xsrc[XL];
-  int xdst[XL];
-  bool xmine[XL];
+  const int k_lo = blockIdx.y * k_per_block, k_hi = min(K, k_lo + k_per_block), k_range = k_hi - k_lo;
+  const int w_rows = (int)min((long)RING_ROWS, N - n0);
+#if defined(__HIP_DEVICE_COMPILE__)
+  const __amdgpu_buffer_rsrc_t x_src = operand_descriptor(X, addressing::tile_descriptor(0, ldx, k_lo, k_hi, M));
+  const __amdgpu_buffer_rsrc_t w_src = operand_descriptor(W, addressing::ring_w_descriptor(tiled, n0, k_lo, k_hi, w_rows, K, ldw));
+#endif
+  unsigned x_off[XI];
+  int x_piece[XI];
 #pragma unroll
-  for (int i = 0; i < XL; ++i) {
-    const int token = i * 32 + tid / 8;
-    xsrc[i] = X + addressing::shared_x_base(token, M, ldx);
-    xdst[i] = ((token / 16) * 8 + xp) * 16 + ((token + 2 * xp) & 15);
-    xmine[i] = token < MB * 16;
+  for (int p = 0; p < XI; ++p) {
+    const int row = (p * 8 + wave) * 8 + lane / 8;
+    x_piece[p] = addressing::tile_piece(lane, row);
+    x_off[p] = addressing::tile_lane_offset(row, M, ldx, x_piece[p]);
   }
-  int xfrag[MB][2];
-#pragma unroll
-  for (int c = 0; c < MB; ++c)
-#pragma unroll
-    for (int h = 0; h < 2; ++h) xfrag[c][h] = (c * 8 + lg * 2 + h) * 16 + ((lr + 2 * (lg * 2 + h)) & 15);
+  const int frow = lane % 32, piece = quarter * 2 + lane / 32;     // a fragment: row (token) frow, the 8 k of the piece
+  const unsigned w_off = addressing::ring_w_lane_offset(tiled, rows32 * 32 + frow, w_rows, K, ldw, piece);
+  const int place = (piece ^ ((frow >> 1) & 7)) * 8;
 
-  f32x4_t acc[MB];
+  Frag wq[AHEAD];
+  auto fetch_x = [&](const int s, const int buf) {
+#if defined(__HIP_DEVICE_COMPILE__)
 #pragma unroll
-  for (int c = 0; c < MB; ++c) acc[c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int p = 0; p < XI; ++p)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(x_src, (lds_ptr_t)(lds + (buf * XROWS + (p * 8 + wave) * 8) * KSTEP), 16,
+                                               addressing::tile_slab_offset(x_off[p], s * KSTEP, x_piece[p], k_range), 0, 0, 0);
+#endif
+  };
+  auto fetch_w = [&](const int s, const int j) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    wq[j].n = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(w_src, addressing::ring_w_step_offset(tiled, w_off, s * KSTEP, piece, k_range), 0, 0));
+#endif
+  };
 
-  Frag wq[DEPTH][2];
-  u32x4_t xq[DEPTH][XL];
-  // every step issues the same loads, also beyond the range (clamped, never used): the count
-  // of loads in flight is then a constant the compiler can wait on exactly
-  auto fetch = [&](const int s, const int j) {
-    const int kk = k_of(s);
+  f32x16_t acc[T];
 #pragma unroll
-    for (int i = 0; i < XL; ++i) xq[j][i] = *reinterpret_cast<const u32x4_t*>(xsrc[i] + addressing::shared_x_step(kk, xp, kb1));
+  for (int c = 0; c < T; ++c)
 #pragma unroll
-    for (int h = 0; h < 2; ++h) wq[j][h] = load_frag(wrow + addressing::shared_w_step(tiled, kk, h, lg, kb1));
-  };
-#pragma unroll
-  for (int j = 0; j < DEPTH; ++j) fetch(j, j);
+    for (int v = 0; v < 16; ++v) acc[c][v] = 0.f;
 
-  // the tile of step s + 1 goes to LDS (the other of two buffers) before step s computes, so
-  // that the one barrier per step finds every wave's writes long done
-  auto stage = [&](const int s, const int j) {
-    const bool x_ok = k_of(s) + xp * 8 < kb1;          // 8-element pieces beyond the range count as zero
-    u32x4_t* xs = lds.xs[s & 1];
+  const int steps = (k_range + KSTEP - 1) / KSTEP;
 #pragma unroll
-    for (int i = 0; i < XL; ++i)
-      if (xmine[i]) xs[xdst[i]] = x_ok ? xq[j][i] : u32x4_t{0u, 0u, 0u, 0u};
-  };
-  auto step = [&](const int s, const int j, auto more_to_fetch) {
-    const int kk = k_of(s);
-    stage(s + 1, (j + 1) % DEPTH);
-    const u32x4_t* xs = lds.xs[s & 1];
-    Frag x[MB][2], w[2];
-#pragma unroll
-    for (int c = 0; c < MB; ++c)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) x[c][h].n = xs[xfrag[c][h]];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) w[h].n = kk + lg * 16 + h * 8 < kb1 ? wq[j][h].n : u32x4_t{0u, 0u, 0u, 0u};
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int c = 0; c < MB; ++c) acc[c] = mfma16(w[h], x[c][h], acc[c]);
-    if (decltype(more_to_fetch)::value) fetch(s + DEPTH, j);
-    __syncthreads();
-  };
-  stage(0, 0);
-  __syncthreads();
-  // whole rounds of DEPTH steps have no branch, so that the waits stay exact; the last steps
-  // fetch nothing more
-  int s0 = 0;
-  for (; s0 + DEPTH <= steps; s0 += DEPTH) {
-#pragma unroll
-    for (int j = 0; j < DEPTH; ++j) step(s0 + j, j, std::true_type{});
+  for (int j = 0; j < AHEAD; ++j) {
+    fetch_x(j, j);
+    fetch_w(j, j);
+    __builtin_amdgcn_sched_barrier(0);      // in this order: the waits in the loop count on it
   }
+  int buf = 0;
+  auto step = [&](const int s, const int j) {
+    // step s has landed for every wave, and everybody has left the buffer of step s - 1
+    block_barrier_keeping_loads<(AHEAD - 1) * (XI + 1)>();
+    const uint16_t* x_base = lds + (buf * XROWS + frow) * KSTEP + place;
+    Frag x[T];
 #pragma unroll
-  for (int j = 0; j < DEPTH; ++j)
-    if (s0 + j < steps) step(s0 + j, j, std::false_type{});
-  // (the last step ended with a barrier: the result tile may take the place of the activation tiles)
-
-  // acc[c][r] is C^T[n0 + wave*16 + lg*4 + r][c*16 + lr]
+    for (int c = 0; c < T; ++c) x[c].n = *reinterpret_cast<const u32x4_t*>(x_base + c * 32 * KSTEP);
+    fetch_x(s + AHEAD, buf == 0 ? NB - 1 : buf - 1);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int c = 0; c < MB; ++c)
+    for (int c = 0; c < T; ++c) acc[c] = mfma32(wq[j], x[c], acc[c]);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch_w(s + AHEAD, j);                  // behind the last use of the registers it fills: in others the loop ends with copies
+    buf = buf == NB - 1 ? 0 : buf + 1;
+  };
+  // Whole rounds of AHEAD steps without a branch, the last steps perhaps beyond the range (zeros): with one the compiler moves
+  // the weights in flight to other registers, and waits for all of them
+  for (int s0 = 0; s0 < steps; s0 += AHEAD) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) lds.tile[wave * 16 + lg * 4 + r][c * 16 + lr] = acc[c][r];
+    for (int j = 0; j < AHEAD; ++j) step(s0 + j, j);
+  }
+  __builtin_amdgcn_s_waitcnt(0x0F70);       // nothing may still be on its way into LDS when the sums take it over
   __syncthreads();
 
-  const int cols = MB * 16;
+  // acc[c][v] is C^T[n0 + rows32*32 + 8*(v/4) + 4*(lane/32) + v%4][c*32 + lane%32], a quarter of it: quarters 2 and 3 hand
+  // theirs to 0 and 1, and what is left are two tiles [64][TOKENS] to be added
+  float* red = reinterpret_cast<float*>(lds);
+  auto at = [&](const int c, const int v) {
+    return ((quarter % 2) * RING_ROWS + rows32 * 32 + 8 * (v / 4) + 4 * (lane / 32) + v % 4) * PITCH + c * 32 + frow;
+  };
+  if (quarter >= 2) {
+#pragma unroll
+    for (int c = 0; c < T; ++c)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) red[at(c, v)] = acc[c][v];
+  }
+  __syncthreads();
+  if (quarter < 2) {
+#pragma unroll
+    for (int c = 0; c < T; ++c)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) red[at(c, v)] += acc[c][v];
+  }
+  __syncthreads();
+  auto total = [&](const int n, const int m) { return red[n * PITCH + m] + red[(RING_ROWS + n) * PITCH + m]; };
+
   if (splits == 1 && EPI == EPI_SWIGLU) {
     // rows [gate 16 | up 16 | gate 16 | up 16]: 32 features per block
-    for (int idx = tid; idx < 32 * cols; idx += 256) {
+    for (int idx = tid; idx < 32 * M; idx += 512) {
       const int j = idx % 16, pair = (idx / 16) % 2, m = idx / 32;
-      if (m >= M || n0 + pair * 32 + 16 + j >= N) continue;
-      const float g = lds.tile[pair * 32 + j][m], u = lds.tile[pair * 32 + 16 + j][m];
+      if (n0 + pair * 32 + 16 + j >= N) continue;
+      const float g = total(pair * 32 + j, m), u = total(pair * 32 + 16 + j, m);
       reinterpret_cast<bf16_t*>(Cv)[(long)m * ldc + n0 / 2 + pair * 16 + j] = from_float<bf16_t>(g / (1.0f + expf(-g)) * u);
     }
     return;
   }
   float* mine = part + (long)blockIdx.y * M * N;
-  for (int idx = tid; idx < ROWS * cols; idx += 256) {
-    const int nl = idx % ROWS, m = idx / ROWS;
-    if (m >= M || n0 + nl >= N) continue;
-    if (splits == 1) epilogue_store<EPI>(Cv, ldc, m, n0 + nl, lds.tile[nl][m]);
-    else mine[(long)m * N + n0 + nl] = lds.tile[nl][m];   // the consumer adds the splits in split order
+  for (int idx = tid; idx < RING_ROWS * M; idx += 512) {
+    const int nl = idx % RING_ROWS, m = idx / RING_ROWS;
+    if (n0 + nl >= N) continue;
+    if (splits == 1) epilogue_store<EPI>(Cv, ldc, m, n0 + nl, total(nl, m));
+    else mine[(long)m * N + n0 + nl] = total(nl, m);   // the consumer adds the splits in split order
   }
 }
 
@@ -428,23 +436,32 @@ static int launch_mb(int epi, dim3 grid, hipStream_t stream, void* C, long ldc, 
   return pi_check_launch("gemm_skinny");
 }
 
-template <int MB>
-static int launch_shared(int epi, dim3 grid, hipStream_t stream, void* C, long ldc, const bf16_t* X, long ldx, const bf16_t* W,
-                         long ldw, int M, int N, int K, int kpb, float* part, int tiled) {
-#define GO(E) hipLaunchKernelGGL((gemm_skinny_shared_kernel<MB, E, SHARED_DEPTH>), grid, dim3(256), 0, stream, C, ldc, X, ldx, W, ldw, M, N, K, kpb, part, tiled)
+template <int T, int EPI>
+static int launch_ring_of(dim3 grid, hipStream_t stream, void* C, long ldc, const bf16_t* X, long ldx, const bf16_t* W, long ldw, int M, int N, int K,
+                          int kpb, float* part, int tiled) {
+  constexpr size_t ring = RING_BUFFERS * (T == 2 ? 64 : 128) * KSTEP * sizeof(uint16_t), sums = 2 * RING_ROWS * (T * 32 + 1) * sizeof(float);
+  constexpr size_t bytes = ring > sums ? ring : sums;        // at most 80 KB: two blocks to a unit
+  static const hipError_t configured = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_skinny_ring_kernel<T, EPI>),
+                                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+  if (configured != hipSuccess) return pi_fail("gemm_skinny: cannot reserve %zu bytes of LDS: %s", bytes, hipGetErrorString(configured));
+  hipLaunchKernelGGL((gemm_skinny_ring_kernel<T, EPI>), grid, dim3(512), bytes, stream, C, ldc, X, ldx, W, ldw, M, N, K, kpb, part, tiled);
+  return pi_check_launch("gemm_skinny (rings)");
+}
+
+template <int T>
+static int launch_ring(int epi, dim3 grid, hipStream_t stream, void* C, long ldc, const bf16_t* X, long ldx, const bf16_t* W, long ldw, int M, int N,
+                       int K, int kpb, float* part, int tiled) {
   switch (epi) {
-    case EPI_BF16: GO(EPI_BF16); break;
-    case EPI_F32: GO(EPI_F32); break;
-    case EPI_ACCUM: GO(EPI_ACCUM); break;
-    case EPI_SWIGLU: GO(EPI_SWIGLU); break;
-    default: return pi_fail("gemm_skinny: unknown epilogue %d", epi);
+    case EPI_BF16: return launch_ring_of<T, EPI_BF16>(grid, stream, C, ldc, X, ldx, W, ldw, M, N, K, kpb, part, tiled);
+    case EPI_F32: return launch_ring_of<T, EPI_F32>(grid, stream, C, ldc, X, ldx, W, ldw, M, N, K, kpb, part, tiled);
+    case EPI_ACCUM: return launch_ring_of<T, EPI_ACCUM>(grid, stream, C, ldc, X, ldx, W, ldw, M, N, K, kpb, part, tiled);
+    case EPI_SWIGLU: return launch_ring_of<T, EPI_SWIGLU>(grid, stream, C, ldc, X, ldx, W, ldw, M, N, K, kpb, part, tiled);
   }
-#undef GO
-  return pi_check_launch("gemm_skinny (shared activations)");
+  return pi_fail("gemm_skinny: unknown epilogue %d", epi);
 }
 
 // Rows of the weight matrix per block for M tokens (the caller sizes its k-split by it).
-extern "C" int pi_gemm_skinny_rows_per_block(int M) { return M > SHARED_FROM_TOKENS ? SHARED_ROWS_PER_BLOCK : ROWS_PER_BLOCK; }
+extern "C" int pi_gemm_skinny_rows_per_block(int M) { return M > SHARED_FROM_TOKENS ? RING_ROWS : ROWS_PER_BLOCK; }
 
 // splits > 1: the partial products go to `part` (float32 [splits, M, N]) and C is not touched;
 // *splits_out tells how many splits were made (no empty ones).
@@ -473,18 +490,14 @@ extern "C" int pi_gemm_skinny(void* C, int epilogue, long ldc, const void* X, lo
   const int mb = (M + 15) / 16;
   const bf16_t *x = (const bf16_t*)X, *w = (const bf16_t*)W;
   if (M > SHARED_FROM_TOKENS) {
-#define SHARED(B) case B: return launch_shared<B>(epilogue, grid, stream, C, ldc, x, ldx, w, ldw, M, N, K, kpb, (float*)part, tiled)
-    switch (mb) {
-      SHARED(3); SHARED(4); SHARED(5); SHARED(6); SHARED(7);
-      default: return launch_shared<8>(epilogue, grid, stream, C, ldc, x, ldx, w, ldw, M, N, K, kpb, (float*)part, tiled);
-    }
-#undef SHARED
+    PI_REQUIRE(ldx < RING_MAX_STRIDE && ldw < RING_MAX_STRIDE && K < RING_MAX_STRIDE, "gemm_skinny: K (%d) or row strides (%ld, %ld) are too long for 32-bit offsets", K, ldx, ldw);
+    if (M <= 64) return launch_ring<2>(epilogue, grid, stream, C, ldc, x, ldx, w, ldw, M, N, K, kpb, (float*)part, tiled);
+    if (M <= 96) return launch_ring<3>(epilogue, grid, stream, C, ldc, x, ldx, w, ldw, M, N, K, kpb, (float*)part, tiled);
+    return launch_ring<4>(epilogue, grid, stream, C, ldc, x, ldx, w, ldw, M, N, K, kpb, (float*)part, tiled);
   }
   switch (mb) {
     case 1: return launch_mb<1>(epilogue, grid, stream, C, ldc, x, ldx, w, ldw, M, N, K, kpb, (float*)part, tiled);
-    case 2: return launch_mb<2>(epilogue, grid, stream, C, ldc, x, ldx, w, ldw, M, N, K, kpb, (float*)part, tiled);
-    case 3: return launch_mb<3>(epilogue, grid, stream, C, ldc, x, ldx, w, ldw, M, N, K, kpb, (float*)part, tiled);
-    default: return launch_mb<4>(epilogue, grid, stream, C, ldc, x, ldx, w, ldw, M, N, K, kpb, (float*)part, tiled);
+    default: return launch_mb<2>(epilogue, grid, stream, C, ldc, x, ldx, w, ldw, M, N, K, kpb, (float*)part, tiled);
   }
 }
 

@@ -31,8 +31,9 @@ SKINNY_MAX_ROWS = 128          # up to this many tokens the weight-streaming ker
 ROWS_PER_BLOCK = 32            # weight rows per block of the skinny kernel
 BLOCKS_PER_UNIT = 2            # blocks of it wanted per compute unit to keep HBM busy (measured: 512 on 256 units; 384 and 768 are slower)
 SHARED_FROM_TOKENS = 32        # more tokens than this: the skinny kernel that shares activations per block ...
-SHARED_ROWS_PER_BLOCK = 64     # ... with this many weight rows per block ...
-SHARED_BLOCKS_PER_UNIT = 1     # ... and one block wanted per compute unit
+SHARED_ROWS_PER_BLOCK = 64     # ... with this many weight rows per block, and no more blocks than compute units (100 tokens, 3,072 x 8,192:
+                               # 22.8 us in six pieces on 288 blocks, 16.9 in five on 240; 6,144 x 4,096 22.8 in three, 18.7 in two)
+RING_MAX_STRIDE = 1 << 21      # elements between rows up to which that kernel's byte offsets fit 31 bits
 FLOAT32_MAX_STRIDE = 1 << 21   # floats between rows up to which the float32 kernels' offsets inside a tile fit 32 bits
 DEFAULT_UNITS = 256            # compute units assumed where no device can be asked (an MI355X)
 PIECES_WORTH = 0.95            # q, k, v of a prompt portion are left in k pieces too where that takes no more than this share of the time:
@@ -73,16 +74,17 @@ def compute_units() -> int:
 
 
 def _gemm_ok(a, w, K, lda, ldw) -> bool:
-    return K % 8 == 0 and lda % 8 == 0 and ldw % 8 == 0 and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+    return (K % 8 == 0 and lda % 8 == 0 and ldw % 8 == 0 and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and not (SHARED_FROM_TOKENS < a.shape[0] <= SKINNY_MAX_ROWS and max(lda, ldw) >= RING_MAX_STRIDE))
 
 
 def _skinny_splits(M: int, N: int, K: int) -> int:
     units = compute_units()
-    if M > SHARED_FROM_TOKENS:     # the kernel that shares an activation tile per block: one block per compute unit
-        groups, wanted = -(-N // SHARED_ROWS_PER_BLOCK), SHARED_BLOCKS_PER_UNIT * units
+    if M > SHARED_FROM_TOKENS:     # the kernel that shares an activation tile per block: at most one block per compute unit
+        splits = units // -(-N // SHARED_ROWS_PER_BLOCK)
     else:
-        groups, wanted = -(-N // ROWS_PER_BLOCK), BLOCKS_PER_UNIT * units
-    splits = max(1, min(-(-wanted // groups), K // 256))
+        splits = -(-BLOCKS_PER_UNIT * units // -(-N // ROWS_PER_BLOCK))
+    splits = max(1, min(splits, K // 256))
     while splits > 1 and splits * M * N > GEMM_PART_FLOATS:
         splits -= 1
     return splits

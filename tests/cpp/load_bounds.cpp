@@ -4,7 +4,7 @@
 //   load_bounds [old-standin] [only] [M N K splits]...
 //
 // Walks the built-in sweep of shapes (and any given as arguments) through the lanes, waves,
-// blocks and steps of gemm_skinny_kernel, gemm_skinny_shared_kernel, gemm_mfma_kernel,
+// blocks and steps of gemm_skinny_kernel, gemm_skinny_ring_kernel, gemm_mfma_kernel,
 // gemm_mfma_big_kernel in its six tile shapes, gemm_float32_rows_kernel and gemm_float32_tile_kernel exactly as the kernels
 // walk them (and, in the built-in sweep, through the
 // key and value fetches of the attention kernels' chunks for every head size and several page sizes), with the matrices row by row (several row
@@ -83,42 +83,6 @@ static bool skinny(const Shape& s, long ldx, long ldw, int tiled, int RT, int qu
           }
         }
       }
-  return true;
-}
-
-// ------------------------------------------------------------------ 33..128 tokens
-static bool shared(const Shape& s, long ldx, long ldw, int tiled, int depth) {
-  const int M = s.M, N = s.N, K = s.K;
-  const A::KSplit cut = A::cut_k(K, s.splits, A::KSTEP);
-  const int MB = (M + 15) / 16, XL = (MB + 1) / 2;
-  const int groups = (N + 63) / 64;
-  for (int by = 0; by < cut.splits; ++by) {
-    const int kb0 = by * cut.k_per_block, kb1 = A::imin(K, kb0 + cut.k_per_block);
-    const int steps = A::shared_steps(kb0, kb1);
-    for (int bx = 0; bx < groups; ++bx)
-      for (int tid = 0; tid < 256; ++tid) {
-        const int wave = tid / 64, lane = tid % 64, lr = lane % 16, lg = lane / 16, xp = tid % 8;
-        const long n0 = (long)bx * 64;
-        for (int st = 0; st < steps + depth; ++st) {
-          const int kk = A::shared_k_of(kb0, steps, st);
-          for (int h = 0; h < 2; ++h) {
-            const long off = A::shared_w_base(tiled, n0, wave, lr, lg, N, K, ldw) + A::shared_w_step(tiled, kk, h, lg, kb1);
-            ++fetches;
-            if (tiled) {
-              if (off < 0 || off + 8 > (long)N * K) return fail("gemm_skinny_shared", "W", s, ldw, tiled, off, "outside the matrix");
-            } else if (!in_row(off, A::lmin(n0 + wave * 16 + lr, (long)N - 1), ldw, K)) {
-              return fail("gemm_skinny_shared", "W", s, ldw, tiled, off, "outside its row");
-            }
-          }
-          for (int i = 0; i < XL; ++i) {
-            const int token = i * 32 + tid / 8;
-            const long off = A::shared_x_base(token, M, ldx) + A::shared_x_step(kk, xp, kb1);
-            ++fetches;
-            if (!in_row(off, A::imin(token, M - 1), ldx, K)) return fail("gemm_skinny_shared", "X", s, ldx, tiled, off, "outside its row");
-          }
-        }
-      }
-  }
   return true;
 }
 
@@ -227,6 +191,46 @@ static const Tiles FLOAT32_TILES[] = {                 // the rings of buffers, 
     {"gemm_float32_tile<128, 128>", 128, 128, 4, false, 1}, {"gemm_float32_tile<128, 64>", 128, 64, 4, false, 2}, {"gemm_float32_tile<64, 64>", 64, 64, 4, false, 3},
 };
 
+// ------------------------------------------------------------------ 33..128 tokens
+// The activations are a tile of 64 or 128 rows; of the weights a block's eight waves take 32 rows by a quarter of each step's
+// k each.  A fetch that is used lies inside its descriptor, at the row and k that the fragment stands for, and any other
+// outside (it reads zeros).
+static bool ring(const Shape& s, long ldx, long ldw, int tiled) {
+  const A::KSplit cut = A::cut_k(s.K, s.splits, A::KSTEP);
+  const Tiles t{"gemm_skinny_ring", s.M <= 64 ? 64 : 128, 64, 8, false, 4};
+  for (int by = 0; by < cut.splits; ++by) {
+    const int k_lo = by * cut.k_per_block, k_hi = A::imin(s.K, k_lo + cut.k_per_block), k_range = k_hi - k_lo;
+    if (!tile_operand(t, "X", s, s.M, s.K, ldx, 0, t.rows_a, k_lo, k_hi)) return false;
+    const int steps = (k_range + 63) / 64, last = (steps + 3) / 4 * 4 + t.ahead;
+    for (long n0 = 0; n0 < s.N; n0 += 64) {
+      const int rows = (int)A::lmin(64, s.N - n0);
+      const A::Descriptor d = A::ring_w_descriptor(tiled, n0, k_lo, k_hi, rows, s.K, ldw);
+      const long operand_bytes = tiled ? (long)s.N * s.K * 2 : ((s.N - 1) * ldw + s.K) * 2;
+      if (d.base < 0 || d.bytes <= 0 || d.base * 2 + d.bytes > operand_bytes || d.bytes >= 0x7ffffff0L)
+        return fail(t.kernel, "W", s, ldw, tiled, d.base, "the descriptor leaves the operand");
+      for (int wave = 0; wave < 8; ++wave)
+        for (int lane = 0; lane < 64; ++lane) {
+          const int row = wave / 4 * 32 + lane % 32, piece = wave % 4 * 2 + lane / 32;
+          const unsigned lane_offset = A::ring_w_lane_offset(tiled, row, rows, s.K, ldw, piece);
+          for (int st = 0; st < last; ++st) {
+            ++fetches;
+            const long off = A::ring_w_step_offset(tiled, lane_offset, st * 64, piece, k_range);
+            const long k = k_lo + st * 64 + piece * 8;
+            if (row >= rows || k >= k_hi) {
+              if (off < d.bytes) return fail(t.kernel, "W", s, ldw, tiled, off, "a fetch that should read zeros lies inside the descriptor");
+              continue;
+            }
+            if (off + 16 > d.bytes) return fail(t.kernel, "W", s, ldw, tiled, off, "a used fetch leaves its descriptor");
+            const long n = n0 + row;
+            const long at = tiled ? (n / 16 * (s.K / 64) + k / 64) * 1024 + k % 16 / 8 * 512 + k % 64 / 16 * 128 + n % 16 * 8 : n * ldw + k;
+            if (d.base * 2 + off != at * 2) return fail(t.kernel, "W", s, ldw, tiled, off, "a used fetch is not the lane's row and k");
+          }
+        }
+    }
+  }
+  return true;
+}
+
 // ------------------------------------------------------------------ attention over the paged cache
 // Every fetch of a chunk's two tiles (attn_load): the keys' fragments (16 bytes) and the values'
 // (8 bytes) of every lane, for a page that is there, one that is missing and one whose id is no
@@ -285,7 +289,7 @@ static bool check(const Shape& s) {
       if (!skinny(s, ld, ld, 0, 2, A::KSTEP)) return false;
       if (s.M <= 16 && s.K % 64 == 0 && !skinny(s, ld, ld, 0, 4, 4 * A::KSTEP)) return false;     // the form that merges key ranges
     } else if (s.M <= 128) {
-      if (!shared(s, ld, ld, 0, 4)) return false;
+      if (!ring(s, ld, ld, 0)) return false;
     }
     for (const Tiles& t : BFLOAT16_TILES)
       if (!tiles(s, ld, ld, t, 1)) return false;
@@ -302,7 +306,7 @@ static bool check(const Shape& s) {
   if (s.N % 16 == 0 && s.K % 64 == 0) {                // the streaming copy of the weights
     if (s.M <= 32 && !skinny(s, s.K, s.K, 1, 2, A::KSTEP)) return false;
     if (s.M <= 16 && !skinny(s, s.K, s.K, 1, 4, 4 * A::KSTEP)) return false;
-    if (s.M > 32 && s.M <= 128 && !shared(s, s.K, s.K, 1, 4)) return false;
+    if (s.M > 32 && s.M <= 128 && !ring(s, s.K, s.K, 1)) return false;
   }
   return true;
 }
