@@ -15,7 +15,14 @@
 
 #define FSTEP 32                      // floats of k per step: 128 bytes of a row
 #define ROWS_MAX_M 32                 // up to this many rows of activations the weight-streaming kernel is taken
-#define ROWS_SPLIT_MIN_K 4096
+#define ROWS_SPLIT_MIN_K 4096         // from this k on a product's pieces are worth a kernel that adds them
+
+// What becomes of a product in one piece: stored, added to C, or, with gate and up rows interleaved in blocks of 16 in W,
+// silu(gate) * up of the same feature stored to C [M, N / 2] (a kernel of its own for it took 4.7 us at eight tokens by 8,192
+// features and 27 at 1,293; the products take as long as without)
+enum { EPI_STORE = 0, EPI_ADD = 1, EPI_SWIGLU = 2 };
+
+__device__ inline float silu_mul(float g, float u) { return g / (1.0f + expf(-g)) * u; }
 
 // ------------------------------------------------------------------ few rows: stream the weights
 // The weights are the row operand, the activations the column operand.  A block is WAVES waves on the same RT * 16
@@ -29,11 +36,12 @@ union RowsLds {
   u32x4_t xs[WAVES][MB * 8 * 16];
 };
 
-template <int MB, int RT, int WAVES, int DEPTH, bool ACCUM>
+template <int MB, int RT, int WAVES, int DEPTH, int EPI>
 __global__ __launch_bounds__(WAVES * 64) void gemm_float32_rows_kernel(float* __restrict__ C, long ldc, const float* __restrict__ X, long ldx,
                                                                        const float* __restrict__ W, long ldw, int M, int N, int K,
                                                                        int k_per_block, float* __restrict__ part) {
   constexpr int ROWS = RT * 16;
+  static_assert(EPI != EPI_SWIGLU || RT == 2, "a gate's rows and its up rows lie in one block");
   __shared__ RowsLds<MB, RT, WAVES> lds;
   const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
   const int lr = lane % 16, lg = lane / 16;
@@ -143,9 +151,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_float32_rows_kernel(float* __
 #pragma unroll
       for (int r = 0; r < 4; ++r) lds.red[wave][t * 16 + lg * 4 + r][c * 16 + lr] = acc[t][c][r];
   __syncthreads();
-  for (int idx = tid; idx < ROWS * MB * 16; idx += WAVES * 64) {
-    const int nl = idx % ROWS, m = idx / ROWS;
-    if (m >= M || n0 + nl >= N) continue;
+  auto total = [&](const int nl, const int m) {
     float v[WAVES];
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) v[w] = lds.red[w][nl][m];
@@ -153,11 +159,24 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_float32_rows_kernel(float* __
     for (int gap = 1; gap < WAVES; gap *= 2)
 #pragma unroll
       for (int w = 0; w < WAVES; w += 2 * gap) v[w] += v[w + gap];
+    return v[0];
+  };
+  if (EPI == EPI_SWIGLU) {
+    for (int idx = tid; idx < 16 * MB * 16; idx += WAVES * 64) {
+      const int j = idx % 16, m = idx / 16;
+      if (m < M && n0 + 16 + j < N) C[m * ldc + n0 / 2 + j] = silu_mul(total(j, m), total(16 + j, m));
+    }
+    return;
+  }
+  for (int idx = tid; idx < ROWS * MB * 16; idx += WAVES * 64) {
+    const int nl = idx % ROWS, m = idx / ROWS;
+    if (m >= M || n0 + nl >= N) continue;
+    const float sum = total(nl, m);
     if (gridDim.y > 1) {
-      part[((long)blockIdx.y * M + m) * N + n0 + nl] = v[0];
+      part[((long)blockIdx.y * M + m) * N + n0 + nl] = sum;
     } else {
       float* c = C + m * ldc + n0 + nl;
-      *c = ACCUM ? *c + v[0] : v[0];
+      *c = EPI == EPI_ADD ? *c + sum : sum;
     }
   }
 }
@@ -169,7 +188,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_float32_rows_kernel(float* __
 // has to be large enough for L2: 32 / 21 / 16 flops per byte at 128 x 128 / 128 x 64 / 64 x 64.  What decides is how the
 // tiles fill the chip, see plan().  Every output is summed over k in the same order in every
 // tile shape; how many pieces k is cut into depends on the rows and columns, so a row's bits depend on what shares its launch.
-template <int TM, int TN, int NB, bool ACCUM>
+template <int TM, int TN, int NB, int EPI>
 __global__ __launch_bounds__(256) void gemm_float32_tile_kernel(float* __restrict__ C, long ldc, const float* __restrict__ A, long lda,
                                                                 const float* __restrict__ W, long ldw, int M, int N, int K, int tiles_n,
                                                                 int k_per_split, float* __restrict__ part) {
@@ -284,6 +303,27 @@ __global__ __launch_bounds__(256) void gemm_float32_tile_kernel(float* __restric
   // acc[i][j][v] is C[m0 + wm*TM/2 + i*32 + 8*(v/4) + 4*(lane/32) + v%4][n0 + wn*TN/2 + j*32 + lane%32]: a store
   // instruction writes 128 contiguous bytes of two rows.  Added into C, sixteen of its values are fetched before the first
   // is used (one after the other 1,600 x 16,384 x 64 took 113 us, 512 x 16,384 x 512 99; 69 and 87 so)
+  if (EPI == EPI_SWIGLU) {
+    // columns 0..15 of a wave's 32 are gate rows of W, 16..31 the up rows of the same features: lane l and lane l + 16 swap
+    // so that the one has gate and up of row v, the other of row v + 1
+    const bool up = frow >= 16;
+#pragma unroll
+    for (int j = 0; j < WN; ++j) {
+      const long n = n0 + wn * (TN / 2) + j * 32;                 // N is a multiple of 32
+      if (n >= N) continue;
+#pragma unroll
+      for (int i = 0; i < WM; ++i) {
+        const long mi = m0 + wm * (TM / 2) + i * 32 + 4 * (lane / 32);
+#pragma unroll
+        for (int v = 0; v < 16; v += 2) {
+          const float own = up ? acc[i][j][v + 1] : acc[i][j][v], other = __shfl_xor(up ? acc[i][j][v] : acc[i][j][v + 1], 16);
+          const long m = mi + 8 * (v / 4) + v % 4 + up;
+          if (m < M) C[m * ldc + n / 2 + frow % 16] = silu_mul(up ? other : own, up ? own : other);
+        }
+      }
+    }
+    return;
+  }
   const bool pieces = gridDim.y > 1;
   float* out = pieces ? part + (long)blockIdx.y * M * N : C;
   const long ld = pieces ? N : ldc;
@@ -297,7 +337,7 @@ __global__ __launch_bounds__(256) void gemm_float32_tile_kernel(float* __restric
       float sum[16];
 #pragma unroll
       for (int v = 0; v < 16; ++v) sum[v] = acc[i][j][v];
-      if (ACCUM && !pieces) {                    // asked for together: one wait for memory, not sixteen
+      if (EPI == EPI_ADD && !pieces) {           // asked for together: one wait for memory, not sixteen
         float old[16];
 #pragma unroll
         for (int v = 0; v < 16; ++v) old[v] = out[min(mi + 8 * (v / 4) + v % 4, (long)M - 1) * ld + n];
@@ -329,13 +369,16 @@ static Float32Plan cut(int tm, int tn, int K, int splits) {
 // once at 4 TB/s by a kernel of their own.  Measured, N x K = 16384 x 2048: 2,048 rows 1,002 us (137 TFLOP/s), 1,293 rows
 // 727 us (1,236 on the vector unit), 378 rows 214 us (118 TFLOP/s); 2048 x 8192: 2,048 rows 525 us, 1,293 rows 412 us in two
 // pieces, 378 rows 119 us in five.
-static Float32Plan plan(int M, int N, int K, long part_floats) {
+// `read_by_next`: the pieces are left to the kernel that reads the result anyway (a norm, a rotation).  They then cost their
+// way through memory and no launch, and a matrix of few rows is streamed by two blocks per unit whatever its k: eight tokens,
+// 2,048 x 2,048 9.9 -> 7.8 us, 3,072 x 2,048 10.0 -> 8.9; and 4.6 us less for each product whose pieces a kernel added.
+static Float32Plan plan(int M, int N, int K, long part_floats, bool read_by_next) {
   const int units = compute_units();
   if (M <= ROWS_MAX_M) {
     // blocks of 32 rows want to be two per unit; a matrix of fewer rows whose k is long is cut over blocks, any other
     // gets its waves in blocks of 16 rows (launch_rows)
-    int splits = K >= ROWS_SPLIT_MIN_K ? 2 * units / ceil_div(N, 32) : 1;
-    while (splits > 1 && (K / splits < 512 || (long)splits * M * N > part_floats)) --splits;
+    int splits = read_by_next || K >= ROWS_SPLIT_MIN_K ? 2 * units / ceil_div(N, 32) : 1;
+    while (splits > 1 && (K / splits < (read_by_next ? 256 : 512) || (long)splits * M * N > part_floats)) --splits;
     return cut(0, 0, K, splits < 1 ? 1 : splits);
   }
   static const struct { int tm, tn; float rate; } shapes[] = {{128, 128, 0.50e6f}, {128, 64, 0.49e6f}, {64, 64, 0.46e6f}};
@@ -348,82 +391,92 @@ static Float32Plan plan(int M, int N, int K, long part_floats) {
       if (splits > 1 && (p.splits != splits || p.k_per_split < 256 || (long)splits * M * N > part_floats)) continue;
       const long rounds = (tiles * p.splits + units - 1) / units;
       float us = rounds * (3.f + 2.f * s.tm * s.tn * p.k_per_split / s.rate);
-      if (p.splits > 1) us += 4.f + 2.f * p.splits * M * N * 4.f / 4.0e6f;
+      if (p.splits > 1) us += (read_by_next ? 1.f : 4.f) + (read_by_next ? 1.5f : 2.f) * p.splits * M * N * 4.f / 4.0e6f;
       if (least == 0.f || us < least) { least = us; best = p; }
     }
   }
   return best;
 }
 
-// Pieces that pi_gemm_float32 makes of this product when it may leave pieces in `part_floats` floats: 1 if it writes C.
-extern "C" int pi_gemm_float32_pieces(int M, int N, int K, long part_floats) {
-  return M > 0 && N > 0 && K > 0 ? plan(M, N, K, part_floats).splits : 1;
+// Pieces that pi_gemm_float32 makes of this product when it may leave pieces in `part_floats` floats: 1 if it writes C.  See plan().
+extern "C" int pi_gemm_float32_pieces(int M, int N, int K, long part_floats, int read_by_next) {
+  return M > 0 && N > 0 && K > 0 ? plan(M, N, K, part_floats, read_by_next != 0).splits : 1;
 }
 
-template <int TM, int TN, int NB>
-static int launch_tiles(float* C, long ldc, const float* A, long lda, const float* W, long ldw, int M, int N, int K, int accumulate,
-                        const Float32Plan& p, float* part, hipStream_t stream) {
+template <int TM, int TN, int NB, int EPI>
+static int launch_tiles_of(float* C, long ldc, const float* A, long lda, const float* W, long ldw, int M, int N, int K, const Float32Plan& p, float* part,
+                           hipStream_t stream) {
   constexpr size_t bytes = (size_t)NB * (TM + TN) * 128;
-  static bool configured = false;
-  if (!configured) {
-    for (const void* f : {reinterpret_cast<const void*>(gemm_float32_tile_kernel<TM, TN, NB, true>), reinterpret_cast<const void*>(gemm_float32_tile_kernel<TM, TN, NB, false>)}) {
-      hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-      if (e != hipSuccess) return pi_fail("gemm_float32: cannot reserve %zu bytes of LDS: %s", bytes, hipGetErrorString(e));
-    }
-    configured = true;
-  }
+  static const hipError_t configured = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_float32_tile_kernel<TM, TN, NB, EPI>),
+                                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+  if (configured != hipSuccess) return pi_fail("gemm_float32: cannot reserve %zu bytes of LDS: %s", bytes, hipGetErrorString(configured));
   const int tiles_n = ceil_div(N, TN);
-  const dim3 grid((unsigned)(ceil_div(M, TM) * (long)tiles_n), p.splits), block(256);
-  if (accumulate)
-    hipLaunchKernelGGL((gemm_float32_tile_kernel<TM, TN, NB, true>), grid, block, bytes, stream, C, ldc, A, lda, W, ldw, M, N, K, tiles_n, p.k_per_split, part);
-  else
-    hipLaunchKernelGGL((gemm_float32_tile_kernel<TM, TN, NB, false>), grid, block, bytes, stream, C, ldc, A, lda, W, ldw, M, N, K, tiles_n, p.k_per_split, part);
+  hipLaunchKernelGGL((gemm_float32_tile_kernel<TM, TN, NB, EPI>), dim3((unsigned)(ceil_div(M, TM) * (long)tiles_n), p.splits), dim3(256), bytes, stream, C, ldc,
+                     A, lda, W, ldw, M, N, K, tiles_n, p.k_per_split, part);
   return pi_check_launch("gemm_float32 (tiles)");
+}
+
+template <int EPI>
+static int launch_tiles(float* C, long ldc, const float* A, long lda, const float* W, long ldw, int M, int N, int K, const Float32Plan& p, float* part,
+                        hipStream_t stream) {
+  if (p.tm == 128 && p.tn == 128) return launch_tiles_of<128, 128, 2, EPI>(C, ldc, A, lda, W, ldw, M, N, K, p, part, stream);
+  if (p.tm == 128) return launch_tiles_of<128, 64, 3, EPI>(C, ldc, A, lda, W, ldw, M, N, K, p, part, stream);
+  return launch_tiles_of<64, 64, 4, EPI>(C, ldc, A, lda, W, ldw, M, N, K, p, part, stream);
 }
 
 // Enough waves for the memory whatever the matrix' rows are: blocks of four waves on 32 rows where that gives two per
 // unit, also by cutting k; else blocks of 16 rows with 8 or 16 waves.  Eight tokens, N x K: 16384 x 2048 25.8 us
 // (5.2 TB/s; 35.6 before, on the vector unit), 128256 x 2048 181 us (5.8 TB/s; 197), 3072 x 2048 12.5 us and
 // 2048 x 2048 10.7 us with 16 waves, 2048 x 8192 17.1 us in eight pieces and 4 to add them (with 16 waves instead: 25).
-template <int MB>
-static int launch_rows(float* C, long ldc, const float* A, long lda, const float* W, long ldw, int M, int N, int K, int accumulate,
-                       const Float32Plan& p, float* part, hipStream_t stream) {
+template <int MB, int EPI>
+static int launch_rows(float* C, long ldc, const float* A, long lda, const float* W, long ldw, int M, int N, int K, const Float32Plan& p, float* part,
+                       hipStream_t stream) {
 #define ROWS_GO(RT, WAVES, DEPTH)                                                                                                              \
-  do {                                                                                                                                         \
-    const dim3 grid(ceil_div(N, RT * 16), p.splits), block(WAVES * 64);                                                                        \
-    if (accumulate)                                                                                                                            \
-      hipLaunchKernelGGL((gemm_float32_rows_kernel<MB, RT, WAVES, DEPTH, true>), grid, block, 0, stream, C, ldc, A, lda, W, ldw, M, N, K, p.k_per_split, part);  \
-    else                                                                                                                                       \
-      hipLaunchKernelGGL((gemm_float32_rows_kernel<MB, RT, WAVES, DEPTH, false>), grid, block, 0, stream, C, ldc, A, lda, W, ldw, M, N, K, p.k_per_split, part); \
-  } while (0)
+  hipLaunchKernelGGL((gemm_float32_rows_kernel<MB, RT, WAVES, DEPTH, EPI>), dim3(ceil_div(N, RT * 16), p.splits), dim3(WAVES * 64), 0, stream, C, ldc, \
+                     A, lda, W, ldw, M, N, K, p.k_per_split, part)
   const int units = compute_units();
-  if (p.splits > 1 || N >= 2 * units * 24) ROWS_GO(2, 4, 1);
+  if (p.splits > 1 && p.k_per_split <= 512) ROWS_GO(2, 4, 2);          // a wave's few steps all at once
+  else if (p.splits > 1 || N >= 2 * units * 24) ROWS_GO(2, 4, 1);
+  else if constexpr (EPI == EPI_SWIGLU) ROWS_GO(2, 8, 2);
   else if (MB == 1 && N <= units * 16) ROWS_GO(1, (MB == 1 ? 16 : 8), 2);     // sixteen waves have registers for 16 tokens only
   else ROWS_GO(1, 8, 2);
 #undef ROWS_GO
   return pi_check_launch("gemm_float32 (few rows)");
 }
 
-// C (+)= A . W^T.  `part` (may be null): float32 [part_floats] for the pieces of a product whose k is cut; when
-// pi_gemm_float32_pieces says more than one, the pieces [splits, M, N] are all that is written and C is not touched.
-extern "C" int pi_gemm_float32(void* C, long ldc, const void* A, long lda, const void* W, long ldw, int M, int N, int K, int accumulate,
-                               void* part, long part_floats, hipStream_t stream) {
+template <int EPI>
+static int launch_float32(float* C, long ldc, const float* A, long lda, const float* W, long ldw, int M, int N, int K, const Float32Plan& p, float* part,
+                          hipStream_t stream) {
+  if (p.tm) return launch_tiles<EPI>(C, ldc, A, lda, W, ldw, M, N, K, p, part, stream);
+  return M <= 16 ? launch_rows<1, EPI>(C, ldc, A, lda, W, ldw, M, N, K, p, part, stream) : launch_rows<2, EPI>(C, ldc, A, lda, W, ldw, M, N, K, p, part, stream);
+}
+
+static int check_float32(int M, int N, int K, const void* A, long lda, const void* W, long ldw, long ldc, int cols) {
   PI_REQUIRE(M > 0 && N > 0 && K > 0 && K < (1 << 29), "gemm_float32: bad sizes M=%d N=%d K=%d", M, N, K);
-  PI_REQUIRE(lda >= K && ldw >= K && ldc >= N, "gemm_float32: row strides (%ld, %ld, %ld) smaller than the rows (K=%d, N=%d)", lda, ldw, ldc, K, N);
+  PI_REQUIRE(lda >= K && ldw >= K && ldc >= cols, "gemm_float32: row strides (%ld, %ld, %ld) smaller than the rows (K=%d, %d columns)", lda, ldw, ldc, K, cols);
   PI_REQUIRE(K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0, "gemm_float32: K (%d) and row strides (%ld, %ld) must be multiples of 4", K, lda, ldw);
   PI_REQUIRE(128 * lda < (1L << 28) && 128 * ldw < (1L << 28), "gemm_float32: row strides (%ld, %ld) are too long for 32-bit offsets inside a tile", lda, ldw);
   PI_REQUIRE((uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0, "gemm_float32: operands must be 16-byte aligned");
   PI_REQUIRE((long)ceil_div(M, 64) * ceil_div(N, 64) < 2147483647L, "gemm_float32: too many tiles");
-  const Float32Plan p = plan(M, N, K, part ? part_floats : 0);
+  return 0;
+}
+
+// C (+)= A . W^T.  `part` (may be null): float32 [part_floats] for the pieces of a product whose k is cut; when
+// pi_gemm_float32_pieces says more than one, the pieces [splits, M, N] are all that is written and C is not touched.
+extern "C" int pi_gemm_float32(void* C, long ldc, const void* A, long lda, const void* W, long ldw, int M, int N, int K, int accumulate,
+                               void* part, long part_floats, int read_by_next, hipStream_t stream) {
+  if (check_float32(M, N, K, A, lda, W, ldw, ldc, N)) return -1;
+  const Float32Plan p = plan(M, N, K, part ? part_floats : 0, read_by_next != 0);
   PI_REQUIRE(p.splits == 1 || (part && part_floats >= (long)p.splits * M * N), "gemm_float32: workspace too small (%ld floats for %ld)", part_floats, (long)p.splits * M * N);
-  float *c = (float*)C, *pieces = (float*)part;
-  const float *a = (const float*)A, *w = (const float*)W;
-  if (p.tm == 0) {
-    return M <= 16 ? launch_rows<1>(c, ldc, a, lda, w, ldw, M, N, K, accumulate, p, pieces, stream) : launch_rows<2>(c, ldc, a, lda, w, ldw, M, N, K, accumulate, p, pieces, stream);
-  }
-  if (p.tm == 128 && p.tn == 128) return launch_tiles<128, 128, 2>(c, ldc, a, lda, w, ldw, M, N, K, accumulate, p, pieces, stream);
-  if (p.tm == 128) return launch_tiles<128, 64, 3>(c, ldc, a, lda, w, ldw, M, N, K, accumulate, p, pieces, stream);
-  return launch_tiles<64, 64, 4>(c, ldc, a, lda, w, ldw, M, N, K, accumulate, p, pieces, stream);
+  return accumulate ? launch_float32<EPI_ADD>((float*)C, ldc, (const float*)A, lda, (const float*)W, ldw, M, N, K, p, (float*)part, stream)
+                    : launch_float32<EPI_STORE>((float*)C, ldc, (const float*)A, lda, (const float*)W, ldw, M, N, K, p, (float*)part, stream);
+}
+
+// C [M, N / 2] = silu(gate) * up of the product's columns, gate and up rows interleaved in blocks of 16 in W.
+extern "C" int pi_gemm_float32_swiglu(void* C, long ldc, const void* A, long lda, const void* W, long ldw, int M, int N, int K, hipStream_t stream) {
+  if (check_float32(M, N, K, A, lda, W, ldw, ldc, N / 2)) return -1;
+  PI_REQUIRE(N % 32 == 0, "gemm_float32: the gated epilogue needs N (%d) to be a multiple of 32", N);
+  return launch_float32<EPI_SWIGLU>((float*)C, ldc, (const float*)A, lda, (const float*)W, ldw, M, N, K, plan(M, N, K, 0, false), nullptr, stream);
 }
 
 // ------------------------------------------------------------------ adding pieces

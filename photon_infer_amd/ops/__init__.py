@@ -218,6 +218,10 @@ def gemm_swiglu(out: torch.Tensor, a: torch.Tensor, w_gate_up: torch.Tensor, blo
         from . import fast
         if fast.gemm_swiglu(out, a, w_gate_up, M, 2 * I, a.shape[1], _rows(a, "gemm a"), _rows(w_gate_up, "gemm w"), ws):
             return
+    if _FAST and block == 16 and a.dtype == torch.float32 and w_gate_up.dtype == torch.float32 and out.is_contiguous():
+        from . import fast
+        if fast.gemm_swiglu_float32(out, a, w_gate_up, M, 2 * I, a.shape[1], _rows(a, "gemm a"), _rows(w_gate_up, "gemm w")):
+            return
     gu = torch.empty((M, 2 * I), dtype=a.dtype, device=a.device)
     gemm(gu, a, w_gate_up, ws=ws)
     swiglu(out, gu, block)
@@ -268,7 +272,7 @@ def gemm(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, accumulate: bool =
             return
     if _FAST and a.dtype == torch.float32 and w.dtype == torch.float32 and out.dtype == torch.float32:
         from . import fast
-        if fast.gemm_float32(out, a, w, accumulate, M, N, K, lda, ldw, ldc, ws):
+        if fast.gemm_float32(out, a, w, accumulate, M, N, K, lda, ldw, ldc, may_defer and out.is_contiguous(), ws):
             return
     _lib.call("core", "pi_gemm_general", out.data_ptr(), _dt(out), ldc, a.data_ptr(), _dt(a), lda, w.data_ptr(),
               _dt(w), ldw, M, N, K, int(accumulate), _stream())
@@ -322,6 +326,12 @@ def qkv_projection(h: torch.Tensor, w_qkv: torch.Tensor, dtype: torch.dtype, ws:
     if _FAST and ws is not None and h.dtype == torch.bfloat16 and w_qkv.dtype == torch.bfloat16 and h.is_cuda:
         from . import fast
         p = fast.gemm_pieces(h, w_qkv, ws)
+        if p is not None:
+            ws.counts["qkv_pieces"] += 1
+            return p
+    if _FAST and ws is not None and h.dtype == torch.float32 and w_qkv.dtype == torch.float32 and h.is_cuda and h.shape[0] > 0:
+        from . import fast
+        p = fast.gemm_float32_pieces(h, w_qkv, ws)
         if p is not None:
             ws.counts["qkv_pieces"] += 1
             return p

@@ -34,6 +34,7 @@ SHARED_FROM_TOKENS = 32        # more tokens than this: the skinny kernel that s
 SHARED_ROWS_PER_BLOCK = 64     # ... with this many weight rows per block, and no more blocks than compute units (100 tokens, 3,072 x 8,192:
                                # 22.8 us in six pieces on 288 blocks, 16.9 in five on 240; 6,144 x 4,096 22.8 in three, 18.7 in two)
 RING_MAX_STRIDE = 1 << 21      # elements between rows up to which that kernel's byte offsets fit 31 bits
+FLOAT32_SWIGLU_K = 2048        # up to this k the gated unit is part of the float32 product also where the general kernel streams a few rows faster
 FLOAT32_MAX_STRIDE = 1 << 21   # floats between rows up to which the float32 kernels' offsets inside a tile fit 32 bits
 DEFAULT_UNITS = 256            # compute units assumed where no device can be asked (an MI355X)
 PIECES_WORTH = 0.95            # q, k, v of a prompt portion are left in k pieces too where that takes no more than this share of the time:
@@ -222,17 +223,53 @@ def _general_streams_faster(M: int, N: int, K: int) -> bool:
     return (M <= 2 and K > 512) or (M <= 8 and K >= 8192 and N >= 8192)
 
 
-def gemm_float32(out, a, w, accumulate, M, N, K, lda, ldw, ldc, ws: Optional[KernelWorkspace] = None) -> bool:
+def _float32_product(out, a, w, accumulate, M, N, K, lda, ldw, ldc, ws: Optional[KernelWorkspace], read_by_next: bool) -> Optional[Partials]:
+    """Run the float32 matrix-core product; returns the pieces when k was cut (then ``out`` is not touched)."""
+    made = _lib.load("core").pi_gemm_float32_pieces(M, N, K, GEMM_PART_FLOATS, read_by_next)
+    buf = _piece_buffer(ws, made * M * N, a.device) if made > 1 else None
+    if out is None and buf is None:
+        return None                       # pieces were wanted, and it makes none
+    _lib.call("core", "pi_gemm_float32", None if out is None else out.data_ptr(), ldc, a.data_ptr(), lda, w.data_ptr(), ldw, M, N, K, int(accumulate),
+              None if buf is None else buf.data_ptr(), GEMM_PART_FLOATS if buf is not None else 0, read_by_next, _stream())
+    if buf is None:
+        return None
+    if ws is not None:
+        ws.counts["split_products"] += 1
+    return Partials(buf, made, M, N)
+
+
+def gemm_float32(out, a, w, accumulate, M, N, K, lda, ldw, ldc, may_defer=False, ws: Optional[KernelWorkspace] = None) -> bool:
     """out (+)= a @ w^T, all float32, by the float32 matrix-core kernels; what a product of few tiles leaves in pieces is
-    added at once."""
+    left to the stream's next reader (``may_defer``) or added at once."""
     if not _float32_ok(a, w, K, lda, ldw) or _general_streams_faster(M, N, K):
         return False
-    made = _lib.load("core").pi_gemm_float32_pieces(M, N, K, GEMM_PART_FLOATS)
-    buf = _piece_buffer(ws, made * M * N, a.device) if made > 1 else None
-    _lib.call("core", "pi_gemm_float32", out.data_ptr(), ldc, a.data_ptr(), lda, w.data_ptr(), ldw, M, N, K, int(accumulate),
-              None if buf is None else buf.data_ptr(), GEMM_PART_FLOATS if buf is not None else 0, _stream())
-    if buf is not None:
-        _lib.call("core", "pi_splitk_reduce", out.data_ptr(), EPI_ACCUM if accumulate else EPI_F32, ldc, buf.data_ptr(), made, M, N, _stream())
+    may_defer = may_defer and ws is not None
+    pieces = _float32_product(out, a, w, accumulate, M, N, K, lda, ldw, ldc, ws, may_defer)
+    if pieces is not None and may_defer:
+        ws.pending = PendingUpdate(out, pieces, accumulate)
+        ws.counts["deferred"] += 1
+    elif pieces is not None:
+        _lib.call("core", "pi_splitk_reduce", out.data_ptr(), EPI_ACCUM if accumulate else EPI_F32, ldc, pieces.part.data_ptr(), pieces.splits, M, N, _stream())
+    return True
+
+
+def gemm_float32_pieces(a, w, ws: Optional[KernelWorkspace]) -> Optional[Partials]:
+    """a @ w^T in float32 left in pieces in the workspace, if this product is one whose k-range is cut."""
+    if ws is None:
+        return None
+    M, K = a.shape
+    N = w.shape[0]
+    lda, ldw = a.stride(0) if M > 1 else K, w.stride(0)
+    if a.stride(1) != 1 or w.stride(1) != 1 or not _float32_ok(a, w, K, lda, ldw) or _general_streams_faster(M, N, K):
+        return None
+    return _float32_product(None, a, w, False, M, N, K, lda, ldw, N, ws, True)
+
+
+def gemm_swiglu_float32(out, a, w, M, N, K, lda, ldw) -> bool:
+    """``w`` [N = 2I, K] with gate / up rows interleaved in blocks of 16; out [M, I], all float32."""
+    if not _float32_ok(a, w, K, lda, ldw) or N % 32 or (_general_streams_faster(M, N, K) and K > FLOAT32_SWIGLU_K):
+        return False
+    _lib.call("core", "pi_gemm_float32_swiglu", out.data_ptr(), out.stride(0), a.data_ptr(), lda, w.data_ptr(), ldw, M, N, K, _stream())
     return True
 
 

@@ -48,10 +48,10 @@ class SwiGLU(FeedForward):
         common = torch.float32 if torch.float32 in (g.dtype, u.dtype) else g.dtype
         g, u = g.to(common), u.to(common)
         I = self.intermediate_size
-        if common == torch.bfloat16 and I % INTERLEAVE == 0:
+        if I % INTERLEAVE == 0:
             # one projection for gate and up, rows interleaved in blocks of 16 (gate block, up
             # block, ...): the matrix-core kernels then hold a feature's gate and up value in
-            # the same lane and apply the activation before anything is stored
+            # the same lane, or in two of a wave, and apply the activation before anything is stored
             self.interleave = INTERLEAVE
             self.w_gate_up = torch.stack([g.view(I // INTERLEAVE, INTERLEAVE, -1), u.view(I // INTERLEAVE, INTERLEAVE, -1)],
                                          dim=1).reshape(2 * I, -1).contiguous()

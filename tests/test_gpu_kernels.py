@@ -345,6 +345,40 @@ def test_every_tile_shape_at_its_edges(_ops, monkeypatch, shape, M, N, K):
     close(out, P.swiglu(g.reshape(M, -1), u.reshape(M, -1)).cpu(), 2 ** -7, f"tiles {shape}, swiglu")
 
 
+@pytest.mark.parametrize("M", [1, 3, 16, 17, 32, 33, 65, 200])
+@pytest.mark.parametrize("I,K", [(16, 4), (48, 260), (6160, 200), (528, 4096)])
+def test_float32_product_with_swiglu(_ops, M, I, K):
+    """Gate and up rows interleaved by 16, the unit in the product's epilogue: few rows and tiles, and k long enough for the
+    general kernel.  Sums of K products are off by sqrt(K) roundings of their size at most, the unit's slope is below 1.1."""
+    _ops.use_fast_kernels(True)
+    a = torch.randn(M, K, generator=gen(M))
+    g, u = torch.randn(I, K, generator=gen(I)) / K ** 0.5, torch.randn(I, K, generator=gen(K)) / K ** 0.5
+    w = torch.stack([g.view(I // 16, 16, K), u.view(I // 16, 16, K)], dim=1).reshape(2 * I, K).contiguous()
+    want = P.swiglu(a.double() @ g.double().t(), a.double() @ u.double().t())
+    out = torch.empty(M, I, device=DEV)
+    _ops.gemm_swiglu(out, a.to(DEV), w.to(DEV), 16)
+    close(out, want, 2 ** -23 * (8 + K ** 0.5), f"{M} x {I} x {K}")
+
+
+@pytest.mark.parametrize("M,N,K", [(3, 2048, 2048), (8, 96, 512), (32, 3072, 2048), (33, 256, 1024), (378, 2048, 8192), (1, 2048, 2048)])
+def test_float32_pieces_are_added_by_the_next_reader(_ops, M, N, K):
+    """A product into the stream that stays in pieces, read by the norm, and one for the rotation: against 64 bits."""
+    _ops.use_fast_kernels(True)
+    a, w = torch.randn(M, K, generator=gen(M)).to(DEV), (torch.randn(N, K, generator=gen(N)) / K ** 0.5).to(DEV)
+    x = torch.randn(M, N, generator=gen(K)).to(DEV)
+    want = x.double() + a.double() @ w.double().t()
+    ws = _ops.KernelWorkspace(DEV)
+    _ops.gemm(x, a, w, accumulate=True, may_defer=True, ws=ws)
+    h = torch.empty_like(x)
+    _ops.rmsnorm(h, x, torch.ones(N, device=DEV), 1e-5, ws=ws)
+    assert ws.pending is None
+    close(x, want.cpu(), 2 ** -23 * (8 + K ** 0.5), "stream")
+    close(h, (want / (want.pow(2).mean(-1, keepdim=True) + 1e-5).sqrt()).cpu(), 2 ** -22 * (8 + K ** 0.5), "norm")
+    p = _ops.qkv_projection(a, w, F32, ws)
+    got = p if isinstance(p, torch.Tensor) else p.part[:p.splits * M * N].view(p.splits, M, N).double().sum(0)
+    close(got, (a.double() @ w.double().t()).cpu(), 2 ** -23 * (8 + K ** 0.5), "projection")
+
+
 def test_gemm_reference_vectors(_ops):
     # tests/ops/test_matmul.cpp:90-204
     W = torch.tensor([[1.0, 2.0, 3.0], [4.0, 5.0, 6.0]], device=DEV)
