@@ -240,10 +240,10 @@ def _float32_product(out, a, w, accumulate, M, N, K, lda, ldw, ldc, ws: Optional
 
 def gemm_float32(out, a, w, accumulate, M, N, K, lda, ldw, ldc, may_defer=False, ws: Optional[KernelWorkspace] = None) -> bool:
     """out (+)= a @ w^T, all float32, by the float32 matrix-core kernels; what a product of few tiles leaves in pieces is
-    left to the stream's next reader (``may_defer``) or added at once."""
+    left to the stream's next reader (an update, ``may_defer``) or added at once."""
     if not _float32_ok(a, w, K, lda, ldw) or _general_streams_faster(M, N, K):
         return False
-    may_defer = may_defer and ws is not None
+    may_defer = may_defer and accumulate and ws is not None       # a result that is written, not added, is whole when the call returns
     pieces = _float32_product(out, a, w, accumulate, M, N, K, lda, ldw, ldc, ws, may_defer)
     if pieces is not None and may_defer:
         ws.pending = PendingUpdate(out, pieces, accumulate)
