@@ -143,6 +143,16 @@ __device__ inline float row16_sum(float v) {
   return v;
 }
 
+template <int LANES> __device__ inline float lanes_sum(float v) {
+  static_assert(LANES == 16 || LANES == 32, "a column's lanes");
+  v = row16_sum(v);
+  if constexpr (LANES == 32) {
+    auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  }
+  return v;
+}
+
 static inline int scan_rows_per_lane(int rows) {
   for (int nr = 1; nr <= 16; nr *= 2)
     if (16 * nr >= rows) return nr;
@@ -166,7 +176,14 @@ template <int NR, bool SHORT> struct ScanShape {
 // zeros from `size` on, by one wave.  Fetching and storing are two steps, so that a chunk's fetches are all
 // in flight before the first of them is waited for.  `vec`: size % 4 == 0 and 16-byte accesses are allowed;
 // otherwise the vectors are copied one float at a time by store().
-template <int W, int CH>
+// `NR`: the lanes of a column each read NR rows, four at a time; with 4 or more those fours lie side by side, lane after
+// lane, so that a read falls on all banks (0: the rows as they come).
+template <int W, int NR> __device__ inline int staged_place(int r) {
+  if constexpr (NR >= 4) return r % NR / 4 * (W / NR * 4) + r / NR * 4 + r % 4;
+  return r;
+}
+
+template <int W, int CH, int NR = 0>
 struct StagedVectors {
   static constexpr int Q = W / 4, IT = (CH * Q + PI_WAVE - 1) / PI_WAVE;
   float4 v[IT];
@@ -188,12 +205,12 @@ struct StagedVectors {
 #pragma unroll
       for (int j = 0; j < IT; ++j) {
         const int i = lane + j * PI_WAVE, tt = i / Q, r = (i - tt * Q) * 4;
-        if (tt < cn) *reinterpret_cast<float4*>(dst + tt * W + r) = v[j];
+        if (tt < cn) *reinterpret_cast<float4*>(dst + tt * W + staged_place<W, NR>(r)) = v[j];
       }
     } else {
       for (int i = lane; i < cn * W; i += PI_WAVE) {
         const int tt = i / W, r = i - tt * W;
-        dst[i] = r < size ? src[tt * stride + r] : 0.f;
+        dst[tt * W + staged_place<W, NR>(r)] = r < size ? src[tt * stride + r] : 0.f;
       }
     }
   }
@@ -446,51 +463,75 @@ __global__ __launch_bounds__(PI_WAVE) void delta_prepare_kernel(float* __restric
   if (lane == 0) b[t * b_stride + h] = sigmoid_f(b[t * b_stride + h]);
 }
 
+// What a lane needs of one token: its rows of q^, k^ and the decays, its column's v, and beta.
+template <int NR, int LANES>
+struct DeltaToken {
+  float q[NR], k[NR], g[NR], v, beta;
+  __device__ static inline void rows(float* to, const float* vector, int part) {
+    if constexpr (NR >= 4) {
+#pragma unroll
+      for (int i = 0; i < NR; i += 4) load4(vector + (i / 4 * LANES + part) * 4, to + i);
+    } else {
+#pragma unroll
+      for (int i = 0; i < NR; ++i) to[i] = vector[part * NR + i];
+    }
+  }
+};
+
 // Then the walk: q^, k^ and v from qkv, decays from a, beta from b.  A column of S never meets another
-// column, so a wave walks its four columns alone.
-template <int NR, bool SHORT, int KIND>
-__global__ __launch_bounds__((PI_SCAN_WAVES + 1) * PI_WAVE) void delta_scan_kernel(
+// column, so a wave walks its columns alone.  Bound by the chain from one token's state to the next and by what a wave that
+// has its unit's fourth to itself can issue.  16 heads of 128 x 128, 2,048 tokens of one request: 507 us with chunks fetched
+// and stored to LDS in one go; 471 with a chunk's fetch in flight while the chunk before is walked; 446 with a token read
+// from LDS while the one before is walked; 425 with 32 lanes to a column in blocks of eight columns (two waves of four
+// columns in such blocks, and fours that fall on all banks, gave nothing by themselves).
+template <int SNR, bool SHORT, int KIND, int WALKERS, int LANES>
+__global__ __launch_bounds__((WALKERS + 1) * PI_WAVE) void delta_scan_kernel(
     float* __restrict__ o, long o_stride, const float* __restrict__ qkv, long qkv_stride, const float* __restrict__ decay,
     long decay_stride, const float* __restrict__ beta, long beta_stride, const int* __restrict__ q_start,
     const int* __restrict__ slots, float* __restrict__ state, long state_stride, int H, int G, int d, int dv, int vec) {
-  constexpr int W = ScanShape<NR, SHORT>::W, CH = ScanShape<NR, SHORT>::CH;
+  constexpr int W = ScanShape<SNR, SHORT>::W, CH = ScanShape<SNR, SHORT>::CH, NR = SNR * 16 / LANES;     // rows of a lane: SNR in a state row's order
   __shared__ __attribute__((aligned(16))) float sq[2][CH * W];
   __shared__ __attribute__((aligned(16))) float sk[2][CH * W];
   __shared__ __attribute__((aligned(16))) float sg[2][KIND == SCAN_HEAD_DELTA ? 4 : CH * W];
-  __shared__ float sv[2][CH][PI_SCAN_COLUMNS], sbeta[2][CH], sdecay[2][CH];
-  const int r = blockIdx.x, h = blockIdx.y, z = blockIdx.z;
-  const int wave = threadIdx.x / PI_WAVE, lane = threadIdx.x % PI_WAVE, part = lane % 16;
+  constexpr int COLUMNS = WALKERS * (PI_WAVE / LANES);
+  __shared__ float sv[2][CH][COLUMNS], sbeta[2][CH], sdecay[2][CH];
+  const int r = blockIdx.x, h = blockIdx.y, col0 = blockIdx.z * COLUMNS;
+  const int wave = threadIdx.x / PI_WAVE, lane = threadIdx.x % PI_WAVE, part = lane % LANES;
   const int g = h / (H / G);
   const int qs = q_start[r], n = q_start[r + 1] - qs;
   if (n <= 0) return;
   const int chunks = (n + CH - 1) / CH;
-  const long q_col = (long)g * d, k_col = (long)G * d + (long)g * d, v_col = 2L * G * d + (long)h * dv + z * PI_SCAN_COLUMNS;
+  const long q_col = (long)g * d, k_col = (long)G * d + (long)g * d, v_col = 2L * G * d + (long)h * dv + col0;
 
-  auto fill = [&](int c) {      // the staging wave
-    const int buf = c & 1, t0 = c * CH, cn = n - t0 < CH ? n - t0 : CH;
+  // The staging wave: what a chunk needs is on its way from memory into this wave's registers while the chunk before it is
+  // walked and stored to LDS a chunk later, so that no walk waits for a trip to memory
+  StagedVectors<W, CH, NR> qs_, ks_, gs_;
+  constexpr int XI = (CH * COLUMNS + PI_WAVE - 1) / PI_WAVE;
+  float vs[XI], bt = 0.f, dc = 0.f;
+  auto fetch = [&](int c) {
+    const int t0 = c * CH, cn = n - t0 < CH ? n - t0 : CH;
     const float* src = qkv + (long)(qs + t0) * qkv_stride;
-    StagedVectors<W, CH> qs_, ks_, gs_;
     qs_.fetch(src + q_col, qkv_stride, cn, d, (vec & 1) != 0, lane);
     ks_.fetch(src + k_col, qkv_stride, cn, d, (vec & 1) != 0, lane);
     if constexpr (KIND != SCAN_HEAD_DELTA)
       gs_.fetch(decay + (long)(qs + t0) * decay_stride + (long)h * d, decay_stride, cn, d, (vec & 2) != 0, lane);
-    constexpr int XI = (CH * PI_SCAN_COLUMNS + PI_WAVE - 1) / PI_WAVE;
-    float vs[XI];
 #pragma unroll
     for (int j = 0; j < XI; ++j) {
-      const int i = lane + j * PI_WAVE, tt = i / PI_SCAN_COLUMNS, cc = i % PI_SCAN_COLUMNS;
-      vs[j] = (tt < cn && z * PI_SCAN_COLUMNS + cc < dv) ? src[tt * qkv_stride + v_col + cc] : 0.f;
+      const int i = lane + j * PI_WAVE, tt = i / COLUMNS, cc = i % COLUMNS;
+      vs[j] = (tt < cn && col0 + cc < dv) ? src[tt * qkv_stride + v_col + cc] : 0.f;
     }
-    float bt = 0.f, dc = 0.f;
     if constexpr (KIND != SCAN_DECAYED_OUTER) bt = lane < cn ? beta[(long)(qs + t0 + lane) * beta_stride + h] : 0.f;
     if constexpr (KIND == SCAN_HEAD_DELTA) dc = lane < cn ? decay[(long)(qs + t0 + lane) * decay_stride + h] : 0.f;
+  };
+  auto put = [&](int c) {       // what the last fetch, of chunk c, brought
+    const int buf = c & 1;
     qs_.store(sq[buf], lane);
     ks_.store(sk[buf], lane);
     if constexpr (KIND != SCAN_HEAD_DELTA) gs_.store(sg[buf], lane);
 #pragma unroll
     for (int j = 0; j < XI; ++j) {
       const int i = lane + j * PI_WAVE;
-      if (i < CH * PI_SCAN_COLUMNS) (&sv[buf][0][0])[i] = vs[j];
+      if (i < CH * COLUMNS) (&sv[buf][0][0])[i] = vs[j];
     }
     if (lane < CH) {
       sbeta[buf][lane] = bt;
@@ -499,67 +540,75 @@ __global__ __launch_bounds__((PI_SCAN_WAVES + 1) * PI_WAVE) void delta_scan_kern
   };
 
   float s[NR];
-  const int cw = wave * 4 + lane / 16;                 // this lane's column within the block
-  const int col = z * PI_SCAN_COLUMNS + cw;
+  const int cw = wave * (PI_WAVE / LANES) + lane / LANES;       // this lane's column within the block
+  const int col = col0 + cw;
   const bool live = col < dv;
-  float* Sg = state + (long)slots[r] * state_stride + (((long)h * gridDim.z + z) * PI_SCAN_WAVES + (wave & 3)) * NR * PI_WAVE + lane;
-  if (wave < PI_SCAN_WAVES) {
+  // a state row holds its columns by sixteen, four to a wave of sixteen lanes each, whatever the lanes here are
+  const int by16 = (dv + PI_SCAN_COLUMNS - 1) / PI_SCAN_COLUMNS;
+  const long row = ((long)(h * by16 + col / 16) * PI_SCAN_WAVES + col % 16 / 4) * SNR + part % (LANES / 16) * NR;
+  float* Sg = state + (long)slots[r] * state_stride + row * PI_WAVE + col % 4 * 16 + part / (LANES / 16);
+  if (wave < WALKERS) {
 #pragma unroll
     for (int i = 0; i < NR; ++i) s[i] = Sg[i * PI_WAVE];
   } else {
-    fill(0);
+    fetch(0);
+    put(0);
+    if (chunks > 1) fetch(1);
   }
   __syncthreads();
   for (int c = 0; c < chunks; ++c) {
-    if (wave == PI_SCAN_WAVES) {
-      if (c + 1 < chunks) fill(c + 1);
+    if (wave == WALKERS) {
+      if (c + 1 < chunks) put(c + 1);
+      if (c + 2 < chunks) fetch(c + 2);
     } else {
       const int buf = c & 1, cn = n - c * CH < CH ? n - c * CH : CH;
-#pragma unroll 2
-      for (int tt = 0; tt < cn; ++tt) {
-        const float* qv = &sq[buf][tt * W + part * NR];
-        const float* kv = &sk[buf][tt * W + part * NR];
+      auto take = [&](DeltaToken<NR, LANES>& t, int tt) {
+        t.rows(t.q, &sq[buf][tt * W], part);
+        t.rows(t.k, &sk[buf][tt * W], part);
+        if constexpr (KIND == SCAN_HEAD_DELTA) t.g[0] = sdecay[buf][tt];
+        else t.rows(t.g, &sg[buf][tt * W], part);
+        t.v = sv[buf][tt][cw];
+        t.beta = sbeta[buf][tt];
+      };
+      auto walk = [&](const DeltaToken<NR, LANES>& t, int tt) {
         float u;
         if constexpr (KIND == SCAN_DECAYED_OUTER) {
-          const float* gv = &sg[buf][tt * W + part * NR];
 #pragma unroll
-          for (int i = 0; i < NR; ++i) s[i] *= gv[i];
-          u = sv[buf][tt][cw];
+          for (int i = 0; i < NR; ++i) s[i] *= t.g[i];
+          u = t.v;
         } else {
           float d0 = 0.f, d1 = 0.f;
-          if constexpr (KIND == SCAN_HEAD_DELTA) {
-            const float g1 = sdecay[buf][tt];
 #pragma unroll
-            for (int i = 0; i < NR; ++i) {
-              s[i] *= g1;
-              if (i & 1) d1 = fmaf(s[i], kv[i], d1);
-              else d0 = fmaf(s[i], kv[i], d0);
-            }
-          } else {
-            const float* gv = &sg[buf][tt * W + part * NR];
-#pragma unroll
-            for (int i = 0; i < NR; ++i) {
-              s[i] *= gv[i];
-              if (i & 1) d1 = fmaf(s[i], kv[i], d1);
-              else d0 = fmaf(s[i], kv[i], d0);
-            }
+          for (int i = 0; i < NR; ++i) {
+            s[i] *= t.g[KIND == SCAN_HEAD_DELTA ? 0 : i];
+            if (i & 1) d1 = fmaf(s[i], t.k[i], d1);
+            else d0 = fmaf(s[i], t.k[i], d0);
           }
-          u = sbeta[buf][tt] * (sv[buf][tt][cw] - row16_sum(d0 + d1));
+          u = t.beta * (t.v - lanes_sum<LANES>(d0 + d1));
         }
         float a0 = 0.f, a1 = 0.f;
 #pragma unroll
         for (int i = 0; i < NR; ++i) {
-          s[i] = fmaf(kv[i], u, s[i]);
-          if (i & 1) a1 = fmaf(s[i], qv[i], a1);
-          else a0 = fmaf(s[i], qv[i], a0);
+          s[i] = fmaf(t.k[i], u, s[i]);
+          if (i & 1) a1 = fmaf(s[i], t.q[i], a1);
+          else a0 = fmaf(s[i], t.q[i], a0);
         }
-        const float acc = row16_sum(a0 + a1);
+        const float acc = lanes_sum<LANES>(a0 + a1);
         if (live && part == 0) o[(long)(qs + c * CH + tt) * o_stride + (long)h * dv + col] = acc;
+      };
+      // two tokens in turn, the one read from LDS while the other is walked (past the chunk's last: its last again, unused)
+      DeltaToken<NR, LANES> even, odd;
+      take(even, 0);
+      for (int tt = 0; tt < cn; tt += 2) {
+        take(odd, tt + 1 < cn ? tt + 1 : tt);
+        walk(even, tt);
+        take(even, tt + 2 < cn ? tt + 2 : tt);
+        if (tt + 1 < cn) walk(odd, tt + 1);
       }
     }
     __syncthreads();
   }
-  if (wave < PI_SCAN_WAVES) {
+  if (wave < WALKERS) {
 #pragma unroll
     for (int i = 0; i < NR; ++i) Sg[i * PI_WAVE] = s[i];
   }
@@ -586,17 +635,24 @@ extern "C" int pi_delta_scan(float* o, long o_stride, float* qkv, long qkv_strid
   // bit 0: q and k may be fetched 16 bytes at a time; bit 1: the decays too
   const int vec = (d % 4 == 0 && qkv_stride % 4 == 0 && (uintptr_t)qkv % 16 == 0 ? 1 : 0) |
                   (d % 4 == 0 && a_stride % 4 == 0 && (uintptr_t)a % 16 == 0 ? 2 : 0);
-  const dim3 grid(R, H, (dv + PI_SCAN_COLUMNS - 1) / PI_SCAN_COLUMNS), block((PI_SCAN_WAVES + 1) * PI_WAVE);
-#define PI_LAUNCH_DELTA2(NR_, SHORT_, KIND_)                                                                                                   \
-  hipLaunchKernelGGL((delta_scan_kernel<NR_, SHORT_, KIND_>), grid, block, 0, stream, o, o_stride, qkv, qkv_stride, a, a_stride, b, b_stride, \
-                     q_start, slots, state, state_stride, H, G, d, dv, vec)
-#define PI_LAUNCH_DELTA1(NR_, SHORT_)                                            \
-  do {                                                                           \
-    if (kind == SCAN_HEAD_DELTA) PI_LAUNCH_DELTA2(NR_, SHORT_, SCAN_HEAD_DELTA); \
-    else if (kind == SCAN_DECAYED_OUTER) PI_LAUNCH_DELTA2(NR_, SHORT_, SCAN_DECAYED_OUTER); \
-    else PI_LAUNCH_DELTA2(NR_, SHORT_, SCAN_CHANNEL_DELTA);                      \
+  // Blocks of sixteen columns that leave every other unit idle make way for blocks of eight, a column's rows on twice the lanes
+  const int by16 = (dv + PI_SCAN_COLUMNS - 1) / PI_SCAN_COLUMNS;
+  const bool wide = longest > 2 && (long)R * H * by16 * 2 <= compute_units();
+#define PI_LAUNCH_DELTA2(NR_, SHORT_, KIND_, LANES_)                                                                                           \
+  hipLaunchKernelGGL((delta_scan_kernel<NR_, SHORT_, KIND_, PI_SCAN_WAVES, LANES_>), dim3(R, H, by16 * (LANES_) / 16), dim3((PI_SCAN_WAVES + 1) * PI_WAVE), 0, \
+                     stream, o, o_stride, qkv, qkv_stride, a, a_stride, b, b_stride, q_start, slots, state, state_stride, H, G, d, dv, vec)
+#define PI_LAUNCH_DELTA1(NR_, SHORT_, LANES_)                                            \
+  do {                                                                                   \
+    if (kind == SCAN_HEAD_DELTA) PI_LAUNCH_DELTA2(NR_, SHORT_, SCAN_HEAD_DELTA, LANES_); \
+    else if (kind == SCAN_DECAYED_OUTER) PI_LAUNCH_DELTA2(NR_, SHORT_, SCAN_DECAYED_OUTER, LANES_); \
+    else PI_LAUNCH_DELTA2(NR_, SHORT_, SCAN_CHANNEL_DELTA, LANES_);                      \
   } while (0)
-#define PI_LAUNCH_DELTA(NR_) do { if (longest <= 2) PI_LAUNCH_DELTA1(NR_, true); else PI_LAUNCH_DELTA1(NR_, false); } while (0)
+#define PI_LAUNCH_DELTA(NR_)                                        \
+  do {                                                              \
+    if (longest <= 2) PI_LAUNCH_DELTA1(NR_, true, 16);              \
+    else if ((NR_) >= 8 && wide) PI_LAUNCH_DELTA1(NR_, false, ((NR_) >= 8 ? 32 : 16)); \
+    else PI_LAUNCH_DELTA1(NR_, false, 16);                          \
+  } while (0)
   switch (nr) {
     case 1: PI_LAUNCH_DELTA(1); break;
     case 2: PI_LAUNCH_DELTA(2); break;
