@@ -17,7 +17,7 @@ from typing import Optional
 import torch
 
 from ..errors import KernelError
-from . import _lib
+from . import _lib, fast
 from .workspace import KernelWorkspace, KeyRanges, Partials, stream_layout, stream_layout_takes
 
 PI_F32, PI_BF16 = 0, 1
@@ -70,9 +70,11 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 
 def _rows(t: torch.Tensor, what: str) -> int:
     """Row stride (elements) of a 2-D tensor whose rows are dense."""
-    if t.dim() != 2 or (t.shape[1] > 1 and t.stride(1) != 1):
-        raise KernelError(f"{what}: expected a 2-D tensor with dense rows, got shape {tuple(t.shape)} strides {t.stride()}")
-    return t.stride(0) if t.shape[0] > 1 else max(t.stride(0), t.shape[1])
+    st = t.stride()
+    if len(st) != 2 or (st[1] != 1 and t.shape[1] > 1):
+        raise KernelError(f"{what}: expected a 2-D tensor with dense rows, got shape {tuple(t.shape)} strides {st}")
+    rows, cols = t.shape
+    return st[0] if rows > 1 else max(st[0], cols)
 
 
 def _i32(t: torch.Tensor, what: str, n: Optional[int] = None) -> None:
@@ -172,7 +174,6 @@ def materialize(x: torch.Tensor, ws: Optional[KernelWorkspace]) -> torch.Tensor:
     written)."""
     p = ws.pending if ws is not None else None
     if p is not None and p.is_for(x):
-        from . import fast
         ws.pending = None
         fast.reduce_into(x, p.pieces, accumulate=p.accumulate)
         ws.counts["applied"] += 1
@@ -215,11 +216,9 @@ def gemm_swiglu(out: torch.Tensor, a: torch.Tensor, w_gate_up: torch.Tensor, blo
     if M == 0:
         return
     if _FAST and block == 16 and a.dtype == torch.bfloat16 and w_gate_up.dtype == torch.bfloat16 and out.is_contiguous():
-        from . import fast
         if fast.gemm_swiglu(out, a, w_gate_up, M, 2 * I, a.shape[1], _rows(a, "gemm a"), _rows(w_gate_up, "gemm w"), ws):
             return
     if _FAST and block == 16 and a.dtype == torch.float32 and w_gate_up.dtype == torch.float32 and out.is_contiguous():
-        from . import fast
         if fast.gemm_swiglu_float32(out, a, w_gate_up, M, 2 * I, a.shape[1], _rows(a, "gemm a"), _rows(w_gate_up, "gemm w")):
             return
     gu = torch.empty((M, 2 * I), dtype=a.dtype, device=a.device)
@@ -245,7 +244,6 @@ def gemm(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, accumulate: bool =
             if out.dtype != torch.float32:
                 raise KernelError("gemm: accumulation needs a float32 output")
             materialize(out, ws)
-        from . import fast
         if _FAST and fast.gemm_from_ranges(out, a, w, accumulate, w.shape[0], _rows(w, "gemm w"), _rows(out, "gemm out"),
                                            may_defer and out.dtype == torch.float32 and out.is_contiguous(), ws):
             return
@@ -267,11 +265,9 @@ def gemm(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, accumulate: bool =
     if accumulate:
         materialize(out, ws)
     if _FAST and a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16:
-        from . import fast
         if fast.gemm(out, a, w, accumulate, M, N, K, lda, ldw, ldc, may_defer and out.dtype == torch.float32 and out.is_contiguous(), ws):
             return
     if _FAST and a.dtype == torch.float32 and w.dtype == torch.float32 and out.dtype == torch.float32:
-        from . import fast
         if fast.gemm_float32(out, a, w, accumulate, M, N, K, lda, ldw, ldc, may_defer and out.is_contiguous(), ws):
             return
     _lib.call("core", "pi_gemm_general", out.data_ptr(), _dt(out), ldc, a.data_ptr(), _dt(a), lda, w.data_ptr(),
@@ -324,13 +320,11 @@ def qkv_projection(h: torch.Tensor, w_qkv: torch.Tensor, dtype: torch.dtype, ws:
     (``Partials``), which ``rope_kv_write`` sums on the fly so that the rotation sees float32
     values.  The pieces are good until the next product with the same workspace."""
     if _FAST and ws is not None and h.dtype == torch.bfloat16 and w_qkv.dtype == torch.bfloat16 and h.is_cuda:
-        from . import fast
         p = fast.gemm_pieces(h, w_qkv, ws)
         if p is not None:
             ws.counts["qkv_pieces"] += 1
             return p
     if _FAST and ws is not None and h.dtype == torch.float32 and w_qkv.dtype == torch.float32 and h.is_cuda and h.shape[0] > 0:
-        from . import fast
         p = fast.gemm_float32_pieces(h, w_qkv, ws)
         if p is not None:
             ws.counts["qkv_pieces"] += 1
@@ -423,7 +417,6 @@ def decode_attention_from_projection(out: torch.Tensor, qkv, ctx, rotary, num_he
     filling ``out``, and the product merges them as it reads."""
     if not (_FAST and out.dtype == torch.bfloat16 and out.is_cuda and getattr(ctx, "all_decode", False)):
         return False
-    from . import fast
     if not isinstance(qkv, Partials) and qkv.dtype != torch.bfloat16:
         return False
     T = out.shape[0]
@@ -508,12 +501,10 @@ def paged_attention(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v
         return
     if _FAST and q.dtype == torch.bfloat16 and vd == head_dim and head_dim % 16 == 0 and (plain or scale > 0):
         # the matrix-core kernels take heads whose values are as wide as their keys, options included
-        from . import fast
         if fast.paged_attention(out, q, k_cache, v_cache, block_table, ctx, num_heads, num_kv_heads, head_dim,
                                 page_size, scale, window, pages, ws, slopes, sinks, gate, softcap, out_scale, chunk, gate_stride, keep):
             return
     if _FAST and q.dtype == torch.float32 and vd == head_dim and keep == 0 and not ctx.all_decode:
-        from . import fast
         if fast.paged_attention_float32(out, q, k_cache, v_cache, block_table, ctx, num_heads, num_kv_heads, head_dim,
                                         page_size, scale, window, pages, slopes, sinks, gate, softcap, out_scale, chunk, gate_stride):
             return
@@ -563,13 +554,11 @@ def sample(out: torch.Tensor, logits: torch.Tensor, temperature: Optional[torch.
 # ----------------------------------------------------------------------------- work lists
 def lengths_uneven(kv_lens) -> bool:
     """What a step's ``uneven`` says of its requests' context lengths (see ``fast.lengths_uneven``)."""
-    from . import fast
     return fast.lengths_uneven(kv_lens)
 
 
 def decode_length_bucket(max_kv_len: int) -> int:
     """The context-length bucket that decides a decode step's attention key ranges."""
-    from . import fast
     return fast.decode_length_bucket(max_kv_len)
 
 
@@ -578,14 +567,12 @@ def attention_planner(dtype: torch.dtype, num_heads: int, num_kv_heads: int, hea
     """What makes a step's work lists for an attention mixer of these sizes (a hashable object with
     ``plan(q_lens, kv_lens)``; equal ones share a plan), or None when its kernels need none."""
     if _FAST and dtype == torch.bfloat16 and _lib.build.MODULES["bf16"]:
-        from . import fast
         return fast.attention_planner(dtype, num_heads, num_kv_heads, head_dim, page_size, int(window), torch.device(device), int(chunk or 0), int(keep_first or 0))
     return None
 
 
 def upload_arrays(arrays, device):
     """int32 host arrays by name -> device views of one packed copy."""
-    from . import fast
     return fast.upload_arrays(arrays, device)
 
 
@@ -737,7 +724,6 @@ def gemm_activation(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, activat
     if M == 0:
         return
     if _FAST and a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and out.dtype == torch.bfloat16 and out.is_contiguous():
-        from . import fast
         if fast.gemm_activation(out, a, w, activation, M, N, a.shape[1], _rows(a, "gemm a"), _rows(w, "gemm w")):
             return
     activate(out, qkv_projection(a, w, torch.float32, ws), activation)
@@ -963,7 +949,6 @@ def head_gemm(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, heads: int, a
     if _FAST and a.dtype == torch.bfloat16 and w_rows is not None:
         if w_rows.shape != (heads, N, K) or w_rows.dtype != a.dtype or not w_rows.is_contiguous():
             raise KernelError(f"head product: the row-major weights must be contiguous [{heads}, {N}, {K}] {a.dtype}")
-        from . import fast
         if fast.head_gemm(out, a, w_rows, heads, K, N, a_head, out_head, _rows(a, "head product a"), _rows(out, "head product out"),
                           gate, gate_stride):
             if rot == 0:
@@ -1436,7 +1421,6 @@ def gemm_clamped_glu(out: torch.Tensor, a: torch.Tensor, w_gate_up: torch.Tensor
     if M == 0:
         return
     if _FAST and block == 16 and a.dtype == torch.bfloat16 and w_gate_up.dtype == torch.bfloat16 and out.is_contiguous() and bias.is_contiguous():
-        from . import fast
         if fast.gemm_clamped_glu(out, a, w_gate_up, bias, limit, alpha, M, 2 * I, a.shape[1], _rows(a, "gemm a"), _rows(w_gate_up, "gemm w")):
             if ws is not None:
                 ws.counts["gated_epilogues"] += 1

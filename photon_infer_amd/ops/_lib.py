@@ -97,6 +97,13 @@ def current_stream() -> int:
     return _RAW_STREAM(_CURRENT_DEVICE())
 
 
+def current_device() -> int:
+    """torch's current device, by the same shortest way once the device runtime runs."""
+    if _CURRENT_DEVICE is None or not torch.cuda.is_initialized():
+        return torch.cuda.current_device()
+    return _CURRENT_DEVICE()
+
+
 def load(module: str) -> ctypes.CDLL:
     """The loaded library of ``module``, building it first if it is missing or stale."""
     lib = _LIBS.get(module)
@@ -122,11 +129,16 @@ def load(module: str) -> ctypes.CDLL:
     return lib
 
 
+_ENTRIES: Dict[str, object] = {}      # entry points called before, by name (names are unique over the modules)
+
+
 def call(module: str, name: str, *args) -> None:
-    lib = load(module)
-    rc = getattr(lib, name)(*args)
+    entry = _ENTRIES.get(name)
+    if entry is None:
+        entry = _ENTRIES[name] = getattr(load(module), name)
+    rc = entry(*args)
     if rc != 0:
-        msg = lib._pi_last_error()
+        msg = load(module)._pi_last_error()
         raise KernelError((msg or b"unknown kernel error").decode("utf-8", "replace"))
 
 

@@ -69,7 +69,7 @@ def compute_units() -> int:
     """Compute units of the current device: the split rules below count blocks and waves in
     multiples of it (256 on an MI355X, where they were measured)."""
     try:
-        return _units_of(torch.cuda.current_device())
+        return _units_of(_lib.current_device())
     except Exception:                    # no device in this process (rules asked for on the host)
         return DEFAULT_UNITS
 
@@ -80,7 +80,11 @@ def _gemm_ok(a, w, K, lda, ldw) -> bool:
 
 
 def _skinny_splits(M: int, N: int, K: int) -> int:
-    units = compute_units()
+    return _skinny_splits_of(M, N, K, compute_units())
+
+
+@functools.lru_cache(maxsize=4096)
+def _skinny_splits_of(M: int, N: int, K: int, units: int) -> int:
     if M > SHARED_FROM_TOKENS:     # the kernel that shares an activation tile per block: at most one block per compute unit
         splits = units // -(-N // SHARED_ROWS_PER_BLOCK)
     else:
