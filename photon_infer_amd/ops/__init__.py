@@ -155,7 +155,7 @@ def rmsnorm(out: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, eps: float
         _i32(rows, "rmsnorm rows", M)
     pending = ws.take_pending(x) if ws is not None else None
     if pending is not None:
-        ws.counts["added_by_norm"] += 1
+        ws.counts_of(pending)["added_by_norm"] += 1
     part, splits = (pending.part.data_ptr(), pending.splits) if pending is not None else (None, 0)
     _lib.call("core", "pi_rmsnorm", out.data_ptr(), _dt(out), x.data_ptr(), _ptr(rows), weight.data_ptr(),
               _dt(weight), float(eps), M, D, part, splits, x.shape[0], _stream())
@@ -176,7 +176,7 @@ def materialize(x: torch.Tensor, ws: Optional[KernelWorkspace]) -> torch.Tensor:
     if p is not None and p.is_for(x):
         ws.pending = None
         fast.reduce_into(x, p.pieces, accumulate=p.accumulate)
-        ws.counts["applied"] += 1
+        ws.counts_of(p.pieces)["applied"] += 1
     return x
 
 
@@ -188,8 +188,9 @@ def reset_deferred(ws: Optional[KernelWorkspace]) -> None:
 
 def discard_deferred(x: torch.Tensor, ws: Optional[KernelWorkspace]) -> None:
     """Forget a pending update of ``x`` (the stream is not read again)."""
-    if ws is not None and ws.take_pending(x) is not None:
-        ws.counts["discarded"] += 1
+    pieces = ws.take_pending(x) if ws is not None else None
+    if pieces is not None:
+        ws.counts_of(pieces)["discarded"] += 1
 
 
 def swiglu(out: torch.Tensor, gate_up: torch.Tensor, block: int = 0) -> None:
@@ -322,12 +323,12 @@ def qkv_projection(h: torch.Tensor, w_qkv: torch.Tensor, dtype: torch.dtype, ws:
     if _FAST and ws is not None and h.dtype == torch.bfloat16 and w_qkv.dtype == torch.bfloat16 and h.is_cuda:
         p = fast.gemm_pieces(h, w_qkv, ws)
         if p is not None:
-            ws.counts["qkv_pieces"] += 1
+            ws.counts_of(p)["qkv_pieces"] += 1
             return p
     if _FAST and ws is not None and h.dtype == torch.float32 and w_qkv.dtype == torch.float32 and h.is_cuda and h.shape[0] > 0:
         p = fast.gemm_float32_pieces(h, w_qkv, ws)
         if p is not None:
-            ws.counts["qkv_pieces"] += 1
+            ws.counts_of(p)["qkv_pieces"] += 1
             return p
     out = torch.empty((h.shape[0], w_qkv.shape[0]), dtype=dtype, device=h.device)
     gemm(out, h, w_qkv, ws=ws)
@@ -668,7 +669,7 @@ def rms_join(x: torch.Tensor, y: torch.Tensor, post: torch.Tensor, post_eps: flo
             raise KernelError(f"rms join: expert rows must be contiguous float32 [{T * top}, {D}], got {a.dtype} {tuple(a.shape)}")
         _f32_vector(weights.view(-1), entries, "rms join choice weights")
     elif pieces is not None:
-        ws.counts["added_by_join"] += 1
+        ws.counts_of(pieces)["added_by_join"] += 1
         if (pieces.M, pieces.N) != (T, D):
             raise KernelError(f"rms join: pieces [{pieces.M}, {pieces.N}] of a result [{T}, {D}]")
     else:
@@ -1463,7 +1464,7 @@ def hyper_streams(x: torch.Tensor, *, y: Optional[torch.Tensor] = None, post: Op
     if y is not None:
         _f32_vector(post, n + n * n, "hyper streams mix")
         if pieces is not None:
-            ws.counts["added_by_streams"] += 1
+            ws.counts_of(pieces)["added_by_streams"] += 1
             if (pieces.M, pieces.N) != (T, D):
                 raise KernelError(f"hyper streams: pieces [{pieces.M}, {pieces.N}] of a result [{T}, {D}]")
         elif y.dtype != torch.float32 or not y.is_contiguous() or tuple(y.shape) != (T, D):

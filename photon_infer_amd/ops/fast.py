@@ -122,7 +122,7 @@ def flush(ws: Optional[KernelWorkspace]) -> None:
         return
     p, ws.pending = ws.pending, None
     reduce_into(p.target, p.pieces, accumulate=p.accumulate)
-    ws.counts["flushed"] += 1
+    ws.counts_of(p.pieces)["flushed"] += 1
 
 
 def _piece_buffer(ws: Optional[KernelWorkspace], floats: int, device) -> torch.Tensor:
@@ -238,8 +238,8 @@ def _float32_product(out, a, w, accumulate, M, N, K, lda, ldw, ldc, ws: Optional
     if buf is None:
         return None
     if ws is not None:
-        ws.counts["split_products"] += 1
-    return Partials(buf, made, M, N)
+        ws.float32_counts["split_products"] += 1
+    return Partials(buf, made, M, N, of_float32=True)
 
 
 def gemm_float32(out, a, w, accumulate, M, N, K, lda, ldw, ldc, may_defer=False, ws: Optional[KernelWorkspace] = None) -> bool:
@@ -251,7 +251,7 @@ def gemm_float32(out, a, w, accumulate, M, N, K, lda, ldw, ldc, may_defer=False,
     pieces = _float32_product(out, a, w, accumulate, M, N, K, lda, ldw, ldc, ws, may_defer)
     if pieces is not None and may_defer:
         ws.pending = PendingUpdate(out, pieces, accumulate)
-        ws.counts["deferred"] += 1
+        ws.float32_counts["deferred"] += 1
     elif pieces is not None:
         _lib.call("core", "pi_splitk_reduce", out.data_ptr(), EPI_ACCUM if accumulate else EPI_F32, ldc, pieces.part.data_ptr(), pieces.splits, M, N, _stream())
     return True

@@ -22,12 +22,14 @@ SAMPLE_FLOATS = 1 << 18        # chunk records of the sampling kernels
 
 @dataclass
 class Partials:
-    """A product [M, N] whose k-range was split: ``part`` holds float32 [splits, M, N]."""
+    """A product [M, N] whose k-range was split: ``part`` holds float32 [splits, M, N].  ``of_float32``: the product
+    of a float32 model, whose statistics are kept apart."""
 
     part: torch.Tensor
     splits: int
     M: int
     N: int
+    of_float32: bool = False
 
 
 @dataclass
@@ -84,7 +86,8 @@ def stream_layout(w: torch.Tensor) -> Optional[torch.Tensor]:
 class KernelWorkspace:
     """Buffers are made at first use and kept; ``counts`` says which paths a step took (tests
     read it: ``split_products``, ``deferred``, ``added_by_norm``, ``applied``, ``flushed``,
-    ``discarded``, ``qkv_pieces``, ``ranges_merged_by_product``)."""
+    ``discarded``, ``qkv_pieces``, ``ranges_merged_by_product``).  ``counts`` is about the 16-bit
+    products; ``float32_counts`` has the same entries for pieces of float32 products."""
 
     def __init__(self, device):
         self.device = torch.device(device)
@@ -94,10 +97,15 @@ class KernelWorkspace:
         self._sample_part: Optional[torch.Tensor] = None
         self.pending: Optional[PendingUpdate] = None
         self.counts: Counter = Counter()
+        self.float32_counts: Counter = Counter()
         # weight matrices that have a second copy in the order the weight-streaming kernels read
         # (steps of up to 128 tokens): address of the matrix -> (copy, rows, columns, the matrix
         # itself: while it is kept here, nothing else can come to lie at its address)
         self.stream_copies: Dict[int, Tuple[torch.Tensor, int, int, torch.Tensor]] = {}
+
+    def counts_of(self, pieces: Partials) -> Counter:
+        """The statistics that ``pieces`` belong to."""
+        return self.float32_counts if pieces.of_float32 else self.counts
 
     def _buffer(self, name: str, floats: int) -> torch.Tensor:
         buf = getattr(self, name)

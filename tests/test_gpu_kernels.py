@@ -371,7 +371,8 @@ def test_float32_pieces_are_added_by_the_next_reader(_ops, M, N, K):
     _ops.gemm(x, a, w, accumulate=True, may_defer=True, ws=ws)
     h = torch.empty_like(x)
     _ops.rmsnorm(h, x, torch.ones(N, device=DEV), 1e-5, ws=ws)
-    assert ws.pending is None
+    assert ws.pending is None and not ws.counts                  # the 16-bit products' statistics: nothing of these
+    assert ws.float32_counts["added_by_norm"] == ws.float32_counts["deferred"] == ws.float32_counts["split_products"]
     close(x, want.cpu(), 2 ** -23 * (8 + K ** 0.5), "stream")
     close(h, (want / (want.pow(2).mean(-1, keepdim=True) + 1e-5).sqrt()).cpu(), 2 ** -22 * (8 + K ** 0.5), "norm")
     p = _ops.qkv_projection(a, w, F32, ws)
