@@ -380,6 +380,36 @@ def test_float32_pieces_are_added_by_the_next_reader(_ops, M, N, K):
     close(got, (a.double() @ w.double().t()).cpu(), 2 ** -23 * (8 + K ** 0.5), "projection")
 
 
+@pytest.mark.parametrize("hd,R", [(64, 32), (64, 64), (16, 8), (128, 24), (64, 12), (256, 256)])
+@pytest.mark.parametrize("source", ["tensor", "pieces"])
+def test_neighbours_turned_for_many_tokens_and_for_few(_ops, hd, R, source):
+    """Forty tokens at a time and nine, which go to the kernel of single pairs: the same bits in queries, keys and values."""
+    nh, nkv, T, page = 4, 2, 40, 16
+    cols = (nh + 2 * nkv) * hd
+    x = torch.randn(T, cols, generator=gen(hd + R)).to(BF16).to(DEV)
+    pieces = torch.randn(3, T, cols, generator=gen(R)).to(DEV)
+    pos = torch.arange(5, 5 + T, dtype=torch.int32, device=DEV)
+    table = _ops.rope_table(pos, torch.rand(R // 2, generator=gen(1)).to(DEV))
+    blocks = torch.tensor([[3, 0, 2, 1]], dtype=torch.int32, device=DEV)
+    req = torch.zeros(T, dtype=torch.int32, device=DEV)
+    results = []
+    for step in (T, 9):
+        q = x[:, :nh * hd].clone()
+        kc, vc = torch.zeros(4, nkv, page, hd, dtype=BF16, device=DEV), torch.zeros(4, nkv, hd, page, dtype=BF16, device=DEV)
+        for t in range(0, T, step):
+            e = min(T, t + step)
+            rows, rot = x[t:e], (table[t:e].contiguous(), R, True)
+            if source == "tensor":
+                _ops.rope_kv_write(q[t:e], rows[:, nh * hd:(nh + nkv) * hd], rows[:, (nh + nkv) * hd:], pos[t:e], req[t:e], rot, nh, nkv, hd, kc, vc, blocks, page)
+            else:
+                part = _ops.Partials(pieces[:, t:e].contiguous(), 3, e - t, cols)
+                _ops.rope_kv_write(q[t:e], None, None, pos[t:e], req[t:e], rot, nh, nkv, hd, kc, vc, blocks, page, pieces=part, write_kv=True)
+        results.append((q, kc, vc))
+    for many, few in zip(*results):
+        assert torch.equal(many, few)
+    assert results[0][0].float().abs().max() > 0 and results[0][1].float().abs().max() > 0
+
+
 def test_gemm_reference_vectors(_ops):
     # tests/ops/test_matmul.cpp:90-204
     W = torch.tensor([[1.0, 2.0, 3.0], [4.0, 5.0, 6.0]], device=DEV)
