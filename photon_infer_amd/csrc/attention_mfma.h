@@ -117,6 +117,14 @@ struct KVChunk {
   __device__ inline Frag val(int db) const { return v[db]; }
 };
 
+// One tile of 16 keys on its way to LDS.
+template <int HD>
+struct KVTile {
+  u32x4_t k[HeadFrags<HD>::KS];
+  uint2 v[HD / 16];
+  bool have;
+};
+
 // The same chunk lying in LDS in operand order ([fragment][lane], keys first): a fragment is
 // read when the arithmetic wants it, so that a chunk never occupies registers as a whole.
 template <int HD>
@@ -229,30 +237,43 @@ struct KVLaneOffsets {
   }
 };
 
-// Issue the loads of a chunk of 32 keys.  The loads are unconditional (a missing tile reads
-// page 0 and is zeroed by attn_compute), so that the compiler can count them and wait for one
-// chunk while the next is still in flight.  A tile's base address is the same in every lane
-// (scalar arithmetic); the lane's part is a 32-bit offset.
+// Where a tile of 16 keys lies; a missing one reads page 0 and is zeroed by attn_compute.  The base
+// addresses are the same in every lane (scalar arithmetic); the lane's part is a 32-bit offset.
+template <int HD>
+struct KVTileAt {
+  const char *keys, *values;
+  bool have;
+  __device__ inline KVTileAt(int page, int slot, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache, int nkv, int g,
+                             int page_size, int num_pages) {
+    const long page_elems = addressing::kv_page_elems(nkv, page_size, HD);
+    have = addressing::kv_page_there(page, num_pages);
+    const long pg = addressing::kv_page_or_first(page, num_pages);
+    keys = reinterpret_cast<const char*>(k_cache + addressing::kv_key_tile(pg, page_elems, g, page_size, slot, HD));
+    values = reinterpret_cast<const char*>(v_cache + addressing::kv_value_tile(pg, page_elems, g, page_size, slot, HD));
+  }
+  __device__ inline u32x4_t key(const KVLaneOffsets<HD>& off, int ks) const {
+    // a half fragment's upper lanes read their row's first features again and count as zero
+    const bool held = HD % 32 == 0 || ks + 1 < HeadFrags<HD>::KS || off.tail;
+    const u32x4_t n = *reinterpret_cast<const u32x4_t*>(keys + (held ? off.k + ks * 64 : off.k0));
+    return held ? n : u32x4_t{0u, 0u, 0u, 0u};
+  }
+  __device__ inline uint2 value(const KVLaneOffsets<HD>& off, int db) const { return *reinterpret_cast<const uint2*>(values + off.v[db]); }
+};
+
+// Issue the loads of a chunk of 32 keys.  The loads are unconditional, so that the compiler can
+// count them and wait for one chunk while the next is still in flight.
 template <int HD>
 __device__ inline void attn_load(KVChunk<HD>& kv, const ChunkPages& cp, const bf16_t* __restrict__ k_cache,
                                  const bf16_t* __restrict__ v_cache, const KVLaneOffsets<HD>& off, int nkv, int g,
                                  int page_size, int num_pages) {
-  const long page_elems = addressing::kv_page_elems(nkv, page_size, HD);
 #pragma unroll
   for (int t = 0; t < 2; ++t) {
-    kv.have[t] = addressing::kv_page_there(cp.page[t], num_pages);
-    const long pg = addressing::kv_page_or_first(cp.page[t], num_pages);
-    const char* kp = reinterpret_cast<const char*>(k_cache + addressing::kv_key_tile(pg, page_elems, g, page_size, cp.slot[t], HD));
-    const char* vp = reinterpret_cast<const char*>(v_cache + addressing::kv_value_tile(pg, page_elems, g, page_size, cp.slot[t], HD));
+    const KVTileAt<HD> at(cp.page[t], cp.slot[t], k_cache, v_cache, nkv, g, page_size, num_pages);
+    kv.have[t] = at.have;
 #pragma unroll
-    for (int ks = 0; ks < HeadFrags<HD>::KS; ++ks) {
-      // a half fragment's upper lanes read their row's first features again and count as zero
-      const bool held = HD % 32 == 0 || ks + 1 < HeadFrags<HD>::KS || off.tail;
-      kv.k[t][ks].n = *reinterpret_cast<const u32x4_t*>(kp + (held ? off.k + ks * 64 : off.k0));
-      if (!held) kv.k[t][ks].n = u32x4_t{0u, 0u, 0u, 0u};
-    }
+    for (int ks = 0; ks < HeadFrags<HD>::KS; ++ks) kv.k[t][ks].n = at.key(off, ks);
 #pragma unroll
-    for (int db = 0; db < HD / 16; ++db) kv.v[db].d[t] = *reinterpret_cast<const uint2*>(vp + off.v[db]);
+    for (int db = 0; db < HD / 16; ++db) kv.v[db].d[t] = at.value(off, db);
   }
 }
 

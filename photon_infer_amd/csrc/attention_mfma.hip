@@ -8,13 +8,14 @@
 // of them from the pages into registers while all four compute on the previous 128, which
 // they share through LDS (stored in the very order the matrix-core operands want them, so
 // both the writes and the reads are 16 bytes per lane, lane after lane).  One barrier per 128
-// keys.  Heads of more than 128 features take 64 keys at a time (two of the waves fetch) and
+// keys.  Heads of more than 128 features take 64 keys at a time (each wave fetches 16) and
 // 16 columns per wave: two rounds of 128 would not fit the LDS, nor the state the registers.  A token at absolute position p sees keys lo..p only (lo = 0, or p - window + 1, or the start of p's chunk),
 // whatever portion it arrived in; a wave skips the 32-key chunks none of its columns sees.
 //
 // The host sorts the tiles by the number of keys they walk and deals them out to the blocks
 // of a kv head in rounds, back and forth, so that every block gets about the same work.
 #include "attention_mfma.h"
+#include <type_traits>
 
 #ifndef PLAIN_NJ
 #define PLAIN_NJ 4   // chunks of a fully visible round that are folded as one group (2 or 4)
@@ -104,22 +105,31 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HD <= 64 ? 
       attn_load_q(st, c, q, q_stride, rows[c], heads[c], valid[c], lane);
     }
 
-    // this wave's 32 keys of every round (the first NCH waves fetch): where they lie
-    // (a constant where every wave fetches: behind a branch the compiler waits for the loads at
-    // the branch's end instead of at their first use, and the round loses its overlap: 63 us
-    // instead of 53 for a 2,048-token prompt at head size 64)
-    const bool fetches = NCH == 4 || wave < NCH;
+    // This wave's quarter of every round, a chunk of 32 keys or (NCH 2) a tile of 16: where it lies.  All waves fetch, without a
+    // branch: behind one the compiler waits for the loads at the branch's end instead of at their first use, and the round loses
+    // its overlap (63 us instead of 53 for a 2,048-token prompt at head size 64; at head size 256, where two waves fetched a
+    // chunk each and 146 registers went to memory, 158 us instead of 142 for prompts of 1,501 and 1,126 tokens, 16 heads of one kv head).
+    constexpr bool CHUNKS = NCH == 4;
+    constexpr int KEYS_OF_WAVE = KEYS_PER_ROUND / 4;
     PageCursor cur;
-    cur.start(block_table + (long)r * table_width, table_width, kv_len, page_size, round_of(sc0) * KEYS_PER_ROUND + wave * 32);
+    cur.start(block_table + (long)r * table_width, table_width, kv_len, page_size, round_of(sc0) * KEYS_PER_ROUND + wave * KEYS_OF_WAVE);
     // where the fetch of the window's first round lands, if kept rounds come before it
-    const int jump_key = OPT && gap > 0 && sc0 < head ? head * KEYS_PER_ROUND + wave * 32 : -1;
-    const int land_key = all0 * KEYS_PER_ROUND + wave * 32, land_blk = land_key / page_size, land_slot = land_key - land_blk * page_size;
-    KVChunk<HD> pre;
+    const int jump_key = OPT && gap > 0 && sc0 < head ? head * KEYS_PER_ROUND + wave * KEYS_OF_WAVE : -1;
+    const int land_key = all0 * KEYS_PER_ROUND + wave * KEYS_OF_WAVE, land_blk = land_key / page_size, land_slot = land_key - land_blk * page_size;
+    std::conditional_t<CHUNKS, KVChunk<HD>, KVTile<HD>> pre;
     auto fetch = [&]() {
-      if (!fetches) return;
-      PageCursor two = cur;                        // the chunk's two tiles
+      PageCursor two = cur;                        // the next two tiles (the second is the next wave's if this one fetches tiles)
       const ChunkPages cp = two.next();
-      attn_load<HD>(pre, cp, k_cache, v_cache, off, nkv, g, page_size, num_pages);
+      if constexpr (CHUNKS) {
+        attn_load<HD>(pre, cp, k_cache, v_cache, off, nkv, g, page_size, num_pages);
+      } else {
+        const KVTileAt<HD> at(cp.page[0], cp.slot[0], k_cache, v_cache, nkv, g, page_size, num_pages);
+        pre.have = at.have;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) pre.k[ks] = at.key(off, ks);
+#pragma unroll
+        for (int db = 0; db < HD / 16; ++db) pre.v[db] = at.value(off, db);
+      }
       cur.key += KEYS_PER_ROUND;
       cur.blk += step_blk;
       cur.slot += step_slot;
@@ -132,16 +142,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HD <= 64 ? 
       }
     };
     auto stash = [&](int buf) {
-      if (!fetches) return;
-      u32x4_t* mine = staged + ((buf * NCH + wave) * F) * 64 + lane;
+      if constexpr (CHUNKS) {
+        u32x4_t* mine = staged + ((buf * NCH + wave) * F) * 64 + lane;
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+        for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) mine[(t * KS + ks) * 64] = pre.k[t][ks].n;
+          for (int ks = 0; ks < KS; ++ks) mine[(t * KS + ks) * 64] = pre.k[t][ks].n;
 #pragma unroll
-      for (int db = 0; db < HD / 16; ++db)
-        mine[(2 * KS + db) * 64] = u32x4_t{pre.v[db].d[0].x, pre.v[db].d[0].y, pre.v[db].d[1].x, pre.v[db].d[1].y};
-      if (lane < 2) present[buf][wave][lane] = lane == 0 ? pre.have[0] : pre.have[1];
+        for (int db = 0; db < HD / 16; ++db)
+          mine[(2 * KS + db) * 64] = u32x4_t{pre.v[db].d[0].x, pre.v[db].d[0].y, pre.v[db].d[1].x, pre.v[db].d[1].y};
+        if (lane < 2) present[buf][wave][lane] = lane == 0 ? pre.have[0] : pre.have[1];
+      } else {
+        u32x4_t* mine = staged + ((buf * NCH + wave / 2) * F) * 64 + lane;
+        const int t = wave % 2;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) mine[(t * KS + ks) * 64] = pre.k[ks];
+#pragma unroll
+        for (int db = 0; db < HD / 16; ++db) reinterpret_cast<uint2*>(mine + (2 * KS + db) * 64)[t] = pre.v[db];
+        if (lane == 0) present[buf][wave / 2][t] = pre.have;
+      }
     };
 
     fetch();
