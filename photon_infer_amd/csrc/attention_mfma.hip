@@ -13,7 +13,7 @@
 // whatever portion it arrived in; a wave skips the 32-key chunks none of its columns sees.
 //
 // The host sorts the tiles by the number of keys they walk and deals them out to the blocks
-// of a kv head in rounds, back and forth, so that every block gets about the same work.
+// of a kv head in rounds, the longest of a round to the block that has least so far.
 #include "attention_mfma.h"
 #include <type_traits>
 

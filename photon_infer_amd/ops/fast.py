@@ -435,16 +435,21 @@ def attention_blocks_per_unit(head_dim: int) -> int:
 
 
 def deal_tiles(walks: List[int], seats: int) -> np.ndarray:
-    """[rounds, seats] tile indices (-1: none): the tiles sorted by the keys they walk, longest
-    first, dealt to ``seats`` blocks back and forth so that the blocks' sums come out close."""
-    by_work = sorted(range(len(walks)), key=lambda i: -walks[i])
+    """[rounds, seats] tile indices (-1: none): the tiles sorted by the keys they walk, longest first, a round at a time, and
+    in every round the longest to the block that has least so far.  The blocks' sums then differ by no more than the longest
+    and the shortest tile of one round (a seat left empty counts as a tile of nothing).  Dealt back and forth without a look
+    at the sums, a last round that is not full fell to the blocks with the longest tiles: two prompts of 1,501 and 1,126
+    tokens in tiles of four on 256 blocks ended with 36 rounds of keys in the longest block instead of 32, 28 in the mean
+    (heads of 256: 142 us, now 132)."""
+    work = np.asarray(walks, np.int64)
+    by_work = np.argsort(-work, kind="stable")
     rounds = -(-len(by_work) // seats)
-    order = np.full((rounds, seats), -1, np.int32)
+    order, dealt = np.full((rounds, seats), -1, np.int32), np.zeros(seats, np.int64)
     for k in range(rounds):
         part = by_work[k * seats:(k + 1) * seats]
-        cols = range(len(part)) if k % 2 == 0 else range(seats - 1, seats - 1 - len(part), -1)
-        for c, t in zip(cols, part):
-            order[k, c] = t
+        cols = np.argsort(dealt, kind="stable")[:len(part)]
+        order[k, cols] = part
+        dealt[cols] += work[part]
     return order
 
 

@@ -29,6 +29,17 @@ def test_the_deal_evens_out_the_work():
     assert sorted(walks[t] for t in order[0]) == list(range(97, 129))
 
 
+@pytest.mark.parametrize("lens,rows,seats", [([1501, 1126], 4, 256), ([2048], 32, 24), ([90, 700, 31], 8, 40), ([300], 4, 74)])
+def test_a_last_round_that_is_not_full_goes_to_the_blocks_with_least(lens, rows, seats):
+    """Longest tile to the least loaded block: a round cannot widen the spread of the sums beyond its own tiles' spread."""
+    walks = [(start + min(rows, n - start) - 1) // 128 + 1 for n in lens for start in range(0, n, rows)]
+    order = deal_tiles(walks, seats)
+    work = np.where(order >= 0, np.asarray(walks)[order], 0)
+    sums = work.sum(0)
+    assert sums.max() - sums.min() <= max(r.max() - r.min() for r in work)
+    assert sums.sum() == sum(walks)
+
+
 def test_fewer_tiles_than_seats():
     order = deal_tiles([3, 9], 8)
     assert order.shape == (1, 8)
