@@ -444,6 +444,10 @@ def deal_tiles(walks: List[int], seats: int) -> np.ndarray:
     work = np.asarray(walks, np.int64)
     by_work = np.argsort(-work, kind="stable")
     rounds = -(-len(by_work) // seats)
+    if rounds == 1:
+        order = np.full((1, seats), -1, np.int32)
+        order[0, :len(by_work)] = by_work
+        return order
     order, dealt = np.full((rounds, seats), -1, np.int32), np.zeros(seats, np.int64)
     for k in range(rounds):
         part = by_work[k * seats:(k + 1) * seats]
