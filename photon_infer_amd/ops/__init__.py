@@ -319,11 +319,13 @@ def qkv_projection(h: torch.Tensor, w_qkv: torch.Tensor, dtype: torch.dtype, ws:
     """h @ w_qkv^T for the attention mixer: a tensor [T, N] in ``dtype``, or - when the
     product was split over k and there is a workspace to keep them in - its pieces
     (``Partials``), which ``rope_kv_write`` sums on the fly so that the rotation sees float32
-    values.  The pieces are good until the next product with the same workspace."""
+    values.  The pieces are good until the next product with the same workspace.  A result of bfloat16
+    that is not split may come as one float32 piece too (``fast.keeps_float32``)."""
     if _FAST and ws is not None and h.dtype == torch.bfloat16 and w_qkv.dtype == torch.bfloat16 and h.is_cuda:
-        p = fast.gemm_pieces(h, w_qkv, ws)
+        p = fast.gemm_pieces(h, w_qkv, ws, whole=dtype == torch.bfloat16)
         if p is not None:
-            ws.counts_of(p)["qkv_pieces"] += 1
+            if p.splits > 1:
+                ws.counts_of(p)["qkv_pieces"] += 1
             return p
     if _FAST and ws is not None and h.dtype == torch.float32 and w_qkv.dtype == torch.float32 and h.is_cuda and h.shape[0] > 0:
         p = fast.gemm_float32_pieces(h, w_qkv, ws)

@@ -331,8 +331,18 @@ def gemm_from_ranges(out, kr: KeyRanges, w, accumulate, N, ldw, ldc, may_defer, 
     return True
 
 
-def gemm_pieces(a, w, ws: Optional[KernelWorkspace]) -> Optional[Partials]:
-    """a @ w^T left in pieces in the workspace, if this product is one whose k-range is split."""
+def keeps_float32(M: int, N: int, K: int, units: int) -> bool:
+    """Whether q, k, v that no cut of k leaves in float32 pieces still go to the rotation in float32, as one piece: while
+    their tiles of 128 x 128 do not outnumber the units.  Results of that size are rounded once, behind the rotation,
+    whatever the plan of the day says about pieces; larger ones, which a cut never paid for, are stored in bfloat16 (one
+    float32 piece instead, product and rotation: 543 x 6,144 x 4,096 43.0 -> 46.0 us, 1,280 x 3,072 x 2,048 27.6 -> 31.5;
+    2,048 x 3,072 x 2,048 would be 37.9 -> 42.3).  Not for 32 tokens and fewer, nor for a k too short to be cut in two."""
+    return M > SHARED_FROM_TOKENS and K >= 512 and -(-M // 128) * -(-N // 128) <= units
+
+
+def gemm_pieces(a, w, ws: Optional[KernelWorkspace], whole: bool = False) -> Optional[Partials]:
+    """a @ w^T left in float32 pieces in the workspace, if this product is one whose k-range is split; with ``whole``
+    also a product in one piece (memory of its own) where ``keeps_float32`` says so."""
     if ws is None:
         return None
     M, K = a.shape
@@ -340,18 +350,24 @@ def gemm_pieces(a, w, ws: Optional[KernelWorkspace]) -> Optional[Partials]:
     lda, ldw = a.stride(0) if M > 1 else K, w.stride(0)
     if not _gemm_ok(a, w, K, lda, ldw) or a.stride(1) != 1 or w.stride(1) != 1:
         return None
+    p = None
     if M > SKINNY_MAX_ROWS:
         # a prompt portion of a few hundred tokens has too few tiles for the chip: split k there
         # too, the consumer adds the pieces
         splits = _tile_splits(M, N, K)
-        if splits <= 1 or _tile_splits_of(M, N, K, compute_units(), PIECES_WORTH) <= 1:
-            return None
-        p = _tiles_in_pieces(a, w, M, N, K, lda, ldw, splits, ws)
-        return p if p.splits > 1 else None
-    splits = _skinny_splits(M, N, K)
-    if splits <= 1:
+        if splits > 1 and _tile_splits_of(M, N, K, compute_units(), PIECES_WORTH) > 1:
+            p = _tiles_in_pieces(a, w, M, N, K, lda, ldw, splits, ws)
+    else:
+        splits = _skinny_splits(M, N, K)
+        if splits > 1:
+            p = _skinny(0, EPI_F32, N, a, w, M, N, K, lda, ldw, splits, ws)
+    if p is not None and p.splits > 1:
+        return p
+    if not whole or not keeps_float32(M, N, K, compute_units()):
         return None
-    return _skinny(0, EPI_F32, N, a, w, M, N, K, lda, ldw, splits, ws)
+    out = torch.empty((1, M, N), dtype=torch.float32, device=a.device)
+    gemm(out[0], a, w, False, M, N, K, lda, ldw, N, ws=ws)
+    return Partials(out, 1, M, N)
 
 
 EPI_GATE = 7

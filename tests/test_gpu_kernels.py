@@ -380,6 +380,17 @@ def test_float32_pieces_are_added_by_the_next_reader(_ops, M, N, K):
     close(got, (a.double() @ w.double().t()).cpu(), 2 ** -23 * (8 + K ** 0.5), "projection")
 
 
+@pytest.mark.parametrize("M,N,K", [(33, 8256, 512), (100, 10240, 1024), (128, 16320, 512), (129, 3072, 2048), (641, 3072, 2048), (1280, 3072, 520), (543, 6144, 1024)])
+def test_projections_of_some_hundred_tokens_stay_in_float32_for_the_rotation(_ops, M, N, K):
+    """Few enough tiles: pieces or one float32 piece, never bfloat16 (32-bit sums of K products against 64 bits)."""
+    _ops.use_fast_kernels(True)
+    a, w = torch.randn(M, K, generator=gen(M)).to(BF16).to(DEV), (torch.randn(N, K, generator=gen(N)) / K ** 0.5).to(BF16).to(DEV)
+    p = _ops.qkv_projection(a, w, BF16, _ops.KernelWorkspace(DEV))
+    assert isinstance(p, _ops.Partials) and p.part.dtype == F32 and (p.M, p.N) == (M, N)
+    got = p.part.view(-1)[:p.splits * M * N].view(p.splits, M, N).double().sum(0)
+    close(got, (a.double() @ w.double().t()).cpu(), 2 ** -23 * (8 + K ** 0.5), f"{M} x {N} x {K}")
+
+
 @pytest.mark.parametrize("hd,R", [(64, 32), (64, 64), (16, 8), (128, 24), (64, 12), (256, 256)])
 @pytest.mark.parametrize("source", ["tensor", "pieces"])
 def test_neighbours_turned_for_many_tokens_and_for_few(_ops, hd, R, source):

@@ -170,6 +170,16 @@ def test_a_product_is_left_in_as_many_pieces_as_were_the_fastest(M, N, K, times)
     assert times[fast._tile_splits_of(M, N, K, 256, 1.0) - 1] <= 1.05 * min(times)
 
 
+@pytest.mark.parametrize("N,K,tokens", [(3072, 2048, 1280), (5120, 3072, 768), (6144, 4096, 640), (2560, 1024, 1024), (4608, 3584, 896), (8256, 4096, 128),
+                                        (10240, 8192, 128), (16320, 512, 128)])
+def test_queries_keys_and_values_of_some_hundred_tokens_reach_the_rotation_in_float32(N, K, tokens):
+    """Cut over k or not: from 33 tokens on as long as the result has no more tiles than the chip has units."""
+    from photon_infer_amd.ops import fast
+    for M in range(33, tokens + 1):
+        cut = fast._skinny_splits_of(M, N, K, 256) if M <= fast.SKINNY_MAX_ROWS else fast._tile_splits_of(M, N, K, 256, fast.PIECES_WORTH)
+        assert cut > 1 or fast.keeps_float32(M, N, K, 256), M
+
+
 def test_a_token_count_that_was_not_seen_before_costs_little_to_plan(monkeypatch):
     """In continuous batching the token count changes nearly every step.  Four products of a 1B layer, planned for counts that
     no step had: 13 microseconds in the library (135 in Python), the best of several rounds taken for a busy machine."""
