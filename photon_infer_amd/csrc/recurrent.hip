@@ -463,6 +463,125 @@ __global__ __launch_bounds__(PI_WAVE) void delta_prepare_kernel(float* __restric
   if (lane == 0) b[t * b_stride + h] = sigmoid_f(b[t * b_stride + h]);
 }
 
+// Then the walk: q^, k^ and v from qkv, decays from a, beta from b.  A column of S never meets another
+// column, so a wave walks its four columns alone.
+template <int NR, bool SHORT, int KIND>
+__global__ __launch_bounds__((PI_SCAN_WAVES + 1) * PI_WAVE) void delta_scan_kernel(
+    float* __restrict__ o, long o_stride, const float* __restrict__ qkv, long qkv_stride, const float* __restrict__ decay,
+    long decay_stride, const float* __restrict__ beta, long beta_stride, const int* __restrict__ q_start,
+    const int* __restrict__ slots, float* __restrict__ state, long state_stride, int H, int G, int d, int dv, int vec) {
+  constexpr int W = ScanShape<NR, SHORT>::W, CH = ScanShape<NR, SHORT>::CH;
+  __shared__ __attribute__((aligned(16))) float sq[2][CH * W];
+  __shared__ __attribute__((aligned(16))) float sk[2][CH * W];
+  __shared__ __attribute__((aligned(16))) float sg[2][KIND == SCAN_HEAD_DELTA ? 4 : CH * W];
+  __shared__ float sv[2][CH][PI_SCAN_COLUMNS], sbeta[2][CH], sdecay[2][CH];
+  const int r = blockIdx.x, h = blockIdx.y, z = blockIdx.z;
+  const int wave = threadIdx.x / PI_WAVE, lane = threadIdx.x % PI_WAVE, part = lane % 16;
+  const int g = h / (H / G);
+  const int qs = q_start[r], n = q_start[r + 1] - qs;
+  if (n <= 0) return;
+  const int chunks = (n + CH - 1) / CH;
+  const long q_col = (long)g * d, k_col = (long)G * d + (long)g * d, v_col = 2L * G * d + (long)h * dv + z * PI_SCAN_COLUMNS;
+
+  auto fill = [&](int c) {      // the staging wave
+    const int buf = c & 1, t0 = c * CH, cn = n - t0 < CH ? n - t0 : CH;
+    const float* src = qkv + (long)(qs + t0) * qkv_stride;
+    StagedVectors<W, CH> qs_, ks_, gs_;
+    qs_.fetch(src + q_col, qkv_stride, cn, d, (vec & 1) != 0, lane);
+    ks_.fetch(src + k_col, qkv_stride, cn, d, (vec & 1) != 0, lane);
+    if constexpr (KIND != SCAN_HEAD_DELTA)
+      gs_.fetch(decay + (long)(qs + t0) * decay_stride + (long)h * d, decay_stride, cn, d, (vec & 2) != 0, lane);
+    constexpr int XI = (CH * PI_SCAN_COLUMNS + PI_WAVE - 1) / PI_WAVE;
+    float vs[XI];
+#pragma unroll
+    for (int j = 0; j < XI; ++j) {
+      const int i = lane + j * PI_WAVE, tt = i / PI_SCAN_COLUMNS, cc = i % PI_SCAN_COLUMNS;
+      vs[j] = (tt < cn && z * PI_SCAN_COLUMNS + cc < dv) ? src[tt * qkv_stride + v_col + cc] : 0.f;
+    }
+    float bt = 0.f, dc = 0.f;
+    if constexpr (KIND != SCAN_DECAYED_OUTER) bt = lane < cn ? beta[(long)(qs + t0 + lane) * beta_stride + h] : 0.f;
+    if constexpr (KIND == SCAN_HEAD_DELTA) dc = lane < cn ? decay[(long)(qs + t0 + lane) * decay_stride + h] : 0.f;
+    qs_.store(sq[buf], lane);
+    ks_.store(sk[buf], lane);
+    if constexpr (KIND != SCAN_HEAD_DELTA) gs_.store(sg[buf], lane);
+#pragma unroll
+    for (int j = 0; j < XI; ++j) {
+      const int i = lane + j * PI_WAVE;
+      if (i < CH * PI_SCAN_COLUMNS) (&sv[buf][0][0])[i] = vs[j];
+    }
+    if (lane < CH) {
+      sbeta[buf][lane] = bt;
+      sdecay[buf][lane] = dc;
+    }
+  };
+
+  float s[NR];
+  const int cw = wave * 4 + lane / 16;                 // this lane's column within the block
+  const int col = z * PI_SCAN_COLUMNS + cw;
+  const bool live = col < dv;
+  float* Sg = state + (long)slots[r] * state_stride + (((long)h * gridDim.z + z) * PI_SCAN_WAVES + (wave & 3)) * NR * PI_WAVE + lane;
+  if (wave < PI_SCAN_WAVES) {
+#pragma unroll
+    for (int i = 0; i < NR; ++i) s[i] = Sg[i * PI_WAVE];
+  } else {
+    fill(0);
+  }
+  __syncthreads();
+  for (int c = 0; c < chunks; ++c) {
+    if (wave == PI_SCAN_WAVES) {
+      if (c + 1 < chunks) fill(c + 1);
+    } else {
+      const int buf = c & 1, cn = n - c * CH < CH ? n - c * CH : CH;
+#pragma unroll 2
+      for (int tt = 0; tt < cn; ++tt) {
+        const float* qv = &sq[buf][tt * W + part * NR];
+        const float* kv = &sk[buf][tt * W + part * NR];
+        float u;
+        if constexpr (KIND == SCAN_DECAYED_OUTER) {
+          const float* gv = &sg[buf][tt * W + part * NR];
+#pragma unroll
+          for (int i = 0; i < NR; ++i) s[i] *= gv[i];
+          u = sv[buf][tt][cw];
+        } else {
+          float d0 = 0.f, d1 = 0.f;
+          if constexpr (KIND == SCAN_HEAD_DELTA) {
+            const float g1 = sdecay[buf][tt];
+#pragma unroll
+            for (int i = 0; i < NR; ++i) {
+              s[i] *= g1;
+              if (i & 1) d1 = fmaf(s[i], kv[i], d1);
+              else d0 = fmaf(s[i], kv[i], d0);
+            }
+          } else {
+            const float* gv = &sg[buf][tt * W + part * NR];
+#pragma unroll
+            for (int i = 0; i < NR; ++i) {
+              s[i] *= gv[i];
+              if (i & 1) d1 = fmaf(s[i], kv[i], d1);
+              else d0 = fmaf(s[i], kv[i], d0);
+            }
+          }
+          u = sbeta[buf][tt] * (sv[buf][tt][cw] - row16_sum(d0 + d1));
+        }
+        float a0 = 0.f, a1 = 0.f;
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {
+          s[i] = fmaf(kv[i], u, s[i]);
+          if (i & 1) a1 = fmaf(s[i], qv[i], a1);
+          else a0 = fmaf(s[i], qv[i], a0);
+        }
+        const float acc = row16_sum(a0 + a1);
+        if (live && part == 0) o[(long)(qs + c * CH + tt) * o_stride + (long)h * dv + col] = acc;
+      }
+    }
+    __syncthreads();
+  }
+  if (wave < PI_SCAN_WAVES) {
+#pragma unroll
+    for (int i = 0; i < NR; ++i) Sg[i * PI_WAVE] = s[i];
+  }
+}
+
 // What a lane needs of one token: its rows of q^, k^ and the decays, its column's v, and beta.
 template <int NR, int LANES>
 struct DeltaToken {
@@ -478,22 +597,22 @@ struct DeltaToken {
   }
 };
 
-// Then the walk: q^, k^ and v from qkv, decays from a, beta from b.  A column of S never meets another
-// column, so a wave walks its columns alone.  Bound by the chain from one token's state to the next and by what a wave that
-// has its unit's fourth to itself can issue.  16 heads of 128 x 128, 2,048 tokens of one request: 507 us with chunks fetched
-// and stored to LDS in one go; 471 with a chunk's fetch in flight while the chunk before is walked; 446 with a token read
-// from LDS while the one before is walked; 425 with 32 lanes to a column in blocks of eight columns (two waves of four
-// columns in such blocks, and fours that fall on all banks, gave nothing by themselves).
-template <int SNR, bool SHORT, int KIND, int WALKERS, int LANES>
-__global__ __launch_bounds__((WALKERS + 1) * PI_WAVE) void delta_scan_kernel(
+// The same walk for blocks that have a unit to themselves, reading ahead: bound by the chain from one token's state to the next
+// and by what a wave that has its unit's fourth to itself can issue.  16 heads of 128 x 128, 2,048 tokens of one request: 507 us with
+// chunks fetched and stored to LDS in one go, as above; 471 with a chunk's fetch in flight while the chunk before is walked; 446 with
+// a token read from LDS while the one before is walked; 425 with 32 lanes to a column in blocks of eight columns (two waves of four
+// columns in such blocks, and fours that fall on all banks, gave nothing by themselves).  What is read ahead lies in registers that
+// a unit's other blocks would need, so the form above stays for everything else (pi_delta_scan).
+template <int SNR, int KIND, int LANES>
+__global__ __launch_bounds__((PI_SCAN_WAVES + 1) * PI_WAVE) void delta_scan_ahead_kernel(
     float* __restrict__ o, long o_stride, const float* __restrict__ qkv, long qkv_stride, const float* __restrict__ decay,
     long decay_stride, const float* __restrict__ beta, long beta_stride, const int* __restrict__ q_start,
     const int* __restrict__ slots, float* __restrict__ state, long state_stride, int H, int G, int d, int dv, int vec) {
-  constexpr int W = ScanShape<SNR, SHORT>::W, CH = ScanShape<SNR, SHORT>::CH, NR = SNR * 16 / LANES;     // rows of a lane: SNR in a state row's order
+  constexpr int W = ScanShape<SNR, false>::W, CH = ScanShape<SNR, false>::CH, NR = SNR * 16 / LANES;     // rows of a lane: SNR in a state row's order
   __shared__ __attribute__((aligned(16))) float sq[2][CH * W];
   __shared__ __attribute__((aligned(16))) float sk[2][CH * W];
   __shared__ __attribute__((aligned(16))) float sg[2][KIND == SCAN_HEAD_DELTA ? 4 : CH * W];
-  constexpr int COLUMNS = WALKERS * (PI_WAVE / LANES);
+  constexpr int COLUMNS = PI_SCAN_WAVES * (PI_WAVE / LANES);
   __shared__ float sv[2][CH][COLUMNS], sbeta[2][CH], sdecay[2][CH];
   const int r = blockIdx.x, h = blockIdx.y, col0 = blockIdx.z * COLUMNS;
   const int wave = threadIdx.x / PI_WAVE, lane = threadIdx.x % PI_WAVE, part = lane % LANES;
@@ -547,7 +666,7 @@ __global__ __launch_bounds__((WALKERS + 1) * PI_WAVE) void delta_scan_kernel(
   const int by16 = (dv + PI_SCAN_COLUMNS - 1) / PI_SCAN_COLUMNS;
   const long row = ((long)(h * by16 + col / 16) * PI_SCAN_WAVES + col % 16 / 4) * SNR + part % (LANES / 16) * NR;
   float* Sg = state + (long)slots[r] * state_stride + row * PI_WAVE + col % 4 * 16 + part / (LANES / 16);
-  if (wave < WALKERS) {
+  if (wave < PI_SCAN_WAVES) {
 #pragma unroll
     for (int i = 0; i < NR; ++i) s[i] = Sg[i * PI_WAVE];
   } else {
@@ -557,7 +676,7 @@ __global__ __launch_bounds__((WALKERS + 1) * PI_WAVE) void delta_scan_kernel(
   }
   __syncthreads();
   for (int c = 0; c < chunks; ++c) {
-    if (wave == WALKERS) {
+    if (wave == PI_SCAN_WAVES) {
       if (c + 1 < chunks) put(c + 1);
       if (c + 2 < chunks) fetch(c + 2);
     } else {
@@ -608,7 +727,7 @@ __global__ __launch_bounds__((WALKERS + 1) * PI_WAVE) void delta_scan_kernel(
     }
     __syncthreads();
   }
-  if (wave < WALKERS) {
+  if (wave < PI_SCAN_WAVES) {
 #pragma unroll
     for (int i = 0; i < NR; ++i) Sg[i * PI_WAVE] = s[i];
   }
@@ -635,23 +754,30 @@ extern "C" int pi_delta_scan(float* o, long o_stride, float* qkv, long qkv_strid
   // bit 0: q and k may be fetched 16 bytes at a time; bit 1: the decays too
   const int vec = (d % 4 == 0 && qkv_stride % 4 == 0 && (uintptr_t)qkv % 16 == 0 ? 1 : 0) |
                   (d % 4 == 0 && a_stride % 4 == 0 && (uintptr_t)a % 16 == 0 ? 2 : 0);
-  // Blocks of sixteen columns that leave every other unit idle make way for blocks of eight, a column's rows on twice the lanes
+  // Blocks of sixteen columns that leave every other unit idle make way for blocks of eight, a column's rows on twice the lanes,
+  // which read ahead (16 heads of 128 x 128, 2,048 tokens: 517 us by the plain form, 439 so).  With sixteen lanes only keys of more
+  // than 128 channels with a decay per channel read ahead (4 heads of 256 x 256, four requests of 700 tokens: 324 and 280 us); for
+  // others the registers cost more than they bring (16 heads of 64 x 128, the same requests: 184 us, 294 reading ahead; fifteen
+  // requests of one token beside 200, 8 heads of 64 x 64: 50 and 88; eight of one, 16 heads of 128 x 128: 9.2 and 12.6).
   const int by16 = (dv + PI_SCAN_COLUMNS - 1) / PI_SCAN_COLUMNS;
   const bool wide = longest > 2 && (long)R * H * by16 * 2 <= compute_units();
-#define PI_LAUNCH_DELTA2(NR_, SHORT_, KIND_, LANES_)                                                                                           \
-  hipLaunchKernelGGL((delta_scan_kernel<NR_, SHORT_, KIND_, PI_SCAN_WAVES, LANES_>), dim3(R, H, by16 * (LANES_) / 16), dim3((PI_SCAN_WAVES + 1) * PI_WAVE), 0, \
-                     stream, o, o_stride, qkv, qkv_stride, a, a_stride, b, b_stride, q_start, slots, state, state_stride, H, G, d, dv, vec)
-#define PI_LAUNCH_DELTA1(NR_, SHORT_, LANES_)                                            \
-  do {                                                                                   \
-    if (kind == SCAN_HEAD_DELTA) PI_LAUNCH_DELTA2(NR_, SHORT_, SCAN_HEAD_DELTA, LANES_); \
-    else if (kind == SCAN_DECAYED_OUTER) PI_LAUNCH_DELTA2(NR_, SHORT_, SCAN_DECAYED_OUTER, LANES_); \
-    else PI_LAUNCH_DELTA2(NR_, SHORT_, SCAN_CHANNEL_DELTA, LANES_);                      \
+#define PI_DELTA_ARGS o, o_stride, qkv, qkv_stride, a, a_stride, b, b_stride, q_start, slots, state, state_stride, H, G, d, dv, vec
+#define PI_DELTA_GO(COLUMN_BLOCKS, ...) \
+  hipLaunchKernelGGL((__VA_ARGS__), dim3(R, H, COLUMN_BLOCKS), dim3((PI_SCAN_WAVES + 1) * PI_WAVE), 0, stream, PI_DELTA_ARGS)
+#define PI_LAUNCH_DELTA2(NR_, KIND_)                                                                                  \
+  do {                                                                                                                \
+    constexpr bool LONG_KEYS = (NR_) >= 8;                                                                            \
+    constexpr int AHEAD_NR = LONG_KEYS ? (NR_) : 8;                                                                   \
+    if (longest <= 2) PI_DELTA_GO(by16, delta_scan_kernel<NR_, true, KIND_>);                                         \
+    else if (LONG_KEYS && wide) PI_DELTA_GO(by16 * 2, delta_scan_ahead_kernel<AHEAD_NR, KIND_, 32>);                  \
+    else if ((NR_) >= 16 && (KIND_) != SCAN_HEAD_DELTA) PI_DELTA_GO(by16, delta_scan_ahead_kernel<16, KIND_, 16>);    \
+    else PI_DELTA_GO(by16, delta_scan_kernel<NR_, false, KIND_>);                                                     \
   } while (0)
-#define PI_LAUNCH_DELTA(NR_)                                        \
-  do {                                                              \
-    if (longest <= 2) PI_LAUNCH_DELTA1(NR_, true, 16);              \
-    else if ((NR_) >= 8 && wide) PI_LAUNCH_DELTA1(NR_, false, ((NR_) >= 8 ? 32 : 16)); \
-    else PI_LAUNCH_DELTA1(NR_, false, 16);                          \
+#define PI_LAUNCH_DELTA(NR_)                                                        \
+  do {                                                                              \
+    if (kind == SCAN_HEAD_DELTA) PI_LAUNCH_DELTA2(NR_, SCAN_HEAD_DELTA);            \
+    else if (kind == SCAN_DECAYED_OUTER) PI_LAUNCH_DELTA2(NR_, SCAN_DECAYED_OUTER); \
+    else PI_LAUNCH_DELTA2(NR_, SCAN_CHANNEL_DELTA);                                 \
   } while (0)
   switch (nr) {
     case 1: PI_LAUNCH_DELTA(1); break;
@@ -661,7 +787,8 @@ extern "C" int pi_delta_scan(float* o, long o_stride, float* qkv, long qkv_strid
     default: PI_LAUNCH_DELTA(16); break;
   }
 #undef PI_LAUNCH_DELTA
-#undef PI_LAUNCH_DELTA1
 #undef PI_LAUNCH_DELTA2
+#undef PI_DELTA_GO
+#undef PI_DELTA_ARGS
   return pi_check_launch("delta_scan");
 }

@@ -166,6 +166,12 @@ def dev32(t):
     return t.float().to(DEV).contiguous()
 
 
+# (heads, kv heads, key width, value width) of walks over states with long keys: a request walks with 16 or with 32 lanes to a column
+# by the blocks its step has (on 256 units the first three with 16 beside another request and with 32 alone, the last but one always with 16, the
+# others always with 32), keys of more than 128 channels, and widths that end inside a block, a state row or a 16-byte access
+LONG_KEYS = [(8, 4, 128, 136), (4, 4, 200, 288), (5, 5, 256, 240), (2, 1, 256, 40), (2, 1, 70, 24), (1, 1, 130, 40), (16, 16, 70, 264), (2, 2, 253, 20)]
+
+
 def state_ctx(q_lens, slots):
     """The fields of a StepContext that the kernels of mixers with a state read."""
     q_start = np.zeros(len(q_lens) + 1, np.int32)

@@ -13,7 +13,7 @@ import torch
 
 import plain_muretar as P
 import tiny_muretar as TM
-from gpu_tools import (DEV, RouteRecorder, attention_ctx, close, cut_steps, dev32, in_steps, live_token_need, make_part, paged, randn, run_paged_part,
+from gpu_tools import (DEV, LONG_KEYS, RouteRecorder, attention_ctx, close, cut_steps, dev32, in_steps, live_token_need, make_part, paged, randn, run_paged_part,
                        run_trace, state_ctx)
 from tiny_models import random_tokens
 
@@ -199,7 +199,7 @@ def walk(kind, data, T, slot, cuts, sizes, consts):
 CUTS = ({"a": [83], "b": [10]}, {"a": [1], "b": [1]}, {"a": [2, 17, 1, 40], "b": [3, 2]}, {"a": [9], "b": [10]})
 
 
-@pytest.mark.parametrize("sizes", [(4, 2, 16, 24), (4, 4, 32, 32), (3, 1, 20, 28), (1, 1, 48, 80), (5, 5, 8, 8), (2, 1, 128, 64), (2, 2, 3, 200)])
+@pytest.mark.parametrize("sizes", [(4, 2, 16, 24), (4, 4, 32, 32), (3, 1, 20, 28), (1, 1, 48, 80), (5, 5, 8, 8), (2, 1, 128, 64), (2, 2, 3, 200)] + LONG_KEYS)
 def test_delta_rule_with_a_decay_per_head_whole_in_portions_and_token_by_token(sizes):
     H, G, d, dv = sizes
     T = {"a": 83, "b": 10}
@@ -221,7 +221,7 @@ def test_delta_rule_with_a_decay_per_head_whole_in_portions_and_token_by_token(s
         assert bool((state[0] == 0).all()) and bool((state[2] == 0).all())
 
 
-@pytest.mark.parametrize("sizes", [(2, 24, 16, 8.0), (4, 32, 64, 16.0), (3, 20, 28, 3.5), (1, 40, 40, 1.0), (2, 128, 64, 2.0), (2, 3, 200, 5.0)])
+@pytest.mark.parametrize("sizes", [(2, 24, 16, 8.0), (4, 32, 64, 16.0), (3, 20, 28, 3.5), (1, 40, 40, 1.0), (2, 128, 64, 2.0), (2, 3, 200, 5.0)] + [(H, d, dv, 4.0) for H, _, d, dv in LONG_KEYS])
 def test_gated_linear_attention_walk_whole_in_portions_and_token_by_token(sizes):
     H, d, dv, tau = sizes
     T = {"a": 83, "b": 10}

@@ -13,7 +13,7 @@ import torch
 
 import plain_rorevik as P
 import tiny_rorevik as TR
-from gpu_tools import DEV, attention_ctx, cut_steps, library_calls, live_token_need, run_trace
+from gpu_tools import DEV, LONG_KEYS, attention_ctx, cut_steps, library_calls, live_token_need, run_trace
 from tiny_models import random_tokens
 
 pytestmark = pytest.mark.gpu
@@ -239,7 +239,7 @@ def delta_plain(q, k, v, a, b, dt_bias, A_log, H, d):
     return P.delta_recurrence(P.unit(q) * d ** -0.5, P.unit(k), v, torch.sigmoid(b), decay)
 
 
-@pytest.mark.parametrize("sizes", [(4, 2, 16, 24), (4, 4, 32, 32), (3, 1, 20, 28), (1, 1, 48, 80), (5, 5, 8, 8), (2, 1, 128, 64), (2, 2, 3, 200)])
+@pytest.mark.parametrize("sizes", [(4, 2, 16, 24), (4, 4, 32, 32), (3, 1, 20, 28), (1, 1, 48, 80), (5, 5, 8, 8), (2, 1, 128, 64), (2, 2, 3, 200)] + LONG_KEYS)
 def test_delta_rule_whole_in_portions_and_token_by_token(sizes):
     from photon_infer_amd import ops
     H, G, d, dv = sizes
