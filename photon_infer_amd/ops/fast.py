@@ -34,7 +34,7 @@ SHARED_FROM_TOKENS = 32        # more tokens than this: the skinny kernel that s
 SHARED_ROWS_PER_BLOCK = 64     # ... with this many weight rows per block, and no more blocks than compute units (100 tokens, 3,072 x 8,192:
                                # 22.8 us in six pieces on 288 blocks, 16.9 in five on 240; 6,144 x 4,096 22.8 in three, 18.7 in two)
 RING_MAX_STRIDE = 1 << 21      # elements between rows up to which that kernel's byte offsets fit 31 bits
-FLOAT32_SWIGLU_K = 2048        # up to this k the gated unit is part of the float32 product also where the general kernel streams a few rows faster
+FLOAT32_ROWS = 32              # up to this many rows a float32 product goes to the weight-streaming kernel
 FLOAT32_MAX_STRIDE = 1 << 21   # floats between rows up to which the float32 kernels' offsets inside a tile fit 32 bits
 DEFAULT_UNITS = 256            # compute units assumed where no device can be asked (an MI355X)
 PIECES_WORTH = 0.95            # q, k, v of a prompt portion are left in k pieces too where that takes no more than this share of the time:
@@ -269,9 +269,28 @@ def gemm_float32_pieces(a, w, ws: Optional[KernelWorkspace]) -> Optional[Partial
     return _float32_product(None, a, w, False, M, N, K, lda, ldw, N, ws, True)
 
 
+@functools.lru_cache(maxsize=4096)
+def float32_gate_in_product(M: int, N: int, K: int, units: int) -> bool:
+    """Whether a gated float32 product (N = 2I rows of weights) applies its unit before anything is stored, which needs whole
+    sums, or leaves it to a kernel of its own behind a product whose k may be cut.  More than 32 rows: where the product would
+    not be cut anyway (64 rows, 1,024 features, k 4,096: 85 us whole, 21 in eight pieces with the unit).  Fewer rows stream the
+    weights in blocks of 32 rows: in the product where these nearly are as many as the units (16 rows, 3,072 features, k 2,048:
+    16 and 21 us), or where k is short (8 rows, 512 features, k 512: 7.0 and 7.2; 32 rows, 1,024 features, k 4,096: 31 and 23).
+    One or two rows, which the general kernel streams faster: up to k of 2,048 (8,192 features, one row: 26.9 and 28.8 us, at
+    3,072 39.5 and 39.6, at 4,096 69 and 51), with few features to 1,024 (2,048 features: 9.0 and 10.0; 256: 8.6 and 7.0)."""
+    if M > FLOAT32_ROWS:
+        return _lib.load("core").pi_gemm_float32_pieces(M, N, K, GEMM_PART_FLOATS, 0) == 1
+    blocks, general = N // 32, _general_streams_faster(M, N, K)
+    if 4 * blocks >= 3 * units:
+        return K <= 2048 or not general
+    if general:
+        return K <= 1024 and 8 * blocks >= 3 * units
+    return K <= 1024 if M <= 16 else K <= 512 and 8 * blocks >= units
+
+
 def gemm_swiglu_float32(out, a, w, M, N, K, lda, ldw) -> bool:
     """``w`` [N = 2I, K] with gate / up rows interleaved in blocks of 16; out [M, I], all float32."""
-    if not _float32_ok(a, w, K, lda, ldw) or N % 32 or (_general_streams_faster(M, N, K) and K > FLOAT32_SWIGLU_K):
+    if not _float32_ok(a, w, K, lda, ldw) or N % 32 or not float32_gate_in_product(M, N, K, compute_units()):
         return False
     _lib.call("core", "pi_gemm_float32_swiglu", out.data_ptr(), out.stride(0), a.data_ptr(), lda, w.data_ptr(), ldw, M, N, K, _stream())
     return True

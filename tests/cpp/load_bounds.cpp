@@ -297,7 +297,7 @@ static bool check(const Shape& s) {
   for (int pad = 0; pad <= 12 && s.K % 4 == 0; pad += 12) {    // float32: row strides K and K + 12
     const long ld = s.K + pad;
     if (s.M <= 32) {
-      if (!float32_rows(s, ld, ld, 2, 4, 1) || !float32_rows(s, ld, ld, 1, 8, 2) || !float32_rows(s, ld, ld, 1, 16, 2)) return false;
+      if (!float32_rows(s, ld, ld, 2, 4, 1) || !float32_rows(s, ld, ld, 2, 8, 2) || !float32_rows(s, ld, ld, 1, 8, 2) || !float32_rows(s, ld, ld, 1, 16, 2)) return false;
     } else {
       for (const Tiles& t : FLOAT32_TILES)
         if (!tiles(s, ld, ld, t, 2)) return false;

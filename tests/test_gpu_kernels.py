@@ -346,18 +346,27 @@ def test_every_tile_shape_at_its_edges(_ops, monkeypatch, shape, M, N, K):
 
 
 @pytest.mark.parametrize("M", [1, 3, 16, 17, 32, 33, 65, 200])
-@pytest.mark.parametrize("I,K", [(16, 4), (48, 260), (6160, 200), (528, 4096)])
-def test_float32_product_with_swiglu(_ops, M, I, K):
-    """Gate and up rows interleaved by 16, the unit in the product's epilogue: few rows and tiles, and k long enough for the
-    general kernel.  Sums of K products are off by sqrt(K) roundings of their size at most, the unit's slope is below 1.1."""
+@pytest.mark.parametrize("I,K", [(16, 4), (48, 260), (3088, 328), (6160, 200), (528, 4096)])
+def test_float32_product_with_swiglu(_ops, monkeypatch, M, I, K):
+    """Gate and up rows interleaved by 16, the unit in the product's epilogue wherever the product goes, and as the rule has
+    it, which leaves few features with a long k to two kernels.  Sums of K products are off by sqrt(K) roundings of their size
+    at most, the unit's slope is below 1.1."""
+    from photon_infer_amd.ops import fast
     _ops.use_fast_kernels(True)
     a = torch.randn(M, K, generator=gen(M))
     g, u = torch.randn(I, K, generator=gen(I)) / K ** 0.5, torch.randn(I, K, generator=gen(K)) / K ** 0.5
     w = torch.stack([g.view(I // 16, 16, K), u.view(I // 16, 16, K)], dim=1).reshape(2 * I, K).contiguous()
     want = P.swiglu(a.double() @ g.double().t(), a.double() @ u.double().t())
-    out = torch.empty(M, I, device=DEV)
-    _ops.gemm_swiglu(out, a.to(DEV), w.to(DEV), 16)
-    close(out, want, 2 ** -23 * (8 + K ** 0.5), f"{M} x {I} x {K}")
+    rule = fast.float32_gate_in_product(M, 2 * I, K, fast.compute_units())
+    assert rule or (I, K) in ((16, 4), (48, 260), (528, 4096))
+    for whole in (rule, True):
+        if whole is not rule:
+            monkeypatch.setattr(fast, "float32_gate_in_product", lambda *_: True)
+        out = torch.empty(M, I, device=DEV)
+        with library_calls() as names:
+            _ops.gemm_swiglu(out, a.to(DEV), w.to(DEV), 16)
+        assert (names == ["pi_gemm_float32_swiglu"]) == whole and (whole or names[-1] == "pi_swiglu")
+        close(out, want, 2 ** -23 * (8 + K ** 0.5), f"{M} x {I} x {K}")
 
 
 @pytest.mark.parametrize("M,N,K", [(3, 2048, 2048), (8, 96, 512), (32, 3072, 2048), (33, 256, 1024), (378, 2048, 8192), (1, 2048, 2048)])

@@ -146,6 +146,21 @@ def test_the_float32_path_takes_the_attention_kernel_that_was_the_faster_one(ste
     assert 0.6 < tiles_us / tiles < 1.6 and 0.5 < general_us / general < 1.6       # and the estimates are of that size
 
 
+# (rows, features, k), microseconds of the gated unit in the float32 product, and of product and unit, measured
+FLOAT32_GATED = [
+    (64, 1024, 4096, 85.4, 21.5), (200, 1024, 4096, 86.5, 48.6), (32, 1024, 4096, 30.6, 23.0), (24, 2048, 2048, 18.5, 15.4), (33, 512, 512, 15.9, 13.0),
+    (8, 8192, 4096, 65.0, 68.1), (8, 512, 512, 7.0, 7.2), (2, 1024, 2048, 12.7, 10.3), (1, 4096, 8192, 80.3, 57.9), (1, 8192, 2048, 26.9, 28.8), (1, 2048, 1024, 9.0, 10.0),
+    (16, 3072, 2048, 16.1, 20.7), (32, 3072, 1024, 12.7, 17.2), (24, 256, 1024, 11.8, 10.0), (500, 1536, 2048, 76.0, 80.1), (900, 4096, 512, 77.6, 83.8), (100, 8192, 3072, 113.9, 117.8),
+]
+
+
+@pytest.mark.parametrize("M,I,K,whole,two", FLOAT32_GATED)
+def test_the_float32_gated_unit_is_part_of_the_product_where_that_was_the_faster_way(M, I, K, whole, two):
+    from photon_infer_amd.ops import fast
+    took = whole if fast.float32_gate_in_product(M, 2 * I, K, 256) else two
+    assert took <= 1.03 * min(whole, two)
+
+
 # (rows, columns, k): a tile shape that was measured to be the fastest, or within 3 % of it, for a product in one piece
 @pytest.mark.parametrize("M,N,K,shape", [(543, 28672, 4096, 33), (2048, 16384, 2048, 42), (384, 3072, 2048, 0), (2048, 2048, 8192, 0),
                                          (200, 4096, 14336, 0), (300, 200, 1000, 0), (1100, 28672, 4096, 33)])
