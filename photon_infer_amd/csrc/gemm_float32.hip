@@ -16,6 +16,7 @@
 #define FSTEP 32                      // floats of k per step: 128 bytes of a row
 #define ROWS_MAX_M 32                 // up to this many rows of activations the weight-streaming kernel is taken
 #define ROWS_SPLIT_MIN_K 4096         // from this k on a product's pieces are worth a kernel that adds them
+#define ROWS_WHOLE_K 768              // up to this k a matrix of many rows is left whole for its reader too
 
 // What becomes of a product in one piece: stored, added to C, or, with gate and up rows interleaved in blocks of 16 in W,
 // silu(gate) * up of the same feature stored to C [M, N / 2] (a kernel of its own for it took 4.7 us at eight tokens by 8,192
@@ -370,14 +371,18 @@ static Float32Plan cut(int tm, int tn, int K, int splits) {
 // 727 us (1,236 on the vector unit), 378 rows 214 us (118 TFLOP/s); 2048 x 8192: 2,048 rows 525 us, 1,293 rows 412 us in two
 // pieces, 378 rows 119 us in five.
 // `read_by_next`: the pieces are left to the kernel that reads the result anyway (a norm, a rotation).  They then cost their
-// way through memory and no launch, and a matrix of few rows is streamed by two blocks per unit whatever its k: eight tokens,
-// 2,048 x 2,048 9.9 -> 7.8 us, 3,072 x 2,048 10.0 -> 8.9; and 4.6 us less for each product whose pieces a kernel added.
+// way through memory and no launch, and a matrix of few rows is streamed by two blocks per unit whatever its k: eight tokens and
+// the norm, 2,048 x 2,048 12.4 -> 10.3 us, 3,072 x 2,048 13.1 -> 12.0; and some 2 us less for each product whose pieces a kernel
+// added.  A short k in blocks of 16 rows that nearly are the units' number stays whole (24 tokens and the norm, 3,072 x 768 10.6 us
+// and 14.6 in three pieces; 4,096 x 512 10.1 and 10.9).  More pieces have to promise a hundredth: 129 x 2,048 x 8,192 and the norm
+// takes 65 us in five and 76 in eight, which the rule holds for equal.
 static Float32Plan plan(int M, int N, int K, long part_floats, bool read_by_next) {
   const int units = compute_units();
   if (M <= ROWS_MAX_M) {
     // blocks of 32 rows want to be two per unit; a matrix of fewer rows whose k is long is cut over blocks, any other
     // gets its waves in blocks of 16 rows (launch_rows)
-    int splits = read_by_next || K >= ROWS_SPLIT_MIN_K ? 2 * units / ceil_div(N, 32) : 1;
+    const bool whole = read_by_next ? K <= ROWS_WHOLE_K && 4 * ceil_div(N, 16) >= 3 * units : K < ROWS_SPLIT_MIN_K;
+    int splits = whole ? 1 : 2 * units / ceil_div(N, 32);
     while (splits > 1 && (K / splits < (read_by_next ? 256 : 512) || (long)splits * M * N > part_floats)) --splits;
     return cut(0, 0, K, splits < 1 ? 1 : splits);
   }
@@ -392,7 +397,7 @@ static Float32Plan plan(int M, int N, int K, long part_floats, bool read_by_next
       const long rounds = (tiles * p.splits + units - 1) / units;
       float us = rounds * (3.f + 2.f * s.tm * s.tn * p.k_per_split / s.rate);
       if (p.splits > 1) us += (read_by_next ? 1.f : 4.f) + (read_by_next ? 1.5f : 2.f) * p.splits * M * N * 4.f / 4.0e6f;
-      if (least == 0.f || us < least) { least = us; best = p; }
+      if (least == 0.f || us < (read_by_next && p.splits > best.splits ? 0.99f : 1.f) * least) { least = us; best = p; }
     }
   }
   return best;
@@ -435,8 +440,7 @@ static int launch_rows(float* C, long ldc, const float* A, long lda, const float
   hipLaunchKernelGGL((gemm_float32_rows_kernel<MB, RT, WAVES, DEPTH, EPI>), dim3(ceil_div(N, RT * 16), p.splits), dim3(WAVES * 64), 0, stream, C, ldc, \
                      A, lda, W, ldw, M, N, K, p.k_per_split, part)
   const int units = compute_units();
-  if (p.splits > 1 && p.k_per_split <= 512) ROWS_GO(2, 4, 2);          // a wave's few steps all at once
-  else if (p.splits > 1 || N >= 2 * units * 24) ROWS_GO(2, 4, 1);
+  if (p.splits > 1 || N >= 2 * units * 24) ROWS_GO(2, 4, 1);
   else if constexpr (EPI == EPI_SWIGLU) ROWS_GO(2, 8, 2);
   else if (MB == 1 && N <= units * 16) ROWS_GO(1, (MB == 1 ? 16 : 8), 2);     // sixteen waves have registers for 16 tokens only
   else ROWS_GO(1, 8, 2);

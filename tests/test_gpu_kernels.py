@@ -369,23 +369,27 @@ def test_float32_product_with_swiglu(_ops, monkeypatch, M, I, K):
         close(out, want, 2 ** -23 * (8 + K ** 0.5), f"{M} x {I} x {K}")
 
 
-@pytest.mark.parametrize("M,N,K", [(3, 2048, 2048), (8, 96, 512), (32, 3072, 2048), (33, 256, 1024), (378, 2048, 8192), (1, 2048, 2048)])
-def test_float32_pieces_are_added_by_the_next_reader(_ops, M, N, K):
-    """A product into the stream that stays in pieces, read by the norm, and one for the rotation: against 64 bits."""
+@pytest.mark.parametrize("M,N,K,cut", [(3, 2048, 2048, True), (8, 96, 512, True), (32, 3072, 2048, True), (33, 256, 1024, True), (378, 2048, 8192, True),
+                                       (1, 2048, 2048, False), (24, 3072, 768, False), (40, 16384, 256, False)])
+def test_float32_pieces_are_added_by_the_next_reader(_ops, M, N, K, cut):
+    """A product into the stream that stays in pieces, read by the norm, and one for the rotation: against 64 bits.  Some are whole."""
     _ops.use_fast_kernels(True)
     a, w = torch.randn(M, K, generator=gen(M)).to(DEV), (torch.randn(N, K, generator=gen(N)) / K ** 0.5).to(DEV)
     x = torch.randn(M, N, generator=gen(K)).to(DEV)
     want = x.double() + a.double() @ w.double().t()
     ws = _ops.KernelWorkspace(DEV)
-    _ops.gemm(x, a, w, accumulate=True, may_defer=True, ws=ws)
+    with library_calls() as names:
+        _ops.gemm(x, a, w, accumulate=True, may_defer=True, ws=ws)
+    assert names == (["pi_gemm_float32"] if M > 1 else ["pi_gemm_general"]) and (ws.pending is not None) == cut
     h = torch.empty_like(x)
     _ops.rmsnorm(h, x, torch.ones(N, device=DEV), 1e-5, ws=ws)
     assert ws.pending is None and not ws.counts                  # the 16-bit products' statistics: nothing of these
-    assert ws.float32_counts["added_by_norm"] == ws.float32_counts["deferred"] == ws.float32_counts["split_products"]
+    assert ws.float32_counts["added_by_norm"] == ws.float32_counts["deferred"] == ws.float32_counts["split_products"] == int(cut)
     close(x, want.cpu(), 2 ** -23 * (8 + K ** 0.5), "stream")
     close(h, (want / (want.pow(2).mean(-1, keepdim=True) + 1e-5).sqrt()).cpu(), 2 ** -22 * (8 + K ** 0.5), "norm")
     p = _ops.qkv_projection(a, w, F32, ws)
-    got = p if isinstance(p, torch.Tensor) else p.part[:p.splits * M * N].view(p.splits, M, N).double().sum(0)
+    assert isinstance(p, _ops.Partials) == cut
+    got = p.part[:p.splits * M * N].view(p.splits, M, N).double().sum(0) if cut else p
     close(got, (a.double() @ w.double().t()).cpu(), 2 ** -23 * (8 + K ** 0.5), "projection")
 
 

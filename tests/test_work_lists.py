@@ -146,6 +146,21 @@ def test_the_float32_path_takes_the_attention_kernel_that_was_the_faster_one(ste
     assert 0.6 < tiles_us / tiles < 1.6 and 0.5 < general_us / general < 1.6       # and the estimates are of that size
 
 
+# (rows, columns, k), {pieces of k: microseconds of a float32 product with the norm that adds them}, measured
+FLOAT32_PIECES = [
+    (8, 2048, 2048, {1: 12.4, 4: 10.2, 8: 10.3, 16: 12.8}), (24, 2048, 2048, {1: 14.8, 4: 12.4, 8: 12.3, 16: 15.8}), (24, 3072, 2048, {1: 15.5, 3: 17.6, 5: 15.7, 8: 15.6}),
+    (8, 3072, 768, {1: 9.8, 3: 10.9}), (24, 3072, 768, {1: 10.6, 2: 11.6, 3: 11.7}), (32, 4096, 512, {1: 10.3, 2: 11.1}), (24, 5120, 3072, {1: 37.0, 3: 24.8}),
+    (129, 2048, 8192, {5: 64.9, 8: 75.9}), (1000, 256, 512, {1: 16.7, 2: 12.5}),
+]
+
+
+@pytest.mark.parametrize("M,N,K,times", FLOAT32_PIECES)
+def test_a_float32_product_is_left_in_as_many_pieces_as_were_the_fastest(M, N, K, times):
+    from photon_infer_amd.ops import _lib, fast
+    made = _lib.load("core").pi_gemm_float32_pieces(M, N, K, fast.GEMM_PART_FLOATS, 1)
+    assert times[made] <= 1.05 * min(times.values())
+
+
 # (rows, features, k), microseconds of the gated unit in the float32 product, and of product and unit, measured
 FLOAT32_GATED = [
     (64, 1024, 4096, 85.4, 21.5), (200, 1024, 4096, 86.5, 48.6), (32, 1024, 4096, 30.6, 23.0), (24, 2048, 2048, 18.5, 15.4), (33, 512, 512, 15.9, 13.0),
