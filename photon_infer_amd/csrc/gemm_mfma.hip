@@ -565,15 +565,17 @@ static int launch_big(void* C, long ldc, const void* A, long lda, const void* W,
   return pi_check_launch("gemm_mfma_big");
 }
 
-// shape: 0 a 128 x 128 tile, in whichever kernel is the faster one; else 10 WI + WJ of the larger tiles' kernel (K a multiple of the slab)
+// shape: 0 a 128 x 128 tile, in whichever kernel is the faster one, 20 in the kernel of 256 threads; else 10 WI + WJ of the larger
+// tiles' kernel (K a multiple of the slab)
 template <int EPI>
 static int launch(void* C, long ldc, const void* A, long lda, const void* W, long ldw, int M, int N, int K, int splits, int shape,
                   hipStream_t stream, GluArgs glu = GluArgs{nullptr, 0.f, 0.f, 0}) {
   const addressing::KSplit cut = addressing::cut_k(K, splits, BK);
   const int kps = cut.k_per_block;
   splits = cut.splits;
-  PI_REQUIRE(shape == 0 || K % BK == 0, "gemm_mfma: the larger tiles take whole slabs of %d only, K is %d", BK, K);
+  PI_REQUIRE(shape == 0 || shape == 20 || K % BK == 0, "gemm_mfma: the larger tiles take whole slabs of %d only, K is %d", BK, K);
   switch (shape) {
+    case 20: break;
     case 0:
       if (!tile_plan::ring_128_takes(M, N, K, splits, compute_units())) break;        // else the same tile in a ring
     case 21: return launch_big<EPI, 2, 1, 3, 3>(C, ldc, A, lda, W, ldw, M, N, K, splits, kps, stream, glu);

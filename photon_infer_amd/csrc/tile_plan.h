@@ -8,7 +8,7 @@
 
 namespace tile_plan {
 
-// A block tile: its code (0: the 128 x 128 kernel; 10 WI + WJ of the larger tiles), rows and columns, blocks that a unit
+// A block tile: its code (0: 128 x 128, in the kernel that takes it the faster; 10 WI + WJ of the larger tiles), rows and columns, blocks that a unit
 // holds at a time, and the microseconds of a block that has the chip nearly to itself and of one on a full chip, for k in
 // units of 1,024.  Fitted to measurements on an MI355X of 32 to 512 tiles of every shape at k of 256 to 8,192, weights cold
 // and results float32 (450 products, off by 6 to 8 % in the mean).  543 x 28,672 x 4,096: 336 tiles of 256 x 256 take two rounds of 256

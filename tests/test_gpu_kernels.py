@@ -316,12 +316,15 @@ def test_gemm_with_swiglu_on_large_tiles(_ops, M, I, K):
     close(out, want, 2 ** -7, "fused swiglu on large tiles")
 
 
-@pytest.mark.parametrize("shape", [0, 42, 33, 32, 23, 22, 21])
-@pytest.mark.parametrize("M,N,K", [(129, 96, 64), (193, 512, 192), (257, 800, 320), (640, 1184, 448)])
+EDGES = [(129, 96, 64), (193, 512, 192), (257, 800, 320), (640, 1184, 448)]
+
+
+@pytest.mark.parametrize("shape,M,N,K", [(s, *e) for s in (0, 42, 33, 32, 23, 22, 21, 20) for e in EDGES] +
+                         [(s, *e) for s in (0, 20) for e in ((129, 96, 8), (257, 800, 328), (385, 480, 1000))])
 def test_every_tile_shape_at_its_edges(_ops, monkeypatch, shape, M, N, K):
     """Each block tile with one row more than it holds, columns that end inside a wave's corner, and one slab of k up to
-    several: stored in both types, added, in pieces, and through the gated epilogue (products of bfloat16 in 32-bit sums:
-    the bounds of the tests above)."""
+    several, for the kernel of 256 threads (20; 0 is whichever is faster) also a part of one: stored in both types, added, in
+    pieces, and through the gated epilogue (products of bfloat16 in 32-bit sums: the bounds of the tests above)."""
     from photon_infer_amd.ops import fast
     monkeypatch.setattr(fast, "_tile_shape", lambda *_: shape)
     a = (torch.randn(M, K, generator=gen(M)) * 0.5).to(BF16).to(DEV)
@@ -343,6 +346,19 @@ def test_every_tile_shape_at_its_edges(_ops, monkeypatch, shape, M, N, K):
     out = torch.empty(M, N // 2, dtype=BF16, device=DEV)
     _ops.gemm_swiglu(out, a, w, 16)
     close(out, P.swiglu(g.reshape(M, -1), u.reshape(M, -1)).cpu(), 2 ** -7, f"tiles {shape}, swiglu")
+
+
+@pytest.mark.parametrize("shape,rows,cols", [(20, 128, 128), (21, 128, 128), (22, 128, 256), (23, 128, 384), (32, 192, 256), (33, 192, 384), (42, 256, 256)])
+def test_tiles_in_rectangles_of_dies(_ops, monkeypatch, shape, rows, cols):
+    """Eight row tiles, four column tiles and a long k: every die takes a rectangle of them, the last row and column not whole."""
+    from photon_infer_amd.ops import fast
+    monkeypatch.setattr(fast, "_tile_shape", lambda *_: shape)
+    M, N, K = 8 * rows - 24, 4 * cols - 32, 2048
+    a = (torch.randn(M, K, generator=gen(M)) * 0.5).to(BF16).to(DEV)
+    w = torch.randn(N, K, generator=gen(N)).to(BF16).to(DEV)
+    out = torch.full((M, N), float("nan"), device=DEV)
+    _ops.gemm(out, a, w)
+    close(out, (a.double() @ w.double().t()).cpu(), 2e-6, f"tiles {shape}")
 
 
 @pytest.mark.parametrize("M", [1, 3, 16, 17, 32, 33, 65, 200])
