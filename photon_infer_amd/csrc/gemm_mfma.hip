@@ -664,8 +664,8 @@ extern "C" int pi_gemm_mfma_pieces(int K, int splits) {
 extern "C" int pi_gemm_mfma_shape(int M, int N, int K, int splits, int units) {
   return M > 0 && N > 0 && K > 0 && splits > 0 && units > 0 ? tile_plan::shape_for(M, N, K, splits, units).code : 0;
 }
-extern "C" int pi_gemm_mfma_splits(int M, int N, int K, int units, long part_floats, double worth) {
-  return M > 0 && N > 0 && K > 0 && units > 0 ? tile_plan::splits_for(M, N, K, units, part_floats, worth) : 1;
+extern "C" int pi_gemm_mfma_splits(int M, int N, int K, int units, long part_floats, double worth, int norm) {
+  return M > 0 && N > 0 && K > 0 && units > 0 ? tile_plan::splits_for(M, N, K, units, part_floats, worth, norm != 0) : 1;
 }
 
 // epilogue: 0 store bf16, 1 store f32, 2 add into f32, 3 SwiGLU (W rows interleaved by 16; C is [M, N / 2] bf16),

@@ -10,37 +10,38 @@ namespace tile_plan {
 
 // A block tile: its code (0: 128 x 128, in the kernel that takes it the faster; 10 WI + WJ of the larger tiles), rows and columns, blocks that a unit
 // holds at a time, and the microseconds of a block that has the chip nearly to itself and of one on a full chip, for k in
-// units of 1,024.  Fitted to measurements on an MI355X of 32 to 512 tiles of every shape at k of 256 to 8,192, weights cold
-// and results float32 (450 products, off by 6 to 8 % in the mean).  543 x 28,672 x 4,096: 336 tiles of 256 x 256 take two rounds of 256
-// units, 184 us; 225 of 192 x 384 one, 121 us.
+// units of 1,024.  Fitted on an MI355X to 402 products of 130 to 3,000 rows with twenty matrices of 832 x 2,048 to 28,672 x 4,096
+// in every shape, weights cold, and to 301 of them in one to eight pieces with the norm that adds these: the shape it takes
+// is 0.1 % slower than the fastest in the mean (10 % at worst, 1,293 x 3,072 x 3,072).  543 x 28,672 x 4,096: 336 tiles of
+// 256 x 256 take two rounds of 256 units, 184 us; 225 of 192 x 384 one, 121 us.
 struct Shape {
   int code, rows, cols, slots;
   double alone[3], full[2];
 };
 constexpr Shape SHAPES[] = {
-    {0, 128, 128, 2, {6.533, 4.741, 0.748}, {8.62, 14.413}},
-    {42, 256, 256, 1, {7.699, 13.742, 0.347}, {12.781, 23.51}},
-    {33, 192, 384, 1, {8.2, 17.7, 0.68}, {14.8, 27.9}},
-    {32, 192, 256, 1, {7.117, 10.692, 0.274}, {10.926, 19.844}},
-    {23, 128, 384, 1, {7.3, 12.4, 1.25}, {10, 24.3}},
-    {22, 128, 256, 1, {6.449, 5.174, 2.036}, {8.406, 14.202}},
+    {0, 128, 128, 2, {1.0, 5.84, 0.66}, {4.95, 14.69}},
+    {42, 256, 256, 1, {5.29, 15.8, 0.05}, {8.75, 20.22}},
+    {33, 192, 384, 1, {6.33, 19.74, 0.41}, {9.56, 26.3}},
+    {32, 192, 256, 1, {4.98, 13.26, 0.08}, {7.45, 17.28}},
+    {23, 128, 384, 1, {5.81, 13.05, 1.03}, {5.25, 22.8}},
+    {22, 128, 256, 1, {3.83, 9.42, 0.17}, {5.08, 13.23}},
 };
 // 128 x 128 in the larger tiles' kernel, one block of eight waves to a unit, for whole slabs of k: taken in the place of the
 // 128 x 128 kernel where it is the faster one of the two (256 tiles of k = 8,192 82 us instead of 104; 512 of k = 256 15.5
 // and of k = 2,048 50 us instead of 41, two of whose blocks a unit holds).
-constexpr Shape RING_128 = {21, 128, 128, 1, {5.977, 4.279, 0.323}, {6.392, 9.063}};
+constexpr Shape RING_128 = {21, 128, 128, 1, {3.47, 6.48, 0.05}, {4.15, 8.63}};
 constexpr int SLAB = 64;               // k per slab: the larger tiles take whole slabs only
 constexpr int MAX_SPLITS = 8;
 constexpr int MIN_K = 256;             // a piece keeps at least this much of k
-// What the fit, which is good to some per cent, must promise at least before another shape or one more piece is taken.
-constexpr double SHAPE_GAIN = 0.9735, PIECES_GAIN = 0.9931;
+// What the fit must promise at least before another shape or one more piece is taken.
+constexpr double SHAPE_GAIN = 0.97, PIECES_GAIN = 0.945;
 // Bytes per microsecond of pieces, or of the updated stream, on their way into the norm behind the product, and what every
-// piece takes there besides (writing them is hidden in the times above).  Of 21 sizes of product and norm measured together,
-// 130 to 2,627 rows in one to eight pieces with cold weights, the choice is 1.4 % above the best in the mean (the numbers above are
-// moved inside the fit's error so that it is):
-// 300 x 2,048 x 8,192 takes 68 us in one piece, 28.2 in five and 29.5 in eight, 256 x 4,096 x 4,096 48, 25.7 in three and 28.5.
-// Rows of more than 4,096 columns go through the norm at half that rate (1,267 x 5,376 x 4,544: 104 us in one piece, 175 in two).
-constexpr double PIECES_READ = 6.869e6, WIDE_READ = PIECES_READ / 2, PIECE_US = 0.426;
+// piece takes there besides (writing them is hidden in the times above).  Over the 301 products measured with the norm the
+// choice is 0.8 % above the best in the mean: 300 x 2,048 x 8,192 takes 68 us in one piece, 28.2 in five and 29.5 in eight,
+// 256 x 4,096 x 4,096 48, 25.7 in three and 28.5.  Rows of more than 4,096 columns go through the norm at a third of that
+// rate (1,267 x 5,376 x 4,544: 104 us in one piece, 175 in two), through the rotation of q, k and v at the same (500 x 6,144 x
+// 4,096 with the rotation 48.8 us in one float32 piece, 43.8 in two; 500 x 5,120 x 3,072 41.5, 34.1 in three).
+constexpr double PIECES_READ = 5.8e6, WIDE_READ = PIECES_READ / 3, PIECE_US = 0.09;
 constexpr int WIDE = 4096;
 
 inline double shape_us(const Shape& s, int M, int N, int K, int splits, int units) {
@@ -79,8 +80,9 @@ inline Choice shape_for(int M, int N, int K, int splits, int units) {
 
 // In how many pieces a product is left whose reader adds them: as many as take the least time together with their way
 // through memory, if they take at most `worth` of the time in one piece, and no more than `part_floats` floats hold.
-inline int splits_for(int M, int N, int K, int units, long part_floats, double worth) {
-  const double read = N > WIDE ? WIDE_READ : PIECES_READ;
+// `norm`: the reader is a norm, whose rows may be wide.
+inline int splits_for(int M, int N, int K, int units, long part_floats, double worth, bool norm) {
+  const double read = norm && N > WIDE ? WIDE_READ : PIECES_READ;
   const double whole = shape_for(M, N, K, 1, units).us + 4.0 * M * N / read;      // the kernel adds into the stream
   int best = 1;
   double least = whole;

@@ -67,7 +67,7 @@ _SIGNATURES = {
         "pi_gemm_mfma": [P, I, L, P, L, P, L, I, I, I, I, I, P],
         "pi_gemm_mfma_pieces": [I, I],
         "pi_gemm_mfma_shape": [I, I, I, I, I],
-        "pi_gemm_mfma_splits": [I, I, I, I, L, D],
+        "pi_gemm_mfma_splits": [I, I, I, I, L, D, I],
         "pi_gemm_mfma_clamped_glu": [P, L, P, L, P, L, I, I, I, P, F, F, I, P],
         "pi_gemm_mfma_grouped": [P, I, L, P, L, P, L, L, P, P, P, I, I, I, L, L, F, F, P, L, P],
         "pi_gemm_skinny": [P, I, L, P, L, P, L, I, I, I, I, P, L, P, I, P],

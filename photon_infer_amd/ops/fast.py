@@ -101,8 +101,8 @@ def _tile_shape_of(M: int, N: int, K: int, splits: int, units: int) -> int:
 
 
 @functools.lru_cache(maxsize=4096)
-def _tile_splits_of(M: int, N: int, K: int, units: int, worth: float) -> int:
-    return _lib.load("bf16").pi_gemm_mfma_splits(M, N, K, units, GEMM_PART_FLOATS, worth)
+def _tile_splits_of(M: int, N: int, K: int, units: int, worth: float, norm: bool = True) -> int:
+    return _lib.load("bf16").pi_gemm_mfma_splits(M, N, K, units, GEMM_PART_FLOATS, worth, norm)
 
 
 def _tile_shape(M: int, N: int, K: int, splits: int) -> int:
@@ -111,8 +111,8 @@ def _tile_shape(M: int, N: int, K: int, splits: int) -> int:
 
 
 def _tile_splits(M: int, N: int, K: int) -> int:
-    """k-split of the tile kernels for a product whose reader adds the pieces: as many as take the least time together
-    with the pieces' way through memory."""
+    """k-split of the tile kernels for a product whose reader, a norm, adds the pieces: as many as take the least time
+    together with the pieces' way through memory."""
     return _tile_splits_of(M, N, K, compute_units(), 1.0)
 
 
@@ -352,11 +352,12 @@ def gemm_from_ranges(out, kr: KeyRanges, w, accumulate, N, ldw, ldc, may_defer, 
 
 def keeps_float32(M: int, N: int, K: int, units: int) -> bool:
     """Whether q, k, v that no cut of k leaves in float32 pieces still go to the rotation in float32, as one piece: while
-    their tiles of 128 x 128 do not outnumber the units.  Results of that size are rounded once, behind the rotation,
-    whatever the plan of the day says about pieces; larger ones, which a cut never paid for, are stored in bfloat16 (one
-    float32 piece instead, product and rotation: 543 x 6,144 x 4,096 43.0 -> 46.0 us, 1,280 x 3,072 x 2,048 27.6 -> 31.5;
-    2,048 x 3,072 x 2,048 would be 37.9 -> 42.3).  Not for 32 tokens and fewer, nor for a k too short to be cut in two."""
-    return M > SHARED_FROM_TOKENS and K >= 512 and -(-M // 128) * -(-N // 128) <= units
+    their tiles of 128 x 128 do not outnumber the units, and for a k above 2,048 more of them in proportion (the longer the
+    product takes, the less its float32 result adds).  Results of that size are rounded once, behind the rotation, whatever
+    the tile plan says about pieces; larger ones, which no plan cut, are stored in bfloat16 (one float32 piece instead, product
+    and rotation: 543 x 6,144 x 4,096 43.0 -> 46.0 us, 1,280 x 3,072 x 2,048 27.6 -> 31.5; 2,048 x 3,072 x 2,048 would be
+    37.9 -> 42.3).  Not for 32 tokens and fewer, nor for a k too short to be cut in two."""
+    return M > SHARED_FROM_TOKENS and K >= 512 and -(-M // 128) * -(-N // 128) * 2048 <= units * max(K, 2048)
 
 
 def gemm_pieces(a, w, ws: Optional[KernelWorkspace], whole: bool = False) -> Optional[Partials]:
@@ -373,8 +374,8 @@ def gemm_pieces(a, w, ws: Optional[KernelWorkspace], whole: bool = False) -> Opt
     if M > SKINNY_MAX_ROWS:
         # a prompt portion of a few hundred tokens has too few tiles for the chip: split k there
         # too, the consumer adds the pieces
-        splits = _tile_splits(M, N, K)
-        if splits > 1 and _tile_splits_of(M, N, K, compute_units(), PIECES_WORTH) > 1:
+        splits = _tile_splits_of(M, N, K, compute_units(), PIECES_WORTH, norm=False)
+        if splits > 1:
             p = _tiles_in_pieces(a, w, M, N, K, lda, ldw, splits, ws)
     else:
         splits = _skinny_splits(M, N, K)

@@ -189,21 +189,47 @@ def test_the_float32_gated_unit_is_part_of_the_product_where_that_was_the_faster
     assert took <= 1.03 * min(whole, two)
 
 
-# (rows, columns, k): a tile shape that was measured to be the fastest, or within 3 % of it, for a product in one piece
-@pytest.mark.parametrize("M,N,K,shape", [(543, 28672, 4096, 33), (2048, 16384, 2048, 42), (384, 3072, 2048, 0), (2048, 2048, 8192, 0),
-                                         (200, 4096, 14336, 0), (300, 200, 1000, 0), (1100, 28672, 4096, 33)])
-def test_tile_shapes_follow_the_rounds_they_take(M, N, K, shape):
+# (rows, columns, k), {tile shape: microseconds of the product in one piece}, bfloat16 results, weights cold, measured; 0 is the faster kernel of 128 x 128
+SHAPES_MEASURED = [
+    (543, 28672, 4096, {0: 175.5, 42: 174.4, 33: 121.9, 32: 149.8, 23: 189.0, 22: 163.4}),
+    (2048, 16384, 2048, {0: 147.4, 42: 111.8, 33: 124.7, 32: 126.0, 23: 155.1, 22: 134.6}),
+    (384, 3072, 2048, {0: 17.8, 42: 38.4, 33: 44.4, 32: 32.0, 23: 34.3, 22: 25.0}),
+    (2048, 2048, 8192, {0: 71.2, 42: 141.9, 33: 180.6, 32: 120.5, 23: 172.7, 22: 94.8}),
+    (200, 4096, 14336, {0: 116.6, 42: 265.6, 33: 324.5, 32: 204.2, 23: 314.2, 22: 178.7}),
+    (1150, 28672, 4096, {0: 272.6, 42: 277.0, 33: 232.4, 32: 239.3, 23: 294.0, 22: 244.7}),
+    (1000, 5120, 3072, {0: 56.9, 42: 63.1, 33: 76.6, 32: 51.0, 23: 74.0, 22: 45.3}),
+    (850, 6144, 4096, {0: 60.3, 42: 74.2, 33: 96.9, 32: 65.6, 23: 92.7, 22: 53.9}),
+    (2048, 4096, 4096, {0: 68.0, 42: 78.6, 33: 97.7, 32: 69.0, 23: 93.7, 22: 62.1}),
+    (200, 28672, 4096, {0: 78.7, 42: 89.1, 33: 109.5, 32: 78.0, 23: 105.2, 22: 68.3}),
+    (2627, 3072, 2048, {0: 34.4, 42: 41.3, 33: 47.1, 32: 36.6, 23: 38.4, 22: 33.6}),
+    (300, 16384, 3072, {0: 51.6, 42: 61.3, 33: 81.4, 32: 55.2, 23: 75.9, 22: 46.2}),
+    (3000, 16384, 3072, {0: 311.1, 42: 240.0, 33: 268.8, 32: 254.4, 23: 317.5, 22: 281.9}),
+]
+
+
+@pytest.mark.parametrize("M,N,K,times", SHAPES_MEASURED)
+def test_tile_shapes_follow_the_rounds_they_take(M, N, K, times):
     from photon_infer_amd.ops import fast
-    assert fast._tile_shape_of(M, N, K, 1, 256) == shape
+    assert times[fast._tile_shape_of(M, N, K, 1, 256)] <= 1.03 * min(times.values())
 
 
-# (rows, columns, k), microseconds of the product in one, two, ... pieces with the norm that adds them, measured
+def test_a_k_that_is_no_whole_slabs_takes_the_only_kernel_for_it():
+    from photon_infer_amd.ops import fast
+    assert fast._tile_shape_of(300, 200, 1000, 1, 256) == 0 and fast._tile_shape_of(2048, 16384, 2040, 1, 256) == 0
+
+
+# (rows, columns, k), microseconds of the product in one, two, ... pieces with the norm that adds them, each in its fastest tile shape, weights cold, measured
 PIECES_MEASURED = [
-    (130, 2048, 2048, [23.1, 15.8, 14.3, 13.8, 14.0, 14.2, 14.4, 14.6]), (200, 2048, 2048, [23.2, 16.5, 15.4, 15.1, 15.6, 16.2, 16.9, 17.5]),
-    (300, 2048, 2048, [23.8, 18.1, 17.9, 18.4, 19.6, 20.0, 21.8, 21.3]), (130, 2048, 8192, [74.4, 43.4, 32.5, 27.3, 24.4, 22.7, 21.5, 20.2]),
-    (2048, 2048, 8192, [98.6, 83.6, 85.5, 87.7]), (1400, 2048, 8192, [88.3, 66.9, 72.1, 65.6, 71.4]), (256, 4096, 4096, [49.0, 29.8, 25.8, 24.3, 26.7, 27.8, 29.9, 28.7]),
-    (1000, 4096, 4096, [58.5, 53.4, 57.7, 59.3]), (2048, 4096, 4096, [86.9, 90.5]), (200, 4096, 14336, [135.4, 74.6, 55.8, 47.8, 46.6, 43.2, 42.0, 41.4]),
-    (700, 1024, 1024, [17.6, 14.9, 15.7, 17.0]), (300, 3072, 3072, [43.5, 27.4, 24.3, 24.5, 24.3, 25.0, 26.6, 28.2]), (2600, 2048, 2048, [46.1, 47.8, 59.9]), (1267, 5376, 4544, [104.3, 175.0]),
+    (130, 2048, 2048, [22.9, 15.8, 14.5, 14.0, 14.3, 14.4, 14.5, 14.8]), (200, 2048, 2048, [23.0, 16.5, 15.7, 15.3, 15.8, 16.3, 16.7, 17.2]),
+    (300, 2048, 2048, [24.2, 18.4, 18.0, 18.3, 19.1, 19.8, 20.5, 20.7]), (130, 2048, 8192, [65.4, 37.6, 28.6, 24.8, 22.4, 21.2, 20.2, 20.7]),
+    (300, 2048, 8192, [67.8, 40.6, 31.7, 28.4, 26.3, 30.4, 29.2, 28.1]), (2048, 2048, 8192, [84.2, 79.9, 81.9, 81.2]),
+    (1500, 2048, 8192, [75.1, 67.1, 65.8, 64.6, 67.1]), (256, 4096, 4096, [47.4, 29.7, 25.7, 23.8, 26.4, 25.8, 26.4, 27.8]),
+    (1000, 4096, 4096, [53.7, 51.9, 55.2, 57.9]), (2048, 2048, 2048, [34.7, 37.5, 41.5, 44.4]),
+    (200, 4096, 14336, [124.6, 68.9, 52.7, 44.8, 53.0, 48.5, 47.8, 45.5]), (543, 4096, 14336, [119.3, 101.9, 82.7, 82.3, 77.5, 93.0, 88.3]),
+    (700, 1024, 1024, [17.9, 15.3, 16.0, 16.8]), (300, 3072, 3072, [35.2, 24.7, 22.6, 24.6, 24.3, 23.9, 24.1, 26.9]),
+    (1150, 3072, 3072, [42.2, 41.9, 44.3, 49.3]), (2627, 2048, 2048, [42.4, 46.2, 53.2]), (1267, 5376, 4544, [114.2, 174.3]),
+    (850, 6144, 4096, [89.2, 111.1, 120.6]), (700, 3072, 2048, [30.7, 28.4, 27.6, 29.9, 31.3, 34.1, 36.4]),
+    (1000, 2080, 2048, [31.1, 28.4, 27.2, 30.9, 32.0, 34.5, 36.4, 42.2]), (2627, 832, 2048, [30.5, 28.2, 28.1, 31.2, 33.4, 35.5, 41.8]),
 ]
 
 
@@ -213,13 +239,13 @@ def test_a_product_is_left_in_as_many_pieces_as_were_the_fastest(M, N, K, times)
     assert times[fast._tile_splits_of(M, N, K, 256, 1.0) - 1] <= 1.05 * min(times)
 
 
-@pytest.mark.parametrize("N,K,tokens", [(3072, 2048, 1280), (5120, 3072, 768), (6144, 4096, 640), (2560, 1024, 1024), (4608, 3584, 896), (8256, 4096, 128),
-                                        (10240, 8192, 128), (16320, 512, 128)])
+@pytest.mark.parametrize("N,K,tokens", [(3072, 2048, 1280), (5120, 3072, 1152), (6144, 4096, 1280), (2560, 1024, 1536), (4608, 3584, 1536), (4096, 2560, 1280),
+                                        (9216, 4096, 896), (10240, 8192, 1536), (2048, 2048, 2048), (8256, 4096, 128), (16320, 512, 128)])
 def test_queries_keys_and_values_of_some_hundred_tokens_reach_the_rotation_in_float32(N, K, tokens):
-    """Cut over k or not: from 33 tokens on as long as the result has no more tiles than the chip has units."""
+    """Cut over k or not: from 33 tokens on as long as the result has no more tiles than the chip has units, more with a longer k."""
     from photon_infer_amd.ops import fast
     for M in range(33, tokens + 1):
-        cut = fast._skinny_splits_of(M, N, K, 256) if M <= fast.SKINNY_MAX_ROWS else fast._tile_splits_of(M, N, K, 256, fast.PIECES_WORTH)
+        cut = fast._skinny_splits_of(M, N, K, 256) if M <= fast.SKINNY_MAX_ROWS else fast._tile_splits_of(M, N, K, 256, fast.PIECES_WORTH, norm=False)
         assert cut > 1 or fast.keeps_float32(M, N, K, 256), M
 
 
