@@ -20,7 +20,7 @@ struct Shape {
 };
 constexpr Shape SHAPES[] = {
     {0, 128, 128, 2, {1.0, 5.84, 0.66}, {4.95, 14.69}},
-    {42, 256, 256, 1, {5.29, 15.8, 0.05}, {8.75, 20.22}},
+    {42, 256, 256, 1, {5.29, 15.8, 0.05}, {8.75, 19.82}},
     {33, 192, 384, 1, {6.33, 19.74, 0.41}, {9.56, 26.3}},
     {32, 192, 256, 1, {4.98, 13.26, 0.08}, {7.45, 17.28}},
     {23, 128, 384, 1, {5.81, 13.05, 1.03}, {5.25, 22.8}},
