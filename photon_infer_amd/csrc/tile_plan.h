@@ -37,7 +37,7 @@ constexpr int MIN_K = 256;             // a piece keeps at least this much of k
 constexpr double SHAPE_GAIN = 0.97, PIECES_GAIN = 0.945;
 // Bytes per microsecond of pieces, or of the updated stream, on their way into the norm behind the product, and what every
 // piece takes there besides (writing them is hidden in the times above).  Over the 301 products measured with the norm the
-// choice is 0.8 % above the best in the mean: 300 x 2,048 x 8,192 takes 68 us in one piece, 28.2 in five and 29.5 in eight,
+// choice is 0.9 % above the best in the mean: 300 x 2,048 x 8,192 takes 68 us in one piece, 28.2 in five and 29.5 in eight,
 // 256 x 4,096 x 4,096 48, 25.7 in three and 28.5.  Rows of more than 4,096 columns go through the norm at a third of that
 // rate (1,267 x 5,376 x 4,544: 104 us in one piece, 175 in two), through the rotation of q, k and v at the same (500 x 6,144 x
 // 4,096 with the rotation 48.8 us in one float32 piece, 43.8 in two; 500 x 5,120 x 3,072 41.5, 34.1 in three).

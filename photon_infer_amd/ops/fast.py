@@ -32,7 +32,10 @@ ROWS_PER_BLOCK = 32            # weight rows per block of the skinny kernel
 BLOCKS_PER_UNIT = 2            # blocks of it wanted per compute unit to keep HBM busy (measured: 512 on 256 units; 384 and 768 are slower)
 SHARED_FROM_TOKENS = 32        # more tokens than this: the skinny kernel that shares activations per block ...
 SHARED_ROWS_PER_BLOCK = 64     # ... with this many weight rows per block, and no more blocks than compute units (100 tokens, 3,072 x 8,192:
-                               # 22.8 us in six pieces on 288 blocks, 16.9 in five on 240; 6,144 x 4,096 22.8 in three, 18.7 in two)
+                               # 22.8 us in six pieces on 288 blocks, 16.9 in five on 240; 6,144 x 4,096 22.8 in three, 18.7 in two), though
+                               # a unit would hold two: 64 tokens, k 4,096, blocks for half the units or more in one piece and in two, 8,256
+                               # rows 29.7 and 32.0, 9,216 29.2 and 31.3, 12,160 29.4 and 31.1, 14,720 33.2 and 35.4; the same at 100 tokens
+                               # (35.7 and 39.0, 35.4 and 38.0, 35.4 and 37.6, 39.1 and 41.7), and at k of 2,048 and 8,192
 RING_MAX_STRIDE = 1 << 21      # elements between rows up to which that kernel's byte offsets fit 31 bits
 FLOAT32_ROWS = 32              # up to this many rows a float32 product goes to the weight-streaming kernel
 FLOAT32_MAX_STRIDE = 1 << 21   # floats between rows up to which the float32 kernels' offsets inside a tile fit 32 bits
