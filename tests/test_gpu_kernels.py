@@ -585,7 +585,7 @@ def test_rope_kv_write(_ops, dtype, hd, rot, inter):
 
 
 @pytest.mark.parametrize("hd,page,rotate", [(64, 16, True), (128, 4, True), (64, 8, False), (16, 4, True)])
-@pytest.mark.parametrize("pieces", [0, 3, 6])
+@pytest.mark.parametrize("pieces", [0, 1, 3, 6])
 def test_rope_kv_write_many_tokens(_ops, hd, page, rotate, pieces):
     """Prompts take the kernel with wide accesses: portions that start at any row of the batch
     and at any position, single tokens among them, pages of several sizes; q, k and v as a
@@ -645,7 +645,7 @@ def test_rope_kv_write_many_tokens(_ops, hd, page, rotate, pieces):
 
 @pytest.mark.parametrize("hd,nh,nkv,page,window,rotate", [(64, 8, 2, 16, 0, True), (128, 4, 4, 32, 40, True), (64, 6, 2, 16, 24, False),
                                                           (128, 16, 1, 16, 0, True)])
-@pytest.mark.parametrize("pieces", [False, True])
+@pytest.mark.parametrize("pieces", [0, 1, 3])
 def test_decode_attention_from_projection(_ops, hd, nh, nkv, page, window, rotate, pieces):
     """A step of single tokens through the kernel that rotates, writes the cache and attends at
     once: the cache it leaves and its outputs are, bit for bit, those of the separate kernels
@@ -668,8 +668,8 @@ def test_decode_attention_from_projection(_ops, hd, nh, nkv, page, window, rotat
         kv.v[pg, :, :, sl] = -1e4
     N = (nh + 2 * nkv) * hd
     if pieces:
-        part = (torch.randn(3, R, N, generator=g) * 0.4).to(DEV)
-        qkv = fast.Partials(part, 3, R, N)
+        part = (torch.randn(pieces, R, N, generator=g) * 0.7 * pieces ** -0.5).to(DEV)
+        qkv = fast.Partials(part, pieces, R, N)
     else:
         qkv = (torch.randn(R, N, generator=g) * 0.6).to(BF16).to(DEV)
     freqs = P.rope_frequencies(hd, 10000.0, None)
