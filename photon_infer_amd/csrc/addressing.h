@@ -123,6 +123,29 @@ PI_ADDR unsigned ring_w_step_offset(int tiled, unsigned lane_offset, int k0, int
   return k0 + piece * 8 < k_range ? lane_offset + (unsigned)k0 * (tiled ? 32u : 2u) : OUT_OF_RANGE;
 }
 
+// ---------------------------------------------------------------- gemm_rows_kernel (1..16 tokens, all of k in a block)
+// Through descriptors of a wave's own k-range (whole steps of 64): the weights from the copy, of which 16 rows x 64 k are 2 KB
+// in a row, and M rows of activations.  Offsets of a step s beyond the wave's last, and of rows beyond M, lie outside.
+PI_ADDR Descriptor rows_w_descriptor(long n0, int k0, int steps, int K) {
+  return Descriptor{n0 / 16 * 16 * K + (long)k0 * 16, (long)steps * 2048};
+}
+PI_ADDR Descriptor rows_a_descriptor(int k0, int steps, int M, long lda) {
+  return Descriptor{k0, steps > 0 ? ((M - 1) * lda + (long)steps * KSTEP) * 2 : 0};
+}
+// 16 rows a block: lane row lane % 16, fragment f (its k = 16 (lane / 16) + 8 f .. + 7 of the step).  8 rows, the upper or lower
+// half of 16: lanes with lane % 16 >= 8 hold fragment 1 of row lane % 8, the others fragment 0.
+PI_ADDR unsigned rows_w_lane(int rows, long n0, int lane) {
+  return (unsigned)(rows == 16 ? lane / 16 * 256 + lane % 16 * 16 : lane % 16 / 8 * 1024 + lane / 16 * 256 + (int)(n0 / 8 % 2) * 128 + lane % 8 * 16);
+}
+// Activations: `wide`: token lane % 16, fragment f at + 16 f bytes; else token lane % 8, fragment lane % 16 / 8.
+PI_ADDR unsigned rows_a_lane(bool wide, int lane, int M, long lda) {
+  const int token = wide ? lane % 16 : lane % 8;
+  return token < M ? (unsigned)(token * (int)lda + lane / 16 * 16 + (wide ? 0 : lane % 16 / 8 * 8)) * 2u : OUT_OF_RANGE;
+}
+PI_ADDR unsigned rows_step(unsigned lane_offset, int s, int steps, int step_bytes, int more) {
+  return s < steps && lane_offset != OUT_OF_RANGE ? lane_offset + (unsigned)(s * step_bytes + more) : OUT_OF_RANGE;
+}
+
 // ---------------------------------------------------------------- attention over the paged cache
 // Keys [pages, kv_heads, page, HD], values transposed [pages, kv_heads, HD, page], bfloat16.  A
 // chunk is two tiles of 16 keys; a tile lies in one page (pages hold a multiple of 16 tokens) at

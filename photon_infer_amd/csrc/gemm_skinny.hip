@@ -118,6 +118,38 @@ __device__ inline void merge_ranges_of_tokens(const float* __restrict__ head_bas
   }
 }
 
+// Activations of a norm whose root was left to this reader (gemm_rows_kernel made them): row m holds x * w, and the
+// product of the normalised row is the product of these times 1 / sqrt(mean of x^2 + eps), a factor per row that the
+// epilogue applies in float32.  sums: float32 [M][count], a row's sum of x^2 in pieces.
+struct LeftNorm {
+  const float* sums;
+  int count, width;
+  float eps;
+};
+
+// The factors of rows wave * 4 .. + 3 of a block of four waves, sixteen lanes to a row.  load() asks for the pieces (up to 512
+// a row) before the weights' loop, so that they travel beside it; finish() adds them, the same way in every block, and leaves
+// the factors in LDS.
+struct LeftNormRows {
+  f32x4_t piece[8];
+  __device__ inline void load(const LeftNorm& left, int wave, int lane, int M) {
+    const int m = wave * 4 + lane / 16;
+    const float* row = left.sums + (long)m * left.count;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int at = u * 64 + lane % 16 * 4;
+      piece[u] = m < M && at < left.count ? *reinterpret_cast<const f32x4_t*>(row + at) : f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+  }
+  __device__ inline void finish(const LeftNorm& left, int wave, int lane, float* factors) {
+    const f32x4_t p = ((piece[0] + piece[1]) + (piece[2] + piece[3])) + ((piece[4] + piece[5]) + (piece[6] + piece[7]));
+    float sum = (p[0] + p[1]) + (p[2] + p[3]);
+#pragma unroll
+    for (int off = 1; off < 16; off <<= 1) sum += __shfl_xor(sum, off, PI_WAVE);
+    if (lane % 16 == 0) factors[wave * 4 + lane / 16] = 1.0f / sqrtf(sum / (float)left.width + left.eps);
+  }
+};
+
 template <int MB, int RT>
 union SkinnyLds {
   float red[4][RT * 16][MB * 16 + 1];
@@ -419,6 +451,230 @@ __global__ __launch_bounds__(512, 4) void gemm_skinny_ring_kernel(void* __restri
     if (splits == 1) epilogue_store<EPI>(Cv, ldc, m, n0 + nl, total(nl, m));
     else mine[(long)m * N + n0 + nl] = total(nl, m);   // the consumer adds the splits in split order
   }
+}
+
+// The product of up to 16 tokens with all of k in a block, from the weights' copy.  A block takes 8, 16 or 32 rows and each of
+// its four or eight waves a share of k: nothing is staged or shared, the loads of eight steps (four with 32 rows) are in flight,
+// and the waves' tiles are added once, in LDS.  With 8 rows lanes 8..15 of a column hold the step's second fragment of rows
+// 0..7, so a step is one load and two matrix instructions (one up to 8 tokens: columns 8..15 then hold the tokens' second
+// fragment), of whose results half are of use.
+// Bound by the weights' way from memory, and from 8 tokens on by the activations' from L2, which every block reads.
+//
+// ROWS_FINISH: X[M, N] += A . W^T of a stream, and of the stream's next norm what needs no other block: h = bfloat16(x * w) and
+// the block's share of the rows' sums of x^2.  The root is left to whoever reads h (LEFT): h is rounded once and by as much as
+// the normalised row would be, and the factor is applied to float32 sums.  In place of a product in pieces of k and a norm that
+// adds them, the second of which does little but start.  Weights cold, with that norm, 1 / 8 / 12 tokens, us: 2,048 x 8,192
+// 12.5 / 12.4 / 12.6 -> 8.6 / 9.9 / 11.6; 2,048 x 2,048 7.2 / 7.4 / 7.7 -> 3.9 / 4.3 / 4.7; 3,072 x 8,192 16.9 / 17.2 / 17.6 -> 12.4 /
+// 13.4 / 14.8; 4,096 x 14,336 29.2 / 29.7 / 30.2 -> 23.7 / 24.2 / 25.6; 4,096 x 4,096 14.2 / 14.5 / 14.9 -> 8.8 / 9.3 / 10.1.
+// The reader's part takes 0.2 to 0.5 us where the sums' loads go out behind the weights' (1.0 in front of them).
+//
+// The other epilogues take the place of gemm_skinny_kernel, four waves on 32 rows that staged the activations of a step at a
+// time, where that did not cut k over blocks: 16,384 x 2,048 with the gated unit, 1 / 8 / 16 tokens 15.7 / 15.8 / 15.6 us -> 14.5 /
+// 14.4 / 15.4; 28,672 x 4,096 50.4 / 50.1 / 51.1 -> 43.6 / 44.8 / 46.0; 128,256 x 2,048 93.4 / 96.3 / 102.7 -> 90.8 / 93.2 / 100.7.
+enum { ROWS_FINISH = 8 };      // besides EPI_BF16, EPI_F32 and EPI_SWIGLU
+
+struct FinishTo {              // ROWS_FINISH
+  const void* weight;          // of the norm, bfloat16 or float32
+  bf16_t* h;
+  float* sums;
+};
+
+template <int WAVES, int ROWS, bool WIDE, int EPI, bool LEFT, typename TW>
+__global__ __launch_bounds__(WAVES * 64) void gemm_rows_kernel(void* __restrict__ Cv, long ldc, const bf16_t* __restrict__ A, long lda,
+                                                              const bf16_t* __restrict__ W, int M, int N, int K, FinishTo fin, LeftNorm left) {
+  static_assert(ROWS == 8 || (WIDE && (ROWS == 16 || ROWS == 32)), "8, 16 or 32 rows");
+  constexpr int DEPTH = ROWS == 32 ? 4 : 8;                // steps whose loads are in flight
+  constexpr int RT = ROWS == 32 ? 2 : 1;                   // tiles of 16 rows (or one of 8)
+  constexpr int XF = WIDE ? 2 : 1, WF = ROWS == 8 ? 1 : 2; // fragments of a step: activations, weights of a tile
+  constexpr int PARTS = ROWS == 8 ? 2 * WAVES : WAVES;     // sums to add
+  constexpr int OUT_ROWS = EPI == EPI_SWIGLU ? ROWS / 2 : ROWS, TOKENS = WIDE ? 16 : 8;
+  __shared__ float red[PARTS][ROWS][17];
+  __shared__ float factors[LEFT ? 16 : 1];
+  const int tid = threadIdx.x, lane = tid % 64;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+  const int lr = lane % 16, lg = lane / 16;
+  // blocks go to the dies in turn: every die a run of rows, so that a line of the result is written by one die
+  const int dies = gridDim.x % 8 == 0 ? 8 : 1, block = blockIdx.x % dies * (gridDim.x / dies) + blockIdx.x / dies;
+  const long n0 = (long)block * ROWS;
+  float x = 0.f, wn = 0.f;
+  if constexpr (EPI == ROWS_FINISH) {
+    if (tid / ROWS < M) {
+      x = reinterpret_cast<const float*>(Cv)[(long)(tid / ROWS) * N + n0 + tid % ROWS];
+      wn = to_float(reinterpret_cast<const TW*>(fin.weight)[n0 + tid % ROWS]);
+    }
+  }
+  const addressing::WaveRange range = addressing::wave_share(0, K, WAVES, wave);
+  const int steps = range.k1 > range.k0 ? (range.k1 - range.k0) / KSTEP : 0;
+#if defined(__HIP_DEVICE_COMPILE__)
+  __amdgpu_buffer_rsrc_t w_src[RT];
+#pragma unroll
+  for (int t = 0; t < RT; ++t) w_src[t] = operand_descriptor(W, addressing::rows_w_descriptor(n0 + t * 16, range.k0, steps, K));
+  const __amdgpu_buffer_rsrc_t a_src = operand_descriptor(A, addressing::rows_a_descriptor(range.k0, steps, M, lda));
+#endif
+  const unsigned w_lane = addressing::rows_w_lane(ROWS == 8 ? 8 : 16, n0, lane), a_lane = addressing::rows_a_lane(WIDE, lane, M, lda);
+
+  Frag w[DEPTH][RT][WF], a[DEPTH][XF];
+  constexpr int ACCS = ROWS == 8 ? XF : RT;
+  f32x4_t acc[ACCS];
+#pragma unroll
+  for (int f = 0; f < ACCS; ++f) acc[f] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  auto fetch = [&](const int s, const int j) {
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+      for (int f = 0; f < WF; ++f)
+        w[j][t][f].n = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(w_src[t], addressing::rows_step(w_lane, s, steps, 2048, f * 1024), 0, 0));
+#pragma unroll
+    for (int f = 0; f < XF; ++f)
+      a[j][f].n = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(a_src, addressing::rows_step(a_lane, s, steps, 2 * KSTEP, f * 16), 0, 0));
+#endif
+  };
+#pragma unroll
+  for (int j = 0; j < DEPTH; ++j) fetch(j, j);
+  LeftNormRows rows_left;
+  if constexpr (LEFT) {
+    __builtin_amdgcn_sched_barrier(0);          // behind the weights' loads, whose waits then do not include them
+    if (wave < 4) rows_left.load(left, wave, lane, M);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  for (int s0 = 0; s0 < steps; s0 += DEPTH) {
+    const bool more = s0 + DEPTH < steps;
+#pragma unroll
+    for (int j = 0; j < DEPTH; ++j) {
+#pragma unroll
+      for (int f = 0; f < XF; ++f)
+#pragma unroll
+        for (int t = 0; t < RT; ++t) {
+          f32x4_t& sum = acc[ROWS == 8 ? f : t];
+          sum = mfma16(w[j][t][f % WF], a[j][f], sum);
+        }
+      if (more) fetch(s0 + DEPTH + j, j);
+    }
+  }
+  if constexpr (LEFT) {
+    if (wave < 4) rows_left.finish(left, wave, lane, factors);
+  }
+  // row lg * 4 + i, column lr of a tile; with 8 rows the weights' fragment lg / 2 of row (lg % 2) * 4 + i
+  if constexpr (ROWS != 8) {
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) red[wave][t * 16 + lg * 4 + i][lr] = acc[t][i];
+  } else if constexpr (WIDE) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) red[wave * 2 + lg / 2][(lg % 2) * 4 + i][lr] = lg < 2 ? acc[0][i] : acc[1][i];
+  } else if (lr / 8 == lg / 2) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) red[wave * 2 + lg / 2][(lg % 2) * 4 + i][lr % 8] = acc[0][i];
+  }
+  __syncthreads();
+  for (int at = tid; at < OUT_ROWS * TOKENS; at += WAVES * 64) {          // whole waves
+    const int token = at / OUT_ROWS, row = at % OUT_ROWS;
+    const bool mine = token < M;
+    auto total = [&](const int r, float sum) {
+#pragma unroll
+      for (int p = 0; p < PARTS; ++p) sum += red[p][r][token];
+      return sum;
+    };
+    if constexpr (EPI == ROWS_FINISH) {
+      static_assert(OUT_ROWS * TOKENS <= WAVES * 64, "one result to a thread");
+      x = total(row, x);
+      float square = x * x;
+#pragma unroll
+      for (int off = 1; off < ROWS; off <<= 1) square += __shfl_xor(square, off, PI_WAVE);
+      if (!mine) return;
+      reinterpret_cast<float*>(Cv)[(long)token * N + n0 + row] = x;
+      fin.h[(long)token * N + n0 + row] = from_float<bf16_t>(x * wn);
+      if (row == 0) fin.sums[(long)token * gridDim.x + block] = square;
+    } else if (mine) {
+      const float factor = LEFT ? factors[token] : 1.f;
+      if constexpr (EPI == EPI_SWIGLU) {
+        const float g = total(row, 0.f) * factor, u = total(16 + row, 0.f) * factor;
+        reinterpret_cast<bf16_t*>(Cv)[(long)token * ldc + n0 / 2 + row] = from_float<bf16_t>(g / (1.0f + expf(-g)) * u);
+      } else {
+        epilogue_store<EPI>(Cv, ldc, token, n0 + row, total(row, 0.f) * factor);
+      }
+    }
+  }
+}
+
+// Rows of a block: 8 while blocks of 16 would leave more than a quarter of the units without one (2,048 x 8,192, one token 8.6
+// and 10.0 us; 3,072 x 8,192 13.0 and 12.4, eight tokens 16.9 and 13.4).
+static int finish_rows(int N) { return N / 16 * 4 < 3 * compute_units() ? 8 : 16; }
+
+// Blocks (= pieces of a row's sum of squares) with which the finishing kernel takes a product, 0 where it does not: M up to 16,
+// N % 64 and K % 64, up to 512 blocks (what LeftNormRows holds), and not the many tokens of a long k with 8 rows to a block,
+// whose activations every block reads (2,048 x 8,192: 12 tokens 12.6 in pieces with the norm and 11.6, 16 tokens 12.8 and 13.0).
+extern "C" int pi_gemm_finish_blocks(int M, int N, int K) {
+  if (M < 1 || M > 16 || N < 64 || N % 64 || K < KSTEP || K % KSTEP) return 0;
+  const int rows = finish_rows(N);
+  if (N / rows > 512 || (rows == 8 && M > 12 && K > 4096)) return 0;
+  return N / rows;
+}
+
+// W: the copy in the streaming order (see pi_gemm_skinny).  H bfloat16 [M, N], sums float32 [M, blocks].
+extern "C" int pi_gemm_finish(float* X, const void* A, long lda, const void* W, const void* norm_w, int norm_dtype, void* H, float* sums, long sums_elems,
+                              int M, int N, int K, hipStream_t stream) {
+  const int blocks = pi_gemm_finish_blocks(M, N, K);
+  PI_REQUIRE(blocks > 0, "gemm_finish: not for M=%d N=%d K=%d", M, N, K);
+  PI_REQUIRE(lda >= K && lda % 8 == 0 && lda < RING_MAX_STRIDE && ((uintptr_t)A % 16 == 0) && ((uintptr_t)W % 16 == 0), "gemm_finish: operands must be 16-byte aligned, the row stride (%ld) a multiple of 8", lda);
+  PI_REQUIRE(sums_elems >= (long)M * blocks, "gemm_finish: %ld floats for %ld sums", sums_elems, (long)M * blocks);
+  PI_REQUIRE(norm_dtype == PI_F32 || norm_dtype == PI_BF16, "gemm_finish: unsupported norm weight dtype %d", norm_dtype);
+  // waves: eight for a long k where a unit has no more than a block's worth of loads in flight otherwise
+  const int rows = N / blocks;
+  const bool eight = K > 2048 && (rows == 8 || blocks < compute_units());
+#define GO(WV, RW, WD, T) \
+  hipLaunchKernelGGL((gemm_rows_kernel<WV, RW, WD, ROWS_FINISH, false, T>), dim3(blocks), dim3(WV * 64), 0, stream, X, (long)N, (const bf16_t*)A, lda, \
+                     (const bf16_t*)W, M, N, K, FinishTo{norm_w, (bf16_t*)H, sums}, LeftNorm{})
+#define PICK(WV, T) \
+  do { \
+    if (rows == 16) GO(WV, 16, true, T); \
+    else if (M > 8) GO(WV, 8, true, T); \
+    else GO(WV, 8, false, T); \
+  } while (0)
+  if (eight && norm_dtype == PI_BF16) PICK(8, bf16_t);
+  else if (eight) PICK(8, float);
+  else if (norm_dtype == PI_BF16) PICK(4, bf16_t);
+  else PICK(4, float);
+#undef PICK
+#undef GO
+  return pi_check_launch("gemm_finish");
+}
+
+// C[M, N] = A[M, K] . W[N, K]^T for 1..16 tokens with all of k in a block, W the copy in the streaming order: stored in
+// bfloat16 or float32, added into float32, or through the gated unit (gate and up rows interleaved by 16).  `sums` (or null): A is
+// what pi_gemm_finish left of a norm; float32 [M, count], 16-byte aligned, K the norm's width.
+extern "C" int pi_gemm_rows(void* C, int epilogue, long ldc, const void* A, long lda, const void* W, int M, int N, int K, const float* sums, int count,
+                            float eps, hipStream_t stream) {
+  PI_REQUIRE(M > 0 && M <= 16 && N > 0 && N % 16 == 0 && K > 0 && K % KSTEP == 0, "gemm_rows: takes 1..16 tokens, N in 16 and K in 64, got M=%d N=%d K=%d", M, N, K);
+  PI_REQUIRE(epilogue != EPI_SWIGLU || N % 32 == 0, "gemm_rows: the gated unit takes N (%d) in 32", N);
+  PI_REQUIRE(lda >= K && lda % 8 == 0 && lda < RING_MAX_STRIDE && K < RING_MAX_STRIDE && ((uintptr_t)A % 16 == 0) && ((uintptr_t)W % 16 == 0), "gemm_rows: operands must be 16-byte aligned, the row stride (%ld) a multiple of 8", lda);
+  PI_REQUIRE(!sums || (count > 0 && count <= 512 && count % 4 == 0 && (uintptr_t)sums % 16 == 0), "gemm_rows: a left norm has 4..512 sums a row, got %d", count);
+  // 16 rows to a block while the units take them in one round (3,072 x 2,048, 8 tokens 5.0 us and 6.0; 5,120 x 3,072 11.4 and 8.7)
+  const int rows = epilogue == EPI_SWIGLU || (N / 16 > compute_units() && N % 32 == 0) ? 32 : 16;
+  const LeftNorm left{sums, count, K, eps};
+#define GO(RW, E, L) hipLaunchKernelGGL((gemm_rows_kernel<4, RW, true, E, L, float>), dim3(N / RW), dim3(256), 0, stream, C, ldc, (const bf16_t*)A, lda, (const bf16_t*)W, M, N, K, FinishTo{}, left)
+#define PICK(E) \
+  do { \
+    if (sums && rows == 32) GO(32, E, true); \
+    else if (sums) GO(16, E, true); \
+    else if (rows == 32) GO(32, E, false); \
+    else GO(16, E, false); \
+  } while (0)
+  switch (epilogue) {
+    case EPI_BF16: PICK(EPI_BF16); break;
+    case EPI_F32: PICK(EPI_F32); break;
+    case EPI_ACCUM: PICK(EPI_ACCUM); break;
+    case EPI_SWIGLU:
+      if (sums) GO(32, EPI_SWIGLU, true);
+      else GO(32, EPI_SWIGLU, false);
+      break;
+    default: return pi_fail("gemm_rows: unknown epilogue %d", epilogue);
+  }
+#undef PICK
+#undef GO
+  return pi_check_launch("gemm_rows");
 }
 
 template <int MB>

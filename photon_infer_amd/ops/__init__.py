@@ -18,7 +18,7 @@ import torch
 
 from ..errors import KernelError
 from . import _lib, fast
-from .workspace import KernelWorkspace, KeyRanges, Partials, stream_layout, stream_layout_takes
+from .workspace import KernelWorkspace, KeyRanges, LeftNorm, Partials, stream_layout, stream_layout_takes
 
 PI_F32, PI_BF16 = 0, 1
 MAX_HEAD_DIM = 256              # the matrix-core attention kernels
@@ -172,7 +172,10 @@ def rmsnorm(out: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, eps: float
 def materialize(x: torch.Tensor, ws: Optional[KernelWorkspace]) -> torch.Tensor:
     """Apply an update of ``x`` that is still pending in ``ws``, if there is one (a result whose pieces are unadded is
     written)."""
-    p = ws.pending if ws is not None else None
+    if ws is None:
+        return x
+    ws.left_norm = None                # whoever asks may be about to change the stream
+    p = ws.pending
     if p is not None and p.is_for(x):
         ws.pending = None
         fast.reduce_into(x, p.pieces, accumulate=p.accumulate)
@@ -183,7 +186,17 @@ def materialize(x: torch.Tensor, ws: Optional[KernelWorkspace]) -> torch.Tensor:
 def reset_deferred(ws: Optional[KernelWorkspace]) -> None:
     """Forget a pending update (start of a step: nothing of an earlier, failed step may linger)."""
     if ws is not None:
-        ws.pending = None
+        ws.pending = ws.left_norm = None
+
+
+def whole_norm(h):
+    """``h``, or the normalised rows that a ``LeftNorm`` stands for (for a reader that cannot apply the root itself), made
+    from its stream, which must be as the norm's maker left it."""
+    if not isinstance(h, LeftNorm):
+        return h
+    out = torch.empty_like(h.h)
+    rmsnorm(out, h.x, h.weight, h.eps)
+    return out
 
 
 def discard_deferred(x: torch.Tensor, ws: Optional[KernelWorkspace]) -> None:
@@ -210,6 +223,12 @@ def gemm_swiglu(out: torch.Tensor, a: torch.Tensor, w_gate_up: torch.Tensor, blo
     """out[M, I] = silu(a @ Wg^T) * (a @ Wu^T) where ``w_gate_up`` [2I, K] holds the gate and
     up rows in halves (``block`` 0) or interleaved in blocks of ``block`` rows.  With bfloat16
     operands and blocks of 16 the product and the activation are one kernel."""
+    left = a if isinstance(a, LeftNorm) else None
+    if left is not None:
+        if not (_FAST and block == 16 and w_gate_up.dtype == torch.bfloat16 and out.is_contiguous()):
+            left, a = None, whole_norm(a)
+        else:
+            a = left.h
     _gpu(out, a, w_gate_up)
     M, I = out.shape
     if w_gate_up.shape[0] != 2 * I or a.shape != (M, w_gate_up.shape[1]) or out.dtype != a.dtype:
@@ -217,8 +236,9 @@ def gemm_swiglu(out: torch.Tensor, a: torch.Tensor, w_gate_up: torch.Tensor, blo
     if M == 0:
         return
     if _FAST and block == 16 and a.dtype == torch.bfloat16 and w_gate_up.dtype == torch.bfloat16 and out.is_contiguous():
-        if fast.gemm_swiglu(out, a, w_gate_up, M, 2 * I, a.shape[1], _rows(a, "gemm a"), _rows(w_gate_up, "gemm w"), ws):
+        if fast.gemm_swiglu(out, a, w_gate_up, M, 2 * I, a.shape[1], _rows(a, "gemm a"), _rows(w_gate_up, "gemm w"), ws, left):
             return
+        a = a if left is None else whole_norm(left)
     if _FAST and block == 16 and a.dtype == torch.float32 and w_gate_up.dtype == torch.float32 and out.is_contiguous():
         if fast.gemm_swiglu_float32(out, a, w_gate_up, M, 2 * I, a.shape[1], _rows(a, "gemm a"), _rows(w_gate_up, "gemm w")):
             return
@@ -228,13 +248,22 @@ def gemm_swiglu(out: torch.Tensor, a: torch.Tensor, w_gate_up: torch.Tensor, blo
 
 
 def gemm(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, accumulate: bool = False,
-         may_defer: bool = False, ws: Optional[KernelWorkspace] = None) -> None:
+         may_defer: bool = False, ws: Optional[KernelWorkspace] = None, next_norm=None) -> None:
     """out[M, N] (+)= a[M, K] @ w[N, K]^T with float32 accumulation.
 
     ``ws``: where a product split over k keeps its pieces (without one, memory of this call's own).
     ``may_defer`` (with ``ws``): the caller promises that ``out`` is next read by ``rmsnorm`` or ``materialize``
     - a result that is not accumulated: by ``hyper_streams`` or ``materialize`` - with the same workspace; a
-    product that was split over k may then stay in pieces there."""
+    product that was split over k may then stay in pieces there.
+    ``next_norm`` (with ``may_defer``; (weight, eps)): the RMS norm that reads ``out`` next, whose own reader is a product that
+    takes a ``LeftNorm``: a product of few tokens may then finish ``out`` and leave that in the workspace
+    (``KernelWorkspace.take_left_norm``)."""
+    left = None
+    if isinstance(a, LeftNorm):
+        if _FAST and w.dtype == torch.bfloat16 and not accumulate and not may_defer:
+            left, a = a, a.h
+        else:
+            a = whole_norm(a)
     if isinstance(a, KeyRanges):
         # attention's output of a decode step, its key ranges not merged yet: the weight-streaming
         # kernel merges them as it reads; anything else gets them merged first
@@ -266,8 +295,11 @@ def gemm(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, accumulate: bool =
     if accumulate:
         materialize(out, ws)
     if _FAST and a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16:
-        if fast.gemm(out, a, w, accumulate, M, N, K, lda, ldw, ldc, may_defer and out.dtype == torch.float32 and out.is_contiguous(), ws):
+        may_defer_ = may_defer and out.dtype == torch.float32 and out.is_contiguous()
+        if fast.gemm(out, a, w, accumulate, M, N, K, lda, ldw, ldc, may_defer_, ws, left, next_norm):
             return
+    if left is not None:
+        a = whole_norm(left)
     if _FAST and a.dtype == torch.float32 and w.dtype == torch.float32 and out.dtype == torch.float32:
         if fast.gemm_float32(out, a, w, accumulate, M, N, K, lda, ldw, ldc, may_defer and out.is_contiguous(), ws):
             return
@@ -322,7 +354,8 @@ def qkv_projection(h: torch.Tensor, w_qkv: torch.Tensor, dtype: torch.dtype, ws:
     values.  The pieces are good until the next product with the same workspace.  A result of bfloat16
     that is not split may come as one float32 piece too (``fast.keeps_float32``)."""
     if _FAST and ws is not None and h.dtype == torch.bfloat16 and w_qkv.dtype == torch.bfloat16 and h.is_cuda:
-        p = fast.gemm_pieces(h, w_qkv, ws, whole=dtype == torch.bfloat16)
+        left = h if isinstance(h, LeftNorm) else None
+        p = fast.gemm_pieces(h if left is None else left.h, w_qkv, ws, whole=dtype == torch.bfloat16, left=left)
         if p is not None:
             if p.splits > 1:
                 ws.counts_of(p)["qkv_pieces"] += 1

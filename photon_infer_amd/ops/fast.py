@@ -24,7 +24,7 @@ import torch
 
 from ..errors import KernelError
 from . import _lib
-from .workspace import GEMM_PART_FLOATS, KernelWorkspace, KeyRanges, Partials, PendingUpdate
+from .workspace import GEMM_PART_FLOATS, KernelWorkspace, KeyRanges, LeftNorm, Partials, PendingUpdate
 
 EPI_BF16, EPI_F32, EPI_ACCUM, EPI_SWIGLU = 0, 1, 2, 3
 SKINNY_MAX_ROWS = 128          # up to this many tokens the weight-streaming kernels serve a product (measured against the tile kernel)
@@ -36,6 +36,7 @@ SHARED_ROWS_PER_BLOCK = 64     # ... with this many weight rows per block, and n
                                # a unit would hold two: 64 tokens, k 4,096, blocks for half the units or more in one piece and in two, 8,256
                                # rows 29.7 and 32.0, 9,216 29.2 and 31.3, 12,160 29.4 and 31.1, 14,720 33.2 and 35.4; the same at 100 tokens
                                # (35.7 and 39.0, 35.4 and 38.0, 35.4 and 37.6, 39.1 and 41.7), and at k of 2,048 and 8,192
+FEW_TOKENS = 16                # up to this many tokens a product whose weights have a streaming copy may take all of k in a block (pi_gemm_rows)
 RING_MAX_STRIDE = 1 << 21      # elements between rows up to which that kernel's byte offsets fit 31 bits
 FLOAT32_ROWS = 32              # up to this many rows a float32 product goes to the weight-streaming kernel
 FLOAT32_MAX_STRIDE = 1 << 21   # floats between rows up to which the float32 kernels' offsets inside a tile fit 32 bits
@@ -150,10 +151,23 @@ def _streamed(ws: Optional[KernelWorkspace], w, N: int, K: int, ldw: int):
     return w.data_ptr(), 0
 
 
+def _rows(out_ptr: int, epilogue: int, ldc: int, a, w, M, N, K, lda, ldw, ws: Optional[KernelWorkspace], left: Optional[LeftNorm] = None) -> bool:
+    """A product of up to 16 tokens by the kernel whose blocks take all of k, which reads the weights' streaming copy: False, and
+    nothing done, without one.  ``left``: what ``a`` is the ``h`` of."""
+    w_ptr, tiled = _streamed(ws, w, N, K, ldw)
+    if not tiled or max(lda, K) >= RING_MAX_STRIDE:
+        return False
+    _lib.call("bf16", "pi_gemm_rows", out_ptr, epilogue, ldc, a.data_ptr(), lda, w_ptr, M, N, K, None if left is None else left.sums.data_ptr(),
+              0 if left is None else left.count, 0.0 if left is None else left.eps, _stream())
+    return True
+
+
 def _skinny(out_ptr: int, epilogue: int, ldc: int, a, w, M, N, K, lda, ldw, splits: int,
             ws: Optional[KernelWorkspace], pieces_ws: bool = True) -> Optional[Partials]:
     """Run the weight-streaming kernel; returns the pieces when the product was split.
     ``pieces_ws`` False: the workspace is only asked for the weights' streaming copy."""
+    if splits == 1 and M <= FEW_TOKENS and _rows(out_ptr, epilogue, ldc, a, w, M, N, K, lda, ldw, ws):
+        return None
     buf = _piece_buffer(ws if pieces_ws else None, splits * M * N, a.device) if splits > 1 else None
     made = ctypes.c_int(0)
     w_ptr, tiled = _streamed(ws, w, N, K, ldw)
@@ -183,7 +197,32 @@ def reduce_into(out: torch.Tensor, p: Partials, accumulate: bool) -> None:
               _stream())
 
 
-def gemm(out, a, w, accumulate, M, N, K, lda, ldw, ldc, may_defer=False, ws: Optional[KernelWorkspace] = None) -> bool:
+@functools.lru_cache(maxsize=4096)
+def _finish_blocks(M: int, N: int, K: int) -> int:
+    return _lib.load("bf16").pi_gemm_finish_blocks(M, N, K)
+
+
+def _finish(out, a, w, M, N, K, lda, ldw, next_norm, ws: KernelWorkspace) -> bool:
+    """out += a @ w^T of a few tokens by the kernel that also makes the next norm but for its root, left in the workspace;
+    False, and nothing done, where it does not take the product or the weights have no streaming copy."""
+    weight, eps = next_norm
+    blocks = _finish_blocks(M, N, K)
+    if not blocks or out.dtype != torch.float32 or not weight.is_contiguous() or weight.numel() != N or lda >= RING_MAX_STRIDE:
+        return False
+    w_ptr, tiled = _streamed(ws, w, N, K, ldw)
+    if not tiled:
+        return False
+    h = torch.empty((M, N), dtype=torch.bfloat16, device=out.device)
+    sums = torch.empty((M, blocks), dtype=torch.float32, device=out.device)
+    _lib.call("bf16", "pi_gemm_finish", out.data_ptr(), a.data_ptr(), lda, w_ptr, weight.data_ptr(), 0 if weight.dtype == torch.float32 else 1,
+              h.data_ptr(), sums.data_ptr(), sums.numel(), M, N, K, _stream())
+    ws.left_norm = LeftNorm(out, weight, eps, h, sums, blocks)
+    ws.counts["norms_left"] += 1
+    return True
+
+
+def gemm(out, a, w, accumulate, M, N, K, lda, ldw, ldc, may_defer=False, ws: Optional[KernelWorkspace] = None,
+         left: Optional[LeftNorm] = None, next_norm=None) -> bool:
     if not _gemm_ok(a, w, K, lda, ldw):
         return False
     if accumulate:
@@ -194,6 +233,8 @@ def gemm(out, a, w, accumulate, M, N, K, lda, ldw, ldc, may_defer=False, ws: Opt
         epilogue = EPI_F32
     else:
         return False
+    if left is not None:
+        return M <= FEW_TOKENS and _rows(out.data_ptr(), epilogue, ldc, a, w, M, N, K, lda, ldw, ws, left)
     may_defer = may_defer and ws is not None      # pieces can only wait in a workspace that outlives the call
     if M > SKINNY_MAX_ROWS:
         # few output tiles, long k: split k so that every compute unit has work; the pieces
@@ -206,7 +247,10 @@ def gemm(out, a, w, accumulate, M, N, K, lda, ldw, ldc, may_defer=False, ws: Opt
         _lib.call("bf16", "pi_gemm_mfma", out.data_ptr(), epilogue, ldc, a.data_ptr(), lda, w.data_ptr(), ldw, M, N, K, 1,
                   _tile_shape(M, N, K, 1), _stream())
         return True
-    pieces = _skinny(out.data_ptr(), epilogue, ldc, a, w, M, N, K, lda, ldw, _skinny_splits(M, N, K), ws)
+    splits = _skinny_splits(M, N, K)
+    if may_defer and accumulate and splits > 1 and next_norm is not None and _finish(out, a, w, M, N, K, lda, ldw, next_norm, ws):
+        return True
+    pieces = _skinny(out.data_ptr(), epilogue, ldc, a, w, M, N, K, lda, ldw, splits, ws)
     if pieces is not None:
         if may_defer:
             ws.pending = PendingUpdate(out, pieces, accumulate)          # the next norm of this stream adds them
@@ -363,9 +407,9 @@ def keeps_float32(M: int, N: int, K: int, units: int) -> bool:
     return M > SHARED_FROM_TOKENS and K >= 512 and -(-M // 128) * -(-N // 128) * 2048 <= units * max(K, 2048)
 
 
-def gemm_pieces(a, w, ws: Optional[KernelWorkspace], whole: bool = False) -> Optional[Partials]:
+def gemm_pieces(a, w, ws: Optional[KernelWorkspace], whole: bool = False, left: Optional[LeftNorm] = None) -> Optional[Partials]:
     """a @ w^T left in float32 pieces in the workspace, if this product is one whose k-range is split; with ``whole``
-    also a product in one piece (memory of its own) where ``keeps_float32`` says so."""
+    also a product in one piece (memory of its own) where ``keeps_float32`` says so.  ``left``: what ``a`` is the ``h`` of."""
     if ws is None:
         return None
     M, K = a.shape
@@ -374,6 +418,9 @@ def gemm_pieces(a, w, ws: Optional[KernelWorkspace], whole: bool = False) -> Opt
     if not _gemm_ok(a, w, K, lda, ldw) or a.stride(1) != 1 or w.stride(1) != 1:
         return None
     p = None
+    if left is not None:            # few tokens: one float32 piece, of memory of its own
+        out = torch.empty((1, M, N), dtype=torch.float32, device=a.device)
+        return Partials(out, 1, M, N) if M <= FEW_TOKENS and _rows(out.data_ptr(), EPI_F32, N, a, w, M, N, K, lda, ldw, ws, left) else None
     if M > SKINNY_MAX_ROWS:
         # a prompt portion of a few hundred tokens has too few tiles for the chip: split k there
         # too, the consumer adds the pieces
@@ -407,10 +454,12 @@ def gemm_activation(out, a, w, activation, M, N, K, lda, ldw) -> bool:
     return True
 
 
-def gemm_swiglu(out, a, w, M, N, K, lda, ldw, ws: Optional[KernelWorkspace] = None) -> bool:
+def gemm_swiglu(out, a, w, M, N, K, lda, ldw, ws: Optional[KernelWorkspace] = None, left: Optional[LeftNorm] = None) -> bool:
     """``w`` [N = 2I, K] with gate / up rows interleaved in blocks of 16; out [M, I] bfloat16."""
     if not _gemm_ok(a, w, K, lda, ldw) or N % 32 or out.dtype != torch.bfloat16:
         return False
+    if left is not None:
+        return M <= FEW_TOKENS and _rows(out.data_ptr(), EPI_SWIGLU, out.stride(0), a, w, M, N, K, lda, ldw, ws, left)
     if M > SKINNY_MAX_ROWS:
         _lib.call("bf16", "pi_gemm_mfma", out.data_ptr(), EPI_SWIGLU, out.stride(0), a.data_ptr(), lda, w.data_ptr(), ldw,
                   M, N, K, 1, _tile_shape(M, N, K, 1), _stream())

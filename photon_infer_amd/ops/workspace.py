@@ -65,6 +65,36 @@ class PendingUpdate:
         return t is x or (t.data_ptr() == x.data_ptr() and t.shape == x.shape and t.stride() == x.stride())
 
 
+@dataclass
+class LeftNorm:
+    """The norm of a stream ``x`` [M, D] that the product before it made but for the root (``ops.gemm`` with ``next_norm``):
+    ``h`` holds bfloat16(x * weight), ``sums`` float32 [M, count] every row's sum of x^2 in pieces.  A product that takes it
+    as activations multiplies its float32 rows by 1 / sqrt(sum / D + eps).  Good until ``x`` changes or is freed."""
+
+    x: torch.Tensor
+    weight: torch.Tensor
+    eps: float
+    h: torch.Tensor
+    sums: torch.Tensor
+    count: int
+
+    @property
+    def shape(self):
+        return self.h.shape
+
+    @property
+    def device(self):
+        return self.h.device
+
+    @property
+    def dtype(self):
+        return self.h.dtype
+
+    @property
+    def is_cuda(self):
+        return self.h.is_cuda
+
+
 def stream_layout_takes(w: torch.Tensor) -> bool:
     """Whether ``stream_layout`` has a form for ``w``."""
     return (w.dim() == 2 and w.dtype == torch.bfloat16 and w.is_contiguous() and w.shape[0] > 0 and w.shape[0] % 16 == 0
@@ -86,7 +116,7 @@ def stream_layout(w: torch.Tensor) -> Optional[torch.Tensor]:
 class KernelWorkspace:
     """Buffers are made at first use and kept; ``counts`` says which paths a step took (tests
     read it: ``split_products``, ``deferred``, ``added_by_norm``, ``applied``, ``flushed``,
-    ``discarded``, ``qkv_pieces``, ``ranges_merged_by_product``).  ``counts`` is about the 16-bit
+    ``discarded``, ``qkv_pieces``, ``ranges_merged_by_product``, ``norms_left``).  ``counts`` is about the 16-bit
     products; ``float32_counts`` has the same entries for pieces of float32 products."""
 
     def __init__(self, device):
@@ -96,6 +126,7 @@ class KernelWorkspace:
         self._tile_part: Optional[torch.Tensor] = None
         self._sample_part: Optional[torch.Tensor] = None
         self.pending: Optional[PendingUpdate] = None
+        self.left_norm: Optional[LeftNorm] = None      # what a product has made of the stream's next norm
         self.counts: Counter = Counter()
         self.float32_counts: Counter = Counter()
         # weight matrices that have a second copy in the order the weight-streaming kernels read
@@ -159,6 +190,11 @@ class KernelWorkspace:
         if entry is None or entry[1] != N or entry[2] != K:
             return None
         return entry[0]
+
+    def take_left_norm(self, x: torch.Tensor, weight: torch.Tensor, eps: float) -> Optional[LeftNorm]:
+        """What is left of the norm of ``x`` with these parameters, if a product has made it."""
+        left, self.left_norm = self.left_norm, None
+        return left if left is not None and left.x is x and left.weight is weight and left.eps == eps else None
 
     def take_pending(self, x: torch.Tensor) -> Optional[Partials]:
         """The pieces still to be added to ``x``, if any; they are the caller's to add."""

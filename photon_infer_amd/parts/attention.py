@@ -137,6 +137,11 @@ class PagedAttention(Mixer):
         return KVCacheSpec(self.num_kv_heads, self.head_dim, self.window)
 
     @property
+    def takes_left_norm(self) -> bool:
+        # the activations are read by the q|k|v projection only
+        return not self.values_are_keys
+
+    @property
     def graph_safe(self) -> bool:
         # the kernels take the step's shape from device memory; a position encoding applied by
         # library calls must make the promise itself

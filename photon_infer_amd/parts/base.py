@@ -121,6 +121,10 @@ class StepContext:
     # the stream in pieces (``ops.gemm(..., may_defer=True)``) because the stream's next reader
     # adds them.  False unless an arrangement says so, so a part never defers by itself.
     may_defer: bool = False
+    # Set beside ``may_defer``, or None: (weight, eps) of the norm that reads the stream next, when that norm's own reader takes
+    # a norm whose root is left to it (``ops.gemm(..., next_norm=...)``).
+    next_norm: Any = None
+    after_block_norm: Any = None          # set by the model per block: the same for whoever reads the stream after this block
     may_leave_choices: bool = False       # likewise: a routed feed-forward may leave its result as the experts' rows (``ops.LeftChoices``)
     after_block_consumes: bool = False    # set by the model per block: whoever reads the stream after this block adds pending pieces
     workspace: Any = None                 # the runner's ops.KernelWorkspace: scratch memory of the kernels
@@ -172,6 +176,8 @@ class Part:
 
 
 class Norm(Part):
+    leaves_root = False        # True: ``forward`` returns an ``ops.LeftNorm`` where the product before it has left one
+
     def forward(self, x: torch.Tensor, ctx: Optional[StepContext] = None, rows: Optional[torch.Tensor] = None) -> torch.Tensor:
         """``x`` float32 [N, D] -> normalised rows in the compute dtype ([M, D] when
         ``rows`` (int32 [M]) selects rows of ``x``).  ``ctx`` is the step's context (None
@@ -194,6 +200,8 @@ class PositionEncoding(Part):
 
 
 class Mixer(Part):
+    takes_left_norm = False    # True: ``forward`` takes an ``ops.LeftNorm`` for its activations (its products of them do)
+
     def cache_spec(self):
         """What the mixer keeps per request: ``KVCacheSpec`` / ``PagedCacheSpec`` (per token, in
         pages), ``StateSpec`` (fixed size), or None."""
@@ -214,6 +222,8 @@ class Mixer(Part):
 
 
 class FeedForward(Part):
+    takes_left_norm = False    # as a mixer's
+
     def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext) -> None:
         """Read activations ``h`` [T, D]; add the result into ``x`` (float32)."""
         raise NotImplementedError
@@ -230,6 +240,11 @@ class Block(Part):
     mixer: Mixer
     takes_left_join = False    # True: the block's first reader applies a result that a sandwich block has left (``norm.LEFT_JOIN``)
     reads_deferred = False     # True: the block's first reader of the stream is a norm that adds pending pieces
+
+    @property
+    def first_norm(self):
+        """(weight, eps) of the norm that reads the stream first, when its root may be left to the norm's reader; else None."""
+        return None
 
     def mixers(self) -> List[Mixer]:
         """The block's mixers - and other parts of it that keep something per request (they have a mixer's

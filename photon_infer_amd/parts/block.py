@@ -14,7 +14,7 @@ from .. import ops
 from ..errors import UnsupportedModelError
 from ..weights.loader import TensorSpec
 from .base import BLOCKS, MIXERS, Block, FeedForward, LayerCache, Mixer, Norm, Part, StepContext
-from .norm import LEFT_JOIN, LEFT_UPDATE, LeftJoin
+from .norm import LEFT_JOIN, LEFT_UPDATE, LeftJoin, norm_left_to
 from .token_shift import TokenShift
 
 
@@ -101,20 +101,25 @@ class PreNormBlock(Block):
     def reads_deferred(self) -> bool:
         return bool(getattr(self.norm1, "consumes_deferred", False))
 
+    @property
+    def first_norm(self):
+        return norm_left_to(self.norm1, self.mixer)
+
     def forward(self, x: torch.Tensor, ctx: StepContext, cache: LayerCache) -> None:
         # A mixer or feed-forward may leave its update of x in pieces (ops.gemm(..., may_defer=True))
         # when the stream's next reader adds them: norm2 after the mixer; after the feed-forward,
-        # whoever the model says reads the stream next.
+        # whoever the model says reads the stream next.  Where that reader's norm may be made by the
+        # update itself, ctx.next_norm names it.
         if self.ffn is None:
-            ctx.may_defer = ctx.after_block_consumes
+            ctx.may_defer, ctx.next_norm = ctx.after_block_consumes, ctx.after_block_norm
             self.mixer.forward(self.norm1.forward(x, ctx), x, ctx, cache)
-            ctx.may_defer = False
+            ctx.may_defer, ctx.next_norm = False, None
             return
-        ctx.may_defer = bool(getattr(self.norm2, "consumes_deferred", False))
+        ctx.may_defer, ctx.next_norm = bool(getattr(self.norm2, "consumes_deferred", False)), norm_left_to(self.norm2, self.ffn)
         self.mixer.forward(self.norm1.forward(x, ctx), x, ctx, cache)
-        ctx.may_defer = ctx.after_block_consumes
+        ctx.may_defer, ctx.next_norm = ctx.after_block_consumes, ctx.after_block_norm
         self.ffn.forward(self.norm2.forward(x, ctx), x, ctx)
-        ctx.may_defer = False
+        ctx.may_defer, ctx.next_norm = False, None
 
 
 BLOCKS.register("prenorm", PreNormBlock)

@@ -21,6 +21,7 @@ INTERLEAVE = 16   # rows of a matrix-core tile
 
 class SwiGLU(FeedForward):
     graph_safe = True
+    takes_left_norm = True
 
     def __init__(self, hidden_size: int, intermediate_size: int, activation: str = "silu",
                  names=("gate_proj.weight", "up_proj.weight", "down_proj.weight"), accumulate: bool = True):
@@ -67,7 +68,8 @@ class SwiGLU(FeedForward):
         act = torch.empty((h.shape[0], self.intermediate_size), dtype=self.dtype, device=h.device)
         ws = ctx.workspace if ctx is not None else None
         ops.gemm_swiglu(act, h, self.w_gate_up, self.interleave, ws=ws)
-        ops.gemm(x, act, self.w_down, accumulate=self.accumulate, may_defer=getattr(ctx, "may_defer", False), ws=ws)
+        ops.gemm(x, act, self.w_down, accumulate=self.accumulate, may_defer=getattr(ctx, "may_defer", False), ws=ws,
+                 next_norm=getattr(ctx, "next_norm", None))
 
 
 FEED_FORWARDS.register("swiglu", SwiGLU)

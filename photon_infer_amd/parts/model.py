@@ -164,9 +164,11 @@ class DecoderModel:
                 ops.materialize(x, ws)
             if i + 1 < len(order):
                 ctx.after_block_consumes = bool(self.blocks[order[i + 1].layer].reads_deferred)
+                ctx.after_block_norm = getattr(self.blocks[order[i + 1].layer], "first_norm", None)
             else:                          # the final norm; or nobody (the pieces are then dropped unread)
                 ctx.after_block_consumes = not wanted or bool(getattr(self.final_norm, "consumes_deferred", False))
-            ctx.may_defer = False
+                ctx.after_block_norm = None
+            ctx.may_defer, ctx.next_norm = False, None
             block.forward(x, ctx, caches[i])
         ctx.may_defer = ctx.may_leave_choices = ctx.after_block_consumes = False
         if not wanted:

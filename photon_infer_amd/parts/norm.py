@@ -14,7 +14,7 @@ import torch
 
 from .. import ops
 from ..weights.loader import TensorSpec
-from .base import NORMS, Norm
+from .base import NORMS, Norm, Part
 
 
 # Key in a step's ``scratch``: (streams, a sublayer's result, the numbers it joins them by) - an update of streams that run
@@ -52,9 +52,17 @@ def settle_left_join(x: torch.Tensor, ctx) -> None:
         left.apply(ctx.workspace)
 
 
+def norm_left_to(norm: Norm, reader: Part):
+    """(weight, eps) of ``norm`` when the product before it may make it but for the root, which ``reader`` applies; else None."""
+    if getattr(norm, "leaves_root", False) and norm.dtype == torch.bfloat16 and getattr(reader, "takes_left_norm", False):
+        return norm.weight, norm.eps
+    return None
+
+
 class RMSNorm(Norm):
     consumes_deferred = True   # reads the stream through ops.rmsnorm, which adds a pending update
     takes_left_join = True     # and a result that a sandwich block has left
+    leaves_root = True
     graph_safe = True
 
     def __init__(self, dim: int, eps: float, offset: float = 0.0, tensor_name: str = "weight", mult: float = 1.0):
@@ -87,6 +95,11 @@ class RMSNorm(Norm):
         left = take_left_join(x, ctx)
         if left is not None:
             return left.apply(ctx.workspace, self.weight_f32(), self.eps, self.dtype, rows)
+        if rows is None and ctx is not None and ctx.workspace is not None:
+            # only there when this norm's reader has said that it takes it (norm_left_to)
+            left = ctx.workspace.take_left_norm(x, self.weight, self.eps)
+            if left is not None:
+                return left
         m = x.shape[0] if rows is None else rows.shape[0]
         out = torch.empty((m, self.dim), dtype=self.dtype, device=x.device)
         ops.rmsnorm(out, x, self.weight, self.eps, rows, ws=ctx.workspace if ctx is not None else None)
@@ -101,7 +114,7 @@ class StreamSumRMSNorm(RMSNorm):
     norm's own pass.  An update that a block of such streams has left to the next reader (``HyperConnectionBlock``) is
     applied on the way."""
 
-    consumes_deferred = takes_left_join = False
+    consumes_deferred = takes_left_join = leaves_root = False
 
     def __init__(self, dim: int, eps: float, streams: int, offset: float = 0.0, tensor_name: str = "weight"):
         super().__init__(dim, eps, offset, tensor_name)

@@ -5,7 +5,7 @@
 //
 // Walks the built-in sweep of shapes (and any given as arguments) through the lanes, waves,
 // blocks and steps of gemm_skinny_kernel, gemm_skinny_ring_kernel, gemm_mfma_kernel,
-// gemm_mfma_big_kernel in its six tile shapes, gemm_float32_rows_kernel and gemm_float32_tile_kernel exactly as the kernels
+// gemm_mfma_big_kernel in its six tile shapes, gemm_rows_kernel, gemm_float32_rows_kernel and gemm_float32_tile_kernel exactly as the kernels
 // walk them (and, in the built-in sweep, through the
 // key and value fetches of the attention kernels' chunks for every head size and several page sizes), with the matrices row by row (several row
 // strides) and, where the sizes allow, in the weight-streaming kernels' tiled order.  Prints
@@ -231,6 +231,39 @@ static bool ring(const Shape& s, long ldx, long ldw, int tiled) {
   return true;
 }
 
+// ------------------------------------------------------------------ 1..16 tokens, all of k in a block
+// Every fetch of gemm_rows_kernel with 8 or 16 rows a tile, four or eight waves: the weights' copy and the activations
+// through descriptors of a wave's own k.  A used fetch is the lane's row (token) and k; any other lies outside its descriptor.
+static bool few_rows(const Shape& s, long lda) {
+  for (int rows : {8, 16})
+    for (int waves : {4, 8})
+      for (int wide = rows == 16 || s.M > 8; wide < 2; ++wide)
+        for (long n0 = 0; n0 < s.N; n0 += rows)
+          for (int wave = 0; wave < waves; ++wave) {
+            const A::WaveRange r = A::wave_share(0, s.K, waves, wave);
+            const int steps = r.k1 > r.k0 ? (r.k1 - r.k0) / 64 : 0;
+            const A::Descriptor dw = A::rows_w_descriptor(n0, r.k0, steps, s.K), da = A::rows_a_descriptor(r.k0, steps, s.M, lda);
+            if (steps > 0 && (dw.base < 0 || dw.base * 2 + dw.bytes > (long)s.N * s.K * 2)) return fail("gemm_rows", "W", s, s.K, 1, dw.base, "the descriptor leaves the operand");
+            if (steps > 0 && (da.base < 0 || da.base * 2 + da.bytes > ((s.M - 1) * lda + s.K) * 2)) return fail("gemm_rows", "A", s, lda, 0, da.base, "the descriptor leaves the operand");
+            for (int lane = 0; lane < 64; ++lane)
+              for (int st = 0; st < steps + 16; ++st)
+                for (int f = 0; f < 2; ++f) {
+                  ++fetches;
+                  const long w = A::rows_step(A::rows_w_lane(rows, n0, lane), st, steps, 2048, rows == 16 ? f * 1024 : 0);
+                  const long a = A::rows_step(A::rows_a_lane(wide, lane, s.M, lda), st, steps, 128, wide ? f * 16 : 0);
+                  const int wf = rows == 16 ? f : lane % 16 / 8, af = wide ? f : lane % 16 / 8;
+                  const long n = n0 + (rows == 16 ? lane % 16 : lane % 8), token = wide ? lane % 16 : lane % 8;
+                  if (st >= steps ? w < dw.bytes : w + 16 > dw.bytes) return fail("gemm_rows", "W", s, s.K, 1, w, "on the wrong side of its descriptor");
+                  if (st >= steps || token >= s.M ? a < da.bytes : a + 16 > da.bytes) return fail("gemm_rows", "A", s, lda, 0, a, "on the wrong side of its descriptor");
+                  const long k = r.k0 + st * 64 + lane / 16 * 16;
+                  if (st < steps && dw.base * 2 + w != (n / 16 * (s.K / 64) + k / 64) * 2048 + wf * 1024 + lane / 16 * 256 + n % 16 * 16)
+                    return fail("gemm_rows", "W", s, s.K, 1, w, "a used fetch is not the lane's row and k");
+                  if (st < steps && token < s.M && da.base * 2 + a != (token * lda + k + af * 8) * 2) return fail("gemm_rows", "A", s, lda, 0, a, "a used fetch is not the lane's token and k");
+                }
+          }
+  return true;
+}
+
 // ------------------------------------------------------------------ attention over the paged cache
 // Every fetch of a chunk's two tiles (attn_load): the keys' fragments (16 bytes) and the values'
 // (8 bytes) of every lane, for a page that is there, one that is missing and one whose id is no
@@ -307,6 +340,7 @@ static bool check(const Shape& s) {
     if (s.M <= 32 && !skinny(s, s.K, s.K, 1, 2, A::KSTEP)) return false;
     if (s.M <= 16 && !skinny(s, s.K, s.K, 1, 4, 4 * A::KSTEP)) return false;
     if (s.M > 32 && s.M <= 128 && !ring(s, s.K, s.K, 1)) return false;
+    if (s.M <= 16 && s.N % 64 == 0 && s.N < 2048 && (!few_rows(s, s.K) || !few_rows(s, s.K + 8))) return false;
   }
   return true;
 }

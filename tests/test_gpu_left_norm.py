@@ -1,0 +1,170 @@
+"""Products of a few tokens that finish the residual stream and leave its norm's root to the reader.
+
+``ops.gemm(..., next_norm=...)`` against float64: the stream, what is left of the norm, and the products that take it,
+at the edges of the kernel's sizes: one token to sixteen (one matrix instruction to 8, two beyond), blocks of 8 and of 16
+weight rows, k shares that are empty, partial and of more steps than are in flight, bfloat16 and float32 norm weights.
+"""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV, F32, BF16 = "cuda", torch.float32, torch.bfloat16
+# bfloat16 has 8 significant bits: one rounding to it is off by 2^-8 of the value at most (half of the last place of a value
+# just above a power of two); float32 sums of some thousand terms add some 1e-6 of the terms' sum, which is left out
+ROUND = 2.0 ** -8
+
+
+def gen(seed):
+    return torch.Generator(device=DEV).manual_seed(seed)
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from photon_infer_amd import ops as o
+    o.ensure_loaded(BF16)
+    return o
+
+
+def made(ops, M, N, K, w_dtype=BF16, eps=1e-5, pad=0):
+    g = gen(M * 7 + N + K)
+    a = (torch.randn(M, K + pad, generator=g, device=DEV)).to(BF16)[:, :K]
+    w = (torch.randn(N, K, generator=g, device=DEV) * K ** -0.5).to(BF16)
+    x0 = torch.randn(M, N, generator=g, device=DEV)
+    weight = (torch.rand(N, generator=g, device=DEV) + 0.5).to(w_dtype)
+    ws = ops.KernelWorkspace(DEV)
+    assert ws.add_stream_copy(w)
+    x = x0.clone()
+    ops.gemm(x, a, w, accumulate=True, may_defer=True, ws=ws, next_norm=(weight, eps))
+    return ws, x, x0.double() + a.double() @ w.double().t(), weight
+
+
+@pytest.mark.parametrize("M", [1, 7, 8, 9, 16])
+@pytest.mark.parametrize("N,K,w_dtype", [(64, 512, BF16), (64, 1088, F32), (192, 3136, BF16), (2048, 2048, BF16), (2048, 4160, F32),
+                                         (3072, 576, BF16), (3136, 4544, F32), (4096, 2112, BF16)])
+def test_finished_stream_and_left_norm_against_float64(ops, M, N, K, w_dtype):
+    from photon_infer_amd.ops import fast
+    if not fast._finish_blocks(M, N, K) or fast._skinny_splits(M, N, K) < 2:
+        pytest.skip("a size that the pieces keep")
+    ws, x, want, weight = made(ops, M, N, K, w_dtype, pad=8)
+    assert ws.counts["norms_left"] == 1 and ws.pending is None
+    left = ws.take_left_norm(x, weight, 1e-5)
+    assert isinstance(left, ops.LeftNorm) and ws.left_norm is None
+    assert ((x.double() - want).abs() <= 2e-6 * (want.abs() + 1.0) * max(1.0, (K / 64) ** 0.5)).all()
+    assert torch.equal(left.h, (x * weight.float()).to(BF16))
+    sums = (x.double() ** 2).sum(1)
+    assert (left.sums.double().sum(1) - sums).abs().max() <= 1e-5 * sums.max()
+    # its readers: a product in pieces of k and whole, float32 and bfloat16, and the gated unit
+    norm = (x.double() / torch.sqrt(sums[:, None] / N + 1e-5)) * weight.double()
+    g = gen(5)
+    for rows, k_pieces in ((96, True), (16384 if N <= 2048 else 1024, False)):
+        w2 = (torch.randn(rows, N, generator=g, device=DEV) * N ** -0.5).to(BF16)
+        want2 = norm @ w2.double().t()
+        size = (norm.abs() @ w2.double().abs().t())               # what the rounding of the activations may sum up to
+        got = ops.qkv_projection(left, w2, F32, ws)
+        if isinstance(got, ops.Partials):
+            got = got.part.view(-1)[:got.splits * M * rows].view(got.splits, M, rows).sum(0)
+        assert ((got.double() - want2).abs() <= ROUND * size).all()
+        out = torch.empty(M, rows, dtype=BF16, device=DEV)
+        ops.gemm(out, left, w2, ws=ws)
+        assert ((out.double() - want2).abs() <= ROUND * (size + want2.abs())).all()
+        if rows % 32 == 0:
+            unit = torch.empty(M, rows // 2, dtype=BF16, device=DEV)
+            ops.gemm_swiglu(unit, left, w2, 16, ws=ws)
+            z = want2.view(M, rows // 32, 2, 16)
+            s = size.view(M, rows // 32, 2, 16)
+            wanted = (torch.nn.functional.silu(z[:, :, 0]) * z[:, :, 1]).reshape(M, -1)
+            slack = (1.1 * s[:, :, 0] * z[:, :, 1].abs() + s[:, :, 1] * z[:, :, 0].abs()).reshape(M, -1)
+            assert ((unit.double() - wanted).abs() <= ROUND * (1.1 * slack + wanted.abs() + 1e-3)).all()
+
+
+def test_rows_that_are_not_finite_stay_by_themselves_and_zero_rows_keep_their_eps(ops):
+    M, N, K = 8, 256, 512
+    g = gen(3)
+    a = torch.randn(M, K, generator=g, device=DEV).to(BF16)
+    a[2, 5], a[6, 100] = float("inf"), float("nan")
+    a[4] = 0
+    w = (torch.randn(N, K, generator=g, device=DEV) * 0.05).to(BF16)
+    weight = torch.ones(N, dtype=BF16, device=DEV)
+    ws = ops.KernelWorkspace(DEV)
+    ws.add_stream_copy(w)
+    x = torch.zeros(M, N, device=DEV)
+    ops.gemm(x, a, w, accumulate=True, may_defer=True, ws=ws, next_norm=(weight, 1e-5))
+    left = ws.take_left_norm(x, weight, 1e-5)
+    out = torch.empty(M, 64, dtype=F32, device=DEV)
+    ops.gemm(out, left, (torch.randn(64, N, generator=g, device=DEV) * 0.05).to(BF16), ws=ws)
+    good = [0, 1, 3, 4, 5, 7]
+    assert torch.isfinite(x[good]).all() and torch.isfinite(out[good]).all() and (out[4] == 0).all()
+    assert not torch.isfinite(x[2]).any() and torch.isnan(x[6]).all() and torch.isnan(out[2]).all() and torch.isnan(out[6]).all()
+
+
+def test_whoever_else_reads_or_changes_the_stream_finds_it_finished(ops):
+    """Another norm, another update of the stream and a reader that takes no left norm."""
+    ws, x, want, weight = made(ops, 3, 256, 512)
+    other = torch.ones(256, dtype=BF16, device=DEV)
+    assert ws.take_left_norm(x, other, 1e-5) is None and ws.left_norm is None          # another norm's: dropped, not handed on
+    ws, x, want, weight = made(ops, 3, 256, 512)
+    a, w = torch.ones(3, 64, dtype=BF16, device=DEV), torch.ones(256, 64, dtype=BF16, device=DEV)
+    ops.gemm(x, a, w, accumulate=True, ws=ws)
+    assert ws.left_norm is None and (x.double() - want - 64).abs().max() < 1e-4
+    ws, x, want, weight = made(ops, 3, 256, 512)
+    left = ws.take_left_norm(x, weight, 1e-5)
+    whole = torch.empty(3, 256, dtype=BF16, device=DEV)
+    ops.rmsnorm(whole, x, weight, 1e-5)
+    assert torch.equal(ops.whole_norm(left), whole)
+    wide = torch.randn(40, 256, generator=gen(1), device=DEV)                          # float32 weights: no product here takes it
+    got, same = torch.empty(3, 40, device=DEV), torch.empty(3, 40, device=DEV)
+    ops.gemm(got, left, wide, ws=ws)
+    ops.gemm(same, whole, wide, ws=ws)
+    assert torch.equal(got, same)
+    # without a streaming copy, or without the caller's word that the norm is next, the update stays in pieces
+    for copies, norm in ((False, True), (True, False)):
+        ws = ops.KernelWorkspace(DEV)
+        w = torch.ones(2048, 512, dtype=BF16, device=DEV)
+        if copies:
+            ws.add_stream_copy(w)
+        x = torch.zeros(2, 2048, device=DEV)
+        ops.gemm(x, torch.ones(2, 512, dtype=BF16, device=DEV), w, accumulate=True, may_defer=True, ws=ws,
+                 next_norm=(torch.ones(2048, device=DEV), 1e-5) if norm else None)
+        assert ws.left_norm is None and ws.pending is not None and ws.counts["norms_left"] == 0
+
+
+@pytest.mark.parametrize("batch", [1, 5, 12])
+def test_a_models_decode_steps_leave_their_norms(tmp_path, batch):
+    """A model whose matrices have streaming copies: decode steps leave the norms of whole layers to the next projection,
+    with and without graphs, to the same tokens, and their logits are those of the steps that make every norm."""
+    from photon_infer_amd import EngineOptions, ModelRunner, StepEntry
+    from photon_infer_amd.config import LlamaConfig
+    from photon_infer_amd.parts import PreNormBlock
+
+    cfg = LlamaConfig.from_dict(dict(architectures=["LlamaForCausalLM"], hidden_size=512, intermediate_size=1024, num_attention_heads=8,
+                                     num_key_value_heads=2, head_dim=64, num_hidden_layers=3, vocab_size=1024, max_position_embeddings=512,
+                                     rms_norm_eps=1e-5, rope_theta=10000.0, tie_word_embeddings=True))
+    from photon_infer_amd.registry import build_model_spec
+    g = gen(9)
+    tensors = {s.name: (torch.rand(s.shape, generator=g, device=DEV) + 0.5 if s.role == "norm" else torch.randn(s.shape, generator=g, device=DEV) * 0.04).to(BF16)
+               for s in build_model_spec(cfg).tensor_specs()}
+
+    def run(graphs, leave):
+        runner = ModelRunner(None, EngineOptions(max_batch=batch, max_cache_tokens=batch * 64, max_model_len=128, use_graphs=graphs, keep_logits=True),
+                             config=cfg, tensors=dict(tensors))
+        if not leave:
+            for b in runner.model.blocks:
+                b.norm1.leaves_root = b.norm2.leaves_root = False
+        for i in range(batch):
+            runner.admit(i)
+            runner.step([StepEntry(i, list(range(3 + i, 12 + 2 * i)))])
+        rows = []
+        for t in range(4):
+            runner.decode_step([StepEntry(i, [17 * t + i], [0]) for i in range(batch)], [0.0] * batch, [0.0] * batch)
+            rows.append(runner.decode_logits.clone())
+        return torch.stack(rows).double(), runner.workspace.counts
+
+    assert PreNormBlock is not None
+    eager, counts = run(False, True)
+    assert counts["norms_left"] > 0, counts
+    graphed, _ = run(True, True)
+    assert torch.equal(eager, graphed)
+    whole, counts = run(False, False)
+    assert counts["norms_left"] == 0
+    # three layers of bfloat16 activations: their roundings, not their sizes, differ
+    assert (eager - whole).norm() <= 0.02 * whole.norm()
