@@ -415,7 +415,8 @@ static int launch_decode(bool fused, const DecodeSource& src, void* out, long ou
   PI_REQUIRE(out_stride % 4 == 0 && ((uintptr_t)out % 8 == 0), "attention_decode: out rows must be 8-byte aligned");
   if (!fused)
     PI_REQUIRE(q_stride % 8 == 0 && ((uintptr_t)q % 16 == 0), "attention_decode: q rows must be 16-byte aligned");
-  PI_REQUIRE(waves == 1 || ((waves == 2 || waves == 4) && splits == 1), "attention_decode: %d waves per block over %d ranges", waves, splits);
+  PI_REQUIRE(waves == 1 || waves == 2 || waves == 4, "attention_decode: %d waves per block", waves);
+  PI_REQUIRE(!uneven || splits == 1, "attention_decode: waves that may leave go with one range, got %d", splits);
   if (splits > 1)
     PI_REQUIRE(part && part_elems >= (long)R * nh * splits * (hd + 4), "attention_decode: workspace too small for %d ranges", splits);
   const dim3 grid(splits, nkv, R), block(64 * waves);

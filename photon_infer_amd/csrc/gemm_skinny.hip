@@ -47,17 +47,15 @@ struct RangeSource {
   int heads, head_dim, count;
 };
 
-// Lane group lg merges the key ranges of tokens lg, lg + 4, .. (TOK of them per round) for the
-// lane's four features of one head and leaves them, rounded to bfloat16, where the product's
-// operand reads expect them.  CNT > 0: up to CNT ranges, all loads of a round asked for before
+// Merges the key ranges of tokens first, first + stride, .. (TOK of them per round) for four features of one head, rounds
+// them to bfloat16 and hands them to store(token, packed).  CNT > 0: up to CNT ranges, all loads of a round asked for before
 // the first is used (one trip to memory); CNT == 0: any number, in two passes.  Ranges are added
 // in range order with the shared arithmetic (range_weight / range_add / range_finish).
-template <int CNT, int TOK>
+template <int CNT, int TOK, typename Store>
 __device__ inline void merge_ranges_of_tokens(const float* __restrict__ head_base, long token_stride, int count, int rec, int hd,
-                                              int f0, int lg, int lr, int M, uint2* __restrict__ xs2) {
-  const int piece = lr / 2;                              // the 16-byte piece of the k step the lane's features lie in
+                                              int f0, int first, int stride, int M, Store store) {
 #pragma unroll 1
-  for (int t0 = lg; t0 < M; t0 += 4 * TOK) {
+  for (int t0 = first; t0 < M; t0 += stride * TOK) {
     f32x4_t sum[TOK];
     float l_tot[TOK];
     if constexpr (CNT > 0) {
@@ -65,7 +63,7 @@ __device__ inline void merge_ranges_of_tokens(const float* __restrict__ head_bas
       f32x4_t o[TOK][CNT];
 #pragma unroll
       for (int j = 0; j < TOK; ++j) {
-        const float* base = head_base + (long)min(t0 + 4 * j, M - 1) * token_stride;
+        const float* base = head_base + (long)min(t0 + stride * j, M - 1) * token_stride;
 #pragma unroll
         for (int u = 0; u < CNT; ++u) {
           const int r = min(u, count - 1);
@@ -108,14 +106,24 @@ __device__ inline void merge_ranges_of_tokens(const float* __restrict__ head_bas
     }
 #pragma unroll
     for (int j = 0; j < TOK; ++j) {
-      const int token = t0 + 4 * j;
+      const int token = t0 + stride * j;
       if (token >= M) break;
       uint2 packed;
       packed.x = pack_bf16x2(range_finish(sum[j][0], l_tot[j]), range_finish(sum[j][1], l_tot[j]));
       packed.y = pack_bf16x2(range_finish(sum[j][2], l_tot[j]), range_finish(sum[j][3], l_tot[j]));
-      xs2[(piece * 16 + ((token + 2 * piece) & 15)) * 2 + (lr & 1)] = packed;
+      store(token, packed);
     }
   }
+}
+
+// tokens per round x ranges per token held in registers at once: about IN_FLIGHT either way
+template <int IN_FLIGHT, typename Store>
+__device__ inline void merge_ranges(const float* __restrict__ head_base, long token_stride, int count, int rec, int hd, int f0, int first,
+                                    int stride, int M, Store store) {
+  if (count <= 4) merge_ranges_of_tokens<4, IN_FLIGHT / 4>(head_base, token_stride, count, rec, hd, f0, first, stride, M, store);
+  else if (count <= 8) merge_ranges_of_tokens<8, IN_FLIGHT / 8>(head_base, token_stride, count, rec, hd, f0, first, stride, M, store);
+  else if (count <= 16) merge_ranges_of_tokens<16, IN_FLIGHT / 16>(head_base, token_stride, count, rec, hd, f0, first, stride, M, store);
+  else merge_ranges_of_tokens<0, 1>(head_base, token_stride, count, rec, hd, f0, first, stride, M, store);
 }
 
 // Activations of a norm whose root was left to this reader (gemm_rows_kernel made them): row m holds x * w, and the
@@ -230,11 +238,10 @@ __global__ __launch_bounds__(256) void gemm_skinny_kernel(void* __restrict__ Cv,
       const float* head_base = rs.ranges + (long)head * rs.count * rec;
       const long token_stride = (long)rs.heads * rs.count * rec;
       uint2* xs2 = reinterpret_cast<uint2*>(xs);
-      // tokens per lane group x ranges per token held in registers at once: about 16 either way
-      if (rs.count <= 4) merge_ranges_of_tokens<4, 4>(head_base, token_stride, rs.count, rec, rs.head_dim, f0, lg, lr, M, xs2);
-      else if (rs.count <= 8) merge_ranges_of_tokens<8, 2>(head_base, token_stride, rs.count, rec, rs.head_dim, f0, lg, lr, M, xs2);
-      else if (rs.count <= 16) merge_ranges_of_tokens<16, 1>(head_base, token_stride, rs.count, rec, rs.head_dim, f0, lg, lr, M, xs2);
-      else merge_ranges_of_tokens<0, 1>(head_base, token_stride, rs.count, rec, rs.head_dim, f0, lg, lr, M, xs2);
+      const int piece = lr / 2;                            // the 16-byte piece of the k step the lane's features lie in
+      merge_ranges<16>(head_base, token_stride, rs.count, rec, rs.head_dim, f0, lg, 4, M, [&](const int token, const uint2 packed) {
+        xs2[(piece * 16 + ((token + 2 * piece) & 15)) * 2 + (lr & 1)] = packed;
+      });
     } else {
       const bool x_ok = whole || kk + xp * 8 < k1;
 #pragma unroll
@@ -479,9 +486,14 @@ struct FinishTo {              // ROWS_FINISH
   float* sums;
 };
 
-template <int WAVES, int ROWS, bool WIDE, int EPI, bool LEFT, typename TW>
+// Source: nothing (A), or a RangeSource: attention's key ranges, which the block merges into LDS while its weights travel,
+// a thread four features of every token.
+template <int WAVES, int ROWS, bool WIDE, int EPI, bool LEFT, typename TW, typename... Source>
 __global__ __launch_bounds__(WAVES * 64) void gemm_rows_kernel(void* __restrict__ Cv, long ldc, const bf16_t* __restrict__ A, long lda,
-                                                              const bf16_t* __restrict__ W, int M, int N, int K, FinishTo fin, LeftNorm left) {
+                                                              const bf16_t* __restrict__ W, int M, int N, int K, FinishTo fin, LeftNorm left,
+                                                              Source... source) {
+  constexpr bool RANGES = sizeof...(Source) > 0;
+  extern __shared__ __attribute__((aligned(16))) uint2 merged[];     // RANGES: [K / 8][TOKENS], a piece's tokens turned by the piece
   static_assert(ROWS == 8 || (WIDE && (ROWS == 16 || ROWS == 32)), "8, 16 or 32 rows");
   constexpr int DEPTH = ROWS == 32 ? 4 : 8;                // steps whose loads are in flight
   constexpr int RT = ROWS == 32 ? 2 : 1;                   // tiles of 16 rows (or one of 8)
@@ -526,12 +538,22 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_rows_kernel(void* __restrict_
       for (int f = 0; f < WF; ++f)
         w[j][t][f].n = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(w_src[t], addressing::rows_step(w_lane, s, steps, 2048, f * 1024), 0, 0));
 #pragma unroll
-    for (int f = 0; f < XF; ++f)
+    for (int f = 0; f < (RANGES ? 0 : XF); ++f)
       a[j][f].n = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(a_src, addressing::rows_step(a_lane, s, steps, 2 * KSTEP, f * 16), 0, 0));
 #endif
   };
 #pragma unroll
   for (int j = 0; j < DEPTH; ++j) fetch(j, j);
+  if constexpr (RANGES) {
+    const RangeSource rs{source...};
+    const int rec = rs.head_dim + 4;
+    for (int quad = tid; quad < K / 4; quad += WAVES * 64) {
+      const int head = quad * 4 / rs.head_dim, f0 = quad * 4 - head * rs.head_dim, piece = quad / 2;
+      merge_ranges<16>(rs.ranges + (long)head * rs.count * rec, (long)rs.heads * rs.count * rec, rs.count, rec, rs.head_dim, f0, 0, 1, M,
+                   [&](const int token, const uint2 packed) { merged[(piece * TOKENS + (token + piece) % TOKENS) * 2 + quad % 2] = packed; });
+    }
+    __syncthreads();
+  }
   LeftNormRows rows_left;
   if constexpr (LEFT) {
     __builtin_amdgcn_sched_barrier(0);          // behind the weights' loads, whose waits then do not include them
@@ -542,6 +564,15 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_rows_kernel(void* __restrict_
     const bool more = s0 + DEPTH < steps;
 #pragma unroll
     for (int j = 0; j < DEPTH; ++j) {
+      if constexpr (RANGES) {
+        // (of tokens beyond M what LDS holds, which only reaches columns that are never stored)
+#pragma unroll
+        for (int f = 0; f < XF; ++f) {
+          const int piece = range.k0 / 8 + (s0 + j) * 8 + lg * 2 + (WIDE ? f : lr / 8), token = WIDE ? lr : lr % 8;
+          a[j][f] = zero_frag();
+          if (s0 + j < steps) a[j][f].n = *reinterpret_cast<const u32x4_t*>(merged + (piece * TOKENS + (token + piece) % TOKENS) * 2);
+        }
+      }
 #pragma unroll
       for (int f = 0; f < XF; ++f)
 #pragma unroll
@@ -640,6 +671,49 @@ extern "C" int pi_gemm_finish(float* X, const void* A, long lda, const void* W, 
 #undef PICK
 #undef GO
   return pi_check_launch("gemm_finish");
+}
+
+// Attention's key ranges as activations of the finishing product: blocks of 8 rows, each of which merges them all, so not for
+// more bytes than a block reads in the time of the merging kernel.  2,048 x 2,048 with the norm behind it, us: one token with 2
+// ranges of 32 heads of 64 9.5 -> 5.5, eight with 4 (280 KB) 10.8 -> 9.0, of which the merge is 4.5; the merging kernel takes 3.5
+// and the product then 4.3.  The records' maxima and sums through LDS, 16 rows to a block, or twice the loads in flight: 9.5, 9.3, 9.0.
+#define FINISH_RANGE_BYTES (320 << 10)
+#define FINISH_RANGE_LDS (64 << 10)
+
+// Blocks, as pi_gemm_finish_blocks, with which the finishing kernel merges the ranges itself; 0: it does not.
+extern "C" int pi_gemm_finish_ranges_blocks(int M, int N, int heads, int head_dim, int count) {
+  const long K = (long)heads * head_dim;
+  if (head_dim < 8 || head_dim % 8 || count < 1 || K > 8192 || !pi_gemm_finish_blocks(M, N, (int)K) || finish_rows(N) != 8) return 0;
+  if ((long)M * heads * count * (head_dim + 4) * 4 > FINISH_RANGE_BYTES || K * (M > 8 ? 16 : 8) * 2 > FINISH_RANGE_LDS) return 0;
+  return N / 8;
+}
+
+template <bool WIDE, typename TW>
+static int launch_finish_ranges(float* X, const RangeSource& rs, const bf16_t* W, const void* norm_w, bf16_t* H, float* sums, int M, int N, int K, hipStream_t stream) {
+  const auto kernel = gemm_rows_kernel<8, 8, WIDE, ROWS_FINISH, false, TW, RangeSource>;
+  static const hipError_t configured = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, FINISH_RANGE_LDS);
+  if (configured != hipSuccess) return pi_fail("gemm_finish: cannot reserve %d bytes of LDS: %s", FINISH_RANGE_LDS, hipGetErrorString(configured));
+  hipLaunchKernelGGL(kernel, dim3(N / 8), dim3(512), (size_t)K * (WIDE ? 16 : 8) * 2, stream, X, (long)N, (const bf16_t*)nullptr, 0L, W, M, N, K,
+                     FinishTo{norm_w, H, sums}, LeftNorm{}, rs);
+  return pi_check_launch("gemm_finish (key ranges merged on the way in)");
+}
+
+// pi_gemm_finish whose activations are attention's key ranges (`ranges`: float32 [M, heads, count, head_dim + 4], see RangeSource).
+extern "C" int pi_gemm_finish_ranges(float* X, const void* ranges, int heads, int head_dim, int count, const void* W, const void* norm_w, int norm_dtype,
+                                     void* H, float* sums, long sums_elems, int M, int N, hipStream_t stream) {
+  const int blocks = pi_gemm_finish_ranges_blocks(M, N, heads, head_dim, count), K = heads * head_dim;
+  PI_REQUIRE(blocks > 0, "gemm_finish: not for %d ranges of %d heads of %d, M=%d N=%d", count, heads, head_dim, M, N);
+  PI_REQUIRE(((uintptr_t)ranges % 16 == 0) && ((uintptr_t)W % 16 == 0), "gemm_finish: operands must be 16-byte aligned");
+  PI_REQUIRE(sums_elems >= (long)M * blocks, "gemm_finish: %ld floats for %ld sums", sums_elems, (long)M * blocks);
+  PI_REQUIRE(norm_dtype == PI_F32 || norm_dtype == PI_BF16, "gemm_finish: unsupported norm weight dtype %d", norm_dtype);
+  const RangeSource rs{(const float*)ranges, heads, head_dim, count};
+  const bf16_t* w = (const bf16_t*)W;
+  if (M > 8) {
+    if (norm_dtype == PI_BF16) return launch_finish_ranges<true, bf16_t>(X, rs, w, norm_w, (bf16_t*)H, sums, M, N, K, stream);
+    return launch_finish_ranges<true, float>(X, rs, w, norm_w, (bf16_t*)H, sums, M, N, K, stream);
+  }
+  if (norm_dtype == PI_BF16) return launch_finish_ranges<false, bf16_t>(X, rs, w, norm_w, (bf16_t*)H, sums, M, N, K, stream);
+  return launch_finish_ranges<false, float>(X, rs, w, norm_w, (bf16_t*)H, sums, M, N, K, stream);
 }
 
 // C[M, N] = A[M, K] . W[N, K]^T for 1..16 tokens with all of k in a block, W the copy in the streaming order: stored in

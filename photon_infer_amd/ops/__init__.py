@@ -275,7 +275,7 @@ def gemm(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, accumulate: bool =
                 raise KernelError("gemm: accumulation needs a float32 output")
             materialize(out, ws)
         if _FAST and fast.gemm_from_ranges(out, a, w, accumulate, w.shape[0], _rows(w, "gemm w"), _rows(out, "gemm out"),
-                                           may_defer and out.dtype == torch.float32 and out.is_contiguous(), ws):
+                                           may_defer and out.dtype == torch.float32 and out.is_contiguous(), ws, next_norm):
             return
         merged = torch.empty((a.tokens, a.heads * a.head_dim), dtype=torch.bfloat16, device=out.device)
         fast.merge_ranges(merged, a)

@@ -73,6 +73,8 @@ _SIGNATURES = {
         "pi_gemm_skinny": [P, I, L, P, L, P, L, I, I, I, I, P, L, P, I, P],
         "pi_gemm_rows": [P, I, L, P, L, P, I, I, I, P, I, F, P],
         "pi_gemm_finish_blocks": [I, I, I],
+        "pi_gemm_finish_ranges_blocks": [I, I, I, I, I],
+        "pi_gemm_finish_ranges": [P, P, I, I, I, P, P, I, P, P, L, I, I, P],
         "pi_gemm_finish": [P, P, L, P, P, I, P, P, L, I, I, I, P],
         "pi_attention_tile_rows": [I, I, I],
         "pi_attention_prefill_mfma": [P, L, P, L, P, P, P, I, P, P, P, P, P, P, P, P, I, I, I, I, I, I, F, I, L, P, P, P, L, F, F, I, I, P],

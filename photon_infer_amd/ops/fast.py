@@ -49,6 +49,7 @@ FUSED_DECODE_HEAD_DIMS = (64, 128)                 # ... and of its form that st
 MAX_DECODE_SPLITS = 64         # the combine kernel holds one key range per lane
 DECODE_WAVES_PER_UNIT = 2      # waves of the decode attention kernel per compute unit that fill the chip (measured at batch 1 to 64: more is never faster)
 DECODE_MIN_KEYS_PER_SPLIT = 128
+RANGES_TO_SHARE = 32           # ranges of all requests from which on two waves of a block share one (decode_range_waves)
 # Waves that share a block's keys, against ranges with their merging kernel or one wave (lists of attention times, 32 heads, 8 kv
 # heads, 600 to 4,096 keys each).  Blocks have to fill their rounds over the units this far: 384 of them, 1.5 rounds, at 4,096
 # keys 75.7 -> 81.0 us (up to 1,024 keys 23.8 -> 21.4), 320 at head size 128 126 -> 140; 192, three quarters of one round,
@@ -57,6 +58,7 @@ DECODE_MIN_KEYS_PER_SPLIT = 128
 # for lengths that are uneven: 64 requests of 2,000 to 4,000 keys 83 -> 76, of 4,096 each 96.5 -> 99.5 and with the second
 # waves gone at once 97.  From 10 % between the longest and the mean on the waves gain.
 DECODE_WAVES_FILL, DECODE_WAVES_FILL_LONG, DECODE_WAVES_LONG, DECODE_WAVES_MIN_KEYS = 0.75, 0.8, 1024, 512
+PLAIN_HEADS = (None, None, None, 0, 0.0, 1.0, 0, 0)   # a decode attention's options: none
 UNEVEN = 1.1                   # longest context over the mean from which a step's lengths are uneven
 
 
@@ -202,11 +204,19 @@ def _finish_blocks(M: int, N: int, K: int) -> int:
     return _lib.load("bf16").pi_gemm_finish_blocks(M, N, K)
 
 
+@functools.lru_cache(maxsize=4096)
+def _finish_ranges_blocks(M: int, N: int, heads: int, head_dim: int, count: int) -> int:
+    return _lib.load("bf16").pi_gemm_finish_ranges_blocks(M, N, heads, head_dim, count)
+
+
 def _finish(out, a, w, M, N, K, lda, ldw, next_norm, ws: KernelWorkspace) -> bool:
-    """out += a @ w^T of a few tokens by the kernel that also makes the next norm but for its root, left in the workspace;
-    False, and nothing done, where it does not take the product or the weights have no streaming copy."""
+    """out += a @ w^T of a few tokens by the kernel that also makes the next norm but for its root, left in the workspace (in
+    the place of pieces of k, whose order of sums hangs on the step anyway; a product that is not cut keeps the one order that
+    steps up to 32 tokens have); False, and nothing done, where it does not take the product or the weights have no streaming copy.  ``a`` may be
+    ``KeyRanges``, where the kernel merges as many."""
     weight, eps = next_norm
-    blocks = _finish_blocks(M, N, K)
+    ranges = a if isinstance(a, KeyRanges) else None
+    blocks = _finish_blocks(M, N, K) if ranges is None else _finish_ranges_blocks(M, N, ranges.heads, ranges.head_dim, ranges.count)
     if not blocks or out.dtype != torch.float32 or not weight.is_contiguous() or weight.numel() != N or lda >= RING_MAX_STRIDE:
         return False
     w_ptr, tiled = _streamed(ws, w, N, K, ldw)
@@ -214,8 +224,13 @@ def _finish(out, a, w, M, N, K, lda, ldw, next_norm, ws: KernelWorkspace) -> boo
         return False
     h = torch.empty((M, N), dtype=torch.bfloat16, device=out.device)
     sums = torch.empty((M, blocks), dtype=torch.float32, device=out.device)
-    _lib.call("bf16", "pi_gemm_finish", out.data_ptr(), a.data_ptr(), lda, w_ptr, weight.data_ptr(), 0 if weight.dtype == torch.float32 else 1,
-              h.data_ptr(), sums.data_ptr(), sums.numel(), M, N, K, _stream())
+    norm = (weight.data_ptr(), 0 if weight.dtype == torch.float32 else 1, h.data_ptr(), sums.data_ptr(), sums.numel())
+    if ranges is None:
+        _lib.call("bf16", "pi_gemm_finish", out.data_ptr(), a.data_ptr(), lda, w_ptr, *norm, M, N, K, _stream())
+    else:
+        _lib.call("bf16", "pi_gemm_finish_ranges", out.data_ptr(), ranges.part.data_ptr(), ranges.heads, ranges.head_dim, ranges.count, w_ptr, *norm,
+                  M, N, _stream())
+        ws.counts["ranges_merged_by_product"] += 1
     ws.left_norm = LeftNorm(out, weight, eps, h, sums, blocks)
     ws.counts["norms_left"] += 1
     return True
@@ -361,10 +376,17 @@ def merge_ranges(out: torch.Tensor, kr: KeyRanges) -> None:
               kr.part.data_ptr(), kr.heads, kr.head_dim, kr.count, None, None, 0, 1.0, _stream())
 
 
-def gemm_from_ranges(out, kr: KeyRanges, w, accumulate, N, ldw, ldc, may_defer, ws: Optional[KernelWorkspace]) -> bool:
+def gemm_from_ranges(out, kr: KeyRanges, w, accumulate, N, ldw, ldc, may_defer, ws: Optional[KernelWorkspace], next_norm=None) -> bool:
     """out (+)= merged(kr) @ w^T by the weight-streaming kernel, which merges the key ranges as it
-    stages its activations; the same bits as merging first."""
+    stages its activations; the same bits as merging first.  With ``next_norm`` by the kernel that finishes ``out`` and leaves
+    the norm, if it merges as many ranges; False if it only takes them merged."""
     M, K = kr.tokens, kr.heads * kr.head_dim
+    splits = _skinny_splits(M, N, K)
+    if next_norm is not None and may_defer and accumulate and splits > 1 and ws is not None and w.dtype == torch.bfloat16 and w.stride(1) == 1:
+        if _finish(out, kr, w, M, N, K, 0, ldw, next_norm, ws):
+            return True
+        if _finish_blocks(M, N, K) and _streamed(ws, w, N, K, ldw)[1]:
+            return False
     if not ranges_product_ok(M, kr.head_dim, N * K * 2) or w.dtype != torch.bfloat16 or w.stride(1) != 1 or ldw % 8 or w.data_ptr() % 16:
         return False
     if accumulate:
@@ -375,7 +397,6 @@ def gemm_from_ranges(out, kr: KeyRanges, w, accumulate, N, ldw, ldc, may_defer, 
         epilogue = EPI_F32
     else:
         return False
-    splits = _skinny_splits(M, N, K)
     buf = _piece_buffer(ws, splits * M * N, w.device) if splits > 1 else None
     made = ctypes.c_int(0)
     w_ptr, tiled = _streamed(ws, w, N, K, ldw)
@@ -733,6 +754,16 @@ def decode_block_waves(splits: int, R: int, num_kv_heads: int, max_kv_len: int, 
     return 2 if rounds < 3 and bucket > DECODE_WAVES_MIN_KEYS * max(1, head_dim // 64) else 1
 
 
+def decode_range_waves(splits: int, R: int) -> Tuple[int, int]:
+    """(ranges, waves that share one) in place of ``splits`` ranges of a wave each: two waves of a block walk a range's keys as
+    fast as two ranges do (8 requests of 4,000 keys, 8 kv heads of 64: 17.0 us either way; one request 6.8 and 7.5, 16 27.6 and
+    28.4; four waves 21.5, 9.6 and 36.9), and where the output projection merges the ranges, every block of it all of them, it has
+    half as many.  A merging kernel is no faster for it (4 requests of 16,000 latents, 64 ranges: 2 us a step slower)."""
+    if R <= RANGES_MAX_TOKENS and splits > 1 and R * splits >= RANGES_TO_SHARE:
+        return -(-splits // 2), 2
+    return splits, 1
+
+
 def lengths_uneven(kv_lens) -> bool:
     """Whether a step's contexts differ enough for waves that share one: the longest against the mean."""
     if len(kv_lens) <= RANGES_MAX_TOKENS:
@@ -741,13 +772,17 @@ def lengths_uneven(kv_lens) -> bool:
     return int(lens.max()) * len(lens) > UNEVEN * int(lens.sum())
 
 
-def _waves_or_ranges(ctx, splits: int, R: int, num_kv_heads: int, head_dim: int, longest: int, bound: int, plan=None) -> Tuple[int, int, Optional[int]]:
+def _waves_or_ranges(ctx, splits: int, R: int, num_kv_heads: int, head_dim: int, longest: int, bound: int, plan=None,
+                     plain: bool = True) -> Tuple[int, int, Optional[int]]:
     """(ranges, waves, where the device reads whether the waves are to share at all) of a decode attention; ``bound`` > 0: a
-    token sees so many keys at most; ``plan``: the requests are the single tokens of a step with portions, which the host knows."""
+    token sees so many keys at most; ``plain``: heads without options; ``plan``: the requests are the single tokens of a step with portions, which the host knows."""
     bounded = 0 < bound < decode_length_bucket(longest)
     waves = decode_block_waves(splits, R, num_kv_heads, min(longest, bound) if bounded else longest, head_dim)
     if waves == 1 or splits > 1:
-        return (1, waves, None) if waves > 1 else (splits, 1, None)
+        if waves > 1:
+            return 1, waves, None
+        # as the kernel that starts from the projection, to the same bits
+        return (*(decode_range_waves(splits, R) if plain and head_dim in FUSED_DECODE_HEAD_DIMS else (splits, 1)), None)
     if bounded:                                       # the contexts' lengths do not say how many keys are seen
         return 1, 1, None
     if plan is not None:
@@ -786,7 +821,7 @@ def paged_attention(out, q, k_cache, v_cache, block_table, ctx, num_heads, num_k
         # (a token's keys end at its chunk's start, whatever the context)
         splits = _decode_splits_that_fit(ws, n_req, num_heads, num_kv_heads, head_dim, min(longest, chunk + keep) if chunk else longest)
         bound = min(window or 1 << 30, chunk + keep if chunk else 1 << 30) if window or chunk else 0
-        splits, waves, uneven = _waves_or_ranges(ctx, splits, n_req, num_kv_heads, head_dim, longest, bound, plan)
+        splits, waves, uneven = _waves_or_ranges(ctx, splits, n_req, num_kv_heads, head_dim, longest, bound, plan, opt == PLAIN_HEADS)
         part = _attn_part(ws, n_req * num_heads * splits * (head_dim + 4), q.device)
         _lib.call("bf16", "pi_attention_decode", out.data_ptr(), out.stride(0), q.data_ptr(), q.stride(0),
                   k_cache.data_ptr(), v_cache.data_ptr(), block_table.data_ptr(), block_table.shape[1],
@@ -895,7 +930,10 @@ def decode_attention_from_projection(out, qkv, ctx, table, num_heads, num_kv_hea
     splits = _decode_splits_that_fit(ws, R, num_heads, num_kv_heads, head_dim, ctx.max_kv_len)
     leave = leave_ranges > 0 and ws is not None and splits > 1 and ranges_product_ok(R, head_dim, leave_ranges)
     waves, uneven = 1, None
-    if not leave:
+    if leave:
+        splits, waves = decode_range_waves(splits, R)
+        leave = splits > 1
+    else:
         splits, waves, uneven = _waves_or_ranges(ctx, splits, R, num_kv_heads, head_dim, ctx.max_kv_len, window)
     part = _attn_part(ws, R * num_heads * splits * (head_dim + 4), out.device)
     _lib.call("bf16", "pi_attention_decode_fused", out.data_ptr(), out.stride(0),

@@ -77,6 +77,38 @@ def test_finished_stream_and_left_norm_against_float64(ops, M, N, K, w_dtype):
             assert ((unit.double() - wanted).abs() <= ROUND * (1.1 * slack + wanted.abs() + 1e-3)).all()
 
 
+@pytest.mark.parametrize("M,heads,head_dim,count,inside", [(1, 8, 64, 2, True), (1, 32, 64, 16, True), (1, 32, 64, 40, False), (3, 5, 128, 13, True), (2, 8, 80, 9, True), (7, 24, 128, 3, True),
+                                                          (8, 32, 64, 4, True), (9, 32, 64, 3, True), (16, 32, 64, 2, True), (16, 24, 128, 2, False), (16, 32, 64, 8, False)])
+def test_key_ranges_into_a_finished_stream(ops, M, heads, head_dim, count, inside):
+    """Attention's key ranges as activations: merged by the finishing product where they are few, by the merging kernel
+    before it elsewhere; empty ranges, ranges of unlike maxima."""
+    N, K = 512, heads * head_dim
+    g = gen(count + K)
+    part = torch.randn(M, heads, count, head_dim + 4, generator=g, device=DEV)
+    part[..., head_dim] *= 3
+    part[..., head_dim + 1] = part[..., head_dim + 1].abs() + 0.5
+    if count > 2:
+        part[:, :, 1, head_dim], part[:, :, 1, :head_dim], part[:, :, 1, head_dim + 1] = float("-inf"), 0.0, 0.0
+    rows = torch.arange(M, dtype=torch.int32, device=DEV)
+    ranges = ops.KeyRanges(part, count, M, heads, head_dim, rows)
+    weights = torch.exp2(part[..., head_dim].double() - part[..., head_dim].double().amax(-1, keepdim=True))
+    merged = (part[..., :head_dim].double() * weights[..., None]).sum(2) / (part[..., head_dim + 1].double() * weights).sum(2)[..., None]
+    w = (torch.randn(N, K, generator=g, device=DEV) * K ** -0.5).to(BF16)
+    weight = (torch.rand(N, generator=g, device=DEV) + 0.5).to(BF16)
+    ws = ops.KernelWorkspace(DEV)
+    ws.add_stream_copy(w)
+    x0 = torch.randn(M, N, generator=g, device=DEV)
+    x = x0.clone()
+    ops.gemm(x, ranges, w, accumulate=True, may_defer=True, ws=ws, next_norm=(weight, 1e-5))
+    assert ws.counts["norms_left"] == 1 and ws.counts["ranges_merged_by_product"] == int(inside)
+    a = merged.reshape(M, K)
+    want = x0.double() + a @ w.double().t()
+    assert ((x.double() - want).abs() <= ROUND * (a.abs() @ w.double().abs().t()) + 1e-5).all()
+    left = ws.take_left_norm(x, weight, 1e-5)
+    assert torch.equal(left.h, (x * weight.float()).to(BF16))
+    assert (left.sums.double().sum(1) - (x.double() ** 2).sum(1)).abs().max() <= 1e-5 * (x.double() ** 2).sum(1).max()
+
+
 def test_rows_that_are_not_finite_stay_by_themselves_and_zero_rows_keep_their_eps(ops):
     M, N, K = 8, 256, 512
     g = gen(3)
