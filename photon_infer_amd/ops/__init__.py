@@ -24,6 +24,8 @@ PI_F32, PI_BF16 = 0, 1
 MAX_HEAD_DIM = 256              # the matrix-core attention kernels
 GENERAL_MAX_HEAD_DIM = 640      # the general attention kernel (key rows of a latent cache are wide)
 
+FEW_TOKENS = fast.FEW_TOKENS    # up to this many tokens a product may take all of k in a block (weights with a streaming copy)
+
 _FAST = True
 
 
@@ -1452,11 +1454,12 @@ def gemm_clamped_glu(out: torch.Tensor, a: torch.Tensor, w_gate_up: torch.Tensor
     if x is not None:
         materialize(x, ws)
     M, I = out.shape
-    if w_gate_up.shape[0] != 2 * I or a.shape != (M, w_gate_up.shape[1]) or bias.dtype != torch.float32 or bias.numel() != 2 * I:
+    if w_gate_up.shape[0] != 2 * I or tuple(a.shape) != (M, w_gate_up.shape[1]) or bias.dtype != torch.float32 or bias.numel() != 2 * I:
         raise KernelError(f"gemm_clamped_glu: shapes do not agree: a {tuple(a.shape)}, w {tuple(w_gate_up.shape)}, out {tuple(out.shape)}")
     if M == 0:
         return
-    if _FAST and block == 16 and a.dtype == torch.bfloat16 and w_gate_up.dtype == torch.bfloat16 and out.is_contiguous() and bias.is_contiguous():
+    if (_FAST and block == 16 and a.dtype == torch.bfloat16 and w_gate_up.dtype == torch.bfloat16 and out.is_contiguous() and bias.is_contiguous()
+            and not isinstance(a, LeftNorm)):        # (few tokens: not that kernel's)
         if fast.gemm_clamped_glu(out, a, w_gate_up, bias, limit, alpha, M, 2 * I, a.shape[1], _rows(a, "gemm a"), _rows(w_gate_up, "gemm w")):
             if ws is not None:
                 ws.counts["gated_epilogues"] += 1

@@ -37,6 +37,9 @@ SHARED_ROWS_PER_BLOCK = 64     # ... with this many weight rows per block, and n
                                # rows 29.7 and 32.0, 9,216 29.2 and 31.3, 12,160 29.4 and 31.1, 14,720 33.2 and 35.4; the same at 100 tokens
                                # (35.7 and 39.0, 35.4 and 38.0, 35.4 and 37.6, 39.1 and 41.7), and at k of 2,048 and 8,192
 FEW_TOKENS = 16                # up to this many tokens a product whose weights have a streaming copy may take all of k in a block (pi_gemm_rows)
+FEW_TOKENS_WHOLE_K = 4096      # ... and does in the place of pieces that a kernel of its own would add, up to this k (M = 1 / 12: 1,024 x 2,048 5.4 / 5.9
+                               # us in pieces and 3.3 / 4.2, 4,384 x 2,048 8.8 / 9.5 and 6.3 / 7.4, 6,560 x 3,072 12.7 / 13.7 and 9.6 / 10.6; 2,048 x
+                               # 8,192 11 / 11 and 10 / 13)
 RING_MAX_STRIDE = 1 << 21      # elements between rows up to which that kernel's byte offsets fit 31 bits
 FLOAT32_ROWS = 32              # up to this many rows a float32 product goes to the weight-streaming kernel
 FLOAT32_MAX_STRIDE = 1 << 21   # floats between rows up to which the float32 kernels' offsets inside a tile fit 32 bits
@@ -264,6 +267,8 @@ def gemm(out, a, w, accumulate, M, N, K, lda, ldw, ldc, may_defer=False, ws: Opt
         return True
     splits = _skinny_splits(M, N, K)
     if may_defer and accumulate and splits > 1 and next_norm is not None and _finish(out, a, w, M, N, K, lda, ldw, next_norm, ws):
+        return True
+    if splits > 1 and not may_defer and M <= FEW_TOKENS and K <= FEW_TOKENS_WHOLE_K and _rows(out.data_ptr(), epilogue, ldc, a, w, M, N, K, lda, ldw, ws):
         return True
     pieces = _skinny(out.data_ptr(), epilogue, ldc, a, w, M, N, K, lda, ldw, splits, ws)
     if pieces is not None:

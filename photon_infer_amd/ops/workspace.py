@@ -191,6 +191,9 @@ class KernelWorkspace:
             return None
         return entry[0]
 
+    def has_stream_copy(self, w: torch.Tensor) -> bool:
+        return w.dim() == 2 and self.stream_copy_of(w, w.shape[0], w.shape[1]) is not None
+
     def take_left_norm(self, x: torch.Tensor, weight: torch.Tensor, eps: float) -> Optional[LeftNorm]:
         """What is left of the norm of ``x`` with these parameters, if a product has made it."""
         left, self.left_norm = self.left_norm, None

@@ -36,6 +36,7 @@ UNIT_EPS = 1e-6      # inside the root of the unit vectors' length
 
 class ChannelDeltaRule(Mixer):
     graph_safe = True        # slots and request boundaries are read on the device
+    takes_left_norm = True   # the activations are read by products only, before the stream is updated
 
     def __init__(self, hidden_size: int, num_heads: int, num_kv_heads: int, key_dim: int, value_dim: int, conv_taps: int,
                  decay_rank: int, gate_rank: int, eps: float, out_scale: float = 1.0, accumulate: bool = True):
@@ -99,7 +100,7 @@ class ChannelDeltaRule(Mixer):
         y = torch.empty((T, self.v_size), dtype=self.dtype, device=h.device)
         ops.head_norm_gate(y, o, gate, self.w_norm, self.eps, self.num_heads, self.value_dim, self.out_scale)
         ops.gemm(x, y, self.w_o, accumulate=self.accumulate,
-                 may_defer=self.accumulate and getattr(ctx, "may_defer", False), ws=ws)
+                 may_defer=self.accumulate and getattr(ctx, "may_defer", False), ws=ws, next_norm=getattr(ctx, "next_norm", None))
 
 
 MIXERS.register("channel_delta_rule", ChannelDeltaRule)
@@ -116,7 +117,7 @@ class GatedDeltaRule(Mixer):
 
     One projection gives everything that is read from h, as float32: rows [q | k | v | b | a | g]."""
 
-    graph_safe = True
+    graph_safe = takes_left_norm = True
 
     def __init__(self, hidden_size: int, num_heads: int, num_kv_heads: int, key_dim: int, value_dim: int, conv_taps: int, eps: float,
                  accumulate: bool = True):
@@ -167,7 +168,7 @@ class GatedDeltaRule(Mixer):
                        H, self.num_kv_heads, self.key_dim, self.value_dim, self.key_dim ** -0.5, UNIT_EPS, kind="head_delta")
         y = torch.empty((T, self.v_size), dtype=self.dtype, device=h.device)
         ops.head_norm_gate(y, o, proj[:, C + 2 * H:], self.w_norm, self.eps, H, self.value_dim, gate="silu")
-        ops.gemm(x, y, self.w_o, accumulate=self.accumulate, may_defer=self.accumulate and getattr(ctx, "may_defer", False), ws=ws)
+        ops.gemm(x, y, self.w_o, accumulate=self.accumulate, may_defer=self.accumulate and getattr(ctx, "may_defer", False), ws=ws, next_norm=getattr(ctx, "next_norm", None))
 
 
 MIXERS.register("gated_delta_rule", GatedDeltaRule)

@@ -41,6 +41,7 @@ from .base import MIXERS, PAGE, LayerCache, Mixer, PagedCacheSpec, PagedTensor, 
 
 class LatentAttention(Mixer):
     graph_safe = True        # every kernel takes positions, requests and pages from device memory
+    takes_left_norm = True   # the activations are read by the first projection only
 
     def __init__(self, hidden_size: int, num_heads: int, head_dim: int, rot_dim: int, value_dim: int, q_rank: int, kv_rank: int,
                  scale: float, eps: float, position: Optional[PositionEncoding] = None, accumulate: bool = True,
@@ -149,7 +150,8 @@ class LatentAttention(Mixer):
                                 value_dim=v_rows)
         out = torch.empty((T, self.o_size), dtype=self.dtype, device=h.device)
         ops.head_gemm(out, att, self.w_uv, H, a_head=v_rows, w_rows=self.w_uv_rows, gate=gates)
-        ops.gemm(x, out, self.w_o, accumulate=self.accumulate, may_defer=getattr(ctx, "may_defer", False), ws=ws)
+        ops.gemm(x, out, self.w_o, accumulate=self.accumulate, may_defer=getattr(ctx, "may_defer", False), ws=ws,
+                 next_norm=getattr(ctx, "next_norm", None))
 
 
 MIXERS.register("latent_attention", LatentAttention)

@@ -86,6 +86,7 @@ class ClampedGLU(FeedForward):
     stream in the same kernel, so that the product only accumulates."""
 
     graph_safe = True
+    takes_left_norm = True
 
     def __init__(self, hidden_size: int, intermediate_size: int, limit: float, alpha: float = 1.702,
                  names=("gate", "up", "down"), bias_suffix: str = ".b"):
@@ -130,7 +131,7 @@ class ClampedGLU(FeedForward):
         # the down projection's bias is added to the stream itself on the way, so that the product only accumulates
         ops.gemm_clamped_glu(act, h, self.w_gate_up, self.b_gate_up, self.limit, self.alpha, self.interleave, ws=ws,
                              x=x, x_bias=self.b_down)
-        ops.gemm(x, act, self.w_down, accumulate=True, may_defer=getattr(ctx, "may_defer", False), ws=ws)
+        ops.gemm(x, act, self.w_down, accumulate=True, may_defer=getattr(ctx, "may_defer", False), ws=ws, next_norm=getattr(ctx, "next_norm", None))
 
 
 FEED_FORWARDS.register("clamped_glu", ClampedGLU)

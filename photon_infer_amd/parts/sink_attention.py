@@ -56,6 +56,7 @@ def distance_slopes(num_heads: int) -> torch.Tensor:
 
 class SinkWindowAttention(Mixer):
     graph_safe = True        # every kernel takes positions, requests and pages from device memory
+    takes_left_norm = True   # the activations are read by the first projection only
 
     def __init__(self, hidden_size: int, num_heads: int, num_kv_heads: int, head_dim: int, value_dim: int, scale: float,
                  window: Optional[int], eps: float, temp_coef: float = 0.0, temp_every: int = 1, qk_norm: bool = True,
@@ -161,7 +162,8 @@ class SinkWindowAttention(Mixer):
         ops.paged_attention(attn, q, cache.k, cache.v, table, ctx, self.num_heads, self.num_kv_heads, self.head_dim,
                             cache.page_size, self.scale, self.window or 0, ws, value_dim=self.value_dim,
                             slopes=self.slopes, sinks=self.sinks, gate=gate, softcap=self.softcap, chunk=self.chunk or 0, keep_first=self.keep_first)
-        ops.gemm(x, attn, self.w_o, accumulate=self.accumulate, may_defer=getattr(ctx, "may_defer", False), ws=ws)
+        ops.gemm(x, attn, self.w_o, accumulate=self.accumulate, may_defer=getattr(ctx, "may_defer", False), ws=ws,
+                 next_norm=getattr(ctx, "next_norm", None))
 
 
 MIXERS.register("sink_window_attention", SinkWindowAttention)

@@ -29,6 +29,7 @@ from .base import MIXERS, LayerCache, Mixer, StateSpec, StepContext
 
 class StateSpaceMixer(Mixer):
     graph_safe = True        # slots and request boundaries are read on the device
+    takes_left_norm = True   # the activations are read by products only, before the stream is updated
 
     def __init__(self, hidden_size: int, num_heads: int, value_dim: int, state_dim: int, groups: int, norm_groups: int,
                  conv_taps: int, eps: float, out_scale: float = 1.0, accumulate: bool = True):
@@ -76,7 +77,7 @@ class StateSpaceMixer(Mixer):
         act = torch.empty((T, inner), dtype=self.dtype, device=h.device)
         ops.gated_group_norm(act, y, proj[:, :inner], self.w_norm, self.eps, self.norm_groups, self.out_scale)
         ops.gemm(x, act, self.w_o, accumulate=self.accumulate,
-                 may_defer=self.accumulate and getattr(ctx, "may_defer", False), ws=ws)
+                 may_defer=self.accumulate and getattr(ctx, "may_defer", False), ws=ws, next_norm=getattr(ctx, "next_norm", None))
 
 
 MIXERS.register("state_space", StateSpaceMixer)
