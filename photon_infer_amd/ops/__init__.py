@@ -453,9 +453,9 @@ def decode_attention_from_projection(out: torch.Tensor, qkv, ctx, rotary, num_he
     caller hands the result straight to ``gemm`` with that matrix; when the keys were split into
     ranges, the kernel may then return them unmerged (``KeyRanges``, in the workspace) instead of
     filling ``out``, and the product merges them as it reads."""
-    if not (_FAST and out.dtype == torch.bfloat16 and out.is_cuda and getattr(ctx, "all_decode", False)):
+    if not (_FAST and out.dtype in (torch.bfloat16, torch.float32) and out.is_cuda and getattr(ctx, "all_decode", False)):
         return False
-    if not isinstance(qkv, Partials) and qkv.dtype != torch.bfloat16:
+    if not isinstance(qkv, Partials) and qkv.dtype != out.dtype:
         return False
     T = out.shape[0]
     table = None
@@ -470,6 +470,9 @@ def decode_attention_from_projection(out: torch.Tensor, qkv, ctx, rotary, num_he
     pages = _check_cache(k_cache, v_cache, num_kv_heads, head_dim, page_size, out.dtype)
     if block_table.dim() != 2 or block_table.dtype != torch.int32 or not block_table.is_contiguous():
         raise KernelError("attention: block table must be contiguous int32 [requests, width]")
+    if out.dtype == torch.float32:
+        return fast.decode_attention_float32(out, qkv, ctx, table, num_heads, num_kv_heads, head_dim, k_cache, v_cache, block_table, page_size, scale,
+                                             window, pages, write_kv)
     return fast.decode_attention_from_projection(out, qkv, ctx, table, num_heads, num_kv_heads, head_dim, k_cache, v_cache,
                                                  block_table, page_size, scale, window, pages, write_kv, ws, leave_ranges)
 

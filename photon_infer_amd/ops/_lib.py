@@ -31,6 +31,8 @@ _SIGNATURES = {
         "pi_gemm_general": [P, I, L, P, I, L, P, I, L, I, I, I, I, P],
         "pi_attention_float32_tile_tokens": [I, I],
         "pi_attention_float32": [P, L, P, L, P, P, P, I, P, P, I, I, I, I, I, I, F, I, L, P, P, P, L, F, F, I, P],
+        "pi_attention_float32_decode_takes": [I, I, I],
+        "pi_attention_float32_decode": [P, L, P, I, I, I, P, I, P, P, P, I, P, P, I, I, I, I, I, F, I, L, I, P, L, P],
         "pi_gemm_float32_pieces": [I, I, I, L, I],
         "pi_gemm_float32": [P, L, P, L, P, L, I, I, I, I, P, L, I, P],
         "pi_gemm_float32_swiglu": [P, L, P, L, P, L, I, I, I, P],

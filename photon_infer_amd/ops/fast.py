@@ -913,6 +913,42 @@ def paged_attention_float32(out, q, k_cache, v_cache, block_table, ctx, num_head
     return True
 
 
+# Key ranges of the float32 decode attention: blocks per compute unit that fill the chip (32 heads on 8 kv heads of 64, 64 requests of
+# 2,000 keys: 85 us with four, 105 with two; heads of 128 take registers for two: 8 requests of 2,000 34 and 43), and keys of the
+# step's length bucket that a range keeps (8 requests of 600: 15.1 us with 128, 17.1 with 256), from a bucket on that is worth the
+# merging kernel (one request of 150: 12.5 us in one range, 13.0 in two)
+FLOAT32_DECODE_BLOCKS_PER_UNIT, FLOAT32_DECODE_MIN_KEYS, FLOAT32_DECODE_MIN_BUCKET = {64: 4, 128: 2}, 128, 512
+
+
+def float32_decode_ranges(R: int, num_kv_heads: int, head_dim: int, max_kv_len: int) -> int:
+    """Key ranges per request and kv head, by the step's length bucket (the same eagerly and replayed)."""
+    bucket = decode_length_bucket(max_kv_len)
+    if bucket < FLOAT32_DECODE_MIN_BUCKET:
+        return 1
+    return max(1, min(MAX_DECODE_SPLITS, FLOAT32_DECODE_BLOCKS_PER_UNIT[head_dim] * compute_units() // (R * num_kv_heads), bucket // FLOAT32_DECODE_MIN_KEYS))
+
+
+def decode_attention_float32(out, qkv, ctx, table, num_heads, num_kv_heads, head_dim, k_cache, v_cache, block_table, page_size, scale, window, pages,
+                             write_kv) -> bool:
+    """``decode_attention_from_projection`` of the float32 path; the kernel always fills ``out``."""
+    R = ctx.R
+    if page_size % 16 or k_cache.data_ptr() % 16 or v_cache.data_ptr() % 16 or not _lib.load("core").pi_attention_float32_decode_takes(num_heads, num_kv_heads, head_dim):
+        return False
+    if not isinstance(qkv, Partials):
+        if qkv.stride(1) != 1 or (R > 1 and qkv.stride(0) != qkv.shape[1]):
+            return False
+        qkv = Partials(qkv, 1, qkv.shape[0], qkv.shape[1])
+    if qkv.M != R or qkv.N < (num_heads + (2 * num_kv_heads if write_kv else 0)) * head_dim:
+        return False
+    ranges = float32_decode_ranges(R, num_kv_heads, head_dim, min(ctx.max_kv_len, window) if window else ctx.max_kv_len)
+    part = torch.empty(R * num_heads * ranges * (head_dim + 2), dtype=torch.float32, device=out.device) if ranges > 1 else None
+    _lib.call("core", "pi_attention_float32_decode", out.data_ptr(), out.stride(0), qkv.part.data_ptr(), qkv.splits, qkv.N, R,
+              None if table is None else table.data_ptr(), int(bool(write_kv)), k_cache.data_ptr(), v_cache.data_ptr(), block_table.data_ptr(),
+              block_table.shape[1], ctx.q_start.data_ptr(), ctx.kv_len.data_ptr(), R, num_heads, num_kv_heads, head_dim, page_size, float(scale),
+              int(window), pages, ranges, None if part is None else part.data_ptr(), 0 if part is None else part.numel(), _stream())
+    return True
+
+
 def decode_attention_from_projection(out, qkv, ctx, table, num_heads, num_kv_heads, head_dim, k_cache, v_cache,
                                      block_table, page_size, scale, window, pages, write_kv,
                                      ws: Optional[KernelWorkspace] = None, leave_ranges: int = 0):
