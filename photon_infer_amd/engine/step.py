@@ -305,6 +305,7 @@ class ModelRunner:
             logit_rows=views["logit_rows"], uneven=views["uneven"],
             q_lens=q_lens, kv_lens=kv_lens, max_q_len=max(q_lens), max_kv_len=max(kv_lens),
             all_decode=all(n == 1 for n in q_lens), host_slots=slots, workspace=self.workspace,
+            every_row=T == R == logit_rows.size,          # single tokens, and a row is wanted once at most
         )
         for planner, prefix, names, finish in planned:
             ctx.plans[planner] = finish({name: views[prefix + name] for name in names})
@@ -457,7 +458,7 @@ class _DecodeGraph:
             req_of_token=d["req_of_token"], q_start=d["q_start"], kv_len=d["kv_len"], slots=d["slots"],
             block_tables={g: d[f"table{g}"].view(R, self.width) for g in range(G)}, logit_rows=d["logit_rows"],
             uneven=d["uneven"], q_lens=[1] * R, kv_lens=(), max_q_len=1, max_kv_len=length_bucket, all_decode=True,
-            workspace=runner.workspace)
+            workspace=runner.workspace, every_row=True)
         self.feed_rows = d["feed_rows"]
         self.temps = d["temps"].view(torch.float32)
         self.uniforms = d["uniforms"].view(torch.float32)

@@ -129,6 +129,30 @@ def embedding(out: torch.Tensor, table: torch.Tensor, ids: torch.Tensor, scale: 
               table.shape[0], float(scale), copies, _stream())
 
 
+EMBEDDING_NORM_MAX_WIDTH = 8192
+
+
+def embedding_norm(x: torch.Tensor, table: torch.Tensor, ids: torch.Tensor, scale: float, weight: torch.Tensor, eps: float, h_dtype: torch.dtype,
+                   ws: KernelWorkspace) -> bool:
+    """``embedding`` into ``x`` [T, D] together with the RMS norm that reads it next, left in ``ws`` for ``take_left_norm``.
+    False, and nothing done, for widths and weights that the kernel does not take."""
+    _gpu(x, table, ids, weight)
+    T, D = x.shape
+    if (not _FAST or D % 4 or D > EMBEDDING_NORM_MAX_WIDTH or not weight.is_contiguous() or weight.shape != (D,) or table.data_ptr() % 16 or weight.data_ptr() % 16
+            or h_dtype not in (torch.float32, torch.bfloat16)):
+        return False
+    if x.dtype != torch.float32 or not x.is_contiguous():
+        raise KernelError("embedding: output must be contiguous float32")
+    if table.dim() != 2 or table.shape[1] != D or not table.is_contiguous():
+        raise KernelError(f"embedding: table shape {tuple(table.shape)} does not match width {D}")
+    _i32(ids, "embedding ids", T)
+    h = torch.empty((T, D), dtype=h_dtype, device=x.device)
+    _lib.call("core", "pi_embedding_norm", x.data_ptr(), h.data_ptr(), _dt(h), table.data_ptr(), _dt(table), ids.data_ptr(), float(scale), weight.data_ptr(),
+              _dt(weight), float(eps), T, D, table.shape[0], _stream())
+    ws.left_norm = LeftNorm(x, weight, eps, h, None, 0)
+    return True
+
+
 def softcap_(x: torch.Tensor, cap: float) -> None:
     """x <- cap * tanh(x / cap), in place, float32."""
     _gpu(x)

@@ -16,6 +16,7 @@ P, I, L, F, D = c_void_p, c_int, c_long, c_float, c_double
 _SIGNATURES = {
     "core": {
         "pi_embedding": [P, P, I, P, I, I, I, F, I, P],
+        "pi_embedding_norm": [P, P, I, P, I, P, F, P, I, F, I, I, I, P],
         "pi_softcap": [P, L, F, P],
         "pi_embedding_positions": [P, P, P, I, P, P, F, I, I, I, I, P],
         "pi_clamped_glu": [P, I, P, I, P, P, P, I, F, F, I, I, P, I, I, P],

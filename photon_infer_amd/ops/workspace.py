@@ -69,13 +69,14 @@ class PendingUpdate:
 class LeftNorm:
     """The norm of a stream ``x`` [M, D] that the product before it made but for the root (``ops.gemm`` with ``next_norm``):
     ``h`` holds bfloat16(x * weight), ``sums`` float32 [M, count] every row's sum of x^2 in pieces.  A product that takes it
-    as activations multiplies its float32 rows by 1 / sqrt(sum / D + eps).  Good until ``x`` changes or is freed."""
+    as activations multiplies its float32 rows by 1 / sqrt(sum / D + eps).  Good until ``x`` changes or is freed.  ``count``
+    0: ``h`` is the norm itself, whole."""
 
     x: torch.Tensor
     weight: torch.Tensor
     eps: float
     h: torch.Tensor
-    sums: torch.Tensor
+    sums: Optional[torch.Tensor]
     count: int
 
     @property

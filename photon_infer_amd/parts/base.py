@@ -116,6 +116,7 @@ class StepContext:
     max_q_len: int = 0
     max_kv_len: int = 0
     all_decode: bool = False
+    every_row: bool = False               # a step of single tokens whose logits are all wanted: logit_rows are 0 .. T - 1
     host_slots: Sequence[int] = ()        # the requests' state slots, on the host
     # Set by whoever arranges the parts, for the part that runs next: it may leave its update of
     # the stream in pieces (``ops.gemm(..., may_defer=True)``) because the stream's next reader
@@ -124,6 +125,7 @@ class StepContext:
     # Set beside ``may_defer``, or None: (weight, eps) of the norm that reads the stream next, when that norm's own reader takes
     # a norm whose root is left to it (``ops.gemm(..., next_norm=...)``).
     next_norm: Any = None
+    opening_norm: Any = None              # set by the model for the embedding: (weight, eps, dtype) of the norm that reads the stream first
     after_block_norm: Any = None          # set by the model per block: the same for whoever reads the stream after this block
     may_leave_choices: bool = False       # likewise: a routed feed-forward may leave its result as the experts' rows (``ops.LeftChoices``)
     after_block_consumes: bool = False    # set by the model per block: whoever reads the stream after this block adds pending pieces
@@ -252,6 +254,11 @@ class Block(Part):
         receives a list of ``LayerCache`` in this order instead of a single one."""
         m = getattr(self, "mixer", None)
         return [m] if m is not None else []
+
+    @property
+    def opening_norm(self):
+        """(weight, eps, dtype) of the RMS norm that reads the stream first, when whoever makes the stream may make it too; else None."""
+        return None
 
     def forward(self, x: torch.Tensor, ctx: StepContext, cache) -> None:
         raise NotImplementedError

@@ -117,6 +117,10 @@ class PreNormBlock(Block):
     def first_norm(self):
         return norm_left_to(self.norm1, self.mixer)
 
+    @property
+    def opening_norm(self):
+        return (self.norm1.weight, self.norm1.eps, self.norm1.dtype) if getattr(self.norm1, "leaves_root", False) else None
+
     def forward(self, x: torch.Tensor, ctx: StepContext, cache: LayerCache) -> None:
         # A mixer or feed-forward may leave its update of x in pieces (ops.gemm(..., may_defer=True))
         # when the stream's next reader adds them: norm2 after the mixer; after the feed-forward,

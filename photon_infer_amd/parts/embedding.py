@@ -41,6 +41,9 @@ class TokenEmbedding(Part):
         embeddings that look at more than the ids."""
         shape = (token_ids.shape[0], self.copies, self.hidden_size) if self.copies else (token_ids.shape[0], self.hidden_size)
         x = torch.empty(shape, dtype=torch.float32, device=token_ids.device)
+        norm = getattr(ctx, "opening_norm", None)
+        if norm is not None and not self.copies and ctx.workspace is not None and ops.embedding_norm(x, self.weight, token_ids, self.scale, *norm, ctx.workspace):
+            return x
         ops.embedding(x, self.weight, token_ids, self.scale)
         return x
 
@@ -82,6 +85,7 @@ class PositionedEmbedding(TokenEmbedding):
 
 class LMHead(Part):
     graph_safe = True
+    takes_left_norm = True
 
     def __init__(self, vocab_size: int, hidden_size: int, tied: bool, tensor_name: str = "weight", softcap: Optional[float] = None):
         self.vocab_size = int(vocab_size)

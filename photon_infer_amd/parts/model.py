@@ -18,7 +18,7 @@ from ..errors import ConfigError
 from ..weights.loader import TensorSpec
 from .base import Block, KVCacheSpec, LayerCache, Norm, PagedCacheSpec, PagedTensor, StateSpec, StepContext
 from .embedding import LMHead, TokenEmbedding
-from .norm import settle_left_join
+from .norm import norm_left_to, settle_left_join
 
 
 @dataclass(frozen=True)
@@ -151,8 +151,10 @@ class DecoderModel:
         ws = ctx.workspace
         ops.reset_deferred(ws)             # nothing of an earlier (failed) step may linger
         ctx.scratch.clear()
-        x = self.embedding.forward(ctx.token_ids, ctx)
         order = self.spec.run_order
+        ctx.opening_norm = getattr(self.blocks[order[0].layer], "opening_norm", None) if order else None
+        x = self.embedding.forward(ctx.token_ids, ctx)
+        ctx.opening_norm = None
         wanted = ctx.logit_rows.shape[0] > 0
         for i, entry in enumerate(order):
             block = self.blocks[entry.layer]
@@ -167,7 +169,7 @@ class DecoderModel:
                 ctx.after_block_norm = getattr(self.blocks[order[i + 1].layer], "first_norm", None)
             else:                          # the final norm; or nobody (the pieces are then dropped unread)
                 ctx.after_block_consumes = not wanted or bool(getattr(self.final_norm, "consumes_deferred", False))
-                ctx.after_block_norm = None
+                ctx.after_block_norm = norm_left_to(self.final_norm, self.head) if wanted and ctx.every_row else None
             ctx.may_defer, ctx.next_norm = False, None
             block.forward(x, ctx, caches[i])
         ctx.may_defer = ctx.may_leave_choices = ctx.after_block_consumes = False
@@ -178,7 +180,7 @@ class DecoderModel:
             settle_left_join(x, ctx)
         if not getattr(self.final_norm, "consumes_deferred", False):
             ops.materialize(x, ws)
-        return self.head.forward(self.final_norm.forward(x, ctx, rows=ctx.logit_rows), ctx)
+        return self.head.forward(self.final_norm.forward(x, ctx, rows=None if ctx.every_row else ctx.logit_rows), ctx)
 
     def streamed_weights(self) -> List[torch.Tensor]:
         """The weight matrices that every decode step reads whole (see ``Part.streamed_weights``)."""

@@ -96,10 +96,10 @@ class RMSNorm(Norm):
         if left is not None:
             return left.apply(ctx.workspace, self.weight_f32(), self.eps, self.dtype, rows)
         if rows is None and ctx is not None and ctx.workspace is not None:
-            # only there when this norm's reader has said that it takes it (norm_left_to)
+            # without its root only when this norm's reader has said that it takes it (norm_left_to)
             left = ctx.workspace.take_left_norm(x, self.weight, self.eps)
             if left is not None:
-                return left
+                return left if left.count else left.h
         m = x.shape[0] if rows is None else rows.shape[0]
         out = torch.empty((m, self.dim), dtype=self.dtype, device=x.device)
         ops.rmsnorm(out, x, self.weight, self.eps, rows, ws=ctx.workspace if ctx is not None else None)

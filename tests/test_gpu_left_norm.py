@@ -129,6 +129,30 @@ def test_rows_that_are_not_finite_stay_by_themselves_and_zero_rows_keep_their_ep
     assert not torch.isfinite(x[2]).any() and torch.isnan(x[6]).all() and torch.isnan(out[2]).all() and torch.isnan(out[6]).all()
 
 
+@pytest.mark.parametrize("T,D,table_dtype,w_dtype,h_dtype", [(1, 64, BF16, BF16, BF16), (3, 1000, BF16, F32, BF16), (8, 2048, BF16, BF16, BF16), (5, 8192, F32, F32, F32),
+                                                           (300, 2052, F32, BF16, BF16)])
+def test_embedding_and_its_norm_in_one_kernel(ops, T, D, table_dtype, w_dtype, h_dtype):
+    g = gen(D)
+    table = torch.randn(50, D, generator=g, device=DEV).to(table_dtype)
+    weight = (torch.rand(D, generator=g, device=DEV) + 0.5).to(w_dtype)
+    ids = torch.randint(0, 50, (T,), generator=g, device=DEV).to(torch.int32)
+    if T > 2:
+        ids[1] = 50                                     # not in the table: a row that is not a number, and no fault
+    for scale in (1.0, 3.5):
+        x, plain, ws = torch.empty(T, D, device=DEV), torch.empty(T, D, device=DEV), ops.KernelWorkspace(DEV)
+        assert ops.embedding_norm(x, table, ids, scale, weight, 1e-5, h_dtype, ws)
+        ops.embedding(plain, table, ids, scale)
+        assert torch.equal(x.view(torch.int32), plain.view(torch.int32))
+        left = ws.take_left_norm(x, weight, 1e-5)
+        assert left.count == 0 and left.h.dtype == h_dtype
+        good = [t for t in range(T) if ids[t] < 50]
+        want = plain[good].double() / torch.sqrt((plain[good].double() ** 2).mean(1, keepdim=True) + 1e-5) * weight.double()
+        slack = want.abs() * (ROUND if h_dtype == BF16 else 1e-6)
+        assert ((left.h[good].double() - want).abs() <= slack * 1.001).all()
+        assert torch.isnan(left.h[[t for t in range(T) if t not in good]].float()).all()
+    assert not ops.embedding_norm(torch.empty(1, 30, device=DEV), torch.zeros(4, 30, device=DEV), ids[:1] * 0, 1.0, torch.ones(30, device=DEV), 1e-5, F32, ws)
+
+
 def test_whoever_else_reads_or_changes_the_stream_finds_it_finished(ops):
     """Another norm, another update of the stream and a reader that takes no left norm."""
     ws, x, want, weight = made(ops, 3, 256, 512)
@@ -166,7 +190,6 @@ def test_a_models_decode_steps_leave_their_norms(tmp_path, batch):
     with and without graphs, to the same tokens, and their logits are those of the steps that make every norm."""
     from photon_infer_amd import EngineOptions, ModelRunner, StepEntry
     from photon_infer_amd.config import LlamaConfig
-    from photon_infer_amd.parts import PreNormBlock
 
     cfg = LlamaConfig.from_dict(dict(architectures=["LlamaForCausalLM"], hidden_size=512, intermediate_size=1024, num_attention_heads=8,
                                      num_key_value_heads=2, head_dim=64, num_hidden_layers=3, vocab_size=1024, max_position_embeddings=512,
@@ -180,6 +203,7 @@ def test_a_models_decode_steps_leave_their_norms(tmp_path, batch):
         runner = ModelRunner(None, EngineOptions(max_batch=batch, max_cache_tokens=batch * 64, max_model_len=128, use_graphs=graphs, keep_logits=True),
                              config=cfg, tensors=dict(tensors))
         if not leave:
+            runner.model.final_norm.leaves_root = False
             for b in runner.model.blocks:
                 b.norm1.leaves_root = b.norm2.leaves_root = False
         for i in range(batch):
@@ -191,7 +215,6 @@ def test_a_models_decode_steps_leave_their_norms(tmp_path, batch):
             rows.append(runner.decode_logits.clone())
         return torch.stack(rows).double(), runner.workspace.counts
 
-    assert PreNormBlock is not None
     eager, counts = run(False, True)
     assert counts["norms_left"] > 0, counts
     graphed, _ = run(True, True)
