@@ -2,91 +2,17 @@
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 from ctypes import c_double, c_float, c_int, c_long, c_void_p
 from typing import Dict
 
 import torch
 
 from ..errors import KernelError, KernelLibraryMissing
-from . import build
+from . import build, signatures
 
-P, I, L, F, D = c_void_p, c_int, c_long, c_float, c_double
-
-# entry point -> argument types (all return int: 0 = ok)
-_SIGNATURES = {
-    "core": {
-        "pi_embedding": [P, P, I, P, I, I, I, F, I, P],
-        "pi_embedding_norm": [P, P, I, P, I, P, F, P, I, F, I, I, I, P],
-        "pi_softcap": [P, L, F, P],
-        "pi_embedding_positions": [P, P, P, I, P, P, F, I, I, I, I, P],
-        "pi_clamped_glu": [P, I, P, I, P, P, P, I, F, F, I, I, P, I, I, P],
-        "pi_causal_conv_silu": [P, L, P, L, P, P, I, I, I, P, P, I, I, P, L, P],
-        "pi_state_space_scan": [P, L, P, L, P, L, P, P, P, P, P, I, I, I, P, L, I, I, I, I, P],
-        "pi_state_space_chunk": [I, I],
-        "pi_state_space_chunks": [P, L, P, L, P, L, P, P, P, P, P, I, I, I, P, P, P, L, I, I, I, I, P],
-        "pi_gated_group_norm": [P, I, L, P, L, P, L, P, F, F, I, I, I, P],
-        "pi_delta_scan": [P, L, P, L, P, L, P, P, P, L, P, P, I, I, I, P, L, I, I, I, I, F, F, I, F, P],
-        "pi_rmsnorm": [P, I, P, P, P, I, F, I, I, P, I, L, P],
-        "pi_swiglu": [P, P, I, I, I, I, P],
-        "pi_rope_kv_write": [P, L, P, L, P, L, I, P, P, P, I, I, I, I, I, I, I, P, P, P, I, I, L, P, I, I, I, I, I, I, P, P],
-        "pi_gemm_general": [P, I, L, P, I, L, P, I, L, I, I, I, I, P],
-        "pi_attention_float32_tile_tokens": [I, I],
-        "pi_attention_float32": [P, L, P, L, P, P, P, I, P, P, I, I, I, I, I, I, F, I, L, P, P, P, L, F, F, I, P],
-        "pi_attention_float32_decode_takes": [I, I, I],
-        "pi_attention_float32_decode": [P, L, P, I, I, I, P, I, P, P, P, I, P, P, I, I, I, I, I, F, I, L, I, P, L, P],
-        "pi_gemm_float32_pieces": [I, I, I, L, I],
-        "pi_gemm_float32": [P, L, P, L, P, L, I, I, I, I, P, L, I, P],
-        "pi_gemm_float32_swiglu": [P, L, P, L, P, L, I, I, I, P],
-        "pi_splitk_reduce": [P, I, L, P, I, I, I, P],
-        "pi_paged_attention_general": [P, L, P, L, P, P, I, P, I, P, P, I, I, I, I, I, F, I, L, I, P, L, I, P, P, P, L, F, F, I, I, P],
-        "pi_branch_norm_add": [P, P, I, P, P, P, P, P, F, F, I, I, P],
-        "pi_cast_stream": [P, I, P, L, P],
-        "pi_qk_norm_kv_write": [P, L, P, I, P, L, P, P, P, P, F, F, I, I, I, I, I, I, I, P, P, P, I, I, L, P, I, L, I, I, P],
-        "pi_latent_kv_write": [P, L, I, P, L, P, P, P, P, P, F, I, I, I, I, I, P, P, P, I, I, L, P, I, L, I, P, P],
-        "pi_head_gemm": [P, L, I, P, L, I, P, I, I, I, I, I, I, P, I, P, L, P],
-        "pi_matrix_memory_scan": [P, L, P, L, I, I, I, I, I, P, P, F, F, P, P, I, P, L, I, I, I, I, I, I, P, L, P],
-        "pi_head_norm_gate": [P, I, P, L, P, L, P, F, I, I, I, F, I, P],
-        "pi_route": [P, P, P, L, I, I, I, I, I, I, I, P, F, I, P],
-        "pi_group_entries": [P, I, I, P, P, P, P, P, I, I, P],
-        "pi_gather_rows": [P, P, I, P, I, I, I, P, P],
-        "pi_grouped_gemm_general": [P, I, L, P, I, L, P, I, L, L, P, P, P, I, I, I, P],
-        "pi_combine_choices": [P, P, P, P, I, I, I, I, P, I, P, I, P],
-        "pi_activation": [P, I, P, L, I, I, P],
-        "pi_layer_norm": [P, I, P, P, P, P, F, I, I, I, P],
-        "pi_sandwich_norm_add": [P, P, I, P, P, P, P, P, P, P, P, P, F, I, I, P],
-        "pi_rms_join": [P, P, I, P, P, I, P, P, I, I, P, I, P, F, P, F, I, I, P],
-        "pi_retention": [P, I, P, L, P, I, P, I, I, P, F, F, P, P, I, I, I, P, L, I, I, I, I, P, L, P],
-        "pi_diff_combine": [P, I, P, I, F, F, F, I, I, I, I, I, P],
-        "pi_paged_attention_general_ranges": [I, I, I],
-        "pi_rope_table": [P, P, P, I, I, F, P],
-        "pi_qk_rope_norm_write": [P, L, I, P, L, P, I, P, P, I, I, F, P, P, I, I, I, I, I, I, P, P, P, P, P, P, I, I, L, P],
-        "pi_hyper_streams": [P, I, I, I, P, P, I, P, I, P, I, P, P, F, P, I, P, P, L, I, P, P, I, P],
-        "pi_token_shift": [P, I, P, P, P, L, I, P, P, P, I, I, P],
-        "pi_min_gru": [P, I, L, P, L, P, I, P, P, P, I, I, I, P, L, I, I, P, L, P],
-        "pi_sample": [P, P, L, P, P, I, I, P, L, P],
-        "pi_sample_static": [P, P, L, P, P, I, I, P],
-    },
-    "bf16": {
-        "pi_gemm_mfma": [P, I, L, P, L, P, L, I, I, I, I, I, P],
-        "pi_gemm_mfma_pieces": [I, I],
-        "pi_gemm_mfma_shape": [I, I, I, I, I],
-        "pi_gemm_mfma_splits": [I, I, I, I, L, D, I],
-        "pi_gemm_mfma_clamped_glu": [P, L, P, L, P, L, I, I, I, P, F, F, I, P],
-        "pi_gemm_mfma_grouped": [P, I, L, P, L, P, L, L, P, P, P, I, I, I, L, L, F, F, P, L, P],
-        "pi_gemm_skinny": [P, I, L, P, L, P, L, I, I, I, I, P, L, P, I, P],
-        "pi_gemm_rows": [P, I, L, P, L, P, I, I, I, P, I, F, P],
-        "pi_gemm_finish_blocks": [I, I, I],
-        "pi_gemm_finish_ranges_blocks": [I, I, I, I, I],
-        "pi_gemm_finish_ranges": [P, P, I, I, I, P, P, I, P, P, L, I, I, P],
-        "pi_gemm_finish": [P, P, L, P, P, I, P, P, L, I, I, I, P],
-        "pi_attention_tile_rows": [I, I, I],
-        "pi_attention_prefill_mfma": [P, L, P, L, P, P, P, I, P, P, P, P, P, P, P, P, I, I, I, I, I, I, F, I, L, P, P, P, L, F, F, I, I, P],
-        "pi_attention_combine_rows": [P, L, P, I, P, I, I, I, P, P, L, F, P],
-        "pi_attention_decode": [P, L, P, L, P, P, P, I, P, P, P, I, I, I, I, I, F, I, L, I, I, P, P, L, P, P, P, L, F, F, I, I, P],
-        "pi_attention_decode_fused": [P, L, P, L, P, I, I, I, P, I, P, P, P, I, P, P, I, I, I, I, I, F, I, L, I, I, P, P, L, I, P],
-        "pi_gemm_skinny_ranges": [P, I, L, P, I, I, I, P, L, I, I, I, P, L, P, I, P],
-    },
-}
+_CTYPES = {signatures.P: c_void_p, signatures.I: c_int, signatures.L: c_long, signatures.F: c_float, signatures.D: c_double}
 
 _LIBS: Dict[str, ctypes.CDLL] = {}
 
@@ -122,12 +48,12 @@ def load(module: str) -> ctypes.CDLL:
         lib = ctypes.CDLL(path)
     except OSError as e:
         raise KernelLibraryMissing(f"cannot load kernel library {path}: {e}") from e
-    for name, argtypes in _SIGNATURES[module].items():
+    for name, types in signatures.SIGNATURES[module].items():
         try:
             fn = getattr(lib, name)
         except AttributeError:
             raise KernelLibraryMissing(f"kernel library {path} lacks entry point {name}") from None
-        fn.argtypes = argtypes
+        fn.argtypes = [_CTYPES[t] for t in types]
         fn.restype = c_int
     err = getattr(lib, f"pi_{module}_last_error")
     err.restype = ctypes.c_char_p
@@ -138,12 +64,30 @@ def load(module: str) -> ctypes.CDLL:
 
 
 _ENTRIES: Dict[str, object] = {}      # entry points called before, by name (names are unique over the modules)
+_LAUNCHER = None
+
+
+def _bound(module: str, name: str):
+    """The entry point as a builtin of the launcher, an extension of the interpreter whose functions turn their arguments
+    into the entry point's types by themselves: a call of thirteen arguments costs 0.3 us so and 2.4 through ctypes, and
+    a step that is not a replayed graph makes some 130 of them."""
+    global _LAUNCHER
+    if _LAUNCHER is None:
+        path = build.build_module("launch")
+        try:
+            loader = importlib.machinery.ExtensionFileLoader("photon_launch", path)
+            launcher = importlib.util.module_from_spec(importlib.util.spec_from_file_location("photon_launch", path, loader=loader))
+            loader.exec_module(launcher)
+        except ImportError as e:
+            raise KernelLibraryMissing(f"cannot load the launcher {path}: {e}") from e
+        _LAUNCHER = launcher
+    return _LAUNCHER.bind(name, ctypes.cast(getattr(load(module), name), c_void_p).value)
 
 
 def call(module: str, name: str, *args) -> None:
     entry = _ENTRIES.get(name)
     if entry is None:
-        entry = _ENTRIES[name] = getattr(load(module), name)
+        entry = _ENTRIES[name] = _bound(module, name)
     rc = entry(*args)
     if rc != 0:
         msg = load(module)._pi_last_error()

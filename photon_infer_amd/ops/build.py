@@ -20,6 +20,7 @@ from concurrent.futures import ThreadPoolExecutor
 from typing import Dict, List
 
 from ..errors import KernelLibraryMissing
+from . import signatures
 
 CSRC_DIR = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "csrc")
 
@@ -31,11 +32,13 @@ MODULES: Dict[str, List[str]] = {
     "bf16": ["gemm_mfma.hip", "gemm_skinny.hip", "attention_mfma.hip", "attention_decode.hip"],
     # host only: cache manager bookkeeping (needs no GPU and no hipcc)
     "runtime": ["runtime/cache.cpp"],
+    # host only: the interpreter's way to the kernel modules' entry points
+    "launch": ["runtime/launch.cpp"],
     # host only: the engine for C / C++ programs (hosts an interpreter; links libpython)
     "api": ["api/photon_engine.cpp"],
 }
 HEADERS = ["common.h", "mfma.h", "addressing.h", "attention_mfma.h", "sampling.h", "token_tiles.h", "tile_plan.h"]
-HOST_MODULES = {"runtime", "api"}
+HOST_MODULES = {"runtime", "launch", "api"}
 HOST_HEADERS = {"api": ["api/photon_engine.h"]}
 HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-Wall"]
 
@@ -125,6 +128,8 @@ def _build_dir() -> str:
 def source_hash(module: str) -> str:
     host = module in HOST_MODULES
     h = hashlib.sha256(" ".join(HOST_FLAGS + sanitize_flags() if host else HIPCC_FLAGS).encode())
+    if module == "launch":
+        h.update(signatures.launch_table().encode())
     for name in MODULES[module] + (HOST_HEADERS.get(module, []) if host else HEADERS):
         h.update(" ".join(FILE_FLAGS.get(name, [])).encode())
         path = os.path.join(CSRC_DIR, name)
@@ -176,6 +181,10 @@ def build_module(module: str, force: bool = False, quiet: bool = False) -> str:
         compile_flags = compile_flags + python_embed_flags()[0]
         link_libs = python_embed_flags()[1]
     bdir = _build_dir()
+    if module == "launch":
+        compile_flags = compile_flags + [python_embed_flags()[0][0], "-I", bdir]
+        with open(os.path.join(bdir, "launch_entries.inc"), "w") as f:
+            f.write(signatures.launch_table())
     sources = MODULES[module]
     missing = [s for s in sources if not os.path.isfile(os.path.join(CSRC_DIR, s))]
     if missing:

@@ -177,7 +177,7 @@ def _skinny(out_ptr: int, epilogue: int, ldc: int, a, w, M, N, K, lda, ldw, spli
     made = ctypes.c_int(0)
     w_ptr, tiled = _streamed(ws, w, N, K, ldw)
     _lib.call("bf16", "pi_gemm_skinny", out_ptr, epilogue, ldc, a.data_ptr(), lda, w_ptr, ldw, M, N, K, splits,
-              None if buf is None else buf.data_ptr(), 0 if buf is None else buf.numel(), ctypes.byref(made), tiled, _stream())
+              None if buf is None else buf.data_ptr(), 0 if buf is None else buf.numel(), ctypes.addressof(made), tiled, _stream())
     if made.value > 1:
         if ws is not None:
             ws.counts["split_products"] += 1
@@ -407,7 +407,7 @@ def gemm_from_ranges(out, kr: KeyRanges, w, accumulate, N, ldw, ldc, may_defer, 
     w_ptr, tiled = _streamed(ws, w, N, K, ldw)
     _lib.call("bf16", "pi_gemm_skinny_ranges", out.data_ptr(), epilogue, ldc, kr.part.data_ptr(), kr.heads, kr.head_dim, kr.count,
               w_ptr, ldw, M, N, splits, None if buf is None else buf.data_ptr(), 0 if buf is None else buf.numel(),
-              ctypes.byref(made), tiled, _stream())
+              ctypes.addressof(made), tiled, _stream())
     if ws is not None:
         ws.counts["ranges_merged_by_product"] += 1
     if made.value > 1:

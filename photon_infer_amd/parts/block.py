@@ -131,7 +131,8 @@ class PreNormBlock(Block):
             self.mixer.forward(self.norm1.forward(x, ctx), x, ctx, cache)
             ctx.may_defer, ctx.next_norm = False, None
             return
-        ctx.may_defer, ctx.next_norm = bool(getattr(self.norm2, "consumes_deferred", False)), norm_left_to(self.norm2, self.ffn)
+        ctx.may_defer = bool(getattr(self.norm2, "consumes_deferred", False))
+        ctx.next_norm = norm_left_to(self.norm2, self.ffn) if ctx.T <= ops.FEW_TOKENS else None
         self.mixer.forward(self.norm1.forward(x, ctx), x, ctx, cache)
         ctx.may_defer, ctx.next_norm = ctx.after_block_consumes, ctx.after_block_norm
         self.ffn.forward(self.norm2.forward(x, ctx), x, ctx)

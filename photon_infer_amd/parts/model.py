@@ -156,6 +156,7 @@ class DecoderModel:
         x = self.embedding.forward(ctx.token_ids, ctx)
         ctx.opening_norm = None
         wanted = ctx.logit_rows.shape[0] > 0
+        few = ctx.T <= ops.FEW_TOKENS      # products of more tokens leave no norms
         for i, entry in enumerate(order):
             block = self.blocks[entry.layer]
             # A block meets an update of the stream that is still in pieces only if it says that
@@ -166,10 +167,10 @@ class DecoderModel:
                 ops.materialize(x, ws)
             if i + 1 < len(order):
                 ctx.after_block_consumes = bool(self.blocks[order[i + 1].layer].reads_deferred)
-                ctx.after_block_norm = getattr(self.blocks[order[i + 1].layer], "first_norm", None)
+                ctx.after_block_norm = getattr(self.blocks[order[i + 1].layer], "first_norm", None) if few else None
             else:                          # the final norm; or nobody (the pieces are then dropped unread)
                 ctx.after_block_consumes = not wanted or bool(getattr(self.final_norm, "consumes_deferred", False))
-                ctx.after_block_norm = norm_left_to(self.final_norm, self.head) if wanted and ctx.every_row else None
+                ctx.after_block_norm = norm_left_to(self.final_norm, self.head) if few and wanted and ctx.every_row else None
             ctx.may_defer, ctx.next_norm = False, None
             block.forward(x, ctx, caches[i])
         ctx.may_defer = ctx.may_leave_choices = ctx.after_block_consumes = False

@@ -95,7 +95,7 @@ class RMSNorm(Norm):
         left = take_left_join(x, ctx)
         if left is not None:
             return left.apply(ctx.workspace, self.weight_f32(), self.eps, self.dtype, rows)
-        if rows is None and ctx is not None and ctx.workspace is not None:
+        if rows is None and ctx is not None and ctx.workspace is not None and ctx.workspace.left_norm is not None:
             # without its root only when this norm's reader has said that it takes it (norm_left_to)
             left = ctx.workspace.take_left_norm(x, self.weight, self.eps)
             if left is not None:

@@ -1,0 +1,69 @@
+"""The interpreter's way to the kernel libraries' entry points (csrc/runtime/launch.cpp): argument types as the entry points
+have them, errors as the binding has them.  The entry points here refuse their sizes before they touch a device."""
+import ctypes
+import threading
+
+import pytest
+
+from photon_infer_amd.errors import KernelError
+from photon_infer_amd.ops import _lib, signatures
+
+
+def bound(name, argtypes, function):
+    """The launcher's builtin for ``name``, with a Python function in the entry point's place."""
+    _lib._bound("core", "pi_rmsnorm")
+    keep = ctypes.CFUNCTYPE(ctypes.c_int, *argtypes)(function)
+    return _lib._LAUNCHER.bind(name, ctypes.cast(keep, ctypes.c_void_p).value), keep
+
+
+def rebind(name):
+    _lib._bound("core", name)
+
+
+def test_arguments_arrive_as_the_entry_point_has_them():
+    types = signatures.SIGNATURES["core"]["pi_softcap"]
+    assert types == [signatures.P, signatures.L, signatures.F, signatures.P]
+    got = []
+    call, keep = bound("pi_softcap", [ctypes.c_void_p, ctypes.c_long, ctypes.c_float, ctypes.c_void_p], lambda *a: got.append(a) or 7)
+    try:
+        assert call(1 << 46, -5, 0.1, None) == 7
+        assert call(None, (1 << 63) + 1, 3, True) == 7                 # whole numbers wrap, whole numbers are floats, True is 1
+        assert got[0][:2] == (1 << 46, -5) and abs(got[0][2] - 0.1) < 1e-8 and got[0][3] is None
+        assert got[1] == (None, -(1 << 63) + 1, 3.0, 1)
+        for wrong in ((1, 2, 3.0), (1, 2, 3.0, None, 5), ("a", 2, 3.0, None), (1, 2.5, 3.0, None), (1, 2, "x", None), (1, None, 3.0, None)):
+            with pytest.raises(TypeError):
+                call(*wrong)
+        assert len(got) == 2
+    finally:
+        rebind("pi_softcap")
+
+
+def test_errors_of_an_entry_point_and_unknown_names():
+    for _ in range(2):
+        with pytest.raises(KernelError, match="rmsnorm: bad sizes M=-1 D=5"):
+            _lib.call("core", "pi_rmsnorm", None, 0, None, None, None, 0, 1e-5, -1, 5, None, 0, 0, 0)
+    with pytest.raises(KeyError):
+        _lib._LAUNCHER.bind("pi_no_such_entry", 1)
+    with pytest.raises(ValueError):
+        _lib._LAUNCHER.bind("pi_rmsnorm", 0)
+    rebind("pi_rmsnorm")
+
+
+def test_every_entry_point_is_in_the_launchers_table_and_threads_keep_their_messages():
+    for module, entries in signatures.SIGNATURES.items():
+        for name in entries:
+            assert callable(_lib._bound(module, name)), name
+    seen = {}
+
+    def ask(i):
+        try:
+            _lib.call("core", "pi_rmsnorm", None, 0, None, None, None, 0, 1e-5, -i, 5, None, 0, 0, 0)
+        except KernelError as e:
+            seen[i] = str(e)
+
+    threads = [threading.Thread(target=ask, args=(i,)) for i in range(1, 9)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert all(f"M=-{i} D" in seen[i] for i in range(1, 9)), seen
