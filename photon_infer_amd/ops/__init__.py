@@ -274,7 +274,8 @@ def gemm_swiglu(out: torch.Tensor, a: torch.Tensor, w_gate_up: torch.Tensor, blo
 
 
 def gemm(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, accumulate: bool = False,
-         may_defer: bool = False, ws: Optional[KernelWorkspace] = None, next_norm=None) -> None:
+         may_defer: bool = False, ws: Optional[KernelWorkspace] = None, next_norm=None,
+         whole: bool = False) -> None:
     """out[M, N] (+)= a[M, K] @ w[N, K]^T with float32 accumulation.
 
     ``ws``: where a product split over k keeps its pieces (without one, memory of this call's own).
@@ -283,7 +284,9 @@ def gemm(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, accumulate: bool =
     product that was split over k may then stay in pieces there.
     ``next_norm`` (with ``may_defer``; (weight, eps)): the RMS norm that reads ``out`` next, whose own reader is a product that
     takes a ``LeftNorm``: a product of few tokens may then finish ``out`` and leave that in the workspace
-    (``KernelWorkspace.take_left_norm``)."""
+    (``KernelWorkspace.take_left_norm``).
+    ``whole``: a product of few tokens that would be cut over k, its pieces added by a kernel of their own, may take all of k in a
+    block instead where the weights have a streaming copy: other sums in another order than without one."""
     left = None
     if isinstance(a, LeftNorm):
         if _FAST and w.dtype == torch.bfloat16 and not accumulate and not may_defer:
@@ -322,7 +325,7 @@ def gemm(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, accumulate: bool =
         materialize(out, ws)
     if _FAST and a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16:
         may_defer_ = may_defer and out.dtype == torch.float32 and out.is_contiguous()
-        if fast.gemm(out, a, w, accumulate, M, N, K, lda, ldw, ldc, may_defer_, ws, left, next_norm):
+        if fast.gemm(out, a, w, accumulate, M, N, K, lda, ldw, ldc, may_defer_, ws, left, next_norm, whole):
             return
     if left is not None:
         a = whole_norm(left)

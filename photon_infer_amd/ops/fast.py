@@ -240,7 +240,7 @@ def _finish(out, a, w, M, N, K, lda, ldw, next_norm, ws: KernelWorkspace) -> boo
 
 
 def gemm(out, a, w, accumulate, M, N, K, lda, ldw, ldc, may_defer=False, ws: Optional[KernelWorkspace] = None,
-         left: Optional[LeftNorm] = None, next_norm=None) -> bool:
+         left: Optional[LeftNorm] = None, next_norm=None, whole: bool = False) -> bool:
     if not _gemm_ok(a, w, K, lda, ldw):
         return False
     if accumulate:
@@ -268,7 +268,7 @@ def gemm(out, a, w, accumulate, M, N, K, lda, ldw, ldc, may_defer=False, ws: Opt
     splits = _skinny_splits(M, N, K)
     if may_defer and accumulate and splits > 1 and next_norm is not None and _finish(out, a, w, M, N, K, lda, ldw, next_norm, ws):
         return True
-    if splits > 1 and not may_defer and M <= FEW_TOKENS and K <= FEW_TOKENS_WHOLE_K and _rows(out.data_ptr(), epilogue, ldc, a, w, M, N, K, lda, ldw, ws):
+    if whole and splits > 1 and not may_defer and M <= FEW_TOKENS and K <= FEW_TOKENS_WHOLE_K and _rows(out.data_ptr(), epilogue, ldc, a, w, M, N, K, lda, ldw, ws):
         return True
     pieces = _skinny(out.data_ptr(), epilogue, ldc, a, w, M, N, K, lda, ldw, splits, ws)
     if pieces is not None:

@@ -211,7 +211,7 @@ class PagedAttention(Mixer):
                 # the output, or its key ranges still to be merged, which the product does as it reads them
                 ops.gemm(x, done if isinstance(done, ops.KeyRanges) else attn, self.w_o, accumulate=self.accumulate,
                          may_defer=self.accumulate and not self.o_bias and getattr(ctx, "may_defer", False), ws=ws,
-                         next_norm=getattr(ctx, "next_norm", None))
+                         next_norm=getattr(ctx, "next_norm", None), whole=True)
                 if self.o_bias and not self.bias_to_caller:
                     ops.add_row_bias(x, self.b_o)
                 return
@@ -249,7 +249,7 @@ class PagedAttention(Mixer):
         # where the arrangement allows it, the product stays in pieces for the stream's next reader
         ops.gemm(x, attn, self.w_o, accumulate=self.accumulate,
                  may_defer=self.accumulate and not self.o_bias and getattr(ctx, "may_defer", False), ws=ws,
-                 next_norm=getattr(ctx, "next_norm", None))
+                 next_norm=getattr(ctx, "next_norm", None), whole=True)
         if self.o_bias and not self.bias_to_caller:
             ops.add_row_bias(x, self.b_o)
 

@@ -86,12 +86,12 @@ class ChannelDeltaRule(Mixer):
         T, ws, C = h.shape[0], ctx.workspace, self.channels
         f32 = lambda n: torch.empty((T, n), dtype=torch.float32, device=h.device)
         proj = f32(C + self.num_heads)
-        ops.gemm(proj, h, self.w_in, ws=ws)
+        ops.gemm(proj, h, self.w_in, ws=ws, whole=True)
         low = torch.empty((T, self.decay_rank + self.gate_rank), dtype=self.dtype, device=h.device)
-        ops.gemm(low, h, self.w_low, ws=ws)
+        ops.gemm(low, h, self.w_low, ws=ws, whole=True)
         a, gate = f32(self.a_size), f32(self.v_size)
-        ops.gemm(a, low[:, :self.decay_rank], self.w_a2, ws=ws)
-        ops.gemm(gate, low[:, self.decay_rank:], self.w_g2, ws=ws)
+        ops.gemm(a, low[:, :self.decay_rank], self.w_a2, ws=ws, whole=True)
+        ops.gemm(gate, low[:, self.decay_rank:], self.w_g2, ws=ws, whole=True)
         qkv = f32(C)
         ops.causal_conv_silu(qkv, proj[:, :C], self.w_conv, None, ctx, cache.state[:, :self.conv_floats])
         o = f32(self.v_size)
@@ -100,7 +100,7 @@ class ChannelDeltaRule(Mixer):
         y = torch.empty((T, self.v_size), dtype=self.dtype, device=h.device)
         ops.head_norm_gate(y, o, gate, self.w_norm, self.eps, self.num_heads, self.value_dim, self.out_scale)
         ops.gemm(x, y, self.w_o, accumulate=self.accumulate,
-                 may_defer=self.accumulate and getattr(ctx, "may_defer", False), ws=ws, next_norm=getattr(ctx, "next_norm", None))
+                 may_defer=self.accumulate and getattr(ctx, "may_defer", False), ws=ws, next_norm=getattr(ctx, "next_norm", None), whole=True)
 
 
 MIXERS.register("channel_delta_rule", ChannelDeltaRule)
@@ -160,7 +160,7 @@ class GatedDeltaRule(Mixer):
         T, ws, C, H = h.shape[0], ctx.workspace, self.channels, self.num_heads
         f32 = lambda n: torch.empty((T, n), dtype=torch.float32, device=h.device)
         proj = f32(C + 2 * H + self.v_size)
-        ops.gemm(proj, h, self.w_in, ws=ws)
+        ops.gemm(proj, h, self.w_in, ws=ws, whole=True)
         qkv = f32(C)
         ops.causal_conv_silu(qkv, proj[:, :C], self.w_conv, None, ctx, cache.state[:, :self.conv_floats])
         o = f32(self.v_size)
@@ -168,7 +168,7 @@ class GatedDeltaRule(Mixer):
                        H, self.num_kv_heads, self.key_dim, self.value_dim, self.key_dim ** -0.5, UNIT_EPS, kind="head_delta")
         y = torch.empty((T, self.v_size), dtype=self.dtype, device=h.device)
         ops.head_norm_gate(y, o, proj[:, C + 2 * H:], self.w_norm, self.eps, H, self.value_dim, gate="silu")
-        ops.gemm(x, y, self.w_o, accumulate=self.accumulate, may_defer=self.accumulate and getattr(ctx, "may_defer", False), ws=ws, next_norm=getattr(ctx, "next_norm", None))
+        ops.gemm(x, y, self.w_o, accumulate=self.accumulate, may_defer=self.accumulate and getattr(ctx, "may_defer", False), ws=ws, next_norm=getattr(ctx, "next_norm", None), whole=True)
 
 
 MIXERS.register("gated_delta_rule", GatedDeltaRule)

@@ -137,7 +137,7 @@ class LatentAttention(Mixer):
                             cache.k if cache.writes else None, cache.v if cache.writes else None, table, cache.page_size,
                             num_gates=self.o_size if self.gate is not None else 0)
         q = torch.empty((T, self.q_size), dtype=self.dtype, device=h.device)
-        ops.gemm(q, cq, self.w_uq, ws=ws)
+        ops.gemm(q, cq, self.w_uq, ws=ws, whole=True)
         # queries in the latent's coordinates, the rotated part behind them
         q_lat = torch.empty((T, H * self.latent_dim), dtype=self.dtype, device=h.device)
         ops.head_gemm(q_lat, q, self.w_uk, H, rot=self.rot_dim, table=rot_table, w_rows=self.w_uk_rows)

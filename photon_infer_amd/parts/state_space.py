@@ -68,7 +68,7 @@ class StateSpaceMixer(Mixer):
     def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext, cache: LayerCache) -> None:
         T, ws, inner = h.shape[0], ctx.workspace, self.inner
         proj = torch.empty((T, self.proj_size), dtype=torch.float32, device=h.device)
-        ops.gemm(proj, h, self.w_in, ws=ws)
+        ops.gemm(proj, h, self.w_in, ws=ws, whole=True)
         xbc = torch.empty((T, self.channels), dtype=torch.float32, device=h.device)
         ops.causal_conv_silu(xbc, proj[:, inner:inner + self.channels], self.w_conv, self.b_conv, ctx, cache.state[:, :self.conv_floats])
         y = torch.empty((T, inner), dtype=torch.float32, device=h.device)
@@ -77,7 +77,7 @@ class StateSpaceMixer(Mixer):
         act = torch.empty((T, inner), dtype=self.dtype, device=h.device)
         ops.gated_group_norm(act, y, proj[:, :inner], self.w_norm, self.eps, self.norm_groups, self.out_scale)
         ops.gemm(x, act, self.w_o, accumulate=self.accumulate,
-                 may_defer=self.accumulate and getattr(ctx, "may_defer", False), ws=ws, next_norm=getattr(ctx, "next_norm", None))
+                 may_defer=self.accumulate and getattr(ctx, "may_defer", False), ws=ws, next_norm=getattr(ctx, "next_norm", None), whole=True)
 
 
 MIXERS.register("state_space", StateSpaceMixer)
