@@ -478,12 +478,21 @@ __global__ __launch_bounds__(512, 4) void gemm_skinny_ring_kernel(void* __restri
 // The other epilogues take the place of gemm_skinny_kernel, four waves on 32 rows that staged the activations of a step at a
 // time, where that did not cut k over blocks: 16,384 x 2,048 with the gated unit, 1 / 8 / 16 tokens 15.7 / 15.8 / 15.6 us -> 14.5 /
 // 14.4 / 15.4; 28,672 x 4,096 50.4 / 50.1 / 51.1 -> 43.6 / 44.8 / 46.0; 128,256 x 2,048 93.4 / 96.3 / 102.7 -> 90.8 / 93.2 / 100.7.
-enum { ROWS_FINISH = 8 };      // besides EPI_BF16, EPI_F32 and EPI_SWIGLU
+enum { ROWS_FINISH = 8, ROWS_CLAMPED = 9 };      // besides EPI_BF16, EPI_F32, EPI_ACCUM and EPI_SWIGLU
 
-struct FinishTo {              // ROWS_FINISH
-  const void* weight;          // of the norm, bfloat16 or float32
+// the clamped gated unit (elementwise.hip's, with its roundings) of a gate and an up value with their biases
+__device__ inline float clamped_unit(float g, float u, float limit, float alpha) {
+  g = fminf(g, limit);
+  u = fminf(fmaxf(u, -limit), limit);
+  return g / (1.0f + expf(-alpha * g)) * (u + 1.0f);
+}
+
+struct FinishTo {
+  const void* weight;          // ROWS_FINISH: of the norm, bfloat16 or float32
   bf16_t* h;
   float* sums;
+  const float* bias;           // ROWS_FINISH: joins the update, [N], or null; ROWS_CLAMPED: of the gate and up rows, [N]
+  float limit, alpha;          // ROWS_CLAMPED: the unit's (clamped_glu)
 };
 
 // Source: nothing (A), or a RangeSource: attention's key ranges, which the block merges into LDS while its weights travel,
@@ -499,7 +508,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_rows_kernel(void* __restrict_
   constexpr int RT = ROWS == 32 ? 2 : 1;                   // tiles of 16 rows (or one of 8)
   constexpr int XF = WIDE ? 2 : 1, WF = ROWS == 8 ? 1 : 2; // fragments of a step: activations, weights of a tile
   constexpr int PARTS = ROWS == 8 ? 2 * WAVES : WAVES;     // sums to add
-  constexpr int OUT_ROWS = EPI == EPI_SWIGLU ? ROWS / 2 : ROWS, TOKENS = WIDE ? 16 : 8;
+  constexpr bool GATED = EPI == EPI_SWIGLU || EPI == ROWS_CLAMPED;
+  constexpr int OUT_ROWS = GATED ? ROWS / 2 : ROWS, TOKENS = WIDE ? 16 : 8;
   __shared__ float red[PARTS][ROWS][17];
   __shared__ float factors[LEFT ? 16 : 1];
   const int tid = threadIdx.x, lane = tid % 64;
@@ -513,6 +523,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_rows_kernel(void* __restrict_
     if (tid / ROWS < M) {
       x = reinterpret_cast<const float*>(Cv)[(long)(tid / ROWS) * N + n0 + tid % ROWS];
       wn = to_float(reinterpret_cast<const TW*>(fin.weight)[n0 + tid % ROWS]);
+      if (fin.bias) x += fin.bias[n0 + tid % ROWS];
     }
   }
   const addressing::WaveRange range = addressing::wave_share(0, K, WAVES, wave);
@@ -620,7 +631,10 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_rows_kernel(void* __restrict_
       if (row == 0) fin.sums[(long)token * gridDim.x + block] = square;
     } else if (mine) {
       const float factor = LEFT ? factors[token] : 1.f;
-      if constexpr (EPI == EPI_SWIGLU) {
+      if constexpr (EPI == ROWS_CLAMPED) {
+        const float g = total(row, 0.f) * factor + fin.bias[n0 + row], u = total(16 + row, 0.f) * factor + fin.bias[n0 + 16 + row];
+        reinterpret_cast<bf16_t*>(Cv)[(long)token * ldc + n0 / 2 + row] = from_float<bf16_t>(clamped_unit(g, u, fin.limit, fin.alpha));
+      } else if constexpr (EPI == EPI_SWIGLU) {
         const float g = total(row, 0.f) * factor, u = total(16 + row, 0.f) * factor;
         reinterpret_cast<bf16_t*>(Cv)[(long)token * ldc + n0 / 2 + row] = from_float<bf16_t>(g / (1.0f + expf(-g)) * u);
       } else {
@@ -644,9 +658,10 @@ extern "C" int pi_gemm_finish_blocks(int M, int N, int K) {
   return N / rows;
 }
 
-// W: the copy in the streaming order (see pi_gemm_skinny).  H bfloat16 [M, N], sums float32 [M, blocks].
+// W: the copy in the streaming order (see pi_gemm_skinny).  H bfloat16 [M, N], sums float32 [M, blocks].  `bias` (or null): float32
+// [N], added to every row of X besides.
 extern "C" int pi_gemm_finish(float* X, const void* A, long lda, const void* W, const void* norm_w, int norm_dtype, void* H, float* sums, long sums_elems,
-                              int M, int N, int K, hipStream_t stream) {
+                              const float* bias, int M, int N, int K, hipStream_t stream) {
   const int blocks = pi_gemm_finish_blocks(M, N, K);
   PI_REQUIRE(blocks > 0, "gemm_finish: not for M=%d N=%d K=%d", M, N, K);
   PI_REQUIRE(lda >= K && lda % 8 == 0 && lda < RING_MAX_STRIDE && ((uintptr_t)A % 16 == 0) && ((uintptr_t)W % 16 == 0), "gemm_finish: operands must be 16-byte aligned, the row stride (%ld) a multiple of 8", lda);
@@ -657,7 +672,7 @@ extern "C" int pi_gemm_finish(float* X, const void* A, long lda, const void* W, 
   const bool eight = K > 2048 && (rows == 8 || blocks < compute_units());
 #define GO(WV, RW, WD, T) \
   hipLaunchKernelGGL((gemm_rows_kernel<WV, RW, WD, ROWS_FINISH, false, T>), dim3(blocks), dim3(WV * 64), 0, stream, X, (long)N, (const bf16_t*)A, lda, \
-                     (const bf16_t*)W, M, N, K, FinishTo{norm_w, (bf16_t*)H, sums}, LeftNorm{})
+                     (const bf16_t*)W, M, N, K, FinishTo{norm_w, (bf16_t*)H, sums, bias, 0.f, 0.f}, LeftNorm{})
 #define PICK(WV, T) \
   do { \
     if (rows == 16) GO(WV, 16, true, T); \
@@ -694,7 +709,7 @@ static int launch_finish_ranges(float* X, const RangeSource& rs, const bf16_t* W
   static const hipError_t configured = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, FINISH_RANGE_LDS);
   if (configured != hipSuccess) return pi_fail("gemm_finish: cannot reserve %d bytes of LDS: %s", FINISH_RANGE_LDS, hipGetErrorString(configured));
   hipLaunchKernelGGL(kernel, dim3(N / 8), dim3(512), (size_t)K * (WIDE ? 16 : 8) * 2, stream, X, (long)N, (const bf16_t*)nullptr, 0L, W, M, N, K,
-                     FinishTo{norm_w, H, sums}, LeftNorm{}, rs);
+                     FinishTo{norm_w, H, sums, nullptr, 0.f, 0.f}, LeftNorm{}, rs);
   return pi_check_launch("gemm_finish (key ranges merged on the way in)");
 }
 
@@ -749,6 +764,22 @@ extern "C" int pi_gemm_rows(void* C, int epilogue, long ldc, const void* A, long
 #undef PICK
 #undef GO
   return pi_check_launch("gemm_rows");
+}
+
+// out[M, N / 2] = the clamped gated unit of A . W^T + bias, gate and up rows of W and bias interleaved by 16, in the product's own
+// kernel (a kernel of its own behind the float32 product took 4.6 us a layer at 12 tokens).  Operands as for pi_gemm_rows.
+extern "C" int pi_gemm_rows_clamped(void* C, long ldc, const void* A, long lda, const void* W, int M, int N, int K, const float* bias, float limit, float alpha,
+                                    const float* sums, int count, float eps, hipStream_t stream) {
+  PI_REQUIRE(M > 0 && M <= 16 && N > 0 && N % 32 == 0 && K > 0 && K % KSTEP == 0 && bias, "gemm_rows_clamped: takes 1..16 tokens, N in 32 and K in 64, got M=%d N=%d K=%d", M, N, K);
+  PI_REQUIRE(lda >= K && lda % 8 == 0 && lda < RING_MAX_STRIDE && K < RING_MAX_STRIDE && ((uintptr_t)A % 16 == 0) && ((uintptr_t)W % 16 == 0), "gemm_rows_clamped: operands must be 16-byte aligned, the row stride (%ld) a multiple of 8", lda);
+  PI_REQUIRE(!sums || (count > 0 && count <= 512 && count % 4 == 0 && (uintptr_t)sums % 16 == 0), "gemm_rows_clamped: a left norm has 4..512 sums a row, got %d", count);
+  const FinishTo unit{nullptr, nullptr, nullptr, bias, limit, alpha};
+  const LeftNorm left{sums, count, K, eps};
+  if (sums)
+    hipLaunchKernelGGL((gemm_rows_kernel<4, 32, true, ROWS_CLAMPED, true, float>), dim3(N / 32), dim3(256), 0, stream, C, ldc, (const bf16_t*)A, lda, (const bf16_t*)W, M, N, K, unit, left);
+  else
+    hipLaunchKernelGGL((gemm_rows_kernel<4, 32, true, ROWS_CLAMPED, false, float>), dim3(N / 32), dim3(256), 0, stream, C, ldc, (const bf16_t*)A, lda, (const bf16_t*)W, M, N, K, unit, left);
+  return pi_check_launch("gemm_rows (clamped unit)");
 }
 
 template <int MB>

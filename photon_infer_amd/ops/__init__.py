@@ -1504,6 +1504,23 @@ def gemm_clamped_glu(out: torch.Tensor, a: torch.Tensor, w_gate_up: torch.Tensor
         clamped_glu(out, gu, bias[:I], bias[I:], limit, alpha, x, x_bias)
 
 
+def clamped_mlp(x: torch.Tensor, act: torch.Tensor, h, w_gate_up: torch.Tensor, bias: torch.Tensor, limit: float, alpha: float, block: int,
+                w_down: torch.Tensor, x_bias: torch.Tensor, next_norm, ws: Optional[KernelWorkspace]) -> bool:
+    """x += (the clamped gated unit of h @ w_gate_up^T + bias) @ w_down^T + x_bias, for a step of a few tokens whose next norm,
+    ``next_norm`` = (weight, eps), is left to its reader (see ``gemm``).  False, and nothing done, for anything else."""
+    if (not _FAST or ws is None or next_norm is None or block != 16 or x.dtype != torch.float32 or act.dtype != torch.bfloat16 or h.dtype != torch.bfloat16
+            or w_gate_up.dtype != torch.bfloat16 or w_down.dtype != torch.bfloat16 or not (x.is_contiguous() and act.is_contiguous() and bias.is_contiguous() and x_bias.is_contiguous())):
+        return False
+    _gpu(x, act, h, w_gate_up, bias, w_down, x_bias)
+    M, I = act.shape
+    if (M == 0 or tuple(h.shape) != (M, w_gate_up.shape[1]) or w_gate_up.shape[0] != 2 * I or tuple(w_down.shape) != (x.shape[1], I) or x.shape[0] != M
+            or bias.dtype != torch.float32 or bias.numel() != 2 * I or x_bias.dtype != torch.float32 or x_bias.numel() != x.shape[1]):
+        return False
+    left = h if isinstance(h, LeftNorm) else None
+    materialize(x, ws)
+    return fast.clamped_mlp(x, act, h if left is None else left.h, w_gate_up, bias, limit, alpha, w_down, x_bias, next_norm, ws, left)
+
+
 # ----------------------------------------------------------------------------- several streams side by side
 HYPER_MAX_STREAMS = 16
 

@@ -212,11 +212,11 @@ def _finish_ranges_blocks(M: int, N: int, heads: int, head_dim: int, count: int)
     return _lib.load("bf16").pi_gemm_finish_ranges_blocks(M, N, heads, head_dim, count)
 
 
-def _finish(out, a, w, M, N, K, lda, ldw, next_norm, ws: KernelWorkspace) -> bool:
+def _finish(out, a, w, M, N, K, lda, ldw, next_norm, ws: KernelWorkspace, bias=None) -> bool:
     """out += a @ w^T of a few tokens by the kernel that also makes the next norm but for its root, left in the workspace (in
     the place of pieces of k, whose order of sums hangs on the step anyway; a product that is not cut keeps the one order that
     steps up to 32 tokens have); False, and nothing done, where it does not take the product or the weights have no streaming copy.  ``a`` may be
-    ``KeyRanges``, where the kernel merges as many."""
+    ``KeyRanges``, where the kernel merges as many.  ``bias`` (float32 [N], not with ranges): added besides."""
     weight, eps = next_norm
     ranges = a if isinstance(a, KeyRanges) else None
     blocks = _finish_blocks(M, N, K) if ranges is None else _finish_ranges_blocks(M, N, ranges.heads, ranges.head_dim, ranges.count)
@@ -229,7 +229,7 @@ def _finish(out, a, w, M, N, K, lda, ldw, next_norm, ws: KernelWorkspace) -> boo
     sums = torch.empty((M, blocks), dtype=torch.float32, device=out.device)
     norm = (weight.data_ptr(), 0 if weight.dtype == torch.float32 else 1, h.data_ptr(), sums.data_ptr(), sums.numel())
     if ranges is None:
-        _lib.call("bf16", "pi_gemm_finish", out.data_ptr(), a.data_ptr(), lda, w_ptr, *norm, M, N, K, _stream())
+        _lib.call("bf16", "pi_gemm_finish", out.data_ptr(), a.data_ptr(), lda, w_ptr, *norm, None if bias is None else bias.data_ptr(), M, N, K, _stream())
     else:
         _lib.call("bf16", "pi_gemm_finish_ranges", out.data_ptr(), ranges.part.data_ptr(), ranges.heads, ranges.head_dim, ranges.count, w_ptr, *norm,
                   M, N, _stream())
@@ -503,6 +503,22 @@ def gemm_clamped_glu(out, a, w, bias, limit, alpha, M, N, K, lda, ldw) -> bool:
     _lib.call("bf16", "pi_gemm_mfma_clamped_glu", out.data_ptr(), out.stride(0), a.data_ptr(), lda, w.data_ptr(), ldw, M, N, K,
               bias.data_ptr(), float(limit), float(alpha), _tile_shape(M, N, K, 1), _stream())
     return True
+
+
+def clamped_mlp(x, act, a, w_gate_up, bias, limit, alpha, w_down, x_bias, next_norm, ws: KernelWorkspace, left: Optional[LeftNorm]) -> bool:
+    """A clamped gated feed-forward of a few tokens as two kernels: the unit (``act``) in the gate | up product, and the down
+    product with its bias finishing the stream ``x`` and leaving its next norm.  False, and nothing done, for what these do not take."""
+    M, I = act.shape
+    K, N = a.shape[1], x.shape[1]
+    lda = a.stride(0) if M > 1 else K
+    if (M > FEW_TOKENS or not _gemm_ok(a, w_gate_up, K, lda, K) or not ws.has_stream_copy(w_gate_up) or not ws.has_stream_copy(w_down) or I % 16
+            or max(lda, K, I) >= RING_MAX_STRIDE or _skinny_splits(M, N, I) < 2 or not _finish_blocks(M, N, I) or next_norm[0].numel() != N or not next_norm[0].is_contiguous()):
+        return False
+    w_ptr, _ = _streamed(ws, w_gate_up, 2 * I, K, K)
+    _lib.call("bf16", "pi_gemm_rows_clamped", act.data_ptr(), act.stride(0), a.data_ptr(), lda, w_ptr, M, 2 * I, K, bias.data_ptr(), float(limit), float(alpha),
+              None if left is None else left.sums.data_ptr(), 0 if left is None else left.count, 0.0 if left is None else left.eps, _stream())
+    ws.counts["gated_epilogues"] += 1
+    return _finish(x, act, w_down, M, N, I, act.stride(0), I, next_norm, ws, x_bias)
 
 
 HEAD_TILES_FROM_TOKENS = 129   # a product per head takes the grouped tile kernel from this many tokens on

@@ -128,6 +128,9 @@ class ClampedGLU(FeedForward):
     def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext) -> None:
         ws = ctx.workspace if ctx is not None else None
         act = torch.empty((h.shape[0], self.intermediate_size), dtype=self.dtype, device=h.device)
+        if ctx is not None and ctx.next_norm is not None and ctx.may_defer and ops.clamped_mlp(
+                x, act, h, self.w_gate_up, self.b_gate_up, self.limit, self.alpha, self.interleave, self.w_down, self.b_down, ctx.next_norm, ws):
+            return
         # the down projection's bias is added to the stream itself on the way, so that the product only accumulates
         ops.gemm_clamped_glu(act, h, self.w_gate_up, self.b_gate_up, self.limit, self.alpha, self.interleave, ws=ws,
                              x=x, x_bias=self.b_down)

@@ -153,6 +153,44 @@ def test_embedding_and_its_norm_in_one_kernel(ops, T, D, table_dtype, w_dtype, h
     assert not ops.embedding_norm(torch.empty(1, 30, device=DEV), torch.zeros(4, 30, device=DEV), ids[:1] * 0, 1.0, torch.ones(30, device=DEV), 1e-5, F32, ws)
 
 
+@pytest.mark.parametrize("M,D,I", [(1, 128, 512), (8, 2048, 1024), (9, 256, 1024), (16, 3072, 576)])
+def test_a_clamped_feed_forward_in_two_kernels(ops, M, D, I):
+    g = gen(D + I)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    wg, wu, w_down = ((rnd(I, D) * 2 * D ** -0.5).to(BF16), (rnd(I, D) * 2 * D ** -0.5).to(BF16), (rnd(D, I) * I ** -0.5).to(BF16))
+    bg, bu, bd, weight = rnd(I), rnd(I), rnd(D), (torch.rand(D, generator=g, device=DEV) + 0.5).to(BF16)
+    pair = lambda a, b: torch.stack([a.view(I // 16, 16, -1), b.view(I // 16, 16, -1)], 1).reshape(2 * I, -1).contiguous()
+    w, bias = pair(wg, wu), pair(bg[:, None], bu[:, None]).view(-1)
+    x0, h = rnd(M, D), rnd(M, D).to(BF16)
+    ws = ops.KernelWorkspace(DEV)
+    ws.add_stream_copy(w), ws.add_stream_copy(w_down)
+    x, act = x0.clone(), torch.empty(M, I, dtype=BF16, device=DEV)
+    assert ops.clamped_mlp(x, act, h, w, bias, 1.5, 1.702, 16, w_down, bd, (weight, 1e-5), ws)
+    # the unit has slopes of at most 1.2 (limit + 1) in the gate and limit in the up value; float32 sums of some 1e-6 of their terms
+    gd, ud = h.double() @ wg.double().t() + bg, h.double() @ wu.double().t() + bu
+    terms = h.double().abs() @ torch.maximum(wg, wu).double().abs().t()
+    gd, ud = gd.clamp(max=1.5), ud.clamp(-1.5, 1.5)
+    unit = gd * torch.sigmoid(1.702 * gd) * (ud + 1)
+    assert ((act.double() - unit).abs() <= ROUND * unit.abs() + 1e-5 * (1 + terms)).all()
+    want = x0.double() + bd + act.double() @ w_down.double().t()
+    assert ((x.double() - want).abs() <= 1e-5 * (1 + want.abs())).all()
+    left = ws.take_left_norm(x, weight, 1e-5)
+    assert torch.equal(left.h, (x * weight.float()).to(BF16)) and ws.counts["norms_left"] == 1
+    # after a norm whose root is left: the same as after the whole norm, but for where it is rounded
+    left2 = ops.LeftNorm(x, weight, 1e-5, left.h, left.sums, left.count)
+    again, act2 = x.clone(), torch.empty_like(act)
+    assert ops.clamped_mlp(again, act2, left2, w, bias, 1.5, 1.702, 16, w_down, bd, (weight, 1e-5), ws)
+    n = x.double() / torch.sqrt((x.double() ** 2).mean(1, keepdim=True) + 1e-5) * weight.double()
+    gd, ud = n @ wg.double().t() + bg, n @ wu.double().t() + bu
+    off = ROUND * (n.abs() @ torch.maximum(wg.abs(), wu.abs()).double().t())
+    gd, ud = gd.clamp(max=1.5), ud.clamp(-1.5, 1.5)
+    unit = gd * torch.sigmoid(1.702 * gd) * (ud + 1)
+    assert ((act2.double() - unit).abs() <= ROUND * unit.abs() + (1.2 * 2.5 + 1.5) * off + 1e-5).all()
+    # no streaming copy of the one or the other: nothing is touched
+    bare, before = ops.KernelWorkspace(DEV), x.clone()
+    assert not ops.clamped_mlp(x, act, h, w, bias, 1.5, 1.702, 16, w_down, bd, (weight, 1e-5), bare) and torch.equal(x, before)
+
+
 def test_whoever_else_reads_or_changes_the_stream_finds_it_finished(ops):
     """Another norm, another update of the stream and a reader that takes no left norm."""
     ws, x, want, weight = made(ops, 3, 256, 512)
