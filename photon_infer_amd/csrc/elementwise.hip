@@ -218,13 +218,21 @@ __global__ void rmsnorm_wide_kernel(TO* __restrict__ out, float* __restrict__ x,
   }
 }
 
-// The embedding of a step and the norm that reads it first: x as embedding_kernel makes it, h its RMS norm, a block to a token, in
-// the place of two kernels that little but start (8 tokens of 2,048: 6.2 + 4.6 us -> 4.4).  The threads, and so the order
-// of the sum, hang on D alone.
-template <typename TE, typename TO, typename TW>
-__global__ __launch_bounds__(512) void embedding_norm_kernel(float* __restrict__ x, TO* __restrict__ h, const TE* __restrict__ table, const int* __restrict__ ids, float scale,
-                                                             const TW* __restrict__ w, float eps, int D, int V) {
-  constexpr int VPT = 4;
+// Threads of a row of the norm, which are the order of its sum too.  Few rows: many threads per row, so that a row's loads are
+// all in flight at once.
+static int norm_threads(int M, int D) { return (D >= 2048 && M <= 256) ? 1024 : (D >= 1024 ? 256 : (D >= 256 ? 128 : 64)); }
+// ... of the kernels with wide accesses: no more threads than groups of four
+static int norm_threads_wide(int M, int D) {
+  const int groups = D / 4, most = norm_threads(M, D);
+  return groups >= most ? most : ((groups + 63) / 64) * 64;
+}
+
+// The embedding of a step and the norm that reads it first: x as embedding_kernel makes it, h its RMS norm as rmsnorm_wide_kernel
+// makes it, to the same bits (the threads and the order of the sum are its own), a block to a token, in the place of two
+// kernels that little but start (8 tokens of 2,048: 6.2 + 4.6 us -> 4.4).
+template <typename TE, typename TO, typename TW, int VPT>
+__global__ __launch_bounds__(1024) void embedding_norm_kernel(float* __restrict__ x, TO* __restrict__ h, const TE* __restrict__ table, const int* __restrict__ ids, float scale,
+                                                              const TW* __restrict__ w, float eps, int D, int V) {
   __shared__ float scratch[16];
   const long t = blockIdx.x;
   const int id = ids[t], groups = D / 4;
@@ -269,8 +277,10 @@ extern "C" int pi_embedding_norm(float* x, void* h, int h_dtype, const void* tab
   PI_REQUIRE(T >= 0 && D > 0 && D % 4 == 0 && D <= 8192 && V > 0, "embedding and norm: bad sizes T=%d D=%d V=%d", T, D, V);
   PI_REQUIRE((uintptr_t)x % 16 == 0 && (uintptr_t)h % 16 == 0 && (uintptr_t)table % 16 == 0 && (uintptr_t)w % 16 == 0, "embedding and norm: tensors must be 16-byte aligned");
   if (T == 0) return 0;
-  const int threads = D >= 2048 ? 512 : D >= 1024 ? 256 : D >= 256 ? 128 : 64;
-#define GO(TE, TO, TW) hipLaunchKernelGGL((embedding_norm_kernel<TE, TO, TW>), dim3(T), dim3(threads), 0, stream, x, (TO*)h, (const TE*)table, ids, scale, (const TW*)w, eps, D, V)
+  const int threads = norm_threads_wide(T, D);
+  // groups of a thread: up to 2 for few rows, up to 8 for many
+#define GO_V(TE, TO, TW, VPT) hipLaunchKernelGGL((embedding_norm_kernel<TE, TO, TW, VPT>), dim3(T), dim3(threads), 0, stream, x, (TO*)h, (const TE*)table, ids, scale, (const TW*)w, eps, D, V)
+#define GO(TE, TO, TW) do { if (D <= 8 * threads) GO_V(TE, TO, TW, 2); else GO_V(TE, TO, TW, 8); } while (0)
 #define PICK(TE, TO) do { if (w_dtype == PI_F32) GO(TE, TO, float); else GO(TE, TO, bf16_t); } while (0)
   PI_REQUIRE((h_dtype == PI_F32 || h_dtype == PI_BF16) && (table_dtype == PI_F32 || table_dtype == PI_BF16) && (w_dtype == PI_F32 || w_dtype == PI_BF16),
              "embedding and norm: unsupported dtypes table=%d out=%d weight=%d", table_dtype, h_dtype, w_dtype);
@@ -280,6 +290,7 @@ extern "C" int pi_embedding_norm(float* x, void* h, int h_dtype, const void* tab
   else PICK(bf16_t, bf16_t);
 #undef PICK
 #undef GO
+#undef GO_V
   return pi_check_launch("embedding_norm");
 }
 
@@ -289,19 +300,16 @@ extern "C" int pi_rmsnorm(void* out, int out_dtype, float* x, const int* rows, c
   PI_REQUIRE(M >= 0 && D > 0, "rmsnorm: bad sizes M=%d D=%d", M, D);
   PI_REQUIRE(part == nullptr || (splits >= 1 && x_rows > 0), "rmsnorm: bad split description (%d splits, %ld rows)", splits, x_rows);
   if (M == 0) return 0;
-  // few rows: many threads per row, so that a row's loads are all in flight at once
-  int threads = (D >= 2048 && M <= 256) ? 1024 : (D >= 1024 ? 256 : (D >= 256 ? 128 : 64));
+  int threads = norm_threads(M, D);
   const long stride = x_rows * (long)D;
   // rows of whole 16-byte groups, at most 8 groups per thread: the kernel with wide accesses
-  // (no more threads than groups)
   bool wide = D % 4 == 0 && ((uintptr_t)x % 16 == 0) && ((uintptr_t)out % 16 == 0) && ((uintptr_t)w % 16 == 0) &&
               (part == nullptr || (uintptr_t)part % 16 == 0);
   int per_thread = 0;
   if (wide) {
-    const int groups = D / 4, most = threads;
-    threads = groups >= most ? most : ((groups + 63) / 64) * 64;
-    per_thread = (groups + threads - 1) / threads;
-    if (per_thread > 8) { wide = false; threads = most; }
+    threads = norm_threads_wide(M, D);
+    per_thread = (D / 4 + threads - 1) / threads;
+    if (per_thread > 8) { wide = false; threads = norm_threads(M, D); }
   }
 #define WIDE(TO, TW, V) \
   hipLaunchKernelGGL((rmsnorm_wide_kernel<TO, TW, V>), dim3(M), dim3(threads), 0, stream, (TO*)out, x, rows, (const TW*)w, eps, D, part, splits, stride)

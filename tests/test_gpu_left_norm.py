@@ -153,6 +153,23 @@ def test_embedding_and_its_norm_in_one_kernel(ops, T, D, table_dtype, w_dtype, h
     assert not ops.embedding_norm(torch.empty(1, 30, device=DEV), torch.zeros(4, 30, device=DEV), ids[:1] * 0, 1.0, torch.ones(30, device=DEV), 1e-5, F32, ws)
 
 
+@pytest.mark.parametrize("T,D,table_dtype,w_dtype,h_dtype", [(1, 64, BF16, BF16, BF16), (3, 1000, BF16, F32, BF16), (5, 1024, F32, F32, F32), (8, 3072, BF16, BF16, BF16),
+                                                           (17, 8192, BF16, BF16, BF16), (256, 4096, BF16, BF16, BF16), (257, 4096, F32, F32, F32),
+                                                           (257, 2048, BF16, BF16, BF16), (300, 2052, F32, BF16, BF16), (257, 8192, BF16, F32, F32)])
+def test_embedding_and_its_norm_have_the_bits_of_the_two_kernels(ops, T, D, table_dtype, w_dtype, h_dtype):
+    """At both sides of every change in the norm's threads: a step's results do not hang on which kernels made its first norm."""
+    g = gen(T + D)
+    table = torch.randn(50, D, generator=g, device=DEV).to(table_dtype)
+    weight = (torch.rand(D, generator=g, device=DEV) + 0.5).to(w_dtype)
+    ids = torch.randint(0, 50, (T,), generator=g, device=DEV).to(torch.int32)
+    for scale in (1.0, 3.7):
+        x, plain, ws, want = torch.empty(T, D, device=DEV), torch.empty(T, D, device=DEV), ops.KernelWorkspace(DEV), torch.empty(T, D, dtype=h_dtype, device=DEV)
+        assert ops.embedding_norm(x, table, ids, scale, weight, 1e-5, h_dtype, ws)
+        ops.embedding(plain, table, ids, scale)
+        ops.rmsnorm(want, plain, weight, 1e-5)
+        assert torch.equal(x, plain) and torch.equal(ws.take_left_norm(x, weight, 1e-5).h, want)
+
+
 @pytest.mark.parametrize("M,D,I", [(1, 128, 512), (8, 2048, 1024), (9, 256, 1024), (16, 3072, 576)])
 def test_a_clamped_feed_forward_in_two_kernels(ops, M, D, I):
     g = gen(D + I)
