@@ -181,10 +181,6 @@ def build_module(module: str, force: bool = False, quiet: bool = False) -> str:
         compile_flags = compile_flags + python_embed_flags()[0]
         link_libs = python_embed_flags()[1]
     bdir = _build_dir()
-    if module == "launch":
-        compile_flags = compile_flags + [python_embed_flags()[0][0], "-I", bdir]
-        with open(os.path.join(bdir, "launch_entries.inc"), "w") as f:
-            f.write(signatures.launch_table())
     sources = MODULES[module]
     missing = [s for s in sources if not os.path.isfile(os.path.join(CSRC_DIR, s))]
     if missing:
@@ -202,7 +198,15 @@ def build_module(module: str, force: bool = False, quiet: bool = False) -> str:
     if not quiet:
         hb.start()
     objs = []
+    table_dir = None
+    stamp = source_hash(module)           # before anything is read for the build: a change on the way makes the library stale, not current
     try:
+        if module == "launch":            # in a folder of this build's own: another process may be building from another table
+            table_dir = tempfile.mkdtemp(prefix=f"{module}.{os.getpid()}.", dir=bdir)
+            with open(os.path.join(table_dir, "launch_entries.inc"), "w") as f:
+                f.write(signatures.launch_table())
+            compile_flags = compile_flags + [python_embed_flags()[0][0], "-I", table_dir]
+
         def compile_one(src: str) -> str:
             obj = os.path.join(bdir, f"{module}_{os.path.splitext(os.path.basename(src))[0]}.{os.getpid()}.o")
             base = [hipcc, *compile_flags, "-I", CSRC_DIR, "-c", os.path.join(CSRC_DIR, src), "-o", obj]
@@ -224,9 +228,11 @@ def build_module(module: str, force: bool = False, quiet: bool = False) -> str:
         _run([hipcc, *link_flags, *objs, *link_libs, "-o", tmp], f"libphoton_{module}.so")
         os.replace(tmp, lib)
         with open(lib + ".hash", "w") as f:
-            f.write(source_hash(module))
+            f.write(stamp)
     finally:
         done.set()
+        if table_dir is not None:
+            shutil.rmtree(table_dir, ignore_errors=True)
         for o in objs:
             try:
                 os.remove(o)

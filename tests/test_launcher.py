@@ -1,12 +1,16 @@
 """The interpreter's way to the kernel libraries' entry points (csrc/runtime/launch.cpp): argument types as the entry points
 have them, errors as the binding has them.  The entry points here refuse their sizes before they touch a device."""
 import ctypes
+import importlib.machinery
+import importlib.util
+import os
+import shutil
 import threading
 
 import pytest
 
 from photon_infer_amd.errors import KernelError
-from photon_infer_amd.ops import _lib, signatures
+from photon_infer_amd.ops import _lib, build, signatures
 
 
 def bound(name, argtypes, function):
@@ -67,3 +71,43 @@ def test_every_entry_point_is_in_the_launchers_table_and_threads_keep_their_mess
     for t in threads:
         t.join()
     assert all(f"M=-{i} D" in seen[i] for i in range(1, 9)), seen
+
+
+def loaded(path):
+    loader = importlib.machinery.ExtensionFileLoader("photon_launch", path)
+    module = importlib.util.module_from_spec(importlib.util.spec_from_file_location("photon_launch", path, loader=loader))
+    loader.exec_module(module)
+    return module
+
+
+@pytest.fixture
+def own_csrc(tmp_path, monkeypatch):
+    """A copy of the launcher's source to build in."""
+    os.makedirs(tmp_path / "csrc" / "runtime")
+    shutil.copy(os.path.join(build.CSRC_DIR, "runtime", "launch.cpp"), tmp_path / "csrc" / "runtime")
+    monkeypatch.setattr(build, "CSRC_DIR", str(tmp_path / "csrc"))
+    return tmp_path
+
+
+def test_a_build_beside_another_compiles_its_own_table(own_csrc, monkeypatch):
+    """Another process with a shorter table builds from start to end while this one is about to compile: the library that
+    counts as current afterwards holds the entry points of the table that its stamp was made from."""
+    run, whole, nested = build._run, dict(signatures.SIGNATURES), []
+
+    def run_with_a_neighbour(cmd, what):
+        if what == "runtime/launch.cpp" and not nested:
+            nested.append(True)
+            monkeypatch.setattr(signatures, "SIGNATURES", {"core": {"pi_rmsnorm": whole["core"]["pi_rmsnorm"]}})
+            build.build_module("launch", force=True, quiet=True)
+            monkeypatch.setattr(signatures, "SIGNATURES", whole)
+        return run(cmd, what)
+
+    monkeypatch.setattr(build, "_run", run_with_a_neighbour)
+    path = build.build_module("launch", quiet=True)
+    assert nested and build.is_current("launch")
+    launcher = loaded(path)
+    for entries in whole.values():
+        for name in entries:
+            assert callable(launcher.bind(name, 1)), name
+    left = sorted(os.listdir(os.path.dirname(path)))
+    assert left == sorted([os.path.basename(path), os.path.basename(path) + ".hash"]), left
