@@ -13,6 +13,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 import tempfile
 import threading
 import time
@@ -103,7 +104,6 @@ def _host_compiler() -> str:
 
 def python_embed_flags():
     """(compile flags, link flags) for a program or library that hosts this interpreter."""
-    import sysconfig
     inc = sysconfig.get_paths()["include"]
     libdir = sysconfig.get_config_var("LIBDIR") or "/usr/lib"
     version = sysconfig.get_config_var("LDVERSION") or sysconfig.get_python_version()
@@ -139,8 +139,15 @@ def source_hash(module: str) -> str:
     return h.hexdigest()
 
 
+def interpreter_tag() -> str:
+    """The binary interface of this interpreter's extensions, as extension file names carry it."""
+    return sysconfig.get_config_var("SOABI") or f"{sys.implementation.cache_tag}-{sysconfig.get_platform()}"
+
+
 def library_path(module: str) -> str:
     tag = os.environ.get("PHOTON_SANITIZE", "").strip().replace(",", "-") if module in HOST_MODULES else ""
+    if module == "launch":                # an extension of the interpreter: each kind of interpreter has its own
+        tag = interpreter_tag() + ("." + tag if tag else "")
     return os.path.join(_build_dir(), f"libphoton_{module}{'.' + tag if tag else ''}.so")
 
 

@@ -111,3 +111,15 @@ def test_a_build_beside_another_compiles_its_own_table(own_csrc, monkeypatch):
             assert callable(launcher.bind(name, 1)), name
     left = sorted(os.listdir(os.path.dirname(path)))
     assert left == sorted([os.path.basename(path), os.path.basename(path) + ".hash"]), left
+
+
+def test_each_interpreter_has_a_launcher_of_its_own(own_csrc, monkeypatch):
+    """An extension built for one interpreter is never what another one finds current."""
+    path = build.build_module("launch", quiet=True)
+    assert build.is_current("launch") and build.interpreter_tag() in os.path.basename(path)
+    config = build.sysconfig.get_config_var
+    monkeypatch.setattr(build.sysconfig, "get_config_var", lambda name: "cpython-399-x86_64-linux-gnu" if name == "SOABI" else config(name))
+    assert build.library_path("launch") != path and not build.is_current("launch")
+    monkeypatch.setattr(build.sysconfig, "get_config_var", lambda name: None if name == "SOABI" else config(name))
+    assert build.library_path("launch") != path and not build.is_current("launch")
+    assert build.library_path("core") == os.path.join(build.CSRC_DIR, "_build", "libphoton_core.so")
