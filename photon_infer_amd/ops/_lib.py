@@ -1,9 +1,11 @@
-"""ctypes binding of the kernel libraries.  Loading fails loudly; nothing falls back."""
+"""Binding of the kernel libraries: the launcher's builtins, or ctypes where the launcher cannot be built.  Loading a kernel
+library fails loudly; no kernel has a substitute."""
 from __future__ import annotations
 
 import ctypes
 import importlib.machinery
 import importlib.util
+import sys
 from ctypes import c_double, c_float, c_int, c_long, c_void_p
 from typing import Dict
 
@@ -64,24 +66,35 @@ def load(module: str) -> ctypes.CDLL:
 
 
 _ENTRIES: Dict[str, object] = {}      # entry points called before, by name (names are unique over the modules)
-_LAUNCHER = None
+_LAUNCHER = None                      # the launcher, or False: there is none for this interpreter
+
+
+def _load_launcher():
+    try:
+        path = build.build_module("launch")
+        loader = importlib.machinery.ExtensionFileLoader("photon_launch", path)
+        launcher = importlib.util.module_from_spec(importlib.util.spec_from_file_location("photon_launch", path, loader=loader))
+        loader.exec_module(launcher)
+        return launcher
+    except (KernelLibraryMissing, ImportError) as e:      # no compiler, or not this interpreter's headers
+        print(f"[photon_infer_amd] no launcher: kernels are called through ctypes, some 2 us slower each ({str(e).strip().splitlines()[0]})", file=sys.stderr, flush=True)
+        return False
 
 
 def _bound(module: str, name: str):
     """The entry point as a builtin of the launcher, an extension of the interpreter whose functions turn their arguments
     into the entry point's types by themselves: a call of thirteen arguments costs 0.3 us so and 2.4 through ctypes, and
-    a step that is not a replayed graph makes some 130 of them."""
+    a step that is not a replayed graph makes some 130 of them.  Where the launcher cannot be built, ctypes' function."""
     global _LAUNCHER
     if _LAUNCHER is None:
-        path = build.build_module("launch")
-        try:
-            loader = importlib.machinery.ExtensionFileLoader("photon_launch", path)
-            launcher = importlib.util.module_from_spec(importlib.util.spec_from_file_location("photon_launch", path, loader=loader))
-            loader.exec_module(launcher)
-        except ImportError as e:
-            raise KernelLibraryMissing(f"cannot load the launcher {path}: {e}") from e
-        _LAUNCHER = launcher
-    return _LAUNCHER.bind(name, ctypes.cast(getattr(load(module), name), c_void_p).value)
+        _LAUNCHER = _load_launcher()
+    entry = getattr(load(module), name)
+    if _LAUNCHER is False:
+        return entry
+    try:
+        return _LAUNCHER.bind(name, ctypes.cast(entry, c_void_p).value)
+    except KeyError as e:
+        raise KernelLibraryMissing(f"the launcher {_LAUNCHER.__file__} lacks entry point {name}") from e
 
 
 def call(module: str, name: str, *args) -> None:

@@ -9,7 +9,7 @@ import threading
 
 import pytest
 
-from photon_infer_amd.errors import KernelError
+from photon_infer_amd.errors import KernelError, KernelLibraryMissing
 from photon_infer_amd.ops import _lib, build, signatures
 
 
@@ -123,3 +123,29 @@ def test_each_interpreter_has_a_launcher_of_its_own(own_csrc, monkeypatch):
     monkeypatch.setattr(build.sysconfig, "get_config_var", lambda name: None if name == "SOABI" else config(name))
     assert build.library_path("launch") != path and not build.is_current("launch")
     assert build.library_path("core") == os.path.join(build.CSRC_DIR, "_build", "libphoton_core.so")
+
+
+@pytest.fixture
+def unbound(monkeypatch):
+    """The binding as it is before the first call."""
+    monkeypatch.setattr(_lib, "_LAUNCHER", None)
+    monkeypatch.setattr(_lib, "_ENTRIES", {})
+
+
+def test_without_the_interpreters_headers_kernels_are_called_through_ctypes(own_csrc, unbound, monkeypatch, capfd):
+    _lib.load("core")                                    # a kernel library that is there
+    monkeypatch.setattr(build, "python_embed_flags", lambda: (["-I/nonexistent"], []))
+    monkeypatch.setattr(build, "HOST_FLAGS", build.HOST_FLAGS + ["-nostdinc"])       # whatever the system's own folders hold
+    for _ in range(3):
+        with pytest.raises(KernelError, match="rmsnorm: bad sizes M=-1 D=5"):
+            _lib.call("core", "pi_rmsnorm", None, 0, None, None, None, 0, 1e-5, -1, 5, None, 0, 0, 0)
+    _lib.call("core", "pi_softcap", 0, 0, 1.0, None)
+    assert capfd.readouterr().err.count("no launcher") == 1
+
+
+def test_a_launcher_that_lacks_an_entry_point_is_a_missing_library(own_csrc, unbound, monkeypatch):
+    whole = signatures.SIGNATURES
+    _lib.load("core")
+    monkeypatch.setattr(signatures, "SIGNATURES", {"core": {"pi_rmsnorm": whole["core"]["pi_rmsnorm"]}})
+    with pytest.raises(KernelLibraryMissing, match="pi_softcap"):
+        _lib.call("core", "pi_softcap", 0, 0, 1.0, None)
