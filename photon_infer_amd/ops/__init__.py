@@ -66,6 +66,12 @@ def _stream() -> int:
     return _lib.current_stream()
 
 
+def _changes(x: Optional[torch.Tensor]) -> None:
+    """For kernels that write ``x`` in place: a norm that was left of the stream before is not one of the stream after."""
+    if x is not None:
+        torch.autograd.graph.increment_version(x)
+
+
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
@@ -220,6 +226,8 @@ def whole_norm(h):
     from its stream, which must be as the norm's maker left it."""
     if not isinstance(h, LeftNorm):
         return h
+    if h.stale:
+        raise KernelError("a norm that was left to its reader cannot be made any more: its stream has been written since")
     out = torch.empty_like(h.h)
     rmsnorm(out, h.x, h.weight, h.eps)
     return out
@@ -303,6 +311,8 @@ def gemm(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, accumulate: bool =
             if out.dtype != torch.float32:
                 raise KernelError("gemm: accumulation needs a float32 output")
             materialize(out, ws)
+            if ws is None:
+                _changes(out)
         if _FAST and fast.gemm_from_ranges(out, a, w, accumulate, w.shape[0], _rows(w, "gemm w"), _rows(out, "gemm out"),
                                            may_defer and out.dtype == torch.float32 and out.is_contiguous(), ws, next_norm):
             return
@@ -323,6 +333,8 @@ def gemm(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, accumulate: bool =
         return
     if accumulate:
         materialize(out, ws)
+        if ws is None:
+            _changes(out)
     if _FAST and a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16:
         may_defer_ = may_defer and out.dtype == torch.float32 and out.is_contiguous()
         if fast.gemm(out, a, w, accumulate, M, N, K, lda, ldw, ldc, may_defer_, ws, left, next_norm, whole):
@@ -699,6 +711,7 @@ def sandwich_norm_add(x: torch.Tensor, a: torch.Tensor, post, eps: float, nxt=No
     _lib.call("core", "pi_sandwich_norm_add", x.data_ptr(), _ptr(h), _dt(h) if h is not None else PI_F32, a.data_ptr(), _ptr(a_bias),
               _ptr(w_a), _ptr(b), _ptr(w_b), post[0].data_ptr(), post[1].data_ptr(), _ptr(nxt[0]) if nxt is not None else None,
               _ptr(nxt[1]) if nxt is not None else None, float(eps), T, D, _stream())
+    _changes(x)
     return h
 
 
@@ -754,6 +767,8 @@ def rms_join(x: torch.Tensor, y: torch.Tensor, post: torch.Tensor, post_eps: flo
     _lib.call("core", "pi_rms_join", x.data_ptr(), _ptr(h), _dt(h) if h is not None else PI_F32, _ptr(a), pieces.part.data_ptr() if pieces is not None else None,
               pieces.splits if pieces is not None else 0, _ptr(entry_row), _ptr(weights), top, entries, _ptr(rows), M, post.data_ptr(), float(post_eps),
               _ptr(nxt), float(next_eps), T, D, _stream())
+    if rows is None:
+        _changes(x)
     return h
 
 
@@ -837,6 +852,7 @@ def branch_norm_add(x: torch.Tensor, a: torch.Tensor, w_outer: torch.Tensor, eps
         h = torch.empty((T, D), dtype=h_dtype, device=x.device)
     _lib.call("core", "pi_branch_norm_add", x.data_ptr(), _ptr(h), _dt(h) if h is not None else PI_F32, a.data_ptr(), _ptr(w_a),
               _ptr(b), _ptr(w_b), w_outer.data_ptr(), float(eps), float(mult), T, D, _stream())
+    _changes(x)
     if h_dtype is None:
         return None
     return x if h is None else h
@@ -1264,6 +1280,7 @@ def combine_choices(out: torch.Tensor, y: torch.Tensor, weights: Optional[torch.
         raise KernelError("combine: one float32 weight per entry is needed")
     _lib.call("core", "pi_combine_choices", out.data_ptr(), y.data_ptr(), _ptr(weights), rows.entry_row.data_ptr(), T, rows.top, D,
               int(bool(accumulate)), _ptr(ids), int(num_real), _ptr(h), _dt(h) if h is not None else PI_F32, _stream())
+    _changes(out)
 
 
 # ----------------------------------------------------------------------------- mixers with a state of fixed size
@@ -1459,6 +1476,7 @@ def clamped_glu(out: torch.Tensor, gate_up: torch.Tensor, gate_bias: Optional[to
     _lib.call("core", "pi_clamped_glu", out.data_ptr(), _dt(out), gate_up.data_ptr(), _dt(gate_up), gate_bias.data_ptr(),
               _ptr(up_bias), _ptr(x_bias) if x is not None else None, _dt(gate_bias), float(limit), float(alpha), T, I,
               _ptr(x), D, int(block), _stream())
+    _changes(x)
 
 
 def add_row_bias(x: torch.Tensor, bias: torch.Tensor) -> None:
@@ -1469,6 +1487,7 @@ def add_row_bias(x: torch.Tensor, bias: torch.Tensor) -> None:
         raise KernelError(f"row bias: expected a contiguous float32 stream [{T}, {D}] and a float32 bias [{D}]")
     _lib.call("core", "pi_clamped_glu", None, PI_F32, None, PI_F32, None, None, bias.data_ptr(), PI_F32, 0.0, 0.0, T, 0,
               x.data_ptr(), D, 0, _stream())
+    _changes(x)
 
 
 def gemm_clamped_glu(out: torch.Tensor, a: torch.Tensor, w_gate_up: torch.Tensor, bias: torch.Tensor, limit: float, alpha: float,
@@ -1574,6 +1593,8 @@ def hyper_streams(x: torch.Tensor, *, y: Optional[torch.Tensor] = None, post: Op
               float(eps), _ptr(rows), M, _ptr(shift), _ptr(state), state.stride(0) if state is not None else 0, state.shape[0] if state is not None else 0,
               _ptr(ctx.slots) if shift is not None else None,
               _ptr(ctx.req_of_token) if shift is not None else None, int(bool(getattr(ctx, "all_decode", False))) if shift is not None else 0, _stream())
+    if y is not None and rows is None:
+        _changes(x)
     return h
 
 

@@ -65,12 +65,17 @@ class PendingUpdate:
         return t is x or (t.data_ptr() == x.data_ptr() and t.shape == x.shape and t.stride() == x.stride())
 
 
+def _version_of(x: torch.Tensor) -> Optional[int]:
+    return None if x.is_inference() else x._version       # (tensors made in inference mode count no versions)
+
+
 @dataclass
 class LeftNorm:
     """The norm of a stream ``x`` [M, D] that the product before it made but for the root (``ops.gemm`` with ``next_norm``):
     ``h`` holds bfloat16(x * weight), ``sums`` float32 [M, count] every row's sum of x^2 in pieces.  A product that takes it
-    as activations multiplies its float32 rows by 1 / sqrt(sum / D + eps).  Good until ``x`` changes or is freed.  ``count``
-    0: ``h`` is the norm itself, whole."""
+    as activations multiplies its float32 rows by 1 / sqrt(sum / D + eps).  Good until ``x`` changes: whoever writes a stream in
+    place raises the tensor's version (torch's own operations do, ``ops._changes`` for the kernels).  ``count`` 0: ``h`` is
+    the norm itself, whole."""
 
     x: torch.Tensor
     weight: torch.Tensor
@@ -78,6 +83,14 @@ class LeftNorm:
     h: torch.Tensor
     sums: Optional[torch.Tensor]
     count: int
+
+    def __post_init__(self):
+        self.version = _version_of(self.x)
+
+    @property
+    def stale(self) -> bool:
+        """The stream has been written since."""
+        return _version_of(self.x) != self.version
 
     @property
     def shape(self):
@@ -196,9 +209,9 @@ class KernelWorkspace:
         return w.dim() == 2 and self.stream_copy_of(w, w.shape[0], w.shape[1]) is not None
 
     def take_left_norm(self, x: torch.Tensor, weight: torch.Tensor, eps: float) -> Optional[LeftNorm]:
-        """What is left of the norm of ``x`` with these parameters, if a product has made it."""
+        """What is left of the norm of ``x`` with these parameters, if a product has made it and ``x`` is as it was then."""
         left, self.left_norm = self.left_norm, None
-        return left if left is not None and left.x is x and left.weight is weight and left.eps == eps else None
+        return left if left is not None and left.x is x and left.weight is weight and left.eps == eps and not left.stale else None
 
     def take_pending(self, x: torch.Tensor) -> Optional[Partials]:
         """The pieces still to be added to ``x``, if any; they are the caller's to add."""

@@ -278,3 +278,27 @@ def test_a_models_decode_steps_leave_their_norms(tmp_path, batch):
     assert counts["norms_left"] == 0
     # three layers of bfloat16 activations: their roundings, not their sizes, differ
     assert (eager - whole).norm() <= 0.02 * whole.norm()
+
+
+def test_every_kernel_that_writes_a_stream_takes_its_norm_back(ops):
+    """Behind an update that left its norm, whatever else changes the stream in place, with the workspace or without."""
+    D, I = 256, 64
+    vec, res = torch.ones(D, device=DEV), lambda: torch.randn(3, D, device=DEV)
+    experts = ops.group_entries(torch.tensor([[0, 1], [1, 0], [0, 1]], dtype=torch.int32, device=DEV), 2)
+    a, w = torch.ones(3, 64, dtype=BF16, device=DEV), torch.ones(D, 64, dtype=BF16, device=DEV)
+    writers = {
+        "row bias": lambda x: ops.add_row_bias(x, vec),
+        "bias on the way": lambda x: ops.clamped_glu(torch.empty(3, I, dtype=BF16, device=DEV), torch.zeros(3, 2 * I, device=DEV), torch.zeros(I, device=DEV),
+                                                     torch.zeros(I, device=DEV), 7.0, 1.7, x, vec),
+        "product without the workspace": lambda x: ops.gemm(x, a, w, accumulate=True),
+        "branch": lambda x: ops.branch_norm_add(x, res(), vec, 1e-5, 1.0),
+        "sandwich": lambda x: ops.sandwich_norm_add(x, res(), (vec, vec), 1e-5),
+        "join": lambda x: ops.rms_join(x, res(), vec, 1e-5),
+        "experts": lambda x: ops.combine_choices(x, torch.randn(experts.rows, D, device=DEV), None, experts, accumulate=True),
+        "torch": lambda x: x.add_(1),
+    }
+    for name, write in writers.items():
+        ws, x, _, weight = made(ops, 3, D, 512)
+        assert ws.left_norm is not None, name
+        write(x)
+        assert ws.take_left_norm(x, weight, 1e-5) is None, name
