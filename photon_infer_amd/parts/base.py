@@ -157,9 +157,19 @@ class Part:
     nothing in Python from it.  Only then may a decode step be captured once as a HIP graph and
     replayed; one part without the promise makes the whole model step eagerly.  The default is
     False: a part has to say so.
+
+    What a class says of norms that are left to their reader (``leaves_root``, ``takes_left_norm``; a block's ``first_norm``
+    and ``opening_norm``) it says of its own ``forward``: a subclass with another ``forward`` says it again or does not.
     """
 
     graph_safe = False
+
+    def __init_subclass__(cls, **kwargs):
+        super().__init_subclass__(**kwargs)
+        if "forward" in cls.__dict__:
+            for name, nothing in (("leaves_root", False), ("takes_left_norm", False), ("first_norm", None), ("opening_norm", None)):
+                if name not in cls.__dict__:
+                    setattr(cls, name, nothing)
 
     def tensor_specs(self) -> List[TensorSpec]:
         return []

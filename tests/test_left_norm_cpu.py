@@ -33,3 +33,44 @@ def test_tensors_that_count_no_versions_keep_their_norms():
         left = left_in(ws, x, weight)
         ops._changes(x)                                  # not an error
         assert ws.take_left_norm(x, weight, 1e-5) is left
+
+
+def test_a_subclass_with_another_forward_makes_no_promise_by_inheritance():
+    """A norm, feed-forward or arrangement that wraps one of the framework's own works on tensors and finished streams,
+    as it does beside parts that leave nothing."""
+    from photon_infer_amd.parts.block import PreNormBlock
+    from photon_infer_amd.parts.mlp import SwiGLU
+    from photon_infer_amd.parts.norm import RMSNorm, norm_left_to
+
+    class DoubledNorm(RMSNorm):
+        def forward(self, x, ctx=None, rows=None):
+            return super().forward(x, ctx, rows) * 2
+
+    class RoundedMLP(SwiGLU):
+        def forward(self, h, x, ctx):
+            super().forward(h.round(), x, ctx)
+
+    class Same(RMSNorm):
+        pass
+
+    class ShiftedBlock(PreNormBlock):
+        def forward(self, x, ctx, cache):
+            super().forward(x.add_(2), ctx, cache)
+
+    class Says(RoundedMLP):
+        takes_left_norm = True
+
+        def forward(self, h, x, ctx):
+            SwiGLU.forward(self, h, x, ctx)
+
+    def norm(kind):
+        n = kind(8, 1e-5)
+        n.load({"weight": torch.ones(8, dtype=BF16)}, BF16, torch.device("cpu"))
+        return n
+
+    assert norm_left_to(norm(RMSNorm), SwiGLU(8, 16)) is not None and norm_left_to(norm(Same), SwiGLU(8, 16)) is not None
+    assert norm_left_to(norm(DoubledNorm), SwiGLU(8, 16)) is None and norm_left_to(norm(RMSNorm), RoundedMLP(8, 16)) is None
+    assert norm_left_to(norm(RMSNorm), Says(8, 16)) is not None
+    for kind, leaves in ((PreNormBlock, True), (ShiftedBlock, False)):
+        block = kind(("n.", norm(RMSNorm)), ("m.", SwiGLU(8, 16)))
+        assert (block.first_norm is not None) == leaves and (block.opening_norm is not None) == leaves, kind
