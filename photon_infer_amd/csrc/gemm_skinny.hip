@@ -732,14 +732,15 @@ extern "C" int pi_gemm_finish_ranges(float* X, const void* ranges, int heads, in
 }
 
 // C[M, N] = A[M, K] . W[N, K]^T for 1..16 tokens with all of k in a block, W the copy in the streaming order: stored in
-// bfloat16 or float32, added into float32, or through the gated unit (gate and up rows interleaved by 16).  `sums` (or null): A is
-// what pi_gemm_finish left of a norm; float32 [M, count], 16-byte aligned, K the norm's width.
+// bfloat16 or float32, added into float32, or through the gated unit (gate and up rows interleaved by 16).  `sums` (or null; not
+// with the sum): A is what pi_gemm_finish left of a norm; float32 [M, count], 16-byte aligned, K the norm's width.
 extern "C" int pi_gemm_rows(void* C, int epilogue, long ldc, const void* A, long lda, const void* W, int M, int N, int K, const float* sums, int count,
                             float eps, hipStream_t stream) {
   PI_REQUIRE(M > 0 && M <= 16 && N > 0 && N % 16 == 0 && K > 0 && K % KSTEP == 0, "gemm_rows: takes 1..16 tokens, N in 16 and K in 64, got M=%d N=%d K=%d", M, N, K);
   PI_REQUIRE(epilogue != EPI_SWIGLU || N % 32 == 0, "gemm_rows: the gated unit takes N (%d) in 32", N);
   PI_REQUIRE(lda >= K && lda % 8 == 0 && lda < RING_MAX_STRIDE && K < RING_MAX_STRIDE && ((uintptr_t)A % 16 == 0) && ((uintptr_t)W % 16 == 0), "gemm_rows: operands must be 16-byte aligned, the row stride (%ld) a multiple of 8", lda);
   PI_REQUIRE(!sums || (count > 0 && count <= 512 && count % 4 == 0 && (uintptr_t)sums % 16 == 0), "gemm_rows: a left norm has 4..512 sums a row, got %d", count);
+  PI_REQUIRE(!sums || epilogue != EPI_ACCUM, "gemm_rows: a sum does not take a left norm");
   // 16 rows to a block while the units take them in one round (3,072 x 2,048, 8 tokens 5.0 us and 6.0; 5,120 x 3,072 11.4 and 8.7)
   const int rows = epilogue == EPI_SWIGLU || (N / 16 > compute_units() && N % 32 == 0) ? 32 : 16;
   const LeftNorm left{sums, count, K, eps};
@@ -754,7 +755,10 @@ extern "C" int pi_gemm_rows(void* C, int epilogue, long ldc, const void* A, long
   switch (epilogue) {
     case EPI_BF16: PICK(EPI_BF16); break;
     case EPI_F32: PICK(EPI_F32); break;
-    case EPI_ACCUM: PICK(EPI_ACCUM); break;
+    case EPI_ACCUM:
+      if (rows == 32) GO(32, EPI_ACCUM, false);
+      else GO(16, EPI_ACCUM, false);
+      break;
     case EPI_SWIGLU:
       if (sums) GO(32, EPI_SWIGLU, true);
       else GO(32, EPI_SWIGLU, false);

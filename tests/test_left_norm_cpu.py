@@ -74,3 +74,11 @@ def test_a_subclass_with_another_forward_makes_no_promise_by_inheritance():
     for kind, leaves in ((PreNormBlock, True), (ShiftedBlock, False)):
         block = kind(("n.", norm(RMSNorm)), ("m.", SwiGLU(8, 16)))
         assert (block.first_norm is not None) == leaves and (block.opening_norm is not None) == leaves, kind
+
+
+def test_a_sum_does_not_take_a_left_norm():
+    """Refused before anything is launched: no kernel is compiled for it (``ops.gemm`` makes the whole norm there)."""
+    from photon_infer_amd.ops import _lib, fast
+    A = 1 << 20                                          # addresses that nobody reads
+    with pytest.raises(KernelError, match="does not take a left norm"):
+        _lib.call("bf16", "pi_gemm_rows", A, fast.EPI_ACCUM, 64, A, 64, A, 1, 64, 64, A, 8, 1e-5, None)
