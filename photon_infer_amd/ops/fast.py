@@ -164,6 +164,8 @@ def _rows(out_ptr: int, epilogue: int, ldc: int, a, w, M, N, K, lda, ldw, ws: Op
         return False
     _lib.call("bf16", "pi_gemm_rows", out_ptr, epilogue, ldc, a.data_ptr(), lda, w_ptr, M, N, K, None if left is None else left.sums.data_ptr(),
               0 if left is None else left.count, 0.0 if left is None else left.eps, _stream())
+    if left is not None:
+        ws.counts["left_norms_read"] += 1
     return True
 
 
@@ -518,6 +520,8 @@ def clamped_mlp(x, act, a, w_gate_up, bias, limit, alpha, w_down, x_bias, next_n
     _lib.call("bf16", "pi_gemm_rows_clamped", act.data_ptr(), act.stride(0), a.data_ptr(), lda, w_ptr, M, 2 * I, K, bias.data_ptr(), float(limit), float(alpha),
               None if left is None else left.sums.data_ptr(), 0 if left is None else left.count, 0.0 if left is None else left.eps, _stream())
     ws.counts["gated_epilogues"] += 1
+    if left is not None:
+        ws.counts["left_norms_read"] += 1
     return _finish(x, act, w_down, M, N, I, act.stride(0), I, next_norm, ws, x_bias)
 
 

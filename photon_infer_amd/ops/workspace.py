@@ -130,7 +130,7 @@ def stream_layout(w: torch.Tensor) -> Optional[torch.Tensor]:
 class KernelWorkspace:
     """Buffers are made at first use and kept; ``counts`` says which paths a step took (tests
     read it: ``split_products``, ``deferred``, ``added_by_norm``, ``applied``, ``flushed``,
-    ``discarded``, ``qkv_pieces``, ``ranges_merged_by_product``, ``norms_left``).  ``counts`` is about the 16-bit
+    ``discarded``, ``qkv_pieces``, ``ranges_merged_by_product``, ``norms_left``, ``left_norms_read``).  ``counts`` is about the 16-bit
     products; ``float32_counts`` has the same entries for pieces of float32 products."""
 
     def __init__(self, device):

@@ -56,8 +56,10 @@ def test_finished_stream_and_left_norm_against_float64(ops, M, N, K, w_dtype):
     # its readers: a product in pieces of k and whole, float32 and bfloat16, and the gated unit
     norm = (x.double() / torch.sqrt(sums[:, None] / N + 1e-5)) * weight.double()
     g = gen(5)
-    for rows, k_pieces in ((96, True), (16384 if N <= 2048 else 1024, False)):
+    for rows in (96, 8224):              # 16 rows to a block, and 32
         w2 = (torch.randn(rows, N, generator=g, device=DEV) * N ** -0.5).to(BF16)
+        assert ws.add_stream_copy(w2)
+        ws.counts["left_norms_read"] = 0
         want2 = norm @ w2.double().t()
         size = (norm.abs() @ w2.double().abs().t())               # what the rounding of the activations may sum up to
         got = ops.qkv_projection(left, w2, F32, ws)
@@ -75,6 +77,99 @@ def test_finished_stream_and_left_norm_against_float64(ops, M, N, K, w_dtype):
             wanted = (torch.nn.functional.silu(z[:, :, 0]) * z[:, :, 1]).reshape(M, -1)
             slack = (1.1 * s[:, :, 0] * z[:, :, 1].abs() + s[:, :, 1] * z[:, :, 0].abs()).reshape(M, -1)
             assert ((unit.double() - wanted).abs() <= ROUND * (1.1 * slack + wanted.abs() + 1e-3)).all()
+        assert ws.counts["left_norms_read"] == 3, ws.counts
+
+
+@pytest.mark.parametrize("M", [1, 8, 16])
+@pytest.mark.parametrize("N,K,scale,eps", [(256, 512, 1e-3, 1e-5), (2048, 2048, 0.1, 0.5), (192, 1024, 1.0, 0.0)])
+def test_readers_apply_the_root_with_its_eps(ops, M, N, K, scale, eps):
+    """Streams whose mean square is small beside eps, of its size, and with no eps at all: a root without it, with another
+    one or of a mean over the pieces would be far off."""
+    g = gen(M + N)
+    a = (torch.randn(M, K, generator=g, device=DEV) * scale).to(BF16)
+    w = (torch.randn(N, K, generator=g, device=DEV) * K ** -0.5).to(BF16)
+    weight, ws = (torch.rand(N, generator=g, device=DEV) + 0.5).to(BF16), ops.KernelWorkspace(DEV)
+    w2 = (torch.randn(96, N, generator=g, device=DEV) * N ** -0.5).to(BF16)
+    assert ws.add_stream_copy(w) and ws.add_stream_copy(w2)
+    x = torch.randn(M, N, generator=g, device=DEV) * scale
+    ops.gemm(x, a, w, accumulate=True, may_defer=True, ws=ws, next_norm=(weight, eps))
+    left = ws.take_left_norm(x, weight, eps)
+    norm = x.double() / torch.sqrt((x.double() ** 2).mean(1, keepdim=True) + eps) * weight.double()
+    out = torch.empty(M, 96, device=DEV)
+    ops.gemm(out, left, w2, ws=ws)
+    assert ws.counts["left_norms_read"] == 1
+    assert ((out.double() - norm @ w2.double().t()).abs() <= ROUND * (norm.abs() @ w2.double().abs().t())).all()
+
+
+@pytest.mark.parametrize("M", [1, 9, 16])
+@pytest.mark.parametrize("N,K", [(16, 512), (64, 4096), (4112, 512), (8224, 576), (1024, 2048)])
+def test_all_of_k_in_a_block_where_the_caller_says_so(ops, M, N, K):
+    """In the place of pieces: stored in float32 and bfloat16, and added; 16 rows to a block and 32."""
+    from photon_infer_amd.ops import fast
+    g = gen(M + N + K)
+    a, w = torch.randn(M, K + 8, generator=g, device=DEV).to(BF16)[:, :K], (torch.randn(N, K, generator=g, device=DEV) * K ** -0.5).to(BF16)
+    ws = ops.KernelWorkspace(DEV)
+    assert ws.add_stream_copy(w) and fast._skinny_splits(M, N, K) > 1
+    want, size = a.double() @ w.double().t(), a.double().abs() @ w.double().abs().t()
+    slack = 2.0 ** -24 * (K / 64 + 8) * size              # float32 sums: a chain of K / 64 steps a wave at most, the waves' sums
+    x0 = torch.randn(M, N, generator=g, device=DEV)
+    f32, b16, x = torch.empty(M, N, device=DEV), torch.empty(M, N, dtype=BF16, device=DEV), x0.clone()
+    ops.gemm(f32, a, w, ws=ws, whole=True)
+    ops.gemm(b16, a, w, ws=ws, whole=True)
+    ops.gemm(x, a, w, accumulate=True, ws=ws, whole=True)
+    assert ws.counts["split_products"] == 0
+    assert ((f32.double() - want).abs() <= slack).all() and torch.equal(b16, f32.to(BF16))
+    assert ((x.double() - x0.double() - want).abs() <= slack + 2.0 ** -23 * (x0.double().abs() + want.abs())).all()
+
+
+@pytest.mark.parametrize("copies", [(True, True), (True, False), (False, True), (False, False)])
+def test_mixers_side_by_side_read_one_norm_of_the_stream_before(ops, copies):
+    """The second mixer reads its activations when the first has written the stream already: whichever of them can apply the
+    root, both see the norm of the stream before."""
+    from photon_infer_amd.parts import StepContext
+    from photon_infer_amd.parts.base import Mixer
+    from photon_infer_amd.parts.block import SideBySide
+    M, D, I = 5, 256, 512
+    g = gen(4)
+    rnd = lambda n, k: (torch.randn(n, k, generator=g, device=DEV) * k ** -0.5).to(BF16)
+
+    class Product(Mixer):
+        takes_left_norm = True
+
+        def __init__(self):
+            self.w_in, self.w_o = rnd(I, D), rnd(D, I) * 8           # a large update
+
+        def streamed_weights(self):
+            return [self.w_in, self.w_o]
+
+        def forward(self, h, x, ctx, cache):
+            y = torch.empty(M, I, dtype=BF16, device=DEV)
+            ops.gemm(y, h, self.w_in, ws=ctx.workspace)
+            ops.gemm(x, y, self.w_o, accumulate=True, may_defer=ctx.may_defer, ws=ctx.workspace, next_norm=ctx.next_norm)
+
+    ws, x, _, weight = made(ops, M, D, 512)
+    mixers = [Product(), Product()]
+    for m, copy in zip(mixers, copies):
+        ws.add_stream_copy(m.w_o)
+        if copy:
+            ws.add_stream_copy(m.w_in)
+    x0 = x.double()
+    norm = x0 / torch.sqrt((x0 ** 2).mean(1, keepdim=True) + 1e-5) * weight.double()
+    left = ws.take_left_norm(x, weight, 1e-5)
+    after = torch.ones(D, dtype=BF16, device=DEV)
+    i32 = torch.zeros(M, dtype=torch.int32, device=DEV)
+    ctx = StepContext(T=M, R=M, dtype=BF16, token_ids=i32, positions=i32, req_of_token=i32, q_start=i32, kv_len=i32, slots=i32, block_tables={}, logit_rows=i32,
+                      may_defer=True, next_norm=(after, 1e-5), workspace=ws)
+    SideBySide([("a.", mixers[0]), ("b.", mixers[1])]).forward(left, x, ctx, [None, None])
+    assert ws.counts["left_norms_read"] == (2 if all(copies) else 0) and ws.pending is None
+    ys = [norm @ m.w_in.double().t() for m in mixers]
+    want = x0 + sum(y @ m.w_o.double().t() for y, m in zip(ys, mixers))
+    # the activations are rounded twice on the way, each by ROUND of the terms that reach the next sum
+    sizes = [(norm.abs() @ m.w_in.double().abs().t() + y.abs()) @ m.w_o.double().abs().t() for y, m in zip(ys, mixers)]
+    assert ((x.double() - want).abs() <= ROUND * sum(sizes) + 1e-5 * want.abs()).all()
+    assert (sum(y @ m.w_o.double().t() for y, m in zip(ys, mixers))).norm() > 4 * x0.norm()
+    final = ws.take_left_norm(x, after, 1e-5)
+    assert torch.equal(final.h, x.to(BF16))
 
 
 @pytest.mark.parametrize("M,heads,head_dim,count,inside", [(1, 8, 64, 2, True), (1, 32, 64, 16, True), (1, 32, 64, 40, False), (3, 5, 128, 13, True), (2, 8, 80, 9, True), (7, 24, 128, 3, True),
@@ -123,7 +218,10 @@ def test_rows_that_are_not_finite_stay_by_themselves_and_zero_rows_keep_their_ep
     ops.gemm(x, a, w, accumulate=True, may_defer=True, ws=ws, next_norm=(weight, 1e-5))
     left = ws.take_left_norm(x, weight, 1e-5)
     out = torch.empty(M, 64, dtype=F32, device=DEV)
-    ops.gemm(out, left, (torch.randn(64, N, generator=g, device=DEV) * 0.05).to(BF16), ws=ws)
+    reader = (torch.randn(64, N, generator=g, device=DEV) * 0.05).to(BF16)
+    ws.add_stream_copy(reader)
+    ops.gemm(out, left, reader, ws=ws)
+    assert ws.counts["left_norms_read"] == 1
     good = [0, 1, 3, 4, 5, 7]
     assert torch.isfinite(x[good]).all() and torch.isfinite(out[good]).all() and (out[4] == 0).all()
     assert not torch.isfinite(x[2]).any() and torch.isnan(x[6]).all() and torch.isnan(out[2]).all() and torch.isnan(out[6]).all()
