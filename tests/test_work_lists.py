@@ -301,3 +301,35 @@ def test_waves_of_bounded_contexts_and_of_steps_that_do_not_know_their_lengths()
     assert fast._waves_or_ranges(bare, 2, 32, 8, 64, 3000, 0) == (1, 2, None) and fast._waves_or_ranges(ctx, 2, 40, 8, 64, 3000, 0) == (2, 1, None)
     for uneven in (False, True):
         assert fast._waves_or_ranges(ctx, 1, 64, 8, 64, 3000, 0, SimpleNamespace(singles_uneven=uneven)) == (1, 1 + uneven, None)
+
+
+@pytest.mark.parametrize("splits,R,made", [(1, 16, (1, 1)), (31, 1, (31, 1)), (32, 1, (16, 2)), (64, 1, (32, 2)), (15, 2, (15, 1)), (16, 2, (8, 2)), (2, 15, (2, 1)),
+                                           (2, 16, (1, 2)), (3, 16, (2, 2)), (4, 8, (2, 2)), (3, 10, (3, 1)), (8, 17, (8, 1))])
+def test_ranges_of_all_requests_from_which_on_two_waves_share_one(splits, R, made):
+    from photon_infer_amd.ops import fast
+    assert fast.decode_range_waves(splits, R) == made
+    assert made[0] * made[1] >= splits
+
+
+def test_key_ranges_of_float32_decode_steps():
+    """One range up to short buckets, then blocks that fill the chip, ranges that keep their keys, and no more than the merging
+    kernel takes; the same within a length bucket."""
+    from photon_infer_amd.ops import fast
+    ranges = fast.float32_decode_ranges
+    assert [ranges(1, 8, 64, n) for n in (1, 256, 257, 512, 513, 1024, 8192, 8193, 1 << 20)] == [1, 1, 4, 4, 8, 8, 64, 64, 64]
+    assert [ranges(R, 8, 64, 4000) for R in (1, 4, 5, 8, 16, 64, 128, 129, 1000)] == [32, 32, 25, 16, 8, 2, 1, 1, 1]
+    assert [ranges(R, 8, 128, 4000) for R in (1, 2, 3, 8, 64)] == [32, 32, 21, 8, 1]
+
+
+def test_products_that_the_finishing_kernel_takes():
+    """Sizes at the edges of its rules, of which the host side answers without a GPU (256 units)."""
+    from photon_infer_amd.ops import fast
+    blocks = lambda *a: fast._finish_blocks.__wrapped__(*a)
+    assert [blocks(M, 2048, 2048) for M in (0, 1, 16, 17)] == [0, 256, 256, 0]
+    assert [blocks(1, N, 2048) for N in (48, 64, 96, 3008, 3072, 8192, 8256)] == [0, 8, 0, 376, 192, 512, 0]
+    assert [blocks(1, 2048, K) for K in (32, 64, 96, 4096, 4160)] == [0, 256, 0, 256, 256]
+    assert [blocks(M, 2048, K) for M, K in ((12, 4160), (13, 4096), (13, 4160))] == [256, 256, 0] and blocks(16, 3072, 8192) == 192
+    ranges = lambda *a: fast._finish_ranges_blocks.__wrapped__(*a)
+    # M, N, heads, head size, ranges: at most 320 KB of them, 64 KB of LDS, blocks of 8 rows
+    assert [ranges(8, 2048, 32, 64, c) for c in (0, 1, 4, 5)] == [0, 256, 256, 0] and [ranges(1, 2048, 32, 64, c) for c in (37, 38)] == [256, 0]
+    assert [ranges(M, 1024, 48, 64, 1) for M in (8, 9)] == [128, 0] and ranges(1, 3072, 32, 64, 2) == 0 and ranges(1, 2048, 32, 60, 2) == 0
