@@ -232,13 +232,14 @@ static bool ring(const Shape& s, long ldx, long ldw, int tiled) {
 }
 
 // ------------------------------------------------------------------ 1..16 tokens, all of k in a block
-// Every fetch of gemm_rows_kernel with 8 or 16 rows a tile, four or eight waves: the weights' copy and the activations
-// through descriptors of a wave's own k.  A used fetch is the lane's row (token) and k; any other lies outside its descriptor.
+// Every fetch of gemm_rows_kernel with 8 or 16 rows a tile (8 where N is in 64), four or eight waves: the weights' copy and the
+// activations through descriptors of a wave's own k.  A used fetch is the lane's row (token) and k; any other lies outside its
+// descriptor.  Of many tiles the first two and the last two.
 static bool few_rows(const Shape& s, long lda) {
   for (int rows : {8, 16})
     for (int waves : {4, 8})
       for (int wide = rows == 16 || s.M > 8; wide < 2; ++wide)
-        for (long n0 = 0; n0 < s.N; n0 += rows)
+        for (long n0 = rows == 8 && s.N % 64 ? s.N : 0; n0 < s.N; n0 += s.N >= 512 && n0 == rows ? s.N - 3 * rows : rows)
           for (int wave = 0; wave < waves; ++wave) {
             const A::WaveRange r = A::wave_share(0, s.K, waves, wave);
             const int steps = r.k1 > r.k0 ? (r.k1 - r.k0) / 64 : 0;
@@ -340,7 +341,7 @@ static bool check(const Shape& s) {
     if (s.M <= 32 && !skinny(s, s.K, s.K, 1, 2, A::KSTEP)) return false;
     if (s.M <= 16 && !skinny(s, s.K, s.K, 1, 4, 4 * A::KSTEP)) return false;
     if (s.M > 32 && s.M <= 128 && !ring(s, s.K, s.K, 1)) return false;
-    if (s.M <= 16 && s.N % 64 == 0 && s.N < 2048 && (!few_rows(s, s.K) || !few_rows(s, s.K + 8))) return false;
+    if (s.M <= 16 && (!few_rows(s, s.K) || !few_rows(s, s.K + 8))) return false;
   }
   return true;
 }
