@@ -259,10 +259,10 @@ def gemm_swiglu(out: torch.Tensor, a: torch.Tensor, w_gate_up: torch.Tensor, blo
     operands and blocks of 16 the product and the activation are one kernel."""
     left = a if isinstance(a, LeftNorm) else None
     if left is not None:
-        if not (_FAST and block == 16 and w_gate_up.dtype == torch.bfloat16 and out.is_contiguous()):
-            left, a = None, whole_norm(a)
-        else:
+        if _FAST and block == 16 and out.dtype == torch.bfloat16 and out.is_contiguous() and w_gate_up.shape[0] % 32 == 0 and fast.applies_root(left, w_gate_up, ws):
             a = left.h
+        else:
+            left, a = None, whole_norm(a)
     _gpu(out, a, w_gate_up)
     M, I = out.shape
     if w_gate_up.shape[0] != 2 * I or a.shape != (M, w_gate_up.shape[1]) or out.dtype != a.dtype:
@@ -272,7 +272,6 @@ def gemm_swiglu(out: torch.Tensor, a: torch.Tensor, w_gate_up: torch.Tensor, blo
     if _FAST and block == 16 and a.dtype == torch.bfloat16 and w_gate_up.dtype == torch.bfloat16 and out.is_contiguous():
         if fast.gemm_swiglu(out, a, w_gate_up, M, 2 * I, a.shape[1], _rows(a, "gemm a"), _rows(w_gate_up, "gemm w"), ws, left):
             return
-        a = a if left is None else whole_norm(left)
     if _FAST and block == 16 and a.dtype == torch.float32 and w_gate_up.dtype == torch.float32 and out.is_contiguous():
         if fast.gemm_swiglu_float32(out, a, w_gate_up, M, 2 * I, a.shape[1], _rows(a, "gemm a"), _rows(w_gate_up, "gemm w")):
             return
@@ -297,7 +296,7 @@ def gemm(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, accumulate: bool =
     block instead where the weights have a streaming copy: other sums in another order than without one."""
     left = None
     if isinstance(a, LeftNorm):
-        if _FAST and w.dtype == torch.bfloat16 and not accumulate and not may_defer:
+        if _FAST and not accumulate and not may_defer and out.dtype in (torch.bfloat16, torch.float32) and fast.applies_root(a, w, ws):
             left, a = a, a.h
         else:
             a = whole_norm(a)
@@ -339,8 +338,6 @@ def gemm(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, accumulate: bool =
         may_defer_ = may_defer and out.dtype == torch.float32 and out.is_contiguous()
         if fast.gemm(out, a, w, accumulate, M, N, K, lda, ldw, ldc, may_defer_, ws, left, next_norm, whole):
             return
-    if left is not None:
-        a = whole_norm(left)
     if _FAST and a.dtype == torch.float32 and w.dtype == torch.float32 and out.dtype == torch.float32:
         if fast.gemm_float32(out, a, w, accumulate, M, N, K, lda, ldw, ldc, may_defer and out.is_contiguous(), ws):
             return
@@ -394,6 +391,8 @@ def qkv_projection(h: torch.Tensor, w_qkv: torch.Tensor, dtype: torch.dtype, ws:
     (``Partials``), which ``rope_kv_write`` sums on the fly so that the rotation sees float32
     values.  The pieces are good until the next product with the same workspace.  A result of bfloat16
     that is not split may come as one float32 piece too (``fast.keeps_float32``)."""
+    if isinstance(h, LeftNorm) and not (_FAST and fast.applies_root(h, w_qkv, ws)):
+        h = whole_norm(h)
     if _FAST and ws is not None and h.dtype == torch.bfloat16 and w_qkv.dtype == torch.bfloat16 and h.is_cuda:
         left = h if isinstance(h, LeftNorm) else None
         p = fast.gemm_pieces(h if left is None else left.h, w_qkv, ws, whole=dtype == torch.bfloat16, left=left)

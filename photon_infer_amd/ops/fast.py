@@ -156,6 +156,14 @@ def _streamed(ws: Optional[KernelWorkspace], w, N: int, K: int, ldw: int):
     return w.data_ptr(), 0
 
 
+def applies_root(left: LeftNorm, w, ws: Optional[KernelWorkspace]) -> bool:
+    """Whether a product of the norm that ``left`` stands for with ``w`` [N, K] is one that applies the root itself: ``_rows``
+    does, which reads the streaming copy.  For any other the norm is made whole, and the product takes its ordinary way."""
+    M, K = left.shape
+    return (ws is not None and w.dim() == 2 and w.dtype == torch.bfloat16 and M <= FEW_TOKENS and w.shape[1] == K and K < RING_MAX_STRIDE
+            and w.is_contiguous() and left.h.is_contiguous() and _gemm_ok(left.h, w, K, K, K) and ws.has_stream_copy(w))
+
+
 def _rows(out_ptr: int, epilogue: int, ldc: int, a, w, M, N, K, lda, ldw, ws: Optional[KernelWorkspace], left: Optional[LeftNorm] = None) -> bool:
     """A product of up to 16 tokens by the kernel whose blocks take all of k, which reads the weights' streaming copy: False, and
     nothing done, without one.  ``left``: what ``a`` is the ``h`` of."""
@@ -254,7 +262,7 @@ def gemm(out, a, w, accumulate, M, N, K, lda, ldw, ldc, may_defer=False, ws: Opt
     else:
         return False
     if left is not None:
-        return M <= FEW_TOKENS and _rows(out.data_ptr(), epilogue, ldc, a, w, M, N, K, lda, ldw, ws, left)
+        return _rows(out.data_ptr(), epilogue, ldc, a, w, M, N, K, lda, ldw, ws, left)
     may_defer = may_defer and ws is not None      # pieces can only wait in a workspace that outlives the call
     if M > SKINNY_MAX_ROWS:
         # few output tiles, long k: split k so that every compute unit has work; the pieces
@@ -448,7 +456,7 @@ def gemm_pieces(a, w, ws: Optional[KernelWorkspace], whole: bool = False, left: 
     p = None
     if left is not None:            # few tokens: one float32 piece, of memory of its own
         out = torch.empty((1, M, N), dtype=torch.float32, device=a.device)
-        return Partials(out, 1, M, N) if M <= FEW_TOKENS and _rows(out.data_ptr(), EPI_F32, N, a, w, M, N, K, lda, ldw, ws, left) else None
+        return Partials(out, 1, M, N) if _rows(out.data_ptr(), EPI_F32, N, a, w, M, N, K, lda, ldw, ws, left) else None
     if M > SKINNY_MAX_ROWS:
         # a prompt portion of a few hundred tokens has too few tiles for the chip: split k there
         # too, the consumer adds the pieces
@@ -487,7 +495,7 @@ def gemm_swiglu(out, a, w, M, N, K, lda, ldw, ws: Optional[KernelWorkspace] = No
     if not _gemm_ok(a, w, K, lda, ldw) or N % 32 or out.dtype != torch.bfloat16:
         return False
     if left is not None:
-        return M <= FEW_TOKENS and _rows(out.data_ptr(), EPI_SWIGLU, out.stride(0), a, w, M, N, K, lda, ldw, ws, left)
+        return _rows(out.data_ptr(), EPI_SWIGLU, out.stride(0), a, w, M, N, K, lda, ldw, ws, left)
     if M > SKINNY_MAX_ROWS:
         _lib.call("bf16", "pi_gemm_mfma", out.data_ptr(), EPI_SWIGLU, out.stride(0), a.data_ptr(), lda, w.data_ptr(), ldw,
                   M, N, K, 1, _tile_shape(M, N, K, 1), _stream())

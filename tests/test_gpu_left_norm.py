@@ -400,3 +400,32 @@ def test_every_kernel_that_writes_a_stream_takes_its_norm_back(ops):
         assert ws.left_norm is not None, name
         write(x)
         assert ws.take_left_norm(x, weight, 1e-5) is None, name
+
+
+@pytest.mark.parametrize("M", [1, 16])
+@pytest.mark.parametrize("rows", [96, 40, 2056])
+def test_readers_without_a_streaming_copy_take_their_ordinary_way(ops, M, rows):
+    """A matrix whose rows are no multiple of 16 has no copy, one that nobody named neither: the norm is made whole, and the
+    product is, to the bit and in pieces where it is cut, that of the whole norm."""
+    N = 512
+    ws, x, _, weight = made(ops, M, N, 1024)
+    left = ws.take_left_norm(x, weight, 1e-5)
+    whole = torch.empty(M, N, dtype=BF16, device=DEV)
+    ops.rmsnorm(whole, x, weight, 1e-5)
+    w2 = (torch.randn(rows, N, generator=gen(rows), device=DEV) * N ** -0.5).to(BF16)
+    for dtype in (F32, BF16):
+        made_, want = torch.empty(M, rows, dtype=dtype, device=DEV), torch.empty(M, rows, dtype=dtype, device=DEV)
+        ops.gemm(made_, left, w2, ws=ws)
+        cut = ws.counts["split_products"]
+        ops.gemm(want, whole, w2, ws=ws)
+        assert torch.equal(made_, want) and cut > 0 and ws.counts["split_products"] == 2 * cut
+        ws.counts["split_products"] = 0
+        pieces = [ops.qkv_projection(h, w2, dtype, ws) for h in (left, whole)]
+        assert all(isinstance(p, ops.Partials) and p.splits > 1 for p in pieces)
+        ws.counts["split_products"] = 0
+    if rows % 32 == 0:
+        unit, want = torch.empty(M, rows // 2, dtype=BF16, device=DEV), torch.empty(M, rows // 2, dtype=BF16, device=DEV)
+        ops.gemm_swiglu(unit, left, w2, 16, ws=ws)
+        ops.gemm_swiglu(want, whole, w2, 16, ws=ws)
+        assert torch.equal(unit, want)
+    assert ws.counts["left_norms_read"] == 0
