@@ -180,6 +180,9 @@ class PagedAttention(Mixer):
     def streamed_weights(self) -> List[torch.Tensor]:
         return [self.w_qkv, self.w_o]
 
+    def norm_readers(self) -> List[torch.Tensor]:
+        return [self.w_qkv]
+
     def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext, cache: LayerCache) -> None:
         T = h.shape[0]
         writes = self.own_kv and cache.writes

@@ -126,7 +126,7 @@ class StepContext:
     # a norm whose root is left to it (``ops.gemm(..., next_norm=...)``).
     next_norm: Any = None
     opening_norm: Any = None              # set by the model for the embedding: (weight, eps, dtype) of the norm that reads the stream first
-    after_block_norm: Any = None          # set by the model per block: the same for whoever reads the stream after this block
+    after_block_norm: Any = None          # set by the model per block: ``next_norm`` for whoever reads the stream after this block
     may_leave_choices: bool = False       # likewise: a routed feed-forward may leave its result as the experts' rows (``ops.LeftChoices``)
     after_block_consumes: bool = False    # set by the model per block: whoever reads the stream after this block adds pending pieces
     workspace: Any = None                 # the runner's ops.KernelWorkspace: scratch memory of the kernels
@@ -185,6 +185,11 @@ class Part:
         copy of each in the order the weight-streaming kernels read (``EngineOptions.stream_copies``);
         a part that names none loses nothing but that."""
         return []
+
+    def norm_readers(self) -> List[torch.Tensor]:
+        """Of a part that takes left norms: the matrices that multiply its activations.  A norm is left to it only where every
+        one of these products applies the root, which those with a streaming copy do."""
+        return self.streamed_weights()
 
 
 class Norm(Part):
@@ -255,7 +260,7 @@ class Block(Part):
 
     @property
     def first_norm(self):
-        """(weight, eps) of the norm that reads the stream first, when its root may be left to the norm's reader; else None."""
+        """(the norm that reads the stream first, the part that reads the norm), where the one may be left to the other; else None."""
         return None
 
     def mixers(self) -> List[Mixer]:

@@ -54,13 +54,16 @@ class SideBySide(Mixer):
     def streamed_weights(self) -> List[torch.Tensor]:
         return [w for _, m in self.branches for w in m.streamed_weights()]
 
+    def norm_readers(self) -> List[torch.Tensor]:
+        return [w for _, m in self.branches for w in m.norm_readers()]
+
     @property
     def takes_left_norm(self) -> bool:
         return all(getattr(m, "takes_left_norm", False) for _, m in self.branches)
 
     def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext, cache) -> None:
         caches = cache if isinstance(cache, (list, tuple)) else [cache]
-        if isinstance(h, ops.LeftNorm) and not all(ctx.workspace.has_stream_copy(w) for w in self.streamed_weights()):
+        if isinstance(h, ops.LeftNorm) and not all(ctx.workspace.has_stream_copy(w) for w in self.norm_readers()):
             h = ops.whole_norm(h)      # a product that cannot apply the root would make the norm of a stream that has changed
         may_defer, next_norm = ctx.may_defer, ctx.next_norm
         for i, ((_, m), c) in enumerate(zip(self.branches, caches)):
@@ -115,7 +118,7 @@ class PreNormBlock(Block):
 
     @property
     def first_norm(self):
-        return norm_left_to(self.norm1, self.mixer)
+        return self.norm1, self.mixer
 
     @property
     def opening_norm(self):
@@ -132,7 +135,7 @@ class PreNormBlock(Block):
             ctx.may_defer, ctx.next_norm = False, None
             return
         ctx.may_defer = bool(getattr(self.norm2, "consumes_deferred", False))
-        ctx.next_norm = norm_left_to(self.norm2, self.ffn) if ctx.T <= ops.FEW_TOKENS else None
+        ctx.next_norm = norm_left_to(self.norm2, self.ffn, ctx.workspace) if ctx.T <= ops.FEW_TOKENS else None
         self.mixer.forward(self.norm1.forward(x, ctx), x, ctx, cache)
         ctx.may_defer, ctx.next_norm = ctx.after_block_consumes, ctx.after_block_norm
         self.ffn.forward(self.norm2.forward(x, ctx), x, ctx)

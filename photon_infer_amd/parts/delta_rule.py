@@ -82,6 +82,9 @@ class ChannelDeltaRule(Mixer):
     def streamed_weights(self) -> List[torch.Tensor]:
         return [self.w_in, self.w_low, self.w_a2, self.w_g2, self.w_o]
 
+    def norm_readers(self) -> List[torch.Tensor]:
+        return [self.w_in, self.w_low]
+
     def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext, cache: LayerCache) -> None:
         T, ws, C = h.shape[0], ctx.workspace, self.channels
         f32 = lambda n: torch.empty((T, n), dtype=torch.float32, device=h.device)
@@ -155,6 +158,9 @@ class GatedDeltaRule(Mixer):
 
     def streamed_weights(self) -> List[torch.Tensor]:
         return [self.w_in, self.w_o]
+
+    def norm_readers(self) -> List[torch.Tensor]:
+        return [self.w_in]
 
     def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext, cache: LayerCache) -> None:
         T, ws, C, H = h.shape[0], ctx.workspace, self.channels, self.num_heads

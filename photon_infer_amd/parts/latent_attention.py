@@ -126,6 +126,9 @@ class LatentAttention(Mixer):
     def streamed_weights(self) -> List[torch.Tensor]:
         return [self.w_in, self.w_uq, self.w_o]
 
+    def norm_readers(self) -> List[torch.Tensor]:
+        return [self.w_in]
+
     def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext, cache: LayerCache) -> None:
         T, ws, H = h.shape[0], ctx.workspace, self.num_heads
         table = ctx.block_tables[cache.group]

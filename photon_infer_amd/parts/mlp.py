@@ -64,6 +64,9 @@ class SwiGLU(FeedForward):
     def streamed_weights(self) -> List[torch.Tensor]:
         return [self.w_gate_up, self.w_down]
 
+    def norm_readers(self) -> List[torch.Tensor]:
+        return [self.w_gate_up]
+
     def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext) -> None:
         act = torch.empty((h.shape[0], self.intermediate_size), dtype=self.dtype, device=h.device)
         ws = ctx.workspace if ctx is not None else None
@@ -124,6 +127,9 @@ class ClampedGLU(FeedForward):
 
     def streamed_weights(self) -> List[torch.Tensor]:
         return [self.w_gate_up, self.w_down]
+
+    def norm_readers(self) -> List[torch.Tensor]:
+        return [self.w_gate_up]
 
     def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext) -> None:
         ws = ctx.workspace if ctx is not None else None

@@ -167,10 +167,11 @@ class DecoderModel:
                 ops.materialize(x, ws)
             if i + 1 < len(order):
                 ctx.after_block_consumes = bool(self.blocks[order[i + 1].layer].reads_deferred)
-                ctx.after_block_norm = getattr(self.blocks[order[i + 1].layer], "first_norm", None) if few else None
+                following = getattr(self.blocks[order[i + 1].layer], "first_norm", None) if few else None
+                ctx.after_block_norm = norm_left_to(*following, ws) if following is not None else None
             else:                          # the final norm; or nobody (the pieces are then dropped unread)
                 ctx.after_block_consumes = not wanted or bool(getattr(self.final_norm, "consumes_deferred", False))
-                ctx.after_block_norm = norm_left_to(self.final_norm, self.head) if few and wanted and ctx.every_row else None
+                ctx.after_block_norm = norm_left_to(self.final_norm, self.head, ws) if few and wanted and ctx.every_row else None
             ctx.may_defer, ctx.next_norm = False, None
             block.forward(x, ctx, caches[i])
         ctx.may_defer = ctx.may_leave_choices = ctx.after_block_consumes = False

@@ -141,6 +141,9 @@ class SinkWindowAttention(Mixer):
     def streamed_weights(self) -> List[torch.Tensor]:
         return [self.w_in, self.w_o]
 
+    def norm_readers(self) -> List[torch.Tensor]:
+        return [self.w_in]
+
     def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext, cache: LayerCache) -> None:
         T, ws = h.shape[0], ctx.workspace
         table = ctx.block_tables[cache.group]

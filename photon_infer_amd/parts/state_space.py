@@ -65,6 +65,9 @@ class StateSpaceMixer(Mixer):
     def streamed_weights(self) -> List[torch.Tensor]:
         return [self.w_in, self.w_o]
 
+    def norm_readers(self) -> List[torch.Tensor]:
+        return [self.w_in]
+
     def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext, cache: LayerCache) -> None:
         T, ws, inner = h.shape[0], ctx.workspace, self.inner
         proj = torch.empty((T, self.proj_size), dtype=torch.float32, device=h.device)

@@ -68,11 +68,18 @@ def test_a_subclass_with_another_forward_makes_no_promise_by_inheritance():
         n.load({"weight": torch.ones(8, dtype=BF16)}, BF16, torch.device("cpu"))
         return n
 
-    assert norm_left_to(norm(RMSNorm), SwiGLU(8, 16)) is not None and norm_left_to(norm(Same), SwiGLU(8, 16)) is not None
-    assert norm_left_to(norm(DoubledNorm), SwiGLU(8, 16)) is None and norm_left_to(norm(RMSNorm), RoundedMLP(8, 16)) is None
-    assert norm_left_to(norm(RMSNorm), Says(8, 16)) is not None
+    def mlp(kind):
+        m = kind(64, 16)
+        m.w_gate_up = torch.zeros(32, 64, dtype=BF16)
+        assert ws.add_stream_copy(m.w_gate_up)
+        return m
+
+    ws = ops.KernelWorkspace("cpu")
+    assert norm_left_to(norm(RMSNorm), mlp(SwiGLU), ws) is not None and norm_left_to(norm(Same), mlp(SwiGLU), ws) is not None
+    assert norm_left_to(norm(DoubledNorm), mlp(SwiGLU), ws) is None and norm_left_to(norm(RMSNorm), mlp(RoundedMLP), ws) is None
+    assert norm_left_to(norm(RMSNorm), mlp(Says), ws) is not None
     for kind, leaves in ((PreNormBlock, True), (ShiftedBlock, False)):
-        block = kind(("n.", norm(RMSNorm)), ("m.", SwiGLU(8, 16)))
+        block = kind(("n.", norm(RMSNorm)), ("m.", SwiGLU(64, 16)))
         assert (block.first_norm is not None) == leaves and (block.opening_norm is not None) == leaves, kind
 
 
@@ -82,3 +89,36 @@ def test_a_sum_does_not_take_a_left_norm():
     A = 1 << 20                                          # addresses that nobody reads
     with pytest.raises(KernelError, match="does not take a left norm"):
         _lib.call("bf16", "pi_gemm_rows", A, fast.EPI_ACCUM, 64, A, 64, A, 1, 64, 64, A, 8, 1e-5, None)
+
+
+def test_a_norm_is_left_only_where_every_product_of_it_applies_the_root():
+    from photon_infer_amd.parts.block import SideBySide
+    from photon_infer_amd.parts.delta_rule import ChannelDeltaRule
+    from photon_infer_amd.parts.embedding import LMHead
+    from photon_infer_amd.parts.mlp import ClampedGLU, SwiGLU
+    from photon_infer_amd.parts.norm import RMSNorm, norm_left_to
+    n = RMSNorm(64, 1e-5)
+    n.load({"weight": torch.ones(64, dtype=BF16)}, BF16, torch.device("cpu"))
+    mat = lambda rows: torch.zeros(rows, 64, dtype=BF16)
+
+    def delta(rows, low):
+        d = ChannelDeltaRule(64, 4, 4, 16, 16, 4, 16, 16, 1e-5)
+        d.w_in, d.w_low = mat(rows), mat(low)
+        return d
+
+    def with_matrix(part, name, rows):
+        setattr(part, name, mat(rows))
+        return part
+
+    for make, fits in ((lambda: with_matrix(SwiGLU(64, 16), "w_gate_up", 32), True), (lambda: with_matrix(ClampedGLU(64, 16, 7.0), "w_gate_up", 32), True),
+                       (lambda: with_matrix(SwiGLU(64, 20), "w_gate_up", 40), False), (lambda: with_matrix(LMHead(32, 64, False), "weight", 32), True),
+                       (lambda: with_matrix(LMHead(33, 64, False), "weight", 33), False), (lambda: delta(208, 32), True), (lambda: delta(196, 32), False),
+                       (lambda: delta(208, 40), False), (lambda: SideBySide([("a.", delta(208, 32)), ("b.", delta(208, 32))]), True),
+                       (lambda: SideBySide([("a.", delta(208, 32)), ("b.", delta(196, 32))]), False)):
+        part = make()
+        for copies in (False, True):
+            ws = ops.KernelWorkspace("cpu")
+            for w in part.norm_readers() if copies else []:
+                ws.add_stream_copy(w)
+            assert (norm_left_to(n, part, ws) is not None) == (fits and copies), (type(part).__name__, copies)
+        assert norm_left_to(n, part, None) is None
