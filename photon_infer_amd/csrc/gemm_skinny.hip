@@ -560,8 +560,11 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_rows_kernel(void* __restrict_
     const int rec = rs.head_dim + 4;
     for (int quad = tid; quad < K / 4; quad += WAVES * 64) {
       const int head = quad * 4 / rs.head_dim, f0 = quad * 4 - head * rs.head_dim, piece = quad / 2;
-      merge_ranges<16>(rs.ranges + (long)head * rs.count * rec, (long)rs.heads * rs.count * rec, rs.count, rec, rs.head_dim, f0, 0, 1, M,
-                   [&](const int token, const uint2 packed) { merged[(piece * TOKENS + (token + piece) % TOKENS) * 2 + quad % 2] = packed; });
+      const float* base = rs.ranges + (long)head * rs.count * rec;
+      const long token_stride = (long)rs.heads * rs.count * rec;
+      auto store = [&](const int token, const uint2 packed) { merged[(piece * TOKENS + (token + piece) % TOKENS) * 2 + quad % 2] = packed; };
+      if (rs.count <= 4) merge_ranges_of_tokens<4, 4>(base, token_stride, rs.count, rec, rs.head_dim, f0, 0, 1, M, store);
+      else merge_ranges_of_tokens<8, 1>(base, token_stride, rs.count, rec, rs.head_dim, f0, 0, 1, M, store);      // up to FINISH_RANGES
     }
     __syncthreads();
   }
@@ -688,17 +691,19 @@ extern "C" int pi_gemm_finish(float* X, const void* A, long lda, const void* W, 
   return pi_check_launch("gemm_finish");
 }
 
-// Attention's key ranges as activations of the finishing product: blocks of 8 rows, each of which merges them all, so not for
-// more bytes than a block reads in the time of the merging kernel.  2,048 x 2,048 with the norm behind it, us: one token with 2
-// ranges of 32 heads of 64 9.5 -> 5.5, eight with 4 (280 KB) 10.8 -> 9.0, of which the merge is 4.5; the merging kernel takes 3.5
-// and the product then 4.3.  The records' maxima and sums through LDS, 16 rows to a block, or twice the loads in flight: 9.5, 9.3, 9.0.
-#define FINISH_RANGE_BYTES (320 << 10)
+// Attention's key ranges as activations of the finishing product: blocks of 8 rows, each of which merges them all, so only for
+// few.  Decode steps of 16 layers, 32 heads of 64, by the merging kernel and inside, us: one token with 2, 4 and 8 ranges (17, 34
+// and 68 KB) 762 / 747, 764 / 747 and 772 / 764; two tokens with 2 and 4, four with 2 771 / 770, 771 / 770 and 796 / 797; three
+// with 4, six with 2 (102 KB) 784 / 798 and 810 / 824; eight with 4 851 / 883, sixteen with 2 1,011 / 1,082 (272 KB); one with
+// 16, whose loads are as many again (136 KB), 809 / 992.
+#define FINISH_RANGE_BYTES (72 << 10)
+#define FINISH_RANGES 8
 #define FINISH_RANGE_LDS (64 << 10)
 
 // Blocks, as pi_gemm_finish_blocks, with which the finishing kernel merges the ranges itself; 0: it does not.
 extern "C" int pi_gemm_finish_ranges_blocks(int M, int N, int heads, int head_dim, int count) {
   const long K = (long)heads * head_dim;
-  if (head_dim < 8 || head_dim % 8 || count < 1 || K > 8192 || !pi_gemm_finish_blocks(M, N, (int)K) || finish_rows(N) != 8) return 0;
+  if (head_dim < 8 || head_dim % 8 || count < 1 || count > FINISH_RANGES || K > 8192 || !pi_gemm_finish_blocks(M, N, (int)K) || finish_rows(N) != 8) return 0;
   if ((long)M * heads * count * (head_dim + 4) * 4 > FINISH_RANGE_BYTES || K * (M > 8 ? 16 : 8) * 2 > FINISH_RANGE_LDS) return 0;
   return N / 8;
 }
