@@ -52,7 +52,8 @@ FUSED_DECODE_HEAD_DIMS = (64, 128)                 # ... and of its form that st
 MAX_DECODE_SPLITS = 64         # the combine kernel holds one key range per lane
 DECODE_WAVES_PER_UNIT = 2      # waves of the decode attention kernel per compute unit that fill the chip (measured at batch 1 to 64: more is never faster)
 DECODE_MIN_KEYS_PER_SPLIT = 128
-RANGES_TO_SHARE = 32           # ranges of all requests from which on two waves of a block share one (decode_range_waves)
+RANGES_TO_SHARE = 32           # ranges of all requests from which on two waves of a block share one (decode_range_waves) ...
+RANGES_SHARED_UP_TO = 4        # ... in steps of up to so many requests
 # Waves that share a block's keys, against ranges with their merging kernel or one wave (lists of attention times, 32 heads, 8 kv
 # heads, 600 to 4,096 keys each).  Blocks have to fill their rounds over the units this far: 384 of them, 1.5 rounds, at 4,096
 # keys 75.7 -> 81.0 us (up to 1,024 keys 23.8 -> 21.4), 320 at head size 128 126 -> 140; 192, three quarters of one round,
@@ -787,13 +788,16 @@ def decode_block_waves(splits: int, R: int, num_kv_heads: int, max_kv_len: int, 
     return 2 if rounds < 3 and bucket > DECODE_WAVES_MIN_KEYS * max(1, head_dim // 64) else 1
 
 
-def decode_range_waves(splits: int, R: int) -> Tuple[int, int]:
-    """(ranges, waves that share one) in place of ``splits`` ranges of a wave each: two waves of a block walk a range's keys as
-    fast as two ranges do (8 requests of 4,000 keys, 8 kv heads of 64: 17.0 us either way; one request 6.8 and 7.5, 16 27.6 and
-    28.4; four waves 21.5, 9.6 and 36.9), and where the output projection merges the ranges, every block of it all of them, it has
-    half as many.  A merging kernel is no faster for it (4 requests of 16,000 latents, 64 ranges: 2 us a step slower)."""
-    if R <= RANGES_MAX_TOKENS and splits > 1 and R * splits >= RANGES_TO_SHARE:
-        return -(-splits // 2), 2
+def decode_range_waves(splits: int, R: int, num_kv_heads: int) -> Tuple[int, int]:
+    """(ranges, waves that share one) in place of ``splits`` ranges of a wave each: whoever merges them has half as many, which
+    steps of up to four requests gain by, as long as the blocks are one round over the units.  Decode steps with ranges of a
+    wave each and of two, us: 1B sizes, one request of 4,000 and 16,000 keys 850 / 804 and 906 / 868, two of 2,000 809 / 795, four of
+    1,000 and 4,000 811 / 803 and 851 / 842; 8B sizes, one of 4,000 1,000 / 976, two of 4,000 1,026 / 1,017, four of 8,000 1,104 /
+    1,102.  264 or 288 blocks: three of 8,000 907 / 922, six and eleven of 1,000 840 / 840 and 931 / 943, twelve of 4,000 1,139 / 1,175.
+    256 blocks, more requests: eight of 4,000 971 / 974, sixteen 1,233 / 1,245."""
+    ranges = -(-splits // 2)
+    if R <= RANGES_SHARED_UP_TO and R * splits >= RANGES_TO_SHARE and R * ranges * num_kv_heads <= compute_units():
+        return ranges, 2
     return splits, 1
 
 
@@ -815,7 +819,7 @@ def _waves_or_ranges(ctx, splits: int, R: int, num_kv_heads: int, head_dim: int,
         if waves > 1:
             return 1, waves, None
         # as the kernel that starts from the projection, to the same bits
-        return (*(decode_range_waves(splits, R) if plain and head_dim in FUSED_DECODE_HEAD_DIMS else (splits, 1)), None)
+        return (*(decode_range_waves(splits, R, num_kv_heads) if plain and head_dim in FUSED_DECODE_HEAD_DIMS else (splits, 1)), None)
     if bounded:                                       # the contexts' lengths do not say how many keys are seen
         return 1, 1, None
     if plan is not None:
@@ -1000,7 +1004,7 @@ def decode_attention_from_projection(out, qkv, ctx, table, num_heads, num_kv_hea
     leave = leave_ranges > 0 and ws is not None and splits > 1 and ranges_product_ok(R, head_dim, leave_ranges)
     waves, uneven = 1, None
     if leave:
-        splits, waves = decode_range_waves(splits, R)
+        splits, waves = decode_range_waves(splits, R, num_kv_heads)
         leave = splits > 1
     else:
         splits, waves, uneven = _waves_or_ranges(ctx, splits, R, num_kv_heads, head_dim, ctx.max_kv_len, window)

@@ -40,8 +40,9 @@ def test_ranges_of_two_waves_and_of_one(ops, monkeypatch, hd, nh, nkv, page, win
     rotary = (torch.cat([angle.cos(), angle.sin()], 1).contiguous(), hd, False)
     ws = ops.KernelWorkspace(DEV)
     splits = fast.decode_splits(R, nkv, max(lens))
-    results = {}
-    for name, share in (("two waves", 0), ("one wave", 1 << 30)):
+    results, shared = {}, False
+    monkeypatch.setattr(fast, "RANGES_SHARED_UP_TO", 16)
+    for name, share in (("two waves", 2), ("one wave", 1 << 30)):
         monkeypatch.setattr(fast, "RANGES_TO_SHARE", share)
         k1, v1, q = k.clone(), v.clone(), torch.empty(R, nh * hd, dtype=BF16, device=DEV)
         fused, apart, merged = (torch.full((R, nh * hd), 7.0, dtype=BF16, device=DEV) for _ in range(3))
@@ -50,8 +51,10 @@ def test_ranges_of_two_waves_and_of_one(ops, monkeypatch, hd, nh, nkv, page, win
         ops.paged_attention(apart, q, k1, v1, table, ctx, nh, nkv, hd, page, scale, window, ws)
         assert torch.equal(fused, apart), name
         left = ops.decode_attention_from_projection(merged, qkv, ctx, rotary, nh, nkv, hd, k1, v1, table, page, scale, window, True, ws, leave_ranges=1 << 20)
-        ranges, waves = fast.decode_range_waves(splits, R)
-        assert (ranges, waves) == ((-(-splits // 2), 2) if share == 0 and splits > 1 else (splits, 1))
+        ranges, waves = fast.decode_range_waves(splits, R, nkv)
+        fits = R * -(-splits // 2) * nkv <= fast.compute_units()
+        assert (ranges, waves) == ((-(-splits // 2), 2) if share == 2 and splits > 1 and fits else (splits, 1))
+        shared |= waves == 2
         if ranges > 1:
             assert isinstance(left, ops.KeyRanges) and left.count == ranges
             fast.merge_ranges(merged, left)
@@ -59,6 +62,7 @@ def test_ranges_of_two_waves_and_of_one(ops, monkeypatch, hd, nh, nkv, page, win
             assert left is True
         assert torch.equal(merged, fused), name
         results[name] = fused
+    assert shared or splits == 1 or R * -(-splits // 2) * nkv > fast.compute_units()
     for r, n in enumerate(lens):
         lo = max(0, n - window) if window else 0
         mine = table[r, :pages[r]].long()

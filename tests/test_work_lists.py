@@ -303,11 +303,13 @@ def test_waves_of_bounded_contexts_and_of_steps_that_do_not_know_their_lengths()
         assert fast._waves_or_ranges(ctx, 1, 64, 8, 64, 3000, 0, SimpleNamespace(singles_uneven=uneven)) == (1, 1 + uneven, None)
 
 
-@pytest.mark.parametrize("splits,R,made", [(1, 16, (1, 1)), (31, 1, (31, 1)), (32, 1, (16, 2)), (64, 1, (32, 2)), (15, 2, (15, 1)), (16, 2, (8, 2)), (2, 15, (2, 1)),
-                                           (2, 16, (1, 2)), (3, 16, (2, 2)), (4, 8, (2, 2)), (3, 10, (3, 1)), (8, 17, (8, 1))])
-def test_ranges_of_all_requests_from_which_on_two_waves_share_one(splits, R, made):
+@pytest.mark.parametrize("splits,R,kv_heads,made", [(1, 16, 8, (1, 1)), (31, 1, 8, (31, 1)), (32, 1, 8, (16, 2)), (64, 1, 8, (32, 2)), (64, 1, 9, (64, 1)), (15, 2, 8, (15, 1)),
+                                                    (16, 2, 8, (8, 2)), (32, 2, 8, (16, 2)), (22, 3, 8, (22, 1)), (20, 3, 8, (10, 2)), (8, 4, 8, (4, 2)), (16, 4, 8, (8, 2)),
+                                                    (16, 4, 9, (16, 1)), (8, 5, 1, (8, 1)), (8, 8, 8, (8, 1)), (4, 16, 8, (4, 1))])
+def test_ranges_of_all_requests_from_which_on_two_waves_share_one(splits, R, kv_heads, made):
+    """As it was the faster way: few requests, enough ranges, and one round of blocks (256 units)."""
     from photon_infer_amd.ops import fast
-    assert fast.decode_range_waves(splits, R) == made
+    assert fast.decode_range_waves(splits, R, kv_heads) == made
     assert made[0] * made[1] >= splits
 
 
