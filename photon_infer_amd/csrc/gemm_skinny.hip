@@ -652,13 +652,15 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_rows_kernel(void* __restrict_
 static int finish_rows(int N) { return N / 16 * 4 < 3 * compute_units() ? 8 : 16; }
 
 // Blocks (= pieces of a row's sum of squares) with which the finishing kernel takes a product, 0 where it does not: M up to 16,
-// N % 64 and K % 64, up to 512 blocks (what LeftNormRows holds), and not the many tokens of a long k with 8 rows to a block,
-// whose activations every block reads (2,048 x 8,192: 12 tokens 12.6 in pieces with the norm and 11.6, 16 tokens 12.8 and 13.0).
+// N % 64 and K % 64, up to 512 blocks (what LeftNormRows holds), and not many tokens, whose activations every block reads, of a long
+// k with 8 rows to a block (2,048 x 8,192: 12 tokens 12.6 in pieces with the norm and 11.6, 16 tokens 12.8 and 13.0; none
+// measured between) or with blocks for a part of a second round (5,120 rows, 320 blocks, k of 5,120 and 13,824 in the mean with
+// the norm and the gap to it: 12 tokens 27.9 and 27.8, 16 tokens 28.4 and 32.1; 8,192 rows, two whole rounds, 16 tokens 62.8 and 62.9).
 extern "C" int pi_gemm_finish_blocks(int M, int N, int K) {
   if (M < 1 || M > 16 || N < 64 || N % 64 || K < KSTEP || K % KSTEP) return 0;
-  const int rows = finish_rows(N);
-  if (N / rows > 512 || (rows == 8 && M > 12 && K > 4096)) return 0;
-  return N / rows;
+  const int rows = finish_rows(N), blocks = N / rows, units = compute_units();
+  if (blocks > 512 || (M > 12 && ((rows == 8 && K > 4096) || (blocks > units && blocks % units)))) return 0;
+  return blocks;
 }
 
 // W: the copy in the streaming order (see pi_gemm_skinny).  H bfloat16 [M, N], sums float32 [M, blocks].  `bias` (or null): float32
