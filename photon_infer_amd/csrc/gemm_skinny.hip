@@ -495,8 +495,9 @@ struct FinishTo {
   float limit, alpha;          // ROWS_CLAMPED: the unit's (clamped_glu)
 };
 
-// Source: nothing (A), or a RangeSource: attention's key ranges, which the block merges into LDS while its weights travel,
-// a thread four features of every token.
+// Source: nothing (A), or a RangeSource: attention's key ranges, up to FINISH_RANGES, which the block merges into LDS while its
+// weights travel, a thread four features of every token.
+#define FINISH_RANGES 16
 template <int WAVES, int ROWS, bool WIDE, int EPI, bool LEFT, typename TW, typename... Source>
 __global__ __launch_bounds__(WAVES * 64) void gemm_rows_kernel(void* __restrict__ Cv, long ldc, const bf16_t* __restrict__ A, long lda,
                                                               const bf16_t* __restrict__ W, int M, int N, int K, FinishTo fin, LeftNorm left,
@@ -563,8 +564,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_rows_kernel(void* __restrict_
       const float* base = rs.ranges + (long)head * rs.count * rec;
       const long token_stride = (long)rs.heads * rs.count * rec;
       auto store = [&](const int token, const uint2 packed) { merged[(piece * TOKENS + (token + piece) % TOKENS) * 2 + quad % 2] = packed; };
-      if (rs.count <= 4) merge_ranges_of_tokens<4, 4>(base, token_stride, rs.count, rec, rs.head_dim, f0, 0, 1, M, store);
-      else merge_ranges_of_tokens<8, 1>(base, token_stride, rs.count, rec, rs.head_dim, f0, 0, 1, M, store);      // up to FINISH_RANGES
+      if (rs.count <= 4) merge_ranges_of_tokens<4, 1>(base, token_stride, rs.count, rec, rs.head_dim, f0, 0, 1, M, store);
+      else if (rs.count <= 8) merge_ranges_of_tokens<8, 1>(base, token_stride, rs.count, rec, rs.head_dim, f0, 0, 1, M, store);
+      else merge_ranges_of_tokens<FINISH_RANGES, 1>(base, token_stride, rs.count, rec, rs.head_dim, f0, 0, 1, M, store);
     }
     __syncthreads();
   }
@@ -693,29 +695,28 @@ extern "C" int pi_gemm_finish(float* X, const void* A, long lda, const void* W, 
   return pi_check_launch("gemm_finish");
 }
 
-// Attention's key ranges as activations of the finishing product: blocks of 8 rows, each of which merges them all, so only for
-// few.  Decode steps of 16 layers, 32 heads of 64, by the merging kernel and inside, us: one token with 2, 4 and 8 ranges (17, 34
-// and 68 KB) 762 / 747, 764 / 747 and 772 / 764; two tokens with 2 and 4, four with 2 771 / 770, 771 / 770 and 796 / 797; three
-// with 4, six with 2 (102 KB) 784 / 798 and 810 / 824; eight with 4 851 / 883, sixteen with 2 1,011 / 1,082 (272 KB); one with
-// 16, whose loads are as many again (136 KB), 809 / 992.
-#define FINISH_RANGE_BYTES (72 << 10)
-#define FINISH_RANGES 8
+// Attention's key ranges as activations of the finishing product: blocks of 8 rows, each of which merges them all, so for one
+// token only.  Decode steps of 16 layers, 32 heads of 64, by the merging kernel and inside, us: one token with 2, 4, 8 and 16
+// ranges (17 to 136 KB) 761 / 748, 760 / 746, 766 / 752 and 773 / 764; two with 4 and 8 771 / 771 and 777 / 774, three with 4 782 /
+// 797, four with 2 and 4 794 / 795 and 800 / 801, eight with 2 834 / 849, sixteen with 2 1,011 / 1,082; of 12 layers, 16 heads: one
+// with 16 411 / 392, eight with 4 433 / 482, sixteen with 2 481 / 537.
+#define FINISH_RANGE_BYTES (144 << 10)
 #define FINISH_RANGE_LDS (64 << 10)
 
 // Blocks, as pi_gemm_finish_blocks, with which the finishing kernel merges the ranges itself; 0: it does not.
 extern "C" int pi_gemm_finish_ranges_blocks(int M, int N, int heads, int head_dim, int count) {
   const long K = (long)heads * head_dim;
-  if (head_dim < 8 || head_dim % 8 || count < 1 || count > FINISH_RANGES || K > 8192 || !pi_gemm_finish_blocks(M, N, (int)K) || finish_rows(N) != 8) return 0;
-  if ((long)M * heads * count * (head_dim + 4) * 4 > FINISH_RANGE_BYTES || K * (M > 8 ? 16 : 8) * 2 > FINISH_RANGE_LDS) return 0;
+  if (M != 1 || head_dim < 8 || head_dim % 8 || count < 1 || count > FINISH_RANGES || K > 8192 || !pi_gemm_finish_blocks(M, N, (int)K) || finish_rows(N) != 8) return 0;
+  if ((long)heads * count * (head_dim + 4) * 4 > FINISH_RANGE_BYTES || K * 8 * 2 > FINISH_RANGE_LDS) return 0;
   return N / 8;
 }
 
-template <bool WIDE, typename TW>
+template <typename TW>
 static int launch_finish_ranges(float* X, const RangeSource& rs, const bf16_t* W, const void* norm_w, bf16_t* H, float* sums, int M, int N, int K, hipStream_t stream) {
-  const auto kernel = gemm_rows_kernel<8, 8, WIDE, ROWS_FINISH, false, TW, RangeSource>;
+  const auto kernel = gemm_rows_kernel<8, 8, false, ROWS_FINISH, false, TW, RangeSource>;
   static const hipError_t configured = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, FINISH_RANGE_LDS);
   if (configured != hipSuccess) return pi_fail("gemm_finish: cannot reserve %d bytes of LDS: %s", FINISH_RANGE_LDS, hipGetErrorString(configured));
-  hipLaunchKernelGGL(kernel, dim3(N / 8), dim3(512), (size_t)K * (WIDE ? 16 : 8) * 2, stream, X, (long)N, (const bf16_t*)nullptr, 0L, W, M, N, K,
+  hipLaunchKernelGGL(kernel, dim3(N / 8), dim3(512), (size_t)K * 8 * 2, stream, X, (long)N, (const bf16_t*)nullptr, 0L, W, M, N, K,
                      FinishTo{norm_w, H, sums, nullptr, 0.f, 0.f}, LeftNorm{}, rs);
   return pi_check_launch("gemm_finish (key ranges merged on the way in)");
 }
@@ -730,12 +731,8 @@ extern "C" int pi_gemm_finish_ranges(float* X, const void* ranges, int heads, in
   PI_REQUIRE(norm_dtype == PI_F32 || norm_dtype == PI_BF16, "gemm_finish: unsupported norm weight dtype %d", norm_dtype);
   const RangeSource rs{(const float*)ranges, heads, head_dim, count};
   const bf16_t* w = (const bf16_t*)W;
-  if (M > 8) {
-    if (norm_dtype == PI_BF16) return launch_finish_ranges<true, bf16_t>(X, rs, w, norm_w, (bf16_t*)H, sums, M, N, K, stream);
-    return launch_finish_ranges<true, float>(X, rs, w, norm_w, (bf16_t*)H, sums, M, N, K, stream);
-  }
-  if (norm_dtype == PI_BF16) return launch_finish_ranges<false, bf16_t>(X, rs, w, norm_w, (bf16_t*)H, sums, M, N, K, stream);
-  return launch_finish_ranges<false, float>(X, rs, w, norm_w, (bf16_t*)H, sums, M, N, K, stream);
+  if (norm_dtype == PI_BF16) return launch_finish_ranges<bf16_t>(X, rs, w, norm_w, (bf16_t*)H, sums, M, N, K, stream);
+  return launch_finish_ranges<float>(X, rs, w, norm_w, (bf16_t*)H, sums, M, N, K, stream);
 }
 
 // C[M, N] = A[M, K] . W[N, K]^T for 1..16 tokens with all of k in a block, W the copy in the streaming order: stored in

@@ -333,7 +333,7 @@ def test_products_that_the_finishing_kernel_takes():
     assert [blocks(M, 2048, K) for M, K in ((12, 4160), (13, 4096), (13, 4160))] == [256, 256, 0] and blocks(16, 3072, 8192) == 192
     assert [blocks(M, N, 5120) for M, N in ((12, 5120), (13, 5120), (16, 4096), (16, 4160), (16, 8192))] == [320, 0, 256, 0, 512]
     ranges = lambda *a: fast._finish_ranges_blocks.__wrapped__(*a)
-    # M, N, heads, head size, ranges: at most 8 of them and 72 KB, 64 KB of LDS, blocks of 8 rows
-    assert [ranges(2, 2048, 32, 64, c) for c in (0, 1, 4, 5)] == [0, 256, 256, 0] and [ranges(1, 2048, 8, 64, c) for c in (8, 9)] == [256, 0]
-    assert [ranges(M, 2048, 32, 64, 2) for M in (4, 5)] == [256, 0] and [ranges(16, 512, 8, 64, c) for c in (2, 3)] == [64, 0]
+    # M, N, heads, head size, ranges: one token, at most 16 ranges and 144 KB, 64 KB of LDS, blocks of 8 rows
+    assert [ranges(1, 2048, 32, 64, c) for c in (0, 1, 16, 17)] == [0, 256, 256, 0] and [ranges(M, 2048, 32, 64, 2) for M in (1, 2, 16)] == [256, 0, 0]
+    assert [ranges(1, 2048, 32, 128, c) for c in (8, 9)] == [256, 0]
     assert ranges(1, 3072, 32, 64, 2) == 0 and ranges(1, 2048, 32, 60, 2) == 0 and [ranges(1, 2048, h, 64, 1) for h in (64, 65)] == [256, 0]
