@@ -791,10 +791,10 @@ def decode_block_waves(splits: int, R: int, num_kv_heads: int, max_kv_len: int, 
 def decode_range_waves(splits: int, R: int, num_kv_heads: int) -> Tuple[int, int]:
     """(ranges, waves that share one) in place of ``splits`` ranges of a wave each: whoever merges them has half as many, which
     steps of up to four requests gain by, as long as the blocks are one round over the units.  Decode steps with ranges of a
-    wave each and of two, us, going on from so many keys: 1B sizes, one request of 4,000 and 16,000 850 / 804 and 906 / 868, two of 2,000 809 / 795, four of
-    1,000 and 4,000 811 / 803 and 851 / 842; 8B sizes, one of 4,000 1,000 / 976, two of 4,000 1,026 / 1,017, four of 8,000 1,104 /
-    1,102.  264 or 288 blocks: three of 8,000 907 / 922, six and eleven of 1,000 840 / 840 and 931 / 943, twelve of 4,000 1,139 / 1,175.
-    256 blocks, more requests: eight of 4,000 971 / 974, sixteen 1,233 / 1,245."""
+    wave each and of two, us, going on from so many keys: 1B sizes, one request of 4,000 and 16,000 850 / 804 and 906 / 868, two of
+    2,000 809 / 795, four of 1,000 and 4,000 811 / 803 and 851 / 842; 8B sizes, one of 4,000 1,000 / 976, two of 4,000 1,026 / 1,017,
+    four of 8,000 1,104 / 1,102.  264 or 288 blocks: three of 8,000 907 / 922, six and eleven of 1,000 840 / 840 and 931 / 943, twelve
+    of 4,000 1,139 / 1,175.  256 blocks, more requests: eight of 4,000 971 / 974, sixteen 1,233 / 1,245."""
     ranges = -(-splits // 2)
     if R <= RANGES_SHARED_UP_TO and R * splits >= RANGES_TO_SHARE and R * ranges * num_kv_heads <= compute_units():
         return ranges, 2
