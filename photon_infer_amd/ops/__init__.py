@@ -490,7 +490,7 @@ def decode_attention_from_projection(out: torch.Tensor, qkv, ctx, rotary, num_he
     ``leave_ranges`` (needs ``ws``; 0, or the bytes of the weight matrix the result goes to): the
     caller hands the result straight to ``gemm`` with that matrix; when the keys were split into
     ranges, the kernel may then return them unmerged (``KeyRanges``, in the workspace) instead of
-    filling ``out``, and the product merges them as it reads."""
+    filling ``out``, and ``gemm`` merges them, in the product or before it."""
     if not (_FAST and out.dtype in (torch.bfloat16, torch.float32) and out.is_cuda and getattr(ctx, "all_decode", False)):
         return False
     if not isinstance(qkv, Partials) and qkv.dtype != out.dtype:

@@ -211,7 +211,7 @@ class PagedAttention(Mixer):
                                                         self.window or 0, writes, ws,
                                                         leave_ranges=self.w_o.numel() * self.w_o.element_size())
             if done:
-                # the output, or its key ranges still to be merged, which the product does as it reads them
+                # the output, or its key ranges still to be merged, by the product as it reads them or before it
                 ops.gemm(x, done if isinstance(done, ops.KeyRanges) else attn, self.w_o, accumulate=self.accumulate,
                          may_defer=self.accumulate and not self.o_bias and getattr(ctx, "may_defer", False), ws=ws,
                          next_norm=getattr(ctx, "next_norm", None), whole=True)
