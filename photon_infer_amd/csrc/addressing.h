@@ -93,7 +93,7 @@ constexpr unsigned OUT_OF_RANGE = 0x7ffffff0u;
 // which 16-byte piece of its row in memory the lane fetches (the pieces of a row are turned by
 // (row / 2) % 8 on their way into LDS)
 PI_ADDR int tile_piece(int lane, int row) { return (lane % 8) ^ ((row >> 1) & 7); }
-// 128 x 128 kernel and the float32 tiles: rows beyond the operand take an offset outside the descriptor
+// 128 x 128 kernel and all float32 tiles: rows beyond the operand take an offset outside the descriptor
 PI_ADDR unsigned tile_lane_offset(int row, int rows, long ld, int piece) {
   return row < rows ? (unsigned)(row * (int)ld + piece * 8) * 2u : OUT_OF_RANGE;
 }
@@ -101,6 +101,10 @@ PI_ADDR unsigned tile_lane_offset(int row, int rows, long ld, int piece) {
 PI_ADDR unsigned tile_slab_offset(unsigned lane_offset, int k0, int piece, int k_range) {
   return k0 + piece * 8 < k_range ? lane_offset + (unsigned)k0 * 2u : OUT_OF_RANGE;
 }
+// float32 tiles in parts: 16 floats (in units of two bytes) a slab, four pieces of a row; a load of 256 threads covers 64 rows
+constexpr int PARTS_SLAB = 32;
+PI_ADDR int parts_piece(int tid) { return tid % 4; }
+PI_ADDR int parts_row(int load, int tid) { return load * 64 + tid / 4; }
 // larger bfloat16 tiles (K a multiple of 64, whole slabs only): rows beyond the operand read the last row
 PI_ADDR unsigned big_lane_offset(int row, int rows, long ld, int piece) {
   return (unsigned)(imin(row, rows - 1) * (int)ld + piece * 8) * 2u;

@@ -1,15 +1,16 @@
-// float32 matrix products on the matrix cores: C[M, N] (+)= A[M, K] . W[N, K]^T with 32-bit operands, products and sums
-// (v_mfma_f32_32x32x2_f32 and v_mfma_f32_16x16x4_f32; 157 TFLOP/s on this chip, twice the vector unit's rate without
-// packed instructions).  They carry the float32 path's products; gemm_general.hip keeps mixed types, odd strides and the
-// products of a few rows that it streams faster (ops/fast.py).
+// float32 matrix products on the matrix cores: C[M, N] (+)= A[M, K] . W[N, K]^T with 32-bit operands and sums, by the
+// instructions that take float32 (v_mfma_f32_32x32x2_f32 and v_mfma_f32_16x16x4_f32; 157 TFLOP/s on this chip, twice the
+// vector unit's rate without packed instructions) or, for large tiles, by six that take bfloat16 (gemm_float32_parts_kernel).
+// They carry the float32 path's products; gemm_general.hip keeps mixed types, odd strides and the products of a few rows that
+// it streams faster (ops/fast.py).
 //
 // K and the row strides are multiples of 4 and the operands 16-byte aligned.  A row of 32 floats is 128 bytes, as a row
 // of 64 bfloat16 is, so both kernels move their operands exactly as the bfloat16 kernels do and share those kernels'
 // address arithmetic (addressing.h), in units of two bytes: every `2 *` below turns floats into such units.
 //
 // Up to 32 rows (decode steps): gemm_float32_rows_kernel, bound by the weights' way from memory.  More rows:
-// gemm_float32_tile_kernel, bound by the matrix cores; where its tiles are few, k is cut over blocks and
-// pi_splitk_reduce adds the pieces in order.
+// gemm_float32_parts_kernel, bound by the matrix cores, or, for few tiles, gemm_float32_tile_kernel; where the tiles do not
+// fill the chip, k is cut over blocks and pi_splitk_reduce adds the pieces in order.
 #include "addressing.h"
 #include "mfma.h"
 
@@ -17,6 +18,7 @@
 #define ROWS_MAX_M 32                 // up to this many rows of activations the weight-streaming kernel is taken
 #define ROWS_SPLIT_MIN_K 4096         // from this k on a product's pieces are worth a kernel that adds them
 #define ROWS_WHOLE_K 768              // up to this k a matrix of many rows is left whole for its reader too
+#define PARTS_WIDE_MAX_STRIDE (1 << 20)  // floats between weight rows up to which 256 of them lie within a descriptor's 2 GB
 
 // What becomes of a product in one piece: stored, added to C, or, with gate and up rows interleaved in blocks of 16 in W,
 // silu(gate) * up of the same feature stored to C [M, N / 2] (a kernel of its own for it took 4.7 us at eight tokens by 8,192
@@ -183,12 +185,81 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_float32_rows_kernel(float* __
 }
 
 // ------------------------------------------------------------------ many rows: tiles
-// Block tile TM x TN, four waves in 2 x 2, slabs of 32 floats of k that go from memory straight into LDS through a ring
-// of NB buffers (rows of 128 bytes, their 16-byte pieces turned by (row / 2) % 8 as in gemm_mfma.hip).  A matrix
-// instruction takes 64 cycles for two registers of operands, so LDS and its reads have time to spare and the tile only
-// has to be large enough for L2: 32 / 21 / 16 flops per byte at 128 x 128 / 128 x 64 / 64 x 64.  What decides is how the
-// tiles fill the chip, see plan().  Every output is summed over k in the same order in every
-// tile shape; how many pieces k is cut into depends on the rows and columns, so a row's bits depend on what shares its launch.
+// Where the block's tile lies among tiles_m x tiles_n.
+struct TilePlace {
+  int m, n;
+};
+__device__ inline TilePlace tile_place(int tiles_n) {
+  const int tiles_m = gridDim.x / tiles_n;
+  if (tiles_n % 8 == 0) {                        // a die streams its own slice of W and walks the row tiles of a column first
+    const int die = blockIdx.x % 8, local = blockIdx.x / 8;
+    return TilePlace{local % tiles_m, die * (tiles_n / 8) + local / tiles_m};
+  }
+  return TilePlace{(int)blockIdx.x / tiles_n, (int)blockIdx.x % tiles_n};
+}
+
+// What becomes of a wave's WM x WN accumulators of 32 x 32, whose first row and column are m_wave and n_wave.
+template <int WM, int WN, int EPI>
+__device__ inline void finish_tiles(const f32x16_t (&acc)[WM][WN], long m_wave, long n_wave, float* __restrict__ C, long ldc, int M, int N,
+                                    float* __restrict__ part) {
+  const int lane = threadIdx.x % 64, frow = lane % 32;
+  // acc[i][j][v] is C[m_wave + i*32 + 8*(v/4) + 4*(lane/32) + v%4][n_wave + j*32 + lane%32]: a store
+  // instruction writes 128 contiguous bytes of two rows.  Added into C, sixteen of its values are fetched before the first
+  // is used (one after the other 1,600 x 16,384 x 64 took 113 us, 512 x 16,384 x 512 99; 69 and 87 so)
+  if (EPI == EPI_SWIGLU) {
+    // columns 0..15 of a wave's 32 are gate rows of W, 16..31 the up rows of the same features: lane l and lane l + 16 swap
+    // so that the one has gate and up of row v, the other of row v + 1
+    const bool up = frow >= 16;
+#pragma unroll
+    for (int j = 0; j < WN; ++j) {
+      const long n = n_wave + j * 32;                 // N is a multiple of 32
+      if (n >= N) continue;
+#pragma unroll
+      for (int i = 0; i < WM; ++i) {
+        const long mi = m_wave + i * 32 + 4 * (lane / 32);
+#pragma unroll
+        for (int v = 0; v < 16; v += 2) {
+          const float own = up ? acc[i][j][v + 1] : acc[i][j][v], other = __shfl_xor(up ? acc[i][j][v] : acc[i][j][v + 1], 16);
+          const long m = mi + 8 * (v / 4) + v % 4 + up;
+          if (m < M) C[m * ldc + n / 2 + frow % 16] = silu_mul(up ? other : own, up ? own : other);
+        }
+      }
+    }
+    return;
+  }
+  const bool pieces = gridDim.y > 1;
+  float* out = pieces ? part + (long)blockIdx.y * M * N : C;
+  const long ld = pieces ? N : ldc;
+#pragma unroll
+  for (int j = 0; j < WN; ++j) {
+    const long n = n_wave + j * 32 + frow;
+    if (n >= N) continue;
+#pragma unroll
+    for (int i = 0; i < WM; ++i) {
+      const long mi = m_wave + i * 32 + 4 * (lane / 32);
+      float sum[16];
+#pragma unroll
+      for (int v = 0; v < 16; ++v) sum[v] = acc[i][j][v];
+      if (EPI == EPI_ADD && !pieces) {           // asked for together: one wait for memory, not sixteen
+        float old[16];
+#pragma unroll
+        for (int v = 0; v < 16; ++v) old[v] = out[min(mi + 8 * (v / 4) + v % 4, (long)M - 1) * ld + n];
+#pragma unroll
+        for (int v = 0; v < 16; ++v) sum[v] = old[v] + sum[v];
+      }
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const long m = mi + 8 * (v / 4) + v % 4;
+        if (m < M) out[m * ld + n] = sum[v];
+      }
+    }
+  }
+}
+
+// Few tiles: TM x TN (64 x 64 is the one in use), four waves in 2 x 2, slabs of 32 floats of k that go from memory straight into
+// LDS through a ring of NB buffers (rows of 128 bytes, their 16-byte pieces turned by (row / 2) % 8 as in gemm_mfma.hip).  A block
+// of these starts and steps faster than one of gemm_float32_parts_kernel: 0.6 us per 32 floats of k alone on its unit, where 64 x 64
+// in parts take 0.9 (a chain of conversion, store, barrier and six products on one accumulator).
 template <int TM, int TN, int NB, int EPI>
 __global__ __launch_bounds__(256) void gemm_float32_tile_kernel(float* __restrict__ C, long ldc, const float* __restrict__ A, long lda,
                                                                 const float* __restrict__ W, long ldw, int M, int N, int K, int tiles_n,
@@ -203,17 +274,8 @@ __global__ __launch_bounds__(256) void gemm_float32_tile_kernel(float* __restric
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
   const int wm = wave / 2, wn = wave % 2;
   const int k_lo = 2 * (int)blockIdx.y * k_per_split, k_hi = 2 * min(K, (int)(blockIdx.y + 1) * k_per_split);
-  const int tiles_m = gridDim.x / tiles_n;
-  int tile_m, tile_n;
-  if (tiles_n % 8 == 0) {                        // a die streams its own slice of W and walks the row tiles of a column first
-    const int die = blockIdx.x % 8, local = blockIdx.x / 8;
-    tile_n = die * (tiles_n / 8) + local / tiles_m;
-    tile_m = local % tiles_m;
-  } else {
-    tile_m = blockIdx.x / tiles_n;
-    tile_n = blockIdx.x % tiles_n;
-  }
-  const long m0 = (long)tile_m * TM, n0 = (long)tile_n * TN;
+  const TilePlace place_of = tile_place(tiles_n);
+  const long m0 = (long)place_of.m * TM, n0 = (long)place_of.n * TN;
   const int a_rows = (int)min((long)TM, M - m0), w_rows = (int)min((long)TN, N - n0);
 #if defined(__HIP_DEVICE_COMPILE__)
   const __amdgpu_buffer_rsrc_t a_src = operand_descriptor(reinterpret_cast<const bf16_t*>(A), addressing::tile_descriptor(m0, 2 * lda, k_lo, k_hi, a_rows));
@@ -300,58 +362,180 @@ __global__ __launch_bounds__(256) void gemm_float32_tile_kernel(float* __restric
     buf = buf == NB - 1 ? 0 : buf + 1;
   }
   __builtin_amdgcn_s_waitcnt(0x0F70);            // nothing may still be on its way into LDS when the block ends
+  finish_tiles<WM, WN, EPI>(acc, m0 + wm * (TM / 2), n0 + wn * (TN / 2), C, ldc, M, N, part);
+}
 
-  // acc[i][j][v] is C[m0 + wm*TM/2 + i*32 + 8*(v/4) + 4*(lane/32) + v%4][n0 + wn*TN/2 + j*32 + lane%32]: a store
-  // instruction writes 128 contiguous bytes of two rows.  Added into C, sixteen of its values are fetched before the first
-  // is used (one after the other 1,600 x 16,384 x 64 took 113 us, 512 x 16,384 x 512 99; 69 and 87 so)
-  if (EPI == EPI_SWIGLU) {
-    // columns 0..15 of a wave's 32 are gate rows of W, 16..31 the up rows of the same features: lane l and lane l + 16 swap
-    // so that the one has gate and up of row v, the other of row v + 1
-    const bool up = frow >= 16;
+// Large tiles, in parts: a float is the sum of three bfloat16 (the bfloat16 nearest to it, the one nearest to what is left, and the
+// rest, which fits), and six of the nine products of parts reach its last bit: lo . lo, lo . mid and mid . lo lie 2^-25 below the
+// product and less.  Six bfloat16 instructions (exact products, 32-bit sums) take 6 x 32 cycles for the 32 x 32 x 16 that float32
+// instructions need 8 x 64 for, and a sum has a sixteenth of the roundings per instruction: 1,293 x 2,048 outputs of k = 2,048 are off
+// from 64 bits by 7.0e-7 of their norm here and by 8.1e-7 with float32 instructions, of k = 8,192 by 1.44e-6 and 1.62e-6.
+//
+// The parts are made once per block, on the way from memory into LDS: a thread fetches 16 bytes of a row a slab (16 floats of k) ahead,
+// splits them (11 instructions per two floats, between the matrix instructions) and stores 8 bytes to each of three planes.  LDS holds
+// two slabs of [32 rows][plane][half of k][row][8 k]: a fragment is 1 KB in lane order, the second half's rows turned by 4 so that
+// four rows' stores fall on different banks.  Four waves in 2 x 2, two blocks per unit, one barrier per slab.
+// Bound by the matrix cores and the chip's power: 2,048 x 16,384 x 2,048 takes 640 us (1.29 PFLOP/s of bfloat16 products at 1.8 GHz,
+// the matrix cores 70 % busy, LDS 26 %, the vector unit 41 %) in tiles of 128 x 256, 996 with float32 instructions in 128 x 128;
+// 1,293 x 16,384 x 2,048 450 us (729), 1,293 x 2,048 x 8,192 235 (371), 378 x 3,072 x 2,048 35 (49).  What orders the steps between
+// the matrix instructions is worth 10 to 20 % in tiles of 192 x 128 (378 x 16,384 x 2,048 184 us as the compiler had them, 148 now).  Not
+// kept: sched_group_barrier for that (one matrix instruction and four or six others in turn: up to 10 % slower), slabs fetched two to
+// four ahead (2 % either way), tiles of 64 x 64 and 64 x 128 in parts.
+//
+// An infinity has no such parts (the rest would be NaN), neither has a float that rounds to one (above 3.39e38); and where an
+// operand's largest float is below 2^-100 the last parts are lost.  A tile that meets one of these is made again from memory with
+// float32 instructions, slowly.  (A NaN needs nothing: its row or column is NaN either way.)
+// Four floats on their way into parts, in steps of some five instructions each: step 2 q + i makes part q of floats 2 i and 2 i + 1.
+struct PartsOf4 {
+  float r[4];
+  uint32_t part[3][2];
+  __device__ inline void begin(const f32x4_t x, float& top) {
 #pragma unroll
-    for (int j = 0; j < WN; ++j) {
-      const long n = n0 + wn * (TN / 2) + j * 32;                 // N is a multiple of 32
-      if (n >= N) continue;
+    for (int e = 0; e < 4; ++e) r[e] = x[e];
+    // fmaxf would quiet NaNs in an instruction of its own
+    asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(top) : "v"(r[0]), "v"(r[1]));
+    asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(top) : "v"(r[2]), "v"(r[3]));
+  }
+  __device__ inline void step(const int u) {
+    const int q = u / 2, i = u % 2;
+    part[q][i] = pack_bf16x2(r[2 * i], r[2 * i + 1]);
+    if (q < 2) {
+      r[2 * i] -= __uint_as_float(part[q][i] << 16);
+      r[2 * i + 1] -= __uint_as_float(part[q][i] & 0xffff0000u);
+    }
+  }
+};
+
+constexpr float PARTS_LARGEST = 3.3895313892515355e38f, PARTS_SMALLEST = 0x1p-100f;
+
+template <int WM, int WN, int EPI>
+__global__ __launch_bounds__(256, 2) void gemm_float32_parts_kernel(float* __restrict__ C, long ldc, const float* __restrict__ A, long lda,
+                                                                    const float* __restrict__ W, long ldw, int M, int N, int K, int tiles_n,
+                                                                    int k_per_split, float* __restrict__ part) {
+  extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
+  constexpr int TM = WM * 64, TN = WN * 64, LOADS = WM + WN;   // a load covers 64 rows
+  constexpr int PLANE = 512, GROUP = 3 * PLANE, BUF = (TM + TN) / 32 * GROUP;
+  constexpr int JP = WN == 4 ? 2 : 1;                          // columns of tiles whose products alternate (128 x 256: 670 -> 637 us)
+  const int tid = threadIdx.x, lane = tid % 64;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+  const int wm = wave / 2, wn = wave % 2;
+  const int k_lo = 2 * (int)blockIdx.y * k_per_split, k_hi = 2 * min(K, (int)(blockIdx.y + 1) * k_per_split), k_range = k_hi - k_lo;
+  const TilePlace tile = tile_place(tiles_n);
+  const long m0 = (long)tile.m * TM, n0 = (long)tile.n * TN;
+  const int a_rows = (int)min((long)TM, M - m0), w_rows = (int)min((long)TN, N - n0);
+#if defined(__HIP_DEVICE_COMPILE__)
+  const __amdgpu_buffer_rsrc_t a_src = operand_descriptor(reinterpret_cast<const bf16_t*>(A), addressing::tile_descriptor(m0, 2 * lda, k_lo, k_hi, a_rows));
+  const __amdgpu_buffer_rsrc_t w_src = operand_descriptor(reinterpret_cast<const bf16_t*>(W), addressing::tile_descriptor(n0, 2 * ldw, k_lo, k_hi, w_rows));
+#endif
+  const int piece = addressing::parts_piece(tid);
+  unsigned offset[LOADS];
+  int store[LOADS];
 #pragma unroll
-      for (int i = 0; i < WM; ++i) {
-        const long mi = m0 + wm * (TM / 2) + i * 32 + 4 * (lane / 32);
+  for (int p = 0; p < LOADS; ++p) {
+    const bool of_a = p < WM;
+    const int row = addressing::parts_row(of_a ? p : p - WM, tid), among = p * 64 + tid / 4;
+    offset[p] = of_a ? addressing::tile_lane_offset(row, a_rows, 2 * lda, piece) : addressing::tile_lane_offset(row, w_rows, 2 * ldw, piece);
+    store[p] = among / 32 * GROUP + (piece / 2 * 32 + (among % 32 ^ piece / 2 * 4)) * 8 + piece % 2 * 4;
+  }
+  u32x4_t got[LOADS];
+  auto fetch = [&](const int p, const int s) {   // beyond the range: zeros
+#if defined(__HIP_DEVICE_COMPILE__)
+    got[p] = __builtin_amdgcn_raw_buffer_load_b128(p < WM ? a_src : w_src, addressing::tile_slab_offset(offset[p], s * addressing::PARTS_SLAB, piece, k_range), 0, 0);
+#endif
+  };
+  float a_top = 0.f, w_top = 0.f;
+  PartsOf4 four;
+  auto put = [&](const int p, const int u, const int buf) {      // step u of load p
+    if (u == 0) four.begin(__builtin_bit_cast(f32x4_t, got[p]), p < WM ? a_top : w_top);
+    four.step(u);
+    if (u < 5) return;
 #pragma unroll
-        for (int v = 0; v < 16; v += 2) {
-          const float own = up ? acc[i][j][v + 1] : acc[i][j][v], other = __shfl_xor(up ? acc[i][j][v] : acc[i][j][v + 1], 16);
-          const long m = mi + 8 * (v / 4) + v % 4 + up;
-          if (m < M) C[m * ldc + n / 2 + frow % 16] = silu_mul(up ? other : own, up ? own : other);
+    for (int q = 0; q < 3; ++q) *reinterpret_cast<uint2*>(lds + buf + store[p] + q * PLANE) = make_uint2(four.part[q][0], four.part[q][1]);
+  };
+
+  f32x16_t acc[WM][WN];
+  auto clear = [&] {
+#pragma unroll
+    for (int i = 0; i < WM; ++i)
+#pragma unroll
+      for (int j = 0; j < WN; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+  };
+  clear();
+  const int slabs = (k_range + addressing::PARTS_SLAB - 1) / addressing::PARTS_SLAB;
+  const int frag = (lane ^ lane / 32 * 4) * 8;
+  const uint16_t* a_base = lds + wm * WM * GROUP + frag;
+  const uint16_t* w_base = lds + (2 * WM + wn * WN) * GROUP + frag;
+#pragma unroll
+  for (int p = 0; p < LOADS; ++p) fetch(p, 0);
+#pragma unroll
+  for (int p = 0; p < LOADS; ++p) {
+#pragma unroll
+    for (int u = 0; u < 6; ++u) put(p, u, 0);
+    fetch(p, 1);
+  }
+  int buf = 0;
+  for (int s = 0; s < slabs; ++s) {
+    __builtin_amdgcn_sched_barrier(0);
+    block_barrier_keeping_loads<63>();           // slab s is there, and everybody has left the other buffer
+    __builtin_amdgcn_sched_barrier(0);
+    Frag fa[WM][3], fb[2][JP][3];
+    auto read_w = [&](const int j) {
+#pragma unroll
+      for (int jj = 0; jj < JP; ++jj)
+#pragma unroll
+        for (int q = 0; q < 3; ++q) fb[j / JP & 1][jj][q].q = *reinterpret_cast<const uint4*>(w_base + buf + (j + jj) * GROUP + q * PLANE);
+    };
+    read_w(0);
+#pragma unroll
+    for (int i = 0; i < WM; ++i)
+#pragma unroll
+      for (int q = 0; q < 3; ++q) fa[i][q].q = *reinterpret_cast<const uint4*>(a_base + buf + i * GROUP + q * PLANE);
+#pragma unroll
+    for (int j = 0; j < WN; j += JP) {
+      if (j + JP < WN) read_w(j + JP);
+      constexpr int of_a[6] = {2, 0, 1, 1, 0, 0}, of_w[6] = {0, 2, 1, 0, 1, 0};      // the smallest terms first
+#pragma unroll
+      for (int n = 0; n < 6 * WM * JP; ++n) {
+        const int t = n / (WM * JP), i = n / JP % WM, jj = n % JP, at = j * 6 * WM + n;
+        acc[i][j + jj] = mfma32(fa[i][of_a[t]], fb[j / JP & 1][jj][of_w[t]], acc[i][j + jj]);
+#pragma unroll
+        for (int u = at * 6 * LOADS / (6 * WM * WN); u < (at + 1) * 6 * LOADS / (6 * WM * WN); ++u) {
+          put(u / 6, u % 6, BUF - buf);
+          if (u % 6 == 5) fetch(u / 6, s + 2);
         }
+        __builtin_amdgcn_sched_barrier(0x104);   // nothing but fragment reads and scalar work moves across: left alone, the compiler bunches the steps
       }
     }
-    return;
+    buf = BUF - buf;
   }
-  const bool pieces = gridDim.y > 1;
-  float* out = pieces ? part + (long)blockIdx.y * M * N : C;
-  const long ld = pieces ? N : ldc;
+
+  block_barrier_keeping_loads<0>();              // everybody is done with LDS
+  int* met = reinterpret_cast<int*>(lds);
+  if (tid == 0) *met = 0;
+  __syncthreads();
+  const int bits = (__any(!(a_top <= PARTS_LARGEST) || !(w_top <= PARTS_LARGEST)) ? 1 : 0) | (__any(a_top > 0.f) ? 2 : 0) |
+                   (__any(a_top >= PARTS_SMALLEST) ? 4 : 0) | (__any(w_top > 0.f) ? 8 : 0) | (__any(w_top >= PARTS_SMALLEST) ? 16 : 0);
+  if (lane == 0) atomicOr(met, bits);
+  __syncthreads();
+  const int all = __builtin_amdgcn_readfirstlane(*met);
+  if ((all & 1) || (all & 6) == 2 || (all & 24) == 8) {
+    clear();
+#pragma unroll 1
+    for (int k = k_lo / 2 + lane / 32; k < k_hi / 2; k += 2) {
+      float fa[WM], fb[WN];
 #pragma unroll
-  for (int j = 0; j < WN; ++j) {
-    const long n = n0 + wn * (TN / 2) + j * 32 + frow;
-    if (n >= N) continue;
+      for (int i = 0; i < WM; ++i) fa[i] = A[min(m0 + wm * (TM / 2) + i * 32 + lane % 32, (long)M - 1) * lda + k];
 #pragma unroll
-    for (int i = 0; i < WM; ++i) {
-      const long mi = m0 + wm * (TM / 2) + i * 32 + 4 * (lane / 32);
-      float sum[16];
+      for (int j = 0; j < WN; ++j) fb[j] = W[min(n0 + wn * (TN / 2) + j * 32 + lane % 32, (long)N - 1) * ldw + k];
 #pragma unroll
-      for (int v = 0; v < 16; ++v) sum[v] = acc[i][j][v];
-      if (EPI == EPI_ADD && !pieces) {           // asked for together: one wait for memory, not sixteen
-        float old[16];
+      for (int i = 0; i < WM; ++i)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) old[v] = out[min(mi + 8 * (v / 4) + v % 4, (long)M - 1) * ld + n];
-#pragma unroll
-        for (int v = 0; v < 16; ++v) sum[v] = old[v] + sum[v];
-      }
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const long m = mi + 8 * (v / 4) + v % 4;
-        if (m < M) out[m * ld + n] = sum[v];
-      }
+        for (int j = 0; j < WN; ++j) acc[i][j] = mfma32_f32(fa[i], fb[j], acc[i][j]);
     }
   }
+  finish_tiles<WM, WN, EPI>(acc, m0 + wm * (TM / 2), n0 + wn * (TN / 2), C, ldc, M, N, part);
 }
 
 // ------------------------------------------------------------------ which kernel, which tile, how many pieces
@@ -365,19 +549,22 @@ static Float32Plan cut(int tm, int tn, int K, int splits) {
   return Float32Plan{tm, tn, c.splits, c.k_per_block};
 }
 
-// Tiles: the shape and the number of pieces with the least time by a model of what was measured: a unit works through
-// its blocks at 0.5 TFLOP/s (less on the smaller tiles), a block starts and ends in 3 us, pieces are written and read
-// once at 4 TB/s by a kernel of their own.  Measured, N x K = 16384 x 2048: 2,048 rows 1,002 us (137 TFLOP/s), 1,293 rows
-// 727 us (1,236 on the vector unit), 378 rows 214 us (118 TFLOP/s); 2048 x 8192: 2,048 rows 525 us, 1,293 rows 412 us in two
-// pieces, 378 rows 119 us in five.
-// `read_by_next`: the pieces are left to the kernel that reads the result anyway (a norm, a rotation).  They then cost their
+// Tiles: the shape and the number of pieces with the least time by a model fitted to 6,800 measurements (24 row counts of 33 to 2,900,
+// thirteen matrices of 512 x 1,024 to 28,672 x 4,096, weights from memory): a block's start, the k that the busiest unit walks, two blocks
+// of it side by side, and the result's way out.  The plan is 0.3 % above the best of these shapes and pieces in the mean, 5.6 % at worst.
+// Float32 instructions (64 x 64) where the parts' larger tiles leave units idle: 64 rows by 2,048 x 8,192 26 us and 51 in tiles of 128 x
+// 128; by 16,384 x 2,048 42 and 45; 100 rows by 16,384 x 2,048 75 and 49.  Pieces that a kernel adds (`after` 0) are written and read
+// once at 4 TB/s, and that takes a launch; if the gated unit then is a kernel too (`after` 2), that as well (512 features, k = 512, 33 to
+// 100 rows: 15.3 us whole, 12.4 in two pieces; 1,293 rows, 1,536 features, k = 2,048 163 and 115).
+// `after` 1: the pieces are left to the kernel that reads the result anyway (a norm, a rotation).  They then cost their
 // way through memory and no launch, and a matrix of few rows is streamed by two blocks per unit whatever its k: eight tokens and
 // the norm, 2,048 x 2,048 12.4 -> 10.3 us, 3,072 x 2,048 13.1 -> 12.0; and some 2 us less for each product whose pieces a kernel
 // added.  A short k in blocks of 16 rows that nearly are the units' number stays whole (24 tokens and the norm, 3,072 x 768 10.6 us
 // and 14.6 in three pieces; 4,096 x 512 10.1 and 10.9).  More pieces have to promise a hundredth: 129 x 2,048 x 8,192 and the norm
 // takes 65 us in five and 76 in eight, which the rule holds for equal.
-static Float32Plan plan(int M, int N, int K, long part_floats, bool read_by_next) {
+static Float32Plan plan(int M, int N, int K, long part_floats, int after) {
   const int units = compute_units();
+  const bool read_by_next = after == 1;
   if (M <= ROWS_MAX_M) {
     // blocks of 32 rows want to be two per unit; a matrix of fewer rows whose k is long is cut over blocks, any other
     // gets its waves in blocks of 16 rows (launch_rows)
@@ -386,26 +573,30 @@ static Float32Plan plan(int M, int N, int K, long part_floats, bool read_by_next
     while (splits > 1 && (K / splits < (read_by_next ? 256 : 512) || (long)splits * M * N > part_floats)) --splits;
     return cut(0, 0, K, splits < 1 ? 1 : splits);
   }
-  static const struct { int tm, tn; float rate; } shapes[] = {{128, 128, 0.50e6f}, {128, 64, 0.49e6f}, {64, 64, 0.46e6f}};
-  Float32Plan best = {128, 128, 1, K};
+  static const struct { int tm, tn; float start, per_k, paired, out; } shapes[] = {      // us, us per k of one block, share of that where two blocks go side by side, us per MB
+      {64, 64, 3.07f, 0.01937f, 0.871f, 0.236f}, {128, 128, 2.75f, 0.04363f, 0.790f, 0.267f}, {192, 128, 3.10f, 0.05737f, 0.838f, 0.301f}, {128, 256, 4.25f, 0.06864f, 0.889f, 0.326f}};
+  Float32Plan best = {64, 64, 1, K};
   float least = 0.f;
+  const float megabytes = (float)M * N * 4e-6f;
   for (const auto& s : shapes) {
     const long tiles = (long)ceil_div(M, s.tm) * ceil_div(N, s.tn);
     for (int splits = 1; splits <= 8; ++splits) {
       const Float32Plan p = cut(s.tm, s.tn, K, splits);
       if (splits > 1 && (p.splits != splits || p.k_per_split < 256 || (long)splits * M * N > part_floats)) continue;
       const long rounds = (tiles * p.splits + units - 1) / units;
-      float us = rounds * (3.f + 2.f * s.tm * s.tn * p.k_per_split / s.rate);
-      if (p.splits > 1) us += (read_by_next ? 1.f : 4.f) + (read_by_next ? 1.5f : 2.f) * p.splits * M * N * 4.f / 4.0e6f;
+      float us = s.start + (rounds % 2 + (rounds - rounds % 2) * s.paired) * s.per_k * p.k_per_split + s.out * p.splits * megabytes;
+      if (p.splits > 1) us += read_by_next ? 1.f + 1.5f * p.splits * megabytes / 4.f : 2.5f + 2.f * p.splits * megabytes / 4.f;
+      if (p.splits > 1 && after == 2) us += 1.f + 1.5f * megabytes / 4.f;
       if (least == 0.f || us < (read_by_next && p.splits > best.splits ? 0.99f : 1.f) * least) { least = us; best = p; }
     }
   }
   return best;
 }
 
-// Pieces that pi_gemm_float32 makes of this product when it may leave pieces in `part_floats` floats: 1 if it writes C.  See plan().
-extern "C" int pi_gemm_float32_pieces(int M, int N, int K, long part_floats, int read_by_next) {
-  return M > 0 && N > 0 && K > 0 ? plan(M, N, K, part_floats, read_by_next != 0).splits : 1;
+// Pieces that pi_gemm_float32 makes of this product when it may leave pieces in `part_floats` floats: 1 if it writes C.  `after`: what
+// becomes of pieces, see plan().
+extern "C" int pi_gemm_float32_pieces(int M, int N, int K, long part_floats, int after) {
+  return M > 0 && N > 0 && K > 0 ? plan(M, N, K, part_floats, after).splits : 1;
 }
 
 template <int TM, int TN, int NB, int EPI>
@@ -421,12 +612,26 @@ static int launch_tiles_of(float* C, long ldc, const float* A, long lda, const f
   return pi_check_launch("gemm_float32 (tiles)");
 }
 
+template <int WM, int WN, int EPI>
+static int launch_parts(float* C, long ldc, const float* A, long lda, const float* W, long ldw, int M, int N, int K, const Float32Plan& p, float* part,
+                        hipStream_t stream) {
+  constexpr size_t bytes = (size_t)2 * (WM + WN) * 2 * 3072;
+  static const hipError_t configured = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_float32_parts_kernel<WM, WN, EPI>),
+                                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+  if (configured != hipSuccess) return pi_fail("gemm_float32: cannot reserve %zu bytes of LDS: %s", bytes, hipGetErrorString(configured));
+  const int tiles_n = ceil_div(N, WN * 64);
+  hipLaunchKernelGGL((gemm_float32_parts_kernel<WM, WN, EPI>), dim3((unsigned)(ceil_div(M, WM * 64) * (long)tiles_n), p.splits), dim3(256), bytes, stream,
+                     C, ldc, A, lda, W, ldw, M, N, K, tiles_n, p.k_per_split, part);
+  return pi_check_launch("gemm_float32 (tiles in parts)");
+}
+
 template <int EPI>
 static int launch_tiles(float* C, long ldc, const float* A, long lda, const float* W, long ldw, int M, int N, int K, const Float32Plan& p, float* part,
                         hipStream_t stream) {
-  if (p.tm == 128 && p.tn == 128) return launch_tiles_of<128, 128, 2, EPI>(C, ldc, A, lda, W, ldw, M, N, K, p, part, stream);
-  if (p.tm == 128) return launch_tiles_of<128, 64, 3, EPI>(C, ldc, A, lda, W, ldw, M, N, K, p, part, stream);
-  return launch_tiles_of<64, 64, 4, EPI>(C, ldc, A, lda, W, ldw, M, N, K, p, part, stream);
+  if (p.tm == 64) return launch_tiles_of<64, 64, 4, EPI>(C, ldc, A, lda, W, ldw, M, N, K, p, part, stream);
+  if (p.tm == 192) return launch_parts<3, 2, EPI>(C, ldc, A, lda, W, ldw, M, N, K, p, part, stream);
+  if (p.tn == 256 && ldw <= PARTS_WIDE_MAX_STRIDE) return launch_parts<2, 4, EPI>(C, ldc, A, lda, W, ldw, M, N, K, p, part, stream);
+  return launch_parts<2, 2, EPI>(C, ldc, A, lda, W, ldw, M, N, K, p, part, stream);
 }
 
 // Enough waves for the memory whatever the matrix' rows are: blocks of four waves on 32 rows where that gives two per
@@ -480,7 +685,7 @@ extern "C" int pi_gemm_float32(void* C, long ldc, const void* A, long lda, const
 extern "C" int pi_gemm_float32_swiglu(void* C, long ldc, const void* A, long lda, const void* W, long ldw, int M, int N, int K, hipStream_t stream) {
   if (check_float32(M, N, K, A, lda, W, ldw, ldc, N / 2)) return -1;
   PI_REQUIRE(N % 32 == 0, "gemm_float32: the gated epilogue needs N (%d) to be a multiple of 32", N);
-  return launch_float32<EPI_SWIGLU>((float*)C, ldc, (const float*)A, lda, (const float*)W, ldw, M, N, K, plan(M, N, K, 0, false), nullptr, stream);
+  return launch_float32<EPI_SWIGLU>((float*)C, ldc, (const float*)A, lda, (const float*)W, ldw, M, N, K, plan(M, N, K, 0, 0), nullptr, stream);
 }
 
 // ------------------------------------------------------------------ adding pieces

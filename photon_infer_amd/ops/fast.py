@@ -357,7 +357,7 @@ def float32_gate_in_product(M: int, N: int, K: int, units: int) -> bool:
     One or two rows, which the general kernel streams faster: up to k of 2,048 (8,192 features, one row: 26.9 and 28.8 us, at
     3,072 39.5 and 39.6, at 4,096 69 and 51), with few features to 1,024 (2,048 features: 9.0 and 10.0; 256: 8.6 and 7.0)."""
     if M > FLOAT32_ROWS:
-        return _lib.load("core").pi_gemm_float32_pieces(M, N, K, GEMM_PART_FLOATS, 0) == 1
+        return _lib.load("core").pi_gemm_float32_pieces(M, N, K, GEMM_PART_FLOATS, 2) == 1
     blocks, general = N // 32, _general_streams_faster(M, N, K)
     if 4 * blocks >= 3 * units:
         return K <= 2048 or not general

@@ -5,7 +5,7 @@
 //
 // Walks the built-in sweep of shapes (and any given as arguments) through the lanes, waves,
 // blocks and steps of gemm_skinny_kernel, gemm_skinny_ring_kernel, gemm_mfma_kernel,
-// gemm_mfma_big_kernel in its six tile shapes, gemm_rows_kernel, gemm_float32_rows_kernel and gemm_float32_tile_kernel exactly as the kernels
+// gemm_mfma_big_kernel in its six tile shapes, gemm_rows_kernel, gemm_float32_rows_kernel, gemm_float32_tile_kernel and gemm_float32_parts_kernel exactly as the kernels
 // walk them (and, in the built-in sweep, through the
 // key and value fetches of the attention kernels' chunks for every head size and several page sizes), with the matrices row by row (several row
 // strides) and, where the sizes allow, in the weight-streaming kernels' tiled order.  Prints
@@ -188,8 +188,43 @@ static const Tiles BFLOAT16_TILES[] = {
     {"gemm_mfma_big<2, 3>", 128, 384, 8, true, 2}, {"gemm_mfma_big<2, 2>", 128, 256, 8, true, 3}, {"gemm_mfma_big<2, 1>", 128, 128, 8, true, 3},
 };
 static const Tiles FLOAT32_TILES[] = {                 // the rings of buffers, less the one in use
-    {"gemm_float32_tile<128, 128>", 128, 128, 4, false, 1}, {"gemm_float32_tile<128, 64>", 128, 64, 4, false, 2}, {"gemm_float32_tile<64, 64>", 64, 64, 4, false, 3},
+    {"gemm_float32_tile<64, 64>", 64, 64, 4, false, 3},
 };
+
+// The float32 tiles in parts: 64 rows a load, slabs of 16 floats, one more slab than there are, and one more.
+static const Tiles FLOAT32_PARTS[] = {
+    {"gemm_float32_parts<2, 2>", 128, 128, 4, false, 2}, {"gemm_float32_parts<3, 2>", 192, 128, 4, false, 2}, {"gemm_float32_parts<2, 4>", 128, 256, 4, false, 2},
+};
+static bool parts_operand(const Tiles& t, const char* operand, const Shape& s, long R, long ld, long row0, int tile, int k_lo, int k_hi) {
+  const int rows = (int)A::lmin(tile, R - row0), k_range = k_hi - k_lo, slabs = (k_range + A::PARTS_SLAB - 1) / A::PARTS_SLAB;
+  const A::Descriptor d = A::tile_descriptor(row0, ld, k_lo, k_hi, rows);
+  if (d.base < 0 || d.bytes <= 0 || d.base * 2 + d.bytes > ((R - 1) * ld + 2 * s.K) * 2 || d.bytes >= 0x7ffffff0L)
+    return fail(t.kernel, operand, s, ld, 0, d.base, "the descriptor leaves the operand");
+  for (int load = 0; load < tile / 64; ++load)
+    for (int tid = 0; tid < 256; ++tid) {
+      const int row = A::parts_row(load, tid), piece = A::parts_piece(tid);
+      for (int sl = 0; sl < slabs + t.ahead; ++sl) {
+        ++fetches;
+        const long off = A::tile_slab_offset(A::tile_lane_offset(row, rows, ld, piece), sl * A::PARTS_SLAB, piece, k_range);
+        const int k = sl * A::PARTS_SLAB + piece * 8;
+        const bool used = row < rows && k < k_range;
+        if (used ? off + 16 > d.bytes : off < d.bytes) return fail(t.kernel, operand, s, ld, 0, off, "on the wrong side of its descriptor");
+        if (used && d.base * 2 + off != ((row0 + row) * ld + k_lo + k) * 2) return fail(t.kernel, operand, s, ld, 0, off, "a used fetch is not the lane's row and k");
+      }
+    }
+  return true;
+}
+static bool parts(const Shape& s, long lda, long ldw, const Tiles& t) {
+  const A::KSplit cut = A::cut_k(s.K, s.splits, 32);
+  for (int by = 0; by < cut.splits; ++by) {
+    const int k_lo = 2 * by * cut.k_per_block, k_hi = 2 * A::imin(s.K, (by + 1) * cut.k_per_block);
+    for (long m0 = 0; m0 < s.M; m0 += t.rows_a)
+      if (!parts_operand(t, "A", s, s.M, 2 * lda, m0, t.rows_a, k_lo, k_hi)) return false;
+    for (long n0 = 0; n0 < s.N; n0 += t.rows_w)
+      if (!parts_operand(t, "W", s, s.N, 2 * ldw, n0, t.rows_w, k_lo, k_hi)) return false;
+  }
+  return true;
+}
 
 // ------------------------------------------------------------------ 33..128 tokens
 // The activations are a tile of 64 or 128 rows; of the weights a block's eight waves take 32 rows by a quarter of each step's
@@ -335,6 +370,8 @@ static bool check(const Shape& s) {
     } else {
       for (const Tiles& t : FLOAT32_TILES)
         if (!tiles(s, ld, ld, t, 2)) return false;
+      for (const Tiles& t : FLOAT32_PARTS)
+        if (!parts(s, ld, ld, t)) return false;
     }
   }
   if (s.N % 16 == 0 && s.K % 64 == 0) {                // the streaming copy of the weights

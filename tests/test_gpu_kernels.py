@@ -293,6 +293,60 @@ def test_float32_products_on_the_matrix_cores(_ops, M, N, K):
     close(odd, (a_full[:, 1:K + 1].double() @ w.double().cpu().t()), rel, "float32, unaligned")
 
 
+# the float32 tiles in parts: a row or a column more than whole tiles, k that ends inside a slab of 16; 128 x 128, 192 x 128, 128 x 256, pieces
+FLOAT32_PARTS = [(193, 16400, 100), (385, 8224, 108), (385, 28000, 260), (1921, 2208, 36), (129, 2048, 8192)]
+
+
+@pytest.mark.parametrize("M,N,K", FLOAT32_PARTS)
+def test_float32_tiles_in_parts(_ops, M, N, K):
+    """Stored, added and through the gated unit: 32-bit sums of K products, off by about 2^-24 sqrt(K) of their size."""
+    _ops.use_fast_kernels(True)
+    rel = 2 ** -24 * (4 + math.sqrt(K))
+    a = torch.randn(M, K + 8, generator=gen(M)).to(DEV)[:, 4:K + 4]
+    w = (torch.randn(N, K + 4, generator=gen(N)) / K ** 0.5).to(DEV)[:, :K]
+    want = a.double() @ w.double().t()
+    full = torch.zeros(M, N + 3, device=DEV)
+    _ops.gemm(full[:, 1:N + 1], a, w)
+    close(full[:, 1:N + 1], want.cpu(), rel, f"{M}x{N}x{K}")
+    assert full[:, 0].abs().max() == 0 and full[:, N + 1:].abs().max() == 0
+    x = torch.randn(M, N, generator=gen(9)).to(DEV)
+    want_x = (want + x.double()).cpu()
+    _ops.gemm(x, a, w, accumulate=True)
+    close(x, want_x, rel, "added")
+    if N % 32 == 0:
+        g, u = want.view(M, N // 32, 2, 16).unbind(2)
+        out = torch.empty(M, N // 2, device=DEV)
+        _ops.gemm_swiglu(out, a, w.contiguous(), 16)
+        close(out, P.swiglu(g.reshape(M, -1).cpu(), u.reshape(M, -1).cpu()), 2 * rel + 2 ** -22, "gated")
+
+
+@pytest.mark.parametrize("M,N,K", FLOAT32_PARTS[:3])
+def test_float32_floats_that_have_no_parts(_ops, M, N, K):
+    """Infinities, a NaN, floats above the largest bfloat16, and operands so small that their last parts would be lost: as 64 bits have them."""
+    rel = 2 ** -24 * (4 + math.sqrt(K))
+
+    def check(a, w, what):
+        want, out = a.double() @ w.double().t(), torch.empty(M, N, device=DEV)
+        _ops.gemm(out, a, w)
+        assert torch.equal(out.isnan(), want.isnan()) and torch.equal(out.isinf(), want.isinf()), what
+        assert torch.equal(out.isposinf(), want.isposinf()), what
+        off, size = [torch.where(want.isfinite(), t, 0.0) for t in (out.double() - want, want)]
+        rows = size.norm(dim=1).clamp_min(1e-300)
+        assert (off.norm(dim=1) <= 2 * rel * rows).all(), what
+        assert (off.norm(dim=0) <= 2 * rel * (off * 0 + rows[:, None]).norm(dim=0)).all(), what
+
+    a, w = torch.randn(M, K, generator=gen(M)).to(DEV), (torch.randn(N, K, generator=gen(N)) / 16).to(DEV)
+    odd = a.clone()
+    odd[3, 5], odd[130, K - 1], odd[131, 0], odd[M - 1, 17] = math.inf, -math.inf, math.nan, 3.4e38
+    check(odd, w, "activations")
+    odd = w.clone()
+    odd[N - 1, 5], odd[70, K - 1] = -math.inf, math.inf
+    check(a, odd, "weights")
+    check(a * 2.0 ** -113, w, "small activations")
+    check(a, w * 2.0 ** -110, "small weights")
+    check(a * 0.0, w, "zeros")
+
+
 @pytest.mark.parametrize("M,N,K,kernel", [(1, 2048, 2048, "pi_gemm_general"), (2, 520, 516, "pi_gemm_general"), (1, 2048, 512, "pi_gemm_float32"),
                                           (3, 2048, 2048, "pi_gemm_float32"), (8, 8192, 8192, "pi_gemm_general"), (9, 8192, 8192, "pi_gemm_float32")])
 def test_few_float32_rows_go_to_the_kernel_that_streams_the_weights_faster(_ops, M, N, K, kernel):
