@@ -84,6 +84,20 @@ __device__ inline float wave_max(float v) {
   return v;
 }
 
+// ---- moves between the lanes of a row of 16 through the data-parallel primitives, no trip through LDS
+template <int CTRL>
+__device__ inline float dpp_move(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
+}
+// the sum over the 16 lanes of a row, in every lane of the row
+__device__ inline float row16_sum(float v) {
+  v += dpp_move<0xB1>(v);       // quad_perm [1, 0, 3, 2]
+  v += dpp_move<0x4E>(v);       // quad_perm [2, 3, 0, 1]
+  v += dpp_move<0x124>(v);      // row_ror 4
+  v += dpp_move<0x128>(v);      // row_ror 8
+  return v;
+}
+
 // A rotated pair: (a, b) turned by the angle whose cosine and sine are c and s.  One spelling
 // for every kernel that rotates, with the roundings fixed, so that a query or key comes out the
 // same wherever it is rotated.

@@ -130,19 +130,6 @@ extern "C" int pi_causal_conv_silu(float* out, long out_stride, const float* in,
 // In memory a request's state is kept in the walk's own order, [head][slice of four columns][i][lane]
 // (NR * 64 floats per slice), so that a wave loads and stores it in whole 256-byte rows.
 // Nothing else reads it; a cleared row is a zero state in any order.
-template <int CTRL>
-__device__ inline float dpp_move(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
-}
-// the sum over the 16 lanes of a row, in every lane of the row
-__device__ inline float row16_sum(float v) {
-  v += dpp_move<0xB1>(v);       // quad_perm [1, 0, 3, 2]
-  v += dpp_move<0x4E>(v);       // quad_perm [2, 3, 0, 1]
-  v += dpp_move<0x124>(v);      // row_ror 4
-  v += dpp_move<0x128>(v);      // row_ror 8
-  return v;
-}
-
 template <int LANES> __device__ inline float lanes_sum(float v) {
   static_assert(LANES == 16 || LANES == 32, "a column's lanes");
   v = row16_sum(v);
@@ -417,13 +404,24 @@ extern "C" int pi_gated_group_norm(void* out, int out_dtype, long out_stride, co
 // over a, beta over b.  One wave per (token, key head) and per (token, head).
 enum ScanKind : int { SCAN_CHANNEL_DELTA = 0, SCAN_HEAD_DELTA = 1, SCAN_DECAYED_OUTER = 2 };
 
+// Tokens that the request of token t brings; called by a whole wave.
+__device__ inline int tokens_beside(const int* __restrict__ q_start, int R, long t) {
+  for (int r0 = 0; r0 < R; r0 += PI_WAVE) {
+    const int r = min(r0 + (int)(threadIdx.x % PI_WAVE), R - 1), from = q_start[r], to = q_start[r + 1];
+    const unsigned long long mine = __ballot(from <= t && t < to);
+    if (mine) return __shfl(to - from, __ffsll(mine) - 1, PI_WAVE);
+  }
+  return 0;
+}
+
 __global__ __launch_bounds__(PI_WAVE) void delta_prepare_kernel(float* __restrict__ qkv, long qkv_stride, float* __restrict__ a,
                                                                long a_stride, const float* __restrict__ dt_bias,
                                                                const float* __restrict__ A_log, float* __restrict__ b,
                                                                long b_stride, int H, int G, int d, float q_scale, float unit_eps,
-                                                               int kind, float inv_tau) {
+                                                               int kind, float inv_tau, const int* __restrict__ q_start, int R, int upto) {
   const long t = blockIdx.x;
   const int j = blockIdx.y, lane = threadIdx.x;
+  if (upto > 0 && tokens_beside(q_start, R, t) > upto) return;
   if (j < G) {
     float* q = qkv + t * qkv_stride + (long)j * d;
     if (kind == SCAN_DECAYED_OUTER) {
@@ -469,7 +467,7 @@ template <int NR, bool SHORT, int KIND>
 __global__ __launch_bounds__((PI_SCAN_WAVES + 1) * PI_WAVE) void delta_scan_kernel(
     float* __restrict__ o, long o_stride, const float* __restrict__ qkv, long qkv_stride, const float* __restrict__ decay,
     long decay_stride, const float* __restrict__ beta, long beta_stride, const int* __restrict__ q_start,
-    const int* __restrict__ slots, float* __restrict__ state, long state_stride, int H, int G, int d, int dv, int vec) {
+    const int* __restrict__ slots, float* __restrict__ state, long state_stride, int H, int G, int d, int dv, int vec, int upto) {
   constexpr int W = ScanShape<NR, SHORT>::W, CH = ScanShape<NR, SHORT>::CH;
   __shared__ __attribute__((aligned(16))) float sq[2][CH * W];
   __shared__ __attribute__((aligned(16))) float sk[2][CH * W];
@@ -479,7 +477,7 @@ __global__ __launch_bounds__((PI_SCAN_WAVES + 1) * PI_WAVE) void delta_scan_kern
   const int wave = threadIdx.x / PI_WAVE, lane = threadIdx.x % PI_WAVE, part = lane % 16;
   const int g = h / (H / G);
   const int qs = q_start[r], n = q_start[r + 1] - qs;
-  if (n <= 0) return;
+  if (n <= 0 || (upto > 0 && n > upto)) return;
   const int chunks = (n + CH - 1) / CH;
   const long q_col = (long)g * d, k_col = (long)G * d + (long)g * d, v_col = 2L * G * d + (long)h * dv + z * PI_SCAN_COLUMNS;
 
@@ -607,7 +605,7 @@ template <int SNR, int KIND, int LANES>
 __global__ __launch_bounds__((PI_SCAN_WAVES + 1) * PI_WAVE) void delta_scan_ahead_kernel(
     float* __restrict__ o, long o_stride, const float* __restrict__ qkv, long qkv_stride, const float* __restrict__ decay,
     long decay_stride, const float* __restrict__ beta, long beta_stride, const int* __restrict__ q_start,
-    const int* __restrict__ slots, float* __restrict__ state, long state_stride, int H, int G, int d, int dv, int vec) {
+    const int* __restrict__ slots, float* __restrict__ state, long state_stride, int H, int G, int d, int dv, int vec, int upto) {
   constexpr int W = ScanShape<SNR, false>::W, CH = ScanShape<SNR, false>::CH, NR = SNR * 16 / LANES;     // rows of a lane: SNR in a state row's order
   __shared__ __attribute__((aligned(16))) float sq[2][CH * W];
   __shared__ __attribute__((aligned(16))) float sk[2][CH * W];
@@ -618,7 +616,7 @@ __global__ __launch_bounds__((PI_SCAN_WAVES + 1) * PI_WAVE) void delta_scan_ahea
   const int wave = threadIdx.x / PI_WAVE, lane = threadIdx.x % PI_WAVE, part = lane % LANES;
   const int g = h / (H / G);
   const int qs = q_start[r], n = q_start[r + 1] - qs;
-  if (n <= 0) return;
+  if (n <= 0 || (upto > 0 && n > upto)) return;
   const int chunks = (n + CH - 1) / CH;
   const long q_col = (long)g * d, k_col = (long)G * d + (long)g * d, v_col = 2L * G * d + (long)h * dv + col0;
 
@@ -735,10 +733,11 @@ __global__ __launch_bounds__((PI_SCAN_WAVES + 1) * PI_WAVE) void delta_scan_ahea
 
 // qkv, a and b are changed in place (unit vectors or scaled queries, decays, beta); o gets the read-outs.
 // kind: a ScanKind.  SCAN_HEAD_DELTA: a is [T, H] and dt_bias [H].  SCAN_DECAYED_OUTER: b is not read, A_log neither,
-// unit_eps neither; tau is the root taken of the sigmoid.
+// unit_eps neither; tau is the root taken of the sigmoid.  `upto` > 0: only the requests that bring up to so many tokens are
+// walked, and `longest` is theirs (the others run in chunks, delta_chunks.hip).
 extern "C" int pi_delta_scan(float* o, long o_stride, float* qkv, long qkv_stride, float* a, long a_stride,
                              const float* dt_bias, const float* A_log, float* b, long b_stride, const int* q_start,
-                             const int* slots, int R, int T, int longest, float* state, long state_stride, int H, int G, int d, int dv,
+                             const int* slots, int R, int T, int longest, int upto, float* state, long state_stride, int H, int G, int d, int dv,
                              float q_scale, float unit_eps, int kind, float tau, hipStream_t stream) {
   PI_REQUIRE(H > 0 && H <= 32767 && G > 0 && H % G == 0 && d > 0 && dv > 0, "state walk: bad sizes heads=%d kv_heads=%d dim=%d vdim=%d", H, G, d, dv);
   PI_REQUIRE(kind >= SCAN_CHANNEL_DELTA && kind <= SCAN_DECAYED_OUTER, "state walk: unknown kind %d", kind);
@@ -749,7 +748,7 @@ extern "C" int pi_delta_scan(float* o, long o_stride, float* qkv, long qkv_strid
   PI_REQUIRE(R >= 0 && T >= 0 && state_stride >= pi_scan_state_floats(H, d, dv), "state walk: a state row of %ld floats cannot hold %d x %d x %d", state_stride, H, d, dv);
   if (R == 0 || T == 0) return 0;
   hipLaunchKernelGGL(delta_prepare_kernel, dim3(T, G + H), dim3(PI_WAVE), 0, stream, qkv, qkv_stride, a, a_stride, dt_bias, A_log, b,
-                     b_stride, H, G, d, q_scale, unit_eps, kind, kind == SCAN_DECAYED_OUTER ? 1.0f / tau : 0.f);
+                     b_stride, H, G, d, q_scale, unit_eps, kind, kind == SCAN_DECAYED_OUTER ? 1.0f / tau : 0.f, q_start, R, upto);
   if (pi_check_launch("delta_prepare")) return -1;
   // bit 0: q and k may be fetched 16 bytes at a time; bit 1: the decays too
   const int vec = (d % 4 == 0 && qkv_stride % 4 == 0 && (uintptr_t)qkv % 16 == 0 ? 1 : 0) |
@@ -761,7 +760,7 @@ extern "C" int pi_delta_scan(float* o, long o_stride, float* qkv, long qkv_strid
   // requests of one token beside 200, 8 heads of 64 x 64: 50 and 88; eight of one, 16 heads of 128 x 128: 9.2 and 12.6).
   const int by16 = (dv + PI_SCAN_COLUMNS - 1) / PI_SCAN_COLUMNS;
   const bool wide = longest > 2 && (long)R * H * by16 * 2 <= compute_units();
-#define PI_DELTA_ARGS o, o_stride, qkv, qkv_stride, a, a_stride, b, b_stride, q_start, slots, state, state_stride, H, G, d, dv, vec
+#define PI_DELTA_ARGS o, o_stride, qkv, qkv_stride, a, a_stride, b, b_stride, q_start, slots, state, state_stride, H, G, d, dv, vec, upto
 #define PI_DELTA_GO(COLUMN_BLOCKS, ...) \
   hipLaunchKernelGGL((__VA_ARGS__), dim3(R, H, COLUMN_BLOCKS), dim3((PI_SCAN_WAVES + 1) * PI_WAVE), 0, stream, PI_DELTA_ARGS)
 #define PI_LAUNCH_DELTA2(NR_, KIND_)                                                                                  \

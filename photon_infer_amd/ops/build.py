@@ -29,7 +29,7 @@ CSRC_DIR = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__
 # matrix-core kernels that only the bfloat16 path uses.
 MODULES: Dict[str, List[str]] = {
     "core": ["elementwise.hip", "gemm_general.hip", "gemm_float32.hip", "attention_general.hip", "attention_float32.hip", "attention_float32_decode.hip", "sampling.hip", "stream_norm.hip",
-             "matrix_memory.hip", "routed_experts.hip", "recurrent.hip", "state_space_chunks.hip", "latent.hip", "gated_recurrence.hip", "hyper_streams.hip", "retention.hip"],
+             "matrix_memory.hip", "routed_experts.hip", "recurrent.hip", "state_space_chunks.hip", "delta_chunks.hip", "latent.hip", "gated_recurrence.hip", "hyper_streams.hip", "retention.hip"],
     "bf16": ["gemm_mfma.hip", "gemm_skinny.hip", "attention_mfma.hip", "attention_decode.hip"],
     # host only: cache manager bookkeeping (needs no GPU and no hipcc)
     "runtime": ["runtime/cache.cpp"],

@@ -265,6 +265,70 @@ def test_delta_rule_whole_in_portions_and_token_by_token(sizes):
         assert bool((state[1] == 0).all())
 
 
+@pytest.mark.parametrize("sizes", [(4, 2, 64, 16), (2, 2, 128, 128), (2, 1, 192, 48), (1, 1, 256, 144)])
+@pytest.mark.parametrize("per_head", [False, True])
+def test_delta_rule_in_chunks_beside_single_tokens(sizes, per_head):
+    """Sixteen tokens at a time: whole and partial chunks, requests that walk beside them, a second portion on top; the
+    bounds of the walk's tests.  Step 2 holds no request that walks."""
+    from photon_infer_amd import ops
+    ops.use_fast_kernels(True)
+    H, G, d, dv = sizes
+    T = {"a": 131, "b": 3, "c": 19, "d": 64, "e": 5}
+    cuts = {"a": [48, 83], "b": [1, 2], "c": [3, 16], "d": [47, 17], "e": [2, 3]}
+    A_log, dt_bias = randn(H, seed=1, scale=0.5) - 1.0, randn(H if per_head else H * d, seed=2)
+    data = {n: delta_inputs(t, H, G, d, dv, 100 * i) for i, (n, t) in enumerate(T.items())}
+    if per_head:
+        data = {n: (q, k, v, a[:, :H].contiguous(), b) for n, (q, k, v, a, b) in data.items()}
+    wide = lambda x: x.repeat_interleave(d, dim=-1) if per_head else x
+    want = {n: delta_plain(q, k, v, wide(a), b, wide(dt_bias), A_log, H, d) for n, (q, k, v, a, b) in data.items()}
+    slot = {n: 5 - i for i, n in enumerate(T)}
+    state = torch.zeros((6, ops.scan_state_floats(H, d, dv) + 3), device=DEV)
+    got = {n: [] for n in T}
+    for number, step in enumerate(in_steps(T, cuts)):
+        cat = lambda idx: torch.cat([data[n][idx][i:j].reshape(j - i, -1) for n, i, j in step])
+        o = torch.full((sum(j - i for _, i, j in step) + 1, H * dv), 7.0, device=DEV)
+        qkv, a, b = dev32(torch.cat([cat(0), cat(1), cat(2)], dim=1)), dev32(cat(3)), dev32(cat(4))
+        with library_calls() as names:
+            ops.delta_scan(o[:-1], qkv, a, dev32(dt_bias), dev32(A_log), b, state_ctx([j - i for _, i, j in step], [slot[n] for n, _, _ in step]),
+                           state[:, :-3], H, G, d, dv, d ** -0.5, 1e-6, kind="head_delta" if per_head else "channel_delta")
+        assert names == ["pi_delta_chunks", "pi_delta_scan"], number
+        assert bool((o[-1] == 7.0).all())
+        for (n, i, j), part in zip(step, torch.split(o[:-1], [j - i for _, i, j in step])):
+            got[n].append(part)
+    for n in T:
+        close(torch.cat(got[n]), want[n][0].reshape(T[n], -1), f"{sizes} {n}", 5e-5)
+        close(ops.unpack_scan_state(state[slot[n], :-3], H, d, dv), want[n][1], f"{sizes} {n} state", 5e-5)
+    assert bool((state[0] == 0).all()) and bool((state[:, -3:] == 0).all())
+
+
+@pytest.mark.parametrize("bad", [math.nan, math.inf])
+@pytest.mark.parametrize("where", ["value", "key", "decay"])
+def test_what_is_not_finite_reaches_no_token_before_it(bad, where):
+    """In chunks: token 37 of 70; a value's column alone, a key's or a decay's head alone, and no other request."""
+    from photon_infer_amd import ops
+    ops.use_fast_kernels(True)
+    H, G, d, dv, T, at = 2, 2, 64, 32, 70, 37
+    q, k, v, a, b = (x.reshape(2 * T, -1) for x in delta_inputs(2 * T, H, G, d, dv, 3))
+    A_log, dt_bias = randn(H, seed=1, scale=0.5) - 1.0, randn(H * d, seed=2)
+
+    def run(k, v, a):
+        state, o = torch.zeros((2, ops.scan_state_floats(H, d, dv)), device=DEV), torch.empty((2 * T, H * dv), device=DEV)
+        ops.delta_scan(o, dev32(torch.cat([q, k, v], dim=1)), dev32(a), dev32(dt_bias), dev32(A_log), dev32(b), state_ctx([T, T], [1, 0]), state,
+                       H, G, d, dv, d ** -0.5, 1e-6)
+        return o
+
+    clean = run(k, v, a)
+    k, v, a = k.clone(), v.clone(), a.clone()
+    {"value": v, "key": k, "decay": a}[where][at, 5] = bad
+    o = run(k, v, a)
+    hit = torch.zeros_like(o, dtype=torch.bool)
+    hit[at:T, 5 if where == "value" else slice(0, dv)] = True
+    # the chunk that holds the token adds its sixteen terms one by one instead of four at a time: 16 roundings of its largest sum
+    assert (o[~hit] - clean[~hit]).abs().max() <= 16 * 2 ** -24 * clean.abs().max()
+    if not (where == "decay" and bad == math.inf):       # softplus of infinity: the channel forgets everything, which is no fault
+        assert not o[hit].isfinite().any()
+
+
 @pytest.mark.parametrize("decode", [False, True])
 def test_a_write_is_recalled_after_hundreds_of_tokens_and_forgotten_by_its_channel_alone(decode):
     """Token 0 writes v0 under key e0 with beta 1.  600 tokens follow with keys in the other channels: with channel 0's
