@@ -127,6 +127,10 @@ extern "C" int pi_causal_conv_silu(float* out, long out_stride, const float* in,
 // parallel in the tokens.  The walk itself is multiply-adds on registers and LDS reads.  One
 // barrier per chunk hands a buffer over.
 //
+// Beyond two tokens per request the grid has requests outermost, so that a long request's blocks lie on all dies (innermost they were every
+// R-th block: of 32 requests all on one die, 64 tokens beside 31 single ones, 32 heads of 64 with a state of 128, 246 us, 68 so), and
+// heads innermost, so that the blocks of a head, which read the same vectors, share a die.
+//
 // In memory a request's state is kept in the walk's own order, [head][slice of four columns][i][lane]
 // (NR * 64 floats per slice), so that a wave loads and stores it in whole 256-byte rows.
 // Nothing else reads it; a cleared row is a zero state in any order.
@@ -151,6 +155,18 @@ extern "C" long pi_scan_state_floats(int heads, int rows, int cols) {
   const int nr = scan_rows_per_lane(rows);
   return (long)heads * ((cols + PI_SCAN_COLUMNS - 1) / PI_SCAN_COLUMNS) * PI_SCAN_WAVES * nr * PI_WAVE;
 }
+
+// Which head, slice of value columns and request a block walks.  In a step of one or two tokens per request all blocks are alike, and
+// requests lie innermost, in any number.
+struct ScanBlock {
+  int head, slice, request;
+};
+template <bool SHORT> __device__ inline ScanBlock scan_block() {
+  if constexpr (SHORT) return ScanBlock{(int)blockIdx.y, (int)blockIdx.z, (int)blockIdx.x};
+  else return ScanBlock{(int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z};
+}
+static inline dim3 scan_grid(bool is_short, int heads, int slices, int requests) { return is_short ? dim3(requests, heads, slices) : dim3(heads, slices, requests); }
+#define PI_SCAN_REQUESTS 65535       // of a launch with requests outermost
 
 // SHORT: a step in which no request brings more than two tokens (decoding) is staged two tokens at a time:
 // few registers and little LDS, so that many blocks share a compute unit while they wait for their states.
@@ -218,7 +234,8 @@ __global__ __launch_bounds__((PI_SCAN_WAVES + 1) * PI_WAVE) void state_space_sca
   __shared__ __attribute__((aligned(16))) float sB[2][CH * W];
   __shared__ __attribute__((aligned(16))) float sC[2][CH * W];
   __shared__ float sx[2][CH][PI_SCAN_COLUMNS], sdt[2][CH], sa[2][CH];
-  const int r = blockIdx.x, h = blockIdx.y, z = blockIdx.z;
+  const ScanBlock at = scan_block<SHORT>();
+  const int h = at.head, z = at.slice, r = at.request;
   const int wave = threadIdx.x / PI_WAVE, lane = threadIdx.x % PI_WAVE, part = lane % 16;
   const int g = h / (H / G);
   const int qs = q_start[r], n = q_start[r + 1] - qs;
@@ -258,7 +275,7 @@ __global__ __launch_bounds__((PI_SCAN_WAVES + 1) * PI_WAVE) void state_space_sca
   const int cw = wave * 4 + lane / 16;                 // this lane's column within the block
   const int col = z * PI_SCAN_COLUMNS + cw;
   const bool live = col < P;
-  float* Sg = state + (long)slots[r] * state_stride + (((long)h * gridDim.z + z) * PI_SCAN_WAVES + (wave & 3)) * NR * PI_WAVE + lane;
+  float* Sg = state + (long)slots[r] * state_stride + (((long)h * ((P + PI_SCAN_COLUMNS - 1) / PI_SCAN_COLUMNS) + z) * PI_SCAN_WAVES + (wave & 3)) * NR * PI_WAVE + lane;
   const float skip = Dskip[h];
   if (wave < PI_SCAN_WAVES) {
 #pragma unroll
@@ -308,11 +325,15 @@ extern "C" int pi_state_space_scan(float* y, long y_stride, const float* xbc, lo
   PI_REQUIRE(R >= 0 && state_stride >= pi_scan_state_floats(H, N, P), "state space: a state row of %ld floats cannot hold %d x %d x %d", state_stride, H, N, P);
   if (R == 0) return 0;
   const int vec = N % 4 == 0 && xbc_stride % 4 == 0 && ((long)H * P) % 4 == 0 && (uintptr_t)xbc % 16 == 0;
-  const dim3 grid(R, H, (P + PI_SCAN_COLUMNS - 1) / PI_SCAN_COLUMNS), block((PI_SCAN_WAVES + 1) * PI_WAVE);
-#define PI_LAUNCH_SS1(NR_, SHORT_)                                                                                                       \
-  hipLaunchKernelGGL((state_space_scan_kernel<NR_, SHORT_>), grid, block, 0, stream, y, y_stride, xbc, xbc_stride, dt_raw, dt_stride, \
-                     dt_bias, A_log, Dskip, q_start, slots, upto, state, state_stride, H, P, N, G, vec)
-#define PI_LAUNCH_SS(NR_) do { if (longest <= 2) PI_LAUNCH_SS1(NR_, true); else PI_LAUNCH_SS1(NR_, false); } while (0)
+  const int slices = (P + PI_SCAN_COLUMNS - 1) / PI_SCAN_COLUMNS;
+#define PI_LAUNCH_SS1(NR_, SHORT_)                                                                                                          \
+  for (int r0 = 0, n; r0 < R; r0 += n) {                                                                                                    \
+    n = (SHORT_) || R - r0 < PI_SCAN_REQUESTS ? R - r0 : PI_SCAN_REQUESTS;                                                                  \
+    hipLaunchKernelGGL((state_space_scan_kernel<NR_, SHORT_>), scan_grid(SHORT_, H, slices, n), dim3((PI_SCAN_WAVES + 1) * PI_WAVE), 0,     \
+                       stream, y, y_stride, xbc, xbc_stride, dt_raw, dt_stride, dt_bias, A_log, Dskip, q_start + r0, slots + r0, upto, state, \
+                       state_stride, H, P, N, G, vec);                                                                                      \
+  }
+#define PI_LAUNCH_SS(NR_) do { if (longest <= 2) { PI_LAUNCH_SS1(NR_, true) } else { PI_LAUNCH_SS1(NR_, false) } } while (0)
   switch (nr) {
     case 1: PI_LAUNCH_SS(1); break;
     case 2: PI_LAUNCH_SS(2); break;
@@ -473,7 +494,9 @@ __global__ __launch_bounds__((PI_SCAN_WAVES + 1) * PI_WAVE) void delta_scan_kern
   __shared__ __attribute__((aligned(16))) float sk[2][CH * W];
   __shared__ __attribute__((aligned(16))) float sg[2][KIND == SCAN_HEAD_DELTA ? 4 : CH * W];
   __shared__ float sv[2][CH][PI_SCAN_COLUMNS], sbeta[2][CH], sdecay[2][CH];
-  const int r = blockIdx.x, h = blockIdx.y, z = blockIdx.z;
+  const int by16 = (dv + PI_SCAN_COLUMNS - 1) / PI_SCAN_COLUMNS;
+  const ScanBlock at = scan_block<SHORT>();
+  const int h = at.head, z = at.slice, r = at.request;
   const int wave = threadIdx.x / PI_WAVE, lane = threadIdx.x % PI_WAVE, part = lane % 16;
   const int g = h / (H / G);
   const int qs = q_start[r], n = q_start[r + 1] - qs;
@@ -517,7 +540,7 @@ __global__ __launch_bounds__((PI_SCAN_WAVES + 1) * PI_WAVE) void delta_scan_kern
   const int cw = wave * 4 + lane / 16;                 // this lane's column within the block
   const int col = z * PI_SCAN_COLUMNS + cw;
   const bool live = col < dv;
-  float* Sg = state + (long)slots[r] * state_stride + (((long)h * gridDim.z + z) * PI_SCAN_WAVES + (wave & 3)) * NR * PI_WAVE + lane;
+  float* Sg = state + (long)slots[r] * state_stride + (((long)h * by16 + z) * PI_SCAN_WAVES + (wave & 3)) * NR * PI_WAVE + lane;
   if (wave < PI_SCAN_WAVES) {
 #pragma unroll
     for (int i = 0; i < NR; ++i) s[i] = Sg[i * PI_WAVE];
@@ -612,7 +635,9 @@ __global__ __launch_bounds__((PI_SCAN_WAVES + 1) * PI_WAVE) void delta_scan_ahea
   __shared__ __attribute__((aligned(16))) float sg[2][KIND == SCAN_HEAD_DELTA ? 4 : CH * W];
   constexpr int COLUMNS = PI_SCAN_WAVES * (PI_WAVE / LANES);
   __shared__ float sv[2][CH][COLUMNS], sbeta[2][CH], sdecay[2][CH];
-  const int r = blockIdx.x, h = blockIdx.y, col0 = blockIdx.z * COLUMNS;
+  const int by16 = (dv + PI_SCAN_COLUMNS - 1) / PI_SCAN_COLUMNS;
+  const ScanBlock at = scan_block<false>();
+  const int h = at.head, col0 = at.slice * COLUMNS, r = at.request;
   const int wave = threadIdx.x / PI_WAVE, lane = threadIdx.x % PI_WAVE, part = lane % LANES;
   const int g = h / (H / G);
   const int qs = q_start[r], n = q_start[r + 1] - qs;
@@ -661,7 +686,6 @@ __global__ __launch_bounds__((PI_SCAN_WAVES + 1) * PI_WAVE) void delta_scan_ahea
   const int col = col0 + cw;
   const bool live = col < dv;
   // a state row holds its columns by sixteen, four to a wave of sixteen lanes each, whatever the lanes here are
-  const int by16 = (dv + PI_SCAN_COLUMNS - 1) / PI_SCAN_COLUMNS;
   const long row = ((long)(h * by16 + col / 16) * PI_SCAN_WAVES + col % 16 / 4) * SNR + part % (LANES / 16) * NR;
   float* Sg = state + (long)slots[r] * state_stride + row * PI_WAVE + col % 4 * 16 + part / (LANES / 16);
   if (wave < PI_SCAN_WAVES) {
@@ -760,17 +784,20 @@ extern "C" int pi_delta_scan(float* o, long o_stride, float* qkv, long qkv_strid
   // requests of one token beside 200, 8 heads of 64 x 64: 50 and 88; eight of one, 16 heads of 128 x 128: 9.2 and 12.6).
   const int by16 = (dv + PI_SCAN_COLUMNS - 1) / PI_SCAN_COLUMNS;
   const bool wide = longest > 2 && (long)R * H * by16 * 2 <= compute_units();
-#define PI_DELTA_ARGS o, o_stride, qkv, qkv_stride, a, a_stride, b, b_stride, q_start, slots, state, state_stride, H, G, d, dv, vec, upto
-#define PI_DELTA_GO(COLUMN_BLOCKS, ...) \
-  hipLaunchKernelGGL((__VA_ARGS__), dim3(R, H, COLUMN_BLOCKS), dim3((PI_SCAN_WAVES + 1) * PI_WAVE), 0, stream, PI_DELTA_ARGS)
-#define PI_LAUNCH_DELTA2(NR_, KIND_)                                                                                  \
-  do {                                                                                                                \
-    constexpr bool LONG_KEYS = (NR_) >= 8;                                                                            \
-    constexpr int AHEAD_NR = LONG_KEYS ? (NR_) : 8;                                                                   \
-    if (longest <= 2) PI_DELTA_GO(by16, delta_scan_kernel<NR_, true, KIND_>);                                         \
-    else if (LONG_KEYS && wide) PI_DELTA_GO(by16 * 2, delta_scan_ahead_kernel<AHEAD_NR, KIND_, 32>);                  \
-    else if ((NR_) >= 16 && (KIND_) != SCAN_HEAD_DELTA) PI_DELTA_GO(by16, delta_scan_ahead_kernel<16, KIND_, 16>);    \
-    else PI_DELTA_GO(by16, delta_scan_kernel<NR_, false, KIND_>);                                                     \
+#define PI_DELTA_ARGS o, o_stride, qkv, qkv_stride, a, a_stride, b, b_stride, q_start + r0, slots + r0, state, state_stride, H, G, d, dv, vec, upto
+#define PI_DELTA_GO(SHORT_, COLUMN_BLOCKS, ...)                                                                                            \
+  for (int r0 = 0, n; r0 < R; r0 += n) {                                                                                                   \
+    n = (SHORT_) || R - r0 < PI_SCAN_REQUESTS ? R - r0 : PI_SCAN_REQUESTS;                                                                 \
+    hipLaunchKernelGGL((__VA_ARGS__), scan_grid(SHORT_, H, COLUMN_BLOCKS, n), dim3((PI_SCAN_WAVES + 1) * PI_WAVE), 0, stream, PI_DELTA_ARGS); \
+  }
+#define PI_LAUNCH_DELTA2(NR_, KIND_)                                                                                            \
+  do {                                                                                                                          \
+    constexpr bool LONG_KEYS = (NR_) >= 8;                                                                                      \
+    constexpr int AHEAD_NR = LONG_KEYS ? (NR_) : 8;                                                                             \
+    if (longest <= 2) { PI_DELTA_GO(true, by16, delta_scan_kernel<NR_, true, KIND_>) }                                          \
+    else if (LONG_KEYS && wide) { PI_DELTA_GO(false, by16 * 2, delta_scan_ahead_kernel<AHEAD_NR, KIND_, 32>) }                  \
+    else if ((NR_) >= 16 && (KIND_) != SCAN_HEAD_DELTA) { PI_DELTA_GO(false, by16, delta_scan_ahead_kernel<16, KIND_, 16>) }    \
+    else { PI_DELTA_GO(false, by16, delta_scan_kernel<NR_, false, KIND_>) }                                                     \
   } while (0)
 #define PI_LAUNCH_DELTA(NR_)                                                        \
   do {                                                                              \
