@@ -39,7 +39,7 @@ import torch
 from .. import ops
 from ..errors import UnsupportedModelError
 from ..weights.loader import TensorSpec
-from .base import MIXERS, PAGE, KVCacheSpec, LayerCache, Mixer, PagedCacheSpec, PagedTensor, PositionEncoding, StepContext
+from .base import MIXERS, PAGE, KVCacheSpec, LayerCache, Mixer, PagedCacheSpec, PagedTensor, PositionEncoding, StepContext, cut_rows
 
 
 POSITION_PREFIX = "position."
@@ -137,6 +137,10 @@ class PagedAttention(Mixer):
         return KVCacheSpec(self.num_kv_heads, self.head_dim, self.window)
 
     @property
+    def cuts_rows(self) -> bool:
+        return not self.values_are_keys
+
+    @property
     def takes_left_norm(self) -> bool:
         # the activations are read by the q|k|v projection only
         return not self.values_are_keys
@@ -183,7 +187,7 @@ class PagedAttention(Mixer):
     def norm_readers(self) -> List[torch.Tensor]:
         return [self.w_qkv]
 
-    def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext, cache: LayerCache) -> None:
+    def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext, cache: LayerCache) -> Optional[torch.Tensor]:
         T = h.shape[0]
         writes = self.own_kv and cache.writes
         rotary = self.position.rotary_params(ctx) if self.position is not None else None
@@ -192,7 +196,7 @@ class PagedAttention(Mixer):
         ws = ctx.workspace
         if self.values_are_keys:
             self._forward_values_are_keys(h, x, ctx, cache, rotary, table)
-            return
+            return None
         if self.qkv_bias:
             if not fused_position:
                 raise UnsupportedModelError("biased projections go with a rotation (or none), not with another position encoding")
@@ -217,7 +221,7 @@ class PagedAttention(Mixer):
                          next_norm=getattr(ctx, "next_norm", None), whole=True)
                 if self.o_bias and not self.bias_to_caller:
                     ops.add_row_bias(x, self.b_o)
-                return
+                return None
         if qkv is not None and not isinstance(qkv, torch.Tensor):
             # the projection is still in pieces (split over k): the rotation kernel sums them
             q = torch.empty((T, self.q_size), dtype=self.dtype, device=h.device)
@@ -249,12 +253,16 @@ class PagedAttention(Mixer):
                 self.num_heads, self.num_kv_heads, self.head_dim, cache.page_size,
                 self.scale, self.window or 0, ws,
             )
+        kept = cut_rows(ctx, x, attn)
+        if kept is not None:
+            x, attn = kept
         # where the arrangement allows it, the product stays in pieces for the stream's next reader
         ops.gemm(x, attn, self.w_o, accumulate=self.accumulate,
                  may_defer=self.accumulate and not self.o_bias and getattr(ctx, "may_defer", False), ws=ws,
                  next_norm=getattr(ctx, "next_norm", None), whole=True)
         if self.o_bias and not self.bias_to_caller:
             ops.add_row_bias(x, self.b_o)
+        return x if kept is not None else None
 
     def _forward_values_are_keys(self, h, x, ctx, cache, rotary, table) -> None:
         T, ws = h.shape[0], ctx.workspace

@@ -129,6 +129,7 @@ class StepContext:
     after_block_norm: Any = None          # set by the model per block: ``next_norm`` for whoever reads the stream after this block
     may_leave_choices: bool = False       # likewise: a routed feed-forward may leave its result as the experts' rows (``ops.LeftChoices``)
     after_block_consumes: bool = False    # set by the model per block: whoever reads the stream after this block adds pending pieces
+    read_rows: Optional[torch.Tensor] = None  # set for a mixer that ``cuts_rows``: the only rows of the stream that are read after it
     workspace: Any = None                 # the runner's ops.KernelWorkspace: scratch memory of the kernels
     plans: Dict[Any, Any] = field(default_factory=dict)     # step planner -> what it made for this step
     scratch: Dict[Any, Any] = field(default_factory=dict)   # what parts share within one step; emptied per step
@@ -147,6 +148,17 @@ class LayerCache:
     tensors: Dict[str, torch.Tensor] = field(default_factory=dict)   # every paged tensor by name: [pages, *page shape]
 
 
+def says_of_rows(part: Any, name: str) -> bool:
+    """What ``part``'s class says of rows that nobody reads, unless the object's ``forward`` has been replaced by another."""
+    return "forward" not in vars(part) and bool(getattr(part, name, False))
+
+
+def cut_rows(ctx: StepContext, *tensors: torch.Tensor):
+    """Copies of the rows of ``tensors`` that are read after this step's last mixer, or None: all are."""
+    rows = getattr(ctx, "read_rows", None)
+    return None if rows is None else tuple(t.index_select(0, rows) for t in tensors)
+
+
 # --------------------------------------------------------------------------- part bases
 class Part:
     """Common behaviour: declare tensors, receive them, know the compute dtype.
@@ -159,7 +171,8 @@ class Part:
     False: a part has to say so.
 
     What a class says of norms that are left to their reader (``leaves_root``, ``takes_left_norm``; a block's ``first_norm``
-    and ``opening_norm``) it says of its own ``forward``: a subclass with another ``forward`` says it again or does not.
+    and ``opening_norm``) and of rows that nobody reads (``rowwise``, ``cuts_rows``, ``ends_in_rows``) it says of its own
+    ``forward``: a subclass with another ``forward`` says it again or does not.
     """
 
     graph_safe = False
@@ -167,7 +180,8 @@ class Part:
     def __init_subclass__(cls, **kwargs):
         super().__init_subclass__(**kwargs)
         if "forward" in cls.__dict__:
-            for name, nothing in (("leaves_root", False), ("takes_left_norm", False), ("first_norm", None), ("opening_norm", None)):
+            for name, nothing in (("leaves_root", False), ("takes_left_norm", False), ("first_norm", None), ("opening_norm", None),
+                                  ("rowwise", False), ("cuts_rows", False), ("ends_in_rows", False)):
                 if name not in cls.__dict__:
                     setattr(cls, name, nothing)
 
@@ -218,6 +232,7 @@ class PositionEncoding(Part):
 
 class Mixer(Part):
     takes_left_norm = False    # True: ``forward`` takes an ``ops.LeftNorm`` for its activations (its products of them do)
+    cuts_rows = False          # True: where ``ctx.read_rows`` names rows, ``forward`` may update a copy of them alone and return it
 
     def cache_spec(self):
         """What the mixer keeps per request: ``KVCacheSpec`` / ``PagedCacheSpec`` (per token, in
@@ -233,13 +248,15 @@ class Mixer(Part):
         step, for all their mixers.  None: nothing to plan."""
         return None
 
-    def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext, cache: LayerCache) -> None:
-        """Read activations ``h`` [T, D]; add the mixer's output into ``x`` (float32)."""
+    def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext, cache: LayerCache) -> Optional[torch.Tensor]:
+        """Read activations ``h`` [T, D]; add the mixer's output into ``x`` (float32).  What is returned is looked at only
+        where ``ctx.read_rows`` was set: those rows with the output added, or None, ``x`` having been updated whole."""
         raise NotImplementedError
 
 
 class FeedForward(Part):
     takes_left_norm = False    # as a mixer's
+    rowwise = False            # True: a token's result takes nothing from other tokens, nor from what ``ctx`` says of them
 
     def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext) -> None:
         """Read activations ``h`` [T, D]; add the result into ``x`` (float32)."""
@@ -257,6 +274,7 @@ class Block(Part):
     mixer: Mixer
     takes_left_join = False    # True: the block's first reader applies a result that a sandwich block has left (``norm.LEFT_JOIN``)
     reads_deferred = False     # True: the block's first reader of the stream is a norm that adds pending pieces
+    ends_in_rows = False       # True: the block has a ``forward_last(x, ctx, cache)``: as ``forward``, the stream after it only at ``ctx.logit_rows``
 
     @property
     def first_norm(self):

@@ -13,7 +13,7 @@ import torch
 from .. import ops
 from ..errors import UnsupportedModelError
 from ..weights.loader import TensorSpec
-from .base import BLOCKS, MIXERS, Block, FeedForward, LayerCache, Mixer, Norm, Part, StepContext
+from .base import BLOCKS, MIXERS, Block, FeedForward, LayerCache, Mixer, Norm, Part, StepContext, says_of_rows
 from .norm import LEFT_JOIN, LEFT_UPDATE, LeftJoin, norm_left_to
 from .token_shift import TokenShift
 
@@ -140,6 +140,36 @@ class PreNormBlock(Block):
         ctx.may_defer, ctx.next_norm = ctx.after_block_consumes, ctx.after_block_norm
         self.ffn.forward(self.norm2.forward(x, ctx), x, ctx)
         ctx.may_defer, ctx.next_norm = False, None
+
+    @property
+    def ends_in_rows(self) -> bool:
+        return self.ffn is not None and says_of_rows(self.ffn, "rowwise")
+
+    def forward_last(self, x: torch.Tensor, ctx: StepContext, cache: LayerCache) -> torch.Tensor:
+        """The block as the last of a model's run: what follows its mixer (and, where the mixer says so, the mixer's last product)
+        takes in only the tokens whose logits are wanted.  The others' keys, values and states are written as ever."""
+        rows = ctx.logit_rows
+        few = 0 < rows.shape[0] <= ops.FEW_TOKENS
+        cuts = says_of_rows(self.mixer, "cuts_rows")
+        ctx.may_defer = bool(getattr(self.norm2, "consumes_deferred", False))
+        ctx.next_norm = norm_left_to(self.norm2, self.ffn, ctx.workspace) if few and cuts else None
+        h = self.norm1.forward(x, ctx)
+        ctx.read_rows = rows if cuts else None
+        cut = self.mixer.forward(h, x, ctx, cache)
+        ctx.read_rows = None
+        if rows.shape[0] == 0:
+            ops.discard_deferred(x, ctx.workspace)
+            ctx.may_defer, ctx.next_norm = False, None
+            return x[:0]
+        if cuts and cut is not None:
+            h, x = self.norm2.forward(cut, ctx), cut
+        else:                                        # the norm adds what is pending to those rows
+            h = self.norm2.forward(x, ctx, rows=rows)
+            x = x.index_select(0, rows)
+        ctx.may_defer, ctx.next_norm = ctx.after_block_consumes, ctx.after_block_norm
+        self.ffn.forward(h, x, ctx)
+        ctx.may_defer, ctx.next_norm = False, None
+        return x
 
 
 BLOCKS.register("prenorm", PreNormBlock)

@@ -36,12 +36,13 @@ import torch
 from .. import ops
 from ..errors import UnsupportedModelError
 from ..weights.loader import TensorSpec
-from .base import MIXERS, PAGE, LayerCache, Mixer, PagedCacheSpec, PagedTensor, PositionEncoding, StepContext
+from .base import MIXERS, PAGE, LayerCache, Mixer, PagedCacheSpec, PagedTensor, PositionEncoding, StepContext, cut_rows
 
 
 class LatentAttention(Mixer):
     graph_safe = True        # every kernel takes positions, requests and pages from device memory
     takes_left_norm = True   # the activations are read by the first projection only
+    cuts_rows = True
 
     def __init__(self, hidden_size: int, num_heads: int, head_dim: int, rot_dim: int, value_dim: int, q_rank: int, kv_rank: int,
                  scale: float, eps: float, position: Optional[PositionEncoding] = None, accumulate: bool = True,
@@ -129,7 +130,7 @@ class LatentAttention(Mixer):
     def norm_readers(self) -> List[torch.Tensor]:
         return [self.w_in]
 
-    def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext, cache: LayerCache) -> None:
+    def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext, cache: LayerCache) -> Optional[torch.Tensor]:
         T, ws, H = h.shape[0], ctx.workspace, self.num_heads
         table = ctx.block_tables[cache.group]
         rot_table = self.position.rotary_params(ctx)[0] if self.rot_dim else None
@@ -153,8 +154,12 @@ class LatentAttention(Mixer):
                                 value_dim=v_rows)
         out = torch.empty((T, self.o_size), dtype=self.dtype, device=h.device)
         ops.head_gemm(out, att, self.w_uv, H, a_head=v_rows, w_rows=self.w_uv_rows, gate=gates)
+        kept = cut_rows(ctx, x, out)
+        if kept is not None:
+            x, out = kept
         ops.gemm(x, out, self.w_o, accumulate=self.accumulate, may_defer=getattr(ctx, "may_defer", False), ws=ws,
                  next_norm=getattr(ctx, "next_norm", None))
+        return x if kept is not None else None
 
 
 MIXERS.register("latent_attention", LatentAttention)

@@ -21,7 +21,7 @@ INTERLEAVE = 16   # rows of a matrix-core tile
 
 class SwiGLU(FeedForward):
     graph_safe = True
-    takes_left_norm = True
+    takes_left_norm = rowwise = True
 
     def __init__(self, hidden_size: int, intermediate_size: int, activation: str = "silu",
                  names=("gate_proj.weight", "up_proj.weight", "down_proj.weight"), accumulate: bool = True):
@@ -89,7 +89,7 @@ class ClampedGLU(FeedForward):
     stream in the same kernel, so that the product only accumulates."""
 
     graph_safe = True
-    takes_left_norm = True
+    takes_left_norm = rowwise = True
 
     def __init__(self, hidden_size: int, intermediate_size: int, limit: float, alpha: float = 1.702,
                  names=("gate", "up", "down"), bias_suffix: str = ".b"):
@@ -152,7 +152,7 @@ class UngatedMLP(FeedForward):
     the normal distribution function.  ``accumulate`` False: the result is written into the tensor handed to
     ``forward`` instead of added to it."""
 
-    graph_safe = True
+    graph_safe = rowwise = True
 
     def __init__(self, hidden_size: int, intermediate_size: int, activation: str, names=("up", "down"), accumulate: bool = True):
         if activation not in ops.ACTIVATIONS:

@@ -27,7 +27,7 @@ import torch
 from .. import ops
 from ..errors import UnsupportedModelError
 from ..weights.loader import TensorSpec
-from .base import FEED_FORWARDS, FeedForward, StepContext
+from .base import FEED_FORWARDS, FeedForward, StepContext, says_of_rows
 from .mlp import INTERLEAVE
 
 
@@ -114,6 +114,10 @@ class RoutedExperts(FeedForward):
     @property
     def graph_safe(self) -> bool:
         return self.shared is None or bool(self.shared.graph_safe)
+
+    @property
+    def rowwise(self) -> bool:
+        return self.shared is None or says_of_rows(self.shared, "rowwise")
 
     def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext) -> None:
         T, ws = h.shape[0], ctx.workspace if ctx is not None else None

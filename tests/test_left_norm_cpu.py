@@ -122,3 +122,35 @@ def test_a_norm_is_left_only_where_every_product_of_it_applies_the_root():
                 ws.add_stream_copy(w)
             assert (norm_left_to(n, part, ws) is not None) == (fits and copies), (type(part).__name__, copies)
         assert norm_left_to(n, part, None) is None
+
+
+def test_a_subclass_with_another_forward_says_nothing_of_rows_by_inheritance():
+    """Whoever mixes tokens in a feed-forward, mixer or arrangement of its own gets all of them."""
+    from photon_infer_amd.parts.attention import PagedAttention
+    from photon_infer_amd.parts.block import PreNormBlock
+    from photon_infer_amd.parts.mlp import GeluMLP, SwiGLU
+
+    class Mixes(SwiGLU):
+        def forward(self, h, x, ctx):
+            super().forward(h + h.roll(1, 0), x, ctx)
+
+    class Named(SwiGLU):
+        pass
+
+    class Averaged(PagedAttention):
+        def forward(self, h, x, ctx, cache):
+            super().forward(h, x, ctx, cache)
+            x.sub_(x.mean(0))
+
+    class Scaled(PreNormBlock):
+        def forward(self, x, ctx, cache):
+            super().forward(x, ctx, cache)
+            x.mul_(2)
+
+    assert SwiGLU.rowwise and Named.rowwise and GeluMLP.rowwise and not Mixes.rowwise
+    assert not Averaged.cuts_rows and not Scaled.ends_in_rows
+    from photon_infer_amd.parts.base import says_of_rows
+    wrapped = SwiGLU(8, 16)
+    assert says_of_rows(wrapped, "rowwise")
+    wrapped.forward = lambda h, x, ctx: None
+    assert not says_of_rows(wrapped, "rowwise")
