@@ -1379,9 +1379,10 @@ def state_space_scan(y: torch.Tensor, xbc: torch.Tensor, dt: torch.Tensor, dt_bi
         chunks = sum(-(-n // chunk) for n in lens if n > upto) if lens else T // chunk + ctx.R
         states = torch.empty((chunks, heads, value_dim, state_dim), dtype=torch.float32, device=y.device)
         decays = torch.empty((chunks, heads), dtype=torch.float32, device=y.device)
+        scores = torch.empty((chunks, groups, chunk, chunk), dtype=torch.float32, device=y.device)
         _lib.call("core", "pi_state_space_chunks", y.data_ptr(), ldy, xbc.data_ptr(), ldx, dt.data_ptr(), ldd, dt_bias.data_ptr(),
                   a_log.data_ptr(), skip.data_ptr(), ctx.q_start.data_ptr(), ctx.slots.data_ptr(), ctx.R, upto + 1, chunks, states.data_ptr(),
-                  decays.data_ptr(), state.data_ptr(), state.stride(0), heads, value_dim, state_dim, groups, _stream())
+                  decays.data_ptr(), scores.data_ptr(), state.data_ptr(), state.stride(0), heads, value_dim, state_dim, groups, _stream())
         longest = max((n for n in lens if n <= upto), default=0) if lens else min(upto, T - longest)
         if longest == 0:
             return
