@@ -25,6 +25,7 @@ MAX_HEAD_DIM = 256              # the matrix-core attention kernels
 GENERAL_MAX_HEAD_DIM = 640      # the general attention kernel (key rows of a latent cache are wide)
 
 FEW_TOKENS = fast.FEW_TOKENS    # up to this many tokens a product may take all of k in a block (weights with a streaming copy)
+STREAMED_TOKENS = {torch.bfloat16: fast.SKINNY_MAX_ROWS, torch.float32: 32}    # up to this many a product's time is that of its weights
 
 _FAST = True
 

@@ -50,6 +50,8 @@ def position_is_rotation(position: Optional[PositionEncoding]) -> bool:
 
 
 class PagedAttention(Mixer):
+    cuts_rows = True
+
     def __init__(
         self,
         hidden_size: int,
@@ -137,10 +139,6 @@ class PagedAttention(Mixer):
         return KVCacheSpec(self.num_kv_heads, self.head_dim, self.window)
 
     @property
-    def cuts_rows(self) -> bool:
-        return not self.values_are_keys
-
-    @property
     def takes_left_norm(self) -> bool:
         # the activations are read by the q|k|v projection only
         return not self.values_are_keys
@@ -187,7 +185,7 @@ class PagedAttention(Mixer):
     def norm_readers(self) -> List[torch.Tensor]:
         return [self.w_qkv]
 
-    def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext, cache: LayerCache) -> Optional[torch.Tensor]:
+    def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext, cache: LayerCache) -> torch.Tensor:
         T = h.shape[0]
         writes = self.own_kv and cache.writes
         rotary = self.position.rotary_params(ctx) if self.position is not None else None
@@ -195,8 +193,7 @@ class PagedAttention(Mixer):
         table = ctx.block_tables[cache.group]
         ws = ctx.workspace
         if self.values_are_keys:
-            self._forward_values_are_keys(h, x, ctx, cache, rotary, table)
-            return None
+            return self._forward_values_are_keys(h, x, ctx, cache, rotary, table)
         if self.qkv_bias:
             if not fused_position:
                 raise UnsupportedModelError("biased projections go with a rotation (or none), not with another position encoding")
@@ -221,7 +218,7 @@ class PagedAttention(Mixer):
                          next_norm=getattr(ctx, "next_norm", None), whole=True)
                 if self.o_bias and not self.bias_to_caller:
                     ops.add_row_bias(x, self.b_o)
-                return None
+                return x
         if qkv is not None and not isinstance(qkv, torch.Tensor):
             # the projection is still in pieces (split over k): the rotation kernel sums them
             q = torch.empty((T, self.q_size), dtype=self.dtype, device=h.device)
@@ -253,18 +250,17 @@ class PagedAttention(Mixer):
                 self.num_heads, self.num_kv_heads, self.head_dim, cache.page_size,
                 self.scale, self.window or 0, ws,
             )
-        kept = cut_rows(ctx, x, attn)
-        if kept is not None:
-            x, attn = kept
+        if getattr(ctx, "read_rows", None) is not None:
+            x, attn = cut_rows(ctx, x, attn)
         # where the arrangement allows it, the product stays in pieces for the stream's next reader
         ops.gemm(x, attn, self.w_o, accumulate=self.accumulate,
                  may_defer=self.accumulate and not self.o_bias and getattr(ctx, "may_defer", False), ws=ws,
                  next_norm=getattr(ctx, "next_norm", None), whole=True)
         if self.o_bias and not self.bias_to_caller:
             ops.add_row_bias(x, self.b_o)
-        return x if kept is not None else None
+        return x
 
-    def _forward_values_are_keys(self, h, x, ctx, cache, rotary, table) -> None:
+    def _forward_values_are_keys(self, h, x, ctx, cache, rotary, table) -> torch.Tensor:
         T, ws = h.shape[0], ctx.workspace
         # float32 results (a tensor, or the pieces of a product split over k): rounded once, behind the norm
         proj = ops.qkv_projection(h, self.w_qkv, torch.float32, ws)
@@ -274,9 +270,12 @@ class PagedAttention(Mixer):
         attn = torch.empty((T, self.o_size), dtype=self.dtype, device=h.device)
         ops.paged_attention(attn, q, cache.k, cache.v, table, ctx, self.num_heads, self.num_kv_heads, self.head_dim, cache.page_size, self.scale,
                             self.window or 0, ws, softcap=self.softcap, out_scale=self.out_scale, feature_gate=gates)
+        if getattr(ctx, "read_rows", None) is not None:
+            x, attn = cut_rows(ctx, x, attn)
         ops.gemm(x, attn, self.w_o, accumulate=self.accumulate, may_defer=not self.o_bias and getattr(ctx, "may_defer", False), ws=ws)
         if self.o_bias and not self.bias_to_caller:
             ops.add_row_bias(x, self.b_o)
+        return x
 
 
 MIXERS.register("attention", PagedAttention)

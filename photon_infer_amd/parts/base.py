@@ -154,9 +154,10 @@ def says_of_rows(part: Any, name: str) -> bool:
 
 
 def cut_rows(ctx: StepContext, *tensors: torch.Tensor):
-    """Copies of the rows of ``tensors`` that are read after this step's last mixer, or None: all are."""
-    rows = getattr(ctx, "read_rows", None)
-    return None if rows is None else tuple(t.index_select(0, rows) for t in tensors)
+    """Copies of the rows of ``tensors`` that ``ctx.read_rows`` names (what has only them already, from a mixer beside, as it is:
+    they are half of the step's tokens at most)."""
+    rows = ctx.read_rows
+    return tuple(t if t.shape[0] == rows.shape[0] else t.index_select(0, rows) for t in tensors)
 
 
 # --------------------------------------------------------------------------- part bases
@@ -232,7 +233,7 @@ class PositionEncoding(Part):
 
 class Mixer(Part):
     takes_left_norm = False    # True: ``forward`` takes an ``ops.LeftNorm`` for its activations (its products of them do)
-    cuts_rows = False          # True: where ``ctx.read_rows`` names rows, ``forward`` may update a copy of them alone and return it
+    cuts_rows = False          # True: where ``ctx.read_rows`` names rows, ``forward`` updates a copy of them alone and returns it
 
     def cache_spec(self):
         """What the mixer keeps per request: ``KVCacheSpec`` / ``PagedCacheSpec`` (per token, in
@@ -249,8 +250,8 @@ class Mixer(Part):
         return None
 
     def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext, cache: LayerCache) -> Optional[torch.Tensor]:
-        """Read activations ``h`` [T, D]; add the mixer's output into ``x`` (float32).  What is returned is looked at only
-        where ``ctx.read_rows`` was set: those rows with the output added, or None, ``x`` having been updated whole."""
+        """Read activations ``h`` [T, D]; add the mixer's output into ``x`` (float32).  A mixer that ``cuts_rows`` returns what
+        it has added to: ``x``, or where ``ctx.read_rows`` was set those rows alone, of which ``x`` may hold no others."""
         raise NotImplementedError
 
 

@@ -61,8 +61,14 @@ class SideBySide(Mixer):
     def takes_left_norm(self) -> bool:
         return all(getattr(m, "takes_left_norm", False) for _, m in self.branches)
 
-    def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext, cache) -> None:
+    @property
+    def cuts_rows(self) -> bool:
+        return all(says_of_rows(m, "cuts_rows") for _, m in self.branches)
+
+    def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext, cache) -> torch.Tensor:
         caches = cache if isinstance(cache, (list, tuple)) else [cache]
+        read = getattr(ctx, "read_rows", None)
+        rows = h.shape[0] if read is None else read.shape[0]
         if isinstance(h, ops.LeftNorm) and not all(ctx.workspace.has_stream_copy(w) for w in self.norm_readers()):
             h = ops.whole_norm(h)      # a product that cannot apply the root would make the norm of a stream that has changed
         may_defer, next_norm = ctx.may_defer, ctx.next_norm
@@ -71,8 +77,10 @@ class SideBySide(Mixer):
             ctx.next_norm = next_norm if last else None      # the stream is finished by the last
             # pieces of an earlier one would be added by a kernel of their own: few tokens take all of k in a block instead
             # (12 tokens, 2,048 x 2,048: 5.7 + 3.3 us and 3.9)
-            ctx.may_defer = may_defer and (last or h.shape[0] > ops.FEW_TOKENS)
-            m.forward(h, x, ctx, c)
+            ctx.may_defer = may_defer and (last or rows > ops.FEW_TOKENS)
+            added = m.forward(h, x, ctx, c)
+            x = x if read is None else added
+        return x
 
 
 MIXERS.register("side_by_side", SideBySide)
@@ -150,19 +158,19 @@ class PreNormBlock(Block):
         takes in only the tokens whose logits are wanted.  The others' keys, values and states are written as ever."""
         rows = ctx.logit_rows
         few = 0 < rows.shape[0] <= ops.FEW_TOKENS
-        cuts = says_of_rows(self.mixer, "cuts_rows")
+        cuts = says_of_rows(self.mixer, "cuts_rows") and not ctx.all_decode      # what single tokens take merges key ranges as it adds
         ctx.may_defer = bool(getattr(self.norm2, "consumes_deferred", False))
         ctx.next_norm = norm_left_to(self.norm2, self.ffn, ctx.workspace) if few and cuts else None
         h = self.norm1.forward(x, ctx)
         ctx.read_rows = rows if cuts else None
-        cut = self.mixer.forward(h, x, ctx, cache)
+        added = self.mixer.forward(h, x, ctx, cache)
         ctx.read_rows = None
         if rows.shape[0] == 0:
             ops.discard_deferred(x, ctx.workspace)
             ctx.may_defer, ctx.next_norm = False, None
             return x[:0]
-        if cuts and cut is not None:
-            h, x = self.norm2.forward(cut, ctx), cut
+        if cuts:
+            h, x = self.norm2.forward(added, ctx), added
         else:                                        # the norm adds what is pending to those rows
             h = self.norm2.forward(x, ctx, rows=rows)
             x = x.index_select(0, rows)

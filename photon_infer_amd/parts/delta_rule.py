@@ -29,7 +29,7 @@ import torch
 from .. import ops
 from ..errors import UnsupportedModelError
 from ..weights.loader import TensorSpec
-from .base import MIXERS, LayerCache, Mixer, StateSpec, StepContext
+from .base import MIXERS, LayerCache, Mixer, StateSpec, StepContext, cut_rows
 
 UNIT_EPS = 1e-6      # inside the root of the unit vectors' length
 
@@ -37,6 +37,7 @@ UNIT_EPS = 1e-6      # inside the root of the unit vectors' length
 class ChannelDeltaRule(Mixer):
     graph_safe = True        # slots and request boundaries are read on the device
     takes_left_norm = True   # the activations are read by products only, before the stream is updated
+    cuts_rows = True
 
     def __init__(self, hidden_size: int, num_heads: int, num_kv_heads: int, key_dim: int, value_dim: int, conv_taps: int,
                  decay_rank: int, gate_rank: int, eps: float, out_scale: float = 1.0, accumulate: bool = True):
@@ -85,7 +86,7 @@ class ChannelDeltaRule(Mixer):
     def norm_readers(self) -> List[torch.Tensor]:
         return [self.w_in, self.w_low]
 
-    def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext, cache: LayerCache) -> None:
+    def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext, cache: LayerCache) -> torch.Tensor:
         T, ws, C = h.shape[0], ctx.workspace, self.channels
         f32 = lambda n: torch.empty((T, n), dtype=torch.float32, device=h.device)
         proj = f32(C + self.num_heads)
@@ -102,8 +103,11 @@ class ChannelDeltaRule(Mixer):
                        self.num_kv_heads, self.key_dim, self.value_dim, self.key_dim ** -0.5, UNIT_EPS)
         y = torch.empty((T, self.v_size), dtype=self.dtype, device=h.device)
         ops.head_norm_gate(y, o, gate, self.w_norm, self.eps, self.num_heads, self.value_dim, self.out_scale)
+        if getattr(ctx, "read_rows", None) is not None:
+            x, y = cut_rows(ctx, x, y)
         ops.gemm(x, y, self.w_o, accumulate=self.accumulate,
                  may_defer=self.accumulate and getattr(ctx, "may_defer", False), ws=ws, next_norm=getattr(ctx, "next_norm", None), whole=True)
+        return x
 
 
 MIXERS.register("channel_delta_rule", ChannelDeltaRule)
@@ -120,7 +124,7 @@ class GatedDeltaRule(Mixer):
 
     One projection gives everything that is read from h, as float32: rows [q | k | v | b | a | g]."""
 
-    graph_safe = takes_left_norm = True
+    graph_safe = takes_left_norm = cuts_rows = True
 
     def __init__(self, hidden_size: int, num_heads: int, num_kv_heads: int, key_dim: int, value_dim: int, conv_taps: int, eps: float,
                  accumulate: bool = True):
@@ -162,7 +166,7 @@ class GatedDeltaRule(Mixer):
     def norm_readers(self) -> List[torch.Tensor]:
         return [self.w_in]
 
-    def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext, cache: LayerCache) -> None:
+    def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext, cache: LayerCache) -> torch.Tensor:
         T, ws, C, H = h.shape[0], ctx.workspace, self.channels, self.num_heads
         f32 = lambda n: torch.empty((T, n), dtype=torch.float32, device=h.device)
         proj = f32(C + 2 * H + self.v_size)
@@ -174,7 +178,10 @@ class GatedDeltaRule(Mixer):
                        H, self.num_kv_heads, self.key_dim, self.value_dim, self.key_dim ** -0.5, UNIT_EPS, kind="head_delta")
         y = torch.empty((T, self.v_size), dtype=self.dtype, device=h.device)
         ops.head_norm_gate(y, o, proj[:, C + 2 * H:], self.w_norm, self.eps, H, self.value_dim, gate="silu")
+        if getattr(ctx, "read_rows", None) is not None:
+            x, y = cut_rows(ctx, x, y)
         ops.gemm(x, y, self.w_o, accumulate=self.accumulate, may_defer=self.accumulate and getattr(ctx, "may_defer", False), ws=ws, next_norm=getattr(ctx, "next_norm", None), whole=True)
+        return x
 
 
 MIXERS.register("gated_delta_rule", GatedDeltaRule)

@@ -130,7 +130,7 @@ class LatentAttention(Mixer):
     def norm_readers(self) -> List[torch.Tensor]:
         return [self.w_in]
 
-    def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext, cache: LayerCache) -> Optional[torch.Tensor]:
+    def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext, cache: LayerCache) -> torch.Tensor:
         T, ws, H = h.shape[0], ctx.workspace, self.num_heads
         table = ctx.block_tables[cache.group]
         rot_table = self.position.rotary_params(ctx)[0] if self.rot_dim else None
@@ -154,12 +154,11 @@ class LatentAttention(Mixer):
                                 value_dim=v_rows)
         out = torch.empty((T, self.o_size), dtype=self.dtype, device=h.device)
         ops.head_gemm(out, att, self.w_uv, H, a_head=v_rows, w_rows=self.w_uv_rows, gate=gates)
-        kept = cut_rows(ctx, x, out)
-        if kept is not None:
-            x, out = kept
+        if getattr(ctx, "read_rows", None) is not None:
+            x, out = cut_rows(ctx, x, out)
         ops.gemm(x, out, self.w_o, accumulate=self.accumulate, may_defer=getattr(ctx, "may_defer", False), ws=ws,
                  next_norm=getattr(ctx, "next_norm", None))
-        return x if kept is not None else None
+        return x
 
 
 MIXERS.register("latent_attention", LatentAttention)

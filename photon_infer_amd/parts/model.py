@@ -194,9 +194,12 @@ class DecoderModel:
     def _ends_in_rows(block: Block, ctx: StepContext) -> bool:
         """Whether the last block is to leave the stream only at the rows whose logits are wanted: nobody reads the others, and a
         prompt wants one of them.  1B sizes, sixteen layers: a prompt of 2,048 tokens 5,290 -> 5,043 us (in 32 bits, three of 517 and
-        less, 15,920 -> 14,870); 512 tokens beside 31 single ones, eight 8B-sized layers 3,099 -> 2,983.  The copy of the rows is a launch
-        (some 4 us), so rows are cut where at least half of them go; up to 16 tokens the weights' bytes set the time of the products."""
-        return says_of_rows(block, "ends_in_rows") and ctx.T > ops.FEW_TOKENS and 2 * ctx.logit_rows.shape[0] <= ctx.T
+        less, 15,920 -> 14,870); 512 tokens beside 31 single ones, eight 8B-sized layers 3,099 -> 2,983.  The copies of the rows are two
+        launches, so rows are cut where at least half of them go, and where the products' time follows the rows: the streaming kernels'
+        hardly does (100 tokens 1,547 and 1,586 us; a step that wants none saves the products themselves)."""
+        wanted = ctx.logit_rows.shape[0]
+        least = ops.FEW_TOKENS if wanted == 0 else ops.STREAMED_TOKENS[ctx.dtype]
+        return says_of_rows(block, "ends_in_rows") and ctx.T > least and 2 * wanted <= ctx.T
 
     def streamed_weights(self) -> List[torch.Tensor]:
         """The weight matrices that every decode step reads whole (see ``Part.streamed_weights``)."""

@@ -45,7 +45,7 @@ import torch
 from .. import ops
 from ..errors import UnsupportedModelError
 from ..weights.loader import TensorSpec
-from .base import MIXERS, PAGE, LayerCache, Mixer, PagedCacheSpec, PagedTensor, StepContext
+from .base import MIXERS, PAGE, LayerCache, Mixer, PagedCacheSpec, PagedTensor, StepContext, cut_rows
 
 
 def distance_slopes(num_heads: int) -> torch.Tensor:
@@ -57,6 +57,7 @@ def distance_slopes(num_heads: int) -> torch.Tensor:
 class SinkWindowAttention(Mixer):
     graph_safe = True        # every kernel takes positions, requests and pages from device memory
     takes_left_norm = True   # the activations are read by the first projection only
+    cuts_rows = True
 
     def __init__(self, hidden_size: int, num_heads: int, num_kv_heads: int, head_dim: int, value_dim: int, scale: float,
                  window: Optional[int], eps: float, temp_coef: float = 0.0, temp_every: int = 1, qk_norm: bool = True,
@@ -144,7 +145,7 @@ class SinkWindowAttention(Mixer):
     def norm_readers(self) -> List[torch.Tensor]:
         return [self.w_in]
 
-    def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext, cache: LayerCache) -> None:
+    def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext, cache: LayerCache) -> torch.Tensor:
         T, ws = h.shape[0], ctx.workspace
         table = ctx.block_tables[cache.group]
         # a float32 tensor, or - where the product was split over k - its pieces, which the next kernel adds
@@ -165,8 +166,11 @@ class SinkWindowAttention(Mixer):
         ops.paged_attention(attn, q, cache.k, cache.v, table, ctx, self.num_heads, self.num_kv_heads, self.head_dim,
                             cache.page_size, self.scale, self.window or 0, ws, value_dim=self.value_dim,
                             slopes=self.slopes, sinks=self.sinks, gate=gate, softcap=self.softcap, chunk=self.chunk or 0, keep_first=self.keep_first)
+        if getattr(ctx, "read_rows", None) is not None:
+            x, attn = cut_rows(ctx, x, attn)
         ops.gemm(x, attn, self.w_o, accumulate=self.accumulate, may_defer=getattr(ctx, "may_defer", False), ws=ws,
                  next_norm=getattr(ctx, "next_norm", None))
+        return x
 
 
 MIXERS.register("sink_window_attention", SinkWindowAttention)

@@ -24,12 +24,13 @@ import torch
 from .. import ops
 from ..errors import UnsupportedModelError
 from ..weights.loader import TensorSpec
-from .base import MIXERS, LayerCache, Mixer, StateSpec, StepContext
+from .base import MIXERS, LayerCache, Mixer, StateSpec, StepContext, cut_rows
 
 
 class StateSpaceMixer(Mixer):
     graph_safe = True        # slots and request boundaries are read on the device
     takes_left_norm = True   # the activations are read by products only, before the stream is updated
+    cuts_rows = True
 
     def __init__(self, hidden_size: int, num_heads: int, value_dim: int, state_dim: int, groups: int, norm_groups: int,
                  conv_taps: int, eps: float, out_scale: float = 1.0, accumulate: bool = True):
@@ -68,7 +69,7 @@ class StateSpaceMixer(Mixer):
     def norm_readers(self) -> List[torch.Tensor]:
         return [self.w_in]
 
-    def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext, cache: LayerCache) -> None:
+    def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext, cache: LayerCache) -> torch.Tensor:
         T, ws, inner = h.shape[0], ctx.workspace, self.inner
         proj = torch.empty((T, self.proj_size), dtype=torch.float32, device=h.device)
         ops.gemm(proj, h, self.w_in, ws=ws, whole=True)
@@ -79,8 +80,11 @@ class StateSpaceMixer(Mixer):
                              cache.state[:, self.conv_floats:], self.num_heads, self.value_dim, self.state_dim, self.groups)
         act = torch.empty((T, inner), dtype=self.dtype, device=h.device)
         ops.gated_group_norm(act, y, proj[:, :inner], self.w_norm, self.eps, self.norm_groups, self.out_scale)
+        if getattr(ctx, "read_rows", None) is not None:
+            x, act = cut_rows(ctx, x, act)
         ops.gemm(x, act, self.w_o, accumulate=self.accumulate,
                  may_defer=self.accumulate and getattr(ctx, "may_defer", False), ws=ws, next_norm=getattr(ctx, "next_norm", None), whole=True)
+        return x
 
 
 MIXERS.register("state_space", StateSpaceMixer)

@@ -16,13 +16,13 @@ def logits_of_steps(folder, dtype):
     from photon_infer_amd import EngineOptions, ModelRunner, StepEntry
 
     runner = ModelRunner(folder, EngineOptions(dtype=dtype, max_batch=24, max_cache_tokens=2048, max_model_len=256, use_graphs=False))
-    long, short = random_tokens(150, 200, 1), random_tokens(41, 200, 2)
+    long, other, short = random_tokens(150, 200, 1), random_tokens(140, 200, 3), random_tokens(41, 200, 2)
     few = [f"few {i}" for i in range(18)]
     for rid in ["a", "b", "c"] + few:
         runner.admit(rid)
     cut = [runner.step([StepEntry("a", long, [149])]),
            runner.step([StepEntry("b", short, [])]),
-           runner.step([StepEntry("c", short[:33], [32, 5]), StepEntry("b", [7], []), StepEntry("a", [9], [0])]),
+           runner.step([StepEntry("c", other, [139, 5]), StepEntry("b", [7], []), StepEntry("a", [9], [0])]),
            runner.step([StepEntry(rid, short[i:i + 2], []) for i, rid in enumerate(few)]),
            runner.step([StepEntry(rid, [3 + i], [0] if i % 7 == 2 else []) for i, rid in enumerate(few)])]
     whole = [runner.step([StepEntry("b", [11], [0]), StepEntry("c", [12], [0]), StepEntry("a", [13], [0])]),
