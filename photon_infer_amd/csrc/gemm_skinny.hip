@@ -25,6 +25,7 @@ enum { EPI_BF16 = 0, EPI_F32 = 1, EPI_ACCUM = 2, EPI_SWIGLU = 3 };
 #define RANGES_ROW_TILES 4      // row tiles per wave where the key ranges are merged on the way in (fewer blocks repeat the merge)
 #define KSTEP addressing::KSTEP
 #define SHARED_FROM_TOKENS 32   // more tokens than this: the kernel that shares an activation tile per block
+#define SHARED_FROM_ELEMENTS 20000000L    // ... and more than 16 tokens on matrices of so many elements
 #define RING_MAX_STRIDE (1L << 21)  // elements between rows, and of k, up to which that kernel's byte offsets fit 31 bits
 
 template <int EPI>
@@ -320,7 +321,7 @@ __global__ __launch_bounds__(256) void gemm_skinny_kernel(void* __restrict__ Cv,
   }
 }
 
-// The same product for 33..128 tokens, where the activations are as many bytes as a block's weights.  A block is eight waves
+// The same product for 33..128 tokens (from 17 on for large matrices, shares_activations), where the activations are as many bytes as a block's weights.  A block is eight waves
 // on 64 weight rows: wave w multiplies rows 32 (w / 4) .. + 31 with T tiles of 32 tokens (v_mfma_f32_32x32x16_bf16), and of
 // every step of 64 k takes the 16 of its quarter w % 4; the quarters are summed through LDS at the end.  So a step's
 // activations are read from LDS twice and not once per 16 rows, and the weights go into registers past LDS.  Activations go
@@ -829,8 +830,14 @@ static int launch_ring(int epi, dim3 grid, hipStream_t stream, void* C, long ldc
   return pi_fail("gemm_skinny: unknown epilogue %d", epi);
 }
 
-// Rows of the weight matrix per block for M tokens (the caller sizes its k-split by it).
-extern "C" int pi_gemm_skinny_rows_per_block(int M) { return M > SHARED_FROM_TOKENS ? RING_ROWS : ROWS_PER_BLOCK; }
+// Which of the two kernels: the caller sizes its k-split by the same rule (fast.py).  For 17 to 32 tokens the one that shares its
+// activations is the better one on matrices of some 40 MB and more (17 / 32 tokens, us, in the norm's or the head's place: 4,096 x 14,336
+// 28.5 / 29.6 -> 26.5 / 26.7, 3,072 x 8,192 17.1 / 18.9 -> 16.0 / 16.3, 6,144 x 4,096 15.6 / 17.5 -> 15.7 / 16.1, 28,672 x 4,096 50.8 / 51.1 ->
+// 46.3 / 46.9, 128,256 x 4,096 199.8 / 211.1 -> 199.3 / 201.6) and the worse one below (2,048 x 8,192 13.0 / 13.5 -> 14.0 / 14.2, 2,048 x 2,048
+// 8.0 / 8.3 -> 8.4 / 8.7).
+static bool shares_activations(int M, int N, int K, long ldx, long ldw) {
+  return M > SHARED_FROM_TOKENS || (M > 16 && (long)N * K >= SHARED_FROM_ELEMENTS && ldx < RING_MAX_STRIDE && ldw < RING_MAX_STRIDE && K < RING_MAX_STRIDE);
+}
 
 // splits > 1: the partial products go to `part` (float32 [splits, M, N]) and C is not touched;
 // *splits_out tells how many splits were made (no empty ones).
@@ -848,7 +855,8 @@ extern "C" int pi_gemm_skinny(void* C, int epilogue, long ldc, const void* X, lo
   PI_REQUIRE(((uintptr_t)X % 16 == 0) && ((uintptr_t)W % 16 == 0), "gemm_skinny: operands must be 16-byte aligned");
   PI_REQUIRE(splits >= 1 && splits <= 65535, "gemm_skinny: bad split count %d", splits);
   PI_REQUIRE(epilogue != EPI_SWIGLU || (splits == 1 && N % 32 == 0), "gemm_skinny: the SwiGLU epilogue needs one split and N (%d) a multiple of 32", N);
-  const int groups = ceil_div(N, pi_gemm_skinny_rows_per_block(M));
+  const bool shared = shares_activations(M, N, K, ldx, ldw);
+  const int groups = ceil_div(N, shared ? RING_ROWS : ROWS_PER_BLOCK);
   const addressing::KSplit cut = addressing::cut_k(K, splits, KSTEP);
   const int kpb = cut.k_per_block;
   splits = cut.splits;                            // no empty splits
@@ -858,7 +866,7 @@ extern "C" int pi_gemm_skinny(void* C, int epilogue, long ldc, const void* X, lo
   const dim3 grid(groups, splits);
   const int mb = (M + 15) / 16;
   const bf16_t *x = (const bf16_t*)X, *w = (const bf16_t*)W;
-  if (M > SHARED_FROM_TOKENS) {
+  if (shared) {
     PI_REQUIRE(ldx < RING_MAX_STRIDE && ldw < RING_MAX_STRIDE && K < RING_MAX_STRIDE, "gemm_skinny: K (%d) or row strides (%ld, %ld) are too long for 32-bit offsets", K, ldx, ldw);
     if (M <= 64) return launch_ring<2>(epilogue, grid, stream, C, ldc, x, ldx, w, ldw, M, N, K, kpb, (float*)part, tiled);
     if (M <= 96) return launch_ring<3>(epilogue, grid, stream, C, ldc, x, ldx, w, ldw, M, N, K, kpb, (float*)part, tiled);

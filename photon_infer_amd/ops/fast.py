@@ -31,6 +31,7 @@ SKINNY_MAX_ROWS = 128          # up to this many tokens the weight-streaming ker
 ROWS_PER_BLOCK = 32            # weight rows per block of the skinny kernel
 BLOCKS_PER_UNIT = 2            # blocks of it wanted per compute unit to keep HBM busy (measured: 512 on 256 units; 384 and 768 are slower)
 SHARED_FROM_TOKENS = 32        # more tokens than this: the skinny kernel that shares activations per block ...
+SHARED_FROM_ELEMENTS = 20_000_000    # ... and more than 16 tokens on matrices of so many elements (both sides: shares_activations, gemm_skinny.hip)
 SHARED_ROWS_PER_BLOCK = 64     # ... with this many weight rows per block, and no more blocks than compute units (100 tokens, 3,072 x 8,192:
                                # 22.8 us in six pieces on 288 blocks, 16.9 in five on 240; 6,144 x 4,096 22.8 in three, 18.7 in two), though
                                # a unit would hold two: 64 tokens, k 4,096, blocks for half the units or more in one piece and in two, 8,256
@@ -95,7 +96,8 @@ def _skinny_splits(M: int, N: int, K: int) -> int:
 
 @functools.lru_cache(maxsize=4096)
 def _skinny_splits_of(M: int, N: int, K: int, units: int) -> int:
-    if M > SHARED_FROM_TOKENS:     # the kernel that shares an activation tile per block: at most one block per compute unit
+    if M > SHARED_FROM_TOKENS or (M > FEW_TOKENS and N * K >= SHARED_FROM_ELEMENTS):
+        # the kernel that shares an activation tile per block: at most one block per compute unit
         splits = units // -(-N // SHARED_ROWS_PER_BLOCK)
     else:
         splits = -(-BLOCKS_PER_UNIT * units // -(-N // ROWS_PER_BLOCK))

@@ -1315,3 +1315,28 @@ def test_temperature_sampling_at_the_edges_of_chunks(_ops, V):
     # the plain implementation agrees on the crafted rows (a few of them: it walks the row in Python)
     for r in (1, 2, 11, 14):
         assert P.sample_temperature(l[r].double(), 1.0, draws[r]) == want[r]
+
+
+@pytest.mark.parametrize("copied", [False, True])
+@pytest.mark.parametrize("M,N,K", [(17, 5008, 4032), (32, 5008, 4032), (17, 4944, 4032), (25, 20064, 1024), (32, 9777, 2056), (31, 9728, 2048)])
+def test_products_of_17_to_32_tokens_on_both_sides_of_the_rule_of_sizes(_ops, M, N, K, copied):
+    """Matrices around 20 million elements, where these tokens change kernels: rows and k that are no whole blocks or steps,
+    whole, added and through the gated unit, from the matrix and from its streaming copy."""
+    if copied and (N % 16 or K % 64):
+        return
+    a, w = (torch.randn(n, K, generator=gen(n)).to(BF16).to(DEV) for n in (M, N))
+    ws = _ops.KernelWorkspace(DEV)
+    assert not copied or ws.add_stream_copy(w)
+    want = a.float() @ w.float().t()
+    # float32 sums of K products in any order: 2^-24 per addition, of which sqrt(K) add up, on both sides
+    bound = 2.0 ** -24 * 4 * K ** 0.5 * (a.float().abs() @ w.float().abs().t())
+    out, added = torch.empty(M, N, device=DEV), torch.ones(M, N, device=DEV)
+    _ops.gemm(out, a, w, ws=ws)
+    _ops.gemm(added, a, w, accumulate=True, ws=ws)
+    assert bool(((out - want).abs() <= bound).all()) and bool(((added - 1 - want).abs() <= bound + 2.0 ** -22 * (1 + want.abs())).all())
+    if N % 32 == 0:
+        act = torch.empty(M, N // 2, dtype=BF16, device=DEV)
+        _ops.gemm_swiglu(act, a, w, 16, ws=ws)
+        g, u = (t.reshape(M, N // 2) for t in want.view(M, N // 32, 2, 16).unbind(2))
+        ref = torch.nn.functional.silu(g) * u
+        assert bool(((act.float() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-3).all())
