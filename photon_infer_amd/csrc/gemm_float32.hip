@@ -198,10 +198,11 @@ __device__ inline TilePlace tile_place(int tiles_n) {
   return TilePlace{(int)blockIdx.x / tiles_n, (int)blockIdx.x % tiles_n};
 }
 
-// What becomes of a wave's WM x WN accumulators of 32 x 32, whose first row and column are m_wave and n_wave.
+// What becomes of a wave's WM x WN accumulators of 32 x 32, whose first row and column are m_wave and n_wave.  Values v whose bit in
+// `chosen` is not set are left out.
 template <int WM, int WN, int EPI>
 __device__ inline void finish_tiles(const f32x16_t (&acc)[WM][WN], long m_wave, long n_wave, float* __restrict__ C, long ldc, int M, int N,
-                                    float* __restrict__ part) {
+                                    float* __restrict__ part, const unsigned chosen = 0xffffu) {
   const int lane = threadIdx.x % 64, frow = lane % 32;
   // acc[i][j][v] is C[m_wave + i*32 + 8*(v/4) + 4*(lane/32) + v%4][n_wave + j*32 + lane%32]: a store
   // instruction writes 128 contiguous bytes of two rows.  Added into C, sixteen of its values are fetched before the first
@@ -221,7 +222,7 @@ __device__ inline void finish_tiles(const f32x16_t (&acc)[WM][WN], long m_wave, 
         for (int v = 0; v < 16; v += 2) {
           const float own = up ? acc[i][j][v + 1] : acc[i][j][v], other = __shfl_xor(up ? acc[i][j][v] : acc[i][j][v + 1], 16);
           const long m = mi + 8 * (v / 4) + v % 4 + up;
-          if (m < M) C[m * ldc + n / 2 + frow % 16] = silu_mul(up ? other : own, up ? own : other);
+          if (m < M && (chosen >> (v + up) & 1)) C[m * ldc + n / 2 + frow % 16] = silu_mul(up ? other : own, up ? own : other);
         }
       }
     }
@@ -250,7 +251,7 @@ __device__ inline void finish_tiles(const f32x16_t (&acc)[WM][WN], long m_wave, 
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         const long m = mi + 8 * (v / 4) + v % 4;
-        if (m < M) out[m * ld + n] = sum[v];
+        if (m < M && (chosen >> v & 1)) out[m * ld + n] = sum[v];
       }
     }
   }
@@ -382,9 +383,12 @@ __global__ __launch_bounds__(256) void gemm_float32_tile_kernel(float* __restric
 // kept: sched_group_barrier for that (one matrix instruction and four or six others in turn: up to 10 % slower), slabs fetched two to
 // four ahead (2 % either way), tiles of 64 x 64 and 64 x 128 in parts.
 //
-// An infinity has no such parts (the rest would be NaN), neither has a float that rounds to one (above 3.39e38); and where an
-// operand's largest float is below 2^-100 the last parts are lost.  A tile that meets one of these is made again from memory with
-// float32 instructions, slowly.  (A NaN needs nothing: its row or column is NaN either way.)
+// An infinity has no such parts (the rest would be NaN), neither has a float that rounds to one (above 3.39e38); a row whose largest
+// float, within the block's k, is below 2^-100 loses its last parts (of a larger row's small floats less is lost than its sums round off:
+// 2^-134 each); and the product of two leading parts may overflow where the floats' does not.  Outputs of such a row of A or W, and
+// infinite ones, are made from memory with float32 instructions, 32 x 32 at a time, in the order of gemm_float32_tile_kernel; the others
+// stay as they are, so that no row's bits hang on what its neighbours hold.  (One infinity in A, 2,048 x 16,384 x 2,048: 620 us become
+// 1,080; 378 x 3,072 x 2,048: 41 and 94.  A NaN needs nothing: its row or column is NaN either way.)
 // Four floats on their way into parts, in steps of some five instructions each: step 2 q + i makes part q of floats 2 i and 2 i + 1.
 struct PartsOf4 {
   float r[4];
@@ -443,10 +447,12 @@ __global__ __launch_bounds__(256, 2) void gemm_float32_parts_kernel(float* __res
     got[p] = __builtin_amdgcn_raw_buffer_load_b128(p < WM ? a_src : w_src, addressing::tile_slab_offset(offset[p], s * addressing::PARTS_SLAB, piece, k_range), 0, 0);
 #endif
   };
-  float a_top = 0.f, w_top = 0.f;
+  float top[LOADS];                              // of this thread's quarter of a row per load
+#pragma unroll
+  for (int p = 0; p < LOADS; ++p) top[p] = 0.f;
   PartsOf4 four;
   auto put = [&](const int p, const int u, const int buf) {      // step u of load p
-    if (u == 0) four.begin(__builtin_bit_cast(f32x4_t, got[p]), p < WM ? a_top : w_top);
+    if (u == 0) four.begin(__builtin_bit_cast(f32x4_t, got[p]), top[p]);
     four.step(u);
     if (u < 5) return;
 #pragma unroll
@@ -512,30 +518,73 @@ __global__ __launch_bounds__(256, 2) void gemm_float32_parts_kernel(float* __res
   }
 
   block_barrier_keeping_loads<0>();              // everybody is done with LDS
-  int* met = reinterpret_cast<int*>(lds);
+  int* met = reinterpret_cast<int*>(lds);        // whether there is an element to be made again; then, per row of A and W, whether it has no parts
   if (tid == 0) *met = 0;
   __syncthreads();
-  const int bits = (__any(!(a_top <= PARTS_LARGEST) || !(w_top <= PARTS_LARGEST)) ? 1 : 0) | (__any(a_top > 0.f) ? 2 : 0) |
-                   (__any(a_top >= PARTS_SMALLEST) ? 4 : 0) | (__any(w_top > 0.f) ? 8 : 0) | (__any(w_top >= PARTS_SMALLEST) ? 16 : 0);
-  if (lane == 0) atomicOr(met, bits);
-  __syncthreads();
-  const int all = __builtin_amdgcn_readfirstlane(*met);
-  if ((all & 1) || (all & 6) == 2 || (all & 24) == 8) {
-    clear();
-#pragma unroll 1
-    for (int k = k_lo / 2 + lane / 32; k < k_hi / 2; k += 2) {
-      float fa[WM], fb[WN];
+  float largest = 0.f;
 #pragma unroll
-      for (int i = 0; i < WM; ++i) fa[i] = A[min(m0 + wm * (TM / 2) + i * 32 + lane % 32, (long)M - 1) * lda + k];
+  for (int i = 0; i < WM; ++i)
 #pragma unroll
-      for (int j = 0; j < WN; ++j) fb[j] = W[min(n0 + wn * (TN / 2) + j * 32 + lane % 32, (long)N - 1) * ldw + k];
+    for (int j = 0; j < WN; ++j)
 #pragma unroll
-      for (int i = 0; i < WM; ++i)
+      for (int v = 0; v < 16; v += 2) asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(largest) : "v"(acc[i][j][v]), "v"(acc[i][j][v + 1]));
+  bool odd = !(largest < INFINITY);
 #pragma unroll
-        for (int j = 0; j < WN; ++j) acc[i][j] = mfma32_f32(fa[i], fb[j], acc[i][j]);
-    }
+  for (int p = 0; p < LOADS; ++p) {
+    const float t = fmaxf(top[p], dpp_move<0xB1>(top[p])), of_row = fmaxf(t, dpp_move<0x4E>(t));      // four lanes to a row
+    const bool none = !(of_row <= PARTS_LARGEST) || (of_row > 0.f && of_row < PARTS_SMALLEST);
+    if (piece == 0) met[1 + p * 64 + tid / 4] = none;
+    odd = odd || none;
   }
-  finish_tiles<WM, WN, EPI>(acc, m0 + wm * (TM / 2), n0 + wn * (TN / 2), C, ldc, M, N, part);
+  if (__any(odd) && lane == 0) atomicOr(met, 1);
+  __syncthreads();
+  const long m_wave = m0 + wm * (TM / 2), n_wave = n0 + wn * (TN / 2);
+  const bool remake = __builtin_amdgcn_readfirstlane(*met) != 0;
+  static_assert((1 + TM + TN) * 4 <= 2048 && 2048 + 4 * WM * WN * 256 <= 4 * BUF, "rows without parts and elements to be made again, in LDS");
+  unsigned* again = reinterpret_cast<unsigned*>(lds + 1024) + wave * WM * WN * 64 + lane;      // [wave][i][j][lane]: a bit per element
+  if (remake) {
+#pragma unroll
+    for (int i = 0; i < WM; ++i)
+#pragma unroll
+      for (int j = 0; j < WN; ++j) {
+        const bool column = met[1 + TM + wn * (TN / 2) + j * 32 + lane % 32];
+        unsigned bits = 0;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          const bool row = met[1 + wm * (TM / 2) + i * 32 + 8 * (v / 4) + 4 * (lane / 32) + v % 4];
+          const bool one = row || column || fabsf(acc[i][j][v]) == INFINITY;
+          bits |= (unsigned)one << v;
+          acc[i][j][v] = one ? -0.f : acc[i][j][v];              // added to C it leaves C as it is, stored it is overwritten below
+        }
+        if (EPI == EPI_SWIGLU) bits |= __shfl_xor(bits, 16);     // gate and up of a feature
+        again[(i * WN + j) * 64] = bits;
+      }
+  }
+  finish_tiles<WM, WN, EPI>(acc, m_wave, n_wave, C, ldc, M, N, part);
+  if (!remake) return;
+#pragma unroll 1
+  for (int t = 0; t < WM * WN; ++t) {            // a thread's elements are those that it has just written
+    const unsigned bits = again[t * 64];
+    if (!__any(bits != 0)) continue;
+    const long m_tile = m_wave + t / WN * 32, n_tile = n_wave + t % WN * 32;
+    const float* a_row = A + min(m_tile + lane % 32, (long)M - 1) * lda;
+    const float* w_row = W + min(n_tile + lane % 32, (long)N - 1) * ldw;
+    f32x16_t made[1][1];
+#pragma unroll
+    for (int v = 0; v < 16; ++v) made[0][0][v] = 0.f;
+#pragma unroll 4
+    for (int k = k_lo / 2; k < k_hi / 2; k += 8) {
+      const int at = k + lane / 32 * 4;          // K is a multiple of 4: the upper lanes' may lie beyond it
+      f32x4_t fa = {0.f, 0.f, 0.f, 0.f}, fb = fa;
+      if (at < k_hi / 2) {
+        fa = *reinterpret_cast<const f32x4_t*>(a_row + at);
+        fb = *reinterpret_cast<const f32x4_t*>(w_row + at);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) made[0][0] = mfma32_f32(fa[e], fb[e], made[0][0]);
+    }
+    finish_tiles<1, 1, EPI>(made, m_tile, n_tile, C, ldc, M, N, part, bits);
+  }
 }
 
 // ------------------------------------------------------------------ which kernel, which tile, how many pieces

@@ -347,6 +347,73 @@ def test_float32_floats_that_have_no_parts(_ops, M, N, K):
     check(a * 0.0, w, "zeros")
 
 
+def _rows_without_parts(M, N, K):
+    """Ordinary operands, and the same with single rows that have no parts: tiny as a whole (up to where float32 itself loses
+    digits), infinite, larger than the largest bfloat16; zeros; and a product that only its parts' leading terms overflow."""
+    a, w = torch.randn(M, K, generator=gen(M)).to(DEV), torch.randn(N, K, generator=gen(N)).to(DEV)
+    odd_a, odd_w = a.clone(), w.clone()
+    for row, by in ((1, -113), (66, -118), (129, -125), (M - 1, -121)):
+        odd_a[row] *= 2.0 ** by
+    for row, by in ((2, -113), (37, -118), (130, -125), (N - 1, -121)):
+        odd_w[row] *= 2.0 ** by
+    odd_a[5], odd_w[6] = 0.0, 0.0
+    odd_a[3, 5], odd_a[70, K - 1], odd_a[71, 17] = math.inf, -math.inf, 3.4e38
+    odd_w[8, 5], odd_w[N - 2, K - 1] = -math.inf, math.inf
+    odd_w[8, 17] = odd_w[N - 2, 17] = 0.5            # beside an infinity no product overflows: it could be one of the other sign
+    odd_a[9, 3], odd_w[9, 3] = 2.0 ** 64 * (2 - 2.0 ** -9), 2.0 ** 62 * (2 - 2.0 ** -9)
+    rows, cols = (odd_a != a).any(1), (odd_w != w).any(1)
+    return a, w, odd_a, odd_w, rows, cols
+
+
+@pytest.mark.parametrize("M,N,K", FLOAT32_PARTS[:3] + [(193, 2048, 8192)])
+def test_float32_rows_that_have_no_parts_among_others(_ops, M, N, K):
+    """Each output as 64 bits have it, whatever lies beside its row and column, and an ordinary one with the bits that it has among
+    ordinary ones.  A sum of K products is off by K roundings of 2^-25 of partial sums that grow with the root of K: some 2^-25 of
+    the sum of sizes whatever K is, sixteen of them over all outputs and twice that as a margin; below 2^-126 an addition rounds to 2^-149."""
+    _ops.use_fast_kernels(True)
+    a, w, odd_a, odd_w, rows, cols = _rows_without_parts(M, N, K)
+    want, size = odd_a.double() @ odd_w.double().t(), odd_a.double().abs() @ odd_w.double().abs().t()
+    want = torch.where(want.abs() > 3.4028235e38, want.sign() * math.inf, want)      # (a NaN stays one)
+    bound = 2.0 ** -20 * size + K * 2.0 ** -149
+    clean, out = torch.empty(M, N, device=DEV), torch.empty(M, N, device=DEV)
+    _ops.gemm(clean, a, w)
+    _ops.gemm(out, odd_a, odd_w)
+    finite = want.isfinite()
+    assert torch.equal(out.isnan(), want.isnan()) and torch.equal(out[~finite & ~want.isnan()].double(), want[~finite & ~want.isnan()])
+    off = (out.double() - want).abs()
+    bad = finite & ~(off <= bound)
+    assert not bad.any(), (int(bad.sum()), bad.any(1).nonzero().flatten().tolist()[:8], bad.any(0).nonzero().flatten().tolist()[:8])
+    kept = ~rows[:, None] & ~cols
+    assert torch.equal(out[kept], clean[kept])
+    added = torch.ones(M, N, device=DEV)
+    _ops.gemm(added, odd_a, odd_w, accumulate=True)
+    assert bool((finite <= ((added.double() - 1 - want).abs() <= bound + 2.0 ** -23 * (1 + want.abs()))).all())
+    if N % 32 == 0:
+        halves = lambda t: (h.reshape(M, -1) for h in t.view(M, N // 32, 2, 16).unbind(2))
+        (g, u), (dg, du) = halves(want), halves(bound)
+        ref = torch.nn.functional.silu(g) * u
+        act, plain = torch.empty(M, N // 2, device=DEV), torch.empty(M, N // 2, device=DEV)
+        _ops.gemm_swiglu(act, odd_a, odd_w, 16)
+        _ops.gemm_swiglu(plain, a, w, 16)
+        fine = g.isfinite() & u.isfinite() & (ref.abs() < 3e38)
+        off = (act.double() - ref).abs()
+        bad = fine & ~(off <= 1.1 * dg * u.abs() + (g.abs() + dg) * du + 2.0 ** -21 * ref.abs() + 2.0 ** -126)
+        assert not bad.any(), int(bad.sum())
+        kept = kept.view(M, N // 32, 2, 16).all(2).reshape(M, -1)
+        assert torch.equal(act[kept], plain[kept])
+
+
+@pytest.mark.parametrize("M,N,K", FLOAT32_PARTS[:3])
+def test_float32_products_that_are_small_though_no_operand_is(_ops, M, N, K):
+    """Terms of parts below 2^-126: both operands around 2^-58, products of their last parts around 2^-134.  Bound as above."""
+    _ops.use_fast_kernels(True)
+    a, w = torch.randn(M, K, generator=gen(M)).to(DEV) * 2.0 ** -58, torch.randn(N, K, generator=gen(N)).to(DEV) * 2.0 ** -58
+    want, size = a.double() @ w.double().t(), a.double().abs() @ w.double().abs().t()
+    out = torch.empty(M, N, device=DEV)
+    _ops.gemm(out, a, w)
+    assert bool(((out.double() - want).abs() <= 2.0 ** -20 * size + K * 2.0 ** -149).all())
+
+
 @pytest.mark.parametrize("M,N,K,kernel", [(1, 2048, 2048, "pi_gemm_general"), (2, 520, 516, "pi_gemm_general"), (1, 2048, 512, "pi_gemm_float32"),
                                           (3, 2048, 2048, "pi_gemm_float32"), (8, 8192, 8192, "pi_gemm_general"), (9, 8192, 8192, "pi_gemm_float32")])
 def test_few_float32_rows_go_to_the_kernel_that_streams_the_weights_faster(_ops, M, N, K, kernel):
