@@ -1352,6 +1352,7 @@ def causal_conv_silu(out: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, b
 # whole chunk of 64 rows is worth some 20 tokens of a walk in a full step.  32 heads of 64, state of 128, beside a request of
 # 128 tokens: 64 single tokens 81 us (walked with it 144, in chunks with it 187), 9 single tokens and 9 requests of 3 64 (69, 75).
 STATE_SPACE_CHUNKS_FROM, STATE_SPACE_CHUNKS_BESIDE = 128, 3
+GRID_MAX = 65535     # blocks of a launch in its second and third dimension: what needs more of them there is walked
 
 
 def state_space_scan(y: torch.Tensor, xbc: torch.Tensor, dt: torch.Tensor, dt_bias: torch.Tensor, a_log: torch.Tensor,
@@ -1373,7 +1374,7 @@ def state_space_scan(y: torch.Tensor, xbc: torch.Tensor, dt: torch.Tensor, dt_bi
     _i32(ctx.slots, "slots", ctx.R)
     longest, upto = int(getattr(ctx, "max_q_len", 0) or T), 0
     chunk = _lib.load("core").pi_state_space_chunk(value_dim, state_dim) if _FAST and longest >= STATE_SPACE_CHUNKS_FROM else 0
-    if chunk and ldx % 4 == 0 and ldy % 4 == 0 and xbc.data_ptr() % 16 == 0 and y.data_ptr() % 16 == 0:
+    if chunk and heads + groups <= GRID_MAX and ldx % 4 == 0 and ldy % 4 == 0 and xbc.data_ptr() % 16 == 0 and y.data_ptr() % 16 == 0:
         upto = STATE_SPACE_CHUNKS_BESIDE - 1
         lens = getattr(ctx, "q_lens", None)
         # without lengths on the host: an upper bound, and requests that may walk

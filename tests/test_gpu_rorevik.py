@@ -228,6 +228,25 @@ def test_single_tokens_walk_beside_a_request_that_runs_in_chunks(lengths_on_host
         assert scan(torch.arange(128), [6], [128])[2] == ["pi_state_space_chunks"]
 
 
+def test_state_space_of_more_heads_than_the_chunked_form_takes():
+    """65,535 heads beside a group: walked, as they are without a request long enough for chunks."""
+    from photon_infer_amd import ops
+    H, Pd, N, G, T = 65535, 4, 16, 1, 128
+    rand = lambda *shape: torch.randn(*shape, generator=torch.Generator(device=DEV).manual_seed(sum(shape)), device=DEV)
+    xbc, dt, params = rand(T, H * Pd + 2 * N), rand(T, H), (rand(H), rand(H), rand(H))
+
+    def scan(q_lens):
+        y, state, done = torch.empty((T, H * Pd), device=DEV), torch.zeros((1, ops.scan_state_floats(H, N, Pd)), device=DEV), 0
+        for n in q_lens:
+            with library_calls() as names:
+                ops.state_space_scan(y[done:done + n], xbc[done:done + n], dt[done:done + n], *params, state_ctx([n], [0]), state, H, Pd, N, G)
+            assert names == ["pi_state_space_scan"]
+            done += n
+        return y, state
+
+    assert all(torch.equal(a, b) for a, b in zip(scan([128]), scan([100, 28])))
+
+
 def delta_inputs(t, H, G, d, dv, seed):
     q, k, v = randn(t, G, d, seed=seed), randn(t, G, d, seed=seed + 1), randn(t, H, dv, seed=seed + 2)
     return q, k, v, randn(t, H * d, seed=seed + 3), randn(t, H, seed=seed + 4)
