@@ -1449,7 +1449,7 @@ def delta_scan(o: torch.Tensor, qkv: torch.Tensor, a: torch.Tensor, dt_bias: tor
     _i32(ctx.slots, "slots", ctx.R)
     longest, upto = int(getattr(ctx, "max_q_len", 0) or T), 0
     chunk = _lib.load("core").pi_delta_chunk(key_dim, value_dim) if _FAST and not outer and longest >= DELTA_CHUNKS_FROM else 0
-    if chunk and ldq % 4 == 0 and qkv.data_ptr() % 16 == 0 and (per_head or (lda % 4 == 0 and a.data_ptr() % 16 == 0)):
+    if chunk and ctx.R <= GRID_MAX and ldq % 4 == 0 and qkv.data_ptr() % 16 == 0 and (per_head or (lda % 4 == 0 and a.data_ptr() % 16 == 0)):
         upto = DELTA_CHUNKS_BESIDE - 1
         lens = getattr(ctx, "q_lens", None)
         # without lengths on the host: an upper bound, and requests that may walk

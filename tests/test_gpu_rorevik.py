@@ -320,6 +320,32 @@ def test_delta_rule_in_chunks_beside_single_tokens(sizes, per_head):
     assert bool((state[0] == 0).all()) and bool((state[:, -3:] == 0).all())
 
 
+def test_delta_rule_of_more_requests_than_the_chunked_form_takes():
+    """65,535 single tokens beside a request of 48: walked, the long one as it is alone."""
+    from photon_infer_amd import ops
+    ops.use_fast_kernels(True)
+    H, G, d, dv, R = 1, 1, 64, 16, 65536
+    lens, T = [1] * (R - 1) + [48], R + 47
+    rand = lambda *shape: torch.randn(*shape, generator=torch.Generator(device=DEV).manual_seed(sum(shape)), device=DEV)
+    qkv, a, b, params = rand(T, 2 * d + dv), rand(T, d), rand(T, 1), (rand(d), rand(1))
+
+    def scan(rows, q_lens, slots):
+        o, state = torch.empty((len(rows), dv), device=DEV), torch.zeros((R, ops.scan_state_floats(H, d, dv)), device=DEV)
+        with library_calls() as names:
+            ops.delta_scan(o, qkv[rows].contiguous(), a[rows].contiguous(), *params, b[rows].contiguous(), state_ctx(q_lens, slots), state, H, G, d, dv, d ** -0.5, 1e-6)
+        return o, state, names
+
+    o, state, names = scan(torch.arange(T), lens, list(range(R)))
+    assert names == ["pi_delta_scan"]
+    alone, left, names = scan(torch.arange(R - 1, T), [48], [R - 1])
+    assert names == ["pi_delta_chunks"]
+    close(o[R - 1:], alone.double().cpu(), "the long request", 5e-5)
+    close(state[R - 1], left[R - 1].double().cpu(), "its state", 5e-5)
+    few, left, _ = scan(torch.arange(7), [1] * 7, list(range(7)))
+    close(o[:7], few.double().cpu(), "single tokens", 5e-5)
+    close(state[:7], left[:7].double().cpu(), "their states", 5e-5)
+
+
 @pytest.mark.parametrize("bad", [math.nan, math.inf])
 @pytest.mark.parametrize("where", ["value", "key", "decay"])
 def test_what_is_not_finite_reaches_no_token_before_it(bad, where):
