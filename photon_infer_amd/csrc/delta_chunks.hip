@@ -9,6 +9,7 @@
 //   1. delta_chunk_prepare_kernel: unit vectors, decays, a, p, X, Y and the rest of every chunk, all chunks at once, in the order in
 //      which the matrix cores take them;
 //   2. delta_chunk_walk_kernel: U, outputs and states from chunk to chunk.
+// Both take a window of the step's chunks at a time, as many as the caller's scratch memory holds.
 //
 // The walk of single tokens is a chain of some 500 cycles per token.  16 heads of 128 x 128, 2,048 tokens of one request: 446 us walked,
 // 143 so (43 and 108 by themselves), eight requests of 375 tokens 414 and 146, 128 tokens 38 and 25, 48 tokens 20 and 19.  Against 64
@@ -36,13 +37,13 @@ __host__ __device__ inline ChunkShape chunk_shape(int d, int dv) {
   return s;
 }
 
-// blockIdx: (chunk, head).  DQ: d / 64.  Bound by issue: a thread's products over pairs of tokens and the sums over sixteen lanes (72 us
+// blockIdx: (chunk behind `first_chunk`, head).  DQ: d / 64.  Bound by issue: a thread's products over pairs of tokens and the sums over sixteen lanes (72 us
 // while it kept all pairs in registers, for half the waves; 43 so).
 template <int DQ>
 __global__ __launch_bounds__(256, 4) void delta_chunk_prepare_kernel(float* __restrict__ scratch, const float* __restrict__ qkv, long qkv_stride,
                                                                   const float* __restrict__ a, long a_stride, const float* __restrict__ dt_bias,
                                                                   const float* __restrict__ A_log, const float* __restrict__ b, long b_stride,
-                                                                  const int* __restrict__ q_start, int R, int from, int H, int G, int dv,
+                                                                  const int* __restrict__ q_start, int R, int from, int first_chunk, int H, int G, int dv,
                                                                   float q_scale, float unit_eps, int per_head) {
   constexpr int D = 64 * DQ, PADDED = D / 4 * 17 * 4;          // a fragment's four rows of lanes 17 pieces apart: their stores fall on all banks
   __shared__ f32x4_t vectors[3 * CHUNK * D / 4];               // q, k, decays; then Y and L q
@@ -50,7 +51,7 @@ __global__ __launch_bounds__(256, 4) void delta_chunk_prepare_kernel(float* __re
   __shared__ float betas[CHUNK];
   static_assert(2 * PADDED <= 3 * CHUNK * D, "Y and L q take the place of the vectors");
   const int h = blockIdx.y, g = h / (H / G), tid = threadIdx.x, at = tid / 16, part = tid % 16;
-  const TokenTile where = find_token_tile(q_start, R, CHUNK, blockIdx.x, from);
+  const TokenTile where = find_token_tile(q_start, R, CHUNK, first_chunk + blockIdx.x, from);
   if (where.req < 0) return;
   const long t0 = q_start[where.req] + (long)where.tile * CHUNK;
   const int tokens = min(CHUNK, (int)(q_start[where.req + 1] - t0));
@@ -206,16 +207,19 @@ __global__ __launch_bounds__(256, 4) void delta_chunk_prepare_kernel(float* __re
 template <int DQ>
 __global__ __launch_bounds__(320) void delta_chunk_walk_kernel(float* __restrict__ o, long o_stride, const float* __restrict__ scratch,
                                                                const int* __restrict__ q_start, const int* __restrict__ slots, int from,
-                                                               float* __restrict__ state, long state_stride, int H, int dv, int nr) {
+                                                               int first_chunk, int count, float* __restrict__ state, long state_stride, int H, int dv, int nr) {
   constexpr int D = 64 * DQ, AHEAD = DQ == 4 ? 2 : DQ == 3 ? 3 : 4;      // as many as there are registers for
   __shared__ f32x4_t of_u[2][4][64], of_o[2][4][64];
   const int h = blockIdx.x, z = blockIdx.y, r = blockIdx.z, lane = threadIdx.x % 64;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
-  const int n = q_start[r + 1] - q_start[r], chunks = token_tiles(n, CHUNK, from);
-  if (chunks == 0) return;
+  // of the request's chunks those from `begin` on that lie in the window
+  const int tokens = q_start[r + 1] - q_start[r], before = token_tiles_before(q_start, r, CHUNK, from);
+  const int begin = max(first_chunk - before, 0), chunks = min(first_chunk + count - before, token_tiles(tokens, CHUNK, from)) - begin;
+  if (chunks <= 0) return;
+  const int n = tokens - begin * CHUNK;
   const ChunkShape shape = chunk_shape(D, dv);
   const long step = (long)H * shape.all;
-  const float* mine = scratch + ((long)token_tiles_before(q_start, r, CHUNK, from) * H + h) * shape.all;
+  const float* mine = scratch + ((long)(before + begin - first_chunk) * H + h) * shape.all;
   auto fragment = [&](int c, int from_float, int tile) { return reinterpret_cast<const f32x4_t*>(mine + c * step + from_float)[tile * 64 + lane]; };
   const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
 
@@ -300,7 +304,7 @@ __global__ __launch_bounds__(320) void delta_chunk_walk_kernel(float* __restrict
     };
 #pragma unroll
     for (int i = 0; i < AHEAD; ++i) fetch(i, i);
-    float* to = o + ((long)q_start[r] + lane / 16 * 4) * o_stride + (long)h * dv + z * 16 + lane % 16;
+    float* to = o + ((long)q_start[r] + begin * CHUNK + lane / 16 * 4) * o_stride + (long)h * dv + z * 16 + lane % 16;
     auto finish = [&](int c) {                   // the outputs of chunk c, whose shares the last barrier has brought
       f32x4_t share[4];
 #pragma unroll
@@ -365,8 +369,8 @@ __global__ __launch_bounds__(320) void delta_chunk_walk_kernel(float* __restrict
 // 0: sizes that the chunked form does not take.
 extern "C" int pi_delta_chunk(int d, int dv) { return d > 0 && d % 64 == 0 && d <= 256 && dv > 0 && dv % 16 == 0 ? CHUNK : 0; }
 
-// The requests that bring `from` tokens or more, with a decay per channel or (`per_head`) per head.  `scratch`: chunks * H * (49 d + 16 dv
-// + 256) floats.  Arguments otherwise as for pi_delta_scan; qkv, a and b are only read.  Rows of q, k and of the decays per channel must be 16-byte aligned.
+// The requests that bring `from` tokens or more, with a decay per channel or (`per_head`) per head; `chunks` of them in all, or an upper
+// bound.  `scratch`: H * (49 d + 16 dv + 256) floats per chunk, for all of them or for fewer, which are then taken one window after the other.  Arguments otherwise as for pi_delta_scan; qkv, a and b are only read.  Rows of q, k and of the decays per channel must be 16-byte aligned.
 extern "C" int pi_delta_chunks(float* o, long o_stride, const float* qkv, long qkv_stride, const float* a, long a_stride, const float* dt_bias,
                                const float* A_log, const float* b, long b_stride, const int* q_start, const int* slots, int R, int from, int chunks,
                                float* scratch, long scratch_floats, float* state, long state_stride, int H, int G, int d, int dv, float q_scale, float unit_eps, int per_head,
@@ -379,18 +383,23 @@ extern "C" int pi_delta_chunks(float* o, long o_stride, const float* qkv, long q
              "delta rule: bad step (%d requests, %d chunks) or a state row of %ld floats that cannot hold %d x %d x %d", R, chunks, state_stride, H, d, dv);
   PI_REQUIRE(qkv_stride % 4 == 0 && (uintptr_t)qkv % 16 == 0 && (uintptr_t)scratch % 16 == 0 && (per_head || (a_stride % 4 == 0 && (uintptr_t)a % 16 == 0)),
              "delta rule: rows must be 16-byte aligned");
-  PI_REQUIRE(scratch_floats >= (long)chunks * H * chunk_shape(d, dv).all, "delta rule: %d chunks of %d heads do not fit %ld floats", chunks, H, scratch_floats);
+  const long window = scratch_floats / ((long)H * chunk_shape(d, dv).all);
+  PI_REQUIRE(window > 0, "delta rule: a chunk of %d heads does not fit %ld floats", H, scratch_floats);
   PI_REQUIRE(dv / 16 <= 65535 && R <= 65535, "delta rule: values of %d, %d requests", dv, R);
-#define GO(DQ_)                                                                                                                                     \
-  case DQ_:                                                                                                                                         \
-    hipLaunchKernelGGL((delta_chunk_prepare_kernel<DQ_>), dim3(chunks, H), dim3(256), 0, stream, scratch, qkv, qkv_stride, a, a_stride, dt_bias,    \
-                       A_log, b, b_stride, q_start, R, from, H, G, dv, q_scale, unit_eps, per_head);                                               \
-    hipLaunchKernelGGL((delta_chunk_walk_kernel<DQ_>), dim3(H, dv / 16, R), dim3(320), 0, stream, o, o_stride, scratch, q_start, slots, from, state, \
-                       state_stride, H, dv, nr);                                                                                                    \
+#define GO(DQ_)                                                                                                                                  \
+  case DQ_:                                                                                                                                      \
+    hipLaunchKernelGGL((delta_chunk_prepare_kernel<DQ_>), dim3(count, H), dim3(256), 0, stream, scratch, qkv, qkv_stride, a, a_stride, dt_bias,  \
+                       A_log, b, b_stride, q_start, R, from, first, H, G, dv, q_scale, unit_eps, per_head);                                     \
+    hipLaunchKernelGGL((delta_chunk_walk_kernel<DQ_>), dim3(H, dv / 16, R), dim3(320), 0, stream, o, o_stride, scratch, q_start, slots, from,    \
+                       first, count, state, state_stride, H, dv, nr);                                                                            \
     break
-  switch (d / 64) {
-    GO(1); GO(2); GO(3); GO(4);
+  for (long at = 0; at < chunks; at += window) {
+    const int first = (int)at, count = (int)(chunks - at < window ? chunks - at : window);
+    switch (d / 64) {
+      GO(1); GO(2); GO(3); GO(4);
+    }
+    if (pi_check_launch("delta_chunks")) return -1;
   }
 #undef GO
-  return pi_check_launch("delta_chunks");
+  return 0;
 }

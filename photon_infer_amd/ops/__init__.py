@@ -1412,6 +1412,9 @@ SCAN_KINDS = {"channel_delta": 0, "head_delta": 1, "decayed_outer": 2}
 # walked and 19.4 in chunks, 32 tokens 16.3 and 18.4; eight requests of 32 55 and 39, of 16 38 and 33), and of the requests beside it
 # that then do so too: all that the walk's form for a token or two does not take.
 DELTA_CHUNKS_FROM, DELTA_CHUNKS_BESIDE = 48, 3
+# What the chunks leave for the walk (34 KB per token of 16 heads of 128 x 128) takes so many floats at most, which is 7,800 such tokens:
+# a larger step is taken in windows.
+DELTA_CHUNKS_FLOATS = 64 << 20
 
 
 def delta_scan(o: torch.Tensor, qkv: torch.Tensor, a: torch.Tensor, dt_bias: torch.Tensor, a_log: Optional[torch.Tensor],
@@ -1454,7 +1457,8 @@ def delta_scan(o: torch.Tensor, qkv: torch.Tensor, a: torch.Tensor, dt_bias: tor
         lens = getattr(ctx, "q_lens", None)
         # without lengths on the host: an upper bound, and requests that may walk
         chunks = sum(-(-n // chunk) for n in lens if n > upto) if lens else T // chunk + ctx.R
-        scratch = torch.empty(chunks * heads * (49 * key_dim + 16 * value_dim + 256), dtype=torch.float32, device=o.device)
+        of_one = heads * (49 * key_dim + 16 * value_dim + 256)
+        scratch = torch.empty(of_one * max(1, min(chunks, DELTA_CHUNKS_FLOATS // of_one)), dtype=torch.float32, device=o.device)
         _lib.call("core", "pi_delta_chunks", o.data_ptr(), ldo, qkv.data_ptr(), ldq, a.data_ptr(), lda, dt_bias.data_ptr(), _ptr(a_log),
                   b.data_ptr(), ldb, ctx.q_start.data_ptr(), ctx.slots.data_ptr(), ctx.R, upto + 1, chunks, scratch.data_ptr(), scratch.numel(), state.data_ptr(),
                   state.stride(0), heads, kv_heads, key_dim, value_dim, float(q_scale), float(unit_eps), int(per_head), _stream())

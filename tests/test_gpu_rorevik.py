@@ -320,6 +320,44 @@ def test_delta_rule_in_chunks_beside_single_tokens(sizes, per_head):
     assert bool((state[0] == 0).all()) and bool((state[:, -3:] == 0).all())
 
 
+@pytest.mark.parametrize("lengths_on_host", [True, False])
+def test_delta_rule_in_windows_of_chunks(monkeypatch, lengths_on_host):
+    """Scratch memory for all nineteen chunks, and for one, two, five, eighteen of them: windows that cut requests, hold several and
+    end with the step give the same bits; requests that walk lie between."""
+    from photon_infer_amd import ops
+    ops.use_fast_kernels(True)
+    H, G, d, dv = 2, 1, 64, 32
+    lens = [1, 150, 2, 3, 64, 16, 1, 40]
+    T, of_one = sum(lens), H * (49 * d + 16 * dv + 256)
+    qkv, a, b = dev32(randn(T, 2 * G * d + H * dv, seed=1)), dev32(randn(T, H * d, seed=2)), dev32(randn(T, H, seed=3))
+    params = dev32(randn(H * d, seed=4)), dev32(randn(H, seed=5, scale=0.5) - 1.0)
+    start, got = dev32(randn(len(lens), ops.scan_state_floats(H, d, dv), seed=6)), []
+    for chunks in (64, 19, 18, 5, 2, 1):
+        monkeypatch.setattr(ops, "DELTA_CHUNKS_FLOATS", chunks * of_one + of_one // 2)
+        o, state, ctx = torch.empty((T, H * dv), device=DEV), start.clone(), state_ctx(lens, list(range(len(lens))))
+        if lengths_on_host:
+            ctx.q_lens = lens
+        ops.delta_scan(o, qkv.clone(), a.clone(), *params, b.clone(), ctx, state, H, G, d, dv, d ** -0.5, 1e-6)
+        got.append((o, state))
+    assert all(torch.equal(x, y) for other in got[1:] for x, y in zip(got[0], other))
+
+
+def test_scratch_memory_of_the_chunked_delta_rule_does_not_grow_with_the_step():
+    """12,000 tokens of 16 heads of 128 x 128 leave 411 MB for the walk; no more than 256 MB of them at a time."""
+    from photon_infer_amd import ops
+    ops.use_fast_kernels(True)
+    H, G, d, dv, T = 16, 16, 128, 128, 12000
+    rand = lambda *shape: torch.randn(*shape, device=DEV)
+    args = torch.empty((T, H * dv), device=DEV), rand(T, 2 * G * d + H * dv), rand(T, H * d), rand(H * d), rand(H), rand(T, H)
+    state, ctx = torch.zeros((1, ops.scan_state_floats(H, d, dv)), device=DEV), state_ctx([T], [0])
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    with library_calls() as names:
+        ops.delta_scan(*args, ctx, state, H, G, d, dv, d ** -0.5, 1e-6)
+    assert names == ["pi_delta_chunks"] and torch.cuda.max_memory_allocated() - before <= 256 << 20
+
+
 def test_delta_rule_of_more_requests_than_the_chunked_form_takes():
     """65,535 single tokens beside a request of 48: walked, the long one as it is alone."""
     from photon_infer_amd import ops
