@@ -321,7 +321,7 @@ __global__ __launch_bounds__(256) void gemm_skinny_kernel(void* __restrict__ Cv,
   }
 }
 
-// The same product for 33..128 tokens (from 17 on for large matrices, shares_activations), where the activations are as many bytes as a block's weights.  A block is eight waves
+// The same product for 33..128 tokens (from 17 on for large matrices, pi_gemm_skinny_shares), where the activations are as many bytes as a block's weights.  A block is eight waves
 // on 64 weight rows: wave w multiplies rows 32 (w / 4) .. + 31 with T tiles of 32 tokens (v_mfma_f32_32x32x16_bf16), and of
 // every step of 64 k takes the 16 of its quarter w % 4; the quarters are summed through LDS at the end.  So a step's
 // activations are read from LDS twice and not once per 16 rows, and the weights go into registers past LDS.  Activations go
@@ -830,12 +830,14 @@ static int launch_ring(int epi, dim3 grid, hipStream_t stream, void* C, long ldc
   return pi_fail("gemm_skinny: unknown epilogue %d", epi);
 }
 
-// Which of the two kernels: the caller sizes its k-split by the same rule (fast.py).  For 17 to 32 tokens the one that shares its
-// activations is the better one on matrices of some 40 MB and more (17 / 32 tokens, us, in the norm's or the head's place: 4,096 x 14,336
+// Which of the two kernels; the caller asks here, and sizes its k-split by the answer (fast.py).  For 17 to 32 tokens the one that shares
+// its activations is the better one on matrices of some 40 MB and more (17 / 32 tokens, us, in the norm's or the head's place: 4,096 x 14,336
 // 28.5 / 29.6 -> 26.5 / 26.7, 3,072 x 8,192 17.1 / 18.9 -> 16.0 / 16.3, 6,144 x 4,096 15.6 / 17.5 -> 15.7 / 16.1, 28,672 x 4,096 50.8 / 51.1 ->
 // 46.3 / 46.9, 128,256 x 4,096 199.8 / 211.1 -> 199.3 / 201.6) and the worse one below (2,048 x 8,192 13.0 / 13.5 -> 14.0 / 14.2, 2,048 x 2,048
-// 8.0 / 8.3 -> 8.4 / 8.7).
-static bool shares_activations(int M, int N, int K, long ldx, long ldw) {
+// 8.0 / 8.3 -> 8.4 / 8.7).  At the line, with the norm that adds the pieces: 5,120 x 4,096 17.8 / 19.1 -> 16.0 / 16.3, 2,560 x 8,192 15.8 /
+// 17.5 -> 15.5 / 15.9, 10,240 x 2,048 19.0 / 20.7 -> 18.5 / 19.9, 2,048 x 10,240 14.6 / 15.9 -> 14.8 / 15.2; with the gated unit 13.0 / 13.6 ->
+// 12.1 / 12.4 for 10,240 x 2,048.
+extern "C" int pi_gemm_skinny_shares(int M, int N, int K, long ldx, long ldw) {
   return M > SHARED_FROM_TOKENS || (M > 16 && (long)N * K >= SHARED_FROM_ELEMENTS && ldx < RING_MAX_STRIDE && ldw < RING_MAX_STRIDE && K < RING_MAX_STRIDE);
 }
 
@@ -855,7 +857,7 @@ extern "C" int pi_gemm_skinny(void* C, int epilogue, long ldc, const void* X, lo
   PI_REQUIRE(((uintptr_t)X % 16 == 0) && ((uintptr_t)W % 16 == 0), "gemm_skinny: operands must be 16-byte aligned");
   PI_REQUIRE(splits >= 1 && splits <= 65535, "gemm_skinny: bad split count %d", splits);
   PI_REQUIRE(epilogue != EPI_SWIGLU || (splits == 1 && N % 32 == 0), "gemm_skinny: the SwiGLU epilogue needs one split and N (%d) a multiple of 32", N);
-  const bool shared = shares_activations(M, N, K, ldx, ldw);
+  const bool shared = pi_gemm_skinny_shares(M, N, K, ldx, ldw);
   const int groups = ceil_div(N, shared ? RING_ROWS : ROWS_PER_BLOCK);
   const addressing::KSplit cut = addressing::cut_k(K, splits, KSTEP);
   const int kpb = cut.k_per_block;

@@ -30,8 +30,7 @@ EPI_BF16, EPI_F32, EPI_ACCUM, EPI_SWIGLU = 0, 1, 2, 3
 SKINNY_MAX_ROWS = 128          # up to this many tokens the weight-streaming kernels serve a product (measured against the tile kernel)
 ROWS_PER_BLOCK = 32            # weight rows per block of the skinny kernel
 BLOCKS_PER_UNIT = 2            # blocks of it wanted per compute unit to keep HBM busy (measured: 512 on 256 units; 384 and 768 are slower)
-SHARED_FROM_TOKENS = 32        # more tokens than this: the skinny kernel that shares activations per block ...
-SHARED_FROM_ELEMENTS = 20_000_000    # ... and more than 16 tokens on matrices of so many elements (both sides: shares_activations, gemm_skinny.hip)
+SHARED_FROM_TOKENS = 32        # more tokens than this: the skinny kernel that shares activations per block (from 17 on for large matrices: pi_gemm_skinny_shares) ...
 SHARED_ROWS_PER_BLOCK = 64     # ... with this many weight rows per block, and no more blocks than compute units (100 tokens, 3,072 x 8,192:
                                # 22.8 us in six pieces on 288 blocks, 16.9 in five on 240; 6,144 x 4,096 22.8 in three, 18.7 in two), though
                                # a unit would hold two: 64 tokens, k 4,096, blocks for half the units or more in one piece and in two, 8,256
@@ -94,9 +93,15 @@ def _skinny_splits(M: int, N: int, K: int) -> int:
     return _skinny_splits_of(M, N, K, compute_units())
 
 
+def _splits(M: int, N: int, K: int, lda: int, ldw: int) -> int:
+    """Pieces of k of the weight-streaming product; rows too far apart for the kernel that shares activations change it."""
+    stride = max(lda, ldw)
+    return _skinny_splits(M, N, K) if stride < RING_MAX_STRIDE else _skinny_splits_of(M, N, K, compute_units(), stride)
+
+
 @functools.lru_cache(maxsize=4096)
-def _skinny_splits_of(M: int, N: int, K: int, units: int) -> int:
-    if M > SHARED_FROM_TOKENS or (M > FEW_TOKENS and N * K >= SHARED_FROM_ELEMENTS):
+def _skinny_splits_of(M: int, N: int, K: int, units: int, stride: int = 0) -> int:
+    if _lib.load("bf16").pi_gemm_skinny_shares(M, N, K, stride, stride):
         # the kernel that shares an activation tile per block: at most one block per compute unit
         splits = units // -(-N // SHARED_ROWS_PER_BLOCK)
     else:
@@ -228,8 +233,8 @@ def _finish_ranges_blocks(M: int, N: int, heads: int, head_dim: int, count: int)
 def _finish(out, a, w, M, N, K, lda, ldw, next_norm, ws: KernelWorkspace, bias=None) -> bool:
     """out += a @ w^T of a few tokens by the kernel that also makes the next norm but for its root, left in the workspace (in
     the place of pieces of k, whose order of sums hangs on the step anyway; a product that is not cut keeps the one order that
-    steps up to 32 tokens have); False, and nothing done, where it does not take the product or the weights have no streaming copy.  ``a`` may be
-    ``KeyRanges``, where the kernel merges as many.  ``bias`` (float32 [N], not with ranges): added besides."""
+    steps up to 16 tokens have, and up to 32 on matrices below 20 million elements); False, and nothing done, where it does not
+    take the product or the weights have no streaming copy.  ``a`` may be ``KeyRanges``, where the kernel merges as many.  ``bias`` (float32 [N], not with ranges): added besides."""
     weight, eps = next_norm
     ranges = a if isinstance(a, KeyRanges) else None
     blocks = _finish_blocks(M, N, K) if ranges is None else _finish_ranges_blocks(M, N, ranges.heads, ranges.head_dim, ranges.count)
@@ -278,7 +283,7 @@ def gemm(out, a, w, accumulate, M, N, K, lda, ldw, ldc, may_defer=False, ws: Opt
         _lib.call("bf16", "pi_gemm_mfma", out.data_ptr(), epilogue, ldc, a.data_ptr(), lda, w.data_ptr(), ldw, M, N, K, 1,
                   _tile_shape(M, N, K, 1), _stream())
         return True
-    splits = _skinny_splits(M, N, K)
+    splits = _splits(M, N, K, lda, ldw)
     if may_defer and accumulate and splits > 1 and next_norm is not None and _finish(out, a, w, M, N, K, lda, ldw, next_norm, ws):
         return True
     if whole and splits > 1 and not may_defer and M <= FEW_TOKENS and K <= FEW_TOKENS_WHOLE_K and _rows(out.data_ptr(), epilogue, ldc, a, w, M, N, K, lda, ldw, ws):
@@ -467,7 +472,7 @@ def gemm_pieces(a, w, ws: Optional[KernelWorkspace], whole: bool = False, left: 
         if splits > 1:
             p = _tiles_in_pieces(a, w, M, N, K, lda, ldw, splits, ws)
     else:
-        splits = _skinny_splits(M, N, K)
+        splits = _splits(M, N, K, lda, ldw)
         if splits > 1:
             p = _skinny(0, EPI_F32, N, a, w, M, N, K, lda, ldw, splits, ws)
     if p is not None and p.splits > 1:

@@ -140,6 +140,28 @@ def test_pieces_that_would_not_fit_the_workspace_are_refused():
         assert fast._skinny_splits(M, N, K) * M * N <= GEMM_PART_FLOATS or fast._skinny_splits(M, N, K) == 1
 
 
+@pytest.mark.parametrize("M", [17, 32])
+def test_k_is_cut_for_the_kernel_that_a_product_of_17_to_32_tokens_takes(monkeypatch, M):
+    """On both sides of the line, and with rows so far apart that the kernel that shares activations does not take them."""
+    import torch
+
+    from photon_infer_amd.ops import fast
+    monkeypatch.setattr(fast, "compute_units", lambda: 256)
+    made = []
+    monkeypatch.setattr(fast, "_skinny", lambda *args: made.append(args[10]))
+
+    def pieces(N, K, lda, ldw):
+        a, w = (torch.empty_strided((rows, K), (stride, 1), dtype=torch.bfloat16) for rows, stride in ((M, lda), (N, ldw)))
+        assert fast.gemm(torch.empty(M, N), a, w, False, M, N, K, lda, ldw, N)
+        return made.pop()
+
+    long = fast.RING_MAX_STRIDE
+    assert pieces(5120, 4096, 4096, 4096) == pieces(5120, 4096, long - 8, 4096) == 3       # 80 blocks of 64 rows: one per unit
+    assert pieces(5120, 4096, long, 4096) == 4                                             # 160 blocks of 32 rows: two per unit
+    assert pieces(4872, 4096, 4096, 4096) == 4                                             # 19.96 million elements
+    assert pieces(8, 2560000, 2560000, 2560000) == 512                                     # k too long as well
+
+
 # (requests' tokens, contexts, heads, kv heads, head size, window, microseconds on the tile kernel, on the general kernel), measured
 FLOAT32_STEPS = [
     ([32], [2048], 32, 8, 64, 0, 150, 127), ([32], [32768], 32, 8, 64, 0, 2316, 1687), ([32], [32768], 24, 8, 128, 0, 3604, 2452),
