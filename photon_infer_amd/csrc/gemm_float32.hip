@@ -609,8 +609,10 @@ static Float32Plan cut(int tm, int tn, int K, int splits) {
 // way through memory and no launch, and a matrix of few rows is streamed by two blocks per unit whatever its k: eight tokens and
 // the norm, 2,048 x 2,048 12.4 -> 10.3 us, 3,072 x 2,048 13.1 -> 12.0; and some 2 us less for each product whose pieces a kernel
 // added.  A short k in blocks of 16 rows that nearly are the units' number stays whole (24 tokens and the norm, 3,072 x 768 10.6 us
-// and 14.6 in three pieces; 4,096 x 512 10.1 and 10.9).  More pieces have to promise a hundredth: 129 x 2,048 x 8,192 and the norm
-// takes 65 us in five and 76 in eight, which the rule holds for equal.
+// and 14.6 in three pieces; 4,096 x 512 10.1 and 10.9).  More pieces have to promise a hundredth: 1,050 x 6,144 x 4,096
+// and the norm takes 352 us whole and 386 in two, 500 x 6,144 x 4,096 180 in four and 184 in five, which the model holds for equal.  Most
+// matrices that it holds for equal would gain by more pieces (1,950 x 3,072 x 2,048 169 and 159, 570 x 4,096 x 4,096 129 in three and 124 in
+// five, 490 x 4,096 x 14,336 332 in four and 315 in eight; 63 x 5,120 x 3,072 30.5 and 30.4).
 static Float32Plan plan(int M, int N, int K, long part_floats, int after) {
   const int units = compute_units();
   const bool read_by_next = after == 1;
