@@ -286,14 +286,16 @@ def test_delta_rule_whole_in_portions_and_token_by_token(sizes):
 
 @pytest.mark.parametrize("sizes", [(4, 2, 64, 16), (2, 2, 128, 128), (2, 1, 192, 48), (1, 1, 256, 144)])
 @pytest.mark.parametrize("per_head", [False, True])
-def test_delta_rule_in_chunks_beside_single_tokens(sizes, per_head):
-    """Sixteen tokens at a time: whole and partial chunks, requests that walk beside them, a second portion on top; the
-    bounds of the walk's tests.  Step 2 holds no request that walks."""
+@pytest.mark.parametrize("lengths_on_host", [True, False])
+def test_delta_rule_in_chunks_beside_single_tokens(sizes, per_head, lengths_on_host):
+    """Sixteen tokens at a time: whole and partial chunks, requests that walk beside them, a second portion on top, in a step in
+    which none walks; the bounds of the walk's tests.  With the lengths on the host, as the engine has them, scratch memory is counted
+    exactly and the second step launches no walk; without them it is an upper bound."""
     from photon_infer_amd import ops
     ops.use_fast_kernels(True)
     H, G, d, dv = sizes
-    T = {"a": 131, "b": 3, "c": 19, "d": 64, "e": 5}
-    cuts = {"a": [48, 83], "b": [1, 2], "c": [3, 16], "d": [47, 17], "e": [2, 3]}
+    T = {"a": 131, "b": 4, "c": 19, "d": 64, "e": 5}
+    cuts = {"a": [48, 83], "b": [1, 3], "c": [3, 16], "d": [47, 17], "e": [2, 3]}
     A_log, dt_bias = randn(H, seed=1, scale=0.5) - 1.0, randn(H if per_head else H * d, seed=2)
     data = {n: delta_inputs(t, H, G, d, dv, 100 * i) for i, (n, t) in enumerate(T.items())}
     if per_head:
@@ -307,10 +309,12 @@ def test_delta_rule_in_chunks_beside_single_tokens(sizes, per_head):
         cat = lambda idx: torch.cat([data[n][idx][i:j].reshape(j - i, -1) for n, i, j in step])
         o = torch.full((sum(j - i for _, i, j in step) + 1, H * dv), 7.0, device=DEV)
         qkv, a, b = dev32(torch.cat([cat(0), cat(1), cat(2)], dim=1)), dev32(cat(3)), dev32(cat(4))
+        ctx = state_ctx([j - i for _, i, j in step], [slot[n] for n, _, _ in step])
+        if lengths_on_host:
+            ctx.q_lens = [j - i for _, i, j in step]
         with library_calls() as names:
-            ops.delta_scan(o[:-1], qkv, a, dev32(dt_bias), dev32(A_log), b, state_ctx([j - i for _, i, j in step], [slot[n] for n, _, _ in step]),
-                           state[:, :-3], H, G, d, dv, d ** -0.5, 1e-6, kind="head_delta" if per_head else "channel_delta")
-        assert names == ["pi_delta_chunks", "pi_delta_scan"], number
+            ops.delta_scan(o[:-1], qkv, a, dev32(dt_bias), dev32(A_log), b, ctx, state[:, :-3], H, G, d, dv, d ** -0.5, 1e-6, kind="head_delta" if per_head else "channel_delta")
+        assert names == ["pi_delta_chunks"] + ["pi_delta_scan"] * (number == 0 or not lengths_on_host), number
         assert bool((o[-1] == 7.0).all())
         for (n, i, j), part in zip(step, torch.split(o[:-1], [j - i for _, i, j in step])):
             got[n].append(part)
