@@ -226,7 +226,7 @@ static bool parts(const Shape& s, long lda, long ldw, const Tiles& t) {
   return true;
 }
 
-// ------------------------------------------------------------------ 33..128 tokens
+// ------------------------------------------------------------------ 33..128 tokens, 17..128 on large matrices
 // The activations are a tile of 64 or 128 rows; of the weights a block's eight waves take 32 rows by a quarter of each step's
 // k each.  A fetch that is used lies inside its descriptor, at the row and k that the fragment stands for, and any other
 // outside (it reads zeros).
@@ -357,9 +357,8 @@ static bool check(const Shape& s) {
     if (s.M <= 32) {
       if (!skinny(s, ld, ld, 0, 2, A::KSTEP)) return false;
       if (s.M <= 16 && s.K % 64 == 0 && !skinny(s, ld, ld, 0, 4, 4 * A::KSTEP)) return false;     // the form that merges key ranges
-    } else if (s.M <= 128) {
-      if (!ring(s, ld, ld, 0)) return false;
     }
+    if (s.M > 16 && s.M <= 128 && !ring(s, ld, ld, 0)) return false;
     for (const Tiles& t : BFLOAT16_TILES)
       if (!tiles(s, ld, ld, t, 1)) return false;
   }
@@ -377,7 +376,7 @@ static bool check(const Shape& s) {
   if (s.N % 16 == 0 && s.K % 64 == 0) {                // the streaming copy of the weights
     if (s.M <= 32 && !skinny(s, s.K, s.K, 1, 2, A::KSTEP)) return false;
     if (s.M <= 16 && !skinny(s, s.K, s.K, 1, 4, 4 * A::KSTEP)) return false;
-    if (s.M > 32 && s.M <= 128 && !ring(s, s.K, s.K, 1)) return false;
+    if (s.M > 16 && s.M <= 128 && !ring(s, s.K, s.K, 1)) return false;
     if (s.M <= 16 && (!few_rows(s, s.K) || !few_rows(s, s.K + 8))) return false;
   }
   return true;

@@ -24,6 +24,7 @@ SHORT_RANGES = [(4, 50, 160), (9, 40, 344), (12, 776, 272), (3, 64, 200), (16, 3
 KERNEL_TEST_SHAPES = [(1, 14, 3), (2, 2, 3), (5, 176, 64), (33, 100, 72), (64, 384, 128), (70, 1001, 96), (1, 256, 64),
                       (130, 64, 200), (257, 320, 136), (8, 2048, 512), (300, 520, 264), (40, 200, 1032), (64, 72, 520),
                       (48, 1001, 96), (35, 130, 2048)]
+KERNEL_TEST_SHAPES += [(17, 5008, 4032), (32, 9777, 2056), (25, 100, 72), (31, 1001, 96), (20, 384, 64)]      # 17 to 32 tokens: two kernels
 MODEL_SHAPES = [(m, n, k) for m in (1, 8, 16, 33, 64, 128, 2048) for n, k in ((3072, 2048), (2048, 2048), (16384, 2048), (2048, 8192))]
 
 
