@@ -18,6 +18,8 @@
 #define ROWS_MAX_M 32                 // up to this many rows of activations the weight-streaming kernel is taken
 #define ROWS_SPLIT_MIN_K 4096         // from this k on a product's pieces are worth a kernel that adds them
 #define ROWS_WHOLE_K 768              // up to this k a matrix of many rows is left whole for its reader too
+#define FEW_TILES_ROWS 64             // rows and columns of a tile of float32 instructions
+#define FEW_TILES_BUFFERS 4           // slabs of it in LDS
 #define PARTS_WIDE_MAX_STRIDE (1 << 20)  // floats between weight rows up to which 256 of them lie within a descriptor's 2 GB
 
 // What becomes of a product in one piece: stored, added to C, or, with gate and up rows interleaved in blocks of 16 in W,
@@ -257,15 +259,16 @@ __device__ inline void finish_tiles(const f32x16_t (&acc)[WM][WN], long m_wave, 
   }
 }
 
-// Few tiles: TM x TN (64 x 64 is the one in use), four waves in 2 x 2, slabs of 32 floats of k that go from memory straight into
-// LDS through a ring of NB buffers (rows of 128 bytes, their 16-byte pieces turned by (row / 2) % 8 as in gemm_mfma.hip).  A block
+// Few tiles: 64 x 64, four waves in 2 x 2, slabs of 32 floats of k that go from memory straight into LDS through a ring of four
+// buffers (rows of 128 bytes, their 16-byte pieces turned by (row / 2) % 8 as in gemm_mfma.hip).  A block
 // of these starts and steps faster than one of gemm_float32_parts_kernel: 0.6 us per 32 floats of k alone on its unit, where 64 x 64
 // in parts take 0.9 (a chain of conversion, store, barrier and six products on one accumulator).
-template <int TM, int TN, int NB, int EPI>
+template <int EPI>
 __global__ __launch_bounds__(256) void gemm_float32_tile_kernel(float* __restrict__ C, long ldc, const float* __restrict__ A, long lda,
                                                                 const float* __restrict__ W, long ldw, int M, int N, int K, int tiles_n,
                                                                 int k_per_split, float* __restrict__ part) {
   extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
+  constexpr int TM = FEW_TILES_ROWS, TN = FEW_TILES_ROWS, NB = FEW_TILES_BUFFERS;
   constexpr int ROW = 64;                        // a row of a slab: 128 bytes, in units of two
   constexpr int AI = TM / 32, WI = TN / 32;      // load instructions of a wave per slab: eight rows each
   constexpr int WM = TM / 64, WN = TN / 64;      // a wave's 32 x 32 tiles
@@ -384,11 +387,12 @@ __global__ __launch_bounds__(256) void gemm_float32_tile_kernel(float* __restric
 // four ahead (2 % either way), tiles of 64 x 64 and 64 x 128 in parts.
 //
 // An infinity has no such parts (the rest would be NaN), neither has a float that rounds to one (above 3.39e38); a row whose largest
-// float, within the block's k, is below 2^-100 loses its last parts (of a larger row's small floats less is lost than its sums round off:
-// 2^-134 each); and the product of two leading parts may overflow where the floats' does not.  Outputs of such a row of A or W, and
-// infinite ones, are made from memory with float32 instructions, 32 x 32 at a time, in the order of gemm_float32_tile_kernel; the others
-// stay as they are, so that no row's bits hang on what its neighbours hold.  (One infinity in A, 2,048 x 16,384 x 2,048: 620 us become
-// 1,080; 378 x 3,072 x 2,048: 41 and 94.  A NaN needs nothing: its row or column is NaN either way.)
+// float, within the block's k, is below 2^-100 loses its last parts (of a larger row's small floats 2^-134 each, less than its sums
+// round off unless they meet zeros wherever the row is large); and the product of two leading parts may overflow where the floats' does
+// not.  Outputs of such a row of A or W, and infinite ones, are made from memory with float32 instructions, 32 x 32 at a time, in the
+// order of gemm_float32_tile_kernel; the others stay as they are, so that no row's bits hang on what its neighbours hold.  (One infinity
+// in A, 2,048 x 16,384 x 2,048: 620 us become 1,080; 378 x 3,072 x 2,048: 41 and 94.  A NaN needs nothing: its row or column is NaN
+// either way.)
 // Four floats on their way into parts, in steps of some five instructions each: step 2 q + i makes part q of floats 2 i and 2 i + 1.
 struct PartsOf4 {
   float r[4];
@@ -625,8 +629,8 @@ static Float32Plan plan(int M, int N, int K, long part_floats, int after) {
     return cut(0, 0, K, splits < 1 ? 1 : splits);
   }
   static const struct { int tm, tn; float start, per_k, paired, out; } shapes[] = {      // us, us per k of one block, share of that where two blocks go side by side, us per MB
-      {64, 64, 3.07f, 0.01937f, 0.871f, 0.236f}, {128, 128, 2.75f, 0.04363f, 0.790f, 0.267f}, {192, 128, 3.10f, 0.05737f, 0.838f, 0.301f}, {128, 256, 4.25f, 0.06864f, 0.889f, 0.326f}};
-  Float32Plan best = {64, 64, 1, K};
+      {FEW_TILES_ROWS, FEW_TILES_ROWS, 3.07f, 0.01937f, 0.871f, 0.236f}, {128, 128, 2.75f, 0.04363f, 0.790f, 0.267f}, {192, 128, 3.10f, 0.05737f, 0.838f, 0.301f}, {128, 256, 4.25f, 0.06864f, 0.889f, 0.326f}};
+  Float32Plan best = {FEW_TILES_ROWS, FEW_TILES_ROWS, 1, K};
   float least = 0.f;
   const float megabytes = (float)M * N * 4e-6f;
   for (const auto& s : shapes) {
@@ -650,15 +654,15 @@ extern "C" int pi_gemm_float32_pieces(int M, int N, int K, long part_floats, int
   return M > 0 && N > 0 && K > 0 ? plan(M, N, K, part_floats, after).splits : 1;
 }
 
-template <int TM, int TN, int NB, int EPI>
-static int launch_tiles_of(float* C, long ldc, const float* A, long lda, const float* W, long ldw, int M, int N, int K, const Float32Plan& p, float* part,
+template <int EPI>
+static int launch_few_tiles(float* C, long ldc, const float* A, long lda, const float* W, long ldw, int M, int N, int K, const Float32Plan& p, float* part,
                            hipStream_t stream) {
-  constexpr size_t bytes = (size_t)NB * (TM + TN) * 128;
-  static const hipError_t configured = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_float32_tile_kernel<TM, TN, NB, EPI>),
+  constexpr size_t bytes = (size_t)FEW_TILES_BUFFERS * 2 * FEW_TILES_ROWS * 128;
+  static const hipError_t configured = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_float32_tile_kernel<EPI>),
                                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
   if (configured != hipSuccess) return pi_fail("gemm_float32: cannot reserve %zu bytes of LDS: %s", bytes, hipGetErrorString(configured));
-  const int tiles_n = ceil_div(N, TN);
-  hipLaunchKernelGGL((gemm_float32_tile_kernel<TM, TN, NB, EPI>), dim3((unsigned)(ceil_div(M, TM) * (long)tiles_n), p.splits), dim3(256), bytes, stream, C, ldc,
+  const int tiles_n = ceil_div(N, FEW_TILES_ROWS);
+  hipLaunchKernelGGL((gemm_float32_tile_kernel<EPI>), dim3((unsigned)(ceil_div(M, FEW_TILES_ROWS) * (long)tiles_n), p.splits), dim3(256), bytes, stream, C, ldc,
                      A, lda, W, ldw, M, N, K, tiles_n, p.k_per_split, part);
   return pi_check_launch("gemm_float32 (tiles)");
 }
@@ -679,7 +683,7 @@ static int launch_parts(float* C, long ldc, const float* A, long lda, const floa
 template <int EPI>
 static int launch_tiles(float* C, long ldc, const float* A, long lda, const float* W, long ldw, int M, int N, int K, const Float32Plan& p, float* part,
                         hipStream_t stream) {
-  if (p.tm == 64) return launch_tiles_of<64, 64, 4, EPI>(C, ldc, A, lda, W, ldw, M, N, K, p, part, stream);
+  if (p.tm == FEW_TILES_ROWS) return launch_few_tiles<EPI>(C, ldc, A, lda, W, ldw, M, N, K, p, part, stream);
   if (p.tm == 192) return launch_parts<3, 2, EPI>(C, ldc, A, lda, W, ldw, M, N, K, p, part, stream);
   if (p.tn == 256 && ldw <= PARTS_WIDE_MAX_STRIDE) return launch_parts<2, 4, EPI>(C, ldc, A, lda, W, ldw, M, N, K, p, part, stream);
   return launch_parts<2, 2, EPI>(C, ldc, A, lda, W, ldw, M, N, K, p, part, stream);
