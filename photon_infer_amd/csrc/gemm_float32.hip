@@ -414,7 +414,7 @@ struct PartsOf4 {
   }
 };
 
-constexpr float PARTS_LARGEST = 3.3895313892515355e38f, PARTS_SMALLEST = 0x1p-100f;
+constexpr float PARTS_LARGEST = 3.3895313892515355e38f, PARTS_SMALLEST = 0x1p-100f, PARTS_OVERFLOW = 0x1p48f;      // K < 2^29: sums of smaller floats stay below 2^126
 
 template <int WM, int WN, int EPI>
 __global__ __launch_bounds__(256, 2) void gemm_float32_parts_kernel(float* __restrict__ C, long ldc, const float* __restrict__ A, long lda,
@@ -522,23 +522,16 @@ __global__ __launch_bounds__(256, 2) void gemm_float32_parts_kernel(float* __res
   }
 
   block_barrier_keeping_loads<0>();              // everybody is done with LDS
-  int* met = reinterpret_cast<int*>(lds);        // whether there is an element to be made again; then, per row of A and W, whether it has no parts
+  int* met = reinterpret_cast<int*>(lds);        // whether an element may have to be made again; then, per row of A and W, whether it has no parts
   if (tid == 0) *met = 0;
   __syncthreads();
-  float largest = 0.f;
-#pragma unroll
-  for (int i = 0; i < WM; ++i)
-#pragma unroll
-    for (int j = 0; j < WN; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; v += 2) asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(largest) : "v"(acc[i][j][v]), "v"(acc[i][j][v + 1]));
-  bool odd = !(largest < INFINITY);
+  bool odd = false;                              // whether this thread knows of a row without parts, or of one with which a sum may overflow
 #pragma unroll
   for (int p = 0; p < LOADS; ++p) {
     const float t = fmaxf(top[p], dpp_move<0xB1>(top[p])), of_row = fmaxf(t, dpp_move<0x4E>(t));      // four lanes to a row
     const bool none = !(of_row <= PARTS_LARGEST) || (of_row > 0.f && of_row < PARTS_SMALLEST);
     if (piece == 0) met[1 + p * 64 + tid / 4] = none;
-    odd = odd || none;
+    odd = odd || none || of_row >= PARTS_OVERFLOW;
   }
   if (__any(odd) && lane == 0) atomicOr(met, 1);
   __syncthreads();
