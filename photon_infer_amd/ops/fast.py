@@ -93,10 +93,9 @@ def _skinny_splits(M: int, N: int, K: int) -> int:
     return _skinny_splits_of(M, N, K, compute_units())
 
 
-def _splits(M: int, N: int, K: int, lda: int, ldw: int) -> int:
-    """Pieces of k of the weight-streaming product; rows too far apart for the kernel that shares activations change it."""
-    stride = max(lda, ldw)
-    return _skinny_splits(M, N, K) if stride < RING_MAX_STRIDE else _skinny_splits_of(M, N, K, compute_units(), stride)
+def _far_rows_splits(M: int, N: int, K: int) -> int:
+    """The same where rows are too far apart for the kernel that shares activations."""
+    return _skinny_splits_of(M, N, K, compute_units(), RING_MAX_STRIDE)
 
 
 @functools.lru_cache(maxsize=4096)
@@ -283,7 +282,7 @@ def gemm(out, a, w, accumulate, M, N, K, lda, ldw, ldc, may_defer=False, ws: Opt
         _lib.call("bf16", "pi_gemm_mfma", out.data_ptr(), epilogue, ldc, a.data_ptr(), lda, w.data_ptr(), ldw, M, N, K, 1,
                   _tile_shape(M, N, K, 1), _stream())
         return True
-    splits = _splits(M, N, K, lda, ldw)
+    splits = _skinny_splits(M, N, K) if lda < RING_MAX_STRIDE > ldw else _far_rows_splits(M, N, K)
     if may_defer and accumulate and splits > 1 and next_norm is not None and _finish(out, a, w, M, N, K, lda, ldw, next_norm, ws):
         return True
     if whole and splits > 1 and not may_defer and M <= FEW_TOKENS and K <= FEW_TOKENS_WHOLE_K and _rows(out.data_ptr(), epilogue, ldc, a, w, M, N, K, lda, ldw, ws):
@@ -472,7 +471,7 @@ def gemm_pieces(a, w, ws: Optional[KernelWorkspace], whole: bool = False, left: 
         if splits > 1:
             p = _tiles_in_pieces(a, w, M, N, K, lda, ldw, splits, ws)
     else:
-        splits = _splits(M, N, K, lda, ldw)
+        splits = _skinny_splits(M, N, K) if lda < RING_MAX_STRIDE > ldw else _far_rows_splits(M, N, K)
         if splits > 1:
             p = _skinny(0, EPI_F32, N, a, w, M, N, K, lda, ldw, splits, ws)
     if p is not None and p.splits > 1:
