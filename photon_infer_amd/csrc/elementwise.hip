@@ -40,6 +40,51 @@ extern "C" int pi_embedding(float* out, const void* table, int table_dtype, cons
   return pi_check_launch("embedding");
 }
 
+// ------------------------------------------------------------------ copies of rows
+// out[m] = in[rows[m]] of one array or two, byte for byte, in units of as many bytes as addresses, strides and widths allow.  A row
+// beyond the array gives bytes of ones, a NaN in either type.  Bound by its launch: one token's stream and activations (12 KB) 1.8 us, 1,024 tokens' 4.8; a library's copies of them were two
+// launches of 4.5, and loading their module took the first prompt of a process 70 to 140 ms.
+struct RowsOf {
+  char* out;
+  const char* in;
+  long stride;        // bytes between rows of `in`; rows of `out` follow each other
+  int bytes, unit;    // of a row, of a unit
+};
+
+template <typename U> __device__ inline void copy_row(char* to, const char* from, int bytes) {
+  for (int i = threadIdx.x; i < bytes / (int)sizeof(U); i += blockDim.x) reinterpret_cast<U*>(to)[i] = reinterpret_cast<const U*>(from)[i];
+}
+
+__global__ __launch_bounds__(256) void copy_rows_kernel(const RowsOf first, const RowsOf second, const int* __restrict__ rows, int count) {
+  const RowsOf& of = blockIdx.y ? second : first;
+  const long m = blockIdx.x;
+  const int row = rows[m];
+  char* to = of.out + m * of.bytes;
+  if (row < 0 || row >= count) {
+    for (int i = threadIdx.x; i < of.bytes; i += blockDim.x) to[i] = (char)0xff;
+    return;
+  }
+  const char* from = of.in + row * of.stride;
+  if (of.unit == 16) copy_row<uint4>(to, from, of.bytes);
+  else if (of.unit == 4) copy_row<uint32_t>(to, from, of.bytes);
+  else copy_row<uint16_t>(to, from, of.bytes);
+}
+
+static RowsOf rows_of(void* out, const void* in, long stride, int bytes) {
+  const uintptr_t all = (uintptr_t)out | (uintptr_t)in | (uintptr_t)stride | (uintptr_t)bytes;
+  return RowsOf{(char*)out, (const char*)in, stride, bytes, all % 16 == 0 ? 16 : all % 4 == 0 ? 4 : 2};
+}
+
+// M rows of `in` (and of `in2` unless it is null), which have `count` rows each, `stride` bytes apart, `bytes` of them wanted.
+extern "C" int pi_copy_rows(void* out, const void* in, long stride, int bytes, void* out2, const void* in2, long stride2, int bytes2,
+                            const int* rows, int M, int count, hipStream_t stream) {
+  PI_REQUIRE(M >= 0 && count > 0 && bytes > 0 && bytes % 2 == 0 && stride >= bytes && stride % 2 == 0, "copy_rows: bad sizes M=%d of %d, %d bytes, %ld apart", M, count, bytes, stride);
+  PI_REQUIRE(!in2 || (bytes2 > 0 && bytes2 % 2 == 0 && stride2 >= bytes2 && stride2 % 2 == 0), "copy_rows: bad sizes of the second array, %d bytes, %ld apart", bytes2, stride2);
+  if (M == 0) return 0;
+  hipLaunchKernelGGL(copy_rows_kernel, dim3(M, in2 ? 2 : 1), dim3(256), 0, stream, rows_of(out, in, stride, bytes), rows_of(out2, in2, stride2, bytes2), rows, count);
+  return pi_check_launch("copy_rows");
+}
+
 // x <- cap * tanh(x / cap) over n float32 numbers, in place (logits that are capped on the way out).
 __global__ void softcap_kernel(float* __restrict__ x, long n, float cap) {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;

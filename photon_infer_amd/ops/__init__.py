@@ -234,6 +234,25 @@ def whole_norm(h):
     return out
 
 
+def copy_rows(rows: torch.Tensor, *tensors: torch.Tensor) -> tuple:
+    """Copies of the rows that ``rows`` (int32) names of tensors [T, any] with T rows each, two of them per launch.  A row beyond the
+    tensors gives a NaN row, no fault."""
+    _gpu(rows, *tensors)
+    M, T = rows.numel(), tensors[0].shape[0] if tensors else 0
+    _i32(rows, "rows to copy", M)
+    for t in tensors:
+        if t.dim() != 2 or t.shape[0] != T or t.stride(1) != 1 or t.element_size() not in (2, 4):
+            raise KernelError(f"copy of rows: wants [{T}, any] with 16 or 32 bits, columns side by side, got {t.dtype} {tuple(t.shape)} strides {t.stride()}")
+    made = tuple(torch.empty((M, t.shape[1]), dtype=t.dtype, device=t.device) for t in tensors)
+    for i in range(0, len(tensors) if M else 0, 2):
+        args = []
+        for out, t in zip(made[i:i + 2], tensors[i:i + 2]):
+            size = t.element_size()
+            args += [out.data_ptr(), t.data_ptr(), (t.stride(0) if T > 1 else t.shape[1]) * size, t.shape[1] * size]
+        _lib.call("core", "pi_copy_rows", *args, *([None, None, 0, 0] if len(args) == 4 else []), rows.data_ptr(), M, T, _stream())
+    return made
+
+
 def discard_deferred(x: torch.Tensor, ws: Optional[KernelWorkspace]) -> None:
     """Forget a pending update of ``x`` (the stream is not read again)."""
     pieces = ws.take_pending(x) if ws is not None else None

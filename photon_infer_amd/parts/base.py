@@ -20,6 +20,7 @@ from typing import Any, Callable, Dict, List, Optional, Sequence, Tuple
 
 import torch
 
+from .. import ops
 from ..errors import UnsupportedModelError
 from ..weights.loader import TensorSpec
 
@@ -157,7 +158,8 @@ def cut_rows(ctx: StepContext, *tensors: torch.Tensor):
     """Copies of the rows of ``tensors`` that ``ctx.read_rows`` names (what has only them already, from a mixer beside, as it is:
     they are half of the step's tokens at most)."""
     rows = ctx.read_rows
-    return tuple(t if t.shape[0] == rows.shape[0] else t.index_select(0, rows) for t in tensors)
+    made = iter(ops.copy_rows(rows, *(t for t in tensors if t.shape[0] != rows.shape[0])))
+    return tuple(t if t.shape[0] == rows.shape[0] else next(made) for t in tensors)
 
 
 # --------------------------------------------------------------------------- part bases

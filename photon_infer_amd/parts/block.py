@@ -173,7 +173,7 @@ class PreNormBlock(Block):
             h, x = self.norm2.forward(added, ctx), added
         else:                                        # the norm adds what is pending to those rows
             h = self.norm2.forward(x, ctx, rows=rows)
-            x = x.index_select(0, rows)
+            x, = ops.copy_rows(rows, x)
         ctx.may_defer, ctx.next_norm = ctx.after_block_consumes, ctx.after_block_norm
         self.ffn.forward(h, x, ctx)
         ctx.may_defer, ctx.next_norm = False, None

@@ -36,6 +36,7 @@ def logits_of_steps(folder, dtype, monkeypatch, cuts=True):
 
     with monkeypatch.context() as m:
         m.setattr(PreNormBlock, "forward_last", seen)
+        m.setattr(torch.Tensor, "index_select", None)      # a library's kernel: loading its module took the first prompt 70 to 140 ms
         cut = [runner.step([StepEntry("a", long, [149])]),
                runner.step([StepEntry("b", short, [])]),
                runner.step([StepEntry("c", other, [139, 5]), StepEntry("b", [7], []), StepEntry("a", [9], [0])]),
@@ -70,6 +71,27 @@ def test_rows_that_nobody_reads_change_nothing(tmp_path, monkeypatch, tiny, name
         # block by one place (2^-8 of it), of which a logit adds up many with either sign
         bound = 3e-5 if dtype == "float32" else 2.0 ** -6
         assert (got - ref).abs().max() <= bound * max(1.0, ref.abs().max().item())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T,D,M", [(1, 1, 1), (40, 2048, 1), (40, 7, 5), (300, 1030, 150), (9, 4100, 3), (33, 64, 0)])
+def test_copies_of_rows(T, D, M, dtype):
+    """Widths and addresses for units of 16, 4 and 2 bytes, strides, one, two and three tensors, rows that are not there."""
+    from photon_infer_amd import ops
+    from photon_infer_amd.errors import KernelError
+    wide, x = randn(T, D + 9, seed=1).to(dtype).to(DEV), randn(T, D + 3, seed=2).float().to(DEV)
+    rows = torch.randperm(T, generator=torch.Generator().manual_seed(3))[:M].to(torch.int32).to(DEV)
+    for tensors in ([x], [x, wide], [wide[:, 8:8 + D], x], [wide[:, 1:1 + D], x[:, 1:], wide]):
+        made = ops.copy_rows(rows, *tensors)
+        assert len(made) == len(tensors)
+        assert all(torch.equal(m, t[rows.long()]) and m.is_contiguous() for m, t in zip(made, tensors))
+    if M:
+        rows[0], rows[-1] = T, -1 if M > 1 else T
+        made = ops.copy_rows(rows, x, wide)
+        for m, t in zip(made, (x, wide)):
+            assert m[0].isnan().all() and m[-1].isnan().all() and torch.equal(m[1:-1], t[rows[1:-1].long()])
+    with pytest.raises(KernelError, match="columns side by side"):
+        ops.copy_rows(rows, x[:, :2 * (D // 2):2] if D > 1 else x.double())
 
 
 # mixers that say that they cut rows and that no design above has in such a block: (kind, parameters)
