@@ -42,8 +42,9 @@ extern "C" int pi_embedding(float* out, const void* table, int table_dtype, cons
 
 // ------------------------------------------------------------------ copies of rows
 // out[m] = in[rows[m]] of one array or two, byte for byte, in units of as many bytes as addresses, strides and widths allow.  A row
-// beyond the array gives bytes of ones, a NaN in either type.  Bound by its launch: one token's stream and activations (12 KB) 1.8 us, 1,024 tokens' 4.8; a library's copies of them were two
-// launches of 4.5, and loading their module took the first prompt of a process 70 to 140 ms.
+// beyond the array gives bytes of ones, a NaN in either type.  Bound by its launch: one token's stream and activations (12 KB) 1.8 us
+// alone, 4.8 in a step; a library's copies of them were two launches of 4.5, and loading their module took the first prompt of a
+// process 70 to 140 ms.
 struct RowsOf {
   char* out;
   const char* in;

@@ -569,7 +569,7 @@ __global__ __launch_bounds__(256, 2) void gemm_float32_parts_kernel(float* __res
     f32x16_t made[1][1];
 #pragma unroll
     for (int v = 0; v < 16; ++v) made[0][0][v] = 0.f;
-#pragma unroll 4
+#pragma unroll 1
     for (int k = k_lo / 2; k < k_hi / 2; k += 8) {
       const int at = k + lane / 32 * 4;          // K is a multiple of 4: the upper lanes' may lie beyond it
       f32x4_t fa = {0.f, 0.f, 0.f, 0.f}, fb = fa;
